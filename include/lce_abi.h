@@ -223,6 +223,40 @@ int lce_ppo_loss_packed(const float* log_prob_packed, const float* entropy_packe
                         float batch_num_tokens, float global_batch_size, float loss_scale_factor, float* out,
                         float* g_log_prob_packed, float* g_entropy_packed, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same loss as a forward / backward pair, for autograd: the forward leaves the gradients unscaled, the backward
+ * multiplies them with the row weights and with the upstream gradient of the loss while it writes them (one launch
+ * instead of a scaling pass and two elementwise products).  Fields as in the two functions above, and
+ *   mask with mask_kind LCE_PPO_MASK_*: fp32 weights, or elements of which the non-zero ones count 1 (what the reference's
+ *     `.to(bool)` makes of a response mask), read in the type they have
+ *   total_nnz >= 0: log_prob, entropy and the gradients are PACKED [total_nnz]; prompt_lens and response_lens [rows] int64
+ *     on the device.  With attention_mask (not NULL; element type LCE_PPO_MASK_U8, _I32 or _I64, row stride
+ *     attention_stride, the first prompt_width columns are the prompts') the two are OUTPUTS: the forward counts them.
+ *     total_nnz < 0: everything is [rows, row_len].
+ *   g_log_prob / g_entropy: unscaled gradients, kept for the backward, like the workspace
+ *   d_log_prob / d_entropy: written by lce_ppo_backward (either may be NULL); g_loss: fp32 on the device
+ * Packed: when lce_ppo_forward returns, checks[0] = sum of all lengths, checks[1] = number of prompts of length 0,
+ * checks[2] = longest response are on the HOST (the call waits for the kernel that adds them up, not for the loss): the
+ * reference's assertions are the caller's.  Rows that fail them have meaningless gradients; nothing is written outside the
+ * vectors.  Not for a capturing stream, for that reason. */
+enum { LCE_PPO_MASK_F32 = 0, LCE_PPO_MASK_U8 = 1, LCE_PPO_MASK_I32 = 2, LCE_PPO_MASK_I64 = 3, LCE_PPO_MASK_F32_NONZERO = 4 };
+typedef struct {
+  const float *log_prob, *entropy, *old_log_prob, *advantages;
+  const void* mask;
+  const float *is_weights, *ref_log_prob;
+  const void* attention_mask;
+  int64_t *prompt_lens, *response_lens;
+  float *out, *g_log_prob, *g_entropy;
+  void* workspace;
+  const float* g_loss;
+  float *d_log_prob, *d_entropy;
+  int64_t total_nnz, rows, row_len, attention_stride, prompt_width, attention_width, workspace_bytes;
+  int64_t checks[3];
+  int mask_kind, attention_kind, kl_type, agg_mode;
+  float kl_coef, clip_low, clip_high, clip_c, entropy_coeff, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor;
+} lce_ppo_call_t;
+int lce_ppo_forward(lce_ppo_call_t* call, void* stream);
+int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
+
 /* Product-level options (process-wide; every entry point works from one snapshot of the settings taken when it starts).
  * LCE_OPT_WORKSPACE_BUDGET (default 0 = the built-in rule, chunks of 8192 vocabulary columns or wider while one
  * d_logits buffer stays within 256 MiB): a byte count; lce_backward_workspace_bytes with vocab_chunk <= 0 then

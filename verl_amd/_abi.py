@@ -53,6 +53,8 @@ SYMBOLS = {
     "lce_ppo_loss_workspace_bytes": (_sz, [_i64, _i64]),
     "lce_ppo_loss": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _f, _i64, _i64, _i, _f, _f, _f, _f, _f, _f, _f, _f, _p, _p, _p, _p, _sz, _p]),
     "lce_ppo_loss_packed": (_i, [_p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _i, _f, _i64, _i64, _i, _f, _f, _f, _f, _f, _f, _f, _f, _p, _p, _p, _p, _sz, _p]),
+    "lce_ppo_forward": (_i, [_p, _p]),
+    "lce_ppo_backward": (_i, [_p, _p]),
     "lce_gemm_nt": (_i, [_p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i64, _i, _i, _p]),
     "lce_gemm_tn": (_i, [_p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i64, _i, _p]),
     "lce_set_variant": (_i, [_i]),
@@ -63,6 +65,19 @@ SYMBOLS = {
     "lce_profile_class_name": (_c.c_char_p, [_i]),
     "lce_profile_read": (_i, [_p, _p, _i]),
 }
+
+# lce_ppo_call_t
+class PpoCall(_c.Structure):
+    _fields_ = (
+        [(n, _p) for n in ("log_prob", "entropy", "old_log_prob", "advantages", "mask", "is_weights", "ref_log_prob", "attention_mask",
+                           "prompt_lens", "response_lens", "out", "g_log_prob", "g_entropy", "workspace", "g_loss", "d_log_prob", "d_entropy")]
+        + [(n, _i64) for n in ("total_nnz", "rows", "row_len", "attention_stride", "prompt_width", "attention_width", "workspace_bytes")]
+        + [("checks", _i64 * 3)]
+        + [(n, _i) for n in ("mask_kind", "attention_kind", "kl_type", "agg_mode")]
+        + [(n, _f) for n in ("kl_coef", "clip_low", "clip_high", "clip_c", "entropy_coeff", "dp_size", "batch_num_tokens",
+                             "global_batch_size", "loss_scale_factor")]
+    )  # fmt: skip
+
 
 _lib = None
 _lock = threading.Lock()

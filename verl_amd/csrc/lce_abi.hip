@@ -493,7 +493,128 @@ size_t lce_ppo_loss_workspace_bytes(int64_t rows, int64_t row_len) {
   int64_t seg_len;
   ppo_geometry(rows, row_len, &segs, &seg_len);
   return ppo_align((size_t)rows * segs * 8 * sizeof(float)) + ppo_align((size_t)rows * 4 * sizeof(double)) +
-         ppo_align((size_t)rows * sizeof(float));
+         ppo_align((size_t)rows * sizeof(float)) + ppo_align((size_t)rows * sizeof(int64_t));
+}
+
+// Host-visible words a kernel reports into while the host waits: pinned slots, handed out per call and given back, at
+// most kMaxHostSlots of them kept (one per thread that is inside such a call at the same time).
+struct HostSlot {
+  int64_t* host = nullptr;
+  int64_t seq = 0;
+};
+static std::mutex g_slot_mu;
+static std::vector<HostSlot> g_slots;
+static constexpr size_t kMaxHostSlots = 16;
+
+static int take_slot(HostSlot* s) {
+  {
+    std::lock_guard<std::mutex> l(g_slot_mu);
+    if (!g_slots.empty()) {
+      *s = g_slots.back();
+      g_slots.pop_back();
+      return LCE_OK;
+    }
+  }
+  void* p = nullptr;
+  if (hipHostMalloc(&p, 64, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) return fail(LCE_E_LAUNCH, "hipHostMalloc failed");
+  s->host = static_cast<int64_t*>(p);
+  s->host[3] = 0;
+  s->seq = 0;
+  return LCE_OK;
+}
+
+static void give_slot(const HostSlot& s) {
+  {
+    std::lock_guard<std::mutex> l(g_slot_mu);
+    if (g_slots.size() < kMaxHostSlots) {
+      g_slots.push_back(s);
+      return;
+    }
+  }
+  (void)hipHostFree(s.host);
+}
+
+// Waits until the kernel has stored `seq` in the slot.  The word is watched rather than an event: the answer is there as
+// soon as the kernel's first workgroup has it, with the launches behind it still running.  Ends when the stream has
+// finished (or failed) without it.
+static int wait_slot(const HostSlot& s, hipStream_t st) {
+  const auto arrived = [&] { return __atomic_load_n(&s.host[3], __ATOMIC_ACQUIRE) == s.seq; };
+  for (;;) {
+    for (int i = 0; i < 2000; ++i) {
+      if (arrived()) return LCE_OK;
+      __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipErrorNotReady) continue;
+    if (arrived()) return LCE_OK;
+    return fail(LCE_E_LAUNCH, "ppo loss: %s", e == hipSuccess ? "the lengths were not reported" : hipGetErrorString(e));
+  }
+}
+
+// the arguments of one call, checked; kernels' arguments and the workspace's parts
+struct PpoPlan {
+  PpoArgs p;
+  PpoAgg g;
+  double* row_tot;
+  float *row_weight, *out;
+  unsigned blocks;
+};
+
+static int ppo_plan(const lce_ppo_call_t& c, PpoPlan* plan) {
+  if (c.rows <= 0 || c.row_len <= 0) return fail(LCE_E_ARG, "ppo loss: rows and row_len must be positive");
+  if (c.rows > ((int64_t)1 << 30) || c.row_len > ((int64_t)1 << 40) / c.rows) return fail(LCE_E_ARG, "ppo loss: too many elements");
+  if (!c.mask || !c.out) return fail(LCE_E_ARG, "null pointer");
+  if (c.mask_kind < PPO_MASK_F32 || c.mask_kind > PPO_MASK_F32_NONZERO) return fail(LCE_E_ARG, "ppo loss: unknown mask_kind %d", c.mask_kind);
+  if (c.log_prob) {
+    if (!c.old_log_prob || !c.advantages || !c.g_log_prob) return fail(LCE_E_ARG, "null pointer");
+    if (!(c.clip_c > 1.f)) return fail(LCE_E_ARG, "clip_ratio_c must be greater than 1");
+  } else if (!c.entropy || c.g_log_prob || c.kl_type != LCE_PPO_KL_NONE) {
+    return fail(LCE_E_ARG, "without log_prob the call aggregates `entropy` alone");
+  }
+  if ((c.entropy == nullptr) != (c.g_entropy == nullptr)) return fail(LCE_E_ARG, "entropy and g_entropy go together");
+  const int kl_base = c.kl_type & ~LCE_PPO_KL_STRAIGHT_THROUGH;
+  if (kl_base < LCE_PPO_KL_NONE || kl_base > LCE_PPO_KL_K3 || (kl_base == LCE_PPO_KL_NONE && c.kl_type != LCE_PPO_KL_NONE))
+    return fail(LCE_E_ARG, "ppo loss: unknown kl_type %d", c.kl_type);
+  if (kl_base != LCE_PPO_KL_NONE && !c.ref_log_prob) return fail(LCE_E_ARG, "the KL penalty needs ref_log_prob");
+  if (c.agg_mode < PPO_TOKEN_MEAN || c.agg_mode > PPO_SEQ_MEAN_TOKEN_MEAN) return fail(LCE_E_ARG, "Invalid loss_agg_mode: %d", c.agg_mode);
+  if (!(c.dp_size > 0.f)) return fail(LCE_E_ARG, "ppo loss: dp_size must be positive");
+  PpoArgs& p = plan->p;
+  ppo_geometry(c.rows, c.row_len, &p.segs, &p.seg_len);
+  const int64_t blocks = c.rows * p.segs;
+  if (blocks > 0x7fffffff) return fail(LCE_E_ARG, "ppo loss: too many rows");
+  plan->blocks = (unsigned)blocks;
+  plan->out = c.out;
+  char* ws = static_cast<char*>(c.workspace);
+  p.partials = reinterpret_cast<float*>(ws);
+  ws += ppo_align((size_t)blocks * 8 * sizeof(float));
+  plan->row_tot = reinterpret_cast<double*>(ws);
+  ws += ppo_align((size_t)c.rows * 4 * sizeof(double));
+  plan->row_weight = reinterpret_cast<float*>(ws);
+  ws += ppo_align((size_t)c.rows * sizeof(float));
+  p.start_out = reinterpret_cast<int64_t*>(ws);  // (only with prompt_len)
+  p.log_prob = c.log_prob; p.entropy = c.entropy; p.old_log_prob = c.old_log_prob; p.advantages = c.advantages;
+  p.mask = c.mask; p.mask_kind = c.mask_kind;
+  p.is_weights = c.is_weights; p.rows = c.rows; p.row_len = c.row_len;
+  p.ref_log_prob = c.ref_log_prob; p.kl_type = kl_base; p.kl_coef = c.kl_coef;
+  // (k2's own gradient is already the straight-through one, verl/trainer/ppo/core_algos.py:2203-2204)
+  p.kl_straight_through = (c.kl_type & LCE_PPO_KL_STRAIGHT_THROUGH) != 0 && kl_base != LCE_PPO_KL_K2;
+  p.clip_low = c.clip_low; p.clip_high = c.clip_high; p.clip_c = c.clip_c; p.entropy_coeff = c.entropy_coeff;
+  p.g_log_prob = c.g_log_prob; p.g_entropy = c.g_entropy;
+  p.pk_start = nullptr; p.pk_len = nullptr; p.prompt_len = nullptr; p.checks = nullptr; p.check_seq = 0; p.total_nnz = c.total_nnz;
+  PpoAgg& g = plan->g;
+  g.mode = c.agg_mode; g.dp_size = c.dp_size; g.batch_num_tokens = c.batch_num_tokens; g.global_batch_size = c.global_batch_size;
+  g.loss_scale_factor = c.loss_scale_factor; g.entropy_coeff = c.entropy_coeff;
+  g.kl_coef = kl_base != LCE_PPO_KL_NONE ? c.kl_coef : 0.f;
+  return LCE_OK;
+}
+
+static int ppo_launch_forward(const PpoPlan& plan, hipStream_t st) {
+  int rc;
+  hipLaunchKernelGGL(ppo_terms_kernel, dim3(plan.blocks), dim3(256), 0, st, plan.p);
+  if ((rc = check_launch("ppo_terms_kernel"))) return rc;
+  hipLaunchKernelGGL(ppo_finish_kernel, dim3(1), dim3(256), 0, st, plan.p.partials, plan.p.rows, plan.p.segs, plan.p.row_len, plan.g,
+                     plan.row_tot, plan.row_weight, plan.out);
+  return check_launch("ppo_finish_kernel");
 }
 
 // shared body of lce_ppo_loss and lce_ppo_loss_packed
@@ -503,50 +624,21 @@ static int ppo_entry(const float* log_prob, const float* entropy, const int64_t*
                      float clip_high, float clip_c, float entropy_coeff, float dp_size, float batch_num_tokens,
                      float global_batch_size, float loss_scale_factor, float* out, float* g_log_prob, float* g_entropy,
                      void* workspace, size_t workspace_bytes, void* stream) {
-  if (rows <= 0 || row_len <= 0) return fail(LCE_E_ARG, "ppo loss: rows and row_len must be positive");
-  if (rows > ((int64_t)1 << 30) || row_len > ((int64_t)1 << 40) / rows) return fail(LCE_E_ARG, "ppo loss: too many elements");
-  if (!mask || !out) return fail(LCE_E_ARG, "null pointer");
-  if (log_prob) {
-    if (!old_log_prob || !advantages || !g_log_prob) return fail(LCE_E_ARG, "null pointer");
-    if (!(clip_c > 1.f)) return fail(LCE_E_ARG, "clip_ratio_c must be greater than 1");
-  } else if (!entropy || g_log_prob || kl_type != LCE_PPO_KL_NONE) {
-    return fail(LCE_E_ARG, "without log_prob the call aggregates `entropy` alone");
-  }
-  if ((entropy == nullptr) != (g_entropy == nullptr)) return fail(LCE_E_ARG, "entropy and g_entropy go together");
+  lce_ppo_call_t c = {};
+  c.log_prob = log_prob; c.entropy = entropy; c.total_nnz = total_nnz; c.old_log_prob = old_log_prob; c.advantages = advantages;
+  c.mask = mask; c.mask_kind = LCE_PPO_MASK_F32; c.is_weights = is_weights; c.ref_log_prob = ref_log_prob; c.kl_type = kl_type;
+  c.kl_coef = kl_coef; c.rows = rows; c.row_len = row_len; c.agg_mode = agg_mode; c.clip_low = clip_low; c.clip_high = clip_high;
+  c.clip_c = clip_c; c.entropy_coeff = entropy_coeff; c.dp_size = dp_size; c.batch_num_tokens = batch_num_tokens;
+  c.global_batch_size = global_batch_size; c.loss_scale_factor = loss_scale_factor; c.out = out; c.g_log_prob = g_log_prob;
+  c.g_entropy = g_entropy; c.workspace = workspace;
   if ((pk_start == nullptr) != (pk_len == nullptr)) return fail(LCE_E_ARG, "packed layout: starts and lengths go together");
   if (pk_start && total_nnz < 0) return fail(LCE_E_ARG, "packed layout: total_nnz must be >= 0");
-  const int kl_base = kl_type & ~LCE_PPO_KL_STRAIGHT_THROUGH;
-  if (kl_base < LCE_PPO_KL_NONE || kl_base > LCE_PPO_KL_K3 || (kl_base == LCE_PPO_KL_NONE && kl_type != LCE_PPO_KL_NONE))
-    return fail(LCE_E_ARG, "ppo loss: unknown kl_type %d", kl_type);
-  if (kl_base != LCE_PPO_KL_NONE && !ref_log_prob) return fail(LCE_E_ARG, "the KL penalty needs ref_log_prob");
-  if (agg_mode < PPO_TOKEN_MEAN || agg_mode > PPO_SEQ_MEAN_TOKEN_MEAN) return fail(LCE_E_ARG, "Invalid loss_agg_mode: %d", agg_mode);
-  if (!(dp_size > 0.f)) return fail(LCE_E_ARG, "ppo loss: dp_size must be positive");
-  if (!workspace || workspace_bytes < lce_ppo_loss_workspace_bytes(rows, row_len))
-    return fail(LCE_E_WORKSPACE, "ppo workspace too small");
+  PpoPlan plan;
+  int rc = ppo_plan(c, &plan);
+  if (rc) return rc;
+  if (!workspace || workspace_bytes < lce_ppo_loss_workspace_bytes(rows, row_len)) return fail(LCE_E_WORKSPACE, "ppo workspace too small");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  PpoArgs p;
-  ppo_geometry(rows, row_len, &p.segs, &p.seg_len);
-  const int64_t blocks = rows * p.segs;
-  if (blocks > 0x7fffffff) return fail(LCE_E_ARG, "ppo loss: too many rows");
-  char* ws = static_cast<char*>(workspace);
-  p.partials = reinterpret_cast<float*>(ws);
-  ws += ppo_align((size_t)blocks * 8 * sizeof(float));
-  double* row_tot = reinterpret_cast<double*>(ws);
-  ws += ppo_align((size_t)rows * 4 * sizeof(double));
-  float* row_weight = reinterpret_cast<float*>(ws);
-  p.log_prob = log_prob; p.entropy = entropy; p.old_log_prob = old_log_prob; p.advantages = advantages; p.mask = mask;
-  p.is_weights = is_weights; p.rows = rows; p.row_len = row_len;
-  p.ref_log_prob = ref_log_prob; p.kl_type = kl_base; p.kl_coef = kl_coef;
-  // (k2's own gradient is already the straight-through one, verl/trainer/ppo/core_algos.py:2203-2204)
-  p.kl_straight_through = (kl_type & LCE_PPO_KL_STRAIGHT_THROUGH) != 0 && kl_base != LCE_PPO_KL_K2;
-  p.clip_low = clip_low; p.clip_high = clip_high; p.clip_c = clip_c; p.entropy_coeff = entropy_coeff;
-  p.g_log_prob = g_log_prob; p.g_entropy = g_entropy;
-  p.pk_start = pk_start; p.pk_len = pk_len; p.total_nnz = total_nnz;
-  PpoAgg g;
-  g.mode = agg_mode; g.dp_size = dp_size; g.batch_num_tokens = batch_num_tokens; g.global_batch_size = global_batch_size;
-  g.loss_scale_factor = loss_scale_factor; g.entropy_coeff = entropy_coeff;
-  g.kl_coef = kl_base != LCE_PPO_KL_NONE ? kl_coef : 0.f;
-  int rc;
+  plan.p.pk_start = pk_start; plan.p.pk_len = pk_len;
   if (pk_start && total_nnz > 0) {
     // packed gradients: the positions no response token maps to (prompts, the last token of each sequence) are zeros
     for (float* gp : {g_log_prob, g_entropy}) {
@@ -556,12 +648,82 @@ static int ppo_entry(const float* log_prob, const float* entropy, const int64_t*
       if ((rc = check_launch("fill_zero_kernel"))) return rc;
     }
   }
-  hipLaunchKernelGGL(ppo_terms_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
-  if ((rc = check_launch("ppo_terms_kernel"))) return rc;
-  hipLaunchKernelGGL(ppo_finish_kernel, dim3(1), dim3(256), 0, st, p.partials, rows, p.segs, row_len, g, row_tot,
-                     row_weight, out);
-  if ((rc = check_launch("ppo_finish_kernel"))) return rc;
-  hipLaunchKernelGGL(ppo_scale_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p, row_weight);
+  if ((rc = ppo_launch_forward(plan, st))) return rc;
+  hipLaunchKernelGGL(ppo_scale_kernel, dim3(plan.blocks), dim3(256), 0, st, plan.p, plan.row_weight, static_cast<const float*>(nullptr), g_log_prob,
+                     g_entropy);
+  return check_launch("ppo_scale_kernel");
+}
+
+// what lce_ppo_forward and lce_ppo_backward check and set up alike
+static int ppo_call_plan(const lce_ppo_call_t* call, PpoPlan* plan) {
+  if (!call) return fail(LCE_E_ARG, "null call");
+  const bool packed = call->total_nnz >= 0;
+  int rc = ppo_plan(*call, plan);
+  if (rc) return rc;
+  if (packed && (!call->log_prob || !call->prompt_lens || !call->response_lens)) return fail(LCE_E_ARG, "ppo loss (packed): null pointer");
+  if (!call->workspace || (size_t)call->workspace_bytes < lce_ppo_loss_workspace_bytes(call->rows, call->row_len))
+    return fail(LCE_E_WORKSPACE, "ppo workspace too small");
+  if (packed) {
+    plan->p.prompt_len = call->prompt_lens;
+    plan->p.pk_len = call->response_lens;
+  }
+  return LCE_OK;
+}
+
+int lce_ppo_forward(lce_ppo_call_t* call, void* stream) {
+  PpoPlan plan;
+  int rc = ppo_call_plan(call, &plan);
+  if (rc) return rc;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (call->total_nnz < 0) return ppo_launch_forward(plan, st);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+    return fail(LCE_E_ARG, "ppo loss (packed): the lengths are checked on the host, which a capturing stream does not allow");
+  if (call->attention_mask) {
+    if (call->prompt_width < 0 || call->attention_width < call->prompt_width || call->attention_stride < call->attention_width)
+      return fail(LCE_E_ARG, "ppo loss: bad attention mask shape");
+    const dim3 grid((unsigned)call->rows), block(256);
+    const int64_t ld = call->attention_stride, pw = call->prompt_width, w = call->attention_width;
+    switch (call->attention_kind) {
+      case LCE_PPO_MASK_U8:
+        hipLaunchKernelGGL(ppo_lengths_kernel<uint8_t>, grid, block, 0, st, static_cast<const uint8_t*>(call->attention_mask), ld, pw, w, call->prompt_lens, call->response_lens);
+        break;
+      case LCE_PPO_MASK_I32:
+        hipLaunchKernelGGL(ppo_lengths_kernel<int32_t>, grid, block, 0, st, static_cast<const int32_t*>(call->attention_mask), ld, pw, w, call->prompt_lens, call->response_lens);
+        break;
+      case LCE_PPO_MASK_I64:
+        hipLaunchKernelGGL(ppo_lengths_kernel<int64_t>, grid, block, 0, st, static_cast<const int64_t*>(call->attention_mask), ld, pw, w, call->prompt_lens, call->response_lens);
+        break;
+      default: return fail(LCE_E_ARG, "ppo loss: unknown attention_kind %d", call->attention_kind);
+    }
+    if ((rc = check_launch("ppo_lengths_kernel"))) return rc;
+  }
+  HostSlot slot;
+  if ((rc = take_slot(&slot))) return rc;
+  void* dev = nullptr;
+  if (hipHostGetDevicePointer(&dev, slot.host, 0) != hipSuccess) {
+    give_slot(slot);
+    return fail(LCE_E_LAUNCH, "hipHostGetDevicePointer failed");
+  }
+  slot.seq += 1;
+  plan.p.checks = static_cast<int64_t*>(dev);
+  plan.p.check_seq = slot.seq;
+  rc = ppo_launch_forward(plan, st);
+  // (a failed launch may still leave a kernel on its way that writes the slot: it is left alone, not reused)
+  if (rc || (rc = wait_slot(slot, st))) return rc;
+  for (int k = 0; k < 3; ++k) call->checks[k] = slot.host[k];
+  give_slot(slot);
+  return LCE_OK;
+}
+
+int lce_ppo_backward(const lce_ppo_call_t* call, void* stream) {
+  PpoPlan plan;
+  int rc = ppo_call_plan(call, &plan);
+  if (rc) return rc;
+  if (!call->g_loss) return fail(LCE_E_ARG, "null pointer");
+  if ((call->d_log_prob && !call->g_log_prob) || (call->d_entropy && !call->g_entropy)) return fail(LCE_E_ARG, "ppo loss: a gradient that the forward did not leave");
+  hipLaunchKernelGGL(ppo_scale_kernel, dim3(plan.blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), plan.p, plan.row_weight, call->g_loss,
+                     call->d_log_prob, call->d_entropy);
   return check_launch("ppo_scale_kernel");
 }
 

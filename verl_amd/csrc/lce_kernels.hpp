@@ -1382,7 +1382,8 @@ struct PpoArgs {
   const float* entropy;   // may be null
   const float* old_log_prob;
   const float* advantages;
-  const float* mask;
+  const void* mask;         // elements of type mask_kind
+  int mask_kind;            // PPO_MASK_*: fp32 weights as they are, or any type of which the non-zero elements count 1
   const float* is_weights;  // may be null: per-token factor on the policy loss (rollout correction), a constant
   const float* ref_log_prob;  // with kl_type != PPO_KL_NONE
   int kl_type;
@@ -1403,13 +1404,114 @@ struct PpoArgs {
   const int64_t* pk_start;
   const int64_t* pk_len;
   int64_t total_nnz;
+  // With prompt_len (then pk_len holds the response lengths and pk_start is null) the starts are added up here from the
+  // lengths, left in start_out [rows] for the backward, and the positions no response token maps to get their zero
+  // gradients here as well.  checks (host memory, may be null) receives what the caller has to refuse: [0] sum of all
+  // lengths, [1] prompts of length 0, [2] longest response, and then check_seq in [3].
+  const int64_t* prompt_len;
+  int64_t* start_out;
+  int64_t* checks;
+  int64_t check_seq;
+};
+
+enum { PPO_MASK_F32 = 0, PPO_MASK_U8 = 1, PPO_MASK_I32 = 2, PPO_MASK_I64 = 3, PPO_MASK_F32_NONZERO = 4 };
+
+LCE_DEV float ppo_mask(const PpoArgs& p, int64_t t) {
+  switch (p.mask_kind) {  // (uniform over the launch)
+    case PPO_MASK_F32: return static_cast<const float*>(p.mask)[t];
+    case PPO_MASK_U8: return static_cast<const uint8_t*>(p.mask)[t] != 0 ? 1.f : 0.f;
+    case PPO_MASK_I32: return static_cast<const int32_t*>(p.mask)[t] != 0 ? 1.f : 0.f;
+    case PPO_MASK_I64: return static_cast<const int64_t*>(p.mask)[t] != 0 ? 1.f : 0.f;
+    default: return static_cast<const float*>(p.mask)[t] != 0.f ? 1.f : 0.f;
+  }
+}
+
+// where row `row` sits in the packed model-output vectors: element c at start + c for c < len
+struct PpoRow {
+  int64_t start, len;
 };
 
 // index of element (row, c) in the model-output vectors, or -1 for a padding position of the packed layout
-LCE_DEV int64_t ppo_out_index(const PpoArgs& p, int64_t row, int64_t c) {
-  if (!p.pk_start) return row * p.row_len + c;
-  const int64_t i = p.pk_start[row] + c;
-  return (c < p.pk_len[row] && i >= 0 && i < p.total_nnz) ? i : -1;
+LCE_DEV int64_t ppo_out_index(const PpoArgs& p, const PpoRow& r, int64_t row, int64_t c) {
+  if (!p.pk_len) return row * p.row_len + c;
+  const int64_t i = r.start + c;
+  return (c < r.len && i >= 0 && i < p.total_nnz) ? i : -1;
+}
+
+// sum over a workgroup of 256 threads, the same in every thread; `part` holds one value per wave
+LCE_DEV int64_t ppo_sum256(int64_t v, int64_t* part) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return part[0] + part[1] + part[2] + part[3];
+}
+
+// Lengths of the prompt and the response of every row of a padded batch: how many positions of the two parts of its
+// attention mask row count (the sum of the elements, as the reference takes it).  One workgroup of 256 threads per row.
+template <typename T>
+__global__ __launch_bounds__(256) void ppo_lengths_kernel(const T* attention_mask, int64_t ld, int64_t prompt_width, int64_t width,
+                                                          int64_t* prompt_len, int64_t* resp_len) {
+  __shared__ int64_t part[4];
+  const T* row = attention_mask + (int64_t)blockIdx.x * ld;
+  int64_t n[2] = {0, 0};
+  for (int64_t c = threadIdx.x; c < prompt_width; c += 256) n[0] += (int64_t)row[c];
+  for (int64_t c = prompt_width + threadIdx.x; c < width; c += 256) n[1] += (int64_t)row[c];
+  const int64_t np = ppo_sum256(n[0], part), nr = ppo_sum256(n[1], part);
+  if (threadIdx.x == 0) {
+    prompt_len[blockIdx.x] = np;
+    resp_len[blockIdx.x] = nr;
+  }
+}
+
+// Packed rows whose lengths are all that is known: every workgroup adds up the lengths before its row itself (a batch
+// has some hundred rows at most; a launch of its own for the prefix sum would cost more), the row's first workgroup
+// zeroes the gradients of the positions that no response token maps to (the prompt but for its last position, and the
+// sequence's last), and workgroup 0 reports what the host has to check.
+LCE_DEV PpoRow ppo_row_from_lengths(const PpoArgs& p, int64_t row, bool first) {
+  __shared__ int64_t part[4];
+  int64_t before = 0;
+  for (int64_t b = threadIdx.x; b < row; b += 256) before += p.prompt_len[b] + p.pk_len[b];
+  before = ppo_sum256(before, part);
+  const int64_t np = p.prompt_len[row];
+  const PpoRow r = {before + np - 1, p.pk_len[row]};
+  if (first) {
+    if (threadIdx.x == 0) p.start_out[row] = r.start;
+    const int64_t last = r.start + r.len;
+    for (int64_t i = before + threadIdx.x; i <= r.start; i += 256) {
+      const int64_t at = i < r.start ? i : last;
+      if (at < 0 || at >= p.total_nnz) continue;  // (lengths that do not fit the outputs: the host refuses them)
+      p.g_log_prob[at] = 0.f;
+      if (p.g_entropy) p.g_entropy[at] = 0.f;
+    }
+  }
+  if (blockIdx.x == 0 && p.checks) {
+    int64_t total = 0, empty = 0, longest = 0;
+    for (int64_t b = threadIdx.x; b < p.rows; b += 256) {
+      const int64_t n = p.pk_len[b];
+      total += p.prompt_len[b] + n;
+      empty += p.prompt_len[b] == 0;
+      longest = n > longest ? n : longest;
+    }
+    total = ppo_sum256(total, part);
+    empty = ppo_sum256(empty, part);
+    for (int off = 32; off > 0; off >>= 1) {
+      const int64_t o = __shfl_xor(longest, off);
+      longest = o > longest ? o : longest;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = longest;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 0; w < 4; ++w) longest = part[w] > longest ? part[w] : longest;
+      p.checks[0] = total;
+      p.checks[1] = empty;
+      p.checks[2] = longest;
+      __threadfence_system();
+      __hip_atomic_store(&p.checks[3], p.check_seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  return r;
 }
 
 // Per-token terms and unscaled gradients; workgroup (row, seg) reduces its segment of one row to
@@ -1420,10 +1522,13 @@ inline __global__ void ppo_terms_kernel(PpoArgs p) {
   const int64_t row = (int64_t)blockIdx.x / p.segs;
   const int64_t c0 = ((int64_t)blockIdx.x % p.segs) * p.seg_len;
   const int64_t c1 = c0 + p.seg_len < p.row_len ? c0 + p.seg_len : p.row_len;
+  PpoRow at = {0, 0};
+  if (p.prompt_len) at = ppo_row_from_lengths(p, row, c0 == 0);
+  else if (p.pk_start) at = {p.pk_start[row], p.pk_len[row]};
   for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) {
     const int64_t t = row * p.row_len + c;
-    const int64_t to = ppo_out_index(p, row, c);
-    const float m = p.mask[t];
+    const int64_t to = ppo_out_index(p, at, row, c);
+    const float m = ppo_mask(p, t);
     const bool on = m != 0.f;  // values outside the mask never reach a sum (NaNs there are harmless)
     float loss = 0.f, dloss = 0.f, nkl = 0.f, clipped = 0.f, dual_clipped = 0.f;
     if (p.log_prob) {
@@ -1586,16 +1691,32 @@ inline __global__ void ppo_finish_kernel(const float* partials, int64_t rows, in
   }
 }
 
-inline __global__ void ppo_scale_kernel(PpoArgs p, const float* row_weight) {
+// d_log_prob, d_entropy = the unscaled gradients of ppo_terms_kernel times the row's weight (and times *g_loss, the
+// upstream gradient of the loss, where there is one).  In and out may be the same vectors.  Packed rows whose starts were
+// added up from the lengths cover their whole sequence, so nothing has to be cleared beforehand.
+inline __global__ void ppo_scale_kernel(PpoArgs p, const float* row_weight, const float* g_loss, float* d_log_prob, float* d_entropy) {
   const int64_t row = (int64_t)blockIdx.x / p.segs;
   const int64_t c0 = ((int64_t)blockIdx.x % p.segs) * p.seg_len;
   const int64_t c1 = c0 + p.seg_len < p.row_len ? c0 + p.seg_len : p.row_len;
-  const float scale = row_weight[row];
+  const float scale = row_weight[row], up = g_loss ? *g_loss : 1.f;
+  PpoRow at = {0, 0};
+  if (p.pk_len) at = {p.prompt_len ? p.start_out[row] : p.pk_start[row], p.pk_len[row]};
+  auto one = [&](int64_t t, float w, float u) {
+    if (d_log_prob) d_log_prob[t] = p.g_log_prob[t] * w * u;
+    if (d_entropy) d_entropy[t] = p.g_entropy[t] * w * u;
+  };
   for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) {
-    const int64_t t = ppo_out_index(p, row, c);
-    if (t < 0) continue;
-    if (p.g_log_prob) p.g_log_prob[t] *= scale;
-    if (p.g_entropy) p.g_entropy[t] *= scale;
+    const int64_t t = ppo_out_index(p, at, row, c);
+    if (t >= 0) one(t, scale, up);
+  }
+  if (p.prompt_len && c0 == 0) {
+    const int64_t before = at.start - p.prompt_len[row] + 1, last = at.start + at.len;
+    for (int64_t i = before + threadIdx.x; i <= at.start; i += blockDim.x) {
+      const int64_t t = i < at.start ? i : last;
+      if (t < 0 || t >= p.total_nnz) continue;
+      if (d_log_prob) d_log_prob[t] = 0.f;
+      if (d_entropy) d_entropy[t] = 0.f;
+    }
   }
 }
 

@@ -29,10 +29,14 @@ _FOLD = {AggregationType.MEAN: np.mean, AggregationType.SUM: np.sum, Aggregation
 
 def reduce_metrics(metrics: dict) -> dict:
     """``verl/utils/metric/utils.py:25-58``: folds every entry in place: a ``Metric`` by its own rule, a plain list by
-    ``np.max`` / ``np.min`` when the key contains "max" / "min", else ``np.mean``."""
+    ``np.max`` / ``np.min`` when the key contains "max" / "min", else ``np.mean``.  Device scalars that nobody has looked at
+    yet are read back for all entries together."""
+    _read_back([m for m in metrics.values() if isinstance(m, Metric)])
     for key, val in metrics.items():
         if isinstance(val, Metric):
             metrics[key] = val.aggregate()
+        elif type(val) is float:  # (what every one of the three makes of a single number)
+            metrics[key] = np.float64(val)
         elif "max" in key:
             metrics[key] = np.max(val)
         elif "min" in key:
@@ -40,6 +44,28 @@ def reduce_metrics(metrics: dict) -> dict:
         else:
             metrics[key] = np.mean(val)
     return metrics
+
+
+def _read_back(metrics: list) -> None:
+    """Replaces the pending device scalars of ``metrics`` by their values, in one copy: of the tensor they are elements
+    of where they share one (a loss reports its statistics as one small vector), else of a stack of them."""
+    pending = [(m, i) for m in metrics for i, v in enumerate(m._items) if isinstance(v, torch.Tensor)]
+    if not pending:
+        return
+    scalars = [m._items[i] for m, i in pending]
+    whole = scalars[0].untyped_storage()
+    if len(scalars) > 1 and whole.nbytes() <= 1024 and all(
+        v.dtype == torch.float32 and v.untyped_storage().data_ptr() == whole.data_ptr() for v in scalars
+    ):
+        flat = scalars[0].as_strided((whole.nbytes() // 4,), (1,), 0).tolist()
+        host = [flat[v.storage_offset()] for v in scalars]
+    elif len(scalars) == 1:
+        host = [float(scalars[0].item())]
+    else:
+        device = scalars[0].device
+        host = torch.stack([v.reshape(()).to(device, torch.float32) for v in scalars]).cpu().tolist()
+    for (m, i), x in zip(pending, host):
+        m._items[i] = x
 
 
 class Metric:
@@ -55,11 +81,7 @@ class Metric:
     def values(self) -> list:
         """The observations as plain numbers, like the reference's attribute; pending device scalars are read back here,
         all of them in one copy."""
-        pending = [i for i, v in enumerate(self._items) if isinstance(v, torch.Tensor)]
-        if pending:
-            host = torch.stack([self._items[i].reshape(()).float() for i in pending]).cpu().tolist()
-            for i, x in zip(pending, host):
-                self._items[i] = x
+        _read_back([self])
         return self._items
 
     @values.setter
@@ -102,7 +124,10 @@ class Metric:
         return list(self.values)
 
     def aggregate(self) -> float:
-        return _FOLD[self.aggregation](self.numbers())
+        numbers = self.values
+        if len(numbers) == 1 and type(numbers[0]) is float:  # (one observation: every rule returns it)
+            return np.float64(numbers[0])
+        return _FOLD[self.aggregation](list(numbers))
 
     @classmethod
     def aggregate_dp(cls, metric_lists: list["Metric"]) -> float:

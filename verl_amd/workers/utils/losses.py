@@ -9,6 +9,7 @@ ready vectors instead of an elementwise autograd graph.  Metric names are the re
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -54,106 +55,126 @@ def agg_numbers(loss_agg_mode, dp_size, batch_num_tokens, global_batch_size, los
     )
 
 
+MASK_F32, MASK_U8, MASK_I32, MASK_I64, MASK_F32_NONZERO = range(5)
+_INT_MASKS = {torch.bool: MASK_U8, torch.uint8: MASK_U8, torch.int32: MASK_I32, torch.int64: MASK_I64}
+
+
+def _f32(t, numel):
+    """``t`` as a contiguous fp32 vector of ``numel`` elements (itself where it is one)."""
+    if t is None:
+        return None
+    if t.dtype != torch.float32:
+        t = t.to(torch.float32)
+    assert t.numel() == numel, "all inputs have the shape of log_prob"
+    return t if t.is_contiguous() else t.contiguous()
+
+
+class _Packed:
+    """Packed model outputs: where the lengths of prompts and responses come from.  Either both vectors, or the attention
+    mask of a padded batch (its first ``prompt_width`` columns are the prompts'), from which the kernel counts them."""
+
+    __slots__ = ("prompt_lens", "response_lens", "attention_mask", "prompt_width", "checks")
+
+    def __init__(self, prompt_lens=None, response_lens=None, attention_mask=None, prompt_width=0):
+        self.prompt_lens, self.response_lens = prompt_lens, response_lens
+        self.attention_mask, self.prompt_width = attention_mask, prompt_width
+        self.checks = None  # (sum of all lengths, prompts of length 0, longest response), filled in by the forward
+
+
 class _FusedPPOLoss(torch.autograd.Function):
-    """``log_prob`` may be None: then the call is ``agg_loss`` of ``entropy`` (the C ABI's aggregation-only form)."""
+    """``log_prob`` may be None: then the call is ``agg_loss`` of ``entropy`` (the C ABI's aggregation-only form).
+    ``packed`` (a ``_Packed``): ``log_prob`` / ``entropy`` are ``[total_nnz]`` over the packed sequences, everything else is
+    ``[batch, max_response_len]``.  ``nonzero_mask``: every non-zero element of the mask counts 1."""
 
     @staticmethod
     def forward(ctx, log_prob, entropy, old_log_prob, advantages, response_mask, is_weights, ref_log_prob, agg, kl,
-                clip_low, clip_high, clip_c, entropy_coeff, packed=None):
-        if packed is not None:
-            return _FusedPPOLoss._forward_packed(ctx, log_prob, entropy, old_log_prob, advantages, response_mask, is_weights,
-                                                 ref_log_prob, agg, kl, clip_low, clip_high, clip_c, entropy_coeff, packed)
+                clip_low, clip_high, clip_c, entropy_coeff, packed=None, nonzero_mask=False):
         lead = log_prob if log_prob is not None else entropy
         assert lead.is_cuda, "fused_ppo_loss runs on the GPU only"
         dev = lead.device
-        shape = lead.shape
-
-        def f32(t):
-            return None if t is None else t.detach().reshape(-1).to(torch.float32).contiguous()
-
-        lp, ent, old, adv, mask = f32(log_prob), f32(entropy), f32(old_log_prob), f32(advantages), f32(response_mask)
-        isw, ref = f32(is_weights), f32(ref_log_prob)
-        n = lead.numel()
-        for t in (lp, ent, old, adv, mask, isw, ref):
-            assert t is None or t.numel() == n, "all inputs have the shape of log_prob"
-        # rows are the sequences the seq-mean modes average over: the last dimension is the response
-        row_len = shape[-1] if len(shape) >= 1 else 1
-        rows = n // row_len if row_len else 0
-        mode, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor = agg
-        kl_type, kl_coef = kl
-        out = torch.empty(16, device=dev, dtype=torch.float32)
-        g_lp = None if lp is None else torch.empty(n, device=dev, dtype=torch.float32)
-        g_ent = None if ent is None else torch.empty(n, device=dev, dtype=torch.float32)
+        total = lead.numel()
+        if packed is None:
+            # rows are the sequences the seq-mean modes average over: the last dimension is the response
+            row_len = lead.shape[-1] if lead.dim() >= 1 else 1
+            rows = total // row_len if row_len else 0
+            n = total
+        else:
+            rows, row_len = response_mask.shape
+            n = rows * row_len
+        lp, ent = _f32(log_prob, total), _f32(entropy, total)
+        old, adv = _f32(old_log_prob, n), _f32(advantages, n)
+        isw, ref = _f32(is_weights, n), _f32(ref_log_prob, n)
+        mask_kind = _INT_MASKS.get(response_mask.dtype) if nonzero_mask or response_mask.dtype == torch.bool else None
+        if mask_kind is not None:
+            assert response_mask.numel() == n, "all inputs have the shape of log_prob"
+            mask = response_mask.contiguous()
+        elif nonzero_mask and response_mask.dtype != torch.float32:
+            mask, mask_kind = response_mask.to(torch.bool).contiguous(), MASK_U8
+        else:
+            mask, mask_kind = _f32(response_mask, n), MASK_F32_NONZERO if nonzero_mask else MASK_F32
+        call = _abi.PpoCall()
+        call.mask_kind = mask_kind
+        call.agg_mode, call.dp_size, call.batch_num_tokens, call.global_batch_size, call.loss_scale_factor = agg
+        call.kl_type, call.kl_coef = kl
+        call.clip_low, call.clip_high, call.clip_c, call.entropy_coeff = clip_low, clip_high, clip_c, entropy_coeff
+        call.rows, call.row_len, call.total_nnz = rows, row_len, -1 if packed is None else total
         lib = _abi.load()
-        with torch.cuda.device(dev):
-            ws_bytes = lib.lce_ppo_loss_workspace_bytes(rows, row_len)
-            ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-            rc = lib.lce_ppo_loss(
-                _abi.ptr(lp), _abi.ptr(ent), _abi.ptr(old), _abi.ptr(adv), mask.data_ptr(), _abi.ptr(isw),
-                _abi.ptr(ref), kl_type, kl_coef, rows, row_len, mode, clip_low, clip_high, clip_c, entropy_coeff,
-                dp_size, batch_num_tokens, global_batch_size, loss_scale_factor, out.data_ptr(), _abi.ptr(g_lp),
-                _abi.ptr(g_ent), ws.data_ptr(), ws_bytes, _abi.current_stream(dev),
-            )  # fmt: skip
-            _abi.check(rc, "lce_ppo_loss")
-        empty = out.new_empty(0)
-        ctx.save_for_backward(g_lp if g_lp is not None else empty, g_ent if g_ent is not None else empty)
-        ctx.has = (lp is not None, ent is not None)
-        ctx.shape = shape
-        ctx.dtypes = (None if log_prob is None else log_prob.dtype, None if entropy is None else entropy.dtype)
-        ctx.mark_non_differentiable(out)
-        return out[0], out
-
-    @staticmethod
-    def _forward_packed(ctx, log_prob, entropy, old_log_prob, advantages, response_mask, is_weights, ref_log_prob, agg, kl,
-                        clip_low, clip_high, clip_c, entropy_coeff, packed):
-        """log_prob / entropy are [total_nnz] model outputs over the packed sequences; everything else is
-        [batch, max_response_len]; packed = (response_start, response_len) int64 [batch] on the device."""
-        assert log_prob is not None and log_prob.is_cuda, "fused_ppo_loss_packed runs on the GPU only"
-        dev = log_prob.device
-        start, length = packed
-        rows, row_len = response_mask.shape
-        total = log_prob.numel()
-
-        def f32(t, n):
-            if t is None:
-                return None
-            t = t.detach().reshape(-1).to(torch.float32).contiguous()
-            assert t.numel() == n
-            return t
-
-        lp, ent = f32(log_prob, total), f32(entropy, total)
-        old, adv, mask = f32(old_log_prob, rows * row_len), f32(advantages, rows * row_len), f32(response_mask, rows * row_len)
-        isw, ref = f32(is_weights, rows * row_len), f32(ref_log_prob, rows * row_len)
-        mode, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor = agg
-        kl_type, kl_coef = kl
+        call.workspace_bytes = lib.lce_ppo_loss_workspace_bytes(rows, row_len)
+        # one allocation: workspace, the unscaled gradients, and the lengths of a packed batch
+        grad_bytes = (total * 4 + 255) // 256 * 256
+        count_lens = packed is not None and packed.attention_mask is not None
+        keep = torch.empty(call.workspace_bytes + 2 * grad_bytes + (16 * rows if count_lens else 0), device=dev, dtype=torch.uint8)
         out = torch.empty(16, device=dev, dtype=torch.float32)
-        g_lp = torch.empty(total, device=dev, dtype=torch.float32)
-        g_ent = None if ent is None else torch.empty(total, device=dev, dtype=torch.float32)
-        lib = _abi.load()
+        at = keep.data_ptr()
+        call.workspace, call.out = at, out.data_ptr()
+        at += call.workspace_bytes
+        call.g_log_prob = at if lp is not None else None
+        call.g_entropy = at + grad_bytes if ent is not None else None
+        at += 2 * grad_bytes
+        ptr = _abi.ptr
+        call.log_prob, call.entropy, call.old_log_prob, call.advantages = ptr(lp), ptr(ent), ptr(old), ptr(adv)
+        call.mask, call.is_weights, call.ref_log_prob = mask.data_ptr(), ptr(isw), ptr(ref)
+        lens = ()
+        if count_lens:
+            am = packed.attention_mask
+            call.attention_mask, call.attention_kind, call.attention_stride = am.data_ptr(), _INT_MASKS[am.dtype], am.stride(0)
+            call.prompt_width, call.attention_width = packed.prompt_width, am.shape[1]
+            call.prompt_lens, call.response_lens = at, at + 8 * rows
+        elif packed is not None:
+            lens = (packed.prompt_lens, packed.response_lens)
+            call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
         with torch.cuda.device(dev):
-            ws_bytes = lib.lce_ppo_loss_workspace_bytes(rows, row_len)
-            ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-            rc = lib.lce_ppo_loss_packed(
-                lp.data_ptr(), _abi.ptr(ent), total, start.data_ptr(), length.data_ptr(), old.data_ptr(), adv.data_ptr(),
-                mask.data_ptr(), _abi.ptr(isw), _abi.ptr(ref), kl_type, kl_coef, rows, row_len, mode, clip_low, clip_high, clip_c,
-                entropy_coeff, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor, out.data_ptr(), g_lp.data_ptr(),
-                _abi.ptr(g_ent), ws.data_ptr(), ws_bytes, _abi.current_stream(dev),
-            )  # fmt: skip
-            _abi.check(rc, "lce_ppo_loss_packed")
-        empty = out.new_empty(0)
-        ctx.save_for_backward(g_lp, g_ent if g_ent is not None else empty)
-        ctx.has = (True, ent is not None)
-        ctx.shape = log_prob.shape
-        ctx.dtypes = (log_prob.dtype, None if entropy is None else entropy.dtype)
+            _abi.check(lib.lce_ppo_forward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_forward")
+        if packed is not None:
+            packed.checks = tuple(call.checks)
+        ctx.save_for_backward(keep, *lens)
+        ctx.call, ctx.base = call, keep.data_ptr()
+        ctx.like = tuple(None if t is None else (t.shape, t.dtype) for t in (log_prob, entropy))
         ctx.mark_non_differentiable(out)
         return out[0], out
 
     @staticmethod
     def backward(ctx, g_loss, _g_out):
-        g_lp, g_ent = ctx.saved_tensors
-        d_lp = (g_lp * g_loss).reshape(ctx.shape).to(ctx.dtypes[0]) if ctx.has[0] else None
-        d_ent = (g_ent * g_loss).reshape(ctx.shape).to(ctx.dtypes[1]) if ctx.has[1] else None
-        return (d_lp, d_ent) + (None,) * 12
+        keep, *lens = ctx.saved_tensors
+        dev = keep.device
+        call = _abi.PpoCall.from_buffer_copy(ctx.call)
+        moved = keep.data_ptr() - ctx.base  # (saved-tensor hooks may bring the buffer back somewhere else)
+        if lens:
+            call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
+        if moved:
+            for name in ("workspace", "g_log_prob", "g_entropy") + (() if lens else ("prompt_lens", "response_lens")):
+                if getattr(call, name) is not None:
+                    setattr(call, name, getattr(call, name) + moved)
+        g_loss = g_loss if g_loss.dtype == torch.float32 else g_loss.to(torch.float32)
+        grads = [
+            torch.empty(like[0], device=dev, dtype=torch.float32) if like is not None and ctx.needs_input_grad[k] else None
+            for k, like in enumerate(ctx.like)
+        ]
+        call.g_loss, call.d_log_prob, call.d_entropy = g_loss.data_ptr(), _abi.ptr(grads[0]), _abi.ptr(grads[1])
+        with torch.cuda.device(dev):
+            _abi.check(_abi.load().lce_ppo_backward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_backward")
+        d = [g if g is None or g.dtype == like[1] else g.to(like[1]) for g, like in zip(grads, ctx.like)]
+        return (*d,) + (None,) * 13
 
 
 def fused_ppo_loss(
@@ -177,6 +198,7 @@ def fused_ppo_loss(
     kl_loss_coef: float = 0.001,
     kl_loss_type: str = "low_var_kl",
     _packed=None,
+    _nonzero_mask=False,
 ):
     """Returns ``(policy_loss, metrics)``: ``policy_loss = pg_loss - entropy_coeff * entropy_loss
     [+ kl_loss_coef * kl_loss]`` (a 0-dim tensor with autograd), ``metrics`` a dict of 0-dim tensors under the
@@ -193,32 +215,30 @@ def fused_ppo_loss(
     kl = (0, 0.0) if ref_log_prob is None else (kl_type_number(kl_loss_type), float(kl_loss_coef))
     loss, out = _FusedPPOLoss.apply(
         log_prob, entropy, old_log_prob, advantages, response_mask, rollout_is_weights, ref_log_prob, agg, kl,
-        float(lo), float(hi), float(clip_ratio_c), float(entropy_coeff), _packed,
+        float(lo), float(hi), float(clip_ratio_c), float(entropy_coeff), _packed, _nonzero_mask,
     )  # fmt: skip
+    _, pg_loss, entropy_loss, clipfrac, ppo_kl, clipfrac_lower, _, _, kl_loss, *_ = out.unbind()
     metrics = {
-        "actor/pg_loss": out[1],
-        "actor/pg_clipfrac": out[3],
-        "actor/ppo_kl": out[4],
-        "actor/pg_clipfrac_lower": out[5],
+        "actor/pg_loss": pg_loss,
+        "actor/pg_clipfrac": clipfrac,
+        "actor/ppo_kl": ppo_kl,
+        "actor/pg_clipfrac_lower": clipfrac_lower,
     }
     if entropy is not None:
-        metrics["actor/entropy_loss"] = out[2]
+        metrics["actor/entropy_loss"] = entropy_loss
     if ref_log_prob is not None:
-        metrics["kl_loss"] = out[8]
+        metrics["kl_loss"] = kl_loss
         metrics["kl_coef"] = kl_loss_coef
     return loss, metrics
 
 
-def response_slices(prompt_lens: torch.Tensor, response_lens: torch.Tensor, total_nnz: int):
-    """``(start, length)`` per sequence of the response slice that ``no_padding_2_padding`` takes out of a packed model
-    output (``verl/workers/utils/padding.py:97-141``): ``start = end of the sequence - response length - 1`` (the
-    left shift by one token), with the reference's two assertions."""
-    prompt_lens = prompt_lens.to(torch.int64)
-    response_lens = response_lens.to(torch.int64)
-    sequence_offsets = (prompt_lens + response_lens).cumsum(dim=0)
-    assert sequence_offsets[-1].item() == total_nnz
-    assert not prompt_lens.eq(0).any(), f"seq_offset - resp_len - 1 assumes prompt_len > 0. Got {prompt_lens}"
-    return (sequence_offsets - response_lens - 1).contiguous(), response_lens.contiguous()
+def _check_lengths(checks, total_nnz, width):
+    """The reference's two assertions on a packed batch (``verl/workers/utils/padding.py:126-128``) and the padded width's,
+    on the sums that the kernel reports."""
+    total, empty_prompts, longest = checks
+    assert total == total_nnz, f"prompt and response lengths add up to {total}, the packed outputs hold {total_nnz} tokens"
+    assert empty_prompts == 0, f"seq_offset - resp_len - 1 assumes prompt_len > 0. Got {empty_prompts} empty prompts"
+    assert longest <= width, "a response is longer than max_response_len"
 
 
 def fused_ppo_loss_packed(
@@ -242,9 +262,11 @@ def fused_ppo_loss_packed(
     assert response_mask.dim() == 2 and old_log_prob.shape == response_mask.shape == advantages.shape
     assert prompt_lens.shape == response_lens.shape == (response_mask.shape[0],)
     dev = log_prob.device
-    start, length = response_slices(prompt_lens.to(dev), response_lens.to(dev), log_prob.numel())
-    assert int(length.max().item()) <= response_mask.shape[1], "a response is longer than max_response_len"
-    return fused_ppo_loss(log_prob, entropy, old_log_prob, advantages, response_mask, _packed=(start, length), **kwargs)
+    packed = _Packed(prompt_lens.to(dev, torch.int64).contiguous(), response_lens.to(dev, torch.int64).contiguous())
+    result = fused_ppo_loss(log_prob, entropy, old_log_prob, advantages, response_mask, _packed=packed, **kwargs)
+    # (the lengths are checked while the loss is on its way: the launches stay inside their buffers whatever they say)
+    _check_lengths(packed.checks, log_prob.numel(), response_mask.shape[1])
+    return result
 
 
 def _cfg(config, name, default=None):
@@ -283,6 +305,15 @@ def batch_lens(data):
     return attention_mask[:, :P].sum(dim=1), attention_mask[:, P:].sum(dim=1)
 
 
+def _packed_lengths(data, dev) -> _Packed:
+    """``batch_lens`` for the kernel: a padded batch's mask of integers on ``dev`` is counted by the loss's own launches."""
+    if not data["prompts"].is_nested:
+        mask, P = data["attention_mask"], data["prompts"].shape[1]
+        if not mask.is_nested and mask.dtype in _INT_MASKS and mask.device == dev and mask.dim() == 2 and mask.shape[1] >= P:
+            return _Packed(attention_mask=mask if mask.stride(1) == 1 else mask.contiguous(), prompt_width=P)
+    return _Packed(*(t.to(dev, torch.int64).contiguous() for t in batch_lens(data)))
+
+
 def _padded(t: torch.Tensor, width: int) -> torch.Tensor:
     """A batch field as exactly ``[batch, width]``: nested (jagged) fields are padded with zeros like
     ``to_padded_tensor``, then cut or zero-padded to ``width`` (a jagged tensor without a cached longest row can come
@@ -293,7 +324,7 @@ def _padded(t: torch.Tensor, width: int) -> torch.Tensor:
         t = t[:, :width]
     elif t.shape[1] < width:
         t = torch.nn.functional.pad(t, (0, width - t.shape[1]))
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def response_width(data, response_lens) -> int:
@@ -330,7 +361,7 @@ def ppo_loss(config, model_output, data, dp_group=None):
     ``ref_log_prob``, and the entries ``dp_size``, ``batch_num_tokens``, ``global_batch_size``.  ``config``: an
     ``ActorConfig``-like object (``clip_ratio*``, ``entropy_coeff``, ``loss_agg_mode``, ``loss_scale_factor``,
     ``use_kl_loss``, ``kl_loss_coef``, ``kl_loss_type``, ``policy_loss.loss_mode``, dict ``global_batch_info``).
-    The response slice, the policy loss, the entropy and KL terms and all metrics are ONE ``lce_ppo_loss_packed``
+    The response slice, the policy loss, the entropy and KL terms and all metrics are ONE ``lce_ppo_forward``
     call; gradients come back in packed order.  Only ``loss_mode == "vanilla"`` has a fused kernel; other modes and
     the sampler-correction outputs (``sc_*``) raise ``NotImplementedError`` instead of taking a slower path."""
     from ...utils.metric import AggregationType, Metric
@@ -359,16 +390,17 @@ def ppo_loss(config, model_output, data, dp_group=None):
         shared.update(info)
     metric_aggregation = metric_aggregation_for(**info)
 
-    prompt_lens, response_lens = batch_lens(data)
-    width = response_width(data, response_lens)
-    if int(response_lens.max().item()) > width:
-        raise ValueError(f"max_response_len = {width} is shorter than the longest response ({int(response_lens.max().item())})")
-    response_mask = _padded(data["response_mask"], width).to(bool)
+    packed = _packed_lengths(data, log_prob.device)
+    width = response_width(data, packed.response_lens)
+    rows = data["responses"].shape[0]
+    response_mask = _padded(data["response_mask"], width)
+    old_log_prob, advantages = _padded(data["old_log_probs"], width), _padded(data["advantages"], width)
+    assert log_prob.dim() == 1 and (entropy is None or entropy.shape == log_prob.shape), "packed outputs are [total_nnz]"
+    assert response_mask.shape == (rows, width) == old_log_prob.shape == advantages.shape
     use_kl = bool(_cfg(config, "use_kl_loss", False))
     is_weights = _get(data, "rollout_is_weights")
-    policy_loss, m = fused_ppo_loss_packed(
-        log_prob, entropy, prompt_lens, response_lens,
-        _padded(data["old_log_probs"], width), _padded(data["advantages"], width), response_mask,
+    policy_loss, m = fused_ppo_loss(
+        log_prob, entropy, old_log_prob, advantages, response_mask, _packed=packed, _nonzero_mask=True,
         clip_ratio=_cfg(config, "clip_ratio"),
         clip_ratio_low=_cfg(config, "clip_ratio_low"),
         clip_ratio_high=_cfg(config, "clip_ratio_high"),
@@ -381,6 +413,10 @@ def ppo_loss(config, model_output, data, dp_group=None):
         kl_loss_type=_cfg(config, "kl_loss_type", "low_var_kl"),
         **info,
     )  # fmt: skip
+    longest = packed.checks[2]
+    if longest > width:
+        raise ValueError(f"max_response_len = {width} is shorter than the longest response ({longest})")
+    _check_lengths(packed.checks, log_prob.numel(), width)
     metrics = Metric.from_dict(
         {k: m[k] for k in ("actor/pg_clipfrac", "actor/ppo_kl", "actor/pg_clipfrac_lower")}, AggregationType.MEAN
     )
