@@ -160,6 +160,14 @@ int lce_logits_backward(const void* logits, int64_t ldl, const int64_t* labels, 
                         const float* stats, const float* dlogprobs, const float* dentropy, void* d_logits, int64_t ldd,
                         void* stream);
 
+/* The same two with the outputs, resp. the upstream gradients, in the type the caller holds them in (LCE_DTYPE_*), so that
+ * no conversion runs before or after them: the value is rounded once from fp32, resp. widened exactly. */
+int lce_logits_forward_as(const void* logits, int64_t ldl, const int64_t* labels, int64_t R, int64_t V, int dtype, void* logprobs,
+                          int logprobs_dtype, void* entropy, int entropy_dtype, float* stats, void* stream);
+int lce_logits_backward_as(const void* logits, int64_t ldl, const int64_t* labels, int64_t R, int64_t V, int dtype,
+                           const float* stats, const void* dlogprobs, int dlogprobs_dtype, const void* dentropy, int dentropy_dtype,
+                           void* d_logits, int64_t ldd, void* stream);
+
 /* Replaces calculate_sum_pi_squared_from_logits (verl/utils/torch_functional.py:687-703; called on the actor's
  * logits at verl/workers/engine/fsdp/transformer_impl.py:1413,1513): out[r] = sum_v softmax(logits[r])_v ^ 2
  * = exp(logsumexp(2 z) - 2 logsumexp(z)), one pass over the row, fp32 arithmetic.  logits [R, V] row stride ldl;

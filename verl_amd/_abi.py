@@ -2,9 +2,12 @@
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("LCE_LIBRARY_PATH") or os.path.join(_HERE, "lib", "liblce_gfx950.so")
@@ -48,6 +51,8 @@ SYMBOLS = {
     ),
     "lce_logits_forward": (_i, [_p, _i64, _p, _i64, _i64, _i, _p, _p, _p, _p]),
     "lce_logits_backward": (_i, [_p, _i64, _p, _i64, _i64, _i, _p, _p, _p, _p, _i64, _p]),
+    "lce_logits_forward_as": (_i, [_p, _i64, _p, _i64, _i64, _i, _p, _i, _p, _i, _p, _p]),
+    "lce_logits_backward_as": (_i, [_p, _i64, _p, _i64, _i64, _i, _p, _p, _i, _p, _i, _p, _i64, _p]),
     "lce_logits_sum_pi_squared": (_i, [_p, _i64, _i64, _i64, _i, _p, _p, _p]),
     "lce_logits_sum_pi_squared_backward": (_i, [_p, _i64, _i64, _i64, _i, _p, _p, _p, _p, _i64, _p]),
     "lce_ppo_loss_workspace_bytes": (_sz, [_i64, _i64]),
@@ -119,15 +124,13 @@ def check(rc: int, what: str) -> None:
         raise LceError(f"{what} failed ({rc}): {msg}")
 
 
-def dtype_code(dtype) -> int:
-    import torch
+_DTYPE_CODES = {torch.bfloat16: DTYPE_BF16, torch.float32: DTYPE_F32, torch.float16: DTYPE_F16}
 
-    if dtype == torch.bfloat16:
-        return DTYPE_BF16
-    if dtype == torch.float32:
-        return DTYPE_F32
-    if dtype == torch.float16:
-        return DTYPE_F16
+
+def dtype_code(dtype) -> int:
+    code = _DTYPE_CODES.get(dtype)
+    if code is not None:
+        return code
     raise NotImplementedError(f"verl_amd supports bfloat16, float16 and float32 inputs, got {dtype}")
 
 
@@ -136,9 +139,16 @@ def ptr(t) -> int | None:
 
 
 def current_stream(device) -> int:
-    import torch
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
-    return torch.cuda.current_stream(device).cuda_stream
+
+_here = contextlib.nullcontext()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)`` where that is not the current device already (the context manager costs a small call
+    more than the call itself does)."""
+    return _here if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def profile_read(reset: bool = True) -> dict[str, tuple[float, int]]:

@@ -164,7 +164,7 @@ def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0,
         return logprobs, entropy, maximum, accumulate, entropy_b, None
     lib = _abi.load()
     cache = None
-    with torch.cuda.device(dev):
+    with _abi.on_device(dev):
         ws_bytes = lib.lce_forward_workspace_bytes(T, H, V, code)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
         cache_bytes = lib.lce_logits_cache_bytes(T, H, V, code) if keep_logits else 0
@@ -236,7 +236,7 @@ def efficient_entropy_backward(
             d_weight.zero_()
     else:
         lib = _abi.load()
-        with torch.cuda.device(dev):
+        with _abi.on_device(dev):
             vchunk = _config._vocab_chunk
             ws_bytes = lib.lce_backward_workspace_bytes(T, H, V, code, vchunk)
             ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)

@@ -39,7 +39,7 @@ def shard_forward(hidden: torch.Tensor, weight_shard: torch.Tensor, labels: torc
     if T == 0:
         return partials
     lib = _abi.load()
-    with torch.cuda.device(dev):
+    with _abi.on_device(dev):
         nws = lib.lce_forward_workspace_bytes(T, H, V, code)
         ws = torch.empty((nws,), device=dev, dtype=torch.uint8)
         rc = lib.lce_forward_shard(
@@ -62,7 +62,7 @@ def merge_shards(partials: torch.Tensor, reduction: typing.Union[int, str] = 0) 
     logprobs = torch.empty((T,) if reduction == 0 else (), **f32)
     entropy, maximum, accumulate, entropy_b = (torch.empty((T,), **f32) for _ in range(4))
     lib = _abi.load()
-    with torch.cuda.device(dev):
+    with _abi.on_device(dev):
         ws = torch.empty((max(4 * T, 16),), device=dev, dtype=torch.uint8)
         rc = lib.lce_merge_shards(
             partials.data_ptr(), R, T, reduction, logprobs.data_ptr(), entropy.data_ptr(), maximum.data_ptr(),
@@ -92,7 +92,7 @@ def shard_backward(dlogprobs: torch.Tensor, dentropy: typing.Optional[torch.Tens
         d_weight.zero_()
         return [d_hidden, d_weight]
     lib = _abi.load()
-    with torch.cuda.device(dev):
+    with _abi.on_device(dev):
         vchunk = _config._vocab_chunk
         nws = lib.lce_backward_workspace_bytes(T, H, V, code, vchunk)
         ws = torch.empty((nws,), device=dev, dtype=torch.uint8)

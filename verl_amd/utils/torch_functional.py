@@ -37,54 +37,81 @@ def _require_gpu(logits: torch.Tensor) -> None:
         )
 
 
-def _logits_forward(logits, labels, want_logprobs: bool, want_entropy: bool, want_stats: bool):
+def _out_code(dtype) -> int:
+    """Type a kernel writes for a result of ``dtype`` (fp32, converted afterwards, where it has no code)."""
+    return _abi._DTYPE_CODES.get(dtype, _abi.DTYPE_F32)
+
+
+_CODE_DTYPES = {code: dtype for dtype, code in _abi._DTYPE_CODES.items()}
+
+
+def _logits_forward(logits, labels, lp_dtype, ent_dtype, want_stats: bool):
+    """``lp_dtype`` / ``ent_dtype``: dtype of that output, None: not wanted."""
     _require_gpu(logits)
     code = _abi.dtype_code(logits.dtype)
     rows, V = _as_rows(logits)
     R = rows.shape[0]
     dev = logits.device
-    lp = torch.empty((R,), device=dev, dtype=torch.float32) if want_logprobs else None
-    ent = torch.empty((R,), device=dev, dtype=torch.float32) if want_entropy else None
+    lp_code, ent_code = _out_code(lp_dtype), _out_code(ent_dtype)
+    lp = torch.empty((R,), device=dev, dtype=_CODE_DTYPES[lp_code]) if lp_dtype is not None else None
+    ent = torch.empty((R,), device=dev, dtype=_CODE_DTYPES[ent_code]) if ent_dtype is not None else None
     # row statistics for the backward (it then needs one pass instead of two)
     # (the caller decides: inside autograd.Function.forward grad mode is off, so it cannot be read here)
     stats = torch.empty((R, 2), device=dev, dtype=torch.float32) if want_stats else None
     y = None
-    if want_logprobs:
+    if lp is not None:
         y = labels.reshape(-1).to(torch.int64).contiguous()
         assert y.shape[0] == R and y.device == dev
     if R > 0:
-        with torch.cuda.device(dev):
-            rc = _abi.load().lce_logits_forward(
-                rows.data_ptr(), rows.stride(0), _abi.ptr(y), R, V, code, _abi.ptr(lp), _abi.ptr(ent), _abi.ptr(stats),
-                _abi.current_stream(dev),
+        with _abi.on_device(dev):
+            rc = _abi.load().lce_logits_forward_as(
+                rows.data_ptr(), rows.stride(0), _abi.ptr(y), R, V, code, _abi.ptr(lp), lp_code, _abi.ptr(ent), ent_code,
+                _abi.ptr(stats), _abi.current_stream(dev),
             )  # fmt: skip
-            _abi.check(rc, "lce_logits_forward")
+            _abi.check(rc, "lce_logits_forward_as")
     return rows, y, lp, ent, stats
+
+
+def _shaped(values, logits, dtype):
+    if logits.dim() != 2:
+        values = values.reshape(logits.shape[:-1])
+    return values if values.dtype == dtype else values.to(dtype)
+
+
+def _upstream(g):
+    """An upstream gradient as the kernel takes it, and the code of its type."""
+    if g is None:
+        return None, _abi.DTYPE_F32
+    g = g.reshape(-1)
+    if g.dtype not in _abi._DTYPE_CODES:
+        g = g.to(torch.float32)
+    return g.contiguous(), _abi._DTYPE_CODES[g.dtype]
 
 
 def _logits_backward(rows, y, stats, g_lp, g_ent, out_shape, out_dtype):
     R, V = rows.shape
     dev = rows.device
     d = torch.empty((R, V), device=dev, dtype=rows.dtype)
-    g_lp = None if g_lp is None else g_lp.reshape(-1).to(torch.float32).contiguous()
-    g_ent = None if g_ent is None else g_ent.reshape(-1).to(torch.float32).contiguous()
+    g_lp, lp_code = _upstream(g_lp)
+    g_ent, ent_code = _upstream(g_ent)
     if R > 0:
-        with torch.cuda.device(dev):
-            rc = _abi.load().lce_logits_backward(
+        with _abi.on_device(dev):
+            rc = _abi.load().lce_logits_backward_as(
                 rows.data_ptr(), rows.stride(0), _abi.ptr(y), R, V, _abi.dtype_code(rows.dtype), _abi.ptr(stats),
-                _abi.ptr(g_lp), _abi.ptr(g_ent), d.data_ptr(), d.stride(0), _abi.current_stream(dev),
+                _abi.ptr(g_lp), lp_code, _abi.ptr(g_ent), ent_code, d.data_ptr(), V, _abi.current_stream(dev),
             )  # fmt: skip
-            _abi.check(rc, "lce_logits_backward")
-    return d.reshape(out_shape).to(out_dtype)
+            _abi.check(rc, "lce_logits_backward_as")
+    d = d if d.shape == out_shape else d.reshape(out_shape)
+    return d if d.dtype == out_dtype else d.to(out_dtype)
 
 
 class _LogprobsFromLogits(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, labels):
-        rows, y, lp, _, stats = _logits_forward(logits, labels, True, False, ctx.needs_input_grad[0])
+        rows, y, lp, _, stats = _logits_forward(logits, labels, logits.dtype, None, ctx.needs_input_grad[0])
         ctx.save_for_backward(rows, y, stats)
         ctx.shape, ctx.dtype = logits.shape, logits.dtype
-        return lp.reshape(logits.shape[:-1]).to(logits.dtype)
+        return _shaped(lp, logits, logits.dtype)
 
     @staticmethod
     def backward(ctx, g):
@@ -95,10 +122,10 @@ class _LogprobsFromLogits(torch.autograd.Function):
 class _EntropyFromLogits(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, out_dtype):
-        rows, _, _, ent, stats = _logits_forward(logits, None, False, True, ctx.needs_input_grad[0])
+        rows, _, _, ent, stats = _logits_forward(logits, None, None, out_dtype, ctx.needs_input_grad[0])
         ctx.save_for_backward(rows, stats)
         ctx.shape, ctx.dtype = logits.shape, logits.dtype
-        return ent.reshape(logits.shape[:-1]).to(out_dtype)
+        return _shaped(ent, logits, out_dtype)
 
     @staticmethod
     def backward(ctx, g):
@@ -111,11 +138,11 @@ class _LogprobsAndEntropyFromLogits(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, logits, labels, entropy_dtype):
-        rows, y, lp, ent, stats = _logits_forward(logits, labels, True, True, ctx.needs_input_grad[0])
+        rows, y, lp, ent, stats = _logits_forward(logits, labels, logits.dtype, entropy_dtype, ctx.needs_input_grad[0])
         ctx.save_for_backward(rows, y, stats)
         ctx.shape, ctx.dtype = logits.shape, logits.dtype
         ctx.set_materialize_grads(False)
-        return lp.reshape(logits.shape[:-1]).to(logits.dtype), ent.reshape(logits.shape[:-1]).to(entropy_dtype)
+        return _shaped(lp, logits, logits.dtype), _shaped(ent, logits, entropy_dtype)
 
     @staticmethod
     def backward(ctx, g_lp, g_ent):
@@ -174,7 +201,7 @@ class _SumPiSquaredFromLogits(torch.autograd.Function):
         keep = ctx.needs_input_grad[0]
         lse = torch.empty((R,), device=dev, dtype=torch.float32) if keep else None
         if R > 0:
-            with torch.cuda.device(dev):
+            with _abi.on_device(dev):
                 rc = _abi.load().lce_logits_sum_pi_squared(
                     rows.data_ptr(), rows.stride(0), R, V, _abi.dtype_code(logits.dtype), out.data_ptr(), _abi.ptr(lse), _abi.current_stream(dev)
                 )
@@ -191,7 +218,7 @@ class _SumPiSquaredFromLogits(torch.autograd.Function):
         d = torch.empty((R, V), device=rows.device, dtype=rows.dtype)
         g = g.reshape(-1).to(torch.float32).contiguous()
         if R > 0:
-            with torch.cuda.device(rows.device):
+            with _abi.on_device(rows.device):
                 rc = _abi.load().lce_logits_sum_pi_squared_backward(
                     rows.data_ptr(), rows.stride(0), R, V, _abi.dtype_code(rows.dtype), lse.data_ptr(), s.data_ptr(), g.data_ptr(),
                     d.data_ptr(), d.stride(0), _abi.current_stream(rows.device),

@@ -143,7 +143,7 @@ class _FusedPPOLoss(torch.autograd.Function):
         elif packed is not None:
             lens = (packed.prompt_lens, packed.response_lens)
             call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
-        with torch.cuda.device(dev):
+        with _abi.on_device(dev):
             _abi.check(lib.lce_ppo_forward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_forward")
         if packed is not None:
             packed.checks = tuple(call.checks)
@@ -171,7 +171,7 @@ class _FusedPPOLoss(torch.autograd.Function):
             for k, like in enumerate(ctx.like)
         ]
         call.g_loss, call.d_log_prob, call.d_entropy = g_loss.data_ptr(), _abi.ptr(grads[0]), _abi.ptr(grads[1])
-        with torch.cuda.device(dev):
+        with _abi.on_device(dev):
             _abi.check(_abi.load().lce_ppo_backward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_backward")
         d = [g if g is None or g.dtype == like[1] else g.to(like[1]) for g, like in zip(grads, ctx.like)]
         return (*d,) + (None,) * 13
