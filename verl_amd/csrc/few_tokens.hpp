@@ -278,7 +278,7 @@ LCE_DEV void dh_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
       const int r = tid / CPR + (256 / CPR) * i;
       int64_t v = Perm::vocab_at(k0 + r);
       v = v < p.vrows ? v : p.vrows - 1;  // dS is zero in such a column
-      pw[i] = *reinterpret_cast<const u32x4_t*>(p.W + v * p.ldw + wcol);
+      pw[i] = load_vec<true>(reinterpret_cast<const u32x4_t*>(p.W + v * p.ldw + wcol));
     }
 #pragma unroll
     for (int i = 0; i < BL; ++i) {

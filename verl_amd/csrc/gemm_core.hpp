@@ -96,13 +96,15 @@ struct Mma<float> {
 // (C = A^T . B); 2 = only B is (C = A . B with A[m][k], B[k][n]).  A ring slot of a K-major operand holds 64 k-rows
 // of 256 columns and its MFMA operand fragments are fetched with the transposing LDS read (ds_read_b64_tr_b16,
 // two per fragment).
-template <typename TIN_, int BM_, int BN_, int BKB_, int NSTAGE_, int WAVES_M_, int WAVES_N_, int SPLIT_ = 0, int TRANS_ = 0>
+// A_ONCE_: the A operand is streamed once by this launch and not read again soon: its loads are marked non-temporal
+template <typename TIN_, int BM_, int BN_, int BKB_, int NSTAGE_, int WAVES_M_, int WAVES_N_, int SPLIT_ = 0, int TRANS_ = 0, int A_ONCE_ = 0>
 struct GemmCfg {
   typedef TIN_ TIN;
   static constexpr bool CORE16 = false;  // (the four-wave 16x16x32 mainloop is GemmCfg16, gemm_core16.hpp)
   static constexpr int BM = BM_, BN = BN_, BKB = BKB_, NSTAGE = NSTAGE_;
   static constexpr int SPLIT = SPLIT_;  // 0 whole stages; 1 split ring, A operand early; 2 split ring, B operand early
   static constexpr int TRANS = TRANS_;
+  static constexpr int A_AUX = A_ONCE_ ? 2 : 0;  // cache policy bits of the global->LDS loads: 2 = nt
   static constexpr bool TRANS_A = TRANS_ == 1, TRANS_B = TRANS_ != 0;
   static_assert(TRANS_ == 0 || (SPLIT_ != 0 && sizeof(TIN_) == 2 && BM_ == 256 && BN_ == 256 && BKB_ == 128), "transposed operands: split ring, 16-bit, 256x256");
   static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
@@ -254,7 +256,7 @@ struct GemmCore {
     char* sa = lds + stage * Cfg::STAGE_BYTES;
     if (idx < Cfg::A_LOADS) {
       __builtin_amdgcn_global_load_lds((gptr_t)(a_base + kbyte + la.voff[idx]),
-                                       (lptr_t)(sa + (idx * Cfg::NW + wave) * 1024), 16, 0, 0);
+                                       (lptr_t)(sa + (idx * Cfg::NW + wave) * 1024), 16, 0, Cfg::A_AUX);
     } else {
       const int j = idx - Cfg::A_LOADS;
       __builtin_amdgcn_global_load_lds((gptr_t)(b_base + kbyte + lb.voff[j]),
@@ -276,7 +278,7 @@ struct GemmCore {
       __builtin_amdgcn_global_load_lds((gptr_t)(b_base + off + lb.voff[j]), (lptr_t)sa, 16, 0, 0);
     } else {
       const int64_t off = Cfg::TRANS_A ? (kbyte / Cfg::BKB) * a_slab : kbyte;
-      __builtin_amdgcn_global_load_lds((gptr_t)(a_base + off + la.voff[j]), (lptr_t)sa, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_t)(a_base + off + la.voff[j]), (lptr_t)sa, 16, 0, Cfg::A_AUX);
     }
   }
   LCE_DEV void issue_slab(char* lds, int stage, int64_t kbyte) const {
