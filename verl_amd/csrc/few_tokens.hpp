@@ -56,8 +56,8 @@ LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 
 template <typename TIN>
 struct FewArgs {
-  const TIN* dS;      // [>= kt rows][ldS]: d_logits of the chunk by (compact) token position; columns in Perm order;
-  int64_t ldS;        //   zero rows beyond the tokens that take part, zero columns beyond the chunk's rows
+  const TIN* dS;      // d_logits of the chunk by (compact) token position, >= kt of them, at ds_at; columns in Perm order;
+  int64_t ldS, pcol;  //   zero rows beyond the tokens that take part, zero columns beyond the chunk's rows
   const TIN* Ht;      // compact copy of hidden, [>= kt rows][ldHt], ldHt >= round_up(H, 256); zero rows beyond the tokens
   int64_t ldHt;
   const TIN* W;       // first row of the chunk, row stride ldw
@@ -109,7 +109,7 @@ LCE_DEV void dw_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
   for (int i = 0; i < (KT * 8 + 255) / 256; ++i) {
     const int id = tid + i * 256, r = id >> 3, c = id & 7;
     if (id < KT * 8) {
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p.dS + (int64_t)r * p.ldS + u0 + c * 8);
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ds_at(p.dS, p.ldS, p.pcol, r, u0 + c * 8));
       *reinterpret_cast<u32x4_t*>(sB + r * 128 + ((c ^ (r & 7)) * 16)) = v;
     }
   }
@@ -283,7 +283,7 @@ LCE_DEV void dh_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
       const int id = tid + i * 256, t = id >> 3, c = id & 7;
-      pb[i] = *reinterpret_cast<const u32x4_t*>(p.dS + (int64_t)t * p.ldS + k0 + c * 8);
+      pb[i] = *reinterpret_cast<const u32x4_t*>(ds_at(p.dS, p.ldS, p.pcol, t, k0 + c * 8));
     }
   };
   auto stash = [&]() {
@@ -366,18 +366,18 @@ __global__ __launch_bounds__(256, 2) void lce_bwd_few_kernel(FewArgs<TIN> p) {
 
 // ------------------------------------------------------------------------------------------------------------------
 // d_logits of a vocabulary chunk from logits that the forward kept (tokens up to half the hidden size): what the
-// d_logits tiles compute from their accumulators, here from x[t * ldx + v], element by element with the same
+// d_logits tiles compute from their accumulators, here from the kept x(t, v), element by element with the same
 // expressions, so the same bits.  One pass over 4 bytes per logit instead of a pass over W.  Workgroup b owns the 64
 // columns [64 b, 64 b + 64) of dS, which lie within one group of the vocabulary order Perm (a whole group of the
 // eight-wave tiles' order, half a group of the 16x16x32 tiles'), and the first `nrows` compact token positions: rows
 // beyond the tokens that take part and columns beyond the chunk's rows (the grid covers whole 256-row tiles) are
 // written as zeros, as the tiles write them.  Eight lanes share a position: they read the 256 bytes of its token's
 // logits behind the 64 columns and write 128 bytes of dS.
-// p: the chunk's DsArgs (W, h, the tile map and the range are not used); x: the kept logit of the chunk's first row
-// for token 0.
+// p: the chunk's DsArgs (W, h, the tile map and the range are not used); x: the kept logits from the chunk's first row
+// on (a multiple of 16), of xtok tokens.
 // ------------------------------------------------------------------------------------------------------------------
 template <typename TIN, typename Perm>
-__global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t ldx, int nrows) {
+__global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t xtok, int nrows) {
   static_assert(sizeof(TIN) == 2 && Perm::GV % 64 == 0, "16-bit d_logits, groups of the vocabulary order in multiples of 64 rows");
   const int tid = threadIdx.x, c = tid & 7;
   const int64_t u0 = (int64_t)blockIdx.x * 64;   // first of this workgroup's 64 columns of dS
@@ -398,14 +398,14 @@ __global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, cons
     }
     // columns c * 8 + (0..3) and c * 8 + (4..7) of the workgroup's 64 are two runs of four consecutive vocabulary rows
     // (both orders Perm keep what one lane of a d_logits tile holds together: four consecutive rows per register quad),
-    // and the cache's rows are padded to whole groups, so each run is one aligned 16-byte load
+    // and the cache is padded to whole groups, so each run is one aligned 16-byte load
     float xv[8];
     int row[8];  // vocabulary row relative to the group's first
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       const int r0 = (int)(Perm::vocab_at(u0 + c * 8 + 4 * hf) - g0);
       f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-      if (tok >= 0 && g0 + r0 < p.vrows) v = *reinterpret_cast<const f32x4_t*>(x + tok * ldx + g0 + r0);
+      if (tok >= 0 && g0 + r0 < p.vrows) v = *reinterpret_cast<const f32x4_t*>(kept_logit(x, xtok, tok, g0 + r0));
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         row[4 * hf + e] = r0 + e;
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, cons
       const bool dead = tok < 0 || g0 + row[e] >= p.vrows;
       d[e] = dlogit<true>(dead ? 0.f : xv[e], p.c, lse2, C0, C1, G, row[e] == rel, dead, p.label_outside == 2);
     }
-    store_run<TIN, 8>(p.dS + (int64_t)pos * p.ldS + u0 + c * 8, d);
+    store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, pos, u0 + c * 8), d);
   }
 }
 

@@ -18,6 +18,7 @@
 // Accumulator layout of one 16 x 16 block: lane l holds column n = l % 16 and rows m = 4 * (l / 16) + r,
 // r = 0..3.  Block (i, j) of a wave covers rows 16 i .. and columns 16 j .. of its 128 x 128.
 #pragma once
+#include <type_traits>
 #include <utility>
 
 #include "gemm_core.hpp"
@@ -31,6 +32,9 @@ struct Mma16<bf16_t> {
   static LCE_DEV void run(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
   }
+  static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
+  }
   // the same instruction as a builtin: the compiler schedules it and knows its latency
   static LCE_DEV f32x4_t known(const f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
     typedef __bf16 v8 __attribute__((ext_vector_type(8)));
@@ -41,6 +45,9 @@ template <>
 struct Mma16<f16_t> {
   static LCE_DEV void run(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  }
+  static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
   }
   static LCE_DEV f32x4_t known(const f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
     typedef _Float16 v8 __attribute__((ext_vector_type(8)));
@@ -68,6 +75,15 @@ struct GemmCfg16 {
   static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
   static constexpr int HL = 8;                       // wave-wide 16-byte-per-lane loads per wave and half slab
 };
+
+// The lane number, worked out anew where it is asked for.  A kernel that walks tiles has no register to spare across its K
+// loop: what follows from the lane number and is wanted at every tile would be kept in scratch memory, and a load from
+// there waits for every load and store issued before it.
+LCE_DEV int lane_anew() {
+  uint32_t zero = 0;
+  asm volatile("" : "+s"(zero));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
 
 template <typename Cfg>
 struct GemmCore16 {
@@ -130,10 +146,11 @@ struct GemmCore16 {
   // The transposing read: in each group of 16 lanes, lane 4e + q supplies the address of X[k0 + e][x0 + 4q ..] and
   // lane i receives X[k0 .. k0+3][x0 + i]; group g of the wave takes the k-octet 8g of the 32 k-values of a k-step,
   // and a second read 4 rows further completes the octet.
-  LCE_DEV void init_tn(const TIN* A, int64_t lda, int64_t m0, const TIN* B, int64_t ldb, int64_t n0) {
+  // With b_pcol, B lies in panels of 64 columns, b_pcol elements apart (ldb = 64: the rows of a panel follow each other).
+  LCE_DEV void init_tn(const TIN* A, int64_t lda, int64_t m0, const TIN* B, int64_t ldb, int64_t n0, int64_t b_pcol = 0) {
     set_lane();
     a_base = reinterpret_cast<const char*>(A + m0);
-    b_base = reinterpret_cast<const char*>(B + n0);
+    b_base = reinterpret_cast<const char*>(b_pcol ? B + (n0 >> 6) * b_pcol : B + n0);
     a_slab = 64 * lda * 2;
     b_slab = 64 * ldb * 2;
 #pragma unroll
@@ -141,13 +158,21 @@ struct GemmCore16 {
       const int row = (j * Cfg::NW + wave) * 2 + (lane >> 5);
       const int c = (lane & 31) ^ tn_swz(row);
       va[j] = (uint32_t)((int64_t)row * lda * 2) + (uint32_t)(c * 16);
-      vb[j] = (uint32_t)((int64_t)row * ldb * 2) + (uint32_t)(c * 16);
+      vb[j] = (uint32_t)((int64_t)row * ldb * 2) + (b_pcol ? (uint32_t)((c >> 3) * b_pcol * 2) + (uint32_t)((c & 7) * 16) : (uint32_t)(c * 16));
     }
-    const int g = lane >> 4, e = (lane & 15) >> 2, q = lane & 3;
+    reads_tn(lane);
+  }
+  LCE_DEV void reads_tn(int ln) {
+    const int g = ln >> 4, e = (ln & 15) >> 2, q = ln & 3;
     const int row = 8 * g + e;  // (k-step 0, first half of the octet)
     const uint32_t in_row = (uint32_t)((((q >> 1) ^ tn_swz(row)) * 16) + (q & 1) * 8);
     a_rd = (uint32_t)(row * 512 + wave_m * Cfg::WM * 2) + in_row;
     b_rd = (uint32_t)(row * 512 + wave_n * Cfg::WN * 2) + in_row;
+  }
+  // another tile of the same matrices after init_tn
+  LCE_DEV void move_tn(const TIN* A, int64_t m0, const TIN* B, int64_t n0, int64_t b_pcol) {
+    a_base = reinterpret_cast<const char*>(A + m0);
+    b_base = reinterpret_cast<const char*>(b_pcol ? B + (n0 >> 6) * b_pcol : B + n0);
   }
   static LCE_DEV int tn_swz(int row) { return ((row & 3) * 4) ^ (((row >> 3) & 1) * 2); }
 
@@ -155,16 +180,17 @@ struct GemmCore16 {
   // LDS row r of an A slab holds memory row perm(r) of the slab (perm: a permutation of 0..63, the order in which B's
   // K index was stored); rows at or beyond `kvalid` > 0 are replaced by rows that exist (B is zero there), and columns at
   // or beyond `mcols` (a last tile of a width that is no multiple of 256) by the row's first chunk: in bounds, and they
-  // feed only results that the epilogue discards.
+  // feed only results that the epilogue discards.  b_slab_bytes: from one K slab of B to the next (its rows' 128 bytes for
+  // rows of ldb elements; a panel where B lies in panels of 64 columns).
   template <typename Perm>
   LCE_DEV void init_mixed(const TIN* A, int64_t lda, int64_t m0, int64_t mcols, int64_t kvalid, Perm perm, const TIN* B, int64_t ldb,
-                          int64_t n0, int64_t N) {
+                          int64_t n0, int64_t N, int64_t b_slab_bytes) {
     static_assert(Cfg::TRANS == 2, "mixed mode");
     set_lane();
     a_base = reinterpret_cast<const char*>(A + m0);
     b_base = reinterpret_cast<const char*>(B + n0 * ldb);
     a_slab = 64 * lda * 2;
-    b_slab = Cfg::BKB;
+    b_slab = b_slab_bytes;
     a_ks_full = kvalid / 64;
     a_ks_last = (kvalid - 1) / 64;
     const int last_row = (int)(kvalid - 1 - a_ks_last * 64);  // of slab a_ks_last
@@ -237,10 +263,12 @@ struct GemmCore16 {
 
   // One k-step: 64 MFMAs on (af, bf); the 16 fragment reads of the next k-step (from ra_n / rb_n, k-step S_N) and HL
   // global->LDS loads are dealt between them.  WAIT: the fragments of this step were read during the previous step
-  // and may still be in flight.  DMA_B: the loads fetch the B operand's half slab `dma_ks` (else A's) into `dma_slot`.
-  template <bool WAIT, int S_N, bool DMA_B>
+  // and may still be in flight.  DMA_B: the loads fetch the B operand's half slab `dma_ks` (else A's) into `dma_slot`; with
+  // FROM, the half slab at `dma_from` instead.  FIRST: the accumulators start here.
+  template <bool WAIT, int S_N, bool DMA_B, bool FROM = false, bool FIRST = false>
   LCE_DEV void kstep(f32x4_t (&acc)[NB][NB], const u32x4_t (&af)[NB], const u32x4_t (&bf)[NB], uint32_t ra_n, uint32_t rb_n,
-                     u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NB], char* lds, int dma_slot, int64_t dma_ks) const {
+                     u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NB], char* lds, int dma_slot, int64_t dma_ks,
+                     const char* dma_from = nullptr) const {
     static_for(std::make_integer_sequence<int, NB * NB>{}, [&](auto mc) {
       constexpr int m = decltype(mc)::value;
       constexpr int i = m / NB, j = m % NB;
@@ -250,9 +278,16 @@ struct GemmCore16 {
         wait_lgkm<(allow > 15 ? 15 : allow)>();
       }
       __builtin_amdgcn_sched_barrier(0);
-      Mma16<TIN>::run(acc[i][j], af[i], bf[j]);
+      if constexpr (FIRST) Mma16<TIN>::first(acc[i][j], af[i], bf[j]);
+      else Mma16<TIN>::run(acc[i][j], af[i], bf[j]);
       if constexpr ((m & 1) == 0 && m / 2 < 16) read_frag<m / 2, S_N>(ra_n, rb_n, af_n, bf_n);
-      if constexpr (m % (NB * NB / HL) == 3) dma(lds, dma_slot, dma_ks, DMA_B, m / (NB * NB / HL));
+      if constexpr (m % (NB * NB / HL) == 3) {
+        constexpr int j8 = m / (NB * NB / HL);
+        if constexpr (FROM)
+          __builtin_amdgcn_global_load_lds((gptr_t)(dma_from + (DMA_B ? vb[j8] : va[j8])), (lptr_t)(lds + dma_slot * SLOT + (j8 * Cfg::NW + wave) * 1024),
+                                           16, 0, 0);
+        else dma(lds, dma_slot, dma_ks, DMA_B, j8);
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
   }
@@ -313,17 +348,77 @@ struct GemmCore16 {
     }
     wait_vm<0>();    // drain the redundant tail fetches before LDS is reused
     wait_lgkm<0>();  // and the reads of the slab after the last
-    // The accumulators are read by ordinary instructions from here on: let the last MFMAs retire.  The MFMAs are inline
-    // assembly, so the compiler knows nothing of their latency, and it is free to place a copy of an accumulator (for the
-    // epilogue, or to spill it) right behind the statement that last wrote it, ahead of this wait (seen in a variant of
-    // the forward: accumulators copied to scratch a few instructions behind the last MFMA, wrong statistics).  Only the
-    // last blocks of the k-step can still be in the matrix pipe when the loop ends, so the last row of blocks is passed
-    // through one more MFMA that the compiler does know (zero operands: acc + 0): behind a builtin it keeps the
-    // distance to a read itself, and the matrix pipe orders it behind the assembly MFMA that wrote the same registers.
+    retire(acc);
+  }
+
+  // The accumulators are read by ordinary instructions from here on: let the last MFMAs retire.  The MFMAs are inline
+  // assembly, so the compiler knows nothing of their latency, and it is free to place a copy of an accumulator (for the
+  // epilogue, or to spill it) right behind the statement that last wrote it, ahead of this wait (seen in a variant of
+  // the forward: accumulators copied to scratch a few instructions behind the last MFMA, wrong statistics).  Only the
+  // last blocks of the k-step can still be in the matrix pipe when the loop ends, so the last row of blocks is passed
+  // through one more MFMA that the compiler does know (zero operands: acc + 0): behind a builtin it keeps the
+  // distance to a read itself, and the matrix pipe orders it behind the assembly MFMA that wrote the same registers.
+  static LCE_DEV void retire(f32x4_t (&acc)[NB][NB]) {
     asm volatile("s_nop 15\n\ts_nop 7" ::);
     const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[NB - 1][j] = Mma16<TIN>::known(acc[NB - 1][j], zero, zero);
+  }
+
+  // ---- a workgroup that walks tiles: the K loops of successive tiles as one stream of slabs -------------------
+  // The loads two slabs ahead of the end of a tile are those of the next tile's first slabs, and the fragments that the last
+  // k-step reads are the next tile's first: between two tiles there is neither a drain nor a first load to wait for.
+  struct Stream {
+    u32x4_t af[NB], bf[NB];  // the next slab's first fragments
+    int sb;                  // slot of its B half
+  };
+  // prologue() of the first tile has been called, and nothing else was loaded since
+  LCE_DEV void stream_begin(char* lds, Stream& s) const {
+    wait_vm<2 * HL>();
+    __builtin_amdgcn_s_barrier();
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    static_for(std::make_integer_sequence<int, 16>{}, [&](auto fc) {
+      read_frag<decltype(fc)::value, 0>(lds0 + SLOT + a_rd, lds0 + b_rd, s.af, s.bf);
+    });
+    s.sb = 0;
+  }
+  // One tile of nk >= 2 slabs at a_base / b_base; a_next / b_next: the next tile's (this one's again when there is none).
+  // STORES: with `stores_behind`, exactly that many stores of this wave lie between the loads of this tile's second slab
+  // and anything loaded here.  The first wait leaves them in flight; the second slab's needs them acknowledged, which
+  // gives them the time of a slab and a half.  Ring slot (s.sb + 4) % 5 is free when this returns, until the barrier that
+  // the caller places before the next call.
+  template <int STORES>
+  LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NB], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
+    static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    int sb = s.sb;
+    auto slab = [&](auto first, int it) {
+      constexpr bool FIRST = decltype(first)::value;
+      u32x4_t af1[NB], bf1[NB];  // the fragments of the slab's second k-step
+      const int sa = sb + 1 >= 5 ? sb + 1 - 5 : sb + 1;
+      const int nb = sb + 2 >= 5 ? sb + 2 - 5 : sb + 2;
+      const int na = sb + 3 >= 5 ? sb + 3 - 5 : sb + 3;
+      const int fr = sb + 4 >= 5 ? sb + 4 - 5 : sb + 4;
+      const bool nx = it + 2 >= nk;
+      const int ks = nx ? it + 2 - nk : it + 2;
+      const char* from_b = (nx ? b_next : b_base) + ks * b_slab;
+      const char* from_a = (nx ? a_next : a_base) + ks * a_slab;
+      kstep<true, 1, true, true, FIRST>(acc, s.af, s.bf, lds0 + sa * SLOT + a_rd, lds0 + sb * SLOT + b_rd, af1, bf1, lds, fr, 0, from_b);
+      if (FIRST && stores_behind) wait_vm<HL + STORES>();
+      else wait_vm<HL>();
+      wait_lgkm<0>();
+      __builtin_amdgcn_s_barrier();
+      kstep<false, 0, false, true>(acc, af1, bf1, lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, s.af, s.bf, lds, sb, 0, from_a);
+      sb = nb;
+    };
+    slab(std::true_type{}, 0);
+    for (int it = 1; it < nk; ++it) slab(std::false_type{}, it);
+    s.sb = sb;
+    // the next tile's first fragments are in registers from here on, whatever the compiler does with those meanwhile
+    wait_lgkm<0>();
+#pragma unroll
+    for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(s.af[i]), "+v"(s.bf[i]));
+    retire(acc);
   }
 
   LCE_DEV void run(char* lds, int64_t K, f32x4_t (&acc)[NB][NB]) const {

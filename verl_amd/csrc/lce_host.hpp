@@ -35,8 +35,12 @@ extern std::vector<hipEvent_t> prof_pool;
 // four-wave 16x16x32 loop (variant 3) above the token counts below.
 constexpr int kDefaultVariantFwd = 2, kDefaultVariantBwd = 1, kVariantCore16 = 3;
 // variant 3 is the default above these token counts (measured at H=3584, V=152064: the forward gains 2-6% from 1024
-// tokens on; forward + backward is 2% slower with it at 1024 tokens, 2% faster at 1536 and 2048, 4% at 3072)
-constexpr int64_t kCore16MinTokensFwd = 512, kCore16MinTokensBwd = 1280;
+// tokens on; the backward runs its gradient GEMMs on it wherever the streaming kernels of few_tokens.hpp end)
+constexpr int64_t kCore16MinTokensFwd = 512, kCore16MinTokensBwd = 128;
+// up to here a backward that fits one vocabulary chunk runs its two gradient GEMMs as launches of their own, d_weight on
+// workgroups that stay (lce_dw16_kernel); beyond, a tile's K loop is long enough to hide its start and its stores, and one
+// mixed launch has the shorter tail
+constexpr int64_t kMidMaxTokens = 2048;
 struct Tuning {
   int variant_fwd = kDefaultVariantFwd, variant_bwd = kDefaultVariantBwd;
   bool variant_forced = false;   // lce_set_variant was called: no size-based choice of the tile
@@ -138,9 +142,7 @@ template <typename TIN> struct Variant2 { typedef GemmCfg<TIN, 256, 256, 128, 2,
 // four waves of 128x128 on v_mfma_f32_16x16x32 (16-bit inputs; fp32 inputs run the split-ring 32x32x2 loop instead)
 template <typename TIN> struct Variant3 { typedef GemmCfg16<TIN> Cfg; };
 template <> struct Variant3<float> { typedef GemmCfg<float, 256, 256, 128, 5, 4, 2, 2> Cfg; };
-// forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring; W is read
-// once, with non-temporal loads (a plain read of 1.09 GB runs at 6.3 TB/s on this card, a non-temporal one at 7.0; the
-// forward at H=3584, V=152064: 1 token 188.5 -> 173.5 us, 64 tokens 193.9 -> 183.8)
+// forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring
 template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
 template <typename TIN> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, 1> Cfg; };
 constexpr int kNumVariants = 4;
@@ -160,10 +162,12 @@ GemmArgs<typename Cfg::TIN> make_gemm_args(const typename Cfg::TIN* A, int64_t l
                                            int64_t ldct, int out_mode) {
   GemmArgs<typename Cfg::TIN> p;
   p.A = A; p.lda = lda; p.B = B; p.ldb = ldb; p.M = M; p.N = N; p.K = K;
+  p.a_pcol = 0;
   p.Cf = Cf; p.ldcf = ldcf; p.Ct = Ct; p.ldct = ldct; p.out_mode = out_mode;
   p.ksplit = 1; p.kslice = K; p.cf_split_stride = 0;
   p.m_dev = nullptr; p.k_dev = nullptr; p.k_gran = 1; p.tn = 0; p.b_rows_valid = 0; p.perm_rows = 0;
   const int tm = (int)((M + Cfg::BM - 1) / Cfg::BM), tn = (int)((N + Cfg::BN - 1) / Cfg::BN);
+  p.n_tiles = tn;
   p.map = TileMap::make(tm, tn, block_rows(tm), 1);
   return p;
 }
@@ -232,7 +236,7 @@ int forward_splits_256(int ntt, int nvt, int max_splits = kMaxSplits) {
   return best;
 }
 
-// Kept logits: fp32 [T][logits_cache_row(V)], element [t][v] = hidden[t] . W[v].  A backward that is given them
+// Kept logits: fp32, T * logits_cache_row(V) of them in panels (kept_logit), element (t, v) = hidden[t] . W[v].  A backward that is given them
 // computes d_logits from 4 bytes per logit instead of from a pass over W and a T x V x H product.  Offered for 16-bit
 // inputs while the cache is no larger than the weight it came from: T * V * 4 <= V * H * 2, i.e. up to H / 2 tokens;
 // beyond that nothing of size T x V is ever kept.
@@ -277,7 +281,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   p.split_span = rows_per_split ? rows_per_split : V;
   p.label_offset = label_offset;
   // xcache: the raw logits are kept for the backward
-  p.xcache = xcache; p.ldx = logits_cache_row(V);
+  p.xcache = xcache;
   p.map = TileMap::make(ntt, S, br, 1);
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   int rc;
@@ -347,15 +351,17 @@ int forward_splits_upper_bound(int64_t T, int64_t V, int max_splits = kMaxSplits
 }
 
 struct BwdLayout {
-  int64_t vchunk, tpad, vpad, ldS, ldST, ldWt, ldHt;
+  int64_t vchunk, tpad, vpad, ldS, pcol, ldST, ldWt, ldHt;  // ldS, pcol: see ds_at
   size_t off_dS[2], off_dST[2], off_Wt, off_Ht, off_dHacc, off_rows, off_inv, off_nrows, off_acounts, off_coef, off_keys[2], off_vals[2], off_hist, off_tokc, off_tokl, total;
   int sort_items, sort_passes;  // label sort (0 items: the one-hot part stays inside the d_logits tiles)
   int nchunks;
   int ksplit;  // K splits of the d_hidden GEMM (each with its own fp32 partial)
   bool tn;     // the gradient GEMMs read dS, a compact copy of hidden and W as they lie in memory (transposing LDS
                // reads for the K-major operands): no dS^T, no h^T
+  bool panels; // d_logits lie in panels of 64 columns
   bool tn_dh;  // ... and the d_hidden GEMM reads W as it lies in memory too: no W^T
   bool few;    // at most 128 tokens, 16-bit inputs: both gradient GEMMs run as the streaming kernels of few_tokens.hpp
+  bool mid;    // 129 to kMidMaxTokens tokens, one chunk, 16x16x32 loop: the two gradient GEMMs are launches of their own
 };
 
 // The d_weight GEMM takes the token-major d_logits and hidden as they are where transposing LDS reads exist (16-bit
@@ -374,6 +380,23 @@ int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
   const int64_t share = work / 256 / 2;
   const int64_t s = share > 0 ? (vchunk + share - 1) / share : 16;
   return (int)(s < 1 ? 1 : s > 16 ? 16 : s);
+}
+
+// K slices of a d_hidden GEMM that is a launch of its own: its tiles times slices run in rounds over the CUs, a slice takes
+// its slabs plus about ten slabs' time for the start and the 256 KB of fp32 it stores, and every slice adds a write and a
+// read of [T, H] fp32 (at 5 TB/s; a slab of 64 takes 1.2 us).  The fewest slab times win.  (333 tokens, H=3584, V=152064: 28
+// tiles x 9 slices are one round of 264 slabs; 16 slices, what the mixed launch would take, two rounds of 149.)
+int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk) {
+  const int64_t tiles = (T + 255) / 256 * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
+  const double per_slice = (double)T * H * 8.0 / 5.0e12 / 1.2e-6;
+  int best = 1;
+  double best_cost = -1.0;
+  for (int s = 1; s <= 32 && s <= slabs; ++s) {
+    const int64_t rounds = (tiles * s + kNumCUs - 1) / kNumCUs;
+    const double cost = (double)rounds * ((slabs + s - 1) / s + 10) + per_slice * s;
+    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = s; }
+  }
+  return best;
 }
 
 // layout for a given chunk width
@@ -403,13 +426,18 @@ BwdLayout bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, size
     L.tn_dh = true;  // W is read in place
   }
   L.nchunks = (int)((V + vchunk - 1) / vchunk);
+  L.mid = !L.few && L.tn && variant == kVariantCore16 && L.nchunks == 1 && T <= kMidMaxTokens;
+  if (L.mid && tu.dh_ksplit <= 0) L.ksplit = dh_ksplit_alone(T, H, vchunk);
   // Row strides are kept away from large powers of two (+128 bytes): with a 16 or 32 KiB stride the
   // 256 rows of an operand tile would all fall into the same L2 channel.
   // tokens / vocabulary rounded up to the K-permutation groups (gt, gv: at most one workgroup tile,
   // which is what the size query assumes; the launch passes the tile variant's wave-tile sizes)
   L.tpad = round_up(T, gt);
   L.vpad = round_up(V, gv);
-  L.ldS = vchunk + 64;
+  // 16-bit d_logits lie in panels of 64 columns where every reader takes them so; the panels are kept 128 bytes apart
+  L.panels = L.tn && (L.few || variant == kVariantCore16);
+  L.ldS = L.panels ? 64 : vchunk + 64;
+  L.pcol = L.panels ? L.tpad * 64 + 64 : 64;
   L.ldST = L.tpad + 64;
   L.ldWt = vchunk + 64;  // one chunk of W^T at a time
   L.ldHt = L.tn ? round_up(H, 256) + 64 : L.tpad + 64;  // tn: row stride of the compact copy of hidden [tpad][.]
@@ -418,7 +446,7 @@ BwdLayout bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, size
   // while the GEMMs of chunk c-1 consume the other pair
   for (int b = 0; b < 2; ++b) {
     L.off_dS[b] = o;
-    if (b == 0 || L.nchunks > 1) o += align256((size_t)L.tpad * L.ldS * esz);
+    if (b == 0 || L.nchunks > 1) o += align256(L.panels ? (size_t)(vchunk / 64) * L.pcol * esz : (size_t)L.tpad * L.ldS * esz);
     L.off_dST[b] = o;
     if (!L.tn && (b == 0 || L.nchunks > 1)) o += align256((size_t)vchunk * L.ldST * esz);
   }
@@ -472,7 +500,8 @@ BwdLayout bwd_layout(const Tuning& tu, int64_t T, int64_t H, int64_t V, size_t e
     if (tu.ws_budget > 0) {
       if ((double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
     } else {
-      int64_t cols = (((int64_t)256 << 20) / (T * (int64_t)esz)) / 256 * 256;
+      // (1 GiB where the logits may be kept: with them nothing of a next chunk runs beside this one's GEMMs)
+      int64_t cols = (((int64_t)(T <= logits_cache_max_tokens(H, esz) ? 1024 : 256) << 20) / (T * (int64_t)esz)) / 256 * 256;
       if (cols < 16384) {
         // many tokens: 16384 columns while one d_logits buffer stays within 1 GiB, never fewer than 8192
         cols = (((int64_t)1 << 30) / (T * (int64_t)esz)) / 256 * 256;
@@ -670,7 +699,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       d.g_lp = dlogprobs; d.g_lp_stride = reduction == LCE_REDUCTION_NONE ? 1 : 0;
       d.g_lp_scale = reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f;
       d.g_ent = dentropy;
-      d.dS = dS[c & 1]; d.ldS = L.ldS; d.dST = L.tn ? nullptr : dST[c & 1]; d.ldST = L.ldST; d.tpad = L.tpad;
+      d.dS = dS[c & 1]; d.ldS = L.ldS; d.pcol = L.pcol; d.dST = L.tn ? nullptr : dST[c & 1]; d.ldST = L.ldST; d.tpad = L.tpad;
       d.rows = rows; d.n_rows = n_rows;
       d.label_outside = lt.labels != nullptr ? tu.label_outside : 0;
       d.tokc = tokc; d.tokl = tokl; d.lab0 = v0;
@@ -698,7 +727,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       if constexpr (sizeof(TIN) == 2) {
         if (L.few) {
           FewArgs<TIN> q;
-          q.dS = dS[cc & 1]; q.ldS = L.ldS; q.Ht = Ht; q.ldHt = L.ldHt; q.W = W + v0 * ldw; q.ldw = ldw;
+          q.dS = dS[cc & 1]; q.ldS = L.ldS; q.pcol = L.pcol; q.Ht = Ht; q.ldHt = L.ldHt; q.W = W + v0 * ldw; q.ldw = ldw;
           q.vrows = vrows; q.ucols = kc; q.H = H;
           q.kt = T <= 64 ? 64 : 128; q.nt = (int)T; q.n_rows = n_rows;
           q.dW = !need_dw ? nullptr
@@ -721,6 +750,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           // W as it lies in memory (K-major for this product), fetched with transposing LDS reads
           p.gh = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, W + v0 * ldw, ldw, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1);
           p.gh.tn = 2;
+          p.gh.a_pcol = L.panels ? L.pcol : 0;
           p.gh.b_rows_valid = vrows;
         } else {
           // Wt = this chunk of W, transposed just before the launch (the previous launch, the last reader of the
@@ -735,6 +765,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
         if (need_dh && L.ksplit > 1) {
           p.gh.ksplit = L.ksplit;
           p.gh.kslice = round_up((kc + L.ksplit - 1) / L.ksplit, Cfg::BK);
+          p.gh.map = TileMap::make(p.gh.map.nrow_tiles, p.gh.n_tiles * L.ksplit, p.gh.map.br, p.gh.map.rows_fastest);
           p.gh.cf_split_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
         }
         // d_weight[v0 : v0 + vrows][H] = dST[vrows][Tpad] . Ht[H][Tpad]^T   (written in the input dtype, or as fp32)
@@ -746,14 +777,35 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           // d_weight[v0 : v0 + vrows][H] = dS[tokens][vrows]^T . hidden[tokens][H], both operands K-major
           p.gw = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, Ht, L.ldHt, vrows, H, round_up(T, 64), dw_f32, H, dw_t, H, grads_f32 ? 0 : 2);
           p.gw.tn = 1;
+          p.gw.a_pcol = L.panels ? L.pcol : 0;
           p.gw.perm_rows = 1;
           p.gw.k_dev = n_rows; p.gw.k_gran = 64;
         } else {
           p.gw = make_gemm_args<Cfg>(dST[cc & 1], L.ldST, Ht, L.ldHt, vrows, H, L.tpad, dw_f32, H, dw_t, H, grads_f32 ? 0 : 2);
           p.gw.k_dev = n_rows; p.gw.k_gran = KPerm<Cfg>::GT;
         }
-        p.n_gh = need_dh ? p.gh.map.total * L.ksplit : 0;
+        p.n_gh = need_dh ? p.gh.map.total : 0;
         p.n_gw = need_dw ? p.gw.map.total : 0;
+        if constexpr (Cfg::CORE16) {
+          if (L.mid && need_dw && dw_t && aligned16(dw_t) && !tu.split_bwd) {
+            // (one chunk: no d_logits tiles share this launch)
+            if (need_dh) {
+              BwdChunkArgs<TIN> q = p;
+              q.n_gw = q.n_ds = 0;
+              ProfScope prof(PC_GEMM_DH, st);
+              launch_chunk(q);
+              if ((rc = check_launch("lce_bwd_chunk16_kernel"))) return rc;
+            }
+            const int64_t tiles = ((p.gw.M + 255) / 256) * ((p.gw.N + 255) / 256);
+            ProfScope prof(PC_GEMM_DW, st);
+            allow_lds(lce_dw16_kernel<Cfg>, Cfg::LDS_BYTES);
+            hipLaunchKernelGGL(lce_dw16_kernel<Cfg>, dim3((unsigned)(tiles < kNumCUs ? p.gw.map.total : kNumCUs)), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st,
+                               p.gw);
+            if ((rc = check_launch("lce_dw16_kernel"))) return rc;
+            p.n_gw = p.n_gh = 0;
+            continue;
+          }
+        }
         if (need_dh && need_dw && p.gh.kslice > p.gw.K) {  // longer tiles go first
           std::swap(p.gh, p.gw);
           std::swap(p.n_gh, p.n_gw);
@@ -784,7 +836,6 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     if constexpr (sizeof(TIN) == 2 && Cfg::BM == 256) {
       if (xcache && L.tn && p.n_ds > 0) {
         // d_logits of this chunk from the logits the forward kept: no pass over W, no T x V x H product
-        const int64_t ldx = logits_cache_row(V);
         const int nrows = L.few ? ((int)(T <= 64 ? 64 : 128) < (int)L.tpad ? (int)(T <= 64 ? 64 : 128) : (int)L.tpad) : (int)L.tpad;
         const int64_t c0 = p.ds.v0 - vocab_offset;  // the chunk's first row of W
         {
@@ -792,7 +843,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           DsArgs<TIN> dq = p.ds;
           dq.rows = rows;  // (the 16x16x32 tiles read the compact copy of hidden and no list; the cache is indexed by token)
           hipLaunchKernelGGL((ds_from_logits_kernel<TIN, KPerm<Cfg>>), dim3((unsigned)(round_up(p.ds.vrows, 256) / 64)), dim3(256), 0, st, dq,
-                             xcache + c0, ldx, nrows);
+                             xcache + c0 * T, T, nrows);
           if ((rc = check_launch("ds_from_logits_kernel"))) return rc;
         }
         p.n_ds = 0;  // (what is left for the launch below: the gradient GEMMs of the previous chunk)

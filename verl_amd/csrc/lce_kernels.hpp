@@ -54,10 +54,16 @@ struct FwdArgs {
   TileMap map;       // rows = token tiles, cols = splits
   int64_t label_offset;  // W holds vocabulary rows [label_offset, label_offset + V) of a larger vocabulary (0 = all of it)
   // When not null (offered while the tokens are at most half the hidden size), the raw logits h . W[v] (fp32, before the division by the
-  // temperature) are kept for the backward, xcache[t * ldx + v] for t < T, v < V (ldx a multiple of 4).
+  // temperature) are kept for the backward: logit (t, v) at kept_logit(xcache, T, t, v).
   float* xcache;
-  int64_t ldx;
 };
+
+// Kept logits lie in panels of 16 vocabulary rows, [panel][token][16] fp32: what one 16 x 16 block of a tile holds is one
+// contiguous kilobyte, and a tile's 256 rows touch a few pages.  (As [token][vocabulary] the rows of a tile are 608 KB
+// apart at V=152064, a page each, and the stores of 16 rows x 64 bytes per instruction cost more than the data: 333
+// tokens, forward with kept logits KEEP_BEFORE -> KEEP_AFTER us.)
+template <typename P>
+LCE_DEV P kept_logit(P x, int64_t T, int64_t t, int64_t v) { return x + ((v >> 4) * T + t) * 16 + (v & 15); }
 
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename Cfg::TIN> p) {
@@ -106,7 +112,6 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename
         for (int j = 0; j < Cfg::FN; ++j) {
           const int64_t t = n0 + g.wave_n * Cfg::WN + j * 32 + ln;
           if (t >= p.T) continue;
-          float* dst = p.xcache + t * p.ldx;
 #pragma unroll
           for (int i = 0; i < Cfg::FM; ++i)
 #pragma unroll
@@ -114,11 +119,11 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename
               const int v = vbase + acc_row(i, 4 * q, hh);
               if (v + 3 < vend) {
                 const f32x4_t x4 = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                *reinterpret_cast<f32x4_t*>(dst + v) = x4;  // (non-temporal stores: 222 instead of 209 us)
+                *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = x4;  // (non-temporal stores: 222 instead of 209 us)
               } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                  if (v + e < vend) dst[v + e] = acc[i][j][4 * q + e];
+                  if (v + e < vend) *kept_logit(p.xcache, p.T, t, v + e) = acc[i][j][4 * q + e];
               }
             }
         }
@@ -349,8 +354,8 @@ struct DsArgs {
   int64_t g_lp_stride;  // 1 or 0
   float g_lp_scale;     // 1, or 1/T for mean
   const float* g_ent;   // [T] or null
-  TIN* dS;              // [T][ldS]      (token-major)
-  int64_t ldS;
+  TIN* dS;              // token-major; entry (t, u) at ds_at(dS, ldS, pcol, t, u)
+  int64_t ldS, pcol;
   TIN* dST;             // [vchunk][ldST] (vocab-major); null when the d_weight GEMM reads dS with transposing LDS reads
   int64_t ldST;
   int64_t tpad;         // tokens rounded up to the GEMM K granule: columns [T, tpad) of dST / rows [T, tpad) of dS are written as zeros
@@ -372,6 +377,14 @@ struct DsArgs {
   int64_t lab0;
   int64_t range_rows;  // few tokens: > 0 = every workgroup of lce_bwd_ds_kernel takes that many vocabulary rows (a multiple of the wave tile's)
 };
+
+// Where d_logits entry (token position t, column u) lies.  16-bit inputs on the kernels that read it so: panels of 64
+// columns, [panel][t][64] (ldS = 64, pcol = elements from panel to panel), so that a K slab of either gradient GEMM is a
+// contiguous piece: 64 columns of 256 tokens for d_hidden, 64 tokens of four panels for d_weight.  Otherwise rows of ldS
+// elements (pcol = 64).  With rows as long as the vocabulary (few tokens: one chunk) the 256 rows of a slab are 304 KB
+// apart, 39 pages of 2 MB that no TLB of a CU holds.
+template <typename P>
+LCE_DEV P ds_at(P dS, int64_t ldS, int64_t pcol, int64_t t, int64_t u) { return dS + (u >> 6) * pcol + t * ldS + (u & 63); }
 
 // The two gradient GEMMs sum over the vocabulary (d_hidden) and over the tokens (d_weight); any
 // permutation of the summation index is allowed as long as both operands of a GEMM use the same one.
@@ -514,7 +527,6 @@ LCE_DEV void ds_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x16_t (&ac
   }
   const bool tok_group_live = p.dST != nullptr && tok0 < p.tpad;  // the whole token group is inside dS^T's columns
   TIN* dst_t = p.dST + (tok0 + (int64_t)ln * FN);            // + vocab row * ldST   (token order: ln*FN + j)
-  TIN* dst_s = p.dS + (vloc0 + hh * 16 * FM);                // + token * ldS + i*16 + r (vocab order: hh, i, r)
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
 #pragma unroll
@@ -542,7 +554,7 @@ LCE_DEV void ds_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x16_t (&ac
           store_run<TIN, 8>(reinterpret_cast<TIN*>(stage_lds + row * Stg::ROW_BYTES + ((c ^ Stg::swz(row)) * 16)), stage[j]);
         } else {
           if (tok_ok[j])
-            store_run<TIN, 8>(dst_s + (tok0 + j * 32 + ln) * p.ldS + i * 16 + half * 8, stage[j]);
+            store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, tok0 + j * 32 + ln, vloc0 + hh * 16 * FM + i * 16 + half * 8), stage[j]);  // (vocab order: hh, i, r)
         }
       }
     }
@@ -557,7 +569,7 @@ LCE_DEV void ds_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x16_t (&ac
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stage_lds + row * Stg::ROW_BYTES + pc * 16);
       const int64_t tok = tok0 + row;
       // rows of tokens that do not take part are zeros (the staged values are); they pad the d_weight GEMM's K
-      if (tok < p.tpad) *reinterpret_cast<u32x4_t*>(p.dS + tok * p.ldS + vloc0 + c * 8) = v;
+      if (tok < p.tpad) *reinterpret_cast<u32x4_t*>(ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + c * 8)) = v;
     }
   }
 }
@@ -633,6 +645,7 @@ struct GemmArgs {
   int64_t lda;
   const TIN* B;
   int64_t ldb;
+  int64_t a_pcol;  // A lies in panels of 64 columns (see ds_at; lda = 64): elements from panel to panel; 0: rows of lda elements
   int64_t M, N, K;
   float* Cf;
   int64_t ldcf;
@@ -640,9 +653,10 @@ struct GemmArgs {
   int64_t ldct;
   int out_mode;
   TileMap map;  // rows = M tiles, cols = N tiles
-  // split K: workgroup `bid` computes tile bid % map.total over k in [s * kslice, min(K, (s + 1) * kslice)),
-  // s = bid / map.total < ksplit, into the fp32 partial Cf + s * cf_split_stride (out_mode 0 or 1 only)
-  int ksplit;
+  // split K: the map's columns are N tiles times slices (n_tiles N tiles, slice by slice), so that the tiles of a launch
+  // spread evenly over the XCDs whatever their number.  Slice s < ksplit covers k in [s * kslice, min(K, (s + 1) * kslice))
+  // into the fp32 partial Cf + s * cf_split_stride (out_mode 0 or 1 only)
+  int ksplit, n_tiles;
   int64_t kslice, cf_split_stride;
   // sizes known only on the device (null = use M / K): rows that exist, M = min(M, *m_dev), and the
   // reduction length, K = min(K, *k_dev rounded up to k_gran); K = 0 gives C = 0
@@ -697,16 +711,16 @@ LCE_DEV void gemm_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* ld
     p.K = k < p.K ? k : p.K;
   }
   int64_t k0 = 0, k1 = p.K;
-  if (p.ksplit > 1) {
-    const int s = bid / p.map.total;  // (the grid holds ksplit copies of the host-sized map)
-    bid -= s * p.map.total;
+  int tm, tn;
+  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
+  if (!map.decode(bid, tm, tn)) return;
+  if (p.ksplit > 1) {  // the map's columns are N tiles x slices
+    const int s = tn / p.n_tiles;
+    tn -= s * p.n_tiles;
     k0 = s * p.kslice;
     k1 = k0 + p.kslice < p.K ? k0 + p.kslice : p.K;
     p.Cf += s * p.cf_split_stride;
   }
-  int tm, tn;
-  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
-  if (!map.decode(bid, tm, tn)) return;
   const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
   const int lane = threadIdx.x & 63, hh = lane >> 5, ln = lane & 31;
   GemmCore<Cfg> g;
@@ -840,16 +854,16 @@ LCE_DEV void gemm_nb_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char*
     p.M = m < p.M ? m : p.M;
   }
   int64_t k0 = 0, k1 = p.K;
-  if (p.ksplit > 1) {
-    const int s = bid / p.map.total;
-    bid -= s * p.map.total;
+  int tm, tn;
+  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
+  if (!map.decode(bid, tm, tn)) return;
+  if (p.ksplit > 1) {  // the map's columns are N tiles x slices
+    const int s = tn / p.n_tiles;
+    tn -= s * p.n_tiles;
     k0 = s * p.kslice;
     k1 = k0 + p.kslice < p.K ? k0 + p.kslice : p.K;
     p.Cf += s * p.cf_split_stride;
   }
-  int tm, tn;
-  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
-  if (!map.decode(bid, tm, tn)) return;
   const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
   const int lane = threadIdx.x & 63, hh = lane >> 5, ln = lane & 31;
   GemmCore<Cfg> g;
@@ -1024,14 +1038,15 @@ inline __global__ void fill_zero_kernel(uint32_t* p, int64_t n) {
 }
 
 // out[r][:C] = in[rows[r]][:C] (in[r] without `rows`) for r < R = *n_rows (R without), zeros for the rows up to the next
-// multiple of 64 (the K granule of the d_weight GEMM); one 16-byte chunk per thread, C a multiple of 16 bytes
+// multiple of 64 (the K granule of the d_weight GEMM), and to 128 (lce_dw16_kernel wants two slabs); one 16-byte chunk per thread, C a multiple of 16 bytes
 template <typename T>
 __global__ void gather_rows_kernel(const T* in, int64_t ldi, int64_t R, int64_t C, T* out, int64_t ldo, int64_t rpad, const int* rows,
                                    const int* n_rows) {
   constexpr int N = 16 / (int)sizeof(T);
   typedef typename VecOf<T, N>::type vec_t;
   if (n_rows) R = *n_rows;
-  const int64_t rend = (R + 63) / 64 * 64 < rpad ? (R + 63) / 64 * 64 : rpad;
+  const int64_t rk = R > 0 && R <= 64 ? 128 : (R + 63) / 64 * 64;
+  const int64_t rend = rk < rpad ? rk : rpad;
   const int64_t per_row = C / N, n = rend * per_row;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
     const int64_t r = q / per_row, c = (q - r * per_row) * N;

@@ -133,16 +133,15 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
       for (int j = 0; j < NB; ++j) {
         const int64_t t = n0 + g.wave_n * Cfg::WN + j * 16 + l16;
         if (t < p.T) {
-          float* dst = p.xcache + t * p.ldx;
 #pragma unroll
           for (int i = 0; i < NB; ++i) {
             const int v = vbase + 16 * i + 4 * g4;
             if (v + 3 < vend) {
-              *reinterpret_cast<f32x4_t*>(dst + v) = acc[i][j];
+              *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = acc[i][j];
             } else {
 #pragma unroll
               for (int r = 0; r < 4; ++r)
-                if (v + r < vend) dst[v + r] = acc[i][j][r];
+                if (v + r < vend) *kept_logit(p.xcache, p.T, t, v + r) = acc[i][j][r];
             }
           }
         }
@@ -264,7 +263,7 @@ LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&a
         }
       }
       // rows of positions without a token are zeros (their constants make them so); they pad the d_weight GEMM's K
-      if (tok < p.tpad) store_run<TIN, 8>(p.dS + tok * p.ldS + vloc0 + ip * 32 + g4 * 8, d);
+      if (tok < p.tpad) store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + ip * 32 + g4 * 8), d);
     }
   }
 }
@@ -326,7 +325,7 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
       const int rel = lab[j] - (int)p.lab0 - vloc0;  // = 16 i + 4 g + r inside the wave tile
       const int64_t tok = tok0 + j * 16 + l16;
       if (rel >= 0 && rel < Cfg::WM && ((rel >> 2) & 3) == g4 && tok < p.tpad)
-        p.dS[tok * p.ldS + vloc0 + (rel >> 5) * 32 + g4 * 8 + ((rel >> 4) & 1) * 4 + (rel & 3)] = (typename Cfg::TIN)0.f;
+        *ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + (rel >> 5) * 32 + g4 * 8 + ((rel >> 4) & 1) * 4 + (rel & 3)) = (typename Cfg::TIN)0.f;
     }
   }
 }
@@ -395,24 +394,24 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
     p.K = k < p.K ? k : p.K;
   }
   int64_t k0 = 0, k1 = p.K;
-  if (p.ksplit > 1) {
-    const int s = bid / p.map.total;  // (the grid holds ksplit copies of the host-sized map)
-    bid -= s * p.map.total;
+  int tm, tn;
+  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
+  if (!map.decode(bid, tm, tn)) return;
+  if (p.ksplit > 1) {  // the map's columns are N tiles x slices
+    const int s = tn / p.n_tiles;
+    tn -= s * p.n_tiles;
     k0 = s * p.kslice;
     k1 = k0 + p.kslice < p.K ? k0 + p.kslice : p.K;
     p.Cf += s * p.cf_split_stride;
   }
-  int tm, tn;
-  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
-  if (!map.decode(bid, tm, tn)) return;
   const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
   GemmCore16<CoreCfg> g;
   f32x4_t acc[Cfg::NB][Cfg::NB];
   if (k0 < k1 && (CoreCfg::TRANS != 2 || k0 < p.b_rows_valid)) {
     // MFMA rows = n, MFMA columns = m
     if constexpr (CoreCfg::TRANS == 2)
-      g.init_mixed(p.B + k0 * p.ldb, p.ldb, n0, p.N - n0, p.b_rows_valid - k0, [](int r) { return KPerm<Cfg>::vocab_at(r); }, p.A + k0, p.lda,
-                   m0, p.M);
+      g.init_mixed(p.B + k0 * p.ldb, p.ldb, n0, p.N - n0, p.b_rows_valid - k0, [](int r) { return KPerm<Cfg>::vocab_at(r); },
+                   p.a_pcol ? p.A + (k0 >> 6) * p.a_pcol : p.A + k0, p.lda, m0, p.M, p.a_pcol ? p.a_pcol * 2 : (int64_t)Cfg::BKB);
     else
       g.init(p.B + k0, p.ldb, n0, p.N, p.A + k0, p.lda, m0, p.M);
     g.run(lds, k1 - k0, acc);
@@ -455,7 +454,7 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
   GemmCore16<Cfg> g;
   f32x4_t acc[Cfg::NB][Cfg::NB];
   if (p.K > 0) {
-    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0);  // MFMA rows = n, MFMA columns = m
+    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);  // MFMA rows = n, MFMA columns = m
     g.run(lds, p.K, acc);
   } else {
     g.set_lane();
@@ -485,6 +484,131 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
       }
     }
   }
+}
+
+// LDS write of 8 bytes as inline assembly, for the same reason as the reads: through the compiler it would wait for the
+// global->LDS loads in flight
+LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_write_b64 %0, %1" ::"v"(lds_addr), "v"(v)); }
+
+// A finished wave tile in 16 bits, C[m][n] with rows in the operand's column order (PermCfg's vocab_at), leaves the wave as
+// whole lines: 16 rows x 128 columns (one block column) at a time go through 4 KB of LDS that belong to this wave, 16-byte
+// chunk c of row r at c ^ r, and are stored four rows x 256 bytes per instruction.  (A CU stores such runs three to four
+// times as fast as the accumulators' own lane order, 16 rows x 64 bytes.)  Two buffers in turn: block column j is
+// written while j - 1 is read back, so that neither waits for the other.  32 stores, exactly, when the tile is FULL.
+template <typename Cfg, typename PermCfg, bool FULL>
+LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NB], int64_t m0, int64_t n0,
+                                int wave_m, int wave_n, uint32_t stage) {
+  typedef typename Cfg::TIN TIN;
+  typedef typename VecOf<TIN, 4>::type vec_t;
+  constexpr int NB = Cfg::NB;
+  const int lane = lane_anew(), g4 = lane >> 4, l16 = lane & 15;
+  const uint32_t wr = stage + (uint32_t)(l16 * 256 + (((g4 >> 1) ^ l16) * 16) + (g4 & 1) * 8);  // chunk 2 i + g4 / 2: ^ i * 32
+  const uint32_t rd = stage + (uint32_t)(g4 * 256 + ((l16 ^ g4) * 16));                          // row 4 k + g4: ^ k * 64, + k * 1024
+  // the store of row 4 k + g4 of block column j, chunk l16: a uniform row pointer and one offset per lane
+  const int64_t n = n0 + wave_m * Cfg::WM;
+  const uint32_t off = (uint32_t)(g4 * p.ldct + l16 * 8) * (uint32_t)sizeof(TIN);
+  const bool n_ok = FULL || n + l16 * 8 < p.N;
+  const int64_t mw = m0 + wave_n * Cfg::WN;
+  char* base = reinterpret_cast<char*>(p.Ct + mw * p.ldct + n);
+  auto write = [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      vec_t o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = round_to<TIN>(acc[i][j][r]);
+      lds_write8((wr ^ (uint32_t)(i * 32)) + (j & 1) * 4096, __builtin_bit_cast(u32x2_t, o));
+    }
+  };
+  auto store = [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    u32x4_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = lds_read16<0>((rd ^ (uint32_t)(k * 64)) + (j & 1) * 4096 + k * 1024);
+    GemmCore16<Cfg>::template wait_lgkm<0>();
+    // (opaque until the wait: the reads are assembly, the compiler does not know when they return)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(v[k]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      constexpr int u0 = 16 * j;
+      const int64_t row = KPerm<PermCfg>::vocab_at(u0 + 4 * k);  // (+ g4: four consecutive rows of C)
+      if (FULL || (n_ok && mw + row + g4 < p.M)) *reinterpret_cast<u32x4_t*>(base + row * p.ldct * (int64_t)sizeof(TIN) + off) = v[k];
+    }
+  };
+  static_for(std::make_integer_sequence<int, NB + 1>{}, [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    if constexpr (j < NB) write(jc);
+    if constexpr (j > 0) {
+      GemmCore16<Cfg>::template wait_lgkm<(j < NB ? NB : 0)>();  // block column j - 1 is in LDS (j's eight writes may be on their way)
+      store(std::integral_constant<int, j - 1>{});
+    }
+  });
+}
+
+// d_weight with tokens between the streaming kernels' range and the sizes where a tile's K loop hides everything else:
+// C[vocab_at(m)][n] = (TIN) sum_k A[k][m] B[k][n] as in gemm16_tn_tile (out_mode 2), by workgroups that stay (one per CU)
+// and walk the tiles, the K loops of successive tiles being one stream of slabs (GemmCore16::stream_tile).  With 333 tokens a
+// tile is six slabs of 1.2 to 1.5 us, and a workgroup per tile paid another 9 us for its start, its first loads, the drain of
+// its last and its stores.
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typename Cfg::TIN> p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  typedef GemmCfg16<typename Cfg::TIN, 1> TnCfg;
+  typedef GemmCore16<TnCfg> Core;
+  if (p.k_dev) {
+    // (at least two slabs, which the stream wants: gather_rows_kernel zeroes that many rows)
+    const int64_t k = *p.k_dev == 0 ? 0 : (*p.k_dev <= 64 ? 128 : ((int64_t)*p.k_dev + 63) / 64 * 64);
+    p.K = k < p.K ? k : p.K;
+  }
+  const int nk = (int)(p.K / 64);
+  Core g;
+  g.set_lane();
+  f32x4_t acc[Cfg::NB][Cfg::NB];
+  int bid = blockIdx.x, tm = 0, tn = 0;
+  auto next_tile = [&]() {  // the first tile at or behind bid (uniform over the workgroup)
+    for (; bid < p.map.total; bid += gridDim.x)
+      if (p.map.decode(bid, tm, tn)) return true;
+    return false;
+  };
+  if (!next_tile()) return;
+  if (nk == 0) {  // no token takes part
+    for (bool more = true; more; bid += gridDim.x, more = next_tile())
+      for (int q = threadIdx.x; q < Cfg::BM * (Cfg::BN / 8); q += Cfg::NTHREADS) {
+        const int64_t m = (int64_t)tm * Cfg::BM + q / (Cfg::BN / 8), n = (int64_t)tn * Cfg::BN + q % (Cfg::BN / 8) * 8;
+        if (m < p.M && n < p.N) *reinterpret_cast<u32x4_t*>(p.Ct + m * p.ldct + n) = u32x4_t{0u, 0u, 0u, 0u};
+      }
+    return;
+  }
+  typename Core::Stream s;
+  g.init_tn(p.B, p.ldb, (int64_t)tn * Cfg::BN, p.A, p.lda, (int64_t)tm * Cfg::BM, p.a_pcol);  // MFMA rows = n, MFMA columns = m
+  g.prologue(lds, p.K);
+  g.stream_begin(lds, s);
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+  bool behind = false, more = true;
+  while (more) {
+    const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
+    bid += gridDim.x;
+    more = next_tile();
+    const char *a_next = g.a_base, *b_next = g.b_base;
+    if (more) {
+      a_next = reinterpret_cast<const char*>(p.B + (int64_t)tn * Cfg::BN);
+      b_next = reinterpret_cast<const char*>(p.a_pcol ? p.A + (int64_t)tm * (Cfg::BM / 64) * p.a_pcol : p.A + (int64_t)tm * Cfg::BM);
+    }
+    g.reads_tn(lane_anew());
+    g.template stream_tile<32>(lds, nk, acc, s, a_next, b_next, behind);
+    g.a_base = a_next;
+    g.b_base = b_next;
+    const int free_slot = s.sb + 4 >= 5 ? s.sb + 4 - 5 : s.sb + 4;
+    const uint32_t stage = lds0 + (uint32_t)(free_slot * TnCfg::STAGE_BYTES) + g.wave * 8192;
+    __builtin_amdgcn_sched_barrier(0);
+    behind = m0 + Cfg::BM <= p.M && n0 + Cfg::BN <= p.N;
+    if (behind) gemm16_store_lines<TnCfg, Cfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
+    else gemm16_store_lines<TnCfg, Cfg, false>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();  // every wave has read its staged rows: the slot is the ring's again
+  }
+  Core::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
 }
 
 // ------------------------------------------------------------------------------------------------
