@@ -62,18 +62,21 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 
 // TRANS_: 0 both operands K-contiguous (row-major A[m][k], B[n][k]); 1 both K-major in memory, A[k][m] and
 // B[k][n], fetched with the transposing LDS read (two ds_read_b64_tr_b16 per fragment); 2 only A K-major (mixed).
-template <typename TIN_, int TRANS_ = 0>
+// NBN_: 16-column blocks per wave along the MFMA columns (tokens): 8 for tiles 256 columns wide, 6 for 192 (ragged token
+// counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
+template <typename TIN_, int TRANS_ = 0, int NBN_ = 8>
 struct GemmCfg16 {
   typedef TIN_ TIN;
   static_assert(sizeof(TIN_) == 2, "16-bit operands");
   static constexpr bool CORE16 = true;
-  static constexpr int BM = 256, BN = 256, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
+  static_assert(NBN_ == 8 || TRANS_ != 1, "both operands K-major: square tiles");
+  static constexpr int BM = 256, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
   static constexpr int WAVES_M = 2, WAVES_N = 2, NW = 4, NTHREADS = 256;
-  static constexpr int WM = 128, WN = 128;
-  static constexpr int NB = 8;                       // 16-row blocks per side of a wave tile
-  static constexpr int STAGE_BYTES = 32768;          // one operand's slab: 256 rows x 128 bytes, or 64 k-rows x 512 bytes
+  static constexpr int WM = 128, WN = 16 * NBN_;
+  static constexpr int NB = 8, NBN = NBN_;           // 16-row / 16-column blocks of a wave tile
+  static constexpr int STAGE_BYTES = 32768;          // one operand's slab: 256 rows x 128 bytes (or BN rows), or 64 k-rows x 512 bytes
   static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
-  static constexpr int HL = 8;                       // wave-wide 16-byte-per-lane loads per wave and half slab
+  static constexpr int HL = 8, HLB = NBN_;           // wave-wide 16-byte-per-lane loads per wave and half slab of A, of B
 };
 
 // The lane number, worked out anew where it is asked for.  A kernel that walks tiles has no register to spare across its K
@@ -88,13 +91,13 @@ LCE_DEV int lane_anew() {
 template <typename Cfg>
 struct GemmCore16 {
   typedef typename Cfg::TIN TIN;
-  static constexpr int NB = Cfg::NB, HL = Cfg::HL, SLOT = Cfg::STAGE_BYTES;
+  static constexpr int NB = Cfg::NB, NBN = Cfg::NBN, HL = Cfg::HL, HLB = Cfg::HLB, SLOT = Cfg::STAGE_BYTES;
   static constexpr bool TN = Cfg::TRANS == 1;
   static constexpr bool TA = Cfg::TRANS != 0, TB = Cfg::TRANS == 1;  // which operand is K-major in memory
 
   const char* a_base;
   const char* b_base;
-  uint32_t va[HL], vb[HL];  // per-lane byte offsets of the loads inside slab 0
+  uint32_t va[HL], vb[HLB];  // per-lane byte offsets of the loads inside slab 0
   uint32_t a_rd, b_rd;      // per-lane LDS read offsets inside a slot (block 0, k-step 0)
   int64_t a_slab, b_slab;   // bytes from one K slab to the next in memory
   int wave, lane, wave_m, wave_n;
@@ -128,10 +131,12 @@ struct GemmCore16 {
       const int row = (j * Cfg::NW + wave) * 8 + lr;
       const int c = pc ^ ((row >> 1) & 7);
       const int ra = row < rows_a ? row : rows_a - 1;
-      const int rb = row < rows_b ? row : rows_b - 1;
-      const int64_t gb = b_rows ? (int64_t)b_rows[n0 + rb] : (int64_t)rb;
       va[j] = (uint32_t)((int64_t)ra * lda * 2) + (uint32_t)(c * 16);
-      vb[j] = (uint32_t)(gb * ldb * 2) + (uint32_t)(c * 16);
+      if (j < HLB) {
+        const int rb = row < rows_b ? row : rows_b - 1;
+        const int64_t gb = b_rows ? (int64_t)b_rows[n0 + rb] : (int64_t)rb;
+        vb[j < HLB ? j : 0] = (uint32_t)(gb * ldb * 2) + (uint32_t)(c * 16);
+      }
     }
     const int r16 = lane & 15, g = lane >> 4;
     const uint32_t off = (uint32_t)(r16 * 128 + ((g ^ (r16 >> 1)) * 16));
@@ -204,10 +209,12 @@ struct GemmCore16 {
       const uint32_t col = (uint32_t)(((int64_t)ca * 8 < mcols ? ca : 0) * 16);
       va[j] = (uint32_t)((int64_t)prow * lda * 2) + col;
       va_tail[j] = (uint32_t)((int64_t)(prow < last_row ? prow : last_row) * lda * 2) + col;
-      const int rowb = (j * Cfg::NW + wave) * 8 + lr;
-      const int cb = pc ^ ((rowb >> 1) & 7);
-      const int rb = rowb < rows_b ? rowb : rows_b - 1;
-      vb[j] = (uint32_t)((int64_t)rb * ldb * 2) + (uint32_t)(cb * 16);
+      if (j < HLB) {
+        const int rowb = (j * Cfg::NW + wave) * 8 + lr;
+        const int cb = pc ^ ((rowb >> 1) & 7);
+        const int rb = rowb < rows_b ? rowb : rows_b - 1;
+        vb[j < HLB ? j : 0] = (uint32_t)((int64_t)rb * ldb * 2) + (uint32_t)(cb * 16);
+      }
     }
     const int g = lane >> 4, e = (lane & 15) >> 2, q = lane & 3;
     const int row = 8 * g + e;
@@ -232,14 +239,15 @@ struct GemmCore16 {
     __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
   }
 
-  // Fragments are read in the order a0, b0 .. b7, a1 .. a7 (F = 0 .. 15): the MFMAs walk the A blocks in the outer
-  // loop, so the first row of eight needs a0 and every b, the later rows one more a each.
-  static constexpr bool frag_is_a(int f) { return f == 0 || f > 8; }
-  static constexpr int frag_blk(int f) { return f == 0 ? 0 : (f <= 8 ? f - 1 : f - 8); }
+  // Fragments are read in the order a0, b0 .. b(NBN-1), a1 .. a7 (F = 0 .. NF-1): the MFMAs walk the A blocks in the outer
+  // loop, so the first row of NBN needs a0 and every b, the later rows one more a each.
+  static constexpr int NF = NB + NBN;
+  static constexpr bool frag_is_a(int f) { return f == 0 || f > NBN; }
+  static constexpr int frag_blk(int f) { return f == 0 ? 0 : (f <= NBN ? f - 1 : f - NBN); }
   static constexpr int CA = TA ? 2 : 1, CB = TB ? 2 : 1;  // LDS instructions per fragment of each operand
   // ra / rb: LDS address of the slot plus a_rd / b_rd; S: k-step inside the slab
   template <int F, int S>
-  LCE_DEV void read_frag(uint32_t ra, uint32_t rb, u32x4_t (&af)[NB], u32x4_t (&bf)[NB]) const {
+  LCE_DEV void read_frag(uint32_t ra, uint32_t rb, u32x4_t (&af)[NB], u32x4_t (&bf)[NBN]) const {
     constexpr bool is_a = frag_is_a(F);
     constexpr int blk = frag_blk(F);
     u32x4_t v;
@@ -256,33 +264,35 @@ struct GemmCore16 {
   }
 
   // LDS instructions issued up to and including fragment f of a k-step (f = -1: none)
-  static constexpr int upto(int f) { return f < 0 ? 0 : (f == 0 ? CA : (f <= 8 ? CA + CB * f : CA + 8 * CB + CA * (f - 8))); }
-  static constexpr int ALLI = 8 * (CA + CB);
+  static constexpr int upto(int f) { return f < 0 ? 0 : (f == 0 ? CA : (f <= NBN ? CA + CB * f : CA + NBN * CB + CA * (f - NBN))); }
+  static constexpr int ALLI = NB * CA + NBN * CB;
   // fragments of the next k-step issued before MFMA m of this one: one after each even MFMA of the first half
-  static constexpr int frags_before(int m) { return (m + 1) / 2 > 16 ? 16 : (m + 1) / 2; }
+  static constexpr int frags_before(int m) { return (m + 1) / 2 > NF ? NF : (m + 1) / 2; }
 
-  // One k-step: 64 MFMAs on (af, bf); the 16 fragment reads of the next k-step (from ra_n / rb_n, k-step S_N) and HL
-  // global->LDS loads are dealt between them.  WAIT: the fragments of this step were read during the previous step
+  // One k-step: NB x NBN MFMAs on (af, bf); the NF fragment reads of the next k-step (from ra_n / rb_n, k-step S_N) and the
+  // global->LDS loads of a half slab are dealt between them.  WAIT: the fragments of this step were read during the previous step
   // and may still be in flight.  DMA_B: the loads fetch the B operand's half slab `dma_ks` (else A's) into `dma_slot`; with
   // FROM, the half slab at `dma_from` instead.  FIRST: the accumulators start here.
   template <bool WAIT, int S_N, bool DMA_B, bool FROM = false, bool FIRST = false>
-  LCE_DEV void kstep(f32x4_t (&acc)[NB][NB], const u32x4_t (&af)[NB], const u32x4_t (&bf)[NB], uint32_t ra_n, uint32_t rb_n,
-                     u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NB], char* lds, int dma_slot, int64_t dma_ks,
+  LCE_DEV void kstep(f32x4_t (&acc)[NB][NBN], const u32x4_t (&af)[NB], const u32x4_t (&bf)[NBN], uint32_t ra_n, uint32_t rb_n,
+                     u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NBN], char* lds, int dma_slot, int64_t dma_ks,
                      const char* dma_from = nullptr) const {
-    static_for(std::make_integer_sequence<int, NB * NB>{}, [&](auto mc) {
+    constexpr int DMAS = DMA_B ? HLB : HL, EVERY = NB * NBN / DMAS;
+    static_assert(2 * NF <= NB * NBN && NB * NBN % DMAS == 0, "one fragment read after every second MFMA");
+    static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
       constexpr int m = decltype(mc)::value;
-      constexpr int i = m / NB, j = m % NB;
-      if constexpr (WAIT && (i == 0 || m % NB == 0)) {
-        constexpr int need = i == 0 ? 1 + j : 8 + i;  // the last fragment this MFMA depends on
+      constexpr int i = m / NBN, j = m % NBN;
+      if constexpr (WAIT && (i == 0 || j == 0)) {
+        constexpr int need = i == 0 ? 1 + j : NBN + i;  // the last fragment this MFMA depends on
         constexpr int allow = (ALLI - upto(need)) + upto(frags_before(m) - 1);
         wait_lgkm<(allow > 15 ? 15 : allow)>();
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (FIRST) Mma16<TIN>::first(acc[i][j], af[i], bf[j]);
       else Mma16<TIN>::run(acc[i][j], af[i], bf[j]);
-      if constexpr ((m & 1) == 0 && m / 2 < 16) read_frag<m / 2, S_N>(ra_n, rb_n, af_n, bf_n);
-      if constexpr (m % (NB * NB / HL) == 3) {
-        constexpr int j8 = m / (NB * NB / HL);
+      if constexpr ((m & 1) == 0 && m / 2 < NF) read_frag<m / 2, S_N>(ra_n, rb_n, af_n, bf_n);
+      if constexpr (m % EVERY == 3) {
+        constexpr int j8 = m / EVERY;
         if constexpr (FROM)
           __builtin_amdgcn_global_load_lds((gptr_t)(dma_from + (DMA_B ? vb[j8] : va[j8])), (lptr_t)(lds + dma_slot * SLOT + (j8 * Cfg::NW + wave) * 1024),
                                            16, 0, 0);
@@ -308,7 +318,7 @@ struct GemmCore16 {
     for (int hf = 0; hf < 4; ++hf) {
       const int64_t ks = hf / 2 < last ? hf / 2 : last;
 #pragma unroll
-      for (int j = 0; j < HL; ++j) dma(lds, hf, ks, (hf & 1) == 0, j);
+      for (int j = 0; j < ((hf & 1) == 0 ? HLB : HL); ++j) dma(lds, hf, ks, (hf & 1) == 0, j);
     }
   }
 
@@ -318,18 +328,18 @@ struct GemmCore16 {
   // between the two k-steps waits for slab i+1 (everything but those youngest loads) and for every wave's reads of slab
   // i; the second k-step then issues A(i+2) into B(i)'s slot and reads the first fragments of slab i+1.  Past the end
   // of K the loader re-fetches the last slab into slots nobody reads (a branch-free body), drained at the end.
-  LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NB]) const {
+  LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
     const int nk = (int)(K / Cfg::BK);
     const int64_t last = nk - 1;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    wait_vm<2 * HL>();  // slab 0 has landed
+      for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    wait_vm<HL + HLB>();  // slab 0 has landed
     __builtin_amdgcn_s_barrier();
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
-    u32x4_t af[2][NB], bf[2][NB];
-    static_for(std::make_integer_sequence<int, 16>{}, [&](auto fc) {
+    u32x4_t af[2][NB], bf[2][NBN];
+    static_for(std::make_integer_sequence<int, NF>{}, [&](auto fc) {
       read_frag<decltype(fc)::value, 0>(lds0 + SLOT + a_rd, lds0 + b_rd, af[0], bf[0]);
     });
     int sb = 0;  // slot of this slab's B half; its A half is in the next slot
@@ -340,7 +350,7 @@ struct GemmCore16 {
       const int fr = sb + 4 >= 5 ? sb + 4 - 5 : sb + 4;  // free slot: takes B(it+2)
       const int64_t ks = it + 2 < last ? it + 2 : last;
       kstep<true, 1, true>(acc, af[0], bf[0], lds0 + sa * SLOT + a_rd, lds0 + sb * SLOT + b_rd, af[1], bf[1], lds, fr, ks);
-      wait_vm<HL>();   // slab it+1 has landed; B(it+2) may still be in flight
+      wait_vm<HLB>();  // slab it+1 has landed; B(it+2) may still be in flight
       wait_lgkm<0>();  // this wave's reads of slab it have returned
       __builtin_amdgcn_s_barrier();
       kstep<false, 0, false>(acc, af[1], bf[1], lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, af[0], bf[0], lds, sb, ks);
@@ -358,26 +368,26 @@ struct GemmCore16 {
   // last blocks of the k-step can still be in the matrix pipe when the loop ends, so the last row of blocks is passed
   // through one more MFMA that the compiler does know (zero operands: acc + 0): behind a builtin it keeps the
   // distance to a read itself, and the matrix pipe orders it behind the assembly MFMA that wrote the same registers.
-  static LCE_DEV void retire(f32x4_t (&acc)[NB][NB]) {
+  static LCE_DEV void retire(f32x4_t (&acc)[NB][NBN]) {
     asm volatile("s_nop 15\n\ts_nop 7" ::);
     const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[NB - 1][j] = Mma16<TIN>::known(acc[NB - 1][j], zero, zero);
+    for (int j = 0; j < NBN; ++j) acc[NB - 1][j] = Mma16<TIN>::known(acc[NB - 1][j], zero, zero);
   }
 
   // ---- a workgroup that walks tiles: the K loops of successive tiles as one stream of slabs -------------------
   // The loads two slabs ahead of the end of a tile are those of the next tile's first slabs, and the fragments that the last
   // k-step reads are the next tile's first: between two tiles there is neither a drain nor a first load to wait for.
   struct Stream {
-    u32x4_t af[NB], bf[NB];  // the next slab's first fragments
-    int sb;                  // slot of its B half
+    u32x4_t af[NB], bf[NBN];  // the next slab's first fragments
+    int sb;                   // slot of its B half
   };
   // prologue() of the first tile has been called, and nothing else was loaded since
   LCE_DEV void stream_begin(char* lds, Stream& s) const {
-    wait_vm<2 * HL>();
+    wait_vm<HL + HLB>();
     __builtin_amdgcn_s_barrier();
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
-    static_for(std::make_integer_sequence<int, 16>{}, [&](auto fc) {
+    static_for(std::make_integer_sequence<int, NF>{}, [&](auto fc) {
       read_frag<decltype(fc)::value, 0>(lds0 + SLOT + a_rd, lds0 + b_rd, s.af, s.bf);
     });
     s.sb = 0;
@@ -388,13 +398,14 @@ struct GemmCore16 {
   // gives them the time of a slab and a half.  Ring slot (s.sb + 4) % 5 is free when this returns, until the barrier that
   // the caller places before the next call.
   template <int STORES>
-  LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NB], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
+  LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
     static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
+    static_assert(NBN == NB, "square tiles");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     int sb = s.sb;
     auto slab = [&](auto first, int it) {
       constexpr bool FIRST = decltype(first)::value;
-      u32x4_t af1[NB], bf1[NB];  // the fragments of the slab's second k-step
+      u32x4_t af1[NB], bf1[NBN];  // the fragments of the slab's second k-step
       const int sa = sb + 1 >= 5 ? sb + 1 - 5 : sb + 1;
       const int nb = sb + 2 >= 5 ? sb + 2 - 5 : sb + 2;
       const int na = sb + 3 >= 5 ? sb + 3 - 5 : sb + 3;
@@ -421,7 +432,7 @@ struct GemmCore16 {
     retire(acc);
   }
 
-  LCE_DEV void run(char* lds, int64_t K, f32x4_t (&acc)[NB][NB]) const {
+  LCE_DEV void run(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
     prologue(lds, K);
     main(lds, K, acc);
   }

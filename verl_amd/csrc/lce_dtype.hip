@@ -36,6 +36,7 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case 3: LCE_RUN(Variant3);
     case kSelT64: LCE_RUN(VariantT64);
     case kSelT128: LCE_RUN(VariantT128);
+    case kSelN192: LCE_RUN(VariantN192);
   }
 #undef LCE_RUN
   return fail(LCE_E_ARG, "tile selector %d out of range", sel);

@@ -54,7 +54,8 @@ struct Tuning {
 };
 
 // tile selectors of the per-type launchers: 0..3 are the variants of lce_set_variant, then the two few-token forward tiles
-enum { kSelT64 = 4, kSelT128 = 5 };
+// and the 16x16x32 loop on tiles 192 tokens wide
+enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6 };
 
 // The launchers of one element type each (lce_dtype.hip compiles them as separate objects).  `sel` is a tile selector;
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
@@ -142,6 +143,9 @@ template <typename TIN> struct Variant2 { typedef GemmCfg<TIN, 256, 256, 128, 2,
 // four waves of 128x128 on v_mfma_f32_16x16x32 (16-bit inputs; fp32 inputs run the split-ring 32x32x2 loop instead)
 template <typename TIN> struct Variant3 { typedef GemmCfg16<TIN> Cfg; };
 template <> struct Variant3<float> { typedef GemmCfg<float, 256, 256, 128, 5, 4, 2, 2> Cfg; };
+// the same loop on tiles 192 tokens wide
+template <typename TIN> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6> Cfg; };
+template <> struct VariantN192<float> : Variant3<float> {};
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring
 template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
 template <typename TIN> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, 1> Cfg; };
@@ -166,7 +170,9 @@ GemmArgs<typename Cfg::TIN> make_gemm_args(const typename Cfg::TIN* A, int64_t l
   p.Cf = Cf; p.ldcf = ldcf; p.Ct = Ct; p.ldct = ldct; p.out_mode = out_mode;
   p.ksplit = 1; p.kslice = K; p.cf_split_stride = 0;
   p.m_dev = nullptr; p.k_dev = nullptr; p.k_gran = 1; p.tn = 0; p.b_rows_valid = 0; p.perm_rows = 0;
-  const int tm = (int)((M + Cfg::BM - 1) / Cfg::BM), tn = (int)((N + Cfg::BN - 1) / Cfg::BN);
+  // (the 16x16x32 loop takes its MFMA columns from A)
+  const int rm = Cfg::CORE16 ? Cfg::BN : Cfg::BM, rn = Cfg::CORE16 ? Cfg::BM : Cfg::BN;
+  const int tm = (int)((M + rm - 1) / rm), tn = (int)((N + rn - 1) / rn);
   p.n_tiles = tn;
   p.map = TileMap::make(tm, tn, block_rows(tm), 1);
   return p;
@@ -203,7 +209,7 @@ int launch_gemm(const typename Cfg::TIN* A, int64_t lda, const typename Cfg::TIN
 // sixteen splits give three rounds of 38.
 constexpr int kNumCUs = 256;
 constexpr int kMaxSplits = 256;
-int forward_splits_256(int ntt, int nvt, int max_splits = kMaxSplits) {
+int forward_splits_256(int ntt, int nvt, int max_splits = kMaxSplits, int64_t* cost_out = nullptr) {
   const int bc = 32 / block_rows(ntt);
   if (max_splits < bc) return max_splits > 1 ? max_splits : 1;  // (a caller with very little room for partial results)
   auto cost_of = [&](int S, int64_t* tiles_out) {
@@ -219,6 +225,7 @@ int forward_splits_256(int ntt, int nvt, int max_splits = kMaxSplits) {
     const int64_t cost = cost_of(S, nullptr);
     if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = S; }
   }
+  if (cost_out) *cost_out = best_cost;
   // Among the split counts within 2 % of the fewest tile-times, one that makes a workgroup walk 48 to 96 tiles is
   // preferred: the longer the walk, the further the 32 workgroups of an XCD drift apart and the fewer of them share a
   // fetched slab; the shorter, the more the rounds' ramp-up shows.  Measured, forward launch (tiles per workgroup: ms):
@@ -234,6 +241,19 @@ int forward_splits_256(int ntt, int nvt, int max_splits = kMaxSplits) {
   }
   if (pick > 0) best = pick;
   return best;
+}
+
+// Token tiles 256 or 192 wide for the 16x16x32 loop?  Every token tile costs a full tile's matrix work whatever its fill, so
+// the width with the fewer tile-times over the whole launch wins; a 192-wide tile-time is three quarters of a 256-wide one
+// and 5 % for its smaller share of operand reuse (equal padded counts, 1536 tokens: 1.289 against 1.275 ms).  Measured,
+// forward at H=3584, V=152064, 256 / 192 wide: 192 tokens 280 / 249 us, 333: 467 / 382, 500: 478 / 520, 576: 657 / 523, 700:
+// 660 / 695, 900: 893 / 838, 1000: 887 / 996, 1152: 1082 / 1001, 1300: 1267 / 1161, 2048: 1668 / 1757.
+bool forward_tiles_192(int64_t T, int64_t V) {
+  int64_t c256 = 0, c192 = 0;
+  const int nvt = (int)((V + 255) / 256);
+  forward_splits_256((int)((T + 255) / 256), nvt, kMaxSplits, &c256);
+  forward_splits_256((int)((T + 191) / 192), nvt, kMaxSplits, &c192);
+  return c192 * 79 < c256 * 100;
 }
 
 // Kept logits: fp32, T * logits_cache_row(V) of them in panels (kept_logit), element (t, v) = hidden[t] . W[v].  A backward that is given them
@@ -257,7 +277,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   const int br = block_rows(ntt), bc = 32 / br;
   const int nrb = (ntt + br - 1) / br;
   // max_splits: the caller's workspace holds partial results of at most that many splits
-  int S = Cfg::BN == 256 ? forward_splits_256(ntt, nvt, max_splits) : bc * ((8 + nrb - 1) / nrb);
+  int S = Cfg::BN > 128 ? forward_splits_256(ntt, nvt, max_splits) : bc * ((8 + nrb - 1) / nrb);
   if (S > nvt) S = nvt;
   if (S > max_splits) S = max_splits;
   // The narrow token tiles serve the HBM-bound case (up to 128 tokens: one streaming read of W).  There each
@@ -341,6 +361,8 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
 // upper bound of the number of vocabulary splits forward_impl picks, over the token-tile widths in use
 int forward_splits_upper_bound(int64_t T, int64_t V, int max_splits = kMaxSplits) {
   int best = forward_splits_256((int)((T + 255) / 256), (int)((V + 255) / 256), max_splits);
+  const int best_192 = forward_splits_256((int)((T + 191) / 192), (int)((V + 255) / 256), max_splits);
+  if (best_192 > best) best = best_192;
   for (int bn = 64; bn <= 128; bn <<= 1) {
     const int ntt = (int)((T + bn - 1) / bn);
     const int br = block_rows(ntt), bc = 32 / br, nrb = (ntt + br - 1) / br;
@@ -361,6 +383,7 @@ struct BwdLayout {
   bool panels; // d_logits lie in panels of 64 columns
   bool tn_dh;  // ... and the d_hidden GEMM reads W as it lies in memory too: no W^T
   bool few;    // at most 128 tokens, 16-bit inputs: both gradient GEMMs run as the streaming kernels of few_tokens.hpp
+  bool mid_192;  // ... d_hidden on token tiles 192 wide
   bool mid;    // 129 to kMidMaxTokens tokens, one chunk, 16x16x32 loop: the two gradient GEMMs are launches of their own
 };
 
@@ -386,16 +409,20 @@ int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
 // its slabs plus about ten slabs' time for the start and the 256 KB of fp32 it stores, and every slice adds a write and a
 // read of [T, H] fp32 (at 5 TB/s; a slab of 64 takes 1.2 us).  The fewest slab times win.  (333 tokens, H=3584, V=152064: 28
 // tiles x 9 slices are one round of 264 slabs; 16 slices, what the mixed launch would take, two rounds of 149.)
-int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk) {
-  const int64_t tiles = (T + 255) / 256 * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
+// `wide`: token tiles 256 wide, else 192, whose slabs take 0.91 of the time here (the operand that all token tiles share, W,
+// arrives at the same rate: 333 tokens, 28 tiles either way, 408 / 370 us; 900 tokens on five narrow tiles 895 us, 1000 on
+// four wide ones 857).
+int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cost_out) {
+  const int64_t tiles = (wide ? (T + 255) / 256 : (T + 191) / 192) * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
   const double per_slice = (double)T * H * 8.0 / 5.0e12 / 1.2e-6;
   int best = 1;
   double best_cost = -1.0;
   for (int s = 1; s <= 32 && s <= slabs; ++s) {
     const int64_t rounds = (tiles * s + kNumCUs - 1) / kNumCUs;
-    const double cost = (double)rounds * ((slabs + s - 1) / s + 10) + per_slice * s;
+    const double cost = (double)rounds * ((slabs + s - 1) / s + 10) * (wide ? 1.0 : 0.91) + per_slice * s;
     if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = s; }
   }
+  *cost_out = best_cost;
   return best;
 }
 
@@ -427,7 +454,13 @@ BwdLayout bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, size
   }
   L.nchunks = (int)((V + vchunk - 1) / vchunk);
   L.mid = !L.few && L.tn && variant == kVariantCore16 && L.nchunks == 1 && T <= kMidMaxTokens;
-  if (L.mid && tu.dh_ksplit <= 0) L.ksplit = dh_ksplit_alone(T, H, vchunk);
+  L.mid_192 = false;
+  if (L.mid) {
+    double c256, c192;
+    const int s256 = dh_ksplit_alone(T, H, vchunk, true, &c256), s192 = dh_ksplit_alone(T, H, vchunk, false, &c192);
+    L.mid_192 = c192 < c256;
+    if (tu.dh_ksplit <= 0) L.ksplit = L.mid_192 ? s192 : s256;
+  }
   // Row strides are kept away from large powers of two (+128 bytes): with a 16 or 32 KiB stride the
   // 256 rows of an operand tile would all fall into the same L2 channel.
   // tokens / vocabulary rounded up to the K-permutation groups (gt, gv: at most one workgroup tile,
@@ -787,30 +820,37 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
         p.n_gh = need_dh ? p.gh.map.total : 0;
         p.n_gw = need_dw ? p.gw.map.total : 0;
         if constexpr (Cfg::CORE16) {
-          if (L.mid && need_dw && dw_t && aligned16(dw_t) && !tu.split_bwd) {
-            // (one chunk: no d_logits tiles share this launch)
-            if (need_dh) {
-              BwdChunkArgs<TIN> q = p;
-              q.n_gw = q.n_ds = 0;
+          // (one chunk: no d_logits tiles share this launch)
+          if (L.mid && !tu.split_bwd && need_dh) {
+            auto launch_dh = [&](auto narrow) {
+              typedef typename std::conditional<decltype(narrow)::value, typename VariantN192<TIN>::Cfg, Cfg>::type DhCfg;
+              GemmArgs<TIN> q = p.gh;
+              const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
+              q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
               ProfScope prof(PC_GEMM_DH, st);
-              launch_chunk(q);
-              if ((rc = check_launch("lce_bwd_chunk16_kernel"))) return rc;
-            }
+              allow_lds(lce_dh16_kernel<DhCfg>, DhCfg::LDS_BYTES);
+              hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3(q.map.total), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q);
+              return check_launch("lce_dh16_kernel");
+            };
+            if ((rc = L.mid_192 ? launch_dh(std::true_type{}) : launch_dh(std::false_type{}))) return rc;
+            p.n_gh = 0;
+          }
+          if (L.mid && !tu.split_bwd && need_dw && dw_t && aligned16(dw_t)) {
             const int64_t tiles = ((p.gw.M + 255) / 256) * ((p.gw.N + 255) / 256);
             ProfScope prof(PC_GEMM_DW, st);
             allow_lds(lce_dw16_kernel<Cfg>, Cfg::LDS_BYTES);
             hipLaunchKernelGGL(lce_dw16_kernel<Cfg>, dim3((unsigned)(tiles < kNumCUs ? p.gw.map.total : kNumCUs)), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st,
                                p.gw);
             if ((rc = check_launch("lce_dw16_kernel"))) return rc;
-            p.n_gw = p.n_gh = 0;
-            continue;
+            p.n_gw = 0;
           }
+          if (p.n_gw + p.n_gh == 0) continue;
         }
-        if (need_dh && need_dw && p.gh.kslice > p.gw.K) {  // longer tiles go first
+        if (p.n_gh && p.n_gw && p.gh.kslice > p.gw.K) {  // longer tiles go first
           std::swap(p.gh, p.gw);
           std::swap(p.n_gh, p.n_gw);
           swapped = true;
-        } else if (!need_dw) {  // an only GEMM sits in the first slot
+        } else if (!p.n_gw) {  // an only GEMM sits in the first slot
           p.gw = p.gh;
           p.n_gw = p.n_gh;
           p.n_gh = 0;

@@ -12,8 +12,8 @@ namespace lce {
 // vocabulary rows (one wave tile) the entries are ordered so that what a lane holds of two neighbouring blocks is one
 // 16-byte run and the four lane groups follow each other (64 contiguous bytes per token and store instruction):
 // row v = 16 i + 4 g + r  ->  position 32 (i / 2) + 8 g + 4 (i % 2) + r.  Tokens keep their order.
-template <typename TIN, int TR>
-struct KPerm<GemmCfg16<TIN, TR>> {
+template <typename TIN, int TR, int NBN>
+struct KPerm<GemmCfg16<TIN, TR, NBN>> {
   static constexpr int GT = 128, GV = 128;
   static __host__ __device__ __forceinline__ int64_t token(int64_t t) { return t; }
   static __host__ __device__ __forceinline__ int64_t token_at(int64_t u) { return u; }
@@ -32,18 +32,18 @@ struct KPerm<GemmCfg16<TIN, TR>> {
 // ------------------------------------------------------------------------------------------------
 // folds one finished tile into the running per-token statistics (FULL: no padded vocabulary rows in the tile)
 template <typename Cfg, bool FULL>
-LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NB], float (&m)[Cfg::NB],
-                        float (&a)[Cfg::NB], float (&b)[Cfg::NB], const int (&lab)[Cfg::NB], int vbase, int vend, int64_t tok0, int g4,
+LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], float (&m)[Cfg::NBN],
+                        float (&a)[Cfg::NBN], float (&b)[Cfg::NBN], const int (&lab)[Cfg::NBN], int vbase, int vend, int64_t tok0, int g4,
                         int l16) {
-  constexpr int NB = Cfg::NB;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
   // The running statistics do not live in registers across the K loop (256 accumulator and 256 ordinary registers are
   // in use there; the compiler keeps them in scratch memory meanwhile).  All of them are asked for here, so that they
   // come back in one batch of loads instead of column by column, each column waiting for its own (forward at 16384
   // tokens: H=896 4.57 -> 4.43 ms, H=1536 6.39 -> 6.28, H=3584 12.91 -> 12.85).
 #pragma unroll
-  for (int j = 0; j < NB; ++j) asm volatile("" : "+v"(m[j]), "+v"(a[j]), "+v"(b[j]));
+  for (int j = 0; j < NBN; ++j) asm volatile("" : "+v"(m[j]), "+v"(a[j]), "+v"(b[j]));
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < NBN; ++j) {
     __builtin_amdgcn_sched_barrier(0);  // one block column at a time (register pressure)
     float x[NB * 4];
 #pragma unroll
@@ -92,7 +92,7 @@ LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, const f32x4_t (&acc
 // KEEP: the tiles also write their logits to p.xcache (FwdArgs), for a backward that then does not recompute them
 template <typename Cfg, bool KEEP>
 LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
-  constexpr int NB = Cfg::NB;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
   int tt, s;
   if (!p.map.decode(blockIdx.x, tt, s)) return;
   const int64_t n0 = (int64_t)tt * Cfg::BN;
@@ -100,10 +100,10 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
   GemmCore16<Cfg> g;
   g.set_lane();
 
-  float m[NB], a[NB], b[NB];
-  int lab[NB];
+  float m[NBN], a[NBN], b[NBN];
+  int lab[NBN];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < NBN; ++j) {
     m[j] = kNegBig;
     a[j] = 0.f;
     b[j] = 0.f;
@@ -112,7 +112,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
     lab[j] = (y >= 0 && y < p.V) ? (int)y : -1;
   }
 
-  f32x4_t acc[NB][NB];
+  f32x4_t acc[NB][NBN];
   const int64_t row0 = (int64_t)s * p.split_stride;
   const int64_t vend64 = row0 + p.split_span < p.V ? row0 + p.split_span : p.V;
   const int vend = (int)vend64;
@@ -130,7 +130,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
       // operations are ever in flight.
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
+      for (int j = 0; j < NBN; ++j) {
         const int64_t t = n0 + g.wave_n * Cfg::WN + j * 16 + l16;
         if (t < p.T) {
 #pragma unroll
@@ -150,7 +150,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
           GemmCore16<Cfg>::template wait_vm<0>();
         } else if (j % 2 == 1 && j >= 3) {
           __builtin_amdgcn_sched_barrier(0);
-          if (j == NB - 1) GemmCore16<Cfg>::template wait_vm<24>();
+          if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<24>();
           else GemmCore16<Cfg>::template wait_vm<32>();
         }
       }
@@ -170,7 +170,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
   // merge the four lane groups (same token, different vocabulary rows), then the two waves along the vocabulary
   f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);  // [WAVES_M][BN]
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < NBN; ++j) {
 #pragma unroll
     for (int off = 16; off <= 32; off <<= 1) {
       const float m2 = __shfl_xor(m[j], off), a2 = __shfl_xor(a[j], off), b2 = __shfl_xor(b[j], off);
@@ -233,12 +233,12 @@ inline __global__ void ds_token_consts_kernel(const int* rows, const int* n_rows
 // it after the common arithmetic (zero when the label's entry is kept out of the tiles, + G when everything is inside).
 // EDGE: the tile reaches beyond the chunk's last row; those entries are zeros.
 template <typename Cfg, bool LABEL, bool EDGE>
-LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NB], const f32x4_t (&tc)[Cfg::NB],
-                           const int (&lab)[Cfg::NB], int64_t tok0, int vloc0, int g4, int l16) {
+LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], const f32x4_t (&tc)[Cfg::NBN],
+                           const int (&lab)[Cfg::NBN], int64_t tok0, int vloc0, int g4, int l16) {
   typedef typename Cfg::TIN TIN;
-  constexpr int NB = Cfg::NB;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < NBN; ++j) {
     const float lse2 = tc[j][0], C0 = tc[j][1], C1 = tc[j][2], G = tc[j][3];
     // the label's entry: block pair rel / 32, lane group (rel / 4) % 4, value 4 ((rel / 16) % 2) + rel % 4 of the run
     const int rel = (LABEL && p.label_outside != 1) ? lab[j] - (int)p.lab0 - vloc0 : -1;  // (1: the tiles hold the softmax terms only)
@@ -273,7 +273,7 @@ LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&a
 // the backward's combined launch, whose tail then is a strip long.)
 template <typename Cfg>
 LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
-  constexpr int NB = Cfg::NB;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
   const int64_t Tc = p.n_rows ? (int64_t)*p.n_rows : p.T;  // tokens that take part
   int tt, vt;
   const TileMap map = p.n_rows ? p.map.with_rows((int)((Tc + Cfg::BN - 1) / Cfg::BN)) : p.map;
@@ -283,10 +283,10 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
   GemmCore16<Cfg> g;
   g.set_lane();
   const int64_t tok0 = n0 + g.wave_n * Cfg::WN;  // first position of this wave's group
-  f32x4_t tc[NB];
-  int lab[NB];
+  f32x4_t tc[NBN];
+  int lab[NBN];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < NBN; ++j) {
     const int64_t pos = tok0 + j * 16 + l16;
     tc[j] = f32x4_t{1.0e30f, 0.f, 0.f, 0.f};
     lab[j] = -1;
@@ -296,14 +296,14 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
     }
   }
   g.init(p.W, p.ldw, (int64_t)vt * Cfg::BM, p.vrows, p.h, p.ldh, n0, Tc, p.rows);
-  f32x4_t acc[NB][NB];
+  f32x4_t acc[NB][NBN];
   g.run(lds, p.H, acc);
   const int vloc0 = vt * Cfg::BM + g.wave_m * Cfg::WM;  // chunk-local vocabulary index of this wave's first row
   // fast path: no padded vocabulary rows and no label in the wave tile
   bool has_label = false;
   if (p.label_outside != 1) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
+    for (int j = 0; j < NBN; ++j) {
       const int rel = lab[j] - (int)p.lab0 - vloc0;
       has_label |= (rel >= 0 && rel < Cfg::WM);
     }
@@ -321,7 +321,7 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
   else ds16_epilogue<Cfg, false, false>(p, acc, tc, lab, tok0, vloc0, g4, l16);
   if (labels_here && p.label_outside == 2) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
+    for (int j = 0; j < NBN; ++j) {
       const int rel = lab[j] - (int)p.lab0 - vloc0;  // = 16 i + 4 g + r inside the wave tile
       const int64_t tok = tok0 + j * 16 + l16;
       if (rel >= 0 && rel < Cfg::WM && ((rel >> 2) & 3) == g4 && tok < p.tpad)
@@ -336,7 +336,7 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
 // for C[m][n] = sum_k A[m][k] B[n][k] lane l holds m = 16 j + l % 16 and n = 16 i + 4 (l / 16) + r.
 // ------------------------------------------------------------------------------------------------
 template <typename Cfg, int MODE, bool EDGE>
-LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NB], int64_t mw, int64_t nw) {
+LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
   typedef typename Cfg::TIN TIN;
   // mw, nw: this lane's row of block column 0 and its first column of block row 0
   // accumulate modes: the old values of block column j + 1 are fetched before column j is added and stored, so that
@@ -354,9 +354,9 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t
   };
   if (MODE & 1) fetch(0);
 #pragma unroll
-  for (int j = 0; j < Cfg::NB; ++j) {
+  for (int j = 0; j < Cfg::NBN; ++j) {
     const int64_t m = mw + j * 16;
-    if ((MODE & 1) && j + 1 < Cfg::NB) fetch(j + 1);
+    if ((MODE & 1) && j + 1 < Cfg::NBN) fetch(j + 1);
     if (EDGE && m >= p.M) continue;
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i) {
@@ -379,7 +379,7 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t
   }
 }
 
-// CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2>: then B is K-major as it lies in memory, B[k][n] with row
+// CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2, NBN>: then B is K-major as it lies in memory, B[k][n] with row
 // stride ldb, its rows in the order KPerm<Cfg>::vocab_at of A's columns (the d_hidden GEMM reading W in place: no W^T);
 // rows of B at or beyond p.b_rows_valid do not exist (A is zero in those columns).
 template <typename Cfg, typename CoreCfg = Cfg>
@@ -395,7 +395,7 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
   }
   int64_t k0 = 0, k1 = p.K;
   int tm, tn;
-  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BM - 1) / Cfg::BM)) : p.map;
+  const TileMap map = p.m_dev ? p.map.with_rows((int)((p.M + Cfg::BN - 1) / Cfg::BN)) : p.map;
   if (!map.decode(bid, tm, tn)) return;
   if (p.ksplit > 1) {  // the map's columns are N tiles x slices
     const int s = tn / p.n_tiles;
@@ -404,9 +404,9 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
     k1 = k0 + p.kslice < p.K ? k0 + p.kslice : p.K;
     p.Cf += s * p.cf_split_stride;
   }
-  const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
+  const int64_t m0 = (int64_t)tm * Cfg::BN, n0 = (int64_t)tn * Cfg::BM;  // (MFMA rows = n, MFMA columns = m)
   GemmCore16<CoreCfg> g;
-  f32x4_t acc[Cfg::NB][Cfg::NB];
+  f32x4_t acc[Cfg::NB][Cfg::NBN];
   if (k0 < k1 && (CoreCfg::TRANS != 2 || k0 < p.b_rows_valid)) {
     // MFMA rows = n, MFMA columns = m
     if constexpr (CoreCfg::TRANS == 2)
@@ -421,10 +421,10 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i)
 #pragma unroll
-      for (int j = 0; j < Cfg::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < Cfg::NBN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   const int64_t mw = m0 + g.wave_n * Cfg::WN + (g.lane & 15), nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
-  const bool edge = m0 + Cfg::BM > p.M || n0 + Cfg::BN > p.N;
+  const bool edge = m0 + Cfg::BN > p.M || n0 + Cfg::BM > p.N;
 #define LCE_EPI16(MODE)                                             \
   if (edge) gemm16_epilogue<Cfg, MODE, true>(p, acc, mw, nw);       \
   else gemm16_epilogue<Cfg, MODE, false>(p, acc, mw, nw)
@@ -630,6 +630,13 @@ template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void gemm16_tn_kernel(GemmArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1>, Cfg>(p, blockIdx.x, lds);
+}
+
+// d_hidden on its own: C[m][n] (+)= sum_k A[m][k] B[k][n] as in gemm16_tile's mixed mode (W read in place)
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Cfg::TIN> p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN>>(p, blockIdx.x, lds);
 }
 
 template <typename Cfg>
