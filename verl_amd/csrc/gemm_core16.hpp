@@ -64,13 +64,15 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 // B[k][n], fetched with the transposing LDS read (two ds_read_b64_tr_b16 per fragment); 2 only A K-major (mixed).
 // NBN_: 16-column blocks per wave along the MFMA columns (tokens): 8 for tiles 256 columns wide, 6 for 192 (ragged token
 // counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
-template <typename TIN_, int TRANS_ = 0, int NBN_ = 8>
+// A_EARLY_: the ring's early operand (see main) is A instead of B.
+template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0>
 struct GemmCfg16 {
   typedef TIN_ TIN;
   static_assert(sizeof(TIN_) == 2, "16-bit operands");
   static constexpr bool CORE16 = true;
   static_assert(NBN_ == 8 || TRANS_ != 1, "both operands K-major: square tiles");
   static constexpr int BM = 256, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
+  static constexpr bool A_EARLY = A_EARLY_ != 0;
   static constexpr int WAVES_M = 2, WAVES_N = 2, NW = 4, NTHREADS = 256;
   static constexpr int WM = 128, WN = 16 * NBN_;
   static constexpr int NB = 8, NBN = NBN_;           // 16-row / 16-column blocks of a wave tile
@@ -92,7 +94,7 @@ template <typename Cfg>
 struct GemmCore16 {
   typedef typename Cfg::TIN TIN;
   static constexpr int NB = Cfg::NB, NBN = Cfg::NBN, HL = Cfg::HL, HLB = Cfg::HLB, SLOT = Cfg::STAGE_BYTES;
-  static constexpr bool TN = Cfg::TRANS == 1;
+  static constexpr bool TN = Cfg::TRANS == 1, AE = Cfg::A_EARLY;
   static constexpr bool TA = Cfg::TRANS != 0, TB = Cfg::TRANS == 1;  // which operand is K-major in memory
 
   const char* a_base;
@@ -310,7 +312,7 @@ struct GemmCore16 {
     __builtin_amdgcn_s_waitcnt(((N & 0xF) | ((N >> 4) << 14)) | 0x0F70);
   }
 
-  // Issues the loads of the first two slabs (half slabs E0 L0 E1 L1 into slots 0..3; E = the B operand).  LDS must be
+  // Issues the loads of the first two slabs (half slabs E0 L0 E1 L1 into slots 0..3; E = the early operand).  LDS must be
   // free: every wave past its last read of the previous tile and its own loads drained (a workgroup barrier after main()).
   LCE_DEV void prologue(char* lds, int64_t K) const {
     const int64_t last = K / Cfg::BK - 1;
@@ -318,15 +320,17 @@ struct GemmCore16 {
     for (int hf = 0; hf < 4; ++hf) {
       const int64_t ks = hf / 2 < last ? hf / 2 : last;
 #pragma unroll
-      for (int j = 0; j < ((hf & 1) == 0 ? HLB : HL); ++j) dma(lds, hf, ks, (hf & 1) == 0, j);
+      for (int j = 0; j < (((hf & 1) == 0) != AE ? HLB : HL); ++j) dma(lds, hf, ks, ((hf & 1) == 0) != AE, j);
     }
   }
 
   // The K loop (K a positive multiple of 64); prologue() must have been called for this tile, and no other vector memory
-  // load may have been issued by this wave since (the waits count outstanding loads).  Slab i reads B from slot 2i % 5
-  // and A from the next slot.  Its first k-step issues the loads of B(i+2) into the slot that A(i-1) left; the barrier
+  // load may have been issued by this wave since (the waits count outstanding loads).  One operand is early (E: B, or A with
+  // A_EARLY), the other late (L).  Slab i reads E from slot 2i % 5 and L from the next slot.  Its first k-step issues the
+  // loads of E(i+2) into the slot that L(i-1) left; the barrier
   // between the two k-steps waits for slab i+1 (everything but those youngest loads) and for every wave's reads of slab
-  // i; the second k-step then issues A(i+2) into B(i)'s slot and reads the first fragments of slab i+1.  Past the end
+  // i; the second k-step then issues L(i+2) into E(i)'s slot and reads the first fragments of slab i+1.  So E has a slab and
+  // a half to arrive and L one slab.  Past the end
   // of K the loader re-fetches the last slab into slots nobody reads (a branch-free body), drained at the end.
   LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
     const int nk = (int)(K / Cfg::BK);
@@ -340,21 +344,21 @@ struct GemmCore16 {
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     u32x4_t af[2][NB], bf[2][NBN];
     static_for(std::make_integer_sequence<int, NF>{}, [&](auto fc) {
-      read_frag<decltype(fc)::value, 0>(lds0 + SLOT + a_rd, lds0 + b_rd, af[0], bf[0]);
+      read_frag<decltype(fc)::value, 0>(lds0 + (AE ? 0 : SLOT) + a_rd, lds0 + (AE ? SLOT : 0) + b_rd, af[0], bf[0]);
     });
-    int sb = 0;  // slot of this slab's B half; its A half is in the next slot
+    int se = 0;  // slot of this slab's early half; its late half is in the next slot
     for (int it = 0; it < nk; ++it) {
-      const int sa = sb + 1 >= 5 ? sb + 1 - 5 : sb + 1;
-      const int nb = sb + 2 >= 5 ? sb + 2 - 5 : sb + 2;
-      const int na = sb + 3 >= 5 ? sb + 3 - 5 : sb + 3;
-      const int fr = sb + 4 >= 5 ? sb + 4 - 5 : sb + 4;  // free slot: takes B(it+2)
+      const int sl = se + 1 >= 5 ? se + 1 - 5 : se + 1;
+      const int ne = se + 2 >= 5 ? se + 2 - 5 : se + 2;
+      const int nl = se + 3 >= 5 ? se + 3 - 5 : se + 3;
+      const int fr = se + 4 >= 5 ? se + 4 - 5 : se + 4;  // free slot: takes E(it+2)
       const int64_t ks = it + 2 < last ? it + 2 : last;
-      kstep<true, 1, true>(acc, af[0], bf[0], lds0 + sa * SLOT + a_rd, lds0 + sb * SLOT + b_rd, af[1], bf[1], lds, fr, ks);
-      wait_vm<HLB>();  // slab it+1 has landed; B(it+2) may still be in flight
-      wait_lgkm<0>();  // this wave's reads of slab it have returned
+      kstep<true, 1, !AE>(acc, af[0], bf[0], lds0 + (AE ? se : sl) * SLOT + a_rd, lds0 + (AE ? sl : se) * SLOT + b_rd, af[1], bf[1], lds, fr, ks);
+      wait_vm<AE ? HL : HLB>();  // slab it+1 has landed; E(it+2) may still be in flight
+      wait_lgkm<0>();            // this wave's reads of slab it have returned
       __builtin_amdgcn_s_barrier();
-      kstep<false, 0, false>(acc, af[1], bf[1], lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, af[0], bf[0], lds, sb, ks);
-      sb = nb;
+      kstep<false, 0, AE>(acc, af[1], bf[1], lds0 + (AE ? ne : nl) * SLOT + a_rd, lds0 + (AE ? nl : ne) * SLOT + b_rd, af[0], bf[0], lds, se, ks);
+      se = ne;
     }
     wait_vm<0>();    // drain the redundant tail fetches before LDS is reused
     wait_lgkm<0>();  // and the reads of the slab after the last
@@ -400,7 +404,7 @@ struct GemmCore16 {
   template <int STORES>
   LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
     static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
-    static_assert(NBN == NB, "square tiles");
+    static_assert(NBN == NB && !AE, "square tiles, B early");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     int sb = s.sb;
     auto slab = [&](auto first, int it) {

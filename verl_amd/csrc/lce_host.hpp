@@ -143,9 +143,12 @@ template <typename TIN> struct Variant2 { typedef GemmCfg<TIN, 256, 256, 128, 2,
 // four waves of 128x128 on v_mfma_f32_16x16x32 (16-bit inputs; fp32 inputs run the split-ring 32x32x2 loop instead)
 template <typename TIN> struct Variant3 { typedef GemmCfg16<TIN> Cfg; };
 template <> struct Variant3<float> { typedef GemmCfg<float, 256, 256, 128, 5, 4, 2, 2> Cfg; };
-// the same loop on tiles 192 tokens wide
-template <typename TIN> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6> Cfg; };
+// the same loop on tiles 192 tokens wide, the weight early: with so few tokens it streams from HBM, and a slab of the narrow
+// tile leaves it less time to arrive (333 tokens: forward 382 -> 365 us, d_hidden 370 -> 330)
+template <typename TIN> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6, 1> Cfg; };
 template <> struct VariantN192<float> : Variant3<float> {};
+// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us)
+template <typename TIN> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1> Cfg; };
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring
 template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
 template <typename TIN> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, 1> Cfg; };
@@ -409,9 +412,7 @@ int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
 // its slabs plus about ten slabs' time for the start and the 256 KB of fp32 it stores, and every slice adds a write and a
 // read of [T, H] fp32 (at 5 TB/s; a slab of 64 takes 1.2 us).  The fewest slab times win.  (333 tokens, H=3584, V=152064: 28
 // tiles x 9 slices are one round of 264 slabs; 16 slices, what the mixed launch would take, two rounds of 149.)
-// `wide`: token tiles 256 wide, else 192, whose slabs take 0.91 of the time here (the operand that all token tiles share, W,
-// arrives at the same rate: 333 tokens, 28 tiles either way, 408 / 370 us; 900 tokens on five narrow tiles 895 us, 1000 on
-// four wide ones 857).
+// `wide`: token tiles 256 wide, else 192, whose slabs take 0.82 of the time (28 tiles either way: 512 tokens 412 us, 333: 330).
 int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cost_out) {
   const int64_t tiles = (wide ? (T + 255) / 256 : (T + 191) / 192) * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
   const double per_slice = (double)T * H * 8.0 / 5.0e12 / 1.2e-6;
@@ -419,7 +420,7 @@ int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cos
   double best_cost = -1.0;
   for (int s = 1; s <= 32 && s <= slabs; ++s) {
     const int64_t rounds = (tiles * s + kNumCUs - 1) / kNumCUs;
-    const double cost = (double)rounds * ((slabs + s - 1) / s + 10) * (wide ? 1.0 : 0.91) + per_slice * s;
+    const double cost = (double)rounds * ((slabs + s - 1) / s + 10) * (wide ? 1.0 : 0.82) + per_slice * s;
     if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = s; }
   }
   *cost_out = best_cost;
@@ -823,7 +824,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           // (one chunk: no d_logits tiles share this launch)
           if (L.mid && !tu.split_bwd && need_dh) {
             auto launch_dh = [&](auto narrow) {
-              typedef typename std::conditional<decltype(narrow)::value, typename VariantN192<TIN>::Cfg, Cfg>::type DhCfg;
+              typedef typename std::conditional<decltype(narrow)::value, typename VariantN192<TIN>::Cfg, typename VariantWEarly<TIN>::Cfg>::type DhCfg;
               GemmArgs<TIN> q = p.gh;
               const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
               q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
