@@ -65,7 +65,12 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 // NBN_: 16-column blocks per wave along the MFMA columns (tokens): 8 for tiles 256 columns wide, 6 for 192 (ragged token
 // counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
 // A_EARLY_: the ring's early operand (see main) is A instead of B.
-template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0>
+// TERMS_: products per slab.  1: the operands are what they are.  6: fp32 operands, each held as three bfloat16 planes
+// x = x1 + x2 + x3 (exact: 3 x 8 significant bits); a slab is multiplied as a1 b1 + a1 b2 + a2 b1 + a1 b3 + a3 b1 + a2 b2 into
+// the same fp32 accumulators.  What is left out, a2 b3 + a3 b2 + a3 b3, is below 2^-26 of |a b|, a quarter of what rounding
+// ONE fp32 product or partial sum costs, and the products themselves are exact.  Six bfloat16 MFMAs take six sixteenths
+// of the matrix pipe's time of the fp32 one.
+template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0, int TERMS_ = 1>
 struct GemmCfg16 {
   typedef TIN_ TIN;
   static_assert(sizeof(TIN_) == 2, "16-bit operands");
@@ -73,6 +78,8 @@ struct GemmCfg16 {
   static_assert(NBN_ == 8 || TRANS_ != 1, "both operands K-major: square tiles");
   static constexpr int BM = 256, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
   static constexpr bool A_EARLY = A_EARLY_ != 0;
+  static constexpr int TERMS = TERMS_;
+  static_assert(TERMS_ == 1 || TERMS_ == 6, "products per slab");
   static constexpr int WAVES_M = 2, WAVES_N = 2, NW = 4, NTHREADS = 256;
   static constexpr int WM = 128, WN = 16 * NBN_;
   static constexpr int NB = 8, NBN = NBN_;           // 16-row / 16-column blocks of a wave tile
@@ -102,6 +109,7 @@ struct GemmCore16 {
   uint32_t va[HL], vb[HLB];  // per-lane byte offsets of the loads inside slab 0
   uint32_t a_rd, b_rd;      // per-lane LDS read offsets inside a slot (block 0, k-step 0)
   int64_t a_slab, b_slab;   // bytes from one K slab to the next in memory
+  int64_t a_plane = 0, b_plane = 0;  // TERMS == 6: bytes from plane to plane
   int wave, lane, wave_m, wave_n;
   // mixed mode: row of A inside a slab that each load fetches, A's row stride in bytes and the number of its rows that exist
   uint32_t va_tail[HL];         // mixed mode: va of the last slab of A that has rows, rows beyond them clamped
@@ -229,14 +237,21 @@ struct GemmCore16 {
   // load j of one operand's half slab number `ks` into ring slot `slot`
   LCE_DEV void dma(char* lds, int slot, int64_t ks, bool is_b, int j) const {
     char* dst = lds + slot * SLOT + (j * Cfg::NW + wave) * 1024;
+    int64_t plane = 0;
+    if constexpr (Cfg::TERMS == 6) {
+      // product number ks % 6 of slab ks / 6: planes (a, b) = (0,0) (0,1) (1,0) (0,2) (2,0) (1,1), two bits each
+      const int n = (int)ks, slab = n / 6, t = 2 * (n - 6 * slab);
+      plane = is_b ? ((0x484 >> t) & 3) * b_plane : ((0x610 >> t) & 3) * a_plane;
+      ks = slab;
+    }
     const char* src;
     if (Cfg::TRANS == 2 && !is_b) {
       // slabs with rows that do not exist take the last slab that has any, with its rows clamped (branch-free: the
       // hand-placed schedule of a k-step must stay one basic block)
       const bool tail = ks >= a_ks_full;
-      src = a_base + (tail ? a_ks_last : ks) * a_slab + (tail ? va_tail[j] : va[j]);
+      src = a_base + (tail ? a_ks_last : ks) * a_slab + plane + (tail ? va_tail[j] : va[j]);
     } else {
-      src = (is_b ? b_base + ks * b_slab + vb[j] : a_base + ks * a_slab + va[j]);
+      src = (is_b ? b_base + ks * b_slab + plane + vb[j] : a_base + ks * a_slab + plane + va[j]);
     }
     __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
   }
@@ -315,7 +330,7 @@ struct GemmCore16 {
   // Issues the loads of the first two slabs (half slabs E0 L0 E1 L1 into slots 0..3; E = the early operand).  LDS must be
   // free: every wave past its last read of the previous tile and its own loads drained (a workgroup barrier after main()).
   LCE_DEV void prologue(char* lds, int64_t K) const {
-    const int64_t last = K / Cfg::BK - 1;
+    const int64_t last = K / Cfg::BK * Cfg::TERMS - 1;
 #pragma unroll
     for (int hf = 0; hf < 4; ++hf) {
       const int64_t ks = hf / 2 < last ? hf / 2 : last;
@@ -333,7 +348,7 @@ struct GemmCore16 {
   // a half to arrive and L one slab.  Past the end
   // of K the loader re-fetches the last slab into slots nobody reads (a branch-free body), drained at the end.
   LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
-    const int nk = (int)(K / Cfg::BK);
+    const int nk = (int)(K / Cfg::BK) * Cfg::TERMS;
     const int64_t last = nk - 1;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -404,7 +419,7 @@ struct GemmCore16 {
   template <int STORES>
   LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
     static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
-    static_assert(NBN == NB && !AE, "square tiles, B early");
+    static_assert(NBN == NB && !AE && Cfg::TERMS == 1, "square tiles, B early");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     int sb = s.sb;
     auto slab = [&](auto first, int it) {

@@ -2,6 +2,7 @@
 // that do not depend on the GEMM element type.  The forward / backward launchers are compiled per element type in
 // lce_dtype.hip.  Nothing here allocates device memory: callers bring the workspace.
 #include "lce_host.hpp"
+#include "lce_terms.hpp"
 
 namespace lce_shared {
 thread_local char err[512] = "";
@@ -195,9 +196,14 @@ static size_t forward_workspace_need(int64_t T, int64_t V, int max_splits) {
   return align256((size_t)forward_splits_upper_bound(T, V > 0 ? V : 1, max_splits) * (size_t)T * 16) + 2 * align256((size_t)T * 4);
 }
 
+// ... and what the bfloat16 planes of fp32 inputs take on top, where they are used (0: they are not)
+static size_t forward_terms_need(int64_t T, int64_t H, int64_t V, int dtype) {
+  if (T <= 0 || H <= 0 || V <= 0 || !use_terms(tuning_snapshot(), T, H, V, dtype)) return 0;
+  return terms_fwd_plan(T, H, V).total;
+}
+
 size_t lce_forward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
-  (void)H; (void)dtype;
-  return forward_workspace_need(T, V, kMaxSplits);
+  return std::max(forward_workspace_need(T, V, kMaxSplits), forward_terms_need(T, H, V, dtype));
 }
 
 // shared body of lce_forward and lce_forward_shard
@@ -231,6 +237,9 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
     // 4.5% faster again once `hidden` is far larger than the memory-side cache (T=65536, H=5120: 671 MB)
     else if (T <= 8192 || (uint64_t)T * (uint64_t)H * esize(dtype) > (512ull << 20)) sel = 1;
   }
+  // (lce_forward_static's built-in buffer has no room for the planes: fp32 tiles there)
+  const size_t terms_need = forward_terms_need(T, H, V, dtype);
+  if (terms_need && workspace_bytes >= terms_need) sel = kSelTerms;
   if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
@@ -349,9 +358,14 @@ int lce_merge_shards(const float* partials, int R, int64_t T, int reduction, flo
   return rc;
 }
 
+static size_t backward_workspace_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype, int64_t vchunk) {
+  if (use_terms(tu, T, H, V, dtype)) return terms_bwd_layout(tu, T, H, V, vchunk).total + 256;
+  return bwd_layout(tu, T, H, V, esize(dtype), vchunk).total + 256;
+}
+
 size_t lce_backward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype, int64_t vchunk) {
   if (T <= 0 || H <= 0 || V <= 0) return 256;
-  return bwd_layout(tuning_snapshot(), T, H, V, esize(dtype), vchunk).total + 256;
+  return backward_workspace_need(tuning_snapshot(), T, H, V, dtype, vchunk);
 }
 
 // shared body of lce_backward and lce_backward_shard
@@ -375,10 +389,10 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
   if (!aligned16(d_hidden) || !aligned16(d_weight)) return fail(LCE_E_ARG, "gradients must be 16-byte aligned");
   if (vchunk < 0) return fail(LCE_E_ARG, "vchunk must be >= 0");
   const Tuning tu = tuning_snapshot();
-  const size_t need = bwd_layout(tu, T, H, V, esz, vchunk).total + 256;
+  const size_t need = backward_workspace_need(tu, T, H, V, dtype, vchunk);
   if (!workspace || workspace_bytes < need) return fail(LCE_E_WORKSPACE, "backward workspace too small: %zu < %zu", workspace_bytes, need);
   char* ws = reinterpret_cast<char*>(align256(reinterpret_cast<size_t>(workspace)));
-  return kBackward[dtype](bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
+  return kBackward[dtype](use_terms(tu, T, H, V, dtype) ? kSelTerms : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
                           accumulate, entropy_b, dlogprobs, dentropy, d_hidden, d_weight, grads_f32, ws, vchunk, st, vocab_offset,
                           tu, xcache);
 }

@@ -3,6 +3,9 @@
 // tile variant.  The build compiles the six combinations side by side; lce_abi.hip calls them through the declarations in
 // lce_host.hpp.
 #include "lce_host.hpp"
+#if LCE_TU_DTYPE == 1
+#include "lce_terms.hpp"
+#endif
 
 #if !defined(LCE_TU_DTYPE) || !defined(LCE_TU_PART)
 #error "compile with -DLCE_TU_DTYPE=<LCE_DTYPE_*> -DLCE_TU_PART=<0|1>"
@@ -37,6 +40,11 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case kSelT64: LCE_RUN(VariantT64);
     case kSelT128: LCE_RUN(VariantT128);
     case kSelN192: LCE_RUN(VariantN192);
+#if LCE_TU_DTYPE == 1
+    case kSelTerms:
+      return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
+                           label_offset, shard_out);
+#endif
   }
 #undef LCE_RUN
   return fail(LCE_E_ARG, "tile selector %d out of range", sel);
@@ -65,6 +73,11 @@ int TU_FN(backward)(int sel, LCE_BWD_PARAMS) {
   switch (sel) {
     case kDefaultVariantBwd: LCE_RUN(Variant1);
     case kVariantCore16: LCE_RUN(Variant3);
+#if LCE_TU_DTYPE == 1
+    case kSelTerms:
+      return backward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
+                            (float*)dw, ws, vchunk, st, vocab_offset, tu);
+#endif
   }
 #undef LCE_RUN
   return fail(LCE_E_ARG, "variant %d out of range", sel);

@@ -9,6 +9,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <mutex>
 #include <utility>
 #include <vector>
@@ -54,8 +55,8 @@ struct Tuning {
 };
 
 // tile selectors of the per-type launchers: 0..3 are the variants of lce_set_variant, then the two few-token forward tiles
-// and the 16x16x32 loop on tiles 192 tokens wide
-enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6 };
+// and the 16x16x32 loop on tiles 192 tokens wide, and the bfloat16 planes of fp32 inputs (lce_terms.hpp)
+enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7 };
 
 // The launchers of one element type each (lce_dtype.hip compiles them as separate objects).  `sel` is a tile selector;
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
@@ -169,7 +170,7 @@ GemmArgs<typename Cfg::TIN> make_gemm_args(const typename Cfg::TIN* A, int64_t l
                                            int64_t ldct, int out_mode) {
   GemmArgs<typename Cfg::TIN> p;
   p.A = A; p.lda = lda; p.B = B; p.ldb = ldb; p.M = M; p.N = N; p.K = K;
-  p.a_pcol = 0;
+  p.a_pcol = 0; p.a_plane = p.b_plane = 0;
   p.Cf = Cf; p.ldcf = ldcf; p.Ct = Ct; p.ldct = ldct; p.out_mode = out_mode;
   p.ksplit = 1; p.kslice = K; p.cf_split_stride = 0;
   p.m_dev = nullptr; p.k_dev = nullptr; p.k_gran = 1; p.tn = 0; p.b_rows_valid = 0; p.perm_rows = 0;
@@ -266,6 +267,47 @@ bool forward_tiles_192(int64_t T, int64_t V) {
 int64_t logits_cache_row(int64_t V) { return round_up(V, 64); }
 int64_t logits_cache_max_tokens(int64_t H, size_t esz) { return esz == 2 ? H / 2 : 0; }
 
+// merges the partial statistics of S splits per token into the five outputs (or a shard's partial), and the reduction
+int forward_merge(const f32x4_t* parts, const float* xlabel, const int64_t* labels, int64_t label_offset, int64_t V, int S, int64_t T, float c,
+                  float temperature, int reduction, float* lp_tok, float* logprobs, float* entropy, float* maximum, float* accumulate,
+                  float* entropy_b, float* shard_out, hipStream_t st) {
+  int rc;
+  if (shard_out) {
+    ProfScope prof(PC_FWD_MERGE, st);
+    f32x4_t* out = reinterpret_cast<f32x4_t*>(shard_out);
+    if (S >= 64)
+      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<64>, dim3((unsigned)((T * 64 + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S,
+                         T, c, 1.0f / temperature, out);
+    else if (S >= 8)
+      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<8>, dim3((unsigned)((T * 8 + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S, T,
+                         c, 1.0f / temperature, out);
+    else
+      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<1>, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S, T,
+                         c, 1.0f / temperature, out);
+    return check_launch("lce_fwd_shard_merge_kernel");
+  }
+  {
+    ProfScope prof(PC_FWD_MERGE, st);
+    if (S >= 64)
+      hipLaunchKernelGGL(lce_fwd_merge_kernel<64>, dim3((unsigned)((T * 64 + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S, T,
+                         c, 1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
+    else if (S >= 8)
+      hipLaunchKernelGGL(lce_fwd_merge_kernel<8>, dim3((unsigned)((T * 8 + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S, T,
+                         c, 1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
+    else
+      hipLaunchKernelGGL(lce_fwd_merge_kernel<1>, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, st, parts, xlabel, labels, label_offset, V, S, T, c,
+                         1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
+    rc = check_launch("lce_fwd_merge_kernel");
+  }
+  if (rc) return rc;
+  if (reduction != LCE_REDUCTION_NONE) {
+    const float scale = reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f;
+    hipLaunchKernelGGL(lce_reduce_sum_kernel, dim3(1), dim3(1024), 0, st, lp_tok, T, scale, logprobs);
+    rc = check_launch("lce_reduce_sum_kernel");
+  }
+  return rc;
+}
+
 template <typename Cfg>
 int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TIN* W, int64_t ldw, const int64_t* labels,
                  int64_t T, int64_t H, int64_t V, float temperature, int reduction, float* logprobs, float* entropy,
@@ -304,7 +346,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   p.split_span = rows_per_split ? rows_per_split : V;
   p.label_offset = label_offset;
   // xcache: the raw logits are kept for the backward
-  p.xcache = xcache;
+  p.xcache = xcache; p.w_plane = p.h_plane = 0;
   p.map = TileMap::make(ntt, S, br, 1);
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   int rc;
@@ -325,40 +367,8 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
     rc = check_launch("lce_fwd_kernel");
   }
   if (rc) return rc;
-  if (shard_out) {
-    ProfScope prof(PC_FWD_MERGE, st);
-    f32x4_t* out = reinterpret_cast<f32x4_t*>(shard_out);
-    if (S >= 64)
-      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<64>, dim3((unsigned)((T * 64 + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S,
-                         T, p.c, 1.0f / temperature, out);
-    else if (S >= 8)
-      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<8>, dim3((unsigned)((T * 8 + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S, T,
-                         p.c, 1.0f / temperature, out);
-    else
-      hipLaunchKernelGGL(lce_fwd_shard_merge_kernel<1>, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S, T,
-                         p.c, 1.0f / temperature, out);
-    return check_launch("lce_fwd_shard_merge_kernel");
-  }
-  {
-    ProfScope prof(PC_FWD_MERGE, st);
-    if (S >= 64)
-      hipLaunchKernelGGL(lce_fwd_merge_kernel<64>, dim3((unsigned)((T * 64 + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S, T,
-                         p.c, 1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
-    else if (S >= 8)
-      hipLaunchKernelGGL(lce_fwd_merge_kernel<8>, dim3((unsigned)((T * 8 + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S, T,
-                         p.c, 1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
-    else
-      hipLaunchKernelGGL(lce_fwd_merge_kernel<1>, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, st, p.parts, p.xlabel, labels, label_offset, V, S, T, p.c,
-                         1.0f / temperature, lp_tok, entropy, maximum, accumulate, entropy_b);
-    rc = check_launch("lce_fwd_merge_kernel");
-  }
-  if (rc) return rc;
-  if (reduction != LCE_REDUCTION_NONE) {
-    const float scale = reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f;
-    hipLaunchKernelGGL(lce_reduce_sum_kernel, dim3(1), dim3(1024), 0, st, lp_tok, T, scale, logprobs);
-    rc = check_launch("lce_reduce_sum_kernel");
-  }
-  return rc;
+  return forward_merge(p.parts, p.xlabel, labels, label_offset, V, S, T, p.c, temperature, reduction, lp_tok, logprobs, entropy, maximum, accumulate,
+                       entropy_b, shard_out, st);
 }
 
 // upper bound of the number of vocabulary splits forward_impl picks, over the token-tile widths in use
@@ -733,7 +743,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       d.g_lp = dlogprobs; d.g_lp_stride = reduction == LCE_REDUCTION_NONE ? 1 : 0;
       d.g_lp_scale = reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f;
       d.g_ent = dentropy;
-      d.dS = dS[c & 1]; d.ldS = L.ldS; d.pcol = L.pcol; d.dST = L.tn ? nullptr : dST[c & 1]; d.ldST = L.ldST; d.tpad = L.tpad;
+      d.dS = dS[c & 1]; d.ldS = L.ldS; d.pcol = L.pcol; d.w_plane = d.h_plane = d.dS_plane = 0; d.dST = L.tn ? nullptr : dST[c & 1]; d.ldST = L.ldST; d.tpad = L.tpad;
       d.rows = rows; d.n_rows = n_rows;
       d.label_outside = lt.labels != nullptr ? tu.label_outside : 0;
       d.tokc = tokc; d.tokl = tokl; d.lab0 = v0;

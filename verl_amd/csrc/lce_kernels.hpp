@@ -56,6 +56,7 @@ struct FwdArgs {
   // When not null (offered while the tokens are at most half the hidden size), the raw logits h . W[v] (fp32, before the division by the
   // temperature) are kept for the backward: logit (t, v) at kept_logit(xcache, T, t, v).
   float* xcache;
+  int64_t w_plane, h_plane;  // W and h in bfloat16 planes (GemmCfg16, TERMS == 6): bytes from plane to plane
 };
 
 // Kept logits lie in panels of 16 vocabulary rows, [panel][token][16] fp32: what one 16 x 16 block of a tile holds is one
@@ -356,6 +357,7 @@ struct DsArgs {
   const float* g_ent;   // [T] or null
   TIN* dS;              // token-major; entry (t, u) at ds_at(dS, ldS, pcol, t, u)
   int64_t ldS, pcol;
+  int64_t w_plane, h_plane, dS_plane;  // everything in bfloat16 planes (GemmCfg16, TERMS == 6): bytes, for dS elements
   TIN* dST;             // [vchunk][ldST] (vocab-major); null when the d_weight GEMM reads dS with transposing LDS reads
   int64_t ldST;
   int64_t tpad;         // tokens rounded up to the GEMM K granule: columns [T, tpad) of dST / rows [T, tpad) of dS are written as zeros
@@ -645,6 +647,7 @@ struct GemmArgs {
   int64_t lda;
   const TIN* B;
   int64_t ldb;
+  int64_t a_plane, b_plane;  // A and B in bfloat16 planes (GemmCfg16, TERMS == 6): bytes from plane to plane
   int64_t a_pcol;  // A lies in panels of 64 columns (see ds_at; lda = 64): elements from panel to panel; 0: rows of lda elements
   int64_t M, N, K;
   float* Cf;

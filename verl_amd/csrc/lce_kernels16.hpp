@@ -12,8 +12,8 @@ namespace lce {
 // vocabulary rows (one wave tile) the entries are ordered so that what a lane holds of two neighbouring blocks is one
 // 16-byte run and the four lane groups follow each other (64 contiguous bytes per token and store instruction):
 // row v = 16 i + 4 g + r  ->  position 32 (i / 2) + 8 g + 4 (i % 2) + r.  Tokens keep their order.
-template <typename TIN, int TR, int NBN, int AE>
-struct KPerm<GemmCfg16<TIN, TR, NBN, AE>> {
+template <typename TIN, int TR, int NBN, int AE, int TERMS>
+struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS>> {
   static constexpr int GT = 128, GV = 128;
   static __host__ __device__ __forceinline__ int64_t token(int64_t t) { return t; }
   static __host__ __device__ __forceinline__ int64_t token_at(int64_t u) { return u; }
@@ -99,6 +99,8 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
   GemmCore16<Cfg> g;
   g.set_lane();
+  g.a_plane = p.w_plane;
+  g.b_plane = p.h_plane;
 
   float m[NBN], a[NBN], b[NBN];
   int lab[NBN];
@@ -263,7 +265,20 @@ LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&a
         }
       }
       // rows of positions without a token are zeros (their constants make them so); they pad the d_weight GEMM's K
-      if (tok < p.tpad) store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + ip * 32 + g4 * 8), d);
+      TIN* dst = ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + ip * 32 + g4 * 8);
+      if constexpr (Cfg::TERMS == 6) {
+        float rest[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) rest[q] = d[q];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          if (tok < p.tpad) store_run<TIN, 8>(dst + t * p.dS_plane, rest);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) rest[q] -= (float)(TIN)rest[q];
+        }
+      } else {
+        if (tok < p.tpad) store_run<TIN, 8>(dst, d);
+      }
     }
   }
 }
@@ -295,6 +310,8 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
       lab[j] = p.tokl[pos];
     }
   }
+  g.a_plane = p.w_plane;
+  g.b_plane = p.h_plane;
   g.init(p.W, p.ldw, (int64_t)vt * Cfg::BM, p.vrows, p.h, p.ldh, n0, Tc, p.rows);
   f32x4_t acc[NB][NBN];
   g.run(lds, p.H, acc);
@@ -409,6 +426,8 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
   f32x4_t acc[Cfg::NB][Cfg::NBN];
   if (k0 < k1 && (CoreCfg::TRANS != 2 || k0 < p.b_rows_valid)) {
     // MFMA rows = n, MFMA columns = m
+    g.a_plane = p.b_plane;
+    g.b_plane = p.a_plane;
     if constexpr (CoreCfg::TRANS == 2)
       g.init_mixed(p.B + k0 * p.ldb, p.ldb, n0, p.N - n0, p.b_rows_valid - k0, [](int r) { return KPerm<Cfg>::vocab_at(r); },
                    p.a_pcol ? p.A + (k0 >> 6) * p.a_pcol : p.A + k0, p.lda, m0, p.M, p.a_pcol ? p.a_pcol * 2 : (int64_t)Cfg::BKB);
@@ -454,6 +473,8 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
   GemmCore16<Cfg> g;
   f32x4_t acc[Cfg::NB][Cfg::NB];
   if (p.K > 0) {
+    g.a_plane = p.b_plane;
+    g.b_plane = p.a_plane;
     g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);  // MFMA rows = n, MFMA columns = m
     g.run(lds, p.K, acc);
   } else {
@@ -611,6 +632,33 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   Core::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
 }
 
+// fp32 rows as three bfloat16 planes, out[r] = three runs of ldo elements: x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 -
+// x2); the differences are exact, so x1 + x2 + x3 = x down to the smallest bfloat16.  Row r is in[rows[r]] (in[r] without
+// `rows`) for r < R = *n_rows (R without), zeros up to the next multiple of 64.  Eight elements per thread; C a multiple of 8.
+inline __global__ void split_planes_kernel(const float* in, int64_t ldi, int64_t R, int64_t C, bf16_t* out, int64_t ldo, int64_t rpad, const int* rows,
+                                           const int* n_rows) {
+  if (n_rows) R = *n_rows;
+  const int64_t rend = (R + 63) / 64 * 64 < rpad ? (R + 63) / 64 * 64 : rpad;
+  const int64_t per_row = C / 8, n = rend * per_row;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = q / per_row, c = (q - r * per_row) * 8;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (r < R) {
+      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(in + (rows ? (int64_t)rows[r] : r) * ldi + c);
+      const f32x4_t lo = src[0], hi = src[1];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = e < 4 ? lo[e & 3] : hi[e & 3];
+    }
+    bf16_t* dst = out + r * 3 * ldo + c;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      store_run<bf16_t, 8>(dst + t * ldo, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] -= (float)(bf16_t)x[e];
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------
 // kernels
 // ------------------------------------------------------------------------------------------------
@@ -641,9 +689,9 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typena
 
 template <typename Cfg>
 LCE_DEV void any_gemm16_tile(const GemmArgs<typename Cfg::TIN>& p, int bid, char* lds) {
-  if (p.tn == 1) gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1>, Cfg>(p, bid, lds);
+  if (p.tn == 1) gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1, 8, 0, Cfg::TERMS>, Cfg>(p, bid, lds);
   // (W early: the whole step 0.2 to 0.5 % faster from 2048 to 16384 tokens)
-  else if (p.tn == 2) gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, 8, 1>>(p, bid, lds);
+  else if (p.tn == 2) gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, 8, 1, Cfg::TERMS>>(p, bid, lds);
   else gemm16_tile<Cfg>(p, bid, lds);
 }
 

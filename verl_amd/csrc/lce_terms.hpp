@@ -1,0 +1,260 @@
+// fp32 inputs on the bfloat16 matrix pipe: every operand is held as three bfloat16 planes whose sum it is, and a K slab is
+// multiplied as six products of planes (GemmCfg16, TERMS == 6).  The fp32 MFMA runs at 157 TFLOP/s dense, the bfloat16 one
+// at 2.5 PFLOP/s; six products for one leave 2.5 times the rate at the clocks both reach, against which stand the passes
+// that make the planes (10 bytes per element of W, forward and backward each).  Measured, fp32 MFMA / planes: H=896,
+// V=151936, 1024 tokens forward + backward 9.90 / 6.39 ms, 2000 tokens forward 4.11 / 2.68, 400 tokens forward 1.09 / 0.90;
+// H=5120, 1500 tokens, half with gradient 56.6 / 36.1.  Error against float64 (2-norm, relative; H=896, V=151936, 2000 tokens):
+// log-probs 7.7e-8 / 7.2e-8, entropies 5.9e-8 / 5.6e-8, d_hidden 1.0e-6 / 5.9e-7, d_weight 7.9e-7 / 4.1e-7: the products are
+// exact and a sixteenth as many partial sums are rounded.
+#pragma once
+#include "lce_host.hpp"
+
+namespace {
+
+// ---- forward ----------------------------------------------------------------------------------
+// The weight is split and multiplied chunk by chunk: a chunk holds whole rounds of tiles over the CUs (as many as 256 MB of
+// planes allow), and its splits are a block of their own in the list of partial statistics.
+struct TermsFwdPlan {
+  int64_t rows;     // vocabulary rows of a chunk
+  int nchunks, splits;  // splits: of all chunks together
+  size_t off_xlabel, off_lp, off_h, off_w, total;
+};
+
+int terms_fwd_splits(int ntt, int64_t rows) { return forward_splits_256(ntt, (int)((rows + 255) / 256)); }
+
+TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V) {
+  TermsFwdPlan p;
+  const int ntt = (int)((T + 255) / 256);
+  const int64_t most = std::max<int64_t>(1, ((int64_t)256 << 20) / (6 * H * 256));  // tiles of a chunk
+  int64_t tiles = most;
+  for (int64_t r = most * ntt / kNumCUs; r >= 1; --r)
+    if (r * kNumCUs / ntt >= 1) { tiles = r * kNumCUs / ntt; break; }
+  p.rows = tiles * 256;
+  p.nchunks = (int)((V + p.rows - 1) / p.rows);
+  p.splits = 0;
+  for (int c = 0; c < p.nchunks; ++c) {
+    const int64_t rows = std::min<int64_t>(p.rows, V - c * p.rows);
+    p.splits += std::min<int>(terms_fwd_splits(ntt, rows), (int)((rows + 255) / 256));
+  }
+  size_t o = align256((size_t)p.splits * T * 16);
+  p.off_xlabel = o; o += align256((size_t)T * 4);
+  p.off_lp = o;     o += align256((size_t)T * 4);
+  p.off_h = o;      o += align256((size_t)round_up(T, 64) * 3 * H * 2);
+  p.off_w = o;      o += align256((size_t)std::min<int64_t>(p.rows, round_up(V, 64)) * 3 * H * 2);
+  p.total = o;
+  return p;
+}
+
+// ---- backward ---------------------------------------------------------------------------------
+struct TermsBwdLayout {
+  int64_t vchunk, tpad, pcol, plane, ldH;  // plane: elements from plane to plane of a d_logits panel
+  size_t off_dS[2], off_W[2], off_H, off_dHacc, off_rows, off_inv, off_nrows, off_acounts, off_tokc, off_tokl, total;
+  int nchunks, ksplit;
+};
+
+TermsBwdLayout terms_bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
+  TermsBwdLayout L;
+  L.vchunk = std::min(round_up(vchunk, 256), round_up(V, 256));
+  L.nchunks = (int)((V + L.vchunk - 1) / L.vchunk);
+  L.ksplit = tu.dh_ksplit > 0 ? tu.dh_ksplit : dh_ksplit(T, H, L.vchunk);
+  L.tpad = round_up(T, 128);
+  L.plane = L.tpad * 64;
+  L.pcol = 3 * L.plane + 64;
+  L.ldH = round_up(H, 256) + 64;
+  size_t o = 0;
+  for (int b = 0; b < 2; ++b) {
+    L.off_dS[b] = o; o += (b == 0 || L.nchunks > 1) ? align256((size_t)(L.vchunk / 64) * L.pcol * 2) : 0;
+    L.off_W[b] = o;  o += (b == 0 || L.nchunks > 1) ? align256((size_t)L.vchunk * 3 * H * 2) : 0;
+  }
+  L.off_H = o;       o += align256((size_t)L.tpad * 3 * L.ldH * 2);
+  L.off_dHacc = o;   o += (size_t)L.ksplit * align256((size_t)T * H * 4);
+  L.off_rows = o;    o += align256((size_t)L.tpad * 4);
+  L.off_inv = o;     o += align256((size_t)T * 4);
+  L.off_nrows = o;   o += 256;
+  L.off_acounts = o; o += align256((size_t)((T + kActiveBlock - 1) / kActiveBlock) * 4);
+  L.off_tokc = o;    o += align256((size_t)L.tpad * 16);
+  L.off_tokl = o;    o += align256((size_t)L.tpad * 4);
+  L.total = o;
+  return L;
+}
+
+// chunk width by the same bound as bwd_layout's (a quarter of one [T, V] plus one fp32 [V, H]); within it a chunk's d_logits
+// planes stay within 256 MB
+TermsBwdLayout terms_bwd_layout(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
+  if (vchunk <= 0) {
+    double gate = (double)T * V + 4.0 * (double)V * H;
+    if (tu.ws_budget > 0 && (double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
+    vchunk = std::min(round_up(V, 256), std::max<int64_t>(2048, (((int64_t)256 << 20) / (6 * T)) / 256 * 256));
+    while (vchunk > 2048 && (double)terms_bwd_layout_for(tu, T, H, V, vchunk).total + 512.0 > gate) vchunk -= 1024;
+    if (vchunk < 2048) vchunk = 2048;
+    const int64_t n = (V + vchunk - 1) / vchunk;
+    vchunk = round_up((V + n - 1) / n, 256);
+  }
+  return terms_bwd_layout_for(tu, T, H, V, vchunk);
+}
+
+// ---- which calls ------------------------------------------------------------------------------
+// ONE rule for forward and backward: the backward recomputes the logits, and where a token's distribution is peaked the
+// rounding errors of a logit and of the forward's statistics cancel only if both come from the same arithmetic (2048
+// tokens x 1024 x 8192, temperature 0.6, worst error of d_hidden relative to its largest entry: 4.7e-6 with the fp32 MFMA
+// both ways, 1.3e-5 with the planes in the forward only).  Where the workspace bound has no room for the planes (small
+// vocabularies), both take the fp32 tiles.
+constexpr int64_t kTermsMinTokens = 256;
+bool use_terms(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype) {
+  if (dtype != LCE_DTYPE_F32 || tu.variant_forced || T < kTermsMinTokens || H % 64 != 0) return false;
+  double gate = (double)T * V + 4.0 * (double)V * H;
+  if (tu.ws_budget > 0 && (double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
+  return (double)terms_bwd_layout(tu, T, H, V, 0).total + 512.0 <= gate;
+}
+
+#if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1
+typedef GemmCfg16<bf16_t, 0, 8, 0, 6> TermsCfg;
+
+int launch_split(const float* in, int64_t ld, int64_t R, int64_t C, bf16_t* out, int64_t ldo, int64_t rpad, const int* rows, const int* n_rows,
+                 hipStream_t st) {
+  ProfScope prof(PC_TRANSPOSE, st);
+  const int64_t blocks = (rpad * (C / 8) + 255) / 256;
+  hipLaunchKernelGGL(split_planes_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, in, ld, R, C, out, ldo, rpad, rows, n_rows);
+  return check_launch("split_planes_kernel");
+}
+
+int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
+                  int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, hipStream_t st,
+                  int64_t label_offset, float* shard_out) {
+  const TermsFwdPlan pl = terms_fwd_plan(T, H, V);
+  bf16_t* h3 = reinterpret_cast<bf16_t*>(ws + pl.off_h);
+  bf16_t* w3 = reinterpret_cast<bf16_t*>(ws + pl.off_w);
+  int rc = launch_split(h, ldh, T, H, h3, H, round_up(T, 64), nullptr, nullptr, st);
+  if (rc) return rc;
+  const int ntt = (int)((T + 255) / 256);
+  FwdArgs<bf16_t> p;
+  p.W = w3; p.ldw = 3 * H; p.h = h3; p.ldh = 3 * H; p.labels = labels; p.T = T; p.H = H;
+  p.w_plane = p.h_plane = H * 2;
+  p.c = kLog2e / temperature;
+  p.xlabel = reinterpret_cast<float*>(ws + pl.off_xlabel);
+  p.xcache = nullptr;
+  f32x4_t* parts = reinterpret_cast<f32x4_t*>(ws);
+  int done = 0;
+  for (int c = 0; c < pl.nchunks; ++c) {
+    const int64_t v0 = c * pl.rows, rows = std::min(pl.rows, V - v0);
+    if ((rc = launch_split(W + v0 * ldw, ldw, rows, H, w3, H, rows, nullptr, nullptr, st))) return rc;
+    p.S = std::min<int>(terms_fwd_splits(ntt, rows), (int)((rows + 255) / 256));
+    p.V = rows;
+    p.label_offset = label_offset + v0;
+    p.parts = parts + (int64_t)done * T;
+    p.split_stride = TermsCfg::BM; p.tile_step = (int64_t)p.S * TermsCfg::BM; p.split_span = rows;
+    p.map = TileMap::make(ntt, p.S, block_rows(ntt), 1);
+    ProfScope prof(PC_FWD, st);
+    allow_lds((lce_fwd16_kernel<TermsCfg, false>), TermsCfg::LDS_BYTES);
+    hipLaunchKernelGGL((lce_fwd16_kernel<TermsCfg, false>), dim3(p.map.total), dim3(TermsCfg::NTHREADS), TermsCfg::LDS_BYTES, st, p);
+    if ((rc = check_launch("lce_fwd16_kernel"))) return rc;
+    done += p.S;
+  }
+  float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + pl.off_lp);
+  return forward_merge(parts, p.xlabel, labels, label_offset, V, done, T, p.c, temperature, reduction, lp_tok, logprobs, entropy, maximum, accumulate,
+                       entropy_b, shard_out, st);
+}
+
+int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
+                   int reduction, const float* maximum, const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
+                   float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu) {
+  typedef TermsCfg Cfg;
+  const bool need_dh = d_hidden != nullptr, need_dw = d_weight != nullptr;
+  const TermsBwdLayout L = terms_bwd_layout(tu, T, H, V, vchunk);
+  bf16_t* dS[2] = {reinterpret_cast<bf16_t*>(ws + L.off_dS[0]), reinterpret_cast<bf16_t*>(ws + L.off_dS[1])};
+  bf16_t* w3[2] = {reinterpret_cast<bf16_t*>(ws + L.off_W[0]), reinterpret_cast<bf16_t*>(ws + L.off_W[1])};
+  bf16_t* h3 = reinterpret_cast<bf16_t*>(ws + L.off_H);
+  float* dHacc = reinterpret_cast<float*>(ws + L.off_dHacc);
+  int* rows = reinterpret_cast<int*>(ws + L.off_rows);
+  int* inv = reinterpret_cast<int*>(ws + L.off_inv);
+  int* n_rows = reinterpret_cast<int*>(ws + L.off_nrows);
+  f32x4_t* tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
+  int* tokl = reinterpret_cast<int*>(ws + L.off_tokl);
+  const int64_t g_stride = reduction == LCE_REDUCTION_NONE ? 1 : 0;
+  const float g_scale = reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f;
+  int rc;
+  {
+    ProfScope prof(PC_ACTIVE_ROWS, st);
+    int* acounts = reinterpret_cast<int*>(ws + L.off_acounts);
+    const unsigned nblk = (unsigned)((T + kActiveBlock - 1) / kActiveBlock);
+    hipLaunchKernelGGL(active_count_kernel, dim3(nblk), dim3(256), 0, st, dlogprobs, g_stride, dentropy, T, acounts);
+    if ((rc = check_launch("active_count_kernel"))) return rc;
+    hipLaunchKernelGGL(active_rows_kernel, dim3(nblk), dim3(256), 0, st, dlogprobs, g_stride, dentropy, T, acounts, rows, inv, n_rows);
+    if ((rc = check_launch("active_rows_kernel"))) return rc;
+    hipLaunchKernelGGL(ds_token_consts_kernel, dim3((unsigned)((L.tpad + 255) / 256)), dim3(256), 0, st, rows, n_rows, T, L.tpad, dlogprobs, g_stride,
+                       g_scale, dentropy, maximum, accumulate, entropy_b, labels, vocab_offset, V, 1.0f / temperature, tokc, tokl);
+    if ((rc = check_launch("ds_token_consts_kernel"))) return rc;
+  }
+  if ((rc = launch_split(h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows, st))) return rc;
+  const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN);
+  // launch c: d_logits of chunk c and the gradient GEMMs of chunk c - 1, as in backward_impl
+  for (int c = 0; c <= L.nchunks; ++c) {
+    BwdChunkArgs<bf16_t> p;
+    p.n_gw = p.n_gh = p.n_ds = 0;
+    if (c < L.nchunks) {
+      const int64_t v0 = (int64_t)c * L.vchunk, vrows = std::min(L.vchunk, V - v0);
+      // (the last reader of this buffer, d_hidden of chunk c - 2, ran in the launch before the last)
+      if ((rc = launch_split(W + v0 * ldw, ldw, vrows, H, w3[c & 1], H, vrows, nullptr, nullptr, st))) return rc;
+      DsArgs<bf16_t>& d = p.ds;
+      d.W = w3[c & 1]; d.ldw = 3 * H; d.h = h3; d.ldh = 3 * L.ldH; d.labels = labels; d.T = T; d.H = H;
+      d.w_plane = H * 2; d.h_plane = L.ldH * 2; d.dS_plane = L.plane;
+      d.v0 = vocab_offset + v0; d.vrows = vrows; d.rcp_tau = 1.0f / temperature; d.c = kLog2e / temperature;
+      d.maximum = maximum; d.accumulate = accumulate; d.entropy_b = entropy_b;
+      d.g_lp = dlogprobs; d.g_lp_stride = g_stride; d.g_lp_scale = g_scale; d.g_ent = dentropy;
+      d.dS = dS[c & 1]; d.ldS = 64; d.pcol = L.pcol; d.dST = nullptr; d.ldST = 0; d.tpad = L.tpad;
+      d.rows = nullptr; d.n_rows = n_rows; d.label_outside = 0;
+      d.tokc = tokc; d.tokl = tokl; d.lab0 = v0; d.range_rows = 0;
+      d.map = TileMap::make(ntt, (int)((vrows + Cfg::BM - 1) / Cfg::BM), block_rows(ntt), 0);
+      p.n_ds = d.map.total;
+    }
+    if (c > 0) {
+      const int cc = c - 1;
+      const int64_t v0 = (int64_t)cc * L.vchunk, vrows = std::min(L.vchunk, V - v0);
+      const int64_t kc = round_up(vrows, KPerm<Cfg>::GV);
+      if (need_dh) {
+        p.gh = make_gemm_args<Cfg>(dS[cc & 1], 64, w3[cc & 1], 3 * H, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1);
+        p.gh.tn = 2; p.gh.b_rows_valid = vrows; p.gh.m_dev = n_rows;
+        p.gh.a_pcol = L.pcol; p.gh.a_plane = L.plane * 2; p.gh.b_plane = H * 2;
+        if (L.ksplit > 1) {
+          p.gh.ksplit = L.ksplit;
+          p.gh.kslice = round_up((kc + L.ksplit - 1) / L.ksplit, Cfg::BK);
+          p.gh.map = TileMap::make(p.gh.map.nrow_tiles, p.gh.n_tiles * L.ksplit, p.gh.map.br, p.gh.map.rows_fastest);
+          p.gh.cf_split_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
+        }
+        p.n_gh = p.gh.map.total;
+      }
+      if (need_dw) {
+        p.gw = make_gemm_args<Cfg>(dS[cc & 1], 64, h3, 3 * L.ldH, vrows, H, round_up(T, 64), d_weight + v0 * H, H, nullptr, 0, 0);
+        p.gw.tn = 1; p.gw.perm_rows = 1; p.gw.k_dev = n_rows; p.gw.k_gran = 64;
+        p.gw.a_pcol = L.pcol; p.gw.a_plane = L.plane * 2; p.gw.b_plane = L.ldH * 2;
+        p.n_gw = p.gw.map.total;
+      }
+      if (p.n_gh && p.n_gw && p.gh.kslice > p.gw.K) {  // longer tiles go first
+        std::swap(p.gh, p.gw);
+        std::swap(p.n_gh, p.n_gw);
+      } else if (!p.n_gw) {
+        p.gw = p.gh;
+        p.n_gw = p.n_gh;
+        p.n_gh = 0;
+      }
+    }
+    ProfScope prof(PC_BWD_CHUNK, st);
+    allow_lds(lce_bwd_chunk16_kernel<Cfg>, Cfg::LDS_BYTES);
+    hipLaunchKernelGGL(lce_bwd_chunk16_kernel<Cfg>, dim3(p.n_gw + p.n_gh + p.n_ds), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
+    if ((rc = check_launch("lce_bwd_chunk16_kernel"))) return rc;
+  }
+  if (need_dh) {
+    ProfScope prof(PC_DH_FINISH, st);
+    LabelTerm lt;
+    lt.labels = nullptr; lt.v0 = vocab_offset; lt.V = V; lt.g_lp = dlogprobs; lt.g_stride = g_stride; lt.scale = 0.f;
+    int64_t blocks = (T * (H / 4) + 255) / 256;
+    if (blocks > 8192) blocks = 8192;
+    hipLaunchKernelGGL((dh_finish_kernel<float, float>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit,
+                       (int64_t)(align256((size_t)T * H * 4) / 4), inv, T, H, d_hidden, lt, W, ldw);
+    if ((rc = check_launch("dh_finish_kernel"))) return rc;
+  }
+  return LCE_OK;
+}
+#endif
+
+}  // namespace
