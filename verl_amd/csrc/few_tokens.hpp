@@ -1,20 +1,16 @@
-// Gradient GEMMs of a backward with few tokens (at most 128), and d_logits from kept logits; 16-bit inputs, gfx950.
+// Few tokens (at most 128; 16-bit inputs, gfx950): the forward up to 64, the gradient GEMMs, and d_logits from kept logits.
 //
-// With T <= 128 both products are one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
-//   d_weight[v][h] = sum_t dS[t][v] * hidden[t][h]      writes [V, H] once; its operands (dS, hidden) are small
+// With T <= 128 every product is one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
+//   logits      W[v] . hidden[t]                        reads W once; nothing is written (or the kept logits)
 //   d_hidden[t][h] = sum_v dS[t][v] * W[v][h]           reads W once; its result is small
+//   d_weight[v][h] = sum_t dS[t][v] * hidden[t][h]      writes [V, H] once; its operands (dS, hidden) are small
 // The 256 x 256 tiles of the general path spend such a pass waiting: a d_weight tile has a K loop of one or two slabs
 // between a cold start and 128 KB of scattered 2-byte stores, and a d_hidden tile keeps two half slabs of W in flight
-// per CU.  The kernels here are shaped for the stream instead:
-//   * several small workgroups per CU (40-80 KB of LDS, <= 168 registers), so that one workgroup's loads overlap
-//     another's MFMAs and stores without a hand-built ring; the next operand tile travels global -> registers while
-//     the current one is multiplied, and is written to LDS after it;
-//   * d_weight: one workgroup owns 64 vocabulary rows and walks all of H, so dS is fetched once per row block and
-//     every store instruction writes 16 rows x 64 contiguous bytes;
-//   * d_hidden: the vocabulary is cut into as many K slices as fill the chip twice over (fp32 partials, summed in a
-//     fixed order afterwards), and W is read as it lies in memory.
-// Both take their K-major operand (hidden[t][.], dS[t][.], W[v][.]) through the transposing LDS read
-// ds_read_b64_tr_b16.  Everything is plain HIP with compiler-placed waits.
+// per CU.  The kernels here are shaped for the stream instead: workgroups that stay, operands of the next stages on their way
+// in registers, and loops without a branch around a load or a store, so that no wait is longer than it has to be.  Reading and
+// writing are separate launches: this card reads 1.09 GB in 155 us and writes it in 185, and takes 340 for the two in a row
+// but 400 to 500 for both at once.  Everything is plain HIP with compiler-placed waits; K-major operands (hidden[t][.],
+// dS[t][.], W[v][.] in the gradients) are read through the transposing LDS read ds_read_b64_tr_b16.
 #pragma once
 #include "gemm_core.hpp"
 #include "lce_kernels.hpp"
@@ -54,6 +50,170 @@ LCE_DEV void mma16(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
 // into different banks (values below 16: valid for rows of 16 chunks and of 32)
 LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 
+// Buffer access to a run of memory: out-of-bounds lanes read zero and store nothing, so the loops below need no branch around
+// a load or a store, and the compiler can wait for exactly the operation it needs (behind a branch it does not know how many
+// younger ones are in flight and waits for all of them).
+typedef __amdgpu_buffer_rsrc_t buf_t;
+// (bytes below 4 GiB: 256 rows of an operand span less)
+LCE_DEV buf_t make_buf(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+constexpr int kBufNowhere = (int)0x80000000u;  // an offset beyond any of these buffers (at most 64 rows of 16 MiB)
+constexpr int kBufNonTemporal = 2;
+
+// ------------------------------------------------------------------------------------------------------------------
+// Forward, up to 64 tokens.  Workgroup = 512 threads = 8 waves, one per CU; it owns a contiguous range of vocabulary rows (the
+// same number for every workgroup) and goes through it in passes of 256 rows, for each of which K is streamed in stages of 64:
+// 256 rows of W x 128 bytes and 64 rows of hidden x 128 bytes.  What bounds it is the read of W, and that by the bytes in
+// flight: DEPTH stages are on their way in registers (128 KB of W per CU) while one is multiplied out of LDS, which holds two,
+// so that a stage costs one barrier; and the stages of the next pass follow those of this one without a gap.
+// The products are those of the d_logits tiles, 32x32x16 blocks with k ascending (rows: vocabulary, columns: tokens), so logits
+// kept here have the bits that a backward without them recomputes.  A wave owns 32 rows x 64 tokens; in a short last pass the
+// waves without rows stand aside (64 tokens: 182 -> 174 us).
+// Measured, kernel and merge, against the 256 x 64 tile with a ring of whole LDS stages (H, V: before -> after): 64 tokens,
+// 3584, 152064: 184 -> 174 us; 4096, 128256: 175 -> 160; 896, 151936: 58 -> 51.5; the same access pattern without any
+// arithmetic takes 170, 163 and 41.  (128 tokens on 64 x 64 wave tiles: 223 us, the 256 x 128 tile takes 213.)
+// ------------------------------------------------------------------------------------------------------------------
+struct FewFwdShape {
+  static constexpr int NT = 64, DEPTH = 4, BM = 256, FN = 2;
+  static constexpr int STAGE = BM * 128 + NT * 128;
+  static constexpr int LDS_BYTES = 2 * STAGE + 8 * 4096;  // two stages, a store tile per wave
+};
+
+template <typename TIN>
+__global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  typedef FewFwdShape S;
+  constexpr int DEPTH = S::DEPTH, FN = S::FN, NT = S::NT;
+  constexpr int WL = S::BM / 64;  // 16-byte chunks of a W stage per thread: row tid / 8 + 64 i, chunk tid % 8 (hidden: one)
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  const int64_t row0 = (int64_t)blockIdx.x * p.split_stride;
+  const int64_t vend64 = row0 + p.split_span < p.V ? row0 + p.split_span : p.V;
+  const int vend = (int)vend64;
+  const int n_k = (int)(p.H / 64), n_kp = (n_k + DEPTH - 1) / DEPTH * DEPTH;  // stages of a pass, rounded up to turns of the loop
+
+  float m[FN], a[FN], b[FN];
+  int lab[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    m[j] = kNegBig;
+    a[j] = 0.f;
+    b[j] = 0.f;
+    const int64_t t = j * 32 + ln;
+    const int64_t y = t < p.T ? p.labels[t] - p.label_offset : -1;
+    lab[j] = (y >= 0 && y < p.V) ? (int)y : -1;
+  }
+
+  // rows beyond the range, tokens beyond T and stages beyond K read as zero
+  const uint32_t w_row = (uint32_t)(p.ldw * sizeof(TIN)), h_row = (uint32_t)(p.ldh * sizeof(TIN));
+  const uint32_t w_at = (uint32_t)(tid >> 3) * w_row + (tid & 7) * 16, h_at = (uint32_t)(tid >> 3) * h_row + (tid & 7) * 16;
+  u32x4_t pw[DEPTH][WL], pb[DEPTH];
+  int64_t f_row = row0;  // the next stage to fetch: first row of its pass, k
+  int f_k = 0;
+  auto fetch = [&](u32x4_t (&w)[WL], u32x4_t& x) {
+    const int64_t left = vend64 - f_row < S::BM ? vend64 - f_row : S::BM;
+    const bool live = f_k < n_k && left > 0;
+    const buf_t wb = make_buf(p.W + f_row * p.ldw + 64 * (int64_t)f_k, live ? left * w_row - 128 * (int64_t)f_k : 0);
+    const buf_t hb = make_buf(p.h + 64 * (int64_t)f_k, live ? p.T * h_row - 128 * (int64_t)f_k : 0);
+#pragma unroll
+    for (int i = 0; i < WL; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(wb, (int)(w_at + 64 * i * w_row), 0, kBufNonTemporal);
+    x = __builtin_amdgcn_raw_buffer_load_b128(hb, (int)h_at, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // (the loads of one stage stay in front of the next one's)
+    if (++f_k == n_kp) {
+      f_k = 0;
+      f_row += S::BM;
+    }
+  };
+  // chunk c of row r lies at c ^ swz(r); rows 32 apart share the pattern
+  auto swz = [](int r) { return (r ^ ((r >> 3) & 1)) & 7; };
+  const int put = (tid >> 3) * 128 + (((tid & 7) ^ swz(tid >> 3)) * 16);
+  const int a_rd = (wave * 32 + ln) * 128, b_rd = S::BM * 128 + ln * 128, sw = swz(ln);
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) fetch(pw[d], pb[d]);
+  int buf = 0;
+  for (int64_t m0 = row0; m0 < vend64; m0 += S::BM) {
+    f32x16_t acc[1][FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
+    const int vbase = (int)m0 + wave * 32;  // this wave's first row
+    const bool busy = vbase < vend;         // (a short last pass leaves the LDS to the waves that have rows)
+    for (int k0 = 0; k0 < n_kp; k0 += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        char* st = lds + buf * S::STAGE;
+        buf ^= 1;
+#pragma unroll
+        for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4_t*>(st + put + i * 8192) = pw[d][i];
+        *reinterpret_cast<u32x4_t*>(st + S::BM * 128 + put) = pb[d];
+        fetch(pw[d], pb[d]);
+        // (a buffer is written again two stages on: every wave has passed the barrier between, after its reads of this stage)
+        __syncthreads();
+        if (busy) {
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) {
+            const int c = ((2 * kk + hh) ^ sw) * 16;
+            const u32x4_t af = *reinterpret_cast<const u32x4_t*>(st + a_rd + c);
+            u32x4_t bf[FN];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const u32x4_t*>(st + b_rd + j * 4096 + c);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) Mma<TIN>::run(acc[0][j], af, bf[j]);
+          }
+        }
+      }
+    }
+    if (p.xcache) {
+      // the logits of this pass, for a backward that then has no need to recompute them.  A 32x32 block passes through 4 KB of
+      // LDS of this wave's own and leaves it as whole lines, 1 KB (16 tokens x 16 rows of a panel) per store; rows in whole
+      // fours, the last ones of W up to the end of the cache's panel.
+      char* sC = lds + 2 * S::STAGE + wave * 4096;
+      const int p4 = lane & 3, pt = lane >> 2;  // as it leaves: quad of rows, token
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int c = 2 * (q & 1) + hh;
+          *reinterpret_cast<f32x4_t*>(sC + (q >> 1) * 2048 + ln * 64 + ((c ^ ((ln >> 1) & 3)) * 16)) =
+              f32x4_t{acc[0][j][4 * q], acc[0][j][4 * q + 1], acc[0][j][4 * q + 2], acc[0][j][4 * q + 3]};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int tl = 16 * (q & 1) + pt;
+          const f32x4_t x4 = *reinterpret_cast<const f32x4_t*>(sC + (q >> 1) * 2048 + tl * 64 + ((p4 ^ ((tl >> 1) & 3)) * 16));
+          const int v = vbase + 16 * (q >> 1) + 4 * p4;
+          const int64_t t = j * 32 + tl;
+          if (t < p.T && v < vend) *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = x4;
+        }
+      }
+    }
+    fold_logits<1, FN>(acc, m, a, b, lab, p.c, vbase, vend, m0 + S::BM <= vend64, hh, p.xlabel + ln);
+  }
+
+  // merge the two lane halves (same token, different vocabulary rows), then the waves
+  __syncthreads();
+  f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);  // [8][NT]
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const float m2 = __shfl_xor(m[j], 32), a2 = __shfl_xor(a[j], 32), b2 = __shfl_xor(b[j], 32);
+    merge_stats(m[j], a[j], b[j], m2, a2, b2, p.c);
+    if (hh == 0) red[wave * NT + j * 32 + ln] = f32x4_t{m[j], a[j], b[j], 0.f};
+  }
+  __syncthreads();
+  if (tid < NT) {
+    const int t = tid;
+    const f32x4_t v0 = red[t];
+    float vm = v0[0], va = v0[1], vb = v0[2];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) {
+      const f32x4_t u = red[w * NT + t];
+      merge_stats(vm, va, vb, u[0], u[1], u[2], p.c);
+    }
+    if (t < p.T) p.parts[(int64_t)blockIdx.x * p.T + t] = f32x4_t{vm, va, vb, 0.f};
+  }
+}
+
 template <typename TIN>
 struct FewArgs {
   const TIN* dS;      // d_logits of the chunk by (compact) token position, >= kt of them, at ds_at; columns in Perm order;
@@ -74,99 +234,103 @@ struct FewArgs {
   int ksplit;         // K slices of d_hidden
   int64_t kslice;     // columns of dS per slice, a multiple of 64
   int accumulate;     // d_hidden partials: 0 store, 1 add to what is there (second and later chunks)
-  int n_dw;           // workgroups of the d_weight part (they come first in the grid)
+  int n_su;           // d_weight: workgroups side by side along the vocabulary
 };
 
 // ------------------------------------------------------------------------------------------------------------------
-// d_weight, few tokens.  Workgroup = 256 threads = 4 waves; it owns dS columns [u0, u0 + 64) and walks H in tiles of
-// HW = 256 or 128 columns; a wave multiplies 64 columns of the tile with all 64 dS columns (HW = 256) or with 32 of
-// them (HW = 128: two waves side by side along each):  C[m = h][n = u] = sum_t Ht[t][h] * dS[t][u].
+// d_weight, few tokens.  Workgroup = 256 threads = 4 waves; it owns HW = 256 columns of H, whose hidden values it keeps in
+// registers as MFMA operands for good, and walks the 64-column blocks of dS bid / n_ht, bid / n_ht + n_su, ...; a wave
+// multiplies its 64 columns of H with all 64 columns of the block:  C[m = h][n = u] = sum_t Ht[t][h] * dS[t][u].
+// What bounds it is the write of [V, H].  The neighbours bid, bid + 1, ... write the pieces of the same rows at about the same
+// time and the chip works its way through d_weight as one window of n_su x 64 rows; each block costs an 8 or 16 KB read of dS
+// (from L2) and no read of hidden.  Measured (with d_hidden, the two together; one launch of workgroups that owned 64 rows and
+// walked H, beside the d_hidden workgroups, before): H=3584, V=152064: 1 token 437 -> 374 us, 64 tokens 462 -> 411;
+// H=896, V=151936, 64 tokens: 159 -> 126; 1.09 GB at 5.3 TB/s here, at 6.5 in d_hidden (1 token).
 // MFMA rows are assigned to h in pairs of blocks: block 2i'+b, row 4g+r  <->  h = 32i' + 8g + 4b + r, so a lane ends
 // up with 8 consecutive h for one u.  With 16-bit output a wave's results pass through a tile of its own in LDS and
-// leave it as whole 128-byte lines, eight lanes per row (measured on the d_weight workgroups alone, H=3584, V=152064:
-// 64 tokens 243 -> 228 us, 4.48 -> 4.78 TB/s; 96 tokens 306 -> 296 us); fp32 output is stored from the registers,
-// 16 rows x 128 bytes per instruction.
+// leave it as whole 128-byte lines, eight lanes per row; fp32 output is stored from the registers, 16 rows x 128 bytes
+// per instruction.
 // ------------------------------------------------------------------------------------------------------------------
-template <typename TIN, typename TOUT, typename Perm, int KT, int HW>
-LCE_DEV void dw_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
-  static_assert(KT % 32 == 0 && KT <= 128, "token positions: whole k-steps of 32");
-  static_assert(HW == 256 || HW == 128, "columns of a hidden tile");
-  constexpr int KS = KT / 32;
-  constexpr int RB = HW * 2, CPR = HW / 8;  // bytes and 16-byte chunks of a hidden tile's row
-  // waves: WAVES_H along the tile's columns x WAVES_U along the 64 dS columns; a wave owns 64 columns of the hidden tile
-  // (MI = 4 MFMA row blocks) and NJ blocks of 16 dS columns
-  constexpr int WH = 64, MI = 4, WAVES_H = HW / WH, WAVES_U = 4 / WAVES_H, NJ = 4 / WAVES_U;
-  constexpr bool STAGE = sizeof(TOUT) == 2;  // 16-bit output: a wave's row piece is one 128-byte line, stored through LDS
-  char* sB = lds;                    // dS tile: KT rows x 128 bytes (64 columns), chunk c of row r at c ^ (r & 7)
-  char* sA = lds + KT * 128;         // hidden tile: KT rows x RB bytes, chunk c of row r at c ^ fw_swz(r)
+template <typename TIN, typename TOUT, typename Perm, int KT>
+__global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
+  static_assert(KT == 64 || KT == 128, "token positions");
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  constexpr int KS = KT / 32, HW = 256, RB = HW * 2, CPR = HW / 8;  // bytes and 16-byte chunks of a row of the hidden tile
+  constexpr int MI = 4, NJ = 4;
+  constexpr bool STAGE = sizeof(TOUT) == 2;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, l16 = lane & 15, e = l16 >> 2, q = l16 & 3;
-  const int wh = wave % WAVES_H, wu = wave / WAVES_H;  // this wave's place along the hidden tile and along the dS columns
-  const int64_t u0 = (int64_t)bid * 64;
-
-  // dS tile -> LDS (KT * 8 chunks of 16 bytes)
-#pragma unroll
-  for (int i = 0; i < (KT * 8 + 255) / 256; ++i) {
-    const int id = tid + i * 256, r = id >> 3, c = id & 7;
-    if (id < KT * 8) {
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ds_at(p.dS, p.ldS, p.pcol, r, u0 + c * 8));
-      *reinterpret_cast<u32x4_t*>(sB + r * 128 + ((c ^ (r & 7)) * 16)) = v;
-    }
-  }
-  constexpr int AL = KT * CPR / 256;  // 16-byte chunks of a hidden tile per thread
-  u32x4_t pre[AL];
-  auto fetch = [&](int64_t h0) {
-#pragma unroll
-    for (int i = 0; i < AL; ++i) {
-      const int id = tid + i * 256, r = id / CPR, c = id % CPR;
-      pre[i] = *reinterpret_cast<const u32x4_t*>(p.Ht + (int64_t)r * p.ldHt + h0 + c * 8);
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int i = 0; i < AL; ++i) {
-      const int id = tid + i * 256, r = id / CPR, c = id % CPR;
-      *reinterpret_cast<u32x4_t*>(sA + r * RB + ((c ^ fw_swz(r)) * 16)) = pre[i];
-    }
-  };
-  fetch(0);
-  // output rows of this lane: dS column u0 + 16 NJ wu + 16 j + l16
-  int64_t vrow[NJ];
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int64_t v = Perm::vocab_at(u0 + 16 * NJ * wu + 16 * j + l16);
-    vrow[j] = v < p.vrows ? v : -1;
-  }
-  // token positions that take part (a device-side count may cut the host's): rows beyond them are not read
-  int ks_n = p.kt / 32;
-  if (p.n_rows) {
-    const int k = (*p.n_rows + 31) / 32;
-    ks_n = k < ks_n ? k : ks_n;
-  }
-  // B fragments (dS) are the same for every h tile: they stay in registers (read once the tile has landed) unless 128
-  // token positions meet 256-column tiles (registers)
-  constexpr bool KEEP_B = KT <= 64 || HW <= 128;
-  u32x4_t bf[KEEP_B ? KS : 1][NJ];
-  auto read_b = [&](int ks, u32x4_t (&out)[NJ]) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      // lanes (e, q) of group g address row 32 ks + 8 g + e (+4), columns 16 NJ wu + 16 j + 4 q ..
-      const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4, col = 16 * NJ * wu + 16 * j + 4 * q;
-      const u32x2_t lo = tr_read_b64(sB + r0 * 128 + (((col >> 3) ^ (r0 & 7)) * 16) + (col & 7) * 2);
-      const u32x2_t hi = tr_read_b64(sB + r1 * 128 + (((col >> 3) ^ (r1 & 7)) * 16) + (col & 7) * 2);
-      out[j] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-    }
-  };
   const int n_ht = (int)((p.H + HW - 1) / HW);
-  for (int ht = 0; ht < n_ht; ++ht) {
-    __syncthreads();  // every wave is done with the previous hidden tile
-    stash();
-    __syncthreads();
-    if (KEEP_B && ht == 0) {
+  const int ht = blockIdx.x % n_ht;
+  const int64_t h0 = (int64_t)ht * HW;
+  const int64_t n_ub = p.ucols / 64;
+  char* sA = lds;               // hidden, 64 token rows x RB bytes at a time; then the four waves' store tiles of 8 KB
+  char* sB = lds + 64 * RB;     // two dS tiles: KT rows x 128 bytes (64 columns), chunk c of row r at c ^ (r & 7)
+  constexpr int BL = KT * 8 / 256;
+  int n_tok = p.kt;  // token positions that take part (a device-side count may cut the host's)
+  if (p.n_rows) n_tok = *p.n_rows < n_tok ? *p.n_rows : n_tok;
+  u32x4_t pre[BL];
+  auto fetch = [&](int64_t ub) {
+    const buf_t panel = make_buf(ds_at(p.dS, p.ldS, p.pcol, 0, ub * 64), n_tok * 128);  // rows of 128 bytes
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) read_b(ks, bf[KEEP_B ? ks : 0]);
+    for (int i = 0; i < BL; ++i) pre[i] = __builtin_amdgcn_raw_buffer_load_b128(panel, tid * 16 + i * 4096, 0, 0);
+  };
+  auto stash = [&](char* to) {
+#pragma unroll
+    for (int i = 0; i < BL; ++i) {
+      const int id = tid + i * 256, r = id >> 3, c = id & 7;
+      *reinterpret_cast<u32x4_t*>(to + r * 128 + ((c ^ (r & 7)) * 16)) = pre[i];
     }
-    if (ht + 1 < n_ht) fetch((int64_t)(ht + 1) * HW);
+  };
+  int64_t ub = blockIdx.x / n_ht;  // (< n_ub: the grid has at most that many)
+  const int64_t ub_last = ub + (n_ub - 1 - ub) / p.n_su * p.n_su;
+  fetch(ub);
+  // hidden tile -> LDS -> fragments
+  u32x4_t af[KS][MI];
+#pragma unroll
+  for (int half = 0; half < KT / 64; ++half) {
+    if (half) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64 * CPR / 256; ++i) {
+      const int id = tid + i * 256, r = id / CPR, c = id % CPR;
+      *reinterpret_cast<u32x4_t*>(sA + r * RB + ((c ^ fw_swz(r)) * 16)) =
+          *reinterpret_cast<const u32x4_t*>(p.Ht + (int64_t)(64 * half + r) * p.ldHt + h0 + c * 8);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        // block i = 2i' + b: the run of lane q starts at column 64 wave + 32 i' + 8 q + 4 b
+        const int col = 64 * wave + 32 * (i >> 1) + 8 * q + 4 * (i & 1);
+        const int r0 = 32 * k2 + 8 * g + e, r1 = r0 + 4;
+        const u32x2_t lo = tr_read_b64(sA + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
+        const u32x2_t hi = tr_read_b64(sA + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
+        af[2 * half + k2][i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+      }
+  }
+  const int ks_n = (n_tok + 31) / 32;
+  // where this lane stores, relative to the block's first row (an aligned run of 64 columns of dS is a permutation of the
+  // same 64 rows of the vocabulary): through LDS 16 bytes of eight rows, else runs of 8 columns of four rows
+  int at[STAGE ? 2 * NJ : NJ];
+#pragma unroll
+  for (int k = 0; k < (STAGE ? 2 * NJ : NJ); ++k) {
+    const int row = STAGE ? 8 * k + (lane >> 3) : 16 * k + l16;
+    const int64_t h = h0 + 64 * wave + (STAGE ? ((lane & 7) ^ ((row >> 1) & 7)) * 8 : 8 * g);
+    at[k] = h < p.H ? (int)((Perm::vocab_at(row) * p.H + h) * sizeof(TOUT)) : kBufNowhere;  // (H is a multiple of 8)
+  }
+  const int at1_add = h0 + 64 * wave + 32 + 8 * g < p.H ? 32 * (int)sizeof(TOUT) : kBufNowhere;  // the second run (no STAGE)
+  stash(sB);
+  fetch(ub < ub_last ? ub + p.n_su : ub);
+  // (as many dropped stores as a turn of the loop issues behind its fetch: the compiler waits for the fetch at the top of a turn,
+  // and only with that many younger operations on either way into the loop not for the previous block's stores as well)
+#pragma unroll
+  for (int k = 0; k < (STAGE ? 2 * NJ : 2 * MI / 2 * NJ); ++k)
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{0u, 0u, 0u, 0u}, make_buf(p.dW, 0), kBufNowhere + 16 * k, 0, 0);
+  for (int buf = 0; ub <= ub_last; ub += p.n_su, buf ^= 1) {
+    // one barrier per block: this block's tile is in LDS, and every wave is done with the other buffer
+    __syncthreads();
+    const char* tB = sB + buf * (KT * 128);
     f32x4_t acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -175,27 +339,29 @@ LCE_DEV void dw_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks >= ks_n) break;
-      u32x4_t af[MI];
+      u32x4_t bf[NJ];
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        // block i = 2i' + b: the run of lane q starts at column WH wh + 32 i' + 8 q + 4 b
-        const int col = WH * wh + 32 * (i >> 1) + 8 * q + 4 * (i & 1);
-        const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4;
-        const u32x2_t lo = tr_read_b64(sA + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
-        const u32x2_t hi = tr_read_b64(sA + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
-        af[i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+      for (int j = 0; j < NJ; ++j) {
+        // lanes (e, q) of group g address row 32 ks + 8 g + e (+4), columns 16 j + 4 q ..
+        const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4, col = 16 * j + 4 * q;
+        const u32x2_t lo = tr_read_b64(tB + r0 * 128 + (((col >> 3) ^ (r0 & 7)) * 16) + (col & 7) * 2);
+        const u32x2_t hi = tr_read_b64(tB + r1 * 128 + (((col >> 3) ^ (r1 & 7)) * 16) + (col & 7) * 2);
+        bf[j] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
       }
-      if (!KEEP_B) read_b(ks, bf[0]);
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[i], bf[KEEP_B ? ks : 0][j]);
+        for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[ks][i], bf[j]);
     }
+    stash(sB + (buf ^ 1) * (KT * 128));  // (behind the last block: the last one again)
+    fetch(ub + 2 * p.n_su <= ub_last ? ub + 2 * p.n_su : ub_last);
+    const int64_t u0 = ub * 64, left = p.vrows - u0 < 64 ? p.vrows - u0 : 64;
+    const buf_t out = make_buf(static_cast<TOUT*>(p.dW) + u0 * p.H, (left > 0 ? left : 0) * p.H * sizeof(TOUT));
     if constexpr (STAGE) {
-      // Whole 128-byte lines per store: the wave's 16 NJ rows x 64 columns go through a tile of its own in LDS (16-byte
+      // Whole 128-byte lines per store: the wave's 64 rows x 64 columns go through a tile of its own in LDS (16-byte
       // chunk c of row r at c ^ ((r / 2) % 8), so that the 16 rows x 4 chunks of one write fall into different banks)
       // and leave it eight rows at a time, eight lanes per row.  No barrier: LDS operations of one wave complete in order.
-      char* sC = lds + KT * 128 + KT * RB + wave * (NJ * 2048);
+      char* sC = sA + wave * 8192;
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -206,60 +372,64 @@ LCE_DEV void dw_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
           const int row = 16 * j + l16, c = 4 * ip + g;
           store_run<TOUT, 8>(reinterpret_cast<TOUT*>(sC + row * 128 + ((c ^ ((row >> 1) & 7)) * 16)), d);
         }
-      const int64_t hw0 = (int64_t)ht * HW + WH * wh;
 #pragma unroll
       for (int it = 0; it < NJ * 2; ++it) {
-        const int row = it * 8 + (lane >> 3), pc = lane & 7, c = pc ^ ((row >> 1) & 7);
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sC + row * 128 + pc * 16);
-        const int64_t vr = Perm::vocab_at(u0 + 16 * NJ * wu + row), h = hw0 + c * 8;
-        if (vr < p.vrows && h < p.H) *reinterpret_cast<u32x4_t*>(static_cast<TOUT*>(p.dW) + vr * p.H + h) = v;
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sC + (it * 8 + (lane >> 3)) * 128 + (lane & 7) * 16);
+        __builtin_amdgcn_raw_buffer_store_b128(v, out, at[it], 0, 0);
       }
-      continue;
-    }
-    // lane (g, l16): rows h = h0 + WH wh + 32 i' + 8 g + (0..7) of output row vrow[j]
-    const int64_t hb = (int64_t)ht * HW + WH * wh + 8 * g;
+    } else {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      if (vrow[j] < 0) continue;
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int ip = 0; ip < MI / 2; ++ip) {
-        const int64_t h = hb + 32 * ip;
-        if (h >= p.H) continue;  // (H is a multiple of 8)
-        float d[8];
+        for (int ip = 0; ip < MI / 2; ++ip)
 #pragma unroll
-        for (int x = 0; x < 8; ++x) d[x] = acc[2 * ip + (x >> 2)][j][x & 3];
-        store_run<TOUT, 8>(static_cast<TOUT*>(p.dW) + vrow[j] * p.H + h, d);  // (non-temporal stores: 2.9 instead of 4.1 TB/s)
-      }
+          for (int hf = 0; hf < 2; ++hf) {
+            u32x4_t v;
+            __builtin_memcpy(&v, &acc[2 * ip + hf][j], 16);
+            const int o = at[j] == kBufNowhere ? at[j] : ip ? (at1_add == kBufNowhere ? at1_add : at[j] + at1_add) : at[j];
+            __builtin_amdgcn_raw_buffer_store_b128(v, out, o == kBufNowhere ? o : o + 16 * hf, 0, 0);
+          }
     }
   }
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// d_hidden, few tokens.  Workgroup = 256 threads = 4 waves; it owns columns [h0, h0 + 256) of the result for all NT
-// token rows and one K slice of the chunk's dS columns; wave w multiplies h0 + 64w .. +63:
-//   C[m = h][n = t] = sum_u W[vocab_at(u)][h] * dS[t][u].
+// d_hidden, few tokens.  Workgroup = 512 threads = 8 waves, one per CU; it owns columns [h0, h0 + 256) of the result for all
+// NT token rows and one K slice of the chunk's dS columns; wave w multiplies columns h0 + 64 (w % 4) .. +63 with half of the
+// token rows:  C[m = h][n = t] = sum_u W[vocab_at(u)][h] * dS[t][u].
 // A stage is 64 columns of dS: 64 rows of W (512 bytes of each, fetched in the order of dS's columns) and NT x 128
-// bytes of dS.
+// bytes of dS.  What bounds it is the read of W, and that by the bytes in flight: DEPTH stages are on their way in registers
+// (128 KB of W per CU up to 64 tokens, 96 KB beyond) while one is multiplied out of LDS, which holds two, so that a stage
+// costs one barrier.
 // ------------------------------------------------------------------------------------------------------------------
-template <typename TIN, typename Perm, int NT, int HW>
-LCE_DEV void dh_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
+template <int KT>
+struct FewShape {  // KT: token positions, 64 up to 64 tokens, else 128
+  static constexpr int HW = 256;                                     // columns of H per workgroup
+  static constexpr int DW_LDS = 64 * HW * 2 + 2 * KT * 128;          // hidden (then store tiles), two dS tiles
+  static constexpr int DH_DEPTH = KT <= 64 ? 4 : 3;
+  static constexpr int DH_STAGE = 64 * HW * 2 + KT * 128;            // W rows, dS tile
+  static constexpr int DH_LDS = 2 * DH_STAGE;
+};
+
+template <typename TIN, typename Perm, int NT>
+__global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
   static_assert(NT == 64 || NT == 128, "token rows of a tile");
-  static_assert(HW == 256 || HW == 128, "columns of a tile");
-  constexpr int NJ = NT / 16;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  typedef FewShape<NT> S;
+  constexpr int HW = S::HW, DEPTH = S::DH_DEPTH;
+  constexpr int NJ = NT / 32, MI = 4;       // 16-wide MFMA blocks of a wave: tokens, columns
   constexpr int RB = HW * 2, CPR = HW / 8;  // bytes and 16-byte chunks of a W stage's row
-  constexpr int WH = HW / 4, MI = WH / 16;  // columns and 16-row MFMA blocks of a wave
-  constexpr int WL = 64 * CPR / 256;        // chunks of a W stage per thread
-  char* sA = lds;              // W stage: 64 rows x RB bytes, chunk c of row r at c ^ fw_swz(r)
-  char* sB = lds + 64 * RB;    // dS stage: NT rows x 128 bytes, chunk c of row t at c ^ ((t >> 1) & 7)
+  constexpr int WL = 64 * CPR / 512;        // chunks of a W stage per thread: row tid / CPR + (512 / CPR) i, chunk tid % CPR
+  constexpr int BL = NT * 8 / 512;          // ... of the dS stage
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int wc = wave & 3, wt = wave >> 2;
   const int g = lane >> 4, l16 = lane & 15, e = l16 >> 2, q = l16 & 3;
   const int n_ht = (int)((p.H + HW - 1) / HW);
-  const int ht = bid % n_ht, s = bid / n_ht;
+  const int ht = blockIdx.x % n_ht, s = blockIdx.x / n_ht;
   const int64_t h0 = (int64_t)ht * HW;
   const int64_t k_begin = (int64_t)s * p.kslice;
-  int64_t k_end = k_begin + p.kslice;
-  if (k_end > p.ucols) k_end = p.ucols;
-  float* out = p.dHp + (int64_t)s * p.part_stride;
+  const int64_t k_left = p.ucols - k_begin;
+  const int n_st = k_left <= 0 ? 0 : (int)((k_left < p.kslice ? k_left : p.kslice) / 64);  // stages (both are multiples of 64)
 
   f32x4_t acc[MI][NJ];
 #pragma unroll
@@ -267,73 +437,85 @@ LCE_DEV void dh_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // per thread: WL chunks of the W stage (row r = tid / CPR + (256 / CPR) i, chunk tid % CPR), NT / 32 chunks of the dS stage
-  const int wc = tid % CPR;
-  const int64_t wcol = (h0 + wc * 8 < p.H) ? h0 + wc * 8 : 0;  // (columns beyond H: any in-bounds address; results are not stored)
-  constexpr int BL = NT * 8 / 256;
-  u32x4_t pw[WL], pb[BL];
-  auto fetch = [&](int64_t k0) {
+  // what this lane fetches of a stage, relative to the stage's first row of W (an aligned run of 64 columns of dS is a
+  // permutation of the same 64 rows) and to its panel of dS.  Rows beyond the chunk and columns beyond H read as zero.
+  const int ch = tid % CPR;
+  int w_at[WL];
 #pragma unroll
-    for (int i = 0; i < WL; ++i) {
-      const int r = tid / CPR + (256 / CPR) * i;
-      int64_t v = Perm::vocab_at(k0 + r);
-      v = v < p.vrows ? v : p.vrows - 1;  // dS is zero in such a column
-      pw[i] = load_vec<true>(reinterpret_cast<const u32x4_t*>(p.W + v * p.ldw + wcol));
-    }
+  for (int i = 0; i < WL; ++i) {
+    const int r = tid / CPR + (512 / CPR) * i;
+    w_at[i] = h0 + ch * 8 < p.H ? (int)((Perm::vocab_at(r) * p.ldw + h0 + ch * 8) * sizeof(TIN)) : kBufNowhere;
+  }
+  int n_tok = p.kt;  // token positions that take part (a device-side count may cut the host's)
+  if (p.n_rows) n_tok = *p.n_rows < n_tok ? *p.n_rows : n_tok;
+  u32x4_t pw[DEPTH][WL], pb[DEPTH][BL];
+  auto fetch = [&](u32x4_t (&w)[WL], u32x4_t (&b)[BL], int st) {
+    // (stages behind the last one: W reads as zero; the number of stages is rounded up to whole turns of the loop below)
+    const int64_t k0 = k_begin + 64 * (int64_t)(st < n_st ? st : n_st - 1), left = p.vrows - k0 < 64 ? p.vrows - k0 : 64;
+    const buf_t wb = make_buf(p.W + k0 * p.ldw, (left > 0 && st < n_st ? left : 0) * p.ldw * sizeof(TIN));
 #pragma unroll
-    for (int i = 0; i < BL; ++i) {
-      const int id = tid + i * 256, t = id >> 3, c = id & 7;
-      pb[i] = *reinterpret_cast<const u32x4_t*>(ds_at(p.dS, p.ldS, p.pcol, t, k0 + c * 8));
-    }
+    for (int i = 0; i < WL; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(wb, w_at[i], 0, kBufNonTemporal);
+    const buf_t panel = make_buf(ds_at(p.dS, p.ldS, p.pcol, 0, k0), n_tok * 128);  // rows of 128 bytes
+#pragma unroll
+    for (int i = 0; i < BL; ++i) b[i] = __builtin_amdgcn_raw_buffer_load_b128(panel, tid * 16 + i * 8192, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // (the loads of one stage stay in front of the next one's)
   };
-  auto stash = [&]() {
+  if (n_st > 0) {
 #pragma unroll
-    for (int i = 0; i < WL; ++i) {
-      const int r = tid / CPR + (256 / CPR) * i;
-      *reinterpret_cast<u32x4_t*>(sA + r * RB + ((wc ^ fw_swz(r)) * 16)) = pw[i];
-    }
+    for (int d = 0; d < DEPTH; ++d) fetch(pw[d], pb[d], d);
+  }
+  int buf = 0;
+  for (int st0 = 0; st0 < n_st; st0 += DEPTH) {
 #pragma unroll
-    for (int i = 0; i < BL; ++i) {
-      const int id = tid + i * 256, t = id >> 3, c = id & 7;
-      *reinterpret_cast<u32x4_t*>(sB + t * 128 + ((c ^ ((t >> 1) & 7)) * 16)) = pb[i];
-    }
-  };
-  if (k_begin < k_end) fetch(k_begin);
-  for (int64_t k0 = k_begin; k0 < k_end; k0 += 64) {
-    __syncthreads();
-    stash();
-    __syncthreads();
-    if (k0 + 64 < k_end) fetch(k0 + 64);
+    for (int d = 0; d < DEPTH; ++d) {
+      char* sA = lds + buf * S::DH_STAGE;  // 64 rows x RB bytes, chunk c of row r at c ^ fw_swz(r)
+      char* sB = sA + 64 * RB;             // NT rows x 128 bytes, chunk c of row t at c ^ ((t >> 1) & 7)
+      buf ^= 1;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      u32x4_t af[MI], bf[NJ];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const int col = WH * wave + 16 * i + 4 * q;
-        const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4;
-        const u32x2_t lo = tr_read_b64(sA + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
-        const u32x2_t hi = tr_read_b64(sA + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
-        af[i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+      for (int i = 0; i < WL; ++i) {
+        const int r = tid / CPR + (512 / CPR) * i;
+        *reinterpret_cast<u32x4_t*>(sA + r * RB + ((ch ^ fw_swz(r)) * 16)) = pw[d][i];
       }
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int t = 16 * j + l16, c = 4 * ks + g;  // k = 32 ks + 8 g .. +7 of token row t
-        bf[j] = *reinterpret_cast<const u32x4_t*>(sB + t * 128 + ((c ^ ((t >> 1) & 7)) * 16));
+      for (int i = 0; i < BL; ++i) {
+        const int id = tid + i * 512, t = id >> 3, c = id & 7;
+        *reinterpret_cast<u32x4_t*>(sB + t * 128 + ((c ^ ((t >> 1) & 7)) * 16)) = pb[d][i];
       }
+      fetch(pw[d], pb[d], st0 + d + DEPTH);
+      // (a buffer is written again two stages on: every wave has passed the barrier between, after its reads of this stage)
+      __syncthreads();
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+      for (int ks = 0; ks < 2; ++ks) {
+        u32x4_t af[MI], bf[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[i], bf[j]);
+        for (int i = 0; i < MI; ++i) {
+          const int col = 64 * wc + 16 * i + 4 * q;
+          const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4;
+          const u32x2_t lo = tr_read_b64(sA + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
+          const u32x2_t hi = tr_read_b64(sA + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
+          af[i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int t = (NT / 2) * wt + 16 * j + l16, c = 4 * ks + g;  // k = 32 ks + 8 g .. +7 of token row t
+          bf[j] = *reinterpret_cast<const u32x4_t*>(sB + t * 128 + ((c ^ ((t >> 1) & 7)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[i], bf[j]);
+      }
     }
   }
-  // lane (g, l16): h = h0 + WH wave + 16 i + 4 g + (0..3) of token row 16 j + l16
+  // lane (g, l16): h = h0 + 64 wc + 16 i + 4 g + (0..3) of token row NT/2 wt + 16 j + l16
+  float* out = p.dHp + (int64_t)s * p.part_stride;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int t = 16 * j + l16;
+    const int t = (NT / 2) * wt + 16 * j + l16;
     if (t >= p.nt) continue;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-      const int64_t h = h0 + WH * wave + 16 * i + 4 * g;
+      const int64_t h = h0 + 64 * wc + 16 * i + 4 * g;
       if (h >= p.H) continue;  // (H is a multiple of 4)
       float* dst = out + (int64_t)t * p.H + h;
       f32x4_t v = acc[i][j];
@@ -341,27 +523,6 @@ LCE_DEV void dh_few_tile(const FewArgs<TIN>& p, int bid, char* lds) {
       *reinterpret_cast<f32x4_t*>(dst) = v;
     }
   }
-}
-
-// KT / NT: token positions (64 up to 64 tokens, else 128); HW: columns of H per tile (256 up to 64 tokens, else 128,
-// which keeps the accumulators and the tile in flight within 128 registers a lane)
-template <int KT>
-struct FewShape {
-  static constexpr int NT = KT, HW = KT <= 64 ? 256 : 128, HW_DW = HW;
-  static constexpr int DW = KT * 128 + KT * HW_DW * 2 + HW_DW * 128;  // dS tile, hidden tile, the four waves' store tiles
-  static constexpr int DH = 64 * HW * 2 + NT * 128;
-  static constexpr int LDS_BYTES = DW > DH ? DW : DH;
-};
-
-// One launch: the d_weight workgroups (the writers) first, then the d_hidden workgroups (the readers); the two
-// streams overlap in time.
-template <typename TIN, typename TOUT, typename Perm, int KT>
-__global__ __launch_bounds__(256, 2) void lce_bwd_few_kernel(FewArgs<TIN> p) {
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
-  typedef FewShape<KT> S;
-  const int bid = blockIdx.x;
-  if (bid < p.n_dw) dw_few_tile<TIN, TOUT, Perm, KT, S::HW_DW>(p, bid, lds);
-  else dh_few_tile<TIN, Perm, S::NT, S::HW>(p, bid - p.n_dw, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

@@ -325,7 +325,8 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   int S = Cfg::BN > 128 ? forward_splits_256(ntt, nvt, max_splits) : bc * ((8 + nrb - 1) / nrb);
   if (S > nvt) S = nvt;
   if (S > max_splits) S = max_splits;
-  // The narrow token tiles serve the HBM-bound case (up to 128 tokens: one streaming read of W).  There each
+  // The narrow token tiles serve the HBM-bound case (up to 128 tokens: one streaming read of W; 16-bit inputs of up to 64
+  // tokens have a kernel of their own, forward_few).  There each
   // split takes one contiguous range of rows, the same length for all, instead of whole tiles dealt round robin
   // (594 tiles over 256 splits would be 3 against 2, and a split's tiles would lie 256 tiles apart).  Measured
   // on the kernel, H=3584, V=152064: T=1 203 -> 187 us, T=64 209 -> 190, T=128 221 -> 211; H=4096, V=128256,
@@ -371,6 +372,34 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
                        entropy_b, shard_out, st);
 }
 
+// forward with at most 64 tokens of 16 bits (few_tokens.hpp): one contiguous range of rows per workgroup, one workgroup per CU;
+// whole panels of the kept logits
+template <typename TIN>
+int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
+                int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, hipStream_t st,
+                int64_t label_offset, float* shard_out, int max_splits, float* xcache) {
+  const int most = max_splits < kNumCUs ? max_splits : kNumCUs;
+  FwdArgs<TIN> p;
+  p.split_stride = p.split_span = round_up((V + most - 1) / most, 16);
+  const int S = (int)((V + p.split_stride - 1) / p.split_stride);
+  p.W = W; p.ldw = ldw; p.h = h; p.ldh = ldh; p.labels = labels; p.T = T; p.V = V; p.H = H;
+  p.c = kLog2e / temperature;
+  p.parts = reinterpret_cast<f32x4_t*>(ws);
+  p.xlabel = reinterpret_cast<float*>(ws + align256((size_t)S * T * 16));
+  p.S = S; p.tile_step = 256; p.label_offset = label_offset; p.xcache = xcache; p.w_plane = p.h_plane = 0;
+  float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
+  {
+    ProfScope prof(PC_FWD, st);
+    auto kern = lce_fwd_few_kernel<TIN>;
+    allow_lds(kern, FewFwdShape::LDS_BYTES);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S), dim3(512), FewFwdShape::LDS_BYTES, st, p);
+    int rc = check_launch("lce_fwd_few_kernel");
+    if (rc) return rc;
+  }
+  return forward_merge(p.parts, p.xlabel, labels, label_offset, V, S, T, p.c, temperature, reduction, lp_tok, logprobs, entropy, maximum, accumulate,
+                       entropy_b, shard_out, st);
+}
+
 // upper bound of the number of vocabulary splits forward_impl picks, over the token-tile widths in use
 int forward_splits_upper_bound(int64_t T, int64_t V, int max_splits = kMaxSplits) {
   int best = forward_splits_256((int)((T + 255) / 256), (int)((V + 255) / 256), max_splits);
@@ -408,8 +437,6 @@ bool dw_transposed_reads(size_t esz) { return esz == 2; }
 // vocabulary chunk.  With few tokens one such tile takes longer than a CU's share of the whole launch
 // (d_logits tiles + both GEMMs) and would set the launch's duration; the K range is then cut into
 // slices, with an fp32 partial each, so that a tile takes at most about half of that share.
-int64_t few_tile_columns(int64_t T) { return T <= 64 ? FewShape<64>::HW : FewShape<128>::HW; }
-
 int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
   const int64_t ntt = (T + 255) / 256, nht = (H + 255) / 256, nvt = (vchunk + 255) / 256;
   const int64_t work = ntt * nvt * H + nvt * nht * ntt * 256 + ntt * nht * vchunk;  // in K elements of 256x256 tiles
@@ -454,13 +481,13 @@ BwdLayout bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, size
   L.ksplit = tu.dh_ksplit > 0 ? tu.dh_ksplit : dh_ksplit(T, H, vchunk);
   L.few = tu.few_token_gemms && L.tn && T <= 128;
   if (L.few) {
-    // K slices of the streaming d_hidden kernel: its workgroups (column tiles x slices) fill the chip about twice
-    // over, which is what two resident workgroups per CU take in one round; at least 1024 columns per slice
-    const int64_t n_ht = (H + few_tile_columns(T) - 1) / few_tile_columns(T);
-    int64_t ks = (2 * kNumCUs) / n_ht;
-    const int64_t most = (vchunk + 1023) / 1024;
+    // K slices of the streaming d_hidden kernel: its workgroups (column tiles x slices) fill the chip once, one to a CU;
+    // at least 512 columns per slice
+    const int64_t n_ht = (H + FewShape<64>::HW - 1) / FewShape<64>::HW;
+    int64_t ks = kNumCUs / n_ht;
+    const int64_t most = (vchunk + 511) / 512;
     ks = ks > most ? most : ks;
-    L.ksplit = tu.dh_ksplit > 0 ? tu.dh_ksplit : (int)(ks < 1 ? 1 : ks > 40 ? 40 : ks);
+    L.ksplit = tu.dh_ksplit > 0 ? tu.dh_ksplit : (int)(ks < 1 ? 1 : ks);
     L.tn_dh = true;  // W is read in place
   }
   L.nchunks = (int)((V + vchunk - 1) / vchunk);
@@ -587,18 +614,34 @@ int launch_ds_few_tokens(DsArgs<typename Cfg::TIN> d, int64_t T, int nvt, hipStr
   return check_launch("lce_bwd_ds_kernel");
 }
 
-// Both gradient GEMMs of one vocabulary chunk of a backward with at most 128 tokens, as one launch of the streaming
-// kernels (few_tokens.hpp): d_weight rows of the chunk in the output dtype, d_hidden as L.ksplit fp32 partials.
+// Both gradient GEMMs of one vocabulary chunk of a backward with at most 128 tokens as two launches of the streaming
+// kernels (few_tokens.hpp): d_hidden as L.ksplit fp32 partials, d_weight rows of the chunk in the output dtype.
 template <typename Cfg, typename TOUT, int KT>
-int launch_few_gemms(const FewArgs<typename Cfg::TIN>& q, bool with_dh, hipStream_t st) {
+int launch_few_gemms(FewArgs<typename Cfg::TIN> q, bool with_dh, hipStream_t st) {
   typedef typename Cfg::TIN TIN;
   typedef FewShape<KT> S;
-  const int n_ht = (int)((q.H + S::HW - 1) / S::HW);
-  auto kern = lce_bwd_few_kernel<TIN, TOUT, KPerm<Cfg>, KT>;
-  allow_lds(kern, S::LDS_BYTES);
-  // (q.n_dw = 0: no d_weight workgroups; without d_hidden the grid ends after them)
-  hipLaunchKernelGGL(kern, dim3((unsigned)(q.n_dw + (with_dh ? n_ht * q.ksplit : 0))), dim3(256), S::LDS_BYTES, st, q);
-  return check_launch("lce_bwd_few_kernel");
+  int rc;
+  if (with_dh) {
+    ProfScope prof(PC_GEMM_DH, st);
+    const int n_ht = (int)((q.H + S::HW - 1) / S::HW);
+    auto kern = lce_dh_few_kernel<TIN, KPerm<Cfg>, KT>;
+    allow_lds(kern, S::DH_LDS);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_ht * q.ksplit)), dim3(512), S::DH_LDS, st, q);
+    if ((rc = check_launch("lce_dh_few_kernel"))) return rc;
+  }
+  if (q.dW) {
+    ProfScope prof(PC_GEMM_DW, st);
+    const int n_ht = (int)((q.H + S::HW - 1) / S::HW);
+    // as many workgroups as are resident at once: three per CU up to 64 tokens, two beyond (LDS, registers)
+    q.n_su = ((KT <= 64 ? 3 : 2) * kNumCUs) / n_ht;
+    if (q.n_su < 1) q.n_su = 1;
+    if (q.n_su > q.ucols / 64) q.n_su = (int)(q.ucols / 64);
+    auto kern = lce_dw_few_kernel<TIN, TOUT, KPerm<Cfg>, KT>;
+    allow_lds(kern, S::DW_LDS);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_ht * q.n_su)), dim3(256), S::DW_LDS, st, q);
+    if ((rc = check_launch("lce_dw_few_kernel"))) return rc;
+  }
+  return LCE_OK;
 }
 
 template <typename Cfg>
@@ -779,8 +822,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           q.dHp = dHacc; q.part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
           q.ksplit = L.ksplit; q.kslice = round_up((q.ucols + L.ksplit - 1) / L.ksplit, 64);
           q.accumulate = cc == 0 ? 0 : 1;
-          q.n_dw = need_dw ? (int)(q.ucols / 64) : 0;
-          ProfScope prof(PC_BWD_CHUNK, st);
+          q.n_su = 1;
           if (T <= 64) rc = grads_f32 ? launch_few_gemms<Cfg, float, 64>(q, need_dh, st) : launch_few_gemms<Cfg, TIN, 64>(q, need_dh, st);
           else rc = grads_f32 ? launch_few_gemms<Cfg, float, 128>(q, need_dh, st) : launch_few_gemms<Cfg, TIN, 128>(q, need_dh, st);
           if (rc) return rc;

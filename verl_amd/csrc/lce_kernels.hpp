@@ -61,10 +61,78 @@ struct FwdArgs {
 
 // Kept logits lie in panels of 16 vocabulary rows, [panel][token][16] fp32: what one 16 x 16 block of a tile holds is one
 // contiguous kilobyte, and a tile's 256 rows touch a few pages.  (As [token][vocabulary] the rows of a tile are 608 KB
-// apart at V=152064, a page each, and the stores of 16 rows x 64 bytes per instruction cost more than the data: 333
-// tokens, forward with kept logits KEEP_BEFORE -> KEEP_AFTER us.)
+// apart at V=152064, a page each, and the stores of 16 rows x 64 bytes per instruction cost more than the data.)
 template <typename P>
 LCE_DEV P kept_logit(P x, int64_t T, int64_t t, int64_t v) { return x + ((v >> 4) * T + t) * 16 + (v & 15); }
+
+// Folds the logits of one tile into the running statistics of a lane's tokens (block column j: one token).  `full`: no row of
+// the tile is beyond vend; lab: the tokens' labels as rows of W (or -1); xlabel: where the first block column's raw label
+// logit goes, 32 tokens per block column.
+template <int FM, int FN>
+LCE_DEV void fold_logits(f32x16_t (&acc)[FM][FN], float (&m)[FN], float (&a)[FN], float (&b)[FN], const int (&lab)[FN], float c, int vbase,
+                         int vend, bool full, int hh, float* xlabel) {
+  if (!full) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (vbase + acc_row(i, r, hh) >= vend) acc[i][j][r] = -INFINITY;
+  }
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    __builtin_amdgcn_sched_barrier(0);  // keep one block column in flight at a time (register pressure)
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, acc[i][j][r]);
+    __builtin_amdgcn_sched_barrier(0);
+    const float mn = fmaxf(m[j], tmax);
+    const float sc = fast_exp2((m[j] - mn) * c);
+    const float mc = mn * c;
+    float aj = a[j] * sc, bj = b[j] * sc;
+    m[j] = mn;
+    if (full) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = acc[i][j][r];
+          const float e = fast_exp2(__builtin_fmaf(x, c, -mc));
+          aj += e;
+          bj = __builtin_fmaf(x, e, bj);
+        }
+    } else {
+      // padded vocabulary rows: -inf in the log-sum-exp, 0 in the sum of x * exp
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = acc[i][j][r];
+          const float e = fast_exp2(__builtin_fmaf(x, c, -mc));
+          aj += e;
+          bj = __builtin_fmaf(x == -INFINITY ? 0.f : x, e, bj);
+        }
+    }
+    a[j] = aj;
+    b[j] = bj;
+    // label logit: rare (a token's label falls in this wave tile with probability WM / V)
+    const int rel = lab[j] - vbase;
+    const bool mine = lab[j] >= 0 && lab[j] < vend && rel >= 0 && rel < FM * 32 && (((rel >> 2) & 1) == hh);
+    if (__builtin_amdgcn_ballot_w64(mine) != 0) {
+      float pick = 0.f;
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (mine && acc_row(i, r, hh) == rel) pick = acc[i][j][r];
+      // exactly one lane in the whole grid owns a token's label: plain store, no merge needed
+      if (mine) xlabel[j * 32] = pick;
+    }
+  }
+}
 
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename Cfg::TIN> p) {
@@ -107,7 +175,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename
       // vocabulary rows of a token in four consecutive registers, 16 bytes of that token's row of the cache; the lanes'
       // pieces of a 128-byte line meet in L2.  Issued AHEAD of the next tile's first loads: the K loop waits on counts
       // of outstanding vector-memory operations, and with the stores older than every load it waits for, those counts
-      // mean what they say (64 tokens: 209 instead of 187 us, the same as with the stores behind those loads).
+      // mean what they say.
       if (p.xcache) {
 #pragma unroll
         for (int j = 0; j < Cfg::FN; ++j) {
@@ -138,67 +206,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename
       g.init(p.W, p.ldw, m0 + p.tile_step, vend64, p.h, p.ldh, n0, p.T);
       g.prologue(lds, p.H);
     }
-    if (!full) {
-#pragma unroll
-      for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < Cfg::FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (vbase + acc_row(i, r, hh) >= vend) acc[i][j][r] = -INFINITY;
-    }
-#pragma unroll
-    for (int j = 0; j < Cfg::FN; ++j) {
-      __builtin_amdgcn_sched_barrier(0);  // keep one block column in flight at a time (register pressure)
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, acc[i][j][r]);
-      __builtin_amdgcn_sched_barrier(0);
-      const float mn = fmaxf(m[j], tmax);
-      const float sc = fast_exp2((m[j] - mn) * p.c);
-      const float mc = mn * p.c;
-      float aj = a[j] * sc, bj = b[j] * sc;
-      m[j] = mn;
-      if (full) {
-#pragma unroll
-        for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float x = acc[i][j][r];
-            const float e = fast_exp2(__builtin_fmaf(x, p.c, -mc));
-            aj += e;
-            bj = __builtin_fmaf(x, e, bj);
-          }
-      } else {
-        // padded vocabulary rows: -inf in the log-sum-exp, 0 in the sum of x * exp
-#pragma unroll
-        for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float x = acc[i][j][r];
-            const float e = fast_exp2(__builtin_fmaf(x, p.c, -mc));
-            aj += e;
-            bj = __builtin_fmaf(x == -INFINITY ? 0.f : x, e, bj);
-          }
-      }
-      a[j] = aj;
-      b[j] = bj;
-      // label logit: rare (a token's label falls in this wave tile with probability WM / V)
-      const int rel = lab[j] - vbase;
-      const bool mine = lab[j] >= 0 && lab[j] < vend && rel >= 0 && rel < Cfg::WM && (((rel >> 2) & 1) == hh);
-      if (__builtin_amdgcn_ballot_w64(mine) != 0) {
-        float pick = 0.f;
-#pragma unroll
-        for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (mine && acc_row(i, r, hh) == rel) pick = acc[i][j][r];
-        // exactly one lane in the whole grid owns a token's label: plain store, no merge needed
-        if (mine) p.xlabel[n0 + g.wave_n * Cfg::WN + j * 32 + ln] = pick;
-      }
-    }
+    fold_logits<Cfg::FM, Cfg::FN>(acc, m, a, b, lab, p.c, vbase, vend, full, hh, p.xlabel + n0 + g.wave_n * Cfg::WN + ln);
   }
   __syncthreads();
 
