@@ -191,77 +191,6 @@ inline __global__ __launch_bounds__(256) void sort_scatter_kernel(const uint32_t
   sort_scatter_block(kin, vin, kout, vout, shift, blockIdx.x, nblocks, gh, base);
 }
 
-// Up to kSortBlock tokens: keys and all passes in one workgroup (buffers 0 / 1 alternate; `passes` is even or
-// odd, the caller reads the result from buffer passes % 2).
-inline __global__ __launch_bounds__(256) void label_sort_single_kernel(LabelTerm lt, const int* rows, const int* n_rows, int64_t T, int passes,
-                                                                uint32_t* keys0, int* vals0, uint32_t* keys1, int* vals1) {
-  __shared__ int tab[256];
-  __shared__ int gh[256];
-  const int tid = threadIdx.x;
-  const int64_t n = n_rows ? (int64_t)*n_rows : T;
-  if (n <= 256) {
-    // few tokens: every thread ranks its own item among all of them (stable: ties by position), one pass, no radix
-    // passes (16 -> 4 us with 64 tokens, where the whole backward takes 0.7 ms)
-    uint32_t key = kNoRow;
-    int tok = -1;
-    if (tid < n) {
-      tok = rows ? rows[tid] : tid;
-      float G;
-      key = label_row(lt, tok, G);
-    }
-    tab[tid] = (int)key;  // (bit pattern; compared as unsigned below)
-    __syncthreads();
-    int rank = 0;
-    for (int j = 0; j < 256; ++j) {
-      const uint32_t kj = (uint32_t)tab[j];
-      rank += (kj < key || (kj == key && j < tid)) ? 1 : 0;
-    }
-    uint32_t* kout = (passes & 1) ? keys1 : keys0;  // where the caller reads the result of `passes` radix passes
-    int* vout = (passes & 1) ? vals1 : vals0;
-    kout[rank] = key;
-    vout[rank] = tok;
-    for (int k = 256 + tid; k < kSortBlock; k += 256) {
-      kout[k] = kNoRow;
-      vout[k] = -1;
-    }
-    return;
-  }
-  for (int k = tid; k < kSortBlock; k += 256) {
-    uint32_t key = kNoRow;
-    int tok = -1;
-    if (k < n) {
-      tok = rows ? rows[k] : k;
-      float G;
-      key = label_row(lt, tok, G);
-    }
-    keys0[k] = key;
-    vals0[k] = tok;
-  }
-  __syncthreads();
-  for (int p = 0; p < passes; ++p) {
-    const uint32_t* kin = (p & 1) ? keys1 : keys0;
-    const int* vin = (p & 1) ? vals1 : vals0;
-    uint32_t* kout = (p & 1) ? keys0 : keys1;
-    int* vout = (p & 1) ? vals0 : vals1;
-    sort_hist_block(kin, 8 * p, 0, 1, gh, tab);
-    __syncthreads();
-    // exclusive scan of the 256 digit counts
-    const int own = gh[tid];
-    tab[tid] = own;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const int v = tid >= off ? tab[tid - off] : 0;
-      __syncthreads();
-      tab[tid] += v;
-      __syncthreads();
-    }
-    gh[tid] = tab[tid] - own;
-    __syncthreads();
-    sort_scatter_block(kin, vin, kout, vout, 8 * p, 0, 1, gh, tab);
-    __syncthreads();
-  }
-}
-
 // d_weight[row][:] += sum of G_t * hidden[t][:] over the run of sorted positions with key == row, in order.
 // One workgroup per sorted position; only the first position of a run works.  Runs after the d_weight GEMMs:
 // the rows are read back in the output dtype (rounded once by the GEMM that wrote the softmax terms, which are
@@ -299,61 +228,109 @@ __global__ __launch_bounds__(256) void dw_label_rows_kernel(const uint32_t* keys
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Few tokens (at most 128, 16-bit inputs): a backward of well under a millisecond, where every small launch costs
-// 5 us or more.  One launch before the d_logits pass and one after the gradient GEMMs replace eight:
-//   few_prep_kernel    the list of tokens with a gradient (active_count / active_rows), the label coefficients
-//                      (label_coef) and the compact copy of hidden (gather_rows);
-//   few_finish_kernel  d_hidden from its partials (dh_finish) and the one-hot rows of d_weight (dw_label_rows), which
-//                      finds the tokens that share a label by comparing all pairs instead of sorting them.
-// Results are the same bits as from the separate kernels: same expressions, same order of every sum.
+// Up to kPrepTokens tokens, 16-bit inputs: a backward of a few milliseconds at most, where every small launch costs 5 us or
+// more.  One launch before the d_logits pass and one after the gradient GEMMs replace eight:
+//   token_prep_kernel    the list of tokens with a gradient (active_count / active_rows), the label coefficients
+//                        (label_coef), the compact copy of hidden (gather_rows), the constants of the d_logits tiles
+//                        (ds_token_consts), the label of every listed token;
+//   token_finish_kernel  d_hidden from its partials (dh_finish) and the one-hot rows of d_weight (dw_label_rows), which
+//                        finds the tokens that share a label by comparing a token's with all of them instead of sorting.
+// Results are the same bits as from the separate kernels: same expressions, same order of every sum.  (333 tokens, H=3584:
+// 86 -> 35 us of launches; every workgroup goes through all tokens, which at 4096 would cost more than the launches saved.)
 // ------------------------------------------------------------------------------------------------------------------
+constexpr int kPrepTokens = 2048, kPrepRounds = kPrepTokens / 256;
 
-// Workgroup b: every workgroup lists the tokens itself (ballots over at most 128 gradients); workgroup 0 stores the
-// list; workgroup b then owns compact position b: the row of hidden it copies to Ht[b] (zeros from the list's end up to
-// the next multiple of 64, the K granule of the d_weight product) and that token's label coefficient (wave 0).
-// Grid: tokens rounded up to 64, at most rpad.  a.coef may be null (no coefficients wanted).
-template <typename T>
-__global__ __launch_bounds__(256) void few_prep_kernel(CoefArgs<T> a, T* Ht, int64_t ldHt, int64_t rpad, int* rows, int* inv, int* n_rows) {
+struct TokenPrep {
+  int64_t rpad;           // rows of the compact copy that exist
+  int* rows;
+  int* inv;
+  int* n_rows;
+  uint32_t* keys;         // label row of every listed token by compact position, or kNoRow (null: not wanted)
+  int64_t tpad;           // positions of tokc / tokl
+  f32x4_t* tokc;          // constants of the d_logits tiles (null: not wanted)
+  int* tokl;
+};
+
+// Ordered compaction of a predicate over kPrepTokens items by one workgroup of 256 threads: item r * 256 + tid is on[r].
+// cnt: LDS [kPrepRounds * 4].  Returns how many are on; pos[r]: place of this thread's item among them.
+LCE_DEV int compact_256(const bool (&on)[kPrepRounds], int rounds, int (&pos)[kPrepRounds], int* cnt) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r) {
+    if (r >= rounds) break;
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(on[r]);
+    pos[r] = (int)__popcll(m & ((1ull << lane) - 1ull));
+    if (lane == 0) cnt[r * 4 + wave] = (int)__popcll(m);
+  }
+  __syncthreads();
+  int run = 0;
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r) {
+    if (r >= rounds) break;
+    const int c0 = cnt[r * 4], c1 = cnt[r * 4 + 1], c2 = cnt[r * 4 + 2], c3 = cnt[r * 4 + 3];
+    pos[r] += run + (wave > 0 ? c0 : 0) + (wave > 1 ? c1 : 0) + (wave > 2 ? c2 : 0);
+    run += c0 + c1 + c2 + c3;
+  }
+  return run;
+}
+
+// Every workgroup lists the tokens itself; workgroup 0 stores the list.  PER = 4: a wave owns compact position
+// 4 * blockIdx + wave; PER = 1: the workgroup owns position blockIdx (more workgroups where there are few positions).  A
+// position is the row of hidden copied to Ht (zeros from the list's end up to the next multiple of 64, the K granule of the
+// d_weight product, and to 128, lce_dw16_kernel wants two slabs), the token's label coefficient, its label and its constants.
+// Grid: positions up to the padded tokens.  a.coef may be null (no coefficients wanted).
+template <typename T, int PER>
+__global__ __launch_bounds__(256) void token_prep_kernel(CoefArgs<T> a, LabelTerm lt, T* Ht, int64_t ldHt, TokenPrep p) {
   static_assert(sizeof(T) == 2, "16-bit inputs");
   typedef typename VecOf<T, 8>::type vec_t;
-  __shared__ int list[128];
-  __shared__ int cnt[2];
+  __shared__ int list[kPrepTokens];
+  __shared__ int cnt[kPrepRounds * 4];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  bool on = false;
-  int before = 0;
-  if (wave < 2) {
-    on = tid < a.ntok && token_is_active(a.g_lp, a.g_stride, a.g_ent, tid);
-    const unsigned long long m = __builtin_amdgcn_ballot_w64(on);
-    before = (int)__popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) cnt[wave] = (int)__popcll(m);
+  const int rounds = (int)((a.ntok + 255) / 256);
+  bool on[kPrepRounds];
+  int pos[kPrepRounds];
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r) {
+    const int64_t t = r * 256 + tid;
+    on[r] = t < a.ntok && token_is_active(a.g_lp, a.g_stride, a.g_ent, t);
   }
-  __syncthreads();
-  const int n = cnt[0] + cnt[1];
-  if (wave < 2) {
-    const int pos = (wave ? cnt[0] : 0) + before;
-    if (on) list[pos] = tid;
-    if (blockIdx.x == 0 && tid < a.ntok) {
-      inv[tid] = on ? pos : -1;
-      if (on) rows[pos] = tid;
-      else if (a.coef) a.coef[tid] = 0.f;
+  const int n = compact_256(on, rounds, pos, cnt);
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r) {
+    const int t = r * 256 + tid;
+    if (on[r]) list[pos[r]] = t;
+    if (blockIdx.x == 0 && t < a.ntok) {
+      p.inv[t] = on[r] ? pos[r] : -1;
+      if (on[r]) p.rows[pos[r]] = t;
+      else if (a.coef) a.coef[t] = 0.f;
     }
   }
-  if (blockIdx.x == 0 && tid == 0) *n_rows = n;
+  if (blockIdx.x == 0 && tid == 0) *p.n_rows = n;
   __syncthreads();
-  const int k = blockIdx.x;
-  const int64_t rend = ((int64_t)n + 63) / 64 * 64 < rpad ? ((int64_t)n + 63) / 64 * 64 : rpad;
-  if (k >= rend) return;
+  const int k = PER == 4 ? blockIdx.x * 4 + wave : blockIdx.x;
   const int64_t tok = k < n ? list[k] : -1;
-  for (int64_t c = (int64_t)tid * 8; c < a.H; c += 256 * 8) {
+  const bool first = PER == 4 || wave == 0;  // the wave that works for the position as a whole
+  if (p.tokc && first && lane == 0 && k < p.tpad) token_consts_at(p.tokc, p.tokl, k, tok, a.g_lp, a.g_stride, a.g_scale, a.g_ent, a.maximum,
+                                                                   a.accumulate, a.entropy_b, a.labels, a.v0, a.V, a.rcp_tau);
+  const int64_t rk = n > 0 && n <= 64 ? 128 : ((int64_t)n + 63) / 64 * 64;
+  if (k >= (rk < p.rpad ? rk : p.rpad)) return;
+  for (int64_t c = (int64_t)(PER == 4 ? lane : tid) * 8; c < a.H; c += (PER == 4 ? 64 : 256) * 8) {
     vec_t v;
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (T)0.f;
     if (tok >= 0) v = *reinterpret_cast<const vec_t*>(a.h + tok * a.ldh + c);
     *reinterpret_cast<vec_t*>(Ht + (int64_t)k * ldHt + c) = v;
   }
-  if (tok >= 0 && a.coef && wave == 0) {
-    const float out = label_coef_wave(a, tok);
-    if (lane == 0) a.coef[tok] = out;
+  if (tok >= 0 && first) {
+    float G = 0.f;
+    if (a.coef) {
+      G = label_coef_wave(a, tok);
+      if (lane == 0) a.coef[tok] = G;
+    } else if (p.keys) {
+      G = lt.g_lp[tok * lt.g_stride] * lt.scale;
+    }
+    const int64_t y = a.labels[tok] - a.v0;
+    if (p.keys && lane == 0) p.keys[k] = (G != 0.f && y >= 0 && y < a.V) ? (uint32_t)y : kNoRow;  // (label_row)
   }
 }
 
@@ -361,33 +338,36 @@ __global__ __launch_bounds__(256) void few_prep_kernel(CoefArgs<T> a, T* Ht, int
 // i of the token list; the first position of each label adds sum of G_t * hidden[t][:] over the positions with that
 // label, in order, to the label's row of d_weight (as dw_label_rows_kernel does over a sorted run).
 template <typename T, typename TOUT>
-__global__ __launch_bounds__(256) void few_finish_kernel(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H,
-                                                         TOUT* d_hidden, LabelTerm lt, const T* W, int64_t ldw, int n_dh, const int* rows,
-                                                         const int* n_rows, const T* h, int64_t ldh, TOUT* dW) {
+__global__ __launch_bounds__(256) void token_finish_kernel(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H,
+                                                           TOUT* d_hidden, LabelTerm lt, const T* W, int64_t ldw, int n_dh, const int* rows,
+                                                           const int* n_rows, const uint32_t* keys, const T* h, int64_t ldh, TOUT* dW) {
   if ((int)blockIdx.x < n_dh) {
     dh_finish_body<T, TOUT>(part, S, stride, inv, ntok, H, d_hidden, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)n_dh);
     return;
   }
   constexpr int N = 16 / (int)sizeof(T);
   typedef typename VecOf<T, N>::type vec_t;
-  __shared__ uint32_t keys[128];
-  __shared__ float coefs[128];
-  __shared__ int toks[128];
+  __shared__ int cnt[kPrepRounds * 4];
+  __shared__ int at[kPrepTokens];  // the positions with this label, in order
   const int i = (int)blockIdx.x - n_dh, tid = threadIdx.x;
   const int n = *n_rows;
   if (i >= n) return;
-  if (tid < n && tid < 128) {
-    const int tok = rows[tid];
-    float G;
-    keys[tid] = label_row(lt, tok, G);
-    coefs[tid] = G;
-    toks[tid] = tok;
-  }
-  __syncthreads();
   const uint32_t key = keys[i];
   if (key == kNoRow) return;
-  for (int j = 0; j < i; ++j)
-    if (keys[j] == key) return;  // (the same for every thread) an earlier position owns this row
+  const int rounds = (n + 255) / 256;
+  bool on[kPrepRounds];
+  int pos[kPrepRounds];
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r) {
+    const int j = r * 256 + tid;
+    on[r] = j < n && keys[j] == key;
+  }
+  const int m = compact_256(on, rounds, pos, cnt);
+#pragma unroll
+  for (int r = 0; r < kPrepRounds; ++r)
+    if (on[r]) at[pos[r]] = r * 256 + tid;
+  __syncthreads();
+  if (at[0] != i) return;  // (the same for every thread) an earlier position owns this row
   TOUT* row = dW + (int64_t)key * H;
   for (int64_t c = (int64_t)tid * N; c < H; c += 256 * N) {
     typedef typename VecOf<TOUT, N>::type ovec_t;
@@ -395,10 +375,10 @@ __global__ __launch_bounds__(256) void few_finish_kernel(const float* part, int 
     float acc[N];
 #pragma unroll
     for (int e = 0; e < N; ++e) acc[e] = 0.f;
-    for (int j = i; j < n; ++j) {
-      if (keys[j] != key) continue;
-      const float G = coefs[j];
-      const vec_t hv = *reinterpret_cast<const vec_t*>(h + (int64_t)toks[j] * ldh + c);
+    for (int q = 0; q < m; ++q) {
+      const int64_t tok = rows[at[q]];
+      const float G = lt.g_lp[tok * lt.g_stride] * lt.scale;
+      const vec_t hv = *reinterpret_cast<const vec_t*>(h + tok * ldh + c);
 #pragma unroll
       for (int e = 0; e < N; ++e) acc[e] = __builtin_fmaf(G, (float)hv[e], acc[e]);
     }

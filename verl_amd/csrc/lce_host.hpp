@@ -686,16 +686,26 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
   ca.coef = with_coef ? reinterpret_cast<float*>(ws + L.off_coef) : nullptr;
   if (L.sort_items) lt.labels = labels;
   if (with_coef) { lt.g_lp = ca.coef; lt.g_stride = 1; lt.scale = 1.0f; }
-  // few tokens: the token list, the label coefficients and the compact copy of hidden come from one launch, and the
-  // one-hot rows of d_weight need no sorted list (few_finish_kernel at the end)
-  const bool few_prep = L.few && compact;
-  if (few_prep) {
+  f32x4_t* tokc = nullptr;
+  int* tokl = nullptr;
+  if constexpr (Cfg::CORE16) {
+    tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
+    tokl = reinterpret_cast<int*>(ws + L.off_tokl);
+  }
+  // up to kPrepTokens tokens one launch makes everything the passes below need to know about the tokens, and the one-hot
+  // rows of d_weight need no sorted list (token_finish_kernel at the end)
+  const bool one_prep = compact && L.tn && T <= kPrepTokens;
+  if (one_prep) {
     if constexpr (sizeof(TIN) == 2) {
       ProfScope prof(PC_ACTIVE_ROWS, st);
-      const int64_t r64 = round_up(T, 64);
-      hipLaunchKernelGGL(few_prep_kernel<TIN>, dim3((unsigned)(r64 < L.tpad ? r64 : L.tpad)), dim3(256), 0, st, ca, Ht, L.ldHt, L.tpad, rows,
-                         inv, n_rows);
-      if ((rc = check_launch("few_prep_kernel"))) return rc;
+      TokenPrep tp;
+      tp.rpad = tp.tpad = L.tpad; tp.rows = rows; tp.inv = inv; tp.n_rows = n_rows;
+      tp.keys = L.sort_items && need_dw ? skeys[0] : nullptr;
+      tp.tokc = tokc; tp.tokl = tokl;
+      const int64_t r64 = round_up(T, 64), positions = tokc || L.tpad < r64 ? L.tpad : r64;
+      if (T <= 512) hipLaunchKernelGGL((token_prep_kernel<TIN, 1>), dim3((unsigned)positions), dim3(256), 0, st, ca, lt, Ht, L.ldHt, tp);
+      else hipLaunchKernelGGL((token_prep_kernel<TIN, 4>), dim3((unsigned)((positions + 3) / 4)), dim3(256), 0, st, ca, lt, Ht, L.ldHt, tp);
+      if ((rc = check_launch("token_prep_kernel"))) return rc;
     }
   } else if (compact) {
     ProfScope prof(PC_ACTIVE_ROWS, st);
@@ -706,7 +716,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     hipLaunchKernelGGL(active_rows_kernel, dim3(nblk), dim3(256), 0, st, dlogprobs, ca.g_stride, dentropy, T, acounts, rows, inv, n_rows);
     if ((rc = check_launch("active_rows_kernel"))) return rc;
   }
-  if (L.sort_items && !few_prep) {
+  if (L.sort_items && !one_prep) {
     ProfScope prof(PC_LABEL_ROWS, st);
     if constexpr (sizeof(TIN) == 2) if (with_coef) {
       hipLaunchKernelGGL(label_coef_kernel<TIN>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, ca);
@@ -715,10 +725,6 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     const int nblocks = L.sort_items / kSortBlock;
     if (!need_dw) {
       // (the tokens grouped by label serve the one-hot rows of d_weight only)
-    } else if (nblocks == 1) {
-      hipLaunchKernelGGL(label_sort_single_kernel, dim3(1), dim3(256), 0, st, lt, rows, n_rows, T, L.sort_passes, skeys[0], svals[0],
-                         skeys[1], svals[1]);
-      if ((rc = check_launch("label_sort_single_kernel"))) return rc;
     } else {
       int* hist = reinterpret_cast<int*>(ws + L.off_hist);
       hipLaunchKernelGGL(label_keys_kernel, dim3(L.sort_items / 256), dim3(256), 0, st, lt, rows, n_rows, T, L.sort_items, skeys[0], svals[0]);
@@ -733,11 +739,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       }
     }
   }
-  f32x4_t* tokc = nullptr;
-  int* tokl = nullptr;
-  if constexpr (Cfg::CORE16) {
-    tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
-    tokl = reinterpret_cast<int*>(ws + L.off_tokl);
+  if (tokc && !one_prep) {
     ProfScope prof(PC_ACTIVE_ROWS, st);
     hipLaunchKernelGGL(ds_token_consts_kernel, dim3((unsigned)((L.tpad + 255) / 256)), dim3(256), 0, st, rows, n_rows, T, L.tpad, dlogprobs,
                        (int64_t)(reduction == LCE_REDUCTION_NONE ? 1 : 0), reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f,
@@ -746,8 +748,8 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
   }
   // second operand of the d_weight GEMM (W^T for d_hidden follows chunk by chunk): the listed rows of hidden,
   // as they are (K-major, for the transposing reads), or transposed to h^T [H][T]
-  if (few_prep) {
-    // (few_prep_kernel has written the compact copy)
+  if (one_prep) {
+    // (token_prep_kernel has written the compact copy)
   } else if (L.tn) {
     ProfScope prof(PC_TRANSPOSE, st);
     hipLaunchKernelGGL(gather_rows_kernel<TIN>, dim3(2048), dim3(256), 0, st, h, ldh, T, H, Ht, L.ldHt, L.tpad, rows, n_rows);
@@ -956,21 +958,22 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     launch_chunk(p);
     if ((rc = check_launch("lce_bwd_chunk_kernel"))) return rc;
   }
-  if (few_prep) {
+  if (one_prep) {
     // d_hidden and the one-hot rows of d_weight (every row holds its softmax terms by now), one launch
     if constexpr (sizeof(TIN) == 2) {
       ProfScope prof(PC_DH_FINISH, st);
-      const int n_dh = need_dh ? (int)((T * (H / 4) + 255) / 256) : 0;
+      const int64_t dh_blocks = (T * (H / 4) + 255) / 256;
+      const int n_dh = need_dh ? (int)(dh_blocks < 8192 ? dh_blocks : 8192) : 0;
       const int n_lr = (L.sort_items && need_dw) ? (int)T : 0;
       const int64_t part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
       if (n_dh + n_lr > 0) {
         if (grads_f32)
-          hipLaunchKernelGGL((few_finish_kernel<TIN, float>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
-                             T, H, static_cast<float*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, h, ldh, static_cast<float*>(d_weight));
+          hipLaunchKernelGGL((token_finish_kernel<TIN, float>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
+                             T, H, static_cast<float*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<float*>(d_weight));
         else
-          hipLaunchKernelGGL((few_finish_kernel<TIN, TIN>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
-                             T, H, static_cast<TIN*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, h, ldh, static_cast<TIN*>(d_weight));
-        if ((rc = check_launch("few_finish_kernel"))) return rc;
+          hipLaunchKernelGGL((token_finish_kernel<TIN, TIN>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
+                             T, H, static_cast<TIN*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<TIN*>(d_weight));
+        if ((rc = check_launch("token_finish_kernel"))) return rc;
       }
     }
     return LCE_OK;

@@ -481,6 +481,28 @@ LCE_DEV TokenConsts token_consts(float glp, float gent, float maximum, float acc
   return k;
 }
 
+// the constants and the label of compact position pos, which holds token tok (or none: -1), as the 16x16x32 d_logits tiles read
+// them (DsArgs::tokc, tokl)
+LCE_DEV void token_consts_at(f32x4_t* tokc, int* tokl, int64_t pos, int64_t tok, const float* g_lp, int64_t g_lp_stride, float g_lp_scale,
+                             const float* g_ent, const float* maximum, const float* accumulate, const float* entropy_b, const int64_t* labels,
+                             int64_t vocab_offset, int64_t V, float rcp_tau) {
+  f32x4_t c = {1.0e30f, 0.f, 0.f, 0.f};
+  int lab = -1;
+  if (tok >= 0) {
+    const float glp = g_lp[tok * g_lp_stride] * g_lp_scale;
+    const float gent = g_ent ? g_ent[tok] : 0.f;
+    const TokenConsts k = token_consts(glp, gent, maximum[tok], accumulate[tok], entropy_b[tok], rcp_tau);
+    c[0] = k.lse2;
+    c[1] = k.C0;
+    c[2] = k.C1;
+    c[3] = k.G;
+    const int64_t y = labels[tok] - vocab_offset;
+    lab = (y >= 0 && y < V) ? (int)y : -1;
+  }
+  tokc[pos] = c;
+  tokl[pos] = lab;
+}
+
 // d_logits of one accumulator element; SLOW adds the label one-hot and masks padded rows / tokens
 // (drop: the label's entry is not part of the tile at all, it is added elsewhere in fp32)
 template <bool SLOW>

@@ -209,22 +209,8 @@ inline __global__ void ds_token_consts_kernel(const int* rows, const int* n_rows
   const int64_t pos = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (pos >= tpad) return;
   const int64_t Tc = n_rows ? (int64_t)*n_rows : T;
-  f32x4_t c = {1.0e30f, 0.f, 0.f, 0.f};
-  int lab = -1;
-  if (pos < Tc) {
-    const int64_t tok = rows ? (int64_t)rows[pos] : pos;
-    const float glp = g_lp[tok * g_lp_stride] * g_lp_scale;
-    const float gent = g_ent ? g_ent[tok] : 0.f;
-    const TokenConsts k = token_consts(glp, gent, maximum[tok], accumulate[tok], entropy_b[tok], rcp_tau);
-    c[0] = k.lse2;
-    c[1] = k.C0;
-    c[2] = k.C1;
-    c[3] = k.G;
-    const int64_t y = labels[tok] - vocab_offset;
-    lab = (y >= 0 && y < V) ? (int)y : -1;
-  }
-  tokc[pos] = c;
-  tokl[pos] = lab;
+  token_consts_at(tokc, tokl, pos, pos < Tc ? (rows ? (int64_t)rows[pos] : pos) : -1, g_lp, g_lp_stride, g_lp_scale, g_ent, maximum, accumulate,
+                  entropy_b, labels, vocab_offset, V, rcp_tau);
 }
 
 // One finished tile: d_logits of the wave's 128 tokens x 128 vocabulary entries, written to dS straight from the
