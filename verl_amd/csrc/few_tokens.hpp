@@ -530,56 +530,67 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 // d_logits tiles compute from their accumulators, here from the kept x(t, v), element by element with the same
 // expressions, so the same bits.  One pass over 4 bytes per logit instead of a pass over W.  Workgroup b owns the 64
 // columns [64 b, 64 b + 64) of dS, which lie within one group of the vocabulary order Perm (a whole group of the
-// eight-wave tiles' order, half a group of the 16x16x32 tiles'), and the first `nrows` compact token positions: rows
-// beyond the tokens that take part and columns beyond the chunk's rows (the grid covers whole 256-row tiles) are
-// written as zeros, as the tiles write them.  Eight lanes share a position: they read the 256 bytes of its token's
-// logits behind the 64 columns and write 128 bytes of dS.
+// eight-wave tiles' order, half a group of the 16x16x32 tiles'), and the first `nrows` compact token positions, of which it
+// writes as many as a reader takes: up to the tokens that take part, rounded up to the d_weight product's K granule (64, and
+// two slabs at least).  Positions beyond the tokens and columns beyond the chunk's rows (the grid covers whole 256-row
+// tiles) are written as zeros, as the tiles write them.  Eight lanes share a position: they read the 256 bytes of its
+// token's logits behind the 64 columns and write 128 bytes of dS.  Bound by HBM; the constants come from the per-position
+// table (worked out per workgroup they were six dependent loads and a logarithm per position) and four positions are on
+// their way at once.
 // p: the chunk's DsArgs (W, h, the tile map and the range are not used); x: the kept logits from the chunk's first row
 // on (a multiple of 16), of xtok tokens.
 // ------------------------------------------------------------------------------------------------------------------
 template <typename TIN, typename Perm>
 __global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t xtok, int nrows) {
   static_assert(sizeof(TIN) == 2 && Perm::GV % 64 == 0, "16-bit d_logits, groups of the vocabulary order in multiples of 64 rows");
+  constexpr int U = 4;
   const int tid = threadIdx.x, c = tid & 7;
   const int64_t u0 = (int64_t)blockIdx.x * 64;   // first of this workgroup's 64 columns of dS
   const int64_t g0 = u0 - u0 % Perm::GV;         // first row (= first column) of their group of the vocabulary order
-  const int64_t Tc = p.n_rows ? (int64_t)*p.n_rows : p.T;
-  for (int pos = tid >> 3; pos < nrows; pos += 32) {
-    float lse2 = 0.f, C0 = 0.f, C1 = 0.f, G = 0.f;
-    int64_t tok = -1;
-    int rel = -1;
-    if (pos < Tc) {
-      tok = p.rows ? (int64_t)p.rows[pos] : pos;
-      const float glp = p.g_lp[tok * p.g_lp_stride] * p.g_lp_scale;
-      const float gent = p.g_ent ? p.g_ent[tok] : 0.f;
-      const TokenConsts k = token_consts(glp, gent, p.maximum[tok], p.accumulate[tok], p.entropy_b[tok], p.rcp_tau);
-      lse2 = k.lse2; G = k.G; C1 = k.C1; C0 = k.C0;
-      const int64_t y = p.labels[tok] - p.v0;
-      rel = (p.label_outside != 1 && y >= g0 && y < g0 + Perm::GV) ? (int)(y - g0) : -1;
+  const int Tc = (int)(p.n_rows ? (int64_t)*p.n_rows : p.T);
+  const int used = Tc <= 64 ? 128 : (Tc + 63) / 64 * 64, end = used < nrows ? used : nrows;
+  // columns c * 8 + (0..3) and c * 8 + (4..7) of the workgroup's 64 are two runs of four consecutive vocabulary rows
+  // (both orders Perm keep what one lane of a d_logits tile holds together: four consecutive rows per register quad),
+  // and the cache is padded to whole groups, so each run is one aligned 16-byte load
+  int r0[2];  // vocabulary row relative to the group's first
+  bool live[2];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    r0[hf] = (int)(Perm::vocab_at(u0 + c * 8 + 4 * hf) - g0);
+    live[hf] = g0 + r0[hf] < p.vrows;
+  }
+  for (int base = tid >> 3; base < end; base += 32 * U) {
+    int tok[U];
+    f32x4_t k[U], v[U][2];
+    int rel[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int pos = base + 32 * u;
+      const bool on = pos < Tc;
+      tok[u] = on ? (p.rows ? p.rows[pos] : pos) : -1;
+      k[u] = on ? p.tokc[pos] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const int y = on ? p.tokl[pos] : -1;
+      rel[u] = (p.label_outside != 1 && y >= p.lab0 + g0 && y < p.lab0 + g0 + Perm::GV) ? (int)(y - p.lab0 - g0) : -1;
     }
-    // columns c * 8 + (0..3) and c * 8 + (4..7) of the workgroup's 64 are two runs of four consecutive vocabulary rows
-    // (both orders Perm keep what one lane of a d_logits tile holds together: four consecutive rows per register quad),
-    // and the cache is padded to whole groups, so each run is one aligned 16-byte load
-    float xv[8];
-    int row[8];  // vocabulary row relative to the group's first
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const int r0 = (int)(Perm::vocab_at(u0 + c * 8 + 4 * hf) - g0);
-      f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-      if (tok >= 0 && g0 + r0 < p.vrows) v = *reinterpret_cast<const f32x4_t*>(kept_logit(x, xtok, tok, g0 + r0));
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        row[4 * hf + e] = r0 + e;
-        xv[4 * hf + e] = v[e];
+      for (int hf = 0; hf < 2; ++hf) {
+        v[u][hf] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (tok[u] >= 0 && live[hf]) v[u][hf] = load_vec<true>(reinterpret_cast<const f32x4_t*>(kept_logit(x, xtok, tok[u], g0 + r0[hf])));
       }
-    }
-    float d[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bool dead = tok < 0 || g0 + row[e] >= p.vrows;
-      d[e] = dlogit<true>(dead ? 0.f : xv[e], p.c, lse2, C0, C1, G, row[e] == rel, dead, p.label_outside == 2);
+    for (int u = 0; u < U; ++u) {
+      const int pos = base + 32 * u;
+      float d[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int row = r0[e >> 2] + (e & 3);
+        const bool dead = tok[u] < 0 || g0 + row >= p.vrows;
+        d[e] = dlogit<true>(dead ? 0.f : v[u][e >> 2][e & 3], p.c, k[u][0], k[u][1], k[u][2], k[u][3], row == rel[u], dead, p.label_outside == 2);
+      }
+      if (pos < end) store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, pos, u0 + c * 8), d);
     }
-    store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, pos, u0 + c * 8), d);
   }
 }
 

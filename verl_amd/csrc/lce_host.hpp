@@ -688,7 +688,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
   if (with_coef) { lt.g_lp = ca.coef; lt.g_stride = 1; lt.scale = 1.0f; }
   f32x4_t* tokc = nullptr;
   int* tokl = nullptr;
-  if constexpr (Cfg::CORE16) {
+  if (Cfg::CORE16 || (sizeof(TIN) == 2 && xcache)) {
     tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
     tokl = reinterpret_cast<int*>(ws + L.off_tokl);
   }
