@@ -263,6 +263,11 @@ typedef struct {
   float kl_coef, clip_low, clip_high, clip_c, entropy_coeff, dp_size, batch_num_tokens, global_batch_size, loss_scale_factor;
 } lce_ppo_call_t;
 int lce_ppo_forward(lce_ppo_call_t* call, void* stream);
+/* lce_ppo_forward in two halves, for a caller with work of its own to do before it needs the checks: _begin returns when
+ * everything is launched and leaves a ticket (NULL unless packed), _end waits, fills in checks and takes the ticket back.
+ * Every ticket goes to _end exactly once, with the call and the stream of its _begin. */
+int lce_ppo_forward_begin(lce_ppo_call_t* call, void* stream, void** ticket);
+int lce_ppo_forward_end(lce_ppo_call_t* call, void* stream, void* ticket);
 int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
 
 /* Product-level options (process-wide; every entry point works from one snapshot of the settings taken when it starts).

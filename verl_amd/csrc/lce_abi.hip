@@ -715,7 +715,9 @@ static int ppo_call_plan(const lce_ppo_call_t* call, PpoPlan* plan) {
   return LCE_OK;
 }
 
-int lce_ppo_forward(lce_ppo_call_t* call, void* stream) {
+int lce_ppo_forward_begin(lce_ppo_call_t* call, void* stream, void** ticket) {
+  if (!ticket) return fail(LCE_E_ARG, "null pointer");
+  *ticket = nullptr;
   PpoPlan plan;
   int rc = ppo_call_plan(call, &plan);
   if (rc) return rc;
@@ -755,10 +757,27 @@ int lce_ppo_forward(lce_ppo_call_t* call, void* stream) {
   plan.p.check_seq = slot.seq;
   rc = ppo_launch_forward(plan, st);
   // (a failed launch may still leave a kernel on its way that writes the slot: it is left alone, not reused)
-  if (rc || (rc = wait_slot(slot, st))) return rc;
+  if (rc) return rc;
+  *ticket = new HostSlot(slot);
+  return LCE_OK;
+}
+
+int lce_ppo_forward_end(lce_ppo_call_t* call, void* stream, void* ticket) {
+  if (!call) return fail(LCE_E_ARG, "null call");
+  if (!ticket) return LCE_OK;
+  const HostSlot slot = *static_cast<HostSlot*>(ticket);
+  delete static_cast<HostSlot*>(ticket);
+  const int rc = wait_slot(slot, reinterpret_cast<hipStream_t>(stream));
+  if (rc) return rc;  // (the slot is left alone: see above)
   for (int k = 0; k < 3; ++k) call->checks[k] = slot.host[k];
   give_slot(slot);
   return LCE_OK;
+}
+
+int lce_ppo_forward(lce_ppo_call_t* call, void* stream) {
+  void* ticket = nullptr;
+  const int rc = lce_ppo_forward_begin(call, stream, &ticket);
+  return rc ? rc : lce_ppo_forward_end(call, stream, ticket);
 }
 
 int lce_ppo_backward(const lce_ppo_call_t* call, void* stream) {

@@ -73,12 +73,26 @@ class _Packed:
     """Packed model outputs: where the lengths of prompts and responses come from.  Either both vectors, or the attention
     mask of a padded batch (its first ``prompt_width`` columns are the prompts'), from which the kernel counts them."""
 
-    __slots__ = ("prompt_lens", "response_lens", "attention_mask", "prompt_width", "checks")
+    __slots__ = ("prompt_lens", "response_lens", "attention_mask", "prompt_width", "_pending")
 
     def __init__(self, prompt_lens=None, response_lens=None, attention_mask=None, prompt_width=0):
         self.prompt_lens, self.response_lens = prompt_lens, response_lens
         self.attention_mask, self.prompt_width = attention_mask, prompt_width
-        self.checks = None  # (sum of all lengths, prompts of length 0, longest response), filled in by the forward
+        self._pending = None  # (call, stream, ticket) of the forward
+
+    def launched(self, call, stream, ticket):
+        self._pending = (call, stream, ticket)
+
+    def checks(self):
+        """(sum of all lengths, prompts of length 0, longest response) of the forward that has been launched: waits for the
+        kernel that adds them up.  Once per forward, whatever happens in between."""
+        (call, stream, ticket), self._pending = self._pending, None
+        _abi.check(_abi.load().lce_ppo_forward_end(ctypes.addressof(call), stream, ticket), "lce_ppo_forward_end")
+        return tuple(call.checks)
+
+    def __del__(self):
+        if self._pending is not None:  # (an exception kept the caller from asking)
+            self.checks()
 
 
 class _FusedPPOLoss(torch.autograd.Function):
@@ -144,10 +158,15 @@ class _FusedPPOLoss(torch.autograd.Function):
             lens = (packed.prompt_lens, packed.response_lens)
             call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
         with _abi.on_device(dev):
-            _abi.check(lib.lce_ppo_forward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_forward")
-        if packed is not None:
-            packed.checks = tuple(call.checks)
+            stream = _abi.current_stream(dev)
+            if packed is None:
+                _abi.check(lib.lce_ppo_forward(ctypes.addressof(call), stream), "lce_ppo_forward")
+            else:
+                ticket = ctypes.c_void_p()
+                _abi.check(lib.lce_ppo_forward_begin(ctypes.addressof(call), stream, ctypes.addressof(ticket)), "lce_ppo_forward_begin")
+                packed.launched(call, stream, ticket)
         ctx.save_for_backward(keep, *lens)
+        ctx.set_materialize_grads(False)  # (the vector of statistics takes no gradient: no zeros are made for it)
         ctx.call, ctx.base = call, keep.data_ptr()
         ctx.like = tuple(None if t is None else (t.shape, t.dtype) for t in (log_prob, entropy))
         ctx.mark_non_differentiable(out)
@@ -155,6 +174,8 @@ class _FusedPPOLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_loss, _g_out):
+        if g_loss is None:
+            return (None,) * 15
         keep, *lens = ctx.saved_tensors
         dev = keep.device
         call = _abi.PpoCall.from_buffer_copy(ctx.call)
@@ -265,7 +286,7 @@ def fused_ppo_loss_packed(
     packed = _Packed(prompt_lens.to(dev, torch.int64).contiguous(), response_lens.to(dev, torch.int64).contiguous())
     result = fused_ppo_loss(log_prob, entropy, old_log_prob, advantages, response_mask, _packed=packed, **kwargs)
     # (the lengths are checked while the loss is on its way: the launches stay inside their buffers whatever they say)
-    _check_lengths(packed.checks, log_prob.numel(), response_mask.shape[1])
+    _check_lengths(packed.checks(), log_prob.numel(), response_mask.shape[1])
     return result
 
 
@@ -413,10 +434,6 @@ def ppo_loss(config, model_output, data, dp_group=None):
         kl_loss_type=_cfg(config, "kl_loss_type", "low_var_kl"),
         **info,
     )  # fmt: skip
-    longest = packed.checks[2]
-    if longest > width:
-        raise ValueError(f"max_response_len = {width} is shorter than the longest response ({longest})")
-    _check_lengths(packed.checks, log_prob.numel(), width)
     metrics = Metric.from_dict(
         {k: m[k] for k in ("actor/pg_clipfrac", "actor/ppo_kl", "actor/pg_clipfrac_lower")}, AggregationType.MEAN
     )
@@ -426,4 +443,10 @@ def ppo_loss(config, model_output, data, dp_group=None):
     if use_kl:
         metrics["kl_loss"] = Metric(metric_aggregation, m["kl_loss"])
         metrics["kl_coef"] = _cfg(config, "kl_loss_coef", 0.001)
+    # (last, with everything on the host done: the loss is on its way meanwhile)
+    checks = packed.checks()
+    longest = checks[2]
+    if longest > width:
+        raise ValueError(f"max_response_len = {width} is shorter than the longest response ({longest})")
+    _check_lengths(checks, log_prob.numel(), width)
     return policy_loss, metrics
