@@ -113,8 +113,10 @@ static void launch_logits_fwd(const void* logits, int64_t ldl, const int64_t* la
 
 template <typename TIN>
 static void launch_logits_bwd(const void* logits, int64_t ldl, const int64_t* labels, int64_t R, int64_t V, const float* stats, const void* glp,
-                              int glp_dtype, const void* gent, int gent_dtype, void* dl, int64_t ldd, int segs, hipStream_t st) {
+                              int glp_dtype, const void* gent, int gent_dtype, void* dl, int64_t ldd, hipStream_t st) {
   constexpr int NT = 512;
+  const int64_t part = logits_bwd_part<TIN>(NT) * 16 / (int64_t)sizeof(TIN), parts = (V + part - 1) / part;
+  const int segs = stats && R * parts <= 0x7fffffff ? (int)parts : 1;
   hipLaunchKernelGGL((logits_bwd_kernel<TIN, NT>), dim3((unsigned)(R * segs)), dim3(NT), 0, st, static_cast<const TIN*>(logits), ldl, labels, V,
                      stats, glp, glp_dtype, gent, gent_dtype, static_cast<TIN*>(dl), ldd, segs);
 }
@@ -831,15 +833,9 @@ int lce_logits_backward_as(const void* logits, int64_t ldl, const int64_t* label
   if (!logits || !d_logits || (dlogprobs && !labels)) return fail(LCE_E_ARG, "null pointer");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   ProfScope prof(PC_LOGITS_BWD, st);
-  // a CU takes four workgroups: below 1024 rows a row is shared out, as long as a part holds some trips of the loop
-  int segs = 1;
-  if (stats) {
-    const int64_t most = V / 16384 < 1 ? 1 : V / 16384, want = R < 1024 ? 1024 / R : 1;
-    segs = (int)(want < most ? want : most);
-  }
-  if (dtype == LCE_DTYPE_BF16) launch_logits_bwd<bf16_t>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, segs, st);
-  else if (dtype == LCE_DTYPE_F16) launch_logits_bwd<f16_t>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, segs, st);
-  else launch_logits_bwd<float>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, segs, st);
+  if (dtype == LCE_DTYPE_BF16) launch_logits_bwd<bf16_t>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, st);
+  else if (dtype == LCE_DTYPE_F16) launch_logits_bwd<f16_t>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, st);
+  else launch_logits_bwd<float>(logits, ldl, labels, R, V, stats, dlogprobs, dlogprobs_dtype, dentropy, dentropy_dtype, d_logits, ldd, st);
   return check_launch("logits_bwd_kernel");
 }
 
