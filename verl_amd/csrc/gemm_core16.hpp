@@ -350,10 +350,6 @@ struct GemmCore16 {
   LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
     const int nk = (int)(K / Cfg::BK) * Cfg::TERMS;
     const int64_t last = nk - 1;
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     wait_vm<HL + HLB>();  // slab 0 has landed
     __builtin_amdgcn_s_barrier();
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
@@ -362,19 +358,25 @@ struct GemmCore16 {
       read_frag<decltype(fc)::value, 0>(lds0 + (AE ? 0 : SLOT) + a_rd, lds0 + (AE ? SLOT : 0) + b_rd, af[0], bf[0]);
     });
     int se = 0;  // slot of this slab's early half; its late half is in the next slot
-    for (int it = 0; it < nk; ++it) {
+    auto slab = [&](auto first, int it) {
+      constexpr bool FIRST = decltype(first)::value;
       const int sl = se + 1 >= 5 ? se + 1 - 5 : se + 1;
       const int ne = se + 2 >= 5 ? se + 2 - 5 : se + 2;
       const int nl = se + 3 >= 5 ? se + 3 - 5 : se + 3;
       const int fr = se + 4 >= 5 ? se + 4 - 5 : se + 4;  // free slot: takes E(it+2)
       const int64_t ks = it + 2 < last ? it + 2 : last;
-      kstep<true, 1, !AE>(acc, af[0], bf[0], lds0 + (AE ? se : sl) * SLOT + a_rd, lds0 + (AE ? sl : se) * SLOT + b_rd, af[1], bf[1], lds, fr, ks);
+      kstep<true, 1, !AE, false, FIRST>(acc, af[0], bf[0], lds0 + (AE ? se : sl) * SLOT + a_rd, lds0 + (AE ? sl : se) * SLOT + b_rd, af[1], bf[1], lds,
+                                        fr, ks);
       wait_vm<AE ? HL : HLB>();  // slab it+1 has landed; E(it+2) may still be in flight
       wait_lgkm<0>();            // this wave's reads of slab it have returned
       __builtin_amdgcn_s_barrier();
       kstep<false, 0, AE>(acc, af[1], bf[1], lds0 + (AE ? ne : nl) * SLOT + a_rd, lds0 + (AE ? nl : ne) * SLOT + b_rd, af[0], bf[0], lds, se, ks);
       se = ne;
-    }
+    };
+    // (the first slab starts the accumulators: zeroing them beforehand takes 512 instructions and, while they are ordinary values
+    // to the compiler, the registers of everything else that lives across the loop)
+    slab(std::true_type{}, 0);
+    for (int it = 1; it < nk; ++it) slab(std::false_type{}, it);
     wait_vm<0>();    // drain the redundant tail fetches before LDS is reused
     wait_lgkm<0>();  // and the reads of the slab after the last
     retire(acc);
@@ -389,9 +391,16 @@ struct GemmCore16 {
   // distance to a read itself, and the matrix pipe orders it behind the assembly MFMA that wrote the same registers.
   static LCE_DEV void retire(f32x4_t (&acc)[NB][NBN]) {
     asm volatile("s_nop 15\n\ts_nop 7" ::);
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    stay(acc);
+  }
+
+  // The accumulators are in AGPRs at this point of the program (the compiler otherwise moves many of them into ordinary registers
+  // as soon as a loop ends, ahead of their use, and what lived there into scratch memory).
+  static LCE_DEV void stay(f32x4_t (&acc)[NB][NBN]) {
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) acc[NB - 1][j] = Mma16<TIN>::known(acc[NB - 1][j], zero, zero);
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NBN; ++j) asm volatile("" : "+a"(acc[i][j]));
   }
 
   // ---- a workgroup that walks tiles: the K loops of successive tiles as one stream of slabs -------------------

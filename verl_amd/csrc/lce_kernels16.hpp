@@ -32,19 +32,17 @@ struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS>> {
 // ------------------------------------------------------------------------------------------------
 // folds one finished tile into the running per-token statistics (FULL: no padded vocabulary rows in the tile)
 template <typename Cfg, bool FULL>
-LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], float (&m)[Cfg::NBN],
+LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], float (&m)[Cfg::NBN],
                         float (&a)[Cfg::NBN], float (&b)[Cfg::NBN], const int (&lab)[Cfg::NBN], int vbase, int vend, int64_t tok0, int g4,
                         int l16) {
   constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
-  // The running statistics do not live in registers across the K loop (256 accumulator and 256 ordinary registers are
-  // in use there; the compiler keeps them in scratch memory meanwhile).  All of them are asked for here, so that they
-  // come back in one batch of loads instead of column by column, each column waiting for its own (forward at 16384
-  // tokens: H=896 4.57 -> 4.43 ms, H=1536 6.39 -> 6.28, H=3584 12.91 -> 12.85).
-#pragma unroll
-  for (int j = 0; j < NBN; ++j) asm volatile("" : "+v"(m[j]), "+v"(a[j]), "+v"(b[j]));
 #pragma unroll
   for (int j = 0; j < NBN; ++j) {
-    __builtin_amdgcn_sched_barrier(0);  // one block column at a time (register pressure)
+    // One block column at a time (register pressure).  Its accumulators are in AGPRs up to here: the compiler otherwise reads
+    // all 256 of a lane ahead of the first column and keeps other values in scratch memory meanwhile.
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) asm volatile("" : "+a"(acc[i][j]));
     float x[NB * 4];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -75,6 +73,7 @@ LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, const f32x4_t (&acc
     const float aj = (a4[0] + a4[1]) + (a4[2] + a4[3]), bj = (b4[0] + b4[1]) + (b4[2] + b4[3]);
     a[j] = aj;
     b[j] = bj;
+    asm volatile("" : "+v"(m[j]), "+v"(a[j]), "+v"(b[j]));  // (this column is finished here, not after the branches below)
     // label logit: rare (a token's label falls in this wave tile with probability WM / V)
     const int rel = lab[j] - vbase;
     const bool mine = lab[j] >= 0 && lab[j] < vend && rel >= 0 && rel < Cfg::WM && (((rel >> 2) & 3) == g4);
