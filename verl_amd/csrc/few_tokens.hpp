@@ -50,17 +50,6 @@ LCE_DEV void mma16(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
 // into different banks (values below 16: valid for rows of 16 chunks and of 32)
 LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 
-// Buffer access to a run of memory: out-of-bounds lanes read zero and store nothing, so the loops below need no branch around
-// a load or a store, and the compiler can wait for exactly the operation it needs (behind a branch it does not know how many
-// younger ones are in flight and waits for all of them).
-typedef __amdgpu_buffer_rsrc_t buf_t;
-// (bytes below 4 GiB: 256 rows of an operand span less)
-LCE_DEV buf_t make_buf(const void* p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
-}
-constexpr int kBufNowhere = (int)0x80000000u;  // an offset beyond any of these buffers (at most 64 rows of 16 MiB)
-constexpr int kBufNonTemporal = 2;
-
 // ------------------------------------------------------------------------------------------------------------------
 // Forward, up to 64 tokens.  Workgroup = 512 threads = 8 waves, one per CU; it owns a contiguous range of vocabulary rows (the
 // same number for every workgroup) and goes through it in passes of 256 rows, for each of which K is streamed in stages of 64:

@@ -33,6 +33,17 @@ typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
 #define LCE_DEV __device__ __forceinline__
 
+// Buffer access to a run of memory: out-of-bounds lanes read zero and store nothing, so a loop needs no branch around
+// a load or a store, and the compiler can wait for exactly the operation it needs (behind a branch it does not know how many
+// younger ones are in flight and waits for all of them).
+typedef __amdgpu_buffer_rsrc_t buf_t;
+// (bytes below 4 GiB: 256 rows of an operand span less)
+LCE_DEV buf_t make_buf(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+constexpr int kBufNowhere = (int)0x80000000u;  // an offset beyond any buffer it is used with (those span less than 2 GiB)
+constexpr int kBufNonTemporal = 2;
+
 typedef const void __attribute__((address_space(1))) * gptr_t;
 typedef void __attribute__((address_space(3))) * lptr_t;
 

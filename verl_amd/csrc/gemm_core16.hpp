@@ -403,6 +403,13 @@ struct GemmCore16 {
       for (int j = 0; j < NBN; ++j) asm volatile("" : "+a"(acc[i][j]));
   }
 
+  // the same for one block column, where the epilogues begin with it
+  static LCE_DEV void stay_column(f32x4_t (&acc)[NB][NBN], int j) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) asm volatile("" : "+a"(acc[i][j]));
+  }
+
   // ---- a workgroup that walks tiles: the K loops of successive tiles as one stream of slabs -------------------
   // The loads two slabs ahead of the end of a tile are those of the next tile's first slabs, and the fragments that the last
   // k-step reads are the next tile's first: between two tiles there is neither a drain nor a first load to wait for.

@@ -40,9 +40,7 @@ LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg:
   for (int j = 0; j < NBN; ++j) {
     // One block column at a time (register pressure).  Its accumulators are in AGPRs up to here: the compiler otherwise reads
     // all 256 of a lane ahead of the first column and keeps other values in scratch memory meanwhile.
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) asm volatile("" : "+a"(acc[i][j]));
+    GemmCore16<Cfg>::stay_column(acc, j);
     float x[NB * 4];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -129,27 +127,20 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
       // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are
       // issued 16 at a time and so many are waited for that, with the prologue's 32 loads behind them, fewer than 64
       // operations are ever in flight.
-      __builtin_amdgcn_sched_barrier(0);
+      const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
+      // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
+      const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
+      const int row_at = g4 * 16, panel = (int)p.T * 64;
 #pragma unroll
       for (int j = 0; j < NBN; ++j) {
-        const int64_t t = n0 + g.wave_n * Cfg::WN + j * 16 + l16;
-        if (t < p.T) {
+        GemmCore16<Cfg>::stay_column(acc, j);
+        const int at = t0 + j * 16 < p.T ? (int)(t0 + j * 16) * 64 + row_at : kBufNowhere;
 #pragma unroll
-          for (int i = 0; i < NB; ++i) {
-            const int v = vbase + 16 * i + 4 * g4;
-            if (v + 3 < vend) {
-              *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = acc[i][j];
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (v + r < vend) *kept_logit(p.xcache, p.T, t, v + r) = acc[i][j][r];
-            }
-          }
+        for (int i = 0; i < NB; ++i) {
+          const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, 0);
         }
-        if (!full) {  // (a tile at the end of its split: up to four single stores per block)
-          __builtin_amdgcn_sched_barrier(0);
-          GemmCore16<Cfg>::template wait_vm<0>();
-        } else if (j % 2 == 1 && j >= 3) {
+        if (j % 2 == 1 && j >= 3) {
           __builtin_amdgcn_sched_barrier(0);
           if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<24>();
           else GemmCore16<Cfg>::template wait_vm<32>();
@@ -220,12 +211,13 @@ inline __global__ void ds_token_consts_kernel(const int* rows, const int* n_rows
 // it after the common arithmetic (zero when the label's entry is kept out of the tiles, + G when everything is inside).
 // EDGE: the tile reaches beyond the chunk's last row; those entries are zeros.
 template <typename Cfg, bool LABEL, bool EDGE>
-LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], const f32x4_t (&tc)[Cfg::NBN],
+LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], const f32x4_t (&tc)[Cfg::NBN],
                            const int (&lab)[Cfg::NBN], int64_t tok0, int vloc0, int g4, int l16) {
   typedef typename Cfg::TIN TIN;
   constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
 #pragma unroll
   for (int j = 0; j < NBN; ++j) {
+    GemmCore16<Cfg>::stay_column(acc, j);  // (one block column at a time, as in fwd16_fold)
     const float lse2 = tc[j][0], C0 = tc[j][1], C1 = tc[j][2], G = tc[j][3];
     // the label's entry: block pair rel / 32, lane group (rel / 4) % 4, value 4 ((rel / 16) % 2) + rel % 4 of the run
     const int rel = (LABEL && p.label_outside != 1) ? lab[j] - (int)p.lab0 - vloc0 : -1;  // (1: the tiles hold the softmax terms only)
@@ -257,12 +249,12 @@ LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, const f32x4_t (&a
         for (int q = 0; q < 8; ++q) rest[q] = d[q];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-          if (tok < p.tpad) store_run<TIN, 8>(dst + t * p.dS_plane, rest);
+          store_run<TIN, 8>(dst + t * p.dS_plane, rest);
 #pragma unroll
           for (int q = 0; q < 8; ++q) rest[q] -= (float)(TIN)rest[q];
         }
       } else {
-        if (tok < p.tpad) store_run<TIN, 8>(dst, d);
+        store_run<TIN, 8>(dst, d);
       }
     }
   }
@@ -283,23 +275,20 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
   GemmCore16<Cfg> g;
   g.set_lane();
   const int64_t tok0 = n0 + g.wave_n * Cfg::WN;  // first position of this wave's group
-  f32x4_t tc[NBN];
-  int lab[NBN];
-#pragma unroll
-  for (int j = 0; j < NBN; ++j) {
-    const int64_t pos = tok0 + j * 16 + l16;
-    tc[j] = f32x4_t{1.0e30f, 0.f, 0.f, 0.f};
-    lab[j] = -1;
-    if (pos < p.tpad) {
-      tc[j] = p.tokc[pos];
-      lab[j] = p.tokl[pos];
-    }
-  }
   g.a_plane = p.w_plane;
   g.b_plane = p.h_plane;
   g.init(p.W, p.ldw, (int64_t)vt * Cfg::BM, p.vrows, p.h, p.ldh, n0, Tc, p.rows);
   f32x4_t acc[NB][NBN];
   g.run(lds, p.H, acc);
+  if (tok0 >= p.tpad) return;  // (positions are padded to whole groups: all of this wave's exist, or none)
+  // the constants of the lane's positions, all asked for at once: across the K loop there are no registers for them
+  f32x4_t tc[NBN];
+  int lab[NBN];
+#pragma unroll
+  for (int j = 0; j < NBN; ++j) {
+    tc[j] = p.tokc[tok0 + j * 16 + l16];
+    lab[j] = p.tokl[tok0 + j * 16 + l16];
+  }
   const int vloc0 = vt * Cfg::BM + g.wave_m * Cfg::WM;  // chunk-local vocabulary index of this wave's first row
   // fast path: no padded vocabulary rows and no label in the wave tile
   bool has_label = false;
@@ -326,7 +315,7 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
     for (int j = 0; j < NBN; ++j) {
       const int rel = lab[j] - (int)p.lab0 - vloc0;  // = 16 i + 4 g + r inside the wave tile
       const int64_t tok = tok0 + j * 16 + l16;
-      if (rel >= 0 && rel < Cfg::WM && ((rel >> 2) & 3) == g4 && tok < p.tpad)
+      if (rel >= 0 && rel < Cfg::WM && ((rel >> 2) & 3) == g4)
         *ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + (rel >> 5) * 32 + g4 * 8 + ((rel >> 4) & 1) * 4 + (rel & 3)) = (typename Cfg::TIN)0.f;
     }
   }
@@ -338,7 +327,7 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
 // for C[m][n] = sum_k A[m][k] B[n][k] lane l holds m = 16 j + l % 16 and n = 16 i + 4 (l / 16) + r.
 // ------------------------------------------------------------------------------------------------
 template <typename Cfg, int MODE, bool EDGE>
-LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
+LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
   typedef typename Cfg::TIN TIN;
   // mw, nw: this lane's row of block column 0 and its first column of block row 0
   // accumulate modes: the old values of block column j + 1 are fetched before column j is added and stored, so that
@@ -358,6 +347,7 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t
 #pragma unroll
   for (int j = 0; j < Cfg::NBN; ++j) {
     const int64_t m = mw + j * 16;
+    GemmCore16<Cfg>::stay_column(acc, j);  // (one block column at a time, as in fwd16_fold)
     if ((MODE & 1) && j + 1 < Cfg::NBN) fetch(j + 1);
     if (EDGE && m >= p.M) continue;
 #pragma unroll
@@ -441,57 +431,6 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
 #undef LCE_EPI16
 }
 
-// C[m][n] = sum_k A[k][m] * B[k][n], both operands K-major and allocated in whole 256-column tiles, K (or *k_dev
-// rounded up to k_gran) a multiple of 64.  out_mode 0: Cf = acc; out_mode 2: Ct[PermCfg's vocab_at(m)][n] = (TIN)acc
-// (the rows of C are A's columns, which the d_logits epilogue leaves in KPerm::vocab order).
-template <typename Cfg, typename PermCfg>
-LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* lds) {
-  typedef typename Cfg::TIN TIN;
-  GemmArgs<TIN> p = pin;
-  if (p.k_dev) {
-    const int64_t k = ((int64_t)*p.k_dev + p.k_gran - 1) / p.k_gran * p.k_gran;
-    p.K = k < p.K ? k : p.K;
-  }
-  int tm, tn;
-  if (!p.map.decode(bid, tm, tn)) return;
-  const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
-  GemmCore16<Cfg> g;
-  f32x4_t acc[Cfg::NB][Cfg::NB];
-  if (p.K > 0) {
-    g.a_plane = p.b_plane;
-    g.b_plane = p.a_plane;
-    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);  // MFMA rows = n, MFMA columns = m
-    g.run(lds, p.K, acc);
-  } else {
-    g.set_lane();
-#pragma unroll
-    for (int i = 0; i < Cfg::NB; ++i)
-#pragma unroll
-      for (int j = 0; j < Cfg::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  const int64_t nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
-#pragma unroll
-  for (int j = 0; j < Cfg::NB; ++j) {
-    const int u = g.wave_n * Cfg::WN + j * 16 + (g.lane & 15);  // row inside the tile, in the operand's column order
-    const int64_t m = m0 + ((p.out_mode == 2 || p.perm_rows) ? (int64_t)KPerm<PermCfg>::vocab_at(u) : (int64_t)u);
-    if (m >= p.M) continue;
-#pragma unroll
-    for (int i = 0; i < Cfg::NB; ++i) {
-      const int64_t n = nw + i * 16;
-      if (n >= p.N) continue;  // (N is a multiple of 4)
-      if (p.out_mode == 2) {
-        typedef typename VecOf<TIN, 4>::type vec_t;
-        vec_t o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (TIN)acc[i][j][r];
-        *reinterpret_cast<vec_t*>(p.Ct + m * p.ldct + n) = o;
-      } else {
-        *reinterpret_cast<f32x4_t*>(p.Cf + m * p.ldcf + n) = acc[i][j];
-      }
-    }
-  }
-}
-
 // LDS write of 8 bytes as inline assembly, for the same reason as the reads: through the compiler it would wait for the
 // global->LDS loads in flight
 LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_write_b64 %0, %1" ::"v"(lds_addr), "v"(v)); }
@@ -502,7 +441,7 @@ LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_
 // times as fast as the accumulators' own lane order, 16 rows x 64 bytes.)  Two buffers in turn: block column j is
 // written while j - 1 is read back, so that neither waits for the other.  32 stores, exactly, when the tile is FULL.
 template <typename Cfg, typename PermCfg, bool FULL>
-LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, const f32x4_t (&acc)[Cfg::NB][Cfg::NB], int64_t m0, int64_t n0,
+LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NB], int64_t m0, int64_t n0,
                                 int wave_m, int wave_n, uint32_t stage) {
   typedef typename Cfg::TIN TIN;
   typedef typename VecOf<TIN, 4>::type vec_t;
@@ -518,6 +457,7 @@ LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, const f32x
   char* base = reinterpret_cast<char*>(p.Ct + mw * p.ldct + n);
   auto write = [&](auto jc) {
     constexpr int j = decltype(jc)::value;
+    GemmCore16<Cfg>::stay_column(acc, j);
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       vec_t o;
@@ -550,6 +490,57 @@ LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, const f32x
       store(std::integral_constant<int, j - 1>{});
     }
   });
+}
+
+// C[m][n] = sum_k A[k][m] * B[k][n], both operands K-major and allocated in whole 256-column tiles, K (or *k_dev
+// rounded up to k_gran) a multiple of 64.  out_mode 0: Cf = acc; out_mode 2: Ct[PermCfg's vocab_at(m)][n] = (TIN)acc
+// (the rows of C are A's columns, which the d_logits epilogue leaves in KPerm::vocab order).
+template <typename Cfg, typename PermCfg>
+LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* lds) {
+  typedef typename Cfg::TIN TIN;
+  GemmArgs<TIN> p = pin;
+  if (p.k_dev) {
+    const int64_t k = ((int64_t)*p.k_dev + p.k_gran - 1) / p.k_gran * p.k_gran;
+    p.K = k < p.K ? k : p.K;
+  }
+  int tm, tn;
+  if (!p.map.decode(bid, tm, tn)) return;
+  const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
+  GemmCore16<Cfg> g;
+  f32x4_t acc[Cfg::NB][Cfg::NB];
+  if (p.K > 0) {
+    g.a_plane = p.b_plane;
+    g.b_plane = p.a_plane;
+    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);  // MFMA rows = n, MFMA columns = m
+    g.run(lds, p.K, acc);
+  } else {
+    g.set_lane();
+#pragma unroll
+    for (int i = 0; i < Cfg::NB; ++i)
+#pragma unroll
+      for (int j = 0; j < Cfg::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  if (p.out_mode == 2) {
+    __syncthreads();  // (the ring is the store tiles' now)
+    const uint32_t stage = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 8192;
+    if (m0 + Cfg::BM <= p.M && n0 + Cfg::BN <= p.N) gemm16_store_lines<Cfg, PermCfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
+    else gemm16_store_lines<Cfg, PermCfg, false>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
+    return;
+  }
+  const int64_t nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
+#pragma unroll
+  for (int j = 0; j < Cfg::NB; ++j) {
+    const int u = g.wave_n * Cfg::WN + j * 16 + (g.lane & 15);  // row inside the tile, in the operand's column order
+    const int64_t m = m0 + (p.perm_rows ? (int64_t)KPerm<PermCfg>::vocab_at(u) : (int64_t)u);
+    GemmCore16<Cfg>::stay_column(acc, j);
+    if (m >= p.M) continue;
+#pragma unroll
+    for (int i = 0; i < Cfg::NB; ++i) {
+      const int64_t n = nw + i * 16;
+      if (n >= p.N) continue;  // (N is a multiple of 4)
+      *reinterpret_cast<f32x4_t*>(p.Cf + m * p.ldcf + n) = acc[i][j];
+    }
+  }
 }
 
 // d_weight with tokens between the streaming kernels' range and the sizes where a tile's K loop hides everything else:
