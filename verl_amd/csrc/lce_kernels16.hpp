@@ -330,25 +330,28 @@ template <typename Cfg, int MODE, bool EDGE>
 LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
   typedef typename Cfg::TIN TIN;
   // mw, nw: this lane's row of block column 0 and its first column of block row 0
-  // accumulate modes: the old values of block column j + 1 are fetched before column j is added and stored, so that
-  // a lane always has eight 16-byte loads in flight (measured on the d_hidden GEMM of one 8192-column chunk, 16384 x
-  // 3584 x 8192: 0.900 -> 0.875 ms; the same GEMM storing without reading takes 0.837)
-  f32x4_t prev[2][Cfg::NB];
+  // accumulate modes: the old values of the next AHEAD block columns are on their way while a column is added and stored (the
+  // operand fragments' registers are free by now); one column ahead, a tile's epilogue was 38000 cycles of waiting
+  constexpr int AHEAD = 3;
+  f32x4_t prev[AHEAD + 1][Cfg::NB];
   auto fetch = [&](int j) {
     const int64_t m = mw + j * 16;
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i) {
       const int64_t n = nw + i * 16;
-      prev[j & 1][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (!(EDGE && (m >= p.M || n >= p.N))) prev[j & 1][i] = *reinterpret_cast<const f32x4_t*>(p.Cf + m * p.ldcf + n);
+      prev[j % (AHEAD + 1)][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (!(EDGE && (m >= p.M || n >= p.N))) prev[j % (AHEAD + 1)][i] = *reinterpret_cast<const f32x4_t*>(p.Cf + m * p.ldcf + n);
     }
   };
-  if (MODE & 1) fetch(0);
+  if (MODE & 1) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) fetch(j);
+  }
 #pragma unroll
   for (int j = 0; j < Cfg::NBN; ++j) {
     const int64_t m = mw + j * 16;
     GemmCore16<Cfg>::stay_column(acc, j);  // (one block column at a time, as in fwd16_fold)
-    if ((MODE & 1) && j + 1 < Cfg::NBN) fetch(j + 1);
+    if ((MODE & 1) && j + AHEAD < Cfg::NBN) fetch(j + AHEAD);
     if (EDGE && m >= p.M) continue;
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i) {
@@ -356,7 +359,7 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc
       if (EDGE && n >= p.N) continue;  // (N is a multiple of 4)
       f32x4_t v = acc[i][j];
       if (MODE & 1) {
-        v += prev[j & 1][i];
+        v += prev[j % (AHEAD + 1)][i];
       }
       if (MODE & 2) {
         typedef typename VecOf<TIN, 4>::type vec_t;
@@ -369,6 +372,60 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc
       }
     }
   }
+}
+
+// A full wave tile in fp32, C (+)= acc (ACC: old values are read), as whole lines: one block column (16 rows x 128 columns) at a
+// time goes through 8 KB of LDS that belong to this wave, 16-byte chunk c of row r at c ^ r, and meets memory two rows x 512
+// bytes per instruction.  In the accumulators' own lane order, 16 rows x 64 bytes, reading and writing a tile took 36000
+// cycles whatever was in flight, a twentieth of the K loop of the d_hidden GEMM.  Two buffers in turn; the old values of the
+// next AHEAD columns are on their way while a column is added and stored.
+template <typename Cfg, bool ACC>
+LCE_DEV void gemm16_f32_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw, uint32_t stage) {
+  // mw, nw: the wave tile's first row and column of C
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN, AHEAD = 2;
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15, hi = lane >> 5, cl = lane & 31;
+  const uint32_t wr = stage + (uint32_t)(l16 * 512 + (g4 ^ l16) * 16);   // chunk 4 i + g4: ^ i * 64
+  const uint32_t rd = stage + (uint32_t)(hi * 512 + (cl ^ hi) * 16);     // row 2 k + hi: ^ k * 32, + k * 1024
+  char* base = reinterpret_cast<char*>(p.Cf + mw * p.ldcf + nw);
+  const uint32_t off = (uint32_t)(hi * p.ldcf * 4 + cl * 16);
+  const int64_t row_bytes = p.ldcf * 4;
+  f32x4_t prev[AHEAD + 1][NB];
+  auto fetch = [&](int j) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) prev[j % (AHEAD + 1)][k] = *reinterpret_cast<const f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off);
+  };
+  auto write = [&](int j) {
+    GemmCore16<Cfg>::stay_column(acc, j);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      asm volatile("ds_write_b128 %0, %1" ::"v"((wr ^ (uint32_t)(i * 64)) + (j & 1) * 8192), "a"(acc[i][j]));
+  };
+  if (ACC) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) fetch(j);
+  }
+  write(0);
+  static_for(std::make_integer_sequence<int, NBN>{}, [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    if (ACC && j + AHEAD < NBN) fetch(j + AHEAD);
+    if (j + 1 < NBN) write(j + 1);
+    GemmCore16<Cfg>::template wait_lgkm<(j + 1 < NBN ? NB : 0)>();  // block column j is in LDS (j + 1's writes may be on their way)
+    u32x4_t v[NB];
+    static_for(std::make_integer_sequence<int, NB>{}, [&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      v[k] = lds_read16<k * 1024>((rd ^ (uint32_t)(k * 32)) + (j & 1) * 8192);
+    });
+    GemmCore16<Cfg>::template wait_lgkm<0>();
+#pragma unroll
+    for (int k = 0; k < NB; ++k) asm volatile("" : "+v"(v[k]));  // (the reads are assembly, the compiler does not know when they return)
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      f32x4_t x = __builtin_bit_cast(f32x4_t, v[k]);
+      if (ACC) x += prev[j % (AHEAD + 1)][k];
+      *reinterpret_cast<f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off) = x;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  });
 }
 
 // CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2, NBN>: then B is K-major as it lies in memory, B[k][n] with row
@@ -419,6 +476,14 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
   }
   const int64_t mw = m0 + g.wave_n * Cfg::WN + (g.lane & 15), nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
   const bool edge = m0 + Cfg::BN > p.M || n0 + Cfg::BM > p.N;
+  if (!edge && p.out_mode < 2) {
+    __syncthreads();  // (the ring is the store tiles' now)
+    const uint32_t stage = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 16384;
+    const int64_t mt = m0 + g.wave_n * Cfg::WN, nt = n0 + g.wave_m * Cfg::WM;
+    if (p.out_mode == 1) gemm16_f32_lines<Cfg, true>(p, acc, mt, nt, stage);
+    else gemm16_f32_lines<Cfg, false>(p, acc, mt, nt, stage);
+    return;
+  }
 #define LCE_EPI16(MODE)                                             \
   if (edge) gemm16_epilogue<Cfg, MODE, true>(p, acc, mw, nw);       \
   else gemm16_epilogue<Cfg, MODE, false>(p, acc, mw, nw)
