@@ -239,6 +239,8 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
     // 4.5% faster again once `hidden` is far larger than the memory-side cache (T=65536, H=5120: 671 MB)
     else if (T <= 8192 || (uint64_t)T * (uint64_t)H * esize(dtype) > (512ull << 20)) sel = 1;
   }
+  // (the square tile's stream of slabs wants two of them)
+  if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   // (lce_forward_static's built-in buffer has no room for the planes: fp32 tiles there)
   const size_t terms_need = forward_terms_need(T, H, V, dtype);
   if (terms_need && workspace_bytes >= terms_need) sel = kSelTerms;

@@ -86,6 +86,13 @@ LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg:
   }
 }
 
+// Which forwards run the stream of slabs: the square tile on plain operands.  (The kept logits are stores whose number the
+// stream's waits would have to know; the narrow tile's early operand is the other one.)  It wants two slabs of K at least.
+template <typename Cfg, bool KEEP>
+struct Fwd16Stream {
+  static constexpr bool value = !KEEP && Cfg::NBN == Cfg::NB && !Cfg::A_EARLY && Cfg::TERMS == 1;
+};
+
 // KEEP: the tiles also write their logits to p.xcache (FwdArgs), for a backward that then does not recompute them
 template <typename Cfg, bool KEEP>
 LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
@@ -117,45 +124,73 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
   const int vend = (int)vend64;
   g.init(p.W, p.ldw, row0, vend64, p.h, p.ldh, n0, p.T);
   g.prologue(lds, p.H);
-  for (int64_t m0 = row0; m0 < vend64; m0 += p.tile_step) {
-    g.main(lds, p.H, acc);
-    const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
-    const bool full = m0 + Cfg::BM <= vend64;
-    if constexpr (KEEP) {
-      // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.  Issued AHEAD of the next
-      // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
-      // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are
-      // issued 16 at a time and so many are waited for that, with the prologue's 32 loads behind them, fewer than 64
-      // operations are ever in flight.
-      const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
-      // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
-      const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
-      const int row_at = g4 * 16, panel = (int)p.T * 64;
-#pragma unroll
-      for (int j = 0; j < NBN; ++j) {
-        GemmCore16<Cfg>::stay_column(acc, j);
-        const int at = t0 + j * 16 < p.T ? (int)(t0 + j * 16) * 64 + row_at : kBufNowhere;
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, 0);
-        }
-        if (j % 2 == 1 && j >= 3) {
-          __builtin_amdgcn_sched_barrier(0);
-          if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<24>();
-          else GemmCore16<Cfg>::template wait_vm<32>();
-        }
+  if constexpr (Fwd16Stream<Cfg, KEEP>::value) {
+    // The K loops of successive tiles are one stream of slabs (GemmCore16::stream_tile): nothing is drained between them and
+    // the next tile's first slabs are in LDS while this one is folded in.  Only a last tile with fewer rows, whose loads
+    // are clamped, starts anew.
+    const int nk = (int)(p.H / Cfg::BK);  // (>= 2)
+    typename GemmCore16<Cfg>::Stream st;
+    g.stream_begin(lds, st);
+    for (int64_t m0 = row0; m0 < vend64; m0 += p.tile_step) {
+      const int64_t next = m0 + p.tile_step;
+      const bool flows = next + Cfg::BM <= vend64;
+      const char* a_next = flows ? g.a_base + p.tile_step * p.ldw * 2 : g.a_base;
+      g.template stream_tile<0>(lds, nk, acc, st, a_next, g.b_base, false);
+      g.a_base = a_next;
+      const bool anew = next < vend64 && !flows;
+      if (anew) {
+        GemmCore16<Cfg>::template wait_vm<0>();
+        __syncthreads();
+        g.init(p.W, p.ldw, next, vend64, p.h, p.ldh, n0, p.T);
+        g.prologue(lds, p.H);
       }
-      __builtin_amdgcn_sched_barrier(0);
+      const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
+      if (m0 + Cfg::BM <= vend64) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
+      else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
+      if (anew) g.stream_begin(lds, st);
     }
-    // the next tile's first slabs fly while this tile's statistics are folded in
-    __syncthreads();  // every wave is past its last LDS read and has drained its own loads
-    if (m0 + p.tile_step < vend64) {
-      g.init(p.W, p.ldw, m0 + p.tile_step, vend64, p.h, p.ldh, n0, p.T);
-      g.prologue(lds, p.H);
+    GemmCore16<Cfg>::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
+  } else {
+    for (int64_t m0 = row0; m0 < vend64; m0 += p.tile_step) {
+      g.main(lds, p.H, acc);
+      const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
+      const bool full = m0 + Cfg::BM <= vend64;
+      if constexpr (KEEP) {
+        // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.  Issued AHEAD of the next
+        // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
+        // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are
+        // issued 16 at a time and so many are waited for that, with the prologue's 32 loads behind them, fewer than 64
+        // operations are ever in flight.
+        const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
+        // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
+        const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
+        const int row_at = g4 * 16, panel = (int)p.T * 64;
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) {
+          GemmCore16<Cfg>::stay_column(acc, j);
+          const int at = t0 + j * 16 < p.T ? (int)(t0 + j * 16) * 64 + row_at : kBufNowhere;
+#pragma unroll
+          for (int i = 0; i < NB; ++i) {
+            const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, 0);
+          }
+          if (j % 2 == 1 && j >= 3) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<24>();
+            else GemmCore16<Cfg>::template wait_vm<32>();
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // the next tile's first slabs fly while this tile's statistics are folded in
+      __syncthreads();  // every wave is past its last LDS read and has drained its own loads
+      if (m0 + p.tile_step < vend64) {
+        g.init(p.W, p.ldw, m0 + p.tile_step, vend64, p.h, p.ldh, n0, p.T);
+        g.prologue(lds, p.H);
+      }
+      if (full) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
+      else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
     }
-    if (full) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
-    else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
   }
   __syncthreads();
 
