@@ -383,6 +383,40 @@ def test_ppo_loss_entry_with_the_reference_signature(nested, globals_set):
     assert metrics["kl_coef"] == 0.01
 
 
+@pytest.mark.parametrize("dtype", [torch.int64, torch.bool])
+@pytest.mark.parametrize("layout", ["expanded", "one-row", "windows", "columns-apart", "wider-rows"])
+def test_attention_masks_of_any_strides(layout, dtype):
+    """The lengths of a padded batch are counted from its attention mask whatever its strides: rows expanded from one, a
+    single row whose row stride means nothing, sliding windows over one vector, columns that are not neighbours, rows of a
+    wider tensor.  The same numbers as with a mask of its own memory."""
+    from verl_amd.workers.utils.losses import ppo_loss
+
+    B, P, R = (1 if layout == "one-row" else 4), 6, 9
+    W = P + R
+    if layout == "expanded":
+        mask = torch.ones(1, W, device=DEV, dtype=dtype).expand(B, W)
+    elif layout == "one-row":
+        mask = torch.ones(W, device=DEV, dtype=dtype).as_strided((1, W), (1, 1))
+    elif layout == "windows":  # row b is the vector from element b on: three zeros, then ones
+        mask = torch.cat([torch.zeros(3, device=DEV), torch.ones(W, device=DEV)]).to(dtype).as_strided((B, W), (1, 1))
+    elif layout == "columns-apart":
+        mask = torch.ones(B, 2 * W, device=DEV, dtype=dtype)[:, ::2]
+    else:
+        mask = torch.ones(B, W + 5, device=DEV, dtype=dtype)[:, :W]
+    prompt, resp = mask[:, :P].sum(1).tolist(), mask[:, P:].sum(1).tolist()
+    lp, ent, old, adv, ref, rmask = _packed_case(prompt, resp, R, seed=31)
+    data = {"prompts": torch.zeros(B, P, dtype=torch.long, device=DEV), "responses": torch.zeros(B, R, dtype=torch.long, device=DEV),
+            "response_mask": rmask, "old_log_probs": old, "advantages": adv, "dp_size": 1, "batch_num_tokens": None, "global_batch_size": None}
+    got = []
+    for m in (mask, mask.clone(memory_format=torch.contiguous_format)):
+        lp1, ent1 = lp.clone().requires_grad_(True), ent.clone().requires_grad_(True)
+        loss, _ = ppo_loss(_ActorConfig(), {"log_probs": lp1, "entropy": ent1}, dict(data, attention_mask=m))
+        loss.backward()
+        got.append((loss.detach(), lp1.grad, ent1.grad))
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, atol=0, rtol=0)
+
+
 @pytest.mark.parametrize("fields", ["jagged", "padded-wider", "padded-narrower"])
 def test_ppo_loss_honours_max_response_len(fields):
     """verl/workers/utils/padding.py:112-118: on a nested batch the padded width of the response slice is the non-tensor

@@ -151,7 +151,8 @@ class _FusedPPOLoss(torch.autograd.Function):
         lens = ()
         if count_lens:
             am = packed.attention_mask
-            call.attention_mask, call.attention_kind, call.attention_stride = am.data_ptr(), _INT_MASKS[am.dtype], am.stride(0)
+            call.attention_mask, call.attention_kind = am.data_ptr(), _INT_MASKS[am.dtype]
+            call.attention_stride = am.stride(0) if rows > 1 else am.shape[1]  # (a single row's stride means nothing)
             call.prompt_width, call.attention_width = packed.prompt_width, am.shape[1]
             call.prompt_lens, call.response_lens = at, at + 8 * rows
         elif packed is not None:
@@ -331,7 +332,10 @@ def _packed_lengths(data, dev) -> _Packed:
     if not data["prompts"].is_nested:
         mask, P = data["attention_mask"], data["prompts"].shape[1]
         if not mask.is_nested and mask.dtype in _INT_MASKS and mask.device == dev and mask.dim() == 2 and mask.shape[1] >= P:
-            return _Packed(attention_mask=mask if mask.stride(1) == 1 else mask.contiguous(), prompt_width=P)
+            # (the kernel takes rows of neighbouring elements that do not overlap; expanded rows and sliding windows are copied)
+            if mask.stride(1) != 1 or (mask.shape[0] > 1 and mask.stride(0) < mask.shape[1]):
+                mask = mask.contiguous()
+            return _Packed(attention_mask=mask, prompt_width=P)
     return _Packed(*(t.to(dev, torch.int64).contiguous() for t in batch_lens(data)))
 
 
