@@ -211,6 +211,24 @@ def test_logits_twins_name_the_gpu_only_precondition():
             call()
 
 
+@pytest.mark.parametrize("rows", [3, 5])
+def test_a_batch_with_lengths_for_other_rows_is_refused(rows):
+    """The kernels read one pair of lengths per response: a mask, or nested prompts, with another number of rows must not
+    get as far as a launch, which would read beyond them (or leave the rest out)."""
+    from verl_amd.workers.utils.losses import _packed_lengths
+
+    data = {"prompts": torch.zeros(4, 6, dtype=torch.long), "responses": torch.zeros(4, 5, dtype=torch.long),
+            "attention_mask": torch.ones(rows, 11, dtype=torch.long)}  # fmt: skip
+    cpu = torch.device("cpu")
+    for dtype in (torch.long, torch.int32, torch.bool, torch.float32):  # (float32: the general path)
+        with pytest.raises(AssertionError, match="for 4 responses"):
+            _packed_lengths(dict(data, attention_mask=data["attention_mask"].to(dtype)), cpu)
+    nested = {k: torch.nested.nested_tensor([torch.zeros(2)] * n, layout=torch.jagged) for k, n in (("prompts", rows), ("responses", 4))}
+    with pytest.raises(AssertionError, match="for 4 responses"):
+        _packed_lengths(nested, cpu)
+    assert _packed_lengths(dict(data, attention_mask=torch.ones(4, 11)), cpu).prompt_lens.tolist() == [6.0] * 4
+
+
 def test_metric_aggregation_kinds_of_ppo_loss():
     """verl/workers/utils/losses.py:71-84: any global normaliser switches the loss metrics to SUM; Metric folds as
     verl/utils/metric/utils.py:72-160 (hand-computed numbers)."""

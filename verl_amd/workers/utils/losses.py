@@ -328,15 +328,20 @@ def batch_lens(data):
 
 
 def _packed_lengths(data, dev) -> _Packed:
-    """``batch_lens`` for the kernel: a padded batch's mask of integers on ``dev`` is counted by the loss's own launches."""
+    """``batch_lens`` for the kernel, one pair of lengths per response: a padded batch's mask of integers on ``dev`` is
+    counted by the loss's own launches."""
+    rows = data["responses"].shape[0]
     if not data["prompts"].is_nested:
         mask, P = data["attention_mask"], data["prompts"].shape[1]
         if not mask.is_nested and mask.dtype in _INT_MASKS and mask.device == dev and mask.dim() == 2 and mask.shape[1] >= P:
+            assert mask.shape[0] == rows, f"{mask.shape[0]} rows of the attention mask for {rows} responses"
             # (the kernel takes rows of neighbouring elements that do not overlap; expanded rows and sliding windows are copied)
-            if mask.stride(1) != 1 or (mask.shape[0] > 1 and mask.stride(0) < mask.shape[1]):
+            if mask.stride(1) != 1 or (rows > 1 and mask.stride(0) < mask.shape[1]):
                 mask = mask.contiguous()
             return _Packed(attention_mask=mask, prompt_width=P)
-    return _Packed(*(t.to(dev, torch.int64).contiguous() for t in batch_lens(data)))
+    lens = [t.to(dev, torch.int64).contiguous() for t in batch_lens(data)]
+    assert all(t.shape == (rows,) for t in lens), f"{[tuple(t.shape) for t in lens]} prompt and response lengths for {rows} responses"
+    return _Packed(*lens)
 
 
 def _padded(t: torch.Tensor, width: int) -> torch.Tensor:
