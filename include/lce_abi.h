@@ -241,7 +241,9 @@ int lce_ppo_loss_packed(const float* log_prob_packed, const float* entropy_packe
  *     attention_stride, the first prompt_width columns are the prompts') the two are OUTPUTS: the forward counts them.
  *     total_nnz < 0: everything is [rows, row_len].
  *   g_log_prob / g_entropy: unscaled gradients, kept for the backward, like the workspace
- *   d_log_prob / d_entropy: written by lce_ppo_backward (either may be NULL); g_loss: fp32 on the device
+ *   d_log_prob / d_entropy: written by lce_ppo_backward (either may be NULL); g_loss: fp32 on the device.  Of the other
+ *     pointers lce_ppo_backward looks at g_log_prob, g_entropy, the workspace and, packed, the two vectors of lengths:
+ *     the forward's inputs may be gone by then, and their fields NULL
  * Packed: when lce_ppo_forward returns, checks[0] = sum of all lengths, checks[1] = number of prompts of length 0,
  * checks[2] = longest response are on the HOST (the call waits for the kernel that adds them up, not for the loss): the
  * reference's assertions are the caller's.  Rows that fail them have meaningless gradients; nothing is written outside the

@@ -609,22 +609,25 @@ struct PpoPlan {
   unsigned blocks;
 };
 
-static int ppo_plan(const lce_ppo_call_t& c, PpoPlan* plan) {
+// `scale_only`: for the backward, which reads what the forward left and none of the forward's inputs
+static int ppo_plan(const lce_ppo_call_t& c, PpoPlan* plan, bool scale_only = false) {
   if (c.rows <= 0 || c.row_len <= 0) return fail(LCE_E_ARG, "ppo loss: rows and row_len must be positive");
   if (c.rows > ((int64_t)1 << 30) || c.row_len > ((int64_t)1 << 40) / c.rows) return fail(LCE_E_ARG, "ppo loss: too many elements");
-  if (!c.mask || !c.out) return fail(LCE_E_ARG, "null pointer");
+  if (!scale_only && (!c.mask || !c.out)) return fail(LCE_E_ARG, "null pointer");
   if (c.mask_kind < PPO_MASK_F32 || c.mask_kind > PPO_MASK_F32_NONZERO) return fail(LCE_E_ARG, "ppo loss: unknown mask_kind %d", c.mask_kind);
-  if (c.log_prob) {
+  if (scale_only) {
+    // (no inputs to check)
+  } else if (c.log_prob) {
     if (!c.old_log_prob || !c.advantages || !c.g_log_prob) return fail(LCE_E_ARG, "null pointer");
     if (!(c.clip_c > 1.f)) return fail(LCE_E_ARG, "clip_ratio_c must be greater than 1");
   } else if (!c.entropy || c.g_log_prob || c.kl_type != LCE_PPO_KL_NONE) {
     return fail(LCE_E_ARG, "without log_prob the call aggregates `entropy` alone");
   }
-  if ((c.entropy == nullptr) != (c.g_entropy == nullptr)) return fail(LCE_E_ARG, "entropy and g_entropy go together");
+  if (!scale_only && (c.entropy == nullptr) != (c.g_entropy == nullptr)) return fail(LCE_E_ARG, "entropy and g_entropy go together");
   const int kl_base = c.kl_type & ~LCE_PPO_KL_STRAIGHT_THROUGH;
   if (kl_base < LCE_PPO_KL_NONE || kl_base > LCE_PPO_KL_K3 || (kl_base == LCE_PPO_KL_NONE && c.kl_type != LCE_PPO_KL_NONE))
     return fail(LCE_E_ARG, "ppo loss: unknown kl_type %d", c.kl_type);
-  if (kl_base != LCE_PPO_KL_NONE && !c.ref_log_prob) return fail(LCE_E_ARG, "the KL penalty needs ref_log_prob");
+  if (!scale_only && kl_base != LCE_PPO_KL_NONE && !c.ref_log_prob) return fail(LCE_E_ARG, "the KL penalty needs ref_log_prob");
   if (c.agg_mode < PPO_TOKEN_MEAN || c.agg_mode > PPO_SEQ_MEAN_TOKEN_MEAN) return fail(LCE_E_ARG, "Invalid loss_agg_mode: %d", c.agg_mode);
   if (!(c.dp_size > 0.f)) return fail(LCE_E_ARG, "ppo loss: dp_size must be positive");
   PpoArgs& p = plan->p;
@@ -704,12 +707,12 @@ static int ppo_entry(const float* log_prob, const float* entropy, const int64_t*
 }
 
 // what lce_ppo_forward and lce_ppo_backward check and set up alike
-static int ppo_call_plan(const lce_ppo_call_t* call, PpoPlan* plan) {
+static int ppo_call_plan(const lce_ppo_call_t* call, PpoPlan* plan, bool scale_only = false) {
   if (!call) return fail(LCE_E_ARG, "null call");
   const bool packed = call->total_nnz >= 0;
-  int rc = ppo_plan(*call, plan);
+  int rc = ppo_plan(*call, plan, scale_only);
   if (rc) return rc;
-  if (packed && (!call->log_prob || !call->prompt_lens || !call->response_lens)) return fail(LCE_E_ARG, "ppo loss (packed): null pointer");
+  if (packed && ((!scale_only && !call->log_prob) || !call->prompt_lens || !call->response_lens)) return fail(LCE_E_ARG, "ppo loss (packed): null pointer");
   if (!call->workspace || (size_t)call->workspace_bytes < lce_ppo_loss_workspace_bytes(call->rows, call->row_len))
     return fail(LCE_E_WORKSPACE, "ppo workspace too small");
   if (packed) {
@@ -786,7 +789,7 @@ int lce_ppo_forward(lce_ppo_call_t* call, void* stream) {
 
 int lce_ppo_backward(const lce_ppo_call_t* call, void* stream) {
   PpoPlan plan;
-  int rc = ppo_call_plan(call, &plan);
+  int rc = ppo_call_plan(call, &plan, true);
   if (rc) return rc;
   if (!call->g_loss) return fail(LCE_E_ARG, "null pointer");
   if ((call->d_log_prob && !call->g_log_prob) || (call->d_entropy && !call->g_entropy)) return fail(LCE_E_ARG, "ppo loss: a gradient that the forward did not leave");
