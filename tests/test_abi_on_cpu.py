@@ -211,6 +211,18 @@ def test_logits_twins_name_the_gpu_only_precondition():
             call()
 
 
+def test_response_slices_of_packed_outputs():
+    """verl/workers/utils/padding.py:97-141: where each response starts in the packed outputs, and the two assertions."""
+    from verl_amd.workers.utils.losses import response_slices
+
+    start, length = response_slices(torch.tensor([3, 1, 7]), torch.tensor([5, 0, 2], dtype=torch.int32), 18)
+    assert start.tolist() == [2, 8, 15] and length.tolist() == [5, 0, 2] and start.dtype == length.dtype == torch.int64
+    with pytest.raises(AssertionError):
+        response_slices(torch.tensor([3, 1, 7]), torch.tensor([5, 0, 2]), 17)
+    with pytest.raises(AssertionError, match="prompt_len > 0"):
+        response_slices(torch.tensor([3, 0, 7]), torch.tensor([5, 1, 2]), 18)
+
+
 @pytest.mark.parametrize("rows", [3, 5])
 def test_a_batch_with_lengths_for_other_rows_is_refused(rows):
     """The kernels read one pair of lengths per response: a mask, or nested prompts, with another number of rows must not

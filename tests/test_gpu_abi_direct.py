@@ -191,3 +191,86 @@ def test_diagnostic_gemms_match_torch(variant):
     C2 = torch.zeros(M, N, device=DEV)
     _abi.check(lib.lce_gemm_tn(At.data_ptr(), 512, Bt.data_ptr(), 768, C2.data_ptr(), N, M, N, K, variant, st), "lce_gemm_tn")
     torch.testing.assert_close(C2, want, atol=1e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("kl", [False, True])
+@pytest.mark.parametrize("agg", [0, 2, 4])
+@pytest.mark.parametrize("with_entropy", [False, True])
+def test_ppo_loss_in_one_call(agg, kl, with_entropy):
+    """lce_ppo_loss and lce_ppo_loss_packed, which return loss and gradients of one call, against the forward / backward pair
+    that Python runs: the same launches, so the same bits.  The packed call clears the gradients of the positions that no
+    response token maps to itself."""
+    from verl_amd import _abi
+    from verl_amd.workers.utils import losses as L
+
+    lib = _abi.load()
+    mode = {v: k for k, v in L.AGG_MODES.items()}[agg]
+    prompt, resp, R = [3, 1, 7, 2, 1, 4, 260], [5, 1, 0, 9, 300, 2, 17], 300
+    B, total = len(prompt), sum(prompt) + sum(resp)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rand = lambda *n: torch.rand(*n, device=DEV, generator=g)  # noqa: E731
+    old, adv, ref, isw = -rand(B, R) * 3, rand(B, R) - 0.5, -rand(B, R) * 3, rand(B, R) * 2
+    mask = ((torch.arange(R, device=DEV)[None, :] < torch.tensor(resp, device=DEV)[:, None]) & (rand(B, R) > 0.1)).float()
+    numbers = (4 if kl else 0, 0.05 if kl else 0.0, B, R, agg, 0.2, 0.28, 3.0, 1e-2 if with_entropy else 0.0, 1.0, -1.0, -1.0, -1.0)
+    kw = dict(clip_ratio_low=0.2, clip_ratio_high=0.28, entropy_coeff=numbers[8], loss_agg_mode=mode, rollout_is_weights=isw)
+    if kl:
+        kw.update(ref_log_prob=ref, kl_loss_type="low_var_kl", kl_loss_coef=0.05)
+    nws = lib.lce_ppo_loss_workspace_bytes(B, R)
+    ws = torch.empty(nws, device=DEV, dtype=torch.uint8)
+    stream = torch.cuda.current_stream().cuda_stream
+    P, Rl = torch.tensor(prompt, device=DEV), torch.tensor(resp, device=DEV)
+    start, length = L.response_slices(P, Rl, total)
+    for packed in (False, True):
+        shape = (total,) if packed else (B, R)
+        lp = (-rand(*shape) * 3).requires_grad_(True)
+        ent = (rand(*shape) * 5).requires_grad_(True) if with_entropy else None
+        out = torch.zeros(16, device=DEV)
+        g_lp = torch.full(shape, float("nan"), device=DEV)
+        g_ent = torch.full(shape, float("nan"), device=DEV) if with_entropy else None
+        where = (total, start.data_ptr(), length.data_ptr()) if packed else ()
+        entry = lib.lce_ppo_loss_packed if packed else lib.lce_ppo_loss
+        rc = entry(lp.data_ptr(), _abi.ptr(ent), *where, old.data_ptr(), adv.data_ptr(), mask.data_ptr(), isw.data_ptr(),
+                   ref.data_ptr() if kl else None, *numbers, out.data_ptr(), g_lp.data_ptr(), _abi.ptr(g_ent), ws.data_ptr(), nws, stream)
+        _abi.check(rc, "lce_ppo_loss")
+        if packed:
+            loss, met = L.fused_ppo_loss_packed(lp, ent, P, Rl, old, adv, mask, **kw)
+        else:
+            loss, met = L.fused_ppo_loss(lp, ent, old, adv, mask, **kw)
+        loss.backward()
+        torch.testing.assert_close(out[0], loss.detach(), atol=0, rtol=0)
+        for i, key in ((1, "actor/pg_loss"), (3, "actor/pg_clipfrac"), (4, "actor/ppo_kl"), (5, "actor/pg_clipfrac_lower")):
+            assert out[i].item() == met[key].item(), key
+        torch.testing.assert_close(g_lp, lp.grad, atol=0, rtol=0)
+        if with_entropy:
+            torch.testing.assert_close(g_ent, ent.grad, atol=0, rtol=0)
+
+
+def test_ppo_loss_in_one_call_against_the_oracle():
+    from verl_amd import _abi
+
+    lib = _abi.load()
+    B, R = 9, 700
+    g = torch.Generator(device=DEV).manual_seed(8)
+    lp, old = (-torch.rand(B, R, device=DEV, generator=g) * 3 for _ in range(2))
+    adv, ent = torch.randn(B, R, device=DEV, generator=g), torch.rand(B, R, device=DEV, generator=g)
+    mask = (torch.rand(B, R, device=DEV, generator=g) < 0.7).float()
+    out, g_lp, g_ent = torch.zeros(16, device=DEV), torch.empty(B, R, device=DEV), torch.empty(B, R, device=DEV)
+    nws = lib.lce_ppo_loss_workspace_bytes(B, R)
+    ws = torch.empty(nws, device=DEV, dtype=torch.uint8)
+    rc = lib.lce_ppo_loss(lp.data_ptr(), ent.data_ptr(), old.data_ptr(), adv.data_ptr(), mask.data_ptr(), None, None, 0, 0.0, B, R, 0, 0.2, 0.2,
+                          3.0, 1e-3, 1.0, -1.0, -1.0, -1.0, out.data_ptr(), g_lp.data_ptr(), g_ent.data_ptr(), ws.data_ptr(), nws,
+                          torch.cuda.current_stream().cuda_stream)
+    _abi.check(rc, "lce_ppo_loss")
+    lp2, ent2 = lp.clone().requires_grad_(True), ent.clone().requires_grad_(True)
+    want, _ = O.ppo_actor_loss(lp2, ent2, old, adv, mask, clip_ratio=0.2, entropy_coeff=1e-3)
+    want.backward()
+    torch.testing.assert_close(out[0], want, atol=1e-6, rtol=1e-5)
+    torch.testing.assert_close(g_lp, lp2.grad, atol=1e-8, rtol=1e-5)
+    torch.testing.assert_close(g_ent, ent2.grad, atol=1e-9, rtol=1e-5)
+    # nothing is launched without the workspace, or without what the call needs
+    bad = lib.lce_ppo_loss(lp.data_ptr(), ent.data_ptr(), old.data_ptr(), adv.data_ptr(), mask.data_ptr(), None, None, 0, 0.0, B, R, 0, 0.2, 0.2,
+                           3.0, 1e-3, 1.0, -1.0, -1.0, -1.0, out.data_ptr(), g_lp.data_ptr(), g_ent.data_ptr(), ws.data_ptr(), nws - 1, None)
+    assert bad == -2
+    bad = lib.lce_ppo_loss_packed(lp.data_ptr(), None, B * R, None, None, old.data_ptr(), adv.data_ptr(), mask.data_ptr(), None, None, 0, 0.0, B, R, 0,
+                                  0.2, 0.2, 3.0, 0.0, 1.0, -1.0, -1.0, -1.0, out.data_ptr(), g_lp.data_ptr(), None, ws.data_ptr(), nws, None)
+    assert bad == -1

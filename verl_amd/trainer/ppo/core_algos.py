@@ -1,7 +1,7 @@
 """The two functions of the reference's ``verl/trainer/ppo/core_algos.py`` that sit directly behind the fused head:
 ``agg_loss`` (``:1140-1206``) and ``compute_policy_loss_vanilla`` (``:1286-1376``; its deprecated predecessor
 ``compute_policy_loss``, ``:1210-1282``, and the registry lookup ``get_policy_loss_fn``, ``:70-85``), with the reference's names,
-argument order and return values, computed by the HIP PPO-loss kernels (``lce_ppo_loss``).  Both are
+argument order and return values, computed by the HIP PPO-loss kernels (``lce_ppo_forward`` / ``lce_ppo_backward``).  Both are
 differentiable; nothing here runs on the CPU."""
 
 from __future__ import annotations

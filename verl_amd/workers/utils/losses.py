@@ -281,6 +281,18 @@ def fused_ppo_loss(
     return loss, metrics
 
 
+def response_slices(prompt_lens: torch.Tensor, response_lens: torch.Tensor, total_nnz: int):
+    """``(start, length)`` per sequence of the response slice that ``no_padding_2_padding`` takes out of a packed model
+    output (``verl/workers/utils/padding.py:97-141``), what ``lce_ppo_loss_packed`` takes: ``start`` = end of the sequence -
+    response length - 1 (the left shift by one token), with the reference's two assertions.  ``ppo_loss`` and
+    ``fused_ppo_loss_packed`` have their kernels add the lengths up instead."""
+    prompt_lens, response_lens = prompt_lens.to(torch.int64), response_lens.to(torch.int64)
+    ends = (prompt_lens + response_lens).cumsum(dim=0)
+    assert ends[-1].item() == total_nnz
+    assert not prompt_lens.eq(0).any(), f"seq_offset - resp_len - 1 assumes prompt_len > 0. Got {prompt_lens}"
+    return (ends - response_lens - 1).contiguous(), response_lens.contiguous()
+
+
 def _check_lengths(checks, total_nnz, width):
     """The reference's two assertions on a packed batch (``verl/workers/utils/padding.py:126-128``) and the padded width's,
     on the sums that the kernel reports."""
