@@ -19,7 +19,9 @@
 extern "C" {
 #endif
 
-#define LCE_ABI_VERSION 10
+/* 11: the PPO loss as a pair (lce_ppo_forward .. lce_ppo_backward, lce_ppo_call_t), the logits twins in the caller's types,
+ *     larger PPO and fp32 workspaces, another layout of the kept logits */
+#define LCE_ABI_VERSION 11
 
 enum { LCE_DTYPE_BF16 = 0, LCE_DTYPE_F32 = 1, LCE_DTYPE_F16 = 2 };
 enum { LCE_REDUCTION_NONE = 0, LCE_REDUCTION_SUM = 1, LCE_REDUCTION_MEAN = 2 }; /* verl/utils/kernel/kernels.py:102-126 */

@@ -143,6 +143,21 @@ def test_no_fallback_when_library_is_missing(monkeypatch, tmp_path):
         _abi.load()
 
 
+def test_a_library_of_another_version_is_named_as_such(monkeypatch, tmp_path):
+    """An older library lacks some of the symbols: what is reported is its version, not a missing symbol."""
+    import subprocess
+
+    src, lib = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(f"int lce_abi_version(void) {{ return {_abi.ABI_VERSION - 1}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True, timeout=60)
+    monkeypatch.setattr(_abi, "_lib", None)
+    monkeypatch.setattr(_abi, "LIB_PATH", str(lib))
+    with pytest.raises(_abi.LceError, match=f"library {_abi.ABI_VERSION - 1}, binding {_abi.ABI_VERSION}"):
+        _abi.load()
+    header = open(os.path.join(ROOT, "include", "lce_abi.h")).read()
+    assert f"#define LCE_ABI_VERSION {_abi.ABI_VERSION}\n" in header
+
+
 def test_product_code_never_imports_the_oracle():
     pkg = os.path.join(ROOT, "verl_amd")
     for d, _, files in os.walk(pkg):

@@ -13,7 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("LCE_LIBRARY_PATH") or os.path.join(_HERE, "lib", "liblce_gfx950.so")
 
 DTYPE_BF16, DTYPE_F32, DTYPE_F16 = 0, 1, 2
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 # every symbol include/lce_abi.h declares: name -> (restype, argtypes)
 _c = ctypes
@@ -108,12 +108,13 @@ def load() -> ctypes.CDLL:
                 "verl_amd has no CPU or eager fallback."
             )
         lib = ctypes.CDLL(LIB_PATH)
+        # (first, and before another version's library is asked for symbols that it may not have)
+        if lib.lce_abi_version() != ABI_VERSION:
+            raise LceError(f"ABI version mismatch: library {lib.lce_abi_version()}, binding {ABI_VERSION}")
         for name, (res, args) in SYMBOLS.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        if lib.lce_abi_version() != ABI_VERSION:
-            raise LceError(f"ABI version mismatch: library {lib.lce_abi_version()}, binding {ABI_VERSION}")
         _lib = lib
     return _lib
 
