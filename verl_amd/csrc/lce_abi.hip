@@ -199,13 +199,13 @@ static size_t forward_workspace_need(int64_t T, int64_t V, int max_splits) {
 }
 
 // ... and what the bfloat16 planes of fp32 inputs take on top, where they are used (0: they are not)
-static size_t forward_terms_need(int64_t T, int64_t H, int64_t V, int dtype) {
-  if (T <= 0 || H <= 0 || V <= 0 || !use_terms(tuning_snapshot(), T, H, V, dtype)) return 0;
+static size_t forward_terms_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype) {
+  if (T <= 0 || H <= 0 || V <= 0 || !use_terms(tu, T, H, V, dtype)) return 0;
   return terms_fwd_plan(T, H, V).total;
 }
 
 size_t lce_forward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
-  return std::max(forward_workspace_need(T, V, kMaxSplits), forward_terms_need(T, H, V, dtype));
+  return std::max(forward_workspace_need(T, V, kMaxSplits), forward_terms_need(tuning_snapshot(), T, H, V, dtype));
 }
 
 // shared body of lce_forward and lce_forward_shard
@@ -242,7 +242,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   // (lce_forward_static's built-in buffer has no room for the planes: fp32 tiles there)
-  const size_t terms_need = forward_terms_need(T, H, V, dtype);
+  const size_t terms_need = forward_terms_need(tu, T, H, V, dtype);
   if (terms_need && workspace_bytes >= terms_need) sel = kSelTerms;
   if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
