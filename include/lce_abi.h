@@ -23,7 +23,15 @@ extern "C" {
  *     larger PPO and fp32 workspaces, another layout of the kept logits */
 #define LCE_ABI_VERSION 11
 
-enum { LCE_DTYPE_BF16 = 0, LCE_DTYPE_F32 = 1, LCE_DTYPE_F16 = 2 };
+/* LCE_DTYPE_F32_PLANES: fp32 tensors like LCE_DTYPE_F32, with leave to take their products on the bfloat16 matrix pipe, every
+ * operand held as three bfloat16 planes whose sum it is (six products; not less exact than the fp32 MFMA, and 1.2 times as
+ * fast at 400 tokens, 1.5 to 1.6 times from 1000 on; below 256 tokens and with small vocabularies the fp32 MFMA runs all the
+ * same).  For lce_forward,
+ * lce_forward_keep_logits, lce_forward_shard and the lce_backward functions: a backward must be given the code of the
+ * forward that its statistics come from, because the rounding errors of the logits that it recomputes cancel against those
+ * of the statistics.  The planes want the whole workspace that the size queries answer (they answer alike for both codes);
+ * with LCE_DTYPE_F32 what the fp32 MFMA needs is enough.  Every other entry point takes the first three codes. */
+enum { LCE_DTYPE_BF16 = 0, LCE_DTYPE_F32 = 1, LCE_DTYPE_F16 = 2, LCE_DTYPE_F32_PLANES = 3 };
 enum { LCE_REDUCTION_NONE = 0, LCE_REDUCTION_SUM = 1, LCE_REDUCTION_MEAN = 2 }; /* verl/utils/kernel/kernels.py:102-126 */
 enum {
   LCE_OK = 0,
@@ -57,7 +65,8 @@ int lce_forward(const void* hidden, int64_t ldh, const void* weight, int64_t ldw
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The
  * partial statistics go to a buffer of LCE_STATIC_SCRATCH_BYTES that is part of the library's own device image (one
  * copy per GPU, held until the process ends); the call allocates nothing, uses at most as many vocabulary splits as the
- * buffer has room for (so its results may differ from lce_forward's in the last bits of the fp32 sums) and returns
+ * buffer has room for (so its results may differ from lce_forward's in the last bits of the fp32 sums; fp32 inputs:
+ * LCE_DTYPE_F32, here and in the backward) and returns
  * LCE_E_WORKSPACE when there is no room for four (beyond about 116000 tokens).  All calls on one GPU share the
  * buffer, so calls that overlap on one GPU would race for it; calls on one stream do not overlap.  The library keeps, per
  * GPU, the stream of the last call and an event behind its last kernel: a call on another stream while that one has not

@@ -54,3 +54,74 @@ def test_planes_of_fp32_inputs(T, H, V, tau, keep, reduction, vchunk):
             assert ((got.double() - want).norm() / want.norm()).item() <= 3e-6
     if reduction == 0:
         assert (dh[mask == 0] == 0).all()
+
+
+def _forward(lib, code, entry, h, w, y, tau):
+    """The five outputs of a forward through the C ABI, with a workspace as the code asks for, or the library's own."""
+    from verl_amd import _abi
+
+    (T, H), V = h.shape, w.shape[0]
+    out = [torch.empty(T, device=DEV) for _ in range(5)]
+    where = [o.data_ptr() for o in out]
+    st = torch.cuda.current_stream().cuda_stream
+    if entry == "static":
+        rc = lib.lce_forward_static(h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, tau, 0, *where, st)
+    else:
+        n = lib.lce_forward_workspace_bytes(T, H, V, code)
+        n = 8 << 20 if entry == "small" else n  # (what the fp32 MFMA needs: 256 splits of 512 tokens, 2.1 MB)
+        ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+        rc = lib.lce_forward(h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, tau, 0, *where, ws.data_ptr(), n, st)
+    _abi.check(rc, "forward")
+    return out
+
+
+def _backward(lib, code, h, w, y, tau, stats, g_lp, g_ent):
+    from verl_amd import _abi
+
+    (T, H), V = h.shape, w.shape[0]
+    dh, dw = torch.empty_like(h), torch.empty_like(w)
+    n = lib.lce_backward_workspace_bytes(T, H, V, code, 0)
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+    rc = lib.lce_backward(h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, tau, 0, *(s.data_ptr() for s in stats), g_lp.data_ptr(),
+                          g_ent.data_ptr(), dh.data_ptr(), dw.data_ptr(), ws.data_ptr(), n, 0, torch.cuda.current_stream().cuda_stream)
+    _abi.check(rc, "lce_backward")
+    return dh, dw
+
+
+@pytest.mark.parametrize("std", [0.1, 0.3])
+def test_statistics_and_logits_come_from_the_same_arithmetic(std):
+    """The backward recomputes the logits: where a distribution is peaked, their rounding errors cancel against those of the
+    forward's statistics only if both were taken the same way.  The fp32 code takes the fp32 MFMA both ways, whatever
+    workspace the forward had; the other one the planes both ways, whatever was set between the two calls.  The bound is
+    relative: mixing the two doubles the largest error at least (printed), statistics that differ in the last bits of
+    their sums, or another order of the chunks, move it by a few per cent."""
+    from verl_amd import _abi
+    from verl_amd.utils.kernel import kernels
+
+    lib = _abi.load()
+    T, H, V, tau = 512, 1024, 40960, 0.6
+    g = torch.Generator().manual_seed(1)
+    h = torch.randn(T, H, generator=g).to(DEV)
+    w = (torch.randn(V, H, generator=g) * std).to(DEV)
+    y = torch.randint(0, V, (T,), generator=g).to(DEV)
+    g_lp, g_ent = (torch.randn(T, generator=g).to(DEV) for _ in range(2))
+    want, _ = O.lce_backward(g_lp, g_ent, h, w, y, tau, compute_dtype=torch.float64)
+    worst = {}
+    stats = {"full": _forward(lib, _abi.DTYPE_F32, "full", h, w, y, tau)[2:], "static": _forward(lib, _abi.DTYPE_F32, "static", h, w, y, tau)[2:],
+             "small": _forward(lib, _abi.DTYPE_F32, "small", h, w, y, tau)[2:], "planes": _forward(lib, _abi.DTYPE_F32_PLANES, "full", h, w, y, tau)[2:]}
+    for name, code in (("full", _abi.DTYPE_F32), ("static", _abi.DTYPE_F32), ("small", _abi.DTYPE_F32), ("planes", _abi.DTYPE_F32_PLANES)):
+        dh, _ = _backward(lib, code, h, w, y, tau, stats[name], g_lp, g_ent)
+        worst[name] = ((dh.double() - want).abs().max() / want.abs().max()).item()
+    _, _, *kept = kernels.efficient_entropy_forward(h, w, y, 0, tau)
+    kernels.set_workspace_budget(64 << 20)  # (less than the smallest workspace of the planes here, 71 MB)
+    try:
+        dh, _ = kernels.efficient_entropy_backward(g_lp, g_ent, h, w, y, *kept, 0, False, tau)
+    finally:
+        kernels.set_workspace_budget(0)
+    worst["budget"] = ((dh.double() - want).abs().max() / want.abs().max()).item()
+    for a, b in (("static", "planes"), ("planes", "full")):  # (for the record: the two mixtures)
+        dh, _ = _backward(lib, _abi.DTYPE_F32_PLANES if a == "static" else _abi.DTYPE_F32, h, w, y, tau, stats[a], g_lp, g_ent)
+        print(f"std {std}: statistics of {a}, logits of {b}: {((dh.double() - want).abs().max() / want.abs().max()).item():.2e}")
+    print(f"std {std}:", {k: f"{v:.2e}" for k, v in worst.items()})
+    assert max(worst["static"], worst["small"]) < 1.2 * worst["full"] and worst["budget"] < 1.2 * worst["planes"], worst
+    assert worst["planes"] < 1.2 * worst["full"], worst

@@ -13,6 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("LCE_LIBRARY_PATH") or os.path.join(_HERE, "lib", "liblce_gfx950.so")
 
 DTYPE_BF16, DTYPE_F32, DTYPE_F16 = 0, 1, 2
+DTYPE_F32_PLANES = 3  # fp32 with leave to use the bfloat16 matrix pipe: the fused head, forward and backward alike
 ABI_VERSION = 11
 
 # every symbol include/lce_abi.h declares: name -> (restype, argtypes)

@@ -198,14 +198,11 @@ static size_t forward_workspace_need(int64_t T, int64_t V, int max_splits) {
   return align256((size_t)forward_splits_upper_bound(T, V > 0 ? V : 1, max_splits) * (size_t)T * 16) + 2 * align256((size_t)T * 4);
 }
 
-// ... and what the bfloat16 planes of fp32 inputs take on top, where they are used (0: they are not)
-static size_t forward_terms_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype) {
-  if (T <= 0 || H <= 0 || V <= 0 || !use_terms(tu, T, H, V, dtype)) return 0;
-  return terms_fwd_plan(T, H, V).total;
-}
-
+// (answered for LCE_DTYPE_F32: enough for either code of fp32)
 size_t lce_forward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
-  return std::max(forward_workspace_need(T, V, kMaxSplits), forward_terms_need(tuning_snapshot(), T, H, V, dtype));
+  const size_t need = forward_workspace_need(T, V, kMaxSplits);
+  if (T <= 0 || H <= 0 || V <= 0 || (dtype != LCE_DTYPE_F32 && dtype != LCE_DTYPE_F32_PLANES) || !use_terms(tuning_snapshot(), T, H, V)) return need;
+  return dtype == LCE_DTYPE_F32 ? std::max(need, terms_fwd_plan(T, H, V).total) : terms_fwd_plan(T, H, V).total;
 }
 
 // shared body of lce_forward and lce_forward_shard
@@ -213,6 +210,8 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
                          int64_t H, int64_t V, int dtype, float temperature, int reduction, float* logprobs, float* entropy,
                          float* maximum, float* accumulate, float* entropy_b, void* workspace, size_t workspace_bytes,
                          void* stream, int64_t label_offset, float* shard_out, int max_splits = kMaxSplits, float* xcache = nullptr) {
+  const bool planes = dtype == LCE_DTYPE_F32_PLANES;  // fp32 with leave to use them
+  if (planes) dtype = LCE_DTYPE_F32;
   int rc = check_common(hidden, ldh, weight, ldw, labels, T, H, V, dtype, temperature, reduction);
   if (rc) return rc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -224,10 +223,11 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
     return LCE_OK;
   }
   if (!shard_out && (!logprobs || !entropy || !maximum || !accumulate || !entropy_b)) return fail(LCE_E_ARG, "null output pointer");
-  if (!workspace || workspace_bytes < forward_workspace_need(T, V, max_splits))
-    return fail(LCE_E_WORKSPACE, "forward workspace too small: %zu < %zu", workspace_bytes, forward_workspace_need(T, V, max_splits));
-  char* ws = static_cast<char*>(workspace);
   const Tuning tu = tuning_snapshot();
+  const bool terms = planes && use_terms(tu, T, H, V);
+  const size_t need = terms ? terms_fwd_plan(T, H, V).total : forward_workspace_need(T, V, max_splits);
+  if (!workspace || workspace_bytes < need) return fail(LCE_E_WORKSPACE, "forward workspace too small: %zu < %zu", workspace_bytes, need);
+  char* ws = static_cast<char*>(workspace);
   int sel = tu.variant_fwd;
   if (!tu.variant_forced) {
     if (T <= 64) sel = kSelT64;
@@ -241,9 +241,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   }
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
-  // (lce_forward_static's built-in buffer has no room for the planes: fp32 tiles there)
-  const size_t terms_need = forward_terms_need(tu, T, H, V, dtype);
-  if (terms_need && workspace_bytes >= terms_need) sel = kSelTerms;
+  if (terms) sel = kSelTerms;
   if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
@@ -362,14 +360,17 @@ int lce_merge_shards(const float* partials, int R, int64_t T, int reduction, flo
   return rc;
 }
 
-static size_t backward_workspace_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype, int64_t vchunk) {
-  if (use_terms(tu, T, H, V, dtype)) return terms_bwd_layout(tu, T, H, V, vchunk).total + 256;
-  return bwd_layout(tu, T, H, V, esize(dtype), vchunk).total + 256;
+static size_t backward_workspace_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, size_t esz, int64_t vchunk, bool terms) {
+  return (terms ? terms_bwd_layout(tu, T, H, V, vchunk).total : bwd_layout(tu, T, H, V, esz, vchunk).total) + 256;
 }
 
+// (answered for LCE_DTYPE_F32: enough for either code of fp32)
 size_t lce_backward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype, int64_t vchunk) {
   if (T <= 0 || H <= 0 || V <= 0) return 256;
-  return backward_workspace_need(tuning_snapshot(), T, H, V, dtype, vchunk);
+  const Tuning tu = tuning_snapshot();
+  const bool planes = dtype == LCE_DTYPE_F32_PLANES, f32 = planes || dtype == LCE_DTYPE_F32;
+  const size_t of_planes = f32 && use_terms(tu, T, H, V) ? backward_workspace_need(tu, T, H, V, 4, vchunk, true) : 0;
+  return planes && of_planes ? of_planes : std::max(of_planes, backward_workspace_need(tu, T, H, V, f32 ? 4 : 2, vchunk, false));
 }
 
 // shared body of lce_backward and lce_backward_shard
@@ -378,6 +379,8 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
                           const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
                           void* d_hidden, void* d_weight, void* workspace, size_t workspace_bytes, int64_t vchunk,
                           void* stream, int64_t vocab_offset, bool grads_f32 = false, const float* xcache = nullptr) {
+  const bool planes = dtype == LCE_DTYPE_F32_PLANES;
+  if (planes) dtype = LCE_DTYPE_F32;
   int rc = check_common(hidden, ldh, weight, ldw, labels, T, H, V, dtype, temperature, reduction);
   if (rc) return rc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -393,10 +396,11 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
   if (!aligned16(d_hidden) || !aligned16(d_weight)) return fail(LCE_E_ARG, "gradients must be 16-byte aligned");
   if (vchunk < 0) return fail(LCE_E_ARG, "vchunk must be >= 0");
   const Tuning tu = tuning_snapshot();
-  const size_t need = backward_workspace_need(tu, T, H, V, dtype, vchunk);
+  const bool terms = planes && use_terms(tu, T, H, V);
+  const size_t need = backward_workspace_need(tu, T, H, V, esz, vchunk, terms);
   if (!workspace || workspace_bytes < need) return fail(LCE_E_WORKSPACE, "backward workspace too small: %zu < %zu", workspace_bytes, need);
   char* ws = reinterpret_cast<char*>(align256(reinterpret_cast<size_t>(workspace)));
-  return kBackward[dtype](use_terms(tu, T, H, V, dtype) ? kSelTerms : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
+  return kBackward[dtype](terms ? kSelTerms : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
                           accumulate, entropy_b, dlogprobs, dentropy, d_hidden, d_weight, grads_f32, ws, vchunk, st, vocab_offset,
                           tu, xcache);
 }

@@ -94,17 +94,17 @@ TermsBwdLayout terms_bwd_layout(const Tuning& tu, int64_t T, int64_t H, int64_t 
 }
 
 // ---- which calls ------------------------------------------------------------------------------
-// ONE rule for forward and backward: the backward recomputes the logits, and where a token's distribution is peaked the
-// rounding errors of a logit and of the forward's statistics cancel only if both come from the same arithmetic (2048
-// tokens x 1024 x 8192, temperature 0.6, worst error of d_hidden relative to its largest entry: 4.7e-6 with the fp32 MFMA
-// both ways, 1.3e-5 with the planes in the forward only).  Where the workspace bound has no room for the planes (small
-// vocabularies), both take the fp32 tiles.
+// LCE_DTYPE_F32_PLANES gives leave to use them, in forward and backward alike: the backward recomputes the logits, and where a
+// token's distribution is peaked the rounding errors of a logit and of the forward's statistics cancel only if both come from
+// the same arithmetic.  Measured, worst error of d_hidden against float64 relative to its largest entry (512 tokens, H=1024,
+// V=40960, temperature 0.6, weight std 0.1): fp32 MFMA both ways 9.3e-6, planes both ways 7.1e-6, fp32 MFMA in the forward only
+// 1.8e-5, planes in the forward only 2.0e-5.  A caller without the workspace for a forward on planes (lce_forward_static) has
+// only LCE_DTYPE_F32, the fp32 MFMA in both.  With the leave the rule is one of shapes alone, so that nothing set between the
+// two calls can part them: the planes where the default workspace bound has room for them (not for small vocabularies).
 constexpr int64_t kTermsMinTokens = 256;
-bool use_terms(const Tuning& tu, int64_t T, int64_t H, int64_t V, int dtype) {
-  if (dtype != LCE_DTYPE_F32 || tu.variant_forced || T < kTermsMinTokens || H % 64 != 0) return false;
-  double gate = (double)T * V + 4.0 * (double)V * H;
-  if (tu.ws_budget > 0 && (double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
-  return (double)terms_bwd_layout(tu, T, H, V, 0).total + 512.0 <= gate;
+bool use_terms(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
+  if (tu.variant_forced || T < kTermsMinTokens || H % 64 != 0) return false;  // (a forced variant: diagnostics)
+  return (double)terms_bwd_layout(Tuning(), T, H, V, 0).total + 512.0 <= (double)T * V + 4.0 * (double)V * H;
 }
 
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1

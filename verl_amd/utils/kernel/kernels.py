@@ -123,7 +123,8 @@ def _check_inputs(hidden, weight, labels):
         raise NotImplementedError(f"hidden ({hidden.dtype}) and weight ({weight.dtype}) must share a dtype")
     if labels.dtype != torch.int64:
         raise NotImplementedError(f"labels must be int64, got {labels.dtype}")
-    return _abi.dtype_code(hidden.dtype)
+    # (forward and backward both come here, so the two always agree on how fp32 products are taken)
+    return _abi.DTYPE_F32_PLANES if hidden.dtype == torch.float32 else _abi.dtype_code(hidden.dtype)
 
 
 def efficient_entropy_forward(
