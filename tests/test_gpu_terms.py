@@ -125,3 +125,50 @@ def test_statistics_and_logits_come_from_the_same_arithmetic(std):
     print(f"std {std}:", {k: f"{v:.2e}" for k, v in worst.items()})
     assert max(worst["static"], worst["small"]) < 1.2 * worst["full"] and worst["budget"] < 1.2 * worst["planes"], worst
     assert worst["planes"] < 1.2 * worst["full"], worst
+
+
+@pytest.mark.parametrize("where", ["weight -inf", "weight +inf", "weight NaN", "weight beyond bfloat16", "hidden inf", "last hidden -inf"])
+def test_infinities_and_values_beyond_bfloat16(where):
+    """An infinity, and a finite value beyond the largest bfloat16, in either operand: what the planes make of it is finite
+    exactly where the fp32 MFMA's result is, and the same there.  (A weight of -inf whose logit comes out as -inf leaves the
+    other rows' log-probs alone; a token with an infinity spoils its own values only.)"""
+    from verl_amd import _abi
+
+    lib = _abi.load()
+    T, H, V, tau = 300, 128, 40011, 0.8
+    assert lib.lce_forward_workspace_bytes(T, H, V, _abi.DTYPE_F32_PLANES) > lib.lce_forward_workspace_bytes(T, H, V, _abi.DTYPE_BF16)
+    g = torch.Generator().manual_seed(2)
+    h = torch.randn(T, H, generator=g).to(DEV)
+    w = (torch.randn(V, H, generator=g) * 0.05).to(DEV)
+    y = torch.randint(0, V, (T,), generator=g).to(DEV)
+    h[:, 5] = h[:, 5].abs() + 0.25  # one sign, so that an infinite weight gives logits of one sign
+    h[:7, 5] = torch.tensor([1.0, 0.5, 2.0, 1.5, 3.0, 300.0, 299.7])  # (without small terms; large ones)
+    y[3] = 17
+    value = {"weight -inf": -float("inf"), "weight +inf": float("inf"), "weight NaN": float("nan"), "weight beyond bfloat16": -3.4e38}.get(where)
+    if value is not None:
+        w[17, 5] = w[V - 1, 5] = value
+    elif where == "hidden inf":
+        h[7, 3] = float("inf")
+    else:
+        h[T - 1, H - 1] = -float("inf")
+    g_lp, zero = torch.randn(T, generator=g).to(DEV), torch.zeros(T, device=DEV)
+
+    def same(a, b, what, rel):
+        assert torch.equal(a.isfinite(), b.isfinite()), f"{what}: {a.isfinite().sum()} of {a.numel()} values are finite, {b.isfinite().sum()} on the fp32 MFMA"
+        ok = b.isfinite()
+        if ok.any():
+            assert (a[ok] - b[ok]).norm() <= rel * b[ok].norm(), what
+        return int(ok.sum())
+
+    both = []
+    for code in (_abi.DTYPE_F32_PLANES, _abi.DTYPE_F32):
+        out = _forward(lib, code, "full", h, w, y, tau)
+        both.append(out + list(_backward(lib, code, h, w, y, tau, out[2:], g_lp, zero)))
+    # 2-norm, relative: the two ways round a logit differently, by some 2^-24 of its size, and the gradients of a token follow its
+    # logits' absolute error; the largest logits here are about 300 x 0.05 x 4 / 0.8
+    rel = 8 * 75 * 2.0**-24
+    finite = [same(a, b, what, rel) for a, b, what in zip(*both, ["logprobs", "entropy", "maximum", "accumulate", "entropy_b", "d_hidden", "d_weight"])]
+    if where in ("weight -inf", "weight beyond bfloat16"):
+        assert finite[0] >= T - 1
+    elif where.endswith("inf") and "hidden" in where:
+        assert finite[0] == T - 1

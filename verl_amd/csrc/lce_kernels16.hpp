@@ -708,31 +708,101 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   Core::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
 }
 
-// fp32 rows as three bfloat16 planes, out[r] = three runs of ldo elements: x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 -
-// x2); the differences are exact, so x1 + x2 + x3 = x down to the smallest bfloat16.  Row r is in[rows[r]] (in[r] without
-// `rows`) for r < R = *n_rows (R without), zeros up to the next multiple of 64.  Eight elements per thread; C a multiple of 8.
-inline __global__ void split_planes_kernel(const float* in, int64_t ldi, int64_t R, int64_t C, bf16_t* out, int64_t ldo, int64_t rpad, const int* rows,
-                                           const int* n_rows) {
-  if (n_rows) R = *n_rows;
-  const int64_t rend = (R + 63) / 64 * 64 < rpad ? (R + 63) / 64 * 64 : rpad;
-  const int64_t per_row = C / 8, n = rend * per_row;
+// fp32 rows as three bfloat16 planes, out[r] = three runs of ldo elements.  Row r is in[rows[r]] (in[r] without `rows`) for
+// r < R = *n_rows (R without), zeros up to the next multiple of 64.  Eight elements per thread; C a multiple of 8.
+struct SplitArgs {
+  const float* in;
+  int64_t ldi, R, C;
+  bf16_t* out;
+  int64_t ldo, rpad;
+  const int *rows, *n_rows;
+};
+
+// Nearest terms: x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2); the differences are exact, so x1 + x2 + x3 = x down to
+// the smallest bfloat16.  An infinity would be (inf, NaN, NaN), and its products with the small terms of the other operand,
+// which are zeros or of either sign, NaN: values from kWide on are left to split_same_sign.
+constexpr uint32_t kWide = 0x5d000000u;  // 2^59: products of smaller values, and any sum of them, stay far from overflow
+LCE_DEV void split_nearest(const float (&x)[8], float (&p)[3][8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float rest = x[e];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      p[t][e] = (float)(bf16_t)rest;
+      rest -= p[t][e];
+    }
+  }
+}
+
+// Terms of x's own sign, none of them zero unless x is: cut off instead of rounded (3 x 8 bits hold all 24), a zero term
+// replaced by |x| 2^-40.  Every product of an infinity is then an infinity of the right sign, with zero NaN, and so is the sum
+// of the six; a finite value beyond the largest bfloat16 stays finite.  Not for ordinary values: the three products that
+// are left out do not average out over the signs (4e-8 of a product of N(0,1) values on average, as much as an fp32 rounding).
+LCE_DEV void split_same_sign(const float (&x)[8], float (&p)[3][8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, x[e]);
+    const float least = __builtin_copysignf(fmaxf(fabsf(x[e]) * 0x1p-40f, 0x1p-126f), x[e]);
+    float rest = x[e];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const float cut = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, rest) & 0xffff0000u);
+      p[t][e] = cut == 0.f ? least : cut;
+      rest -= cut;
+    }
+    if ((bits & 0x7f800000u) == 0x7f800000u || (bits & 0x7fffffffu) == 0u) {  // infinities, NaN and zero
+      const bool inf = (bits & 0x7fffffffu) == 0x7f800000u;
+      p[0][e] = x[e];
+      p[1][e] = p[2][e] = inf ? __builtin_copysignf(1.f, x[e]) : x[e];
+    }
+  }
+}
+
+template <bool SAME_SIGN>
+LCE_DEV uint32_t split_rows(const SplitArgs& s) {  // returns the largest magnitude this thread has seen, as bits
+  const int64_t R = s.n_rows ? (int64_t)*s.n_rows : s.R;
+  const int64_t rend = (R + 63) / 64 * 64 < s.rpad ? (R + 63) / 64 * 64 : s.rpad;
+  const int64_t per_row = s.C / 8, n = rend * per_row;
+  uint32_t most = 0;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
     const int64_t r = q / per_row, c = (q - r * per_row) * 8;
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (r < R) {
-      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(in + (rows ? (int64_t)rows[r] : r) * ldi + c);
+      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(s.in + (s.rows ? (int64_t)s.rows[r] : r) * s.ldi + c);
       const f32x4_t lo = src[0], hi = src[1];
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = e < 4 ? lo[e & 3] : hi[e & 3];
     }
-    bf16_t* dst = out + r * 3 * ldo + c;
+    float p[3][8];
+    if (SAME_SIGN) {
+      split_same_sign(x, p);
+    } else {
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      store_run<bf16_t, 8>(dst + t * ldo, x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] -= (float)(bf16_t)x[e];
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t magnitude = __builtin_bit_cast(uint32_t, x[e]) & 0x7fffffffu;
+        most = magnitude > most ? magnitude : most;
+      }
+      split_nearest(x, p);
     }
+    bf16_t* dst = s.out + r * 3 * s.ldo + c;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) store_run<bf16_t, 8>(dst + t * s.ldo, p[t]);
   }
+  return most;
+}
+
+// *wide (zero before a call's first launch): some value of the operands split so far is infinite, NaN or kWide and more
+inline __global__ void split_planes_kernel(SplitArgs s, int* wide) {
+  if (split_rows<false>(s) >= kWide) __hip_atomic_store(wide, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Behind every chunk's split: where such a value has been met, both operands are split again, with terms of one sign.  (It
+// may be in either of them and needs the other one's terms that way too.)  Otherwise nothing: 2 us per launch, against a
+// second read of both operands to know beforehand.
+inline __global__ void split_again_kernel(const int* wide, SplitArgs a, SplitArgs b) {
+  if (*wide == 0) return;
+  (void)split_rows<true>(a);
+  (void)split_rows<true>(b);
 }
 
 // ------------------------------------------------------------------------------------------------

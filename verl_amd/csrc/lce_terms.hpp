@@ -17,7 +17,7 @@ namespace {
 struct TermsFwdPlan {
   int64_t rows;     // vocabulary rows of a chunk
   int nchunks, splits;  // splits: of all chunks together
-  size_t off_xlabel, off_lp, off_h, off_w, total;
+  size_t off_xlabel, off_lp, off_wide, off_h, off_w, total;
 };
 
 int terms_fwd_splits(int ntt, int64_t rows) { return forward_splits_256(ntt, (int)((rows + 255) / 256)); }
@@ -39,6 +39,7 @@ TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V) {
   size_t o = align256((size_t)p.splits * T * 16);
   p.off_xlabel = o; o += align256((size_t)T * 4);
   p.off_lp = o;     o += align256((size_t)T * 4);
+  p.off_wide = o;   o += 256;
   p.off_h = o;      o += align256((size_t)round_up(T, 64) * 3 * H * 2);
   p.off_w = o;      o += align256((size_t)std::min<int64_t>(p.rows, round_up(V, 64)) * 3 * H * 2);
   p.total = o;
@@ -110,12 +111,16 @@ bool use_terms(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1
 typedef GemmCfg16<bf16_t, 0, 8, 0, 6> TermsCfg;
 
-int launch_split(const float* in, int64_t ld, int64_t R, int64_t C, bf16_t* out, int64_t ldo, int64_t rpad, const int* rows, const int* n_rows,
-                 hipStream_t st) {
+// The planes of one operand (`s`), and then, where that or the other one (`also`, null: not there yet) holds values that want
+// it, those of both once more (split_again_kernel).
+int launch_split(const SplitArgs& s, const SplitArgs* also, int* wide, hipStream_t st) {
   ProfScope prof(PC_TRANSPOSE, st);
-  const int64_t blocks = (rpad * (C / 8) + 255) / 256;
-  hipLaunchKernelGGL(split_planes_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, in, ld, R, C, out, ldo, rpad, rows, n_rows);
-  return check_launch("split_planes_kernel");
+  const int64_t blocks = (s.rpad * (s.C / 8) + 255) / 256;
+  hipLaunchKernelGGL(split_planes_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, s, wide);
+  int rc = check_launch("split_planes_kernel");
+  if (rc || !also) return rc;
+  hipLaunchKernelGGL(split_again_kernel, dim3(kNumCUs), dim3(256), 0, st, wide, *also, s);
+  return check_launch("split_again_kernel");
 }
 
 int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
@@ -124,8 +129,12 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
   const TermsFwdPlan pl = terms_fwd_plan(T, H, V);
   bf16_t* h3 = reinterpret_cast<bf16_t*>(ws + pl.off_h);
   bf16_t* w3 = reinterpret_cast<bf16_t*>(ws + pl.off_w);
-  int rc = launch_split(h, ldh, T, H, h3, H, round_up(T, 64), nullptr, nullptr, st);
+  int* wide = reinterpret_cast<int*>(ws + pl.off_wide);
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<uint32_t*>(wide), (int64_t)1);
+  int rc = check_launch("fill_zero_kernel");
   if (rc) return rc;
+  const SplitArgs sh = {h, ldh, T, H, h3, H, round_up(T, 64), nullptr, nullptr};
+  if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
   const int ntt = (int)((T + 255) / 256);
   FwdArgs<bf16_t> p;
   p.W = w3; p.ldw = 3 * H; p.h = h3; p.ldh = 3 * H; p.labels = labels; p.T = T; p.H = H;
@@ -137,7 +146,7 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
   int done = 0;
   for (int c = 0; c < pl.nchunks; ++c) {
     const int64_t v0 = c * pl.rows, rows = std::min(pl.rows, V - v0);
-    if ((rc = launch_split(W + v0 * ldw, ldw, rows, H, w3, H, rows, nullptr, nullptr, st))) return rc;
+    if ((rc = launch_split({W + v0 * ldw, ldw, rows, H, w3, H, rows, nullptr, nullptr}, &sh, wide, st))) return rc;
     p.S = std::min<int>(terms_fwd_splits(ntt, rows), (int)((rows + 255) / 256));
     p.V = rows;
     p.label_offset = label_offset + v0;
@@ -168,6 +177,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   int* rows = reinterpret_cast<int*>(ws + L.off_rows);
   int* inv = reinterpret_cast<int*>(ws + L.off_inv);
   int* n_rows = reinterpret_cast<int*>(ws + L.off_nrows);
+  int* wide = n_rows + 1;
   f32x4_t* tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
   int* tokl = reinterpret_cast<int*>(ws + L.off_tokl);
   const int64_t g_stride = reduction == LCE_REDUCTION_NONE ? 1 : 0;
@@ -185,7 +195,10 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
                        g_scale, dentropy, maximum, accumulate, entropy_b, labels, vocab_offset, V, 1.0f / temperature, tokc, tokl);
     if ((rc = check_launch("ds_token_consts_kernel"))) return rc;
   }
-  if ((rc = launch_split(h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows, st))) return rc;
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<uint32_t*>(wide), (int64_t)1);
+  if ((rc = check_launch("fill_zero_kernel"))) return rc;
+  const SplitArgs sh = {h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows};
+  if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
   const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN);
   // launch c: d_logits of chunk c and the gradient GEMMs of chunk c - 1, as in backward_impl
   for (int c = 0; c <= L.nchunks; ++c) {
@@ -194,7 +207,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
     if (c < L.nchunks) {
       const int64_t v0 = (int64_t)c * L.vchunk, vrows = std::min(L.vchunk, V - v0);
       // (the last reader of this buffer, d_hidden of chunk c - 2, ran in the launch before the last)
-      if ((rc = launch_split(W + v0 * ldw, ldw, vrows, H, w3[c & 1], H, vrows, nullptr, nullptr, st))) return rc;
+      if ((rc = launch_split({W + v0 * ldw, ldw, vrows, H, w3[c & 1], H, vrows, nullptr, nullptr}, &sh, wide, st))) return rc;
       DsArgs<bf16_t>& d = p.ds;
       d.W = w3[c & 1]; d.ldw = 3 * H; d.h = h3; d.ldh = 3 * L.ldH; d.labels = labels; d.T = T; d.H = H;
       d.w_plane = H * 2; d.h_plane = L.ldH * 2; d.dS_plane = L.plane;
