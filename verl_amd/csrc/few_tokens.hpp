@@ -69,9 +69,8 @@ struct FewFwdShape {
   static constexpr int LDS_BYTES = 2 * STAGE + 8 * 4096;  // two stages, a store tile per wave
 };
 
-template <typename TIN>
-__global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
+template <typename TIN, int AUX>
+LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache policy of the loads of W
   typedef FewFwdShape S;
   constexpr int DEPTH = S::DEPTH, FN = S::FN, NT = S::NT;
   constexpr int WL = S::BM / 64;  // 16-byte chunks of a W stage per thread: row tid / 8 + 64 i, chunk tid % 8 (hidden: one)
@@ -105,7 +104,7 @@ __global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
     const buf_t wb = make_buf(p.W + f_row * p.ldw + 64 * (int64_t)f_k, live ? left * w_row - 128 * (int64_t)f_k : 0);
     const buf_t hb = make_buf(p.h + 64 * (int64_t)f_k, live ? p.T * h_row - 128 * (int64_t)f_k : 0);
 #pragma unroll
-    for (int i = 0; i < WL; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(wb, (int)(w_at + 64 * i * w_row), 0, kBufNonTemporal);
+    for (int i = 0; i < WL; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(wb, (int)(w_at + 64 * i * w_row), 0, AUX);
     x = __builtin_amdgcn_raw_buffer_load_b128(hb, (int)h_at, 0, 0);
     __builtin_amdgcn_sched_barrier(0);  // (the loads of one stage stay in front of the next one's)
     if (++f_k == n_kp) {
@@ -201,6 +200,14 @@ __global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
     }
     if (t < p.T) p.parts[(int64_t)blockIdx.x * p.T + t] = f32x4_t{vm, va, vb, 0.f};
   }
+}
+
+// (which rows are read how: read_w_once, lce_host.hpp.  A branch around the whole body: none around a load.)
+template <typename TIN>
+__global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  if ((int64_t)blockIdx.x * p.split_stride < p.once_rows) fwd_few_body<TIN, kBufNonTemporal>(p, lds);
+  else fwd_few_body<TIN, 0>(p, lds);
 }
 
 template <typename TIN>

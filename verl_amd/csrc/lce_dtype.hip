@@ -38,13 +38,17 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case 2: LCE_RUN(Variant2);
     case 3: LCE_RUN(Variant3);
     case kSelN192: LCE_RUN(VariantN192);
-    case kSelT128: LCE_RUN(VariantT128);
+    case kSelT128:
+      if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT128Plain);
+      LCE_RUN(VariantT128);
 #if LCE_TU_DTYPE != 1
     case kSelT64:
       return forward_few<TuT>((const TuT*)h, ldh, (const TuT*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
                               label_offset, shard_out, max_splits, xcache);
 #else
-    case kSelT64: LCE_RUN(VariantT64);
+    case kSelT64:
+      if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT64Plain);
+      LCE_RUN(VariantT64);
     case kSelTerms:
       return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
                            label_offset, shard_out);

@@ -150,9 +150,12 @@ template <typename TIN> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6, 1> Cfg
 template <> struct VariantN192<float> : Variant3<float> {};
 // the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us)
 template <typename TIN> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1> Cfg; };
-// forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring
-template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
-template <typename TIN> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, 1> Cfg; };
+// forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring.  ONCE: the loads of W
+// are marked non-temporal (read_w_once)
+template <typename TIN, int ONCE = 1> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, ONCE> Cfg; };
+template <typename TIN, int ONCE = 1> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, ONCE> Cfg; };
+template <typename TIN> using VariantT64Plain = VariantT64<TIN, 0>;
+template <typename TIN> using VariantT128Plain = VariantT128<TIN, 0>;
 constexpr int kNumVariants = 4;
 
 template <typename K>
@@ -160,6 +163,21 @@ void allow_lds(K kernel, int bytes) {
   // dynamic LDS above 64 KiB has to be enabled per kernel; cheap and idempotent
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
+
+// Few tokens: are all of the forward's loads of W marked non-temporal?  W is read once per call, and this card reads 1.09 GB at
+// 7.0 TB/s with such loads and at 6.3 without; so yes where it is large next to the memory-side cache, and where a backward
+// follows, whose writes of d_weight would have to leave the cache before plain loads could enter it (64 tokens, H=3584: step
+// 650 us, 680 with plain loads of the last 64 MB).  But lines that the cache holds because W has just been written (made,
+// loaded, copied) are read faster with plain loads.  So without a backward and with W up to 5/4 of the cache, up to 64 tokens
+// read the last 64 MB of W plainly (a quarter of the cache: several weights in turn still find their parts there) and the
+// rest not, 65 to 128 tokens all of it.  H=896, V=151936 (260 MB), us: all non-temporal / this rule / all plain, 40 tokens:
+// repeated 54.1 / 53.8 / 54.0, three weights in turn 54.3 / 53.7 / 59.5, right after W was drawn 64.4 / 58.9 / 66.4, copied
+// 63.2 / 59.4 / 62.0, behind a large read 56.4 / 56.8 / 60.3, a large write 56.7 / 76.6 / 113.7, and W scaled in place 74.2 /
+// 73.7 / 60.7, the one pattern that stays slower; 100 tokens, all non-temporal / plain: repeated 68.0 / 60.6, three weights
+// 68.5 / 67.9, drawn 80.1 / 75.7, copied 80.8 / 74.7, scaled 91.2 / 69.5, behind a read 71.8 / 68.8, a write 70.4 / 118.9.
+// At 342 MB the two are level, at 445 MB non-temporal loads win (40 tokens: 83.4 against 92.5 plain).
+constexpr int64_t kMallBytes = (int64_t)256 << 20;  // the memory-side cache
+bool read_w_once(int64_t V, int64_t row_bytes, const float* xcache) { return xcache || V * row_bytes > kMallBytes * 5 / 4; }
 
 int block_rows(int nrow_tiles) { return TileMap::block_rows(nrow_tiles); }
 
@@ -347,7 +365,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   p.split_span = rows_per_split ? rows_per_split : V;
   p.label_offset = label_offset;
   // xcache: the raw logits are kept for the backward
-  p.xcache = xcache; p.w_plane = p.h_plane = 0;
+  p.xcache = xcache; p.w_plane = p.h_plane = 0; p.once_rows = 0;
   p.map = TileMap::make(ntt, S, br, 1);
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   int rc;
@@ -387,6 +405,7 @@ int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int6
   p.parts = reinterpret_cast<f32x4_t*>(ws);
   p.xlabel = reinterpret_cast<float*>(ws + align256((size_t)S * T * 16));
   p.S = S; p.tile_step = 256; p.label_offset = label_offset; p.xcache = xcache; p.w_plane = p.h_plane = 0;
+  p.once_rows = read_w_once(V, ldw * (int64_t)sizeof(TIN), xcache) ? V : V - kMallBytes / 4 / (ldw * (int64_t)sizeof(TIN));
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   {
     ProfScope prof(PC_FWD, st);

@@ -141,7 +141,7 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
   p.w_plane = p.h_plane = H * 2;
   p.c = kLog2e / temperature;
   p.xlabel = reinterpret_cast<float*>(ws + pl.off_xlabel);
-  p.xcache = nullptr;
+  p.xcache = nullptr; p.once_rows = 0;
   f32x4_t* parts = reinterpret_cast<f32x4_t*>(ws);
   int done = 0;
   for (int c = 0; c < pl.nchunks; ++c) {
