@@ -95,20 +95,7 @@ class _Packed:
             self.checks()
 
 
-def _grad_bytes(total):
-    return (total * 4 + 255) // 256 * 256
-
-
-def _parts(call, keep, with_log_prob, with_entropy, total):
-    """Sets what of the call lies in ``keep``: the workspace, then the unscaled gradients of ``total`` elements each.
-    Returns the address behind them, where a packed batch has its lengths."""
-    at = keep.data_ptr()
-    call.workspace = at
-    at += call.workspace_bytes
-    call.g_log_prob = at if with_log_prob else None
-    call.g_entropy = at + _grad_bytes(total) if with_entropy else None
-    return at + 2 * _grad_bytes(total)
-
+_POINTERS = _abi.PpoCall.total_nnz.offset  # bytes of the call that are addresses
 
 # a tensor that stands for a batch of them: what autograd hands a backward under is_grads_batched, and what vmap does
 _is_legacy_batched = torch._C._functorch.is_legacy_batchedtensor
@@ -154,12 +141,17 @@ class _FusedPPOLoss(torch.autograd.Function):
         call.rows, call.row_len, call.total_nnz = rows, row_len, -1 if packed is None else total
         lib = _abi.load()
         call.workspace_bytes = lib.lce_ppo_loss_workspace_bytes(rows, row_len)
-        # one allocation (see _parts)
+        # one allocation: workspace, the unscaled gradients, and the lengths of a packed batch
+        grad_bytes = (total * 4 + 255) // 256 * 256
         count_lens = packed is not None and packed.attention_mask is not None
-        keep = torch.empty(call.workspace_bytes + 2 * _grad_bytes(total) + (16 * rows if count_lens else 0), device=dev, dtype=torch.uint8)
+        keep = torch.empty(call.workspace_bytes + 2 * grad_bytes + (16 * rows if count_lens else 0), device=dev, dtype=torch.uint8)
         out = torch.empty(16, device=dev, dtype=torch.float32)
-        call.out = out.data_ptr()
-        at = _parts(call, keep, lp is not None, ent is not None, total)
+        at = keep.data_ptr()
+        call.workspace, call.out = at, out.data_ptr()
+        at += call.workspace_bytes
+        call.g_log_prob = at if lp is not None else None
+        call.g_entropy = at + grad_bytes if ent is not None else None
+        at += 2 * grad_bytes
         ptr = _abi.ptr
         call.log_prob, call.entropy, call.old_log_prob, call.advantages = ptr(lp), ptr(ent), ptr(old), ptr(adv)
         call.mask, call.is_weights, call.ref_log_prob = mask.data_ptr(), ptr(isw), ptr(ref)
@@ -183,10 +175,10 @@ class _FusedPPOLoss(torch.autograd.Function):
                 packed.launched(call, stream, ticket)
         ctx.save_for_backward(keep, *lens)
         ctx.set_materialize_grads(False)  # (the vector of statistics takes no gradient: no zeros are made for it)
-        # (the numbers of the call, without a pointer: where things are is worked out anew in the backward)
+        # for the backward: the numbers of the call, and where in the buffer things are (which may be elsewhere by then); no address
         ctx.numbers = _abi.PpoCall.from_buffer_copy(call)
-        ctypes.memset(ctypes.addressof(ctx.numbers), 0, _abi.PpoCall.total_nnz.offset)
-        ctx.counted = count_lens
+        ctypes.memset(ctypes.addressof(ctx.numbers), 0, _POINTERS)
+        ctx.parts = (call.workspace_bytes, grad_bytes, count_lens)
         ctx.like = tuple(None if t is None else (t.shape, t.dtype) for t in (log_prob, entropy))
         ctx.mark_non_differentiable(out)
         return out[0], out
@@ -197,26 +189,31 @@ class _FusedPPOLoss(torch.autograd.Function):
             return (None,) * 15
         keep, *lens = ctx.saved_tensors
         dev = keep.device
-        assert keep.is_cuda and g_loss.device == dev and all(t.device == dev for t in lens), "the loss's saved tensors are on another device"
-        if keep.data_ptr() % 16:  # (a saved-tensor hook may bring it back anywhere)
+        assert keep.is_cuda and g_loss.device == dev, "the loss's saved tensors are on another device"
+        at = keep.data_ptr()
+        if at % 16:  # (a saved-tensor hook may bring it back anywhere)
             keep = keep.clone()
+            at = keep.data_ptr()
         # An upstream gradient that is itself differentiated (create_graph) or stands for a batch of them (is_grads_batched)
         # is multiplied on by torch; otherwise the kernel reads it where it is.
-        traced = (torch.is_grad_enabled() and g_loss.requires_grad) or _is_legacy_batched(g_loss) or _is_wrapped(g_loss)
+        traced = (g_loss.requires_grad and torch.is_grad_enabled()) or _is_legacy_batched(g_loss) or _is_wrapped(g_loss)
         if traced:
             up = torch.ones((), device=dev, dtype=torch.float32)
         else:
             up = g_loss if g_loss.dtype == torch.float32 else g_loss.to(torch.float32)
         call = _abi.PpoCall.from_buffer_copy(ctx.numbers)
+        ws_bytes, grad_bytes, count_lens = ctx.parts
+        call.workspace, call.g_log_prob, call.g_entropy = at, at + ws_bytes, at + ws_bytes + grad_bytes
+        if count_lens:
+            at += ws_bytes + 2 * grad_bytes
+            call.prompt_lens, call.response_lens = at, at + 8 * call.rows
+        elif lens:
+            assert lens[0].device == lens[1].device == dev, "the loss's saved tensors are on another device"
+            call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
         grads = [
             torch.empty(like[0], device=dev, dtype=torch.float32) if like is not None and ctx.needs_input_grad[k] else None
             for k, like in enumerate(ctx.like)
         ]
-        at = _parts(call, keep, *(like is not None for like in ctx.like), next(like for like in ctx.like if like is not None)[0].numel())
-        if ctx.counted:
-            call.prompt_lens, call.response_lens = at, at + 8 * call.rows
-        elif lens:
-            call.prompt_lens, call.response_lens = lens[0].data_ptr(), lens[1].data_ptr()
         call.g_loss, call.d_log_prob, call.d_entropy = up.data_ptr(), _abi.ptr(grads[0]), _abi.ptr(grads[1])
         with _abi.on_device(dev):
             _abi.check(_abi.load().lce_ppo_backward(ctypes.addressof(call), _abi.current_stream(dev)), "lce_ppo_backward")
