@@ -107,3 +107,20 @@ def test_no_accumulator_is_read_before_it_is_there(tmp_path):
             assert wrong is None, f"{name}: {wrong}"
             looked, kernels = looked + n, kernels + (n > 0)
     assert kernels >= 12 and looked >= 12 * 64, (kernels, looked)  # (forward, d_logits and gradient GEMMs of three element types)
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
+def test_no_kernel_of_the_loop_uses_scratch_memory(tmp_path):
+    """A reload from scratch memory waits for every load and store issued before it, the next tile's among them."""
+    lib = shutil.copy(_abi.LIB_PATH, tmp_path)
+    subprocess.run([OBJDUMP, "--offloading", lib], check=True, capture_output=True, cwd=tmp_path, timeout=120)
+    readelf = os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf")
+    seen = set()
+    for f in sorted(os.listdir(tmp_path)):
+        if not f.endswith("amdgcn-amd-amdhsa--gfx950"):
+            continue
+        notes = subprocess.run([readelf, "--notes", str(tmp_path / f)], check=True, capture_output=True, text=True, timeout=120).stdout
+        for name, rest in re.findall(r"\.name:\s+(\S*GemmCfg16\S*)(.*?)\.wavefront_size", notes, re.S):
+            assert re.search(r"\.private_segment_fixed_size:\s+(\d+)", rest).group(1) == "0", name
+            seen.add(name)
+    assert len(seen) >= 16, seen

@@ -35,11 +35,6 @@ struct Mma16<bf16_t> {
   static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
   }
-  // the same instruction as a builtin: the compiler schedules it and knows its latency
-  static LCE_DEV f32x4_t known(const f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), acc, 0, 0, 0);
-  }
 };
 template <>
 struct Mma16<f16_t> {
@@ -48,10 +43,6 @@ struct Mma16<f16_t> {
   }
   static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
-  }
-  static LCE_DEV f32x4_t known(const f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), acc, 0, 0, 0);
   }
 };
 
@@ -382,13 +373,13 @@ struct GemmCore16 {
     retire(acc);
   }
 
-  // The accumulators are read by ordinary instructions from here on: let the last MFMAs retire.  The MFMAs are inline
-  // assembly, so the compiler knows nothing of their latency, and it is free to place a copy of an accumulator (for the
-  // epilogue, or to spill it) right behind the statement that last wrote it, ahead of this wait (seen in a variant of
-  // the forward: accumulators copied to scratch a few instructions behind the last MFMA, wrong statistics).  Only the
-  // last blocks of the k-step can still be in the matrix pipe when the loop ends, so the last row of blocks is passed
-  // through one more MFMA that the compiler does know (zero operands: acc + 0): behind a builtin it keeps the
-  // distance to a read itself, and the matrix pipe orders it behind the assembly MFMA that wrote the same registers.
+  // The accumulators are read by ordinary instructions from here on: let the last MFMAs deliver.  They are inline assembly, so
+  // the compiler knows nothing of their latency, and would be free to place a copy of an accumulator right behind the
+  // statement that last wrote it, ahead of this wait (seen once, in a variant that zeroed the accumulators beforehand: copied
+  // to scratch a few instructions behind the last MFMA, wrong statistics).  What keeps it from that is the chain of tied
+  // operands from the first slab's products, which start the accumulators, through every k-step to stay(): there is no other
+  // value to copy in between.  That it holds is checked on the listing of the built library
+  // (tests/test_mfma_distance_on_cpu.py), not assumed.
   static LCE_DEV void retire(f32x4_t (&acc)[NB][NBN]) {
     asm volatile("s_nop 15\n\ts_nop 7" ::);
     stay(acc);

@@ -39,8 +39,11 @@ constexpr int kDefaultVariantFwd = 2, kDefaultVariantBwd = 1, kVariantCore16 = 3
 // tokens on; the backward runs its gradient GEMMs on it wherever the streaming kernels of few_tokens.hpp end)
 constexpr int64_t kCore16MinTokensFwd = 512, kCore16MinTokensBwd = 128;
 // up to here a backward that fits one vocabulary chunk runs its two gradient GEMMs as launches of their own, d_weight on
-// workgroups that stay (lce_dw16_kernel); beyond, a tile's K loop is long enough to hide its start and its stores, and one
-// mixed launch has the shorter tail
+// workgroups that stay (lce_dw16_kernel); beyond, a tile's K loop is long enough to hide most of its start and its stores, and
+// one mixed launch has the shorter tail.  Forward + backward, mixed launch / launches of their own, us: H=3584: 1100 tokens
+// 3422 / 3249, 1400: 4084 / 3985, 1700: 4945 / 4785; H=4096: 1100: 3175 / 3115, 1400: 3820 / 3840, 1700: 4487 / 4537, 2000: 5145 /
+// 5065; H=896: level from 1000 on.  The line lies where token_prep_kernel's range ends.  Beyond it a backward still fits
+// one chunk with H=5120 only (kept logits up to 2560 tokens), where launches of their own would gain 2 % (2300: 9170 / 8965).
 constexpr int64_t kMidMaxTokens = 2048;
 struct Tuning {
   int variant_fwd = kDefaultVariantFwd, variant_bwd = kDefaultVariantBwd;

@@ -361,12 +361,13 @@ LCE_DEV void ds16_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
 // the four accumulator registers of a block are four neighbours in a row of C (one 16-byte or 8-byte access):
 // for C[m][n] = sum_k A[m][k] B[n][k] lane l holds m = 16 j + l % 16 and n = 16 i + 4 (l / 16) + r.
 // ------------------------------------------------------------------------------------------------
-template <typename Cfg, int MODE, bool EDGE>
-LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
-  typedef typename Cfg::TIN TIN;
+// A wave tile that reaches beyond C's last row or column, in fp32, C (+)= acc (ACC: old values are read), in the accumulators'
+// own lane order: 16 rows x 64 bytes per instruction.  (Whole tiles: gemm16_f32_lines.)
+template <typename Cfg, bool ACC>
+LCE_DEV void gemm16_edge(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw) {
   // mw, nw: this lane's row of block column 0 and its first column of block row 0
-  // accumulate modes: the old values of the next AHEAD block columns are on their way while a column is added and stored (the
-  // operand fragments' registers are free by now); one column ahead, a tile's epilogue was 38000 cycles of waiting
+  // the old values of the next AHEAD block columns are on their way while a column is added and stored (the operand fragments'
+  // registers are free by now)
   constexpr int AHEAD = 3;
   f32x4_t prev[AHEAD + 1][Cfg::NB];
   auto fetch = [&](int j) {
@@ -375,10 +376,10 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc
     for (int i = 0; i < Cfg::NB; ++i) {
       const int64_t n = nw + i * 16;
       prev[j % (AHEAD + 1)][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (!(EDGE && (m >= p.M || n >= p.N))) prev[j % (AHEAD + 1)][i] = *reinterpret_cast<const f32x4_t*>(p.Cf + m * p.ldcf + n);
+      if (m < p.M && n < p.N) prev[j % (AHEAD + 1)][i] = *reinterpret_cast<const f32x4_t*>(p.Cf + m * p.ldcf + n);
     }
   };
-  if (MODE & 1) {
+  if (ACC) {
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) fetch(j);
   }
@@ -386,34 +387,24 @@ LCE_DEV void gemm16_epilogue(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc
   for (int j = 0; j < Cfg::NBN; ++j) {
     const int64_t m = mw + j * 16;
     GemmCore16<Cfg>::stay_column(acc, j);  // (one block column at a time, as in fwd16_fold)
-    if ((MODE & 1) && j + AHEAD < Cfg::NBN) fetch(j + AHEAD);
-    if (EDGE && m >= p.M) continue;
+    if (ACC && j + AHEAD < Cfg::NBN) fetch(j + AHEAD);
+    if (m >= p.M) continue;
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i) {
       const int64_t n = nw + i * 16;
-      if (EDGE && n >= p.N) continue;  // (N is a multiple of 4)
+      if (n >= p.N) continue;  // (N is a multiple of 4)
       f32x4_t v = acc[i][j];
-      if (MODE & 1) {
-        v += prev[j % (AHEAD + 1)][i];
-      }
-      if (MODE & 2) {
-        typedef typename VecOf<TIN, 4>::type vec_t;
-        vec_t o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (TIN)v[r];
-        *reinterpret_cast<vec_t*>(p.Ct + m * p.ldct + n) = o;
-      } else {
-        *reinterpret_cast<f32x4_t*>(p.Cf + m * p.ldcf + n) = v;
-      }
+      if (ACC) v += prev[j % (AHEAD + 1)][i];
+      *reinterpret_cast<f32x4_t*>(p.Cf + m * p.ldcf + n) = v;
     }
   }
 }
 
 // A full wave tile in fp32, C (+)= acc (ACC: old values are read), as whole lines: one block column (16 rows x 128 columns) at a
 // time goes through 8 KB of LDS that belong to this wave, 16-byte chunk c of row r at c ^ r, and meets memory two rows x 512
-// bytes per instruction.  In the accumulators' own lane order, 16 rows x 64 bytes, reading and writing a tile took 36000
-// cycles whatever was in flight, a twentieth of the K loop of the d_hidden GEMM.  Two buffers in turn; the old values of the
-// next AHEAD columns are on their way while a column is added and stored.
+// bytes per instruction.  In the accumulators' own lane order, 16 rows x 64 bytes, reading and writing a tile took 38300
+// cycles, a sixteenth of the d_hidden GEMM's K loop, with one block column of old values on its way or with three; this way it
+// takes 20600.  Two buffers in turn; the old values of the next AHEAD columns are on their way while a column is added and stored.
 template <typename Cfg, bool ACC>
 LCE_DEV void gemm16_f32_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw, uint32_t stage) {
   // mw, nw: the wave tile's first row and column of C
@@ -463,6 +454,7 @@ LCE_DEV void gemm16_f32_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&ac
   });
 }
 
+// C in fp32 (out_mode 0 or 1: the callers have no other).
 // CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2, NBN>: then B is K-major as it lies in memory, B[k][n] with row
 // stride ldb, its rows in the order KPerm<Cfg>::vocab_at of A's columns (the d_hidden GEMM reading W in place: no W^T);
 // rows of B at or beyond p.b_rows_valid do not exist (A is zero in those columns).
@@ -509,26 +501,17 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
 #pragma unroll
       for (int j = 0; j < Cfg::NBN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  const int64_t mw = m0 + g.wave_n * Cfg::WN + (g.lane & 15), nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
-  const bool edge = m0 + Cfg::BN > p.M || n0 + Cfg::BM > p.N;
-  if (!edge && p.out_mode < 2) {
-    __syncthreads();  // (the ring is the store tiles' now)
-    const uint32_t stage = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 16384;
-    const int64_t mt = m0 + g.wave_n * Cfg::WN, nt = n0 + g.wave_m * Cfg::WM;
-    if (p.out_mode == 1) gemm16_f32_lines<Cfg, true>(p, acc, mt, nt, stage);
-    else gemm16_f32_lines<Cfg, false>(p, acc, mt, nt, stage);
+  if (m0 + Cfg::BN > p.M || n0 + Cfg::BM > p.N) {
+    const int64_t mw = m0 + g.wave_n * Cfg::WN + (g.lane & 15), nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
+    if (p.out_mode == 1) gemm16_edge<Cfg, true>(p, acc, mw, nw);
+    else gemm16_edge<Cfg, false>(p, acc, mw, nw);
     return;
   }
-#define LCE_EPI16(MODE)                                             \
-  if (edge) gemm16_epilogue<Cfg, MODE, true>(p, acc, mw, nw);       \
-  else gemm16_epilogue<Cfg, MODE, false>(p, acc, mw, nw)
-  switch (p.out_mode) {
-    case 0: LCE_EPI16(0); break;
-    case 1: LCE_EPI16(1); break;
-    case 2: LCE_EPI16(2); break;
-    default: LCE_EPI16(3); break;
-  }
-#undef LCE_EPI16
+  __syncthreads();  // (the ring is the store tiles' now)
+  const uint32_t stage = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 16384;
+  const int64_t mt = m0 + g.wave_n * Cfg::WN, nt = n0 + g.wave_m * Cfg::WM;
+  if (p.out_mode == 1) gemm16_f32_lines<Cfg, true>(p, acc, mt, nt, stage);
+  else gemm16_f32_lines<Cfg, false>(p, acc, mt, nt, stage);
 }
 
 // LDS write of 8 bytes as inline assembly, for the same reason as the reads: through the compiler it would wait for the
@@ -654,7 +637,8 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   typedef GemmCfg16<typename Cfg::TIN, 1> TnCfg;
   typedef GemmCore16<TnCfg> Core;
   if (p.k_dev) {
-    // (at least two slabs, which the stream wants: gather_rows_kernel zeroes that many rows)
+    // (at least two slabs, which the stream wants: token_prep_kernel, and beyond its range gather_rows_kernel, zeroes that many
+    // rows of hidden, the d_logits pass those of dS)
     const int64_t k = *p.k_dev == 0 ? 0 : (*p.k_dev <= 64 ? 128 : ((int64_t)*p.k_dev + 63) / 64 * 64);
     p.K = k < p.K ? k : p.K;
   }
