@@ -765,18 +765,22 @@ def main():
     # Algorithmic FLOPs of the step: forward 2*T*V*H, backward 4*Ta*V*H over the Ta tokens that carry an upstream gradient
     # (the mandated recompute of the logits is executed but not counted).  With Ta = T this is the reference's 6*T*V*H.
     algorithmic = (2.0 * T + 2.0 * n_grads * t_active) * V * H / (elapsed / args.steps)
-    if 6.0 * T * V * H / (4.0 * V * H * 2.0) < PEAK_BF16 / PEAK_HBM and "lce_bwd_chunk_kernel" in kernels:
+    streams = [n for n in ("lce_bwd_chunk_kernel", "gemm_nt_kernel(d_hidden)", "gemm_nt_kernel(d_weight)") if n in kernels]
+    if 6.0 * T * V * H / (4.0 * V * H * 2.0) < PEAK_BF16 / PEAK_HBM and streams:
         # few tokens: HBM bounds the step.  Its streaming passes over [V, H] in the input dtype: W read by the forward and
         # by the d_hidden product, d_weight written; with few tokens the forward keeps the fp32 logits (T*V*4 bytes
         # written, then read by the backward) and no pass recomputes them; beyond that the d_logits tiles read W once more.
-        k = kernels["lce_bwd_chunk_kernel"]
+        # (one combined launch, or the two gradient products as launches of their own: then the longer one)
+        name = streams[0] if streams[0] == "lce_bwd_chunk_kernel" else max(streams, key=lambda n: kernels[n]["ms_per_step"])
+        k = kernels[name]
         kept = cache_bytes > 0
         passes_bwd = n_grads if kept else 1.0 + n_grads
-        nbytes = passes_bwd * V * H * 2.0 / k["launches_per_step"]  # (W read for d_hidden, d_weight written; --frozen-head: W read)
+        # (W read for d_hidden, d_weight written; --frozen-head: W read)
+        nbytes = (passes_bwd if name == "lce_bwd_chunk_kernel" else 1.0) * V * H * 2.0 / k["launches_per_step"]
         step_bytes = (1.0 + passes_bwd) * V * H * 2.0 + (2.0 * T * V * 4.0 if kept else 0.0)
-        roofline = {"bound": "hbm", "kernel": "lce_bwd_chunk_kernel", "achieved": nbytes / (k["avg_ms"] * 1e-3) / 1e9,
+        roofline = {"bound": "hbm", "kernel": name, "achieved": nbytes / (k["avg_ms"] * 1e-3) / 1e9,
                     "peak": PEAK_HBM / 1e9, "unit": "GB/s", "frac": nbytes / (k["avg_ms"] * 1e-3) / PEAK_HBM,
-                    "traffic": measured_traffic(workload_name, "lce_bwd_chunk_kernel", state),
+                    "traffic": measured_traffic(workload_name, name, state),
                     "avg_launch_ms": k["avg_ms"], "bytes_per_launch": nbytes, "logits_kept": kept,
                     "step_bytes": step_bytes, "step_GBps": step_bytes / (elapsed / args.steps) / 1e9}
     out = {
