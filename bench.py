@@ -431,11 +431,11 @@ SWEEP_WORKLOAD = "token-sweep"
 
 def run_token_sweep(args):
     """Forward and forward + backward of the Qwen2.5-7B head (H=3584, V=152064, bf16) at token counts from 128 to 2048 in
-    steps of 64 plus ragged counts: the band where the launchers switch code paths (at 64, 128, 512 and 1280 tokens; beyond half the hidden size the backward recomputes its logits) and
+    steps of 64 plus ragged counts: the band where the launchers switch code paths (at 64, 128, 512 and 2048 tokens; beyond half the hidden size the backward recomputes its logits) and
     where the bound changes from HBM (one stream of W per pass: 4 passes of [V, H] forward + backward) to the matrix
     pipes (ridge at 2.5e15 / 8e12 = 312 tokens forward, 417 forward + backward).  Each point: median of `--steps`
     runs; `frac` is the larger of the two floors (algorithmic bytes / 8 TB/s, algorithmic FLOP / 2.5 PFLOP/s) over the
-    measured time.  Token tiles are 256 wide, so the matrix-pipe work is that of T rounded up to 256."""
+    measured time.  Token tiles are 192 or 256 wide, so the matrix-pipe work is that of T rounded up to one of them."""
     import torch
 
     from verl_amd import linear_cross_entropy
