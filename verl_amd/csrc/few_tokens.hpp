@@ -1,4 +1,4 @@
-// Few tokens (at most 128; 16-bit inputs, gfx950): the forward up to 64, the gradient GEMMs, and d_logits from kept logits.
+// Few tokens (16-bit inputs, gfx950): the forward up to 64, d_hidden up to 128, d_weight up to 256, and d_logits from kept logits.
 //
 // With T <= 128 every product is one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
 //   logits      W[v] . hidden[t]                        reads W once; nothing is written (or the kept logits)
@@ -234,63 +234,91 @@ struct FewArgs {
 };
 
 // ------------------------------------------------------------------------------------------------------------------
-// d_weight, few tokens.  Workgroup = 256 threads = 4 waves; it owns HW = 256 columns of H, whose hidden values it keeps in
-// registers as MFMA operands for good, and walks the 64-column blocks of dS bid / n_ht, bid / n_ht + n_su, ...; a wave
-// multiplies its 64 columns of H with all 64 columns of the block:  C[m = h][n = u] = sum_t Ht[t][h] * dS[t][u].
-// What bounds it is the write of [V, H].  The neighbours bid, bid + 1, ... write the pieces of the same rows at about the same
-// time and the chip works its way through d_weight as one window of n_su x 64 rows; each block costs an 8 or 16 KB read of dS
-// (from L2) and no read of hidden.  Measured (with d_hidden, the two together; one launch of workgroups that owned 64 rows and
-// walked H, beside the d_hidden workgroups, before): H=3584, V=152064: 1 token 437 -> 374 us, 64 tokens 462 -> 411;
-// H=896, V=151936, 64 tokens: 159 -> 126; 1.09 GB at 5.3 TB/s here, at 6.5 in d_hidden (1 token).
+// d_weight, up to 256 tokens.  Workgroup = 512 threads = 8 waves, one per CU; it owns 512 columns of H, whose hidden values its
+// waves keep in registers as MFMA operands for good (64 columns of up to KT tokens each: KT / 2 registers), and walks the 64-column
+// blocks of dS id / n_ht, id / n_ht + n_su, ...; a wave multiplies its columns of H with all 64 columns of the block:
+//   C[m = h][n = u] = sum_t Ht[t][h] * dS[t][u].
+// What bounds it is the write of [V, H], up to some 130 tokens at the rate of a plain fill, beyond that with the matrix pipes next
+// to it (two waves per SIMD: one multiplies while the other converts and stores).  The workgroups side by side write the pieces
+// of the same rows at about the same time and the chip works its way through d_weight as one window of n_su x 64 rows.  The stores
+// are marked non-temporal: d_weight is larger than every cache, and unmarked its lines push out the dS that all of
+// the columns' workgroups are about to read (the same kernel with plain stores: 130 tokens 293 us, with these 178; 256: 305, 260).
 // MFMA rows are assigned to h in pairs of blocks: block 2i'+b, row 4g+r  <->  h = 32i' + 8g + 4b + r, so a lane ends
 // up with 8 consecutive h for one u.  With 16-bit output a wave's results pass through a tile of its own in LDS and
 // leave it as whole 128-byte lines, eight lanes per row; fp32 output is stored from the registers, 16 rows x 128 bytes
 // per instruction.
+// Measured, forward + backward in us, H=3584, V=152064, against workgroups of 256 columns and a map that left dS to all XCDs (up to
+// 128 tokens) and lce_dw16_kernel's tiles of 256 x 256 (beyond), both with plain stores: 64 tokens 650 -> 631, 128: 786 -> 717,
+// 130: 903 -> 796, 192: 933 -> 838, 256: 1050 -> 945; H=896, 192 tokens: 353 -> 315.  At 333 tokens a wave would have to share its
+// registers among fewer columns, the LDS reads of dS bind (32 columns: 1287) and the tiles are faster (1240).
 // ------------------------------------------------------------------------------------------------------------------
+constexpr int64_t kDwFewMaxTokens = 256;
+
+// swizzle of the 16-byte chunks of a dS tile's rows of 128 bytes: half a wave's transposing read takes 32 bytes of the rows r .. r+3
+// and r+8 .. r+11, which lie in different banks this way (two rows fill the banks once)
+LCE_DEV int ds_swz(int r) { return (r & 2) ^ ((r & 8) >> 1); }
+
+template <int KT, typename TOUT>
+struct DwFewShape {
+  static_assert(KT % 64 == 0 && KT <= kDwFewMaxTokens, "token positions");
+  static constexpr int HW = 512;                                 // columns of H per workgroup
+  static constexpr int TILE = KT * 128;                          // a block of dS
+  static constexpr int STG = sizeof(TOUT) == 2 ? 8192 : 0;       // a wave's store tile
+  static constexpr int WALK = 2 * TILE + 8 * STG, HID = 64 * HW * 2;  // (64 rows of hidden at a time, before the walk)
+  static constexpr int LDS_BYTES = WALK > HID ? WALK : HID;
+};
+
 template <typename TIN, typename TOUT, typename Perm, int KT>
-__global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
-  static_assert(KT == 64 || KT == 128, "token positions");
+__global__ __launch_bounds__(512, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
+  typedef DwFewShape<KT, TOUT> S;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  constexpr int KS = KT / 32, HW = 256, RB = HW * 2, CPR = HW / 8;  // bytes and 16-byte chunks of a row of the hidden tile
-  constexpr int MI = 4, NJ = 4;
+  constexpr int KS = KT / 32, HW = S::HW, RB = HW * 2, CPR = HW / 8;  // bytes and 16-byte chunks of a row of the hidden tile
+  constexpr int MI = 4, NJ = 4, BL = KT * 8 / 512;
+  constexpr int AHEAD = KT < 256 ? 1 : 0;  // k-steps of dS fragments read ahead (at 256 tokens there are no registers for one)
   constexpr bool STAGE = sizeof(TOUT) == 2;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int STORES = STAGE ? 2 * NJ : MI * NJ;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, l16 = lane & 15, e = l16 >> 2, q = l16 & 3;
   const int n_ht = (int)((p.H + HW - 1) / HW);
-  const int ht = blockIdx.x % n_ht;
-  const int64_t h0 = (int64_t)ht * HW;
+  // each XCD takes a contiguous eighth of the numbering (columns of H fastest): the workgroups that walk the same blocks of dS
+  // sit on one or two XCDs, and dS passes into each L2 about once
+  const int id = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+  if (id >= n_ht * p.n_su) return;
+  const int ht = id % n_ht;
+  const int64_t h0 = (int64_t)ht * HW, hw = h0 + 64 * wave;  // the workgroup's first column, this wave's
+  const bool live = hw < p.H;                                // (H is a multiple of 64)
   const int64_t n_ub = p.ucols / 64;
-  char* sA = lds;               // hidden, 64 token rows x RB bytes at a time; then the four waves' store tiles of 8 KB
-  char* sB = lds + 64 * RB;     // two dS tiles: KT rows x 128 bytes (64 columns), chunk c of row r at c ^ (r & 7)
-  constexpr int BL = KT * 8 / 256;
+  char* sB = lds;                           // two dS tiles: KT rows x 128 bytes, chunk c of row r at c ^ ds_swz(r)
+  char* sC = lds + 2 * S::TILE + wave * S::STG;
   int n_tok = p.kt;  // token positions that take part (a device-side count may cut the host's)
   if (p.n_rows) n_tok = *p.n_rows < n_tok ? *p.n_rows : n_tok;
   u32x4_t pre[BL];
   auto fetch = [&](int64_t ub) {
-    const buf_t panel = make_buf(ds_at(p.dS, p.ldS, p.pcol, 0, ub * 64), n_tok * 128);  // rows of 128 bytes
+    const buf_t panel = make_buf(ds_at(p.dS, p.ldS, p.pcol, 0, ub * 64), n_tok * 128);  // rows of 128 bytes; zeros beyond
 #pragma unroll
-    for (int i = 0; i < BL; ++i) pre[i] = __builtin_amdgcn_raw_buffer_load_b128(panel, tid * 16 + i * 4096, 0, 0);
+    for (int i = 0; i < BL; ++i) pre[i] = __builtin_amdgcn_raw_buffer_load_b128(panel, tid * 16 + i * 8192, 0, 0);
   };
   auto stash = [&](char* to) {
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
-      const int id = tid + i * 256, r = id >> 3, c = id & 7;
-      *reinterpret_cast<u32x4_t*>(to + r * 128 + ((c ^ (r & 7)) * 16)) = pre[i];
+      const int at = tid + i * 512, r = at >> 3, c = at & 7;
+      *reinterpret_cast<u32x4_t*>(to + r * 128 + ((c ^ ds_swz(r)) * 16)) = pre[i];
     }
   };
-  int64_t ub = blockIdx.x / n_ht;  // (< n_ub: the grid has at most that many)
+  int64_t ub = id / n_ht;  // (< n_ub: at most that many side by side)
   const int64_t ub_last = ub + (n_ub - 1 - ub) / p.n_su * p.n_su;
   fetch(ub);
-  // hidden tile -> LDS -> fragments
+  // hidden -> LDS -> fragments, 64 tokens at a time (zeros behind the last token)
   u32x4_t af[KS][MI];
+  const buf_t hid = make_buf(p.Ht, (int64_t)n_tok * p.ldHt * sizeof(TIN));
 #pragma unroll
-  for (int half = 0; half < KT / 64; ++half) {
-    if (half) __syncthreads();
+  for (int part = 0; part < KT / 64; ++part) {
+    if (part) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 64 * CPR / 256; ++i) {
-      const int id = tid + i * 256, r = id / CPR, c = id % CPR;
-      *reinterpret_cast<u32x4_t*>(sA + r * RB + ((c ^ fw_swz(r)) * 16)) =
-          *reinterpret_cast<const u32x4_t*>(p.Ht + (int64_t)(64 * half + r) * p.ldHt + h0 + c * 8);
+    for (int i = 0; i < 64 * CPR / 512; ++i) {
+      const int at = tid + i * 512, r = at / CPR, c = at % CPR;
+      const int from = h0 + c * 8 < p.H ? (int)(((64 * part + r) * p.ldHt + h0 + c * 8) * sizeof(TIN)) : kBufNowhere;
+      *reinterpret_cast<u32x4_t*>(lds + r * RB + ((c ^ fw_swz(r)) * 16)) = __builtin_amdgcn_raw_buffer_load_b128(hid, from, 0, 0);
     }
     __syncthreads();
 #pragma unroll
@@ -300,11 +328,12 @@ __global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
         // block i = 2i' + b: the run of lane q starts at column 64 wave + 32 i' + 8 q + 4 b
         const int col = 64 * wave + 32 * (i >> 1) + 8 * q + 4 * (i & 1);
         const int r0 = 32 * k2 + 8 * g + e, r1 = r0 + 4;
-        const u32x2_t lo = tr_read_b64(sA + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
-        const u32x2_t hi = tr_read_b64(sA + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
-        af[2 * half + k2][i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        const u32x2_t lo = tr_read_b64(lds + r0 * RB + (((col >> 3) ^ fw_swz(r0)) * 16) + (col & 7) * 2);
+        const u32x2_t hi = tr_read_b64(lds + r1 * RB + (((col >> 3) ^ fw_swz(r1)) * 16) + (col & 7) * 2);
+        af[2 * part + k2][i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
       }
   }
+  __syncthreads();
   const int ks_n = (n_tok + 31) / 32;
   // where this lane stores, relative to the block's first row (an aligned run of 64 columns of dS is a permutation of the
   // same 64 rows of the vocabulary): through LDS 16 bytes of eight rows, else runs of 8 columns of four rows
@@ -312,44 +341,50 @@ __global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 #pragma unroll
   for (int k = 0; k < (STAGE ? 2 * NJ : NJ); ++k) {
     const int row = STAGE ? 8 * k + (lane >> 3) : 16 * k + l16;
-    const int64_t h = h0 + 64 * wave + (STAGE ? ((lane & 7) ^ ((row >> 1) & 7)) * 8 : 8 * g);
-    at[k] = h < p.H ? (int)((Perm::vocab_at(row) * p.H + h) * sizeof(TOUT)) : kBufNowhere;  // (H is a multiple of 8)
+    const int64_t h = hw + (STAGE ? ((lane & 7) ^ ((row >> 1) & 7)) * 8 : 8 * g);
+    at[k] = live ? (int)((Perm::vocab_at(row) * p.H + h) * sizeof(TOUT)) : kBufNowhere;
   }
-  const int at1_add = h0 + 64 * wave + 32 + 8 * g < p.H ? 32 * (int)sizeof(TOUT) : kBufNowhere;  // the second run (no STAGE)
   stash(sB);
   fetch(ub < ub_last ? ub + p.n_su : ub);
-  // (as many dropped stores as a turn of the loop issues behind its fetch: the compiler waits for the fetch at the top of a turn,
-  // and only with that many younger operations on either way into the loop not for the previous block's stores as well)
+  // (as many dropped stores as a turn of the loop issues behind its fetch: the compiler waits for the fetch in the next turn, and
+  // only with that many younger operations on either way into the loop not for the previous block's stores as well)
 #pragma unroll
-  for (int k = 0; k < (STAGE ? 2 * NJ : 2 * MI / 2 * NJ); ++k)
+  for (int k = 0; k < STORES; ++k)
     __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{0u, 0u, 0u, 0u}, make_buf(p.dW, 0), kBufNowhere + 16 * k, 0, 0);
   for (int buf = 0; ub <= ub_last; ub += p.n_su, buf ^= 1) {
     // one barrier per block: this block's tile is in LDS, and every wave is done with the other buffer
     __syncthreads();
-    const char* tB = sB + buf * (KT * 128);
+    const char* tB = sB + buf * S::TILE;
     f32x4_t acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks >= ks_n) break;
-      u32x4_t bf[NJ];
+    u32x4_t bf[1 + AHEAD][NJ];
+    auto frags = [&](int ks, u32x4_t (&b)[NJ]) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         // lanes (e, q) of group g address row 32 ks + 8 g + e (+4), columns 16 j + 4 q ..
         const int r0 = 32 * ks + 8 * g + e, r1 = r0 + 4, col = 16 * j + 4 * q;
-        const u32x2_t lo = tr_read_b64(tB + r0 * 128 + (((col >> 3) ^ (r0 & 7)) * 16) + (col & 7) * 2);
-        const u32x2_t hi = tr_read_b64(tB + r1 * 128 + (((col >> 3) ^ (r1 & 7)) * 16) + (col & 7) * 2);
-        bf[j] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        const u32x2_t lo = tr_read_b64(tB + r0 * 128 + (((col >> 3) ^ ds_swz(r0)) * 16) + (col & 7) * 2);
+        const u32x2_t hi = tr_read_b64(tB + r1 * 128 + (((col >> 3) ^ ds_swz(r1)) * 16) + (col & 7) * 2);
+        b[j] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
       }
+    };
+    if (live) {  // (the last workgroup of a row may have waves without columns)
+      if (AHEAD) frags(0, bf[0]);
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+      for (int ks = 0; ks < KS; ++ks) {
+        if (!AHEAD) frags(ks, bf[0]);
+        else if (ks + 1 < KS) frags(ks + 1, bf[(ks + 1) & AHEAD]);  // (zeros behind the last token)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[ks][i], bf[j]);
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) mma16<TIN>(acc[i][j], af[ks][i], bf[ks & AHEAD][j]);
+        if (ks + 1 >= ks_n) break;
+      }
     }
-    stash(sB + (buf ^ 1) * (KT * 128));  // (behind the last block: the last one again)
+    stash(sB + (buf ^ 1) * S::TILE);  // (behind the last block: the last one again)
     fetch(ub + 2 * p.n_su <= ub_last ? ub + 2 * p.n_su : ub_last);
     const int64_t u0 = ub * 64, left = p.vrows - u0 < 64 ? p.vrows - u0 : 64;
     const buf_t out = make_buf(static_cast<TOUT*>(p.dW) + u0 * p.H, (left > 0 ? left : 0) * p.H * sizeof(TOUT));
@@ -357,7 +392,6 @@ __global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
       // Whole 128-byte lines per store: the wave's 64 rows x 64 columns go through a tile of its own in LDS (16-byte
       // chunk c of row r at c ^ ((r / 2) % 8), so that the 16 rows x 4 chunks of one write fall into different banks)
       // and leave it eight rows at a time, eight lanes per row.  No barrier: LDS operations of one wave complete in order.
-      char* sC = sA + wave * 8192;
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -369,22 +403,17 @@ __global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
           store_run<TOUT, 8>(reinterpret_cast<TOUT*>(sC + row * 128 + ((c ^ ((row >> 1) & 7)) * 16)), d);
         }
 #pragma unroll
-      for (int it = 0; it < NJ * 2; ++it) {
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sC + (it * 8 + (lane >> 3)) * 128 + (lane & 7) * 16);
-        __builtin_amdgcn_raw_buffer_store_b128(v, out, at[it], 0, 0);
+      for (int k = 0; k < 2 * NJ; ++k) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sC + (k * 8 + (lane >> 3)) * 128 + (lane & 7) * 16);
+        __builtin_amdgcn_raw_buffer_store_b128(v, out, at[k], 0, kBufNonTemporal);
       }
     } else {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int ip = 0; ip < MI / 2; ++ip)
-#pragma unroll
-          for (int hf = 0; hf < 2; ++hf) {
-            u32x4_t v;
-            __builtin_memcpy(&v, &acc[2 * ip + hf][j], 16);
-            const int o = at[j] == kBufNowhere ? at[j] : ip ? (at1_add == kBufNowhere ? at1_add : at[j] + at1_add) : at[j];
-            __builtin_amdgcn_raw_buffer_store_b128(v, out, o == kBufNowhere ? o : o + 16 * hf, 0, 0);
-          }
+        for (int i = 0; i < MI; ++i)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), out, at[j] == kBufNowhere ? at[j] : at[j] + (32 * (i >> 1) + 4 * (i & 1)) * 4,
+                                                 0, kBufNonTemporal);
     }
   }
 }
@@ -401,7 +430,6 @@ __global__ __launch_bounds__(256, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 template <int KT>
 struct FewShape {  // KT: token positions, 64 up to 64 tokens, else 128
   static constexpr int HW = 256;                                     // columns of H per workgroup
-  static constexpr int DW_LDS = 64 * HW * 2 + 2 * KT * 128;          // hidden (then store tiles), two dS tiles
   static constexpr int DH_DEPTH = KT <= 64 ? 4 : 3;
   static constexpr int DH_STAGE = 64 * HW * 2 + KT * 128;            // W rows, dS tile
   static constexpr int DH_LDS = 2 * DH_STAGE;

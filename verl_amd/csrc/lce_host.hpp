@@ -636,6 +636,19 @@ int launch_ds_few_tokens(DsArgs<typename Cfg::TIN> d, int64_t T, int nvt, hipStr
   return check_launch("lce_bwd_ds_kernel");
 }
 
+// d_weight of one vocabulary chunk by the streaming kernel, KT >= the tokens; as many workgroups as CUs
+template <typename Cfg, typename TOUT, int KT>
+int launch_dw_few(FewArgs<typename Cfg::TIN> q, hipStream_t st) {
+  typedef DwFewShape<KT, TOUT> S;
+  ProfScope prof(PC_GEMM_DW, st);
+  const int64_t n_ht = (q.H + S::HW - 1) / S::HW;
+  q.n_su = (int)std::max<int64_t>(1, std::min<int64_t>(kNumCUs / n_ht, q.ucols / 64));
+  auto kern = lce_dw_few_kernel<typename Cfg::TIN, TOUT, KPerm<Cfg>, KT>;
+  allow_lds(kern, S::LDS_BYTES);
+  hipLaunchKernelGGL(kern, dim3((unsigned)round_up(n_ht * q.n_su, 8)), dim3(512), S::LDS_BYTES, st, q);
+  return check_launch("lce_dw_few_kernel");
+}
+
 // Both gradient GEMMs of one vocabulary chunk of a backward with at most 128 tokens as two launches of the streaming
 // kernels (few_tokens.hpp): d_hidden as L.ksplit fp32 partials, d_weight rows of the chunk in the output dtype.
 template <typename Cfg, typename TOUT, int KT>
@@ -651,19 +664,7 @@ int launch_few_gemms(FewArgs<typename Cfg::TIN> q, bool with_dh, hipStream_t st)
     hipLaunchKernelGGL(kern, dim3((unsigned)(n_ht * q.ksplit)), dim3(512), S::DH_LDS, st, q);
     if ((rc = check_launch("lce_dh_few_kernel"))) return rc;
   }
-  if (q.dW) {
-    ProfScope prof(PC_GEMM_DW, st);
-    const int n_ht = (int)((q.H + S::HW - 1) / S::HW);
-    // as many workgroups as are resident at once: three per CU up to 64 tokens, two beyond (LDS, registers)
-    q.n_su = ((KT <= 64 ? 3 : 2) * kNumCUs) / n_ht;
-    if (q.n_su < 1) q.n_su = 1;
-    if (q.n_su > q.ucols / 64) q.n_su = (int)(q.ucols / 64);
-    auto kern = lce_dw_few_kernel<TIN, TOUT, KPerm<Cfg>, KT>;
-    allow_lds(kern, S::DW_LDS);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(n_ht * q.n_su)), dim3(256), S::DW_LDS, st, q);
-    if ((rc = check_launch("lce_dw_few_kernel"))) return rc;
-  }
-  return LCE_OK;
+  return q.dW ? launch_dw_few<Cfg, TOUT, KT>(q, st) : LCE_OK;
 }
 
 template <typename Cfg>
@@ -912,7 +913,16 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
             if ((rc = L.mid_192 ? launch_dh(std::true_type{}) : launch_dh(std::false_type{}))) return rc;
             p.n_gh = 0;
           }
-          if (L.mid && !tu.split_bwd && need_dw && dw_t && aligned16(dw_t)) {
+          if (L.mid && !tu.split_bwd && need_dw && T <= (grads_f32 ? 192 : kDwFewMaxTokens)) {
+            FewArgs<TIN> q = {};
+            q.dS = dS[cc & 1]; q.ldS = L.ldS; q.pcol = L.pcol; q.Ht = Ht; q.ldHt = L.ldHt;
+            q.vrows = vrows; q.ucols = kc; q.H = H; q.kt = (int)T; q.n_rows = n_rows;
+            q.dW = grads_f32 ? static_cast<void*>(dw_f32) : static_cast<void*>(dw_t);
+            if (T <= 192) rc = grads_f32 ? launch_dw_few<Cfg, float, 192>(q, st) : launch_dw_few<Cfg, TIN, 192>(q, st);
+            else rc = launch_dw_few<Cfg, TIN, 256>(q, st);
+            if (rc) return rc;
+            p.n_gw = 0;
+          } else if (L.mid && !tu.split_bwd && need_dw && dw_t && aligned16(dw_t)) {
             const int64_t tiles = ((p.gw.M + 255) / 256) * ((p.gw.N + 255) / 256);
             ProfScope prof(PC_GEMM_DW, st);
             allow_lds(lce_dw16_kernel<Cfg>, Cfg::LDS_BYTES);
