@@ -155,7 +155,8 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
     if (p.xcache) {
       // the logits of this pass, for a backward that then has no need to recompute them.  A 32x32 block passes through 4 KB of
       // LDS of this wave's own and leaves it as whole lines, 1 KB (16 tokens x 16 rows of a panel) per store; rows in whole
-      // fours, the last ones of W up to the end of the cache's panel.
+      // fours, the last ones of W up to the end of the cache's panel.  Non-temporal (64 tokens, H=3584: step 632 -> 615 us,
+      // 40: 611 -> 597; the stores leave while W streams in, and unmarked they wait for lines of the caches).
       char* sC = lds + 2 * S::STAGE + wave * 4096;
       const int p4 = lane & 3, pt = lane >> 2;  // as it leaves: quad of rows, token
 #pragma unroll
@@ -172,7 +173,7 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
           const f32x4_t x4 = *reinterpret_cast<const f32x4_t*>(sC + (q >> 1) * 2048 + tl * 64 + ((p4 ^ ((tl >> 1) & 3)) * 16));
           const int v = vbase + 16 * (q >> 1) + 4 * p4;
           const int64_t t = j * 32 + tl;
-          if (t < p.T && v < vend) *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = x4;
+          if (t < p.T && v < vend) __builtin_nontemporal_store(x4, reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)));
         }
       }
     }

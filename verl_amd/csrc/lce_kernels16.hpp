@@ -160,7 +160,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
         // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
         // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are
         // issued 16 at a time and so many are waited for that, with the prologue's 32 loads behind them, fewer than 64
-        // operations are ever in flight.
+        // operations are ever in flight.  Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
         const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
         // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
         const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
@@ -172,7 +172,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
 #pragma unroll
           for (int i = 0; i < NB; ++i) {
             const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, kBufNonTemporal);
           }
           if (j % 2 == 1 && j >= 3) {
             __builtin_amdgcn_sched_barrier(0);
