@@ -61,14 +61,15 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 // the same fp32 accumulators.  What is left out, a2 b3 + a3 b2 + a3 b3, is below 2^-26 of |a b|, a quarter of what rounding
 // ONE fp32 product or partial sum costs, and the products themselves are exact.  Six bfloat16 MFMAs take six sixteenths
 // of the matrix pipe's time of the fp32 one.
-template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0, int TERMS_ = 1>
+// A_ONCE_: the loads of A are marked non-temporal (A is read once, or nearly, and larger than the caches).
+template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0, int TERMS_ = 1, int A_ONCE_ = 0>
 struct GemmCfg16 {
   typedef TIN_ TIN;
   static_assert(sizeof(TIN_) == 2, "16-bit operands");
   static constexpr bool CORE16 = true;
   static_assert(NBN_ == 8 || TRANS_ != 1, "both operands K-major: square tiles");
   static constexpr int BM = 256, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
-  static constexpr bool A_EARLY = A_EARLY_ != 0;
+  static constexpr bool A_EARLY = A_EARLY_ != 0, A_ONCE = A_ONCE_ != 0;
   static constexpr int TERMS = TERMS_;
   static_assert(TERMS_ == 1 || TERMS_ == 6, "products per slab");
   static constexpr int WAVES_M = 2, WAVES_N = 2, NW = 4, NTHREADS = 256;
@@ -244,7 +245,8 @@ struct GemmCore16 {
     } else {
       src = (is_b ? b_base + ks * b_slab + plane + vb[j] : a_base + ks * a_slab + plane + va[j]);
     }
-    __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
+    if (Cfg::A_ONCE && !is_b) __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, kBufNonTemporal);  // (constants after inlining)
+    else __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
   }
 
   // Fragments are read in the order a0, b0 .. b(NBN-1), a1 .. a7 (F = 0 .. NF-1): the MFMAs walk the A blocks in the outer
@@ -426,7 +428,7 @@ struct GemmCore16 {
   template <int STORES>
   LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
     static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
-    static_assert(NBN == NB && !AE && Cfg::TERMS == 1, "square tiles, B early");
+    static_assert(NBN == NB && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "square tiles, B early");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     int sb = s.sb;
     auto slab = [&](auto first, int it) {

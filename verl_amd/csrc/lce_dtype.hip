@@ -37,7 +37,9 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case 1: LCE_RUN(Variant1);
     case 2: LCE_RUN(Variant2);
     case 3: LCE_RUN(Variant3);
-    case kSelN192: LCE_RUN(VariantN192);
+    case kSelN192:
+      if (forward_w_once(T, V, ldw * (int64_t)sizeof(TuT))) LCE_RUN(VariantN192Once);
+      LCE_RUN(VariantN192Plain);
     case kSelT128:
       if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT128Plain);
       LCE_RUN(VariantT128);

@@ -148,11 +148,18 @@ template <typename TIN> struct Variant2 { typedef GemmCfg<TIN, 256, 256, 128, 2,
 template <typename TIN> struct Variant3 { typedef GemmCfg16<TIN> Cfg; };
 template <> struct Variant3<float> { typedef GemmCfg<float, 256, 256, 128, 5, 4, 2, 2> Cfg; };
 // the same loop on tiles 192 tokens wide, the weight early: with so few tokens it streams from HBM, and a slab of the narrow
-// tile leaves it less time to arrive (333 tokens: forward 382 -> 365 us, d_hidden 370 -> 330)
-template <typename TIN> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6, 1> Cfg; };
-template <> struct VariantN192<float> : Variant3<float> {};
-// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us)
-template <typename TIN> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1> Cfg; };
+// tile leaves it less time to arrive (333 tokens: forward 382 -> 365 us, d_hidden 370 -> 330).  ONCE: the loads of W are marked
+// non-temporal.  d_hidden with one tile of tokens: step at 130 tokens 790 -> 709 us (H=3584), 1094 -> 985 (5120), 192: 836 -> 756,
+// 315 -> 305 (896): unmarked, W takes the place of the logits' gradient that d_weight reads next (without a d_weight: level, 735 ->
+// 743 at 192 tokens, H=5120).  With two tiles side by side (257
+// to 384 tokens) one's lines may be gone before the other asks: 1184 -> 1158 but 1650 -> 1705 (5120).  Forward: forward_w_once.
+template <typename TIN, int ONCE = 0> struct VariantN192 { typedef GemmCfg16<TIN, 0, 6, 1, 1, ONCE> Cfg; };
+template <int ONCE> struct VariantN192<float, ONCE> : Variant3<float> {};
+template <typename TIN> using VariantN192Plain = VariantN192<TIN, 0>;
+template <typename TIN> using VariantN192Once = VariantN192<TIN, 1>;
+// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us) and read once (step at 256 tokens 953 ->
+// 904 us, 512: 1604 -> 1570; level from 600 tokens on)
+template <typename TIN> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1, 1, 1> Cfg; };
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring.  ONCE: the loads of W
 // are marked non-temporal (read_w_once)
 template <typename TIN, int ONCE = 1> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, ONCE> Cfg; };
@@ -181,6 +188,10 @@ void allow_lds(K kernel, int bytes) {
 // At 342 MB the two are level, at 445 MB non-temporal loads win (40 tokens: 83.4 against 92.5 plain).
 constexpr int64_t kMallBytes = (int64_t)256 << 20;  // the memory-side cache
 bool read_w_once(int64_t V, int64_t row_bytes, const float* xcache) { return xcache || V * row_bytes > kMallBytes * 5 / 4; }
+
+// The same question for the 16x16x32 loop with one tile of 192 tokens.  130 / 192 tokens, forward alone, plain / non-temporal, us:
+// H=3584 (1.09 GB) 228 / 218, 238 / 224; H=896 (272 MB) 68.8 / 71.3, 74.2 / 75.1, and with a backward behind it 214 / 222.
+bool forward_w_once(int64_t T, int64_t V, int64_t row_bytes) { return T <= 192 && V * row_bytes > kMallBytes * 5 / 4; }
 
 int block_rows(int nrow_tiles) { return TileMap::block_rows(nrow_tiles); }
 
@@ -900,8 +911,8 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
         if constexpr (Cfg::CORE16) {
           // (one chunk: no d_logits tiles share this launch)
           if (L.mid && !tu.split_bwd && need_dh) {
-            auto launch_dh = [&](auto narrow) {
-              typedef typename std::conditional<decltype(narrow)::value, typename VariantN192<TIN>::Cfg, typename VariantWEarly<TIN>::Cfg>::type DhCfg;
+            auto launch_dh = [&](auto variant) {
+              typedef typename decltype(variant)::Cfg DhCfg;
               GemmArgs<TIN> q = p.gh;
               const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
               q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
@@ -910,7 +921,8 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
               hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3(q.map.total), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q);
               return check_launch("lce_dh16_kernel");
             };
-            if ((rc = L.mid_192 ? launch_dh(std::true_type{}) : launch_dh(std::false_type{}))) return rc;
+            rc = !L.mid_192 ? launch_dh(VariantWEarly<TIN>{}) : T <= 192 && need_dw ? launch_dh(VariantN192Once<TIN>{}) : launch_dh(VariantN192Plain<TIN>{});
+            if (rc) return rc;
             p.n_gh = 0;
           }
           if (L.mid && !tu.split_bwd && need_dw && T <= (grads_f32 ? 192 : kDwFewMaxTokens)) {

@@ -12,8 +12,8 @@ namespace lce {
 // vocabulary rows (one wave tile) the entries are ordered so that what a lane holds of two neighbouring blocks is one
 // 16-byte run and the four lane groups follow each other (64 contiguous bytes per token and store instruction):
 // row v = 16 i + 4 g + r  ->  position 32 (i / 2) + 8 g + 4 (i % 2) + r.  Tokens keep their order.
-template <typename TIN, int TR, int NBN, int AE, int TERMS>
-struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS>> {
+template <typename TIN, int TR, int NBN, int AE, int TERMS, int AO>
+struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS, AO>> {
   static constexpr int GT = 128, GV = 128;
   static __host__ __device__ __forceinline__ int64_t token(int64_t t) { return t; }
   static __host__ __device__ __forceinline__ int64_t token_at(int64_t u) { return u; }
@@ -816,7 +816,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void gemm16_tn_kernel(GemmArgs<typen
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY>>(p, blockIdx.x, lds);
+  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY, 1, Cfg::A_ONCE>>(p, blockIdx.x, lds);
 }
 
 template <typename Cfg>
