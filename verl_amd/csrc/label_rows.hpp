@@ -334,14 +334,21 @@ __global__ __launch_bounds__(256) void token_prep_kernel(CoefArgs<T> a, LabelTer
   }
 }
 
-// Workgroups [0, n_dh): d_hidden, as dh_finish_kernel with that many workgroups.  Workgroup n_dh + i: compact position
+// Workgroups [0, n_dh): d_hidden, as dh_finish_kernel with that many workgroups (with `by_rows` in use, the slices that
+// lce_dh16_kernel has worked out from the same count of rows).  Workgroup n_dh + i: compact position
 // i of the token list; the first position of each label adds sum of G_t * hidden[t][:] over the positions with that
 // label, in order, to the label's row of d_weight (as dw_label_rows_kernel does over a sorted run).
 template <typename T, typename TOUT>
 __global__ __launch_bounds__(256) void token_finish_kernel(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H,
                                                            TOUT* d_hidden, LabelTerm lt, const T* W, int64_t ldw, int n_dh, const int* rows,
-                                                           const int* n_rows, const uint32_t* keys, const T* h, int64_t ldh, TOUT* dW) {
+                                                           const int* n_rows, const uint32_t* keys, const T* h, int64_t ldh, TOUT* dW,
+                                                           DhSlices by_rows) {
   if ((int)blockIdx.x < n_dh) {
+    if (by_rows.n[0]) {
+      const int64_t rows_n = *n_rows;
+      S = by_rows.count(rows_n);
+      stride = DhSlices::stride(rows_n, H);
+    }
     dh_finish_body<T, TOUT>(part, S, stride, inv, ntok, H, d_hidden, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)n_dh);
     return;
   }

@@ -483,18 +483,35 @@ int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
 // read of [T, H] fp32 (at 5 TB/s; a slab of 64 takes 1.2 us).  The fewest slab times win.  (333 tokens, H=3584, V=152064: 28
 // tiles x 9 slices are one round of 264 slabs; 16 slices, what the mixed launch would take, two rounds of 149.)
 // `wide`: token tiles 256 wide, else 192, whose slabs take 0.82 of the time (28 tiles either way: 512 tokens 412 us, 333: 330).
-int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cost_out) {
+int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cost_out, int most = 32) {
   const int64_t tiles = (wide ? (T + 255) / 256 : (T + 191) / 192) * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
   const double per_slice = (double)T * H * 8.0 / 5.0e12 / 1.2e-6;
   int best = 1;
   double best_cost = -1.0;
-  for (int s = 1; s <= 32 && s <= slabs; ++s) {
+  for (int s = 1; s <= most && s <= slabs; ++s) {
     const int64_t rounds = (tiles * s + kNumCUs - 1) / kNumCUs;
     const double cost = (double)rounds * ((slabs + s - 1) / s + 10) * (wide ? 1.0 : 0.82) + per_slice * s;
     if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = s; }
   }
   *cost_out = best_cost;
   return best;
+}
+
+// The same choice for every number of row tiles that may turn out to take part, within the memory that `ksplit` partials of all
+// T rows have.  Forward + backward in us, slices counted for all tokens / this way: H=4096, V=128256, 1000 tokens, about 500 with
+// gradient 1646 / 1341, about 250: 1931 / 1761, 2000 tokens 3263 / 2555, 400: 1083 / 1029; H=5120 1500 tokens 4016 / 3346; level
+// where every token has one and where the row tiles left fill the CUs as they are.
+DhSlices dh_slices_by_rows(int64_t T, int64_t H, int64_t vchunk, bool wide, int ksplit) {
+  DhSlices d = {};
+  d.tile_rows = wide ? 256 : 192;
+  const int all = d.tiles(T);
+  const int64_t room = (int64_t)ksplit * (int64_t)(align256((size_t)T * H * 4) / 4);
+  for (int r = 1; r <= all; ++r) {
+    const int64_t rows = std::min<int64_t>(T, (int64_t)r * d.tile_rows);
+    double cost;
+    d.n[r - 1] = r == all ? (uint8_t)ksplit : (uint8_t)dh_ksplit_alone(rows, H, vchunk, wide, &cost, (int)std::min<int64_t>(32, room / DhSlices::stride(rows, H)));
+  }
+  return d;
 }
 
 // layout for a given chunk width
@@ -807,6 +824,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       hipLaunchKernelGGL(lce_bwd_chunk_kernel<Cfg>, dim3(q.n_gw + q.n_gh + q.n_ds), dim3(Cfg::NTHREADS), chunk_lds, st, q);
     }
   };
+  DhSlices by_rows = {};
   // launch c (0 <= c <= nchunks): d_logits of chunk c (if any) + the two gradient GEMMs of chunk c-1 (if any)
   for (int c = 0; c <= L.nchunks; ++c) {
     BwdChunkArgs<TIN> p;
@@ -916,9 +934,14 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
               GemmArgs<TIN> q = p.gh;
               const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
               q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
+              int grid = q.map.total;
+              if (one_prep && tu.dh_ksplit <= 0) {
+                by_rows = dh_slices_by_rows(T, H, L.vchunk, DhCfg::BN == 256, L.ksplit);
+                for (int r = 1; r <= tm; ++r) grid = std::max(grid, TileMap::make(r, q.n_tiles * by_rows.n[r - 1], 1, 1).total);
+              }
               ProfScope prof(PC_GEMM_DH, st);
               allow_lds(lce_dh16_kernel<DhCfg>, DhCfg::LDS_BYTES);
-              hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3(q.map.total), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q);
+              hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3((unsigned)grid), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q, by_rows);
               return check_launch("lce_dh16_kernel");
             };
             rc = !L.mid_192 ? launch_dh(VariantWEarly<TIN>{}) : T <= 192 && need_dw ? launch_dh(VariantN192Once<TIN>{}) : launch_dh(VariantN192Plain<TIN>{});
@@ -1013,10 +1036,10 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       if (n_dh + n_lr > 0) {
         if (grads_f32)
           hipLaunchKernelGGL((token_finish_kernel<TIN, float>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
-                             T, H, static_cast<float*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<float*>(d_weight));
+                             T, H, static_cast<float*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<float*>(d_weight), by_rows);
         else
           hipLaunchKernelGGL((token_finish_kernel<TIN, TIN>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
-                             T, H, static_cast<TIN*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<TIN*>(d_weight));
+                             T, H, static_cast<TIN*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<TIN*>(d_weight), by_rows);
         if ((rc = check_launch("token_finish_kernel"))) return rc;
       }
     }

@@ -812,10 +812,18 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void gemm16_tn_kernel(GemmArgs<typen
   gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1>, Cfg>(p, blockIdx.x, lds);
 }
 
-// d_hidden on its own: C[m][n] (+)= sum_k A[m][k] B[k][n] as in gemm16_tile's mixed mode (W read in place)
+// d_hidden on its own: C[m][n] (+)= sum_k A[m][k] B[k][n] as in gemm16_tile's mixed mode (W read in place); with `by_rows` in use
+// the K slices are those of the rows that take part
 template <typename Cfg>
-__global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Cfg::TIN> p) {
+__global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Cfg::TIN> p, DhSlices by_rows) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
+  if (by_rows.n[0]) {
+    const int64_t rows = *p.m_dev;
+    p.ksplit = by_rows.count(rows);
+    p.kslice = ((p.K + p.ksplit - 1) / p.ksplit + Cfg::BK - 1) / Cfg::BK * Cfg::BK;
+    p.cf_split_stride = DhSlices::stride(rows, p.N);
+    p.map.ncol_tiles = p.n_tiles * p.ksplit;
+  }
   gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY, 1, Cfg::A_ONCE>>(p, blockIdx.x, lds);
 }
 
