@@ -157,9 +157,10 @@ template <typename TIN, int ONCE = 0> struct VariantN192 { typedef GemmCfg16<TIN
 template <int ONCE> struct VariantN192<float, ONCE> : Variant3<float> {};
 template <typename TIN> using VariantN192Plain = VariantN192<TIN, 0>;
 template <typename TIN> using VariantN192Once = VariantN192<TIN, 1>;
-// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us) and read once (step at 256 tokens 953 ->
-// 904 us, 512: 1604 -> 1570; level from 600 tokens on)
-template <typename TIN> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1, 1, 1> Cfg; };
+// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us).  ONCE, up to two tiles of tokens and with a
+// d_weight to follow: step at 256 tokens 953 -> 904 us, 512: 1604 -> 1570; from 600 tokens on level, and without a d_weight
+// the other way (450 tokens, H=5120: 1520 -> 1540, 1000: 2728 -> 2767)
+template <typename TIN, int ONCE = 0> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1, 1, ONCE> Cfg; };
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring.  ONCE: the loads of W
 // are marked non-temporal (read_w_once)
 template <typename TIN, int ONCE = 1> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, ONCE> Cfg; };
@@ -944,7 +945,9 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
               hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3((unsigned)grid), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q, by_rows);
               return check_launch("lce_dh16_kernel");
             };
-            rc = !L.mid_192 ? launch_dh(VariantWEarly<TIN>{}) : T <= 192 && need_dw ? launch_dh(VariantN192Once<TIN>{}) : launch_dh(VariantN192Plain<TIN>{});
+            const bool once = need_dw && T <= (L.mid_192 ? 192 : 512);
+            if (L.mid_192) rc = once ? launch_dh(VariantN192<TIN, 1>{}) : launch_dh(VariantN192<TIN, 0>{});
+            else rc = once ? launch_dh(VariantWEarly<TIN, 1>{}) : launch_dh(VariantWEarly<TIN, 0>{});
             if (rc) return rc;
             p.n_gh = 0;
           }
