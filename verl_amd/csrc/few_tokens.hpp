@@ -1,4 +1,5 @@
-// Few tokens (16-bit inputs, gfx950): the forward up to 64, d_hidden up to 128, d_weight up to 256, and d_logits from kept logits.
+// Few tokens (gfx950).  16-bit inputs: the forward up to 64, d_hidden up to 128, d_weight up to 256, and d_logits from kept
+// logits; fp32 inputs: the forward up to 128.
 //
 // With T <= 128 every product is one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
 //   logits      W[v] . hidden[t]                        reads W once; nothing is written (or the kept logits)
@@ -62,50 +63,48 @@ LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 // Measured, kernel and merge, against the 256 x 64 tile with a ring of whole LDS stages (H, V: before -> after): 64 tokens,
 // 3584, 152064: 184 -> 174 us; 4096, 128256: 175 -> 160; 896, 151936: 58 -> 51.5; the same access pattern without any
 // arithmetic takes 170, 163 and 41.  (128 tokens on 64 x 64 wave tiles: 223 us, the 256 x 128 tile takes 213.)
+// fp32 inputs run it up to 128 tokens, on the fp32 MFMA, which is the bound from some 40 tokens on (64 tokens, 1.09 G products of W's
+// elements: 445 us at its peak rate): the narrowest of 32, 64, 96 and 128 tokens that holds them.  Against the 256 x 64 and 256 x 128
+// tiles, H=3584: 1 to 32 tokens 750 -> 440 us, 64: 746 -> 673, 65 to 96: 1335 -> 936, 128: 1335 -> 1220; H=896: 202 -> 113, 202 -> 188,
+// 360 -> 285, 354 -> 333.
 // ------------------------------------------------------------------------------------------------------------------
+template <typename TIN, int NT_>
 struct FewFwdShape {
-  static constexpr int NT = 64, DEPTH = 4, BM = 256, FN = 2;
-  static constexpr int STAGE = BM * 128 + NT * 128;
-  static constexpr int LDS_BYTES = 2 * STAGE + 8 * 4096;  // two stages, a store tile per wave
+  static constexpr int NT = NT_, DEPTH = sizeof(TIN) == 2 || NT == 32 ? 4 : 3, BM = 256, FN = NT / 32;
+  static constexpr int BK = 128 / (int)sizeof(TIN);  // K elements of a stage
+  static constexpr int HROWS = (NT + 63) / 64 * 64;  // rows of a stage of hidden in LDS (64 are fetched at a time)
+  static constexpr int STAGE = BM * 128 + HROWS * 128;
+  static constexpr int LDS_BYTES = 2 * STAGE + (sizeof(TIN) == 2 ? 8 * 4096 : 0);  // two stages, a store tile per wave
 };
 
-template <typename TIN, int AUX>
-LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache policy of the loads of W
-  typedef FewFwdShape S;
-  constexpr int DEPTH = S::DEPTH, FN = S::FN, NT = S::NT;
-  constexpr int WL = S::BM / 64;  // 16-byte chunks of a W stage per thread: row tid / 8 + 64 i, chunk tid % 8 (hidden: one)
+// The products of W's rows [row0, vend64) with the NT hidden rows, 256 rows of W at a time; `pass(acc, m0, vbase, busy)` gets those of
+// rows vbase .. vbase + 31 (this wave's; busy: some exist) in acc[0][j][.], column j * 32 + lane % 32.  h_off: byte offset of hidden row
+// tid / 8 + 64 i (kBufNowhere: reads as zero) in the h_bytes behind h.
+template <typename TIN, int NT, int AUX, typename F>
+LCE_DEV void few_products(const TIN* W, int64_t ldw, int64_t row0, int64_t vend64, int64_t H, const TIN* h, int64_t h_bytes,
+                          const uint32_t (&h_off)[FewFwdShape<TIN, NT>::HROWS / 64], char* lds, F&& pass) {
+  typedef FewFwdShape<TIN, NT> S;
+  constexpr int DEPTH = S::DEPTH, FN = S::FN, HL = S::HROWS / 64;
+  constexpr int WL = S::BM / 64;  // 16-byte chunks of a W stage per thread: row tid / 8 + 64 i, chunk tid % 8
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
-  const int64_t row0 = (int64_t)blockIdx.x * p.split_stride;
-  const int64_t vend64 = row0 + p.split_span < p.V ? row0 + p.split_span : p.V;
   const int vend = (int)vend64;
-  const int n_k = (int)(p.H / 64), n_kp = (n_k + DEPTH - 1) / DEPTH * DEPTH;  // stages of a pass, rounded up to turns of the loop
-
-  float m[FN], a[FN], b[FN];
-  int lab[FN];
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    m[j] = kNegBig;
-    a[j] = 0.f;
-    b[j] = 0.f;
-    const int64_t t = j * 32 + ln;
-    const int64_t y = t < p.T ? p.labels[t] - p.label_offset : -1;
-    lab[j] = (y >= 0 && y < p.V) ? (int)y : -1;
-  }
+  const int n_k = (int)(H / S::BK), n_kp = (n_k + DEPTH - 1) / DEPTH * DEPTH;  // stages of a pass, rounded up to turns of the loop
 
   // rows beyond the range, tokens beyond T and stages beyond K read as zero
-  const uint32_t w_row = (uint32_t)(p.ldw * sizeof(TIN)), h_row = (uint32_t)(p.ldh * sizeof(TIN));
-  const uint32_t w_at = (uint32_t)(tid >> 3) * w_row + (tid & 7) * 16, h_at = (uint32_t)(tid >> 3) * h_row + (tid & 7) * 16;
-  u32x4_t pw[DEPTH][WL], pb[DEPTH];
+  const uint32_t w_row = (uint32_t)(ldw * sizeof(TIN));
+  const uint32_t w_at = (uint32_t)(tid >> 3) * w_row + (tid & 7) * 16;
+  u32x4_t pw[DEPTH][WL], pb[DEPTH][HL];
   int64_t f_row = row0;  // the next stage to fetch: first row of its pass, k
   int f_k = 0;
-  auto fetch = [&](u32x4_t (&w)[WL], u32x4_t& x) {
+  auto fetch = [&](u32x4_t (&w)[WL], u32x4_t (&x)[HL]) {
     const int64_t left = vend64 - f_row < S::BM ? vend64 - f_row : S::BM;
     const bool live = f_k < n_k && left > 0;
-    const buf_t wb = make_buf(p.W + f_row * p.ldw + 64 * (int64_t)f_k, live ? left * w_row - 128 * (int64_t)f_k : 0);
-    const buf_t hb = make_buf(p.h + 64 * (int64_t)f_k, live ? p.T * h_row - 128 * (int64_t)f_k : 0);
+    const buf_t wb = make_buf(W + f_row * ldw + S::BK * (int64_t)f_k, live ? left * w_row - 128 * (int64_t)f_k : 0);
+    const buf_t hb = make_buf(h + S::BK * (int64_t)f_k, live ? h_bytes - 128 * (int64_t)f_k : 0);
 #pragma unroll
     for (int i = 0; i < WL; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(wb, (int)(w_at + 64 * i * w_row), 0, AUX);
-    x = __builtin_amdgcn_raw_buffer_load_b128(hb, (int)h_at, 0, 0);
+#pragma unroll
+    for (int i = 0; i < HL; ++i) x[i] = __builtin_amdgcn_raw_buffer_load_b128(hb, (int)h_off[i], 0, 0);
     __builtin_amdgcn_sched_barrier(0);  // (the loads of one stage stay in front of the next one's)
     if (++f_k == n_kp) {
       f_k = 0;
@@ -134,7 +133,8 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
         buf ^= 1;
 #pragma unroll
         for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4_t*>(st + put + i * 8192) = pw[d][i];
-        *reinterpret_cast<u32x4_t*>(st + S::BM * 128 + put) = pb[d];
+#pragma unroll
+        for (int i = 0; i < HL; ++i) *reinterpret_cast<u32x4_t*>(st + S::BM * 128 + put + i * 8192) = pb[d][i];
         fetch(pw[d], pb[d]);
         // (a buffer is written again two stages on: every wave has passed the barrier between, after its reads of this stage)
         __syncthreads();
@@ -152,7 +152,37 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
         }
       }
     }
-    if (p.xcache) {
+    pass(acc, m0, vbase, busy);
+  }
+}
+
+// Forward.  AUX: cache policy of the loads of W
+template <typename TIN, int NT, int AUX>
+LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
+  typedef FewFwdShape<TIN, NT> S;
+  constexpr int FN = S::FN, HL = S::HROWS / 64;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  const int64_t row0 = (int64_t)blockIdx.x * p.split_stride;
+  const int64_t vend64 = row0 + p.split_span < p.V ? row0 + p.split_span : p.V;
+  const int vend = (int)vend64;
+  float m[FN], a[FN], b[FN];
+  int lab[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    m[j] = kNegBig;
+    a[j] = 0.f;
+    b[j] = 0.f;
+    const int64_t t = j * 32 + ln;
+    const int64_t y = t < p.T ? p.labels[t] - p.label_offset : -1;
+    lab[j] = (y >= 0 && y < p.V) ? (int)y : -1;
+  }
+  const uint32_t h_row = (uint32_t)(p.ldh * sizeof(TIN));
+  uint32_t h_off[HL];
+#pragma unroll
+  for (int i = 0; i < HL; ++i) h_off[i] = (uint32_t)((tid >> 3) + 64 * i) * h_row + (tid & 7) * 16;
+  few_products<TIN, NT, AUX>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * h_row, h_off, lds,
+                             [&](f32x16_t (&acc)[1][FN], int64_t m0, int vbase, bool) {
+    if constexpr (sizeof(TIN) == 2) if (p.xcache) {
       // the logits of this pass, for a backward that then has no need to recompute them.  A 32x32 block passes through 4 KB of
       // LDS of this wave's own and leaves it as whole lines, 1 KB (16 tokens x 16 rows of a panel) per store; rows in whole
       // fours, the last ones of W up to the end of the cache's panel.  Non-temporal (64 tokens, H=3584: step 632 -> 615 us,
@@ -178,7 +208,7 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
       }
     }
     fold_logits<1, FN>(acc, m, a, b, lab, p.c, vbase, vend, m0 + S::BM <= vend64, hh, p.xlabel + ln);
-  }
+  });
 
   // merge the two lane halves (same token, different vocabulary rows), then the waves
   __syncthreads();
@@ -204,11 +234,11 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {  // AUX: cache pol
 }
 
 // (which rows are read how: read_w_once, lce_host.hpp.  A branch around the whole body: none around a load.)
-template <typename TIN>
+template <typename TIN, int NT>
 __global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  if ((int64_t)blockIdx.x * p.split_stride < p.once_rows) fwd_few_body<TIN, kBufNonTemporal>(p, lds);
-  else fwd_few_body<TIN, 0>(p, lds);
+  if ((int64_t)blockIdx.x * p.split_stride < p.once_rows) fwd_few_body<TIN, NT, kBufNonTemporal>(p, lds);
+  else fwd_few_body<TIN, NT, 0>(p, lds);
 }
 
 template <typename TIN>

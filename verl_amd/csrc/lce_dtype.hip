@@ -40,22 +40,27 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case kSelN192:
       if (forward_w_once(T, V, ldw * (int64_t)sizeof(TuT))) LCE_RUN(VariantN192Once);
       LCE_RUN(VariantN192Plain);
+#define LCE_FEW(NT)                                                                                                          \
+  return forward_few<TuT, NT>((const TuT*)h, ldh, (const TuT*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, \
+                              ws, st, label_offset, shard_out, max_splits, xcache)
+#if LCE_TU_DTYPE != 1
+    case kSelT64: LCE_FEW(64);
     case kSelT128:
       if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT128Plain);
       LCE_RUN(VariantT128);
-#if LCE_TU_DTYPE != 1
-    case kSelT64:
-      return forward_few<TuT>((const TuT*)h, ldh, (const TuT*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
-                              label_offset, shard_out, max_splits, xcache);
 #else
     case kSelT64:
-      if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT64Plain);
-      LCE_RUN(VariantT64);
+      if (T <= 32) LCE_FEW(32);
+      LCE_FEW(64);
+    case kSelT128:
+      if (T <= 96) LCE_FEW(96);
+      LCE_FEW(128);
     case kSelTerms:
       return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
                            label_offset, shard_out);
 #endif
   }
+#undef LCE_FEW
 #undef LCE_RUN
   return fail(LCE_E_ARG, "tile selector %d out of range", sel);
 }

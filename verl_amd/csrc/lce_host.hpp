@@ -163,9 +163,8 @@ template <typename TIN> using VariantN192Once = VariantN192<TIN, 1>;
 template <typename TIN, int ONCE = 0> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1, 1, ONCE> Cfg; };
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring.  ONCE: the loads of W
 // are marked non-temporal (read_w_once)
-template <typename TIN, int ONCE = 1> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, ONCE> Cfg; };
+template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
 template <typename TIN, int ONCE = 1> struct VariantT128 { typedef GemmCfg<TIN, 256, 128, 128, 3, 4, 2, 0, 0, ONCE> Cfg; };
-template <typename TIN> using VariantT64Plain = VariantT64<TIN, 0>;
 template <typename TIN> using VariantT128Plain = VariantT128<TIN, 0>;
 constexpr int kNumVariants = 4;
 
@@ -405,9 +404,9 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
                        entropy_b, shard_out, st);
 }
 
-// forward with at most 64 tokens of 16 bits (few_tokens.hpp): one contiguous range of rows per workgroup, one workgroup per CU;
-// whole panels of the kept logits
-template <typename TIN>
+// forward with at most 64 tokens of 16 bits or 128 of fp32 (few_tokens.hpp): one contiguous range of rows per workgroup, one
+// workgroup per CU; whole panels of the kept logits
+template <typename TIN, int NT>
 int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                 int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, hipStream_t st,
                 int64_t label_offset, float* shard_out, int max_splits, float* xcache) {
@@ -424,9 +423,10 @@ int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int6
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   {
     ProfScope prof(PC_FWD, st);
-    auto kern = lce_fwd_few_kernel<TIN>;
-    allow_lds(kern, FewFwdShape::LDS_BYTES);
-    hipLaunchKernelGGL(kern, dim3((unsigned)S), dim3(512), FewFwdShape::LDS_BYTES, st, p);
+    typedef FewFwdShape<TIN, NT> Shape;
+    auto kern = lce_fwd_few_kernel<TIN, NT>;
+    allow_lds(kern, Shape::LDS_BYTES);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S), dim3(512), Shape::LDS_BYTES, st, p);
     int rc = check_launch("lce_fwd_few_kernel");
     if (rc) return rc;
   }
