@@ -2,6 +2,7 @@
 // that do not depend on the GEMM element type.  The forward / backward launchers are compiled per element type in
 // lce_dtype.hip.  Nothing here allocates device memory: callers bring the workspace.
 #include "lce_host.hpp"
+#include "lce_few_f32.hpp"
 #include "lce_terms.hpp"
 
 namespace lce_shared {
@@ -361,6 +362,7 @@ int lce_merge_shards(const float* partials, int R, int64_t T, int reduction, flo
 }
 
 static size_t backward_workspace_need(const Tuning& tu, int64_t T, int64_t H, int64_t V, size_t esz, int64_t vchunk, bool terms) {
+  if (esz == 4 && few_f32(tu, T)) return few_f32_layout(tu, T, H, V, vchunk).total + 256;
   return (terms ? terms_bwd_layout(tu, T, H, V, vchunk).total : bwd_layout(tu, T, H, V, esz, vchunk).total) + 256;
 }
 
@@ -400,7 +402,7 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
   const size_t need = backward_workspace_need(tu, T, H, V, esz, vchunk, terms);
   if (!workspace || workspace_bytes < need) return fail(LCE_E_WORKSPACE, "backward workspace too small: %zu < %zu", workspace_bytes, need);
   char* ws = reinterpret_cast<char*>(align256(reinterpret_cast<size_t>(workspace)));
-  return kBackward[dtype](terms ? kSelTerms : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
+  return kBackward[dtype](terms ? kSelTerms : esz == 4 && few_f32(tu, T) ? kSelFewF32 : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
                           accumulate, entropy_b, dlogprobs, dentropy, d_hidden, d_weight, grads_f32, ws, vchunk, st, vocab_offset,
                           tu, xcache);
 }

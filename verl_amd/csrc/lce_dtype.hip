@@ -4,6 +4,7 @@
 // lce_host.hpp.
 #include "lce_host.hpp"
 #if LCE_TU_DTYPE == 1
+#include "lce_few_f32.hpp"
 #include "lce_terms.hpp"
 #endif
 
@@ -92,6 +93,9 @@ int TU_FN(backward)(int sel, LCE_BWD_PARAMS) {
     case kSelTerms:
       return backward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
                             (float*)dw, ws, vchunk, st, vocab_offset, tu);
+    case kSelFewF32:
+      return backward_few_f32((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
+                              (float*)dw, ws, vchunk, st, vocab_offset, tu);
 #endif
   }
 #undef LCE_RUN

@@ -1,0 +1,137 @@
+// Host side of few_tokens_f32.hpp: the backward of fp32 inputs with at most 128 tokens.
+#pragma once
+#include "few_tokens_f32.hpp"
+#include "lce_host.hpp"
+
+namespace {
+
+struct FewF32Layout {
+  int64_t vchunk, pcol;
+  int nchunks, ksplit, nt;  // nt: token positions of the kernels
+  size_t off_dS, off_dHacc, off_rows, off_inv, off_nrows, off_acounts, off_tokc, off_tokl, total;
+};
+
+// Which calls: shapes and diagnostic settings alone.  Measured, forward + backward in ms (the forward is the same), tiles of 256 x 256
+// with transposed copies of W / this way, H=3584, V=152064: 1 token 7.6 / 1.57, 32: 7.8 / 1.74, 64: 8.2 / 2.7, 100: 8.7 / 4.5, 128:
+// 8.8 / 4.6; H=896: 2.7 / 0.47, 2.8 / 0.50, 3.0 / 0.80, 3.1 / 1.31, 3.1 / 1.36; without d_weight, H=3584, 16 tokens 6.4 / 1.32.  Error
+// against float64 (2-norm; H=896, V=151936, 64 tokens): d_hidden 3.8e-6 / 3.8e-6, d_weight 1.2e-7 / 4.2e-8.
+bool few_f32(const Tuning& tu, int64_t T) { return T <= 128 && !tu.variant_forced && tu.few_token_gemms && !tu.split_bwd; }
+
+FewF32Layout few_f32_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
+  FewF32Layout L;
+  L.nt = (int)round_up(T, 32);
+  L.vchunk = std::min(round_up(vchunk, 256), round_up(V, 256));
+  L.nchunks = (int)((V + L.vchunk - 1) / L.vchunk);
+  L.pcol = (int64_t)L.nt * 32 + 32;
+  // K slices of d_hidden: its workgroups fill the chip once, one to a CU; at least 256 rows of W per slice
+  const int64_t n_ht = (H + 255) / 256, fill = std::max<int64_t>(1, kNumCUs / n_ht);
+  L.ksplit = tu.dh_ksplit > 0 ? tu.dh_ksplit : (int)std::min(fill, std::max<int64_t>(1, L.vchunk / 256));
+  size_t o = 0;
+  L.off_dS = o;      o += align256((size_t)(L.vchunk / 32) * L.pcol * 4);
+  L.off_dHacc = o;   o += (size_t)L.ksplit * align256((size_t)T * H * 4);
+  L.off_rows = o;    o += align256((size_t)L.nt * 4);
+  L.off_inv = o;     o += align256((size_t)T * 4);
+  L.off_nrows = o;   o += 256;
+  L.off_acounts = o; o += 256;
+  L.off_tokc = o;    o += align256((size_t)L.nt * 16);
+  L.off_tokl = o;    o += align256((size_t)L.nt * 4);
+  L.total = o;
+  return L;
+}
+
+// one chunk where the bound of bwd_layout (a quarter of one [T, V] plus one fp32 [V, H]) or the budget has room for it
+FewF32Layout few_f32_layout(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
+  if (vchunk <= 0) {
+    double gate = (double)T * V + 4.0 * (double)V * H;
+    if (tu.ws_budget > 0 && (double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
+    vchunk = round_up(V, 256);
+    while (vchunk > 2048 && (double)few_f32_layout_for(tu, T, H, V, vchunk).total + 512.0 > gate) vchunk -= 1024;
+    if (vchunk < 2048) vchunk = 2048;
+    const int64_t n = (V + vchunk - 1) / vchunk;
+    vchunk = round_up((V + n - 1) / n, 256);
+  }
+  return few_f32_layout_for(tu, T, H, V, vchunk);
+}
+
+#if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1 && LCE_TU_PART == 1
+// d_logits, d_hidden and d_weight of one chunk
+template <int NT>
+int launch_few_f32(FewF32Args q, bool need_dh, bool need_dw, hipStream_t st) {
+  int rc;
+  {
+    typedef FewFwdShape<float, NT> S;
+    ProfScope prof(PC_BWD_DS, st);
+    q.span = round_up((q.vrows + kNumCUs - 1) / kNumCUs, 32);
+    allow_lds(lce_ds_few_f32_kernel<NT>, S::LDS_BYTES);
+    hipLaunchKernelGGL(lce_ds_few_f32_kernel<NT>, dim3((unsigned)((q.vrows + q.span - 1) / q.span)), dim3(512), S::LDS_BYTES, st, q);
+    if ((rc = check_launch("lce_ds_few_f32_kernel"))) return rc;
+  }
+  if (need_dh) {
+    typedef FewDhF32Shape<NT> S;
+    ProfScope prof(PC_GEMM_DH, st);
+    q.kslice = round_up((q.vrows + q.ksplit - 1) / q.ksplit, 32);
+    allow_lds(lce_dh_few_f32_kernel<NT>, S::LDS_BYTES);
+    hipLaunchKernelGGL(lce_dh_few_f32_kernel<NT>, dim3((unsigned)((q.H + S::HW - 1) / S::HW * q.ksplit)), dim3(512), S::LDS_BYTES, st, q);
+    if ((rc = check_launch("lce_dh_few_f32_kernel"))) return rc;
+  }
+  if (need_dw) {
+    typedef FewDwF32Shape<NT> S;
+    ProfScope prof(PC_GEMM_DW, st);
+    const int64_t n_ht = (q.H + S::HW - 1) / S::HW;
+    q.n_su = (int)std::max<int64_t>(1, std::min<int64_t>(kNumCUs / n_ht, (q.vrows + 31) / 32));
+    allow_lds(lce_dw_few_f32_kernel<NT>, S::LDS_BYTES);
+    hipLaunchKernelGGL(lce_dw_few_f32_kernel<NT>, dim3((unsigned)round_up(n_ht * q.n_su, 8)), dim3(512), S::LDS_BYTES, st, q);
+    if ((rc = check_launch("lce_dw_few_f32_kernel"))) return rc;
+  }
+  return LCE_OK;
+}
+
+int backward_few_f32(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
+                     int reduction, const float* maximum, const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
+                     float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu) {
+  const FewF32Layout L = few_f32_layout(tu, T, H, V, vchunk);
+  int* rows = reinterpret_cast<int*>(ws + L.off_rows);
+  int* inv = reinterpret_cast<int*>(ws + L.off_inv);
+  int* n_rows = reinterpret_cast<int*>(ws + L.off_nrows);
+  int* acounts = reinterpret_cast<int*>(ws + L.off_acounts);
+  const int64_t g_stride = reduction == LCE_REDUCTION_NONE ? 1 : 0, part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
+  FewF32Args q = {};
+  q.ldw = ldw; q.H = H; q.h = h; q.ldh = ldh; q.T = T; q.rows = rows; q.n_rows = n_rows;
+  q.dS = reinterpret_cast<float*>(ws + L.off_dS); q.pcol = L.pcol;
+  f32x4_t* tokc = reinterpret_cast<f32x4_t*>(ws + L.off_tokc);
+  int* tokl = reinterpret_cast<int*>(ws + L.off_tokl);
+  q.tokc = tokc; q.tokl = tokl; q.c = kLog2e / temperature;
+  q.dHp = reinterpret_cast<float*>(ws + L.off_dHacc); q.part_stride = part_stride; q.ksplit = L.ksplit;
+  int rc;
+  {
+    ProfScope prof(PC_ACTIVE_ROWS, st);
+    hipLaunchKernelGGL(active_count_kernel, dim3(1), dim3(256), 0, st, dlogprobs, g_stride, dentropy, T, acounts);
+    if ((rc = check_launch("active_count_kernel"))) return rc;
+    hipLaunchKernelGGL(active_rows_kernel, dim3(1), dim3(256), 0, st, dlogprobs, g_stride, dentropy, T, acounts, rows, inv, n_rows);
+    if ((rc = check_launch("active_rows_kernel"))) return rc;
+    hipLaunchKernelGGL(ds_token_consts_kernel, dim3(1), dim3(256), 0, st, rows, n_rows, T, (int64_t)L.nt, dlogprobs, g_stride,
+                       reduction == LCE_REDUCTION_MEAN ? 1.0f / (float)T : 1.0f, dentropy, maximum, accumulate, entropy_b, labels, vocab_offset, V,
+                       1.0f / temperature, tokc, tokl);
+    if ((rc = check_launch("ds_token_consts_kernel"))) return rc;
+  }
+  for (int c = 0; c < L.nchunks; ++c) {
+    const int64_t v0 = (int64_t)c * L.vchunk;
+    q.W = W + v0 * ldw; q.vrows = std::min(L.vchunk, V - v0); q.lab0 = v0;
+    q.accumulate = c > 0;
+    q.dW = d_weight ? d_weight + v0 * H : nullptr;
+    const bool dh = d_hidden != nullptr, dw = d_weight != nullptr;
+    rc = L.nt == 32 ? launch_few_f32<32>(q, dh, dw, st) : L.nt == 64 ? launch_few_f32<64>(q, dh, dw, st)
+       : L.nt == 96 ? launch_few_f32<96>(q, dh, dw, st) : launch_few_f32<128>(q, dh, dw, st);
+    if (rc) return rc;
+  }
+  if (!d_hidden) return LCE_OK;
+  ProfScope prof(PC_DH_FINISH, st);
+  LabelTerm lt;
+  lt.labels = nullptr; lt.v0 = vocab_offset; lt.V = V; lt.g_lp = dlogprobs; lt.g_stride = g_stride; lt.scale = 0.f;
+  hipLaunchKernelGGL((dh_finish_kernel<float, float>), dim3((unsigned)((T * (H / 4) + 255) / 256)), dim3(256), 0, st, q.dHp, L.ksplit, part_stride, inv, T,
+                     H, d_hidden, lt, W, ldw);
+  return check_launch("dh_finish_kernel");
+}
+#endif
+
+}  // namespace

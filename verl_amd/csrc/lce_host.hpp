@@ -58,8 +58,9 @@ struct Tuning {
 };
 
 // tile selectors of the per-type launchers: 0..3 are the variants of lce_set_variant, then the two few-token forward tiles
-// and the 16x16x32 loop on tiles 192 tokens wide, and the bfloat16 planes of fp32 inputs (lce_terms.hpp)
-enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7 };
+// and the 16x16x32 loop on tiles 192 tokens wide, the bfloat16 planes of fp32 inputs (lce_terms.hpp), and their backward with
+// few tokens (lce_few_f32.hpp)
+enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8 };
 
 // The launchers of one element type each (lce_dtype.hip compiles them as separate objects).  `sel` is a tile selector;
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
