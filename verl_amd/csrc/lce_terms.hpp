@@ -12,8 +12,7 @@
 namespace {
 
 // ---- forward ----------------------------------------------------------------------------------
-// The weight is split and multiplied chunk by chunk: a chunk holds whole rounds of tiles over the CUs (as many as 256 MB of
-// planes allow), and its splits are a block of their own in the list of partial statistics.
+// The weight is split and multiplied chunk by chunk; a chunk's splits are a block of their own in the list of partial statistics.
 struct TermsFwdPlan {
   int64_t rows;     // vocabulary rows of a chunk
   int nchunks, splits;  // splits: of all chunks together
@@ -25,10 +24,12 @@ int terms_fwd_splits(int ntt, int64_t rows) { return forward_splits_256(ntt, (in
 TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V) {
   TermsFwdPlan p;
   const int ntt = (int)((T + 255) / 256);
-  const int64_t most = std::max<int64_t>(1, ((int64_t)256 << 20) / (6 * H * 256));  // tiles of a chunk
-  int64_t tiles = most;
-  for (int64_t r = most * ntt / kNumCUs; r >= 1; --r)
-    if (r * kNumCUs / ntt >= 1) { tiles = r * kNumCUs / ntt; break; }
+  // whole rounds of tiles over the CUs: as many as 256 MB of planes allow, which the memory-side cache then holds from the split to
+  // the product, but one at least, through memory or not (forward in us, chunks of 256 MB / one round: H=3584, 300 tokens 5698 /
+  // 3392, 1000: 6278 / 5528; H=5120, 300: 10600 / 4902, 1000: 10882 / 8064)
+  const int64_t most = ((int64_t)256 << 20) / (6 * H * 256);  // tiles of a chunk
+  const int64_t rounds = std::max<int64_t>(1, most * ntt / kNumCUs);
+  const int64_t tiles = std::max<int64_t>(1, rounds * kNumCUs / ntt);
   p.rows = tiles * 256;
   p.nchunks = (int)((V + p.rows - 1) / p.rows);
   p.splits = 0;
