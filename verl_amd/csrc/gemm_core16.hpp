@@ -53,8 +53,8 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 
 // TRANS_: 0 both operands K-contiguous (row-major A[m][k], B[n][k]); 1 both K-major in memory, A[k][m] and
 // B[k][n], fetched with the transposing LDS read (two ds_read_b64_tr_b16 per fragment); 2 only A K-major (mixed).
-// NBN_: 16-column blocks per wave along the MFMA columns (tokens): 8 for tiles 256 columns wide, 6 for 192 (ragged token
-// counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
+// NBN_: 16-column blocks per wave along the MFMA columns (tokens): 8 for tiles 256 columns wide, 6 for 192, 5 and 7 for the last of a
+// row of tiles (ragged token counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
 // A_EARLY_: the ring's early operand (see main) is A instead of B.
 // TERMS_: products per slab.  1: the operands are what they are.  6: fp32 operands, each held as three bfloat16 planes
 // x = x1 + x2 + x3 (exact: 3 x 8 significant bits); a slab is multiplied as a1 b1 + a1 b2 + a2 b1 + a1 b3 + a3 b1 + a2 b2 into

@@ -93,13 +93,22 @@ struct Fwd16Stream {
   static constexpr bool value = !KEEP && Cfg::NBN == Cfg::NB && !Cfg::A_EARLY && Cfg::TERMS == 1;
 };
 
+// A last token tile with fewer tokens left is multiplied on the narrowest of 160, 192 and 224 columns that holds them, by a workgroup
+// of the same launch: the matrix work of the columns beyond costs time even where it is padding, at some 1400 W of socket power as energy.
+// Where the tiles are narrow already or the products six (forward in us, H=3584: 130 tokens 231 -> 214, 300: 380 -> 371, 333: 383 -> 374,
+// 352: 384 -> 370; fp32 on planes 300: 3401 -> 3220, 600: 4377 -> 4225); on the square tile's stream it does not show (1100 tokens
+// 1004 -> 1016, 5003: 4049 -> 4080).
+template <typename Cfg>
+struct Fwd16Tails {
+  static constexpr bool value = Cfg::A_EARLY || Cfg::TERMS == 6;
+  template <int NBN>
+  using Narrow = GemmCfg16<typename Cfg::TIN, 0, NBN, Cfg::A_EARLY, Cfg::TERMS, Cfg::A_ONCE>;
+};
+
 // KEEP: the tiles also write their logits to p.xcache (FwdArgs), for a backward that then does not recompute them
 template <typename Cfg, bool KEEP>
-LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, char* lds) {
+LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, char* lds) {
   constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
-  int tt, s;
-  if (!p.map.decode(blockIdx.x, tt, s)) return;
-  const int64_t n0 = (int64_t)tt * Cfg::BN;
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
   GemmCore16<Cfg> g;
   g.set_lane();
@@ -797,7 +806,17 @@ inline __global__ void split_again_kernel(const int* wide, SplitArgs a, SplitArg
 template <typename Cfg, bool KEEP = false>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd16_kernel(FwdArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  fwd16_body<Cfg, KEEP>(p, lds);
+  int tt, s;
+  if (!p.map.decode(blockIdx.x, tt, s)) return;
+  const int64_t n0 = (int64_t)tt * Cfg::BN, left = p.T - n0;
+  if constexpr (Fwd16Tails<Cfg>::value) {
+    if (left <= 160) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<5>, KEEP>(p, n0, s, lds);
+    if constexpr (Cfg::NBN > 6) {
+      if (left <= 192) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<6>, KEEP>(p, n0, s, lds);
+      if (left <= 224) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<7>, KEEP>(p, n0, s, lds);
+    }
+  }
+  fwd16_body<Cfg, KEEP>(p, n0, s, lds);
 }
 
 template <typename Cfg>
