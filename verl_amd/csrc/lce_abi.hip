@@ -234,8 +234,8 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
     if (T <= 64) sel = kSelT64;
     else if (T <= 128) sel = kSelT128;
     else if (esize(dtype) == 2 && forward_tiles_192(T, V)) sel = kSelN192;
+    else if (esize(dtype) == 2) sel = T > kCore16MinTokensFwd ? kVariantCore16 : kSelWEarly;
     else if (T <= 512) sel = 0;  // W (the A operand) streams from HBM: give it the early slot
-    else if (esize(dtype) == 2 && T > kCore16MinTokensFwd) sel = kVariantCore16;
     // the split ring: measured 4-7% faster than the 2-stage ring up to 8192 tokens, equal (+-1%) beyond, and
     // 4.5% faster again once `hidden` is far larger than the memory-side cache (T=65536, H=5120: 671 MB)
     else if (T <= 8192 || (uint64_t)T * (uint64_t)H * esize(dtype) > (512ull << 20)) sel = 1;
@@ -243,7 +243,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   if (terms) sel = kSelTerms;
-  if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192) && esize(dtype) == 2))
+  if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
                          accumulate, entropy_b, ws, st, label_offset, shard_out, max_splits, xcache);

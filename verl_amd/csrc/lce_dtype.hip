@@ -39,8 +39,11 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case 2: LCE_RUN(Variant2);
     case 3: LCE_RUN(Variant3);
     case kSelN192:
-      if (forward_w_once(T, V, ldw * (int64_t)sizeof(TuT))) LCE_RUN(VariantN192Once);
+      if (forward_w_once(T, 192, V, ldw * (int64_t)sizeof(TuT))) LCE_RUN(VariantN192Once);
       LCE_RUN(VariantN192Plain);
+    case kSelWEarly:
+      if (forward_w_once(T, 256, V, ldw * (int64_t)sizeof(TuT))) LCE_RUN(VariantWEarlyOnce);
+      LCE_RUN(VariantWEarlyPlain);
 #define LCE_FEW(NT)                                                                                                          \
   return forward_few<TuT, NT>((const TuT*)h, ldh, (const TuT*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, \
                               ws, st, label_offset, shard_out, max_splits, xcache)

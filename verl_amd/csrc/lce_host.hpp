@@ -36,7 +36,11 @@ extern std::vector<hipEvent_t> prof_pool;
 // four-wave 16x16x32 loop (variant 3) above the token counts below.
 constexpr int kDefaultVariantFwd = 2, kDefaultVariantBwd = 1, kVariantCore16 = 3;
 // variant 3 is the default above these token counts (measured at H=3584, V=152064: the forward gains 2-6% from 1024
-// tokens on; the backward runs its gradient GEMMs on it wherever the streaming kernels of few_tokens.hpp end)
+// tokens on; the backward runs its gradient GEMMs on it wherever the streaming kernels of few_tokens.hpp end).  Up to
+// kCore16MinTokensFwd the forward of 16-bit inputs takes the same loop with the weight early (VariantWEarly), or the narrow tiles:
+// forward in us against the eight-wave loop, H=3584: 193 to 224 tokens 283 -> 242, 256: 289 -> 270, 440: 478 -> 446, 512: 484 -> 457;
+// H=896: 88 -> 79, 90 -> 87, 144 -> 136, 148 -> 139; H=5120: 400 -> 345, 415 -> 375, 676 -> 628, 688 -> 645; beyond, the stream of
+// slabs that only the other order has is 1 to 3 % faster (1000 tokens 832 / 847).
 constexpr int64_t kCore16MinTokensFwd = 512, kCore16MinTokensBwd = 128;
 // up to here a backward that fits one vocabulary chunk runs its two gradient GEMMs as launches of their own, d_weight on
 // workgroups that stay (lce_dw16_kernel); beyond, a tile's K loop is long enough to hide most of its start and its stores, and
@@ -58,9 +62,9 @@ struct Tuning {
 };
 
 // tile selectors of the per-type launchers: 0..3 are the variants of lce_set_variant, then the two few-token forward tiles
-// and the 16x16x32 loop on tiles 192 tokens wide, the bfloat16 planes of fp32 inputs (lce_terms.hpp), and their backward with
+// and the 16x16x32 loop on tiles 192 tokens wide or with the weight early, the bfloat16 planes of fp32 inputs (lce_terms.hpp), and their backward with
 // few tokens (lce_few_f32.hpp)
-enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8 };
+enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8, kSelWEarly = 9 };
 
 // The launchers of one element type each (lce_dtype.hip compiles them as separate objects).  `sel` is a tile selector;
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
@@ -158,10 +162,13 @@ template <typename TIN, int ONCE = 0> struct VariantN192 { typedef GemmCfg16<TIN
 template <int ONCE> struct VariantN192<float, ONCE> : Variant3<float> {};
 template <typename TIN> using VariantN192Plain = VariantN192<TIN, 0>;
 template <typename TIN> using VariantN192Once = VariantN192<TIN, 1>;
-// the square tile with the weight early (d_hidden of its own: 512 tokens 425 -> 412 us).  ONCE, up to two tiles of tokens and with a
+// the square tile with the weight early.  d_hidden of its own (512 tokens 425 -> 412 us); ONCE, up to two tiles of tokens and with a
 // d_weight to follow: step at 256 tokens 953 -> 904 us, 512: 1604 -> 1570; from 600 tokens on level, and without a d_weight
-// the other way (450 tokens, H=5120: 1520 -> 1540, 1000: 2728 -> 2767)
+// the other way (450 tokens, H=5120: 1520 -> 1540, 1000: 2728 -> 2767).  Forward: kCore16MinTokensFwd
 template <typename TIN, int ONCE = 0> struct VariantWEarly { typedef GemmCfg16<TIN, 0, 8, 1, 1, ONCE> Cfg; };
+template <int ONCE> struct VariantWEarly<float, ONCE> : Variant3<float> {};
+template <typename TIN> using VariantWEarlyPlain = VariantWEarly<TIN, 0>;
+template <typename TIN> using VariantWEarlyOnce = VariantWEarly<TIN, 1>;
 // forward with few tokens (one pass over W, HBM-bound): narrow token tiles leave LDS for a deeper ring.  ONCE: the loads of W
 // are marked non-temporal (read_w_once)
 template <typename TIN> struct VariantT64 { typedef GemmCfg<TIN, 256, 64, 128, 4, 4, 2, 0, 0, 1> Cfg; };
@@ -190,9 +197,9 @@ void allow_lds(K kernel, int bytes) {
 constexpr int64_t kMallBytes = (int64_t)256 << 20;  // the memory-side cache
 bool read_w_once(int64_t V, int64_t row_bytes, const float* xcache) { return xcache || V * row_bytes > kMallBytes * 5 / 4; }
 
-// The same question for the 16x16x32 loop with one tile of 192 tokens.  130 / 192 tokens, forward alone, plain / non-temporal, us:
+// The same question for the 16x16x32 loop with one tile of tokens.  130 / 192 tokens, forward alone, plain / non-temporal, us:
 // H=3584 (1.09 GB) 228 / 218, 238 / 224; H=896 (272 MB) 68.8 / 71.3, 74.2 / 75.1, and with a backward behind it 214 / 222.
-bool forward_w_once(int64_t T, int64_t V, int64_t row_bytes) { return T <= 192 && V * row_bytes > kMallBytes * 5 / 4; }
+bool forward_w_once(int64_t T, int64_t tile, int64_t V, int64_t row_bytes) { return T <= tile && V * row_bytes > kMallBytes * 5 / 4; }
 
 int block_rows(int nrow_tiles) { return TileMap::block_rows(nrow_tiles); }
 
