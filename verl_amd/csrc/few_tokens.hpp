@@ -262,6 +262,7 @@ struct FewArgs {
   int64_t kslice;     // columns of dS per slice, a multiple of 64
   int accumulate;     // d_hidden partials: 0 store, 1 add to what is there (second and later chunks)
   int n_su;           // d_weight: workgroups side by side along the vocabulary
+  int by_xcd;         // d_hidden: each XCD takes a contiguous eighth of the workgroups
 };
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -457,6 +458,10 @@ __global__ __launch_bounds__(512, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 // bytes of dS.  What bounds it is the read of W, and that by the bytes in flight: DEPTH stages are on their way in registers
 // (128 KB of W per CU up to 64 tokens, 96 KB beyond) while one is multiplied out of LDS, which holds two, so that a stage
 // costs one barrier.
+// The workgroups of one slice read the same dS.  Numbered across the XCDs, the neighbours of a slice read pieces of the same rows of W at
+// the same time; numbered within them (by_xcd), dS passes into each L2 about once instead of in all eight.  The second from 33 tokens
+// on, where dS is a tenth of W and more: frozen head, 64 tokens, H=3584 410.8 -> 406.0 us, 4096: 377.5 -> 368.2, 5120: 569.4 -> 565.0;
+// step of 1 / 16 tokens at H=3584 566 -> 573, 581 -> 583.
 // ------------------------------------------------------------------------------------------------------------------
 template <int KT>
 struct FewShape {  // KT: token positions, 64 up to 64 tokens, else 128
@@ -480,7 +485,9 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
   const int wc = wave & 3, wt = wave >> 2;
   const int g = lane >> 4, l16 = lane & 15, e = l16 >> 2, q = l16 & 3;
   const int n_ht = (int)((p.H + HW - 1) / HW);
-  const int ht = blockIdx.x % n_ht, s = blockIdx.x / n_ht;
+  const int id = p.by_xcd ? (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  if (id >= n_ht * p.ksplit) return;
+  const int ht = id % n_ht, s = id / n_ht;
   const int64_t h0 = (int64_t)ht * HW;
   const int64_t k_begin = (int64_t)s * p.kslice;
   const int64_t k_left = p.ucols - k_begin;

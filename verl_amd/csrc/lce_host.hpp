@@ -698,7 +698,7 @@ int launch_few_gemms(FewArgs<typename Cfg::TIN> q, bool with_dh, hipStream_t st)
     const int n_ht = (int)((q.H + S::HW - 1) / S::HW);
     auto kern = lce_dh_few_kernel<TIN, KPerm<Cfg>, KT>;
     allow_lds(kern, S::DH_LDS);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(n_ht * q.ksplit)), dim3(512), S::DH_LDS, st, q);
+    hipLaunchKernelGGL(kern, dim3((unsigned)round_up((int64_t)n_ht * q.ksplit, 8)), dim3(512), S::DH_LDS, st, q);
     if ((rc = check_launch("lce_dh_few_kernel"))) return rc;
   }
   return q.dW ? launch_dw_few<Cfg, TOUT, KT>(q, st) : LCE_OK;
@@ -885,7 +885,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           q.dHp = dHacc; q.part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
           q.ksplit = L.ksplit; q.kslice = round_up((q.ucols + L.ksplit - 1) / L.ksplit, 64);
           q.accumulate = cc == 0 ? 0 : 1;
-          q.n_su = 1;
+          q.n_su = 1; q.by_xcd = T > 32;
           if (T <= 64) rc = grads_f32 ? launch_few_gemms<Cfg, float, 64>(q, need_dh, st) : launch_few_gemms<Cfg, TIN, 64>(q, need_dh, st);
           else rc = grads_f32 ? launch_few_gemms<Cfg, float, 128>(q, need_dh, st) : launch_few_gemms<Cfg, TIN, 128>(q, need_dh, st);
           if (rc) return rc;
