@@ -776,29 +776,6 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     hipLaunchKernelGGL(active_rows_kernel, dim3(nblk), dim3(256), 0, st, dlogprobs, ca.g_stride, dentropy, T, acounts, rows, inv, n_rows);
     if ((rc = check_launch("active_rows_kernel"))) return rc;
   }
-  if (L.sort_items && !one_prep) {
-    ProfScope prof(PC_LABEL_ROWS, st);
-    if constexpr (sizeof(TIN) == 2) if (with_coef) {
-      hipLaunchKernelGGL(label_coef_kernel<TIN>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, ca);
-      if ((rc = check_launch("label_coef_kernel"))) return rc;
-    }
-    const int nblocks = L.sort_items / kSortBlock;
-    if (!need_dw) {
-      // (the tokens grouped by label serve the one-hot rows of d_weight only)
-    } else {
-      int* hist = reinterpret_cast<int*>(ws + L.off_hist);
-      hipLaunchKernelGGL(label_keys_kernel, dim3(L.sort_items / 256), dim3(256), 0, st, lt, rows, n_rows, T, L.sort_items, skeys[0], svals[0]);
-      if ((rc = check_launch("label_keys_kernel"))) return rc;
-      for (int ps = 0; ps < L.sort_passes; ++ps) {
-        const int in = ps & 1, out = in ^ 1;
-        hipLaunchKernelGGL(sort_hist_kernel, dim3(nblocks), dim3(256), 0, st, skeys[in], 8 * ps, nblocks, hist);
-        hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(1024), 0, st, hist, 256 * nblocks);
-        hipLaunchKernelGGL(sort_scatter_kernel, dim3(nblocks), dim3(256), 0, st, skeys[in], svals[in], skeys[out], svals[out], 8 * ps,
-                           nblocks, hist);
-        if ((rc = check_launch("label sort pass"))) return rc;
-      }
-    }
-  }
   if (tokc && !one_prep) {
     ProfScope prof(PC_ACTIVE_ROWS, st);
     hipLaunchKernelGGL(ds_token_consts_kernel, dim3((unsigned)((L.tpad + 255) / 256)), dim3(256), 0, st, rows, n_rows, T, L.tpad, dlogprobs,
@@ -1055,6 +1032,31 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       }
     }
     return LCE_OK;
+  }
+  // What only the last two launches below read comes behind the products: a dozen launches of 5 us, each of which the host takes
+  // 8 to 10 for, so that after a synchronisation (an actor step waits for its loss's lengths) the device would wait for them.
+  if (L.sort_items) {
+    ProfScope prof(PC_LABEL_ROWS, st);
+    if constexpr (sizeof(TIN) == 2) if (with_coef) {
+      hipLaunchKernelGGL(label_coef_kernel<TIN>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, ca);
+      if ((rc = check_launch("label_coef_kernel"))) return rc;
+    }
+    const int nblocks = L.sort_items / kSortBlock;
+    if (!need_dw) {
+      // (the tokens grouped by label serve the one-hot rows of d_weight only)
+    } else {
+      int* hist = reinterpret_cast<int*>(ws + L.off_hist);
+      hipLaunchKernelGGL(label_keys_kernel, dim3(L.sort_items / 256), dim3(256), 0, st, lt, rows, n_rows, T, L.sort_items, skeys[0], svals[0]);
+      if ((rc = check_launch("label_keys_kernel"))) return rc;
+      for (int ps = 0; ps < L.sort_passes; ++ps) {
+        const int in = ps & 1, out = in ^ 1;
+        hipLaunchKernelGGL(sort_hist_kernel, dim3(nblocks), dim3(256), 0, st, skeys[in], 8 * ps, nblocks, hist);
+        hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(1024), 0, st, hist, 256 * nblocks);
+        hipLaunchKernelGGL(sort_scatter_kernel, dim3(nblocks), dim3(256), 0, st, skeys[in], svals[in], skeys[out], svals[out], 8 * ps,
+                           nblocks, hist);
+        if ((rc = check_launch("label sort pass"))) return rc;
+      }
+    }
   }
   if (need_dh) {
     // d_hidden = ordered sum of the fp32 partials, rounded once; zero rows for tokens without gradient
