@@ -402,8 +402,9 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
         hipLaunchKernelGGL((lce_fwd16_kernel<Cfg, false>), dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
       }
     } else {
-      allow_lds(lce_fwd_kernel<Cfg>, Cfg::LDS_BYTES);
-      hipLaunchKernelGGL(lce_fwd_kernel<Cfg>, dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
+      auto kern = sizeof(TIN) == 2 && xcache ? lce_fwd_kernel<Cfg, sizeof(TIN) == 2> : lce_fwd_kernel<Cfg, false>;  // (fp32 keeps none)
+      allow_lds(kern, Cfg::LDS_BYTES);
+      hipLaunchKernelGGL(kern, dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
     }
     rc = check_launch("lce_fwd_kernel");
   }

@@ -135,7 +135,43 @@ LCE_DEV void fold_logits(f32x16_t (&acc)[FM][FN], float (&m)[FN], float (&a)[FN]
   }
 }
 
+// The logits of one wave tile, kept for a backward that then has no need to recompute them.  A lane holds 4 + 4 rows of each
+// panel of a token (its partner 32 lanes on the others): two lane swaps, of halves and of rows of 16, and each register of a
+// block column holds 16 tokens x 16 rows, one whole kilobyte per store.  As 16-byte pieces of half lines straight from the
+// registers, which only merge in L2, the kernel took 262 us with and 208 without the stores (100 tokens, H=3584, V=152064: 62 MB,
+// 11 us at the rate of writes); whole lines can be marked non-temporal (half lines so marked: 222 instead of 209): step 692 ->
+// 668 us, 128 tokens 702 -> 678, H=5120 at 100 961 -> 927, H=4096 586 -> 579, H=896 258 -> 255.  They are issued AHEAD of the next tile's first
+// loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older than every load it
+// waits for, those counts mean what they say (behind the loads, with the counts raised by the 16 stores: 0 to 0.5 % slower).
 template <typename Cfg>
+LCE_DEV void keep_logits(const FwdArgs<typename Cfg::TIN>& p, const f32x16_t (&acc)[Cfg::FM][Cfg::FN], int64_t t0, int vbase, int vend, int lane) {
+  const int l16 = lane & 15, quad = lane >> 4, panel = (int)p.T * 64;
+  const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)Cfg::FM * 2 * panel);
+#pragma unroll
+  for (int j = 0; j < Cfg::FN; ++j)
+#pragma unroll
+    for (int i = 0; i < Cfg::FM; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        u32x4_t lo, hi;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t x0 = __builtin_bit_cast(uint32_t, (float)acc[i][j][8 * h + e]), x1 = __builtin_bit_cast(uint32_t, (float)acc[i][j][8 * h + 4 + e]);
+          const auto x = __builtin_amdgcn_permlane32_swap(x0, x1, false, false);
+          const auto y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+          lo[e] = y[0];
+          hi[e] = y[1];
+        }
+        const int64_t t = t0 + j * 32 + l16;
+        const int at = (2 * i + h) * panel + (int)t * 64 + quad * 16;
+        // (rows in whole fours, the last ones of W up to the end of the cache's panel)
+        const bool live = vbase + 32 * i + 16 * h + 4 * quad < vend;
+        __builtin_amdgcn_raw_buffer_store_b128(lo, kept, live && t < p.T ? at : kBufNowhere, 0, kBufNonTemporal);
+        __builtin_amdgcn_raw_buffer_store_b128(hi, kept, live && t + 16 < p.T ? at + 1024 : kBufNowhere, 0, kBufNonTemporal);
+      }
+}
+
+template <typename Cfg, bool KEEP>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   int tt, s;
@@ -171,34 +207,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd_kernel(FwdArgs<typename
     const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
     const bool full = m0 + Cfg::BM <= vend64;
     __builtin_amdgcn_sched_barrier(0);
-    {
-      // the logits of this tile, for a backward that then has no need to recompute them: a lane holds four consecutive
-      // vocabulary rows of a token in four consecutive registers, 16 bytes of that token's row of the cache; the lanes'
-      // pieces of a 128-byte line meet in L2.  Issued AHEAD of the next tile's first loads: the K loop waits on counts
-      // of outstanding vector-memory operations, and with the stores older than every load it waits for, those counts
-      // mean what they say.
-      if (p.xcache) {
-#pragma unroll
-        for (int j = 0; j < Cfg::FN; ++j) {
-          const int64_t t = n0 + g.wave_n * Cfg::WN + j * 32 + ln;
-          if (t >= p.T) continue;
-#pragma unroll
-          for (int i = 0; i < Cfg::FM; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int v = vbase + acc_row(i, 4 * q, hh);
-              if (v + 3 < vend) {
-                const f32x4_t x4 = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                *reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)) = x4;  // (non-temporal stores: 222 instead of 209 us)
-              } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (v + e < vend) *kept_logit(p.xcache, p.T, t, v + e) = acc[i][j][4 * q + e];
-              }
-            }
-        }
-      }
-    }
+    if constexpr (KEEP) keep_logits<Cfg>(p, acc, n0 + g.wave_n * Cfg::WN, vbase, vend, lane);
     __builtin_amdgcn_sched_barrier(0);
     // start fetching the next tile's first slabs now: the loads fly while this tile's statistics are
     // folded in (the epilogue touches neither LDS nor vector memory on its common path)
