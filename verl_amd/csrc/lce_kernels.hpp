@@ -991,6 +991,9 @@ struct LabelTerm {
 // without `inv`), or zeros where inv[t] < 0 (token without upstream gradient).  The sum runs in the
 // fixed order s = 0, 1, ..., so the result does not depend on scheduling.  H a multiple of 4.
 // With a label term, G_t * W[label_t][:] is added in fp32 before the one rounding.
+// Up to 64 slices, with a workgroup or less to a CU where there are few tokens: what bounds it is the chain of loads, so 16 of
+// them are in flight at a time (8 tokens of H=896, 64 slices: 19 us as the compiler had it, now 6 to 8; 128 tokens: 20, now 8.5; one column
+// per thread in place of four, for more workgroups, is no faster).
 // (bid of nblocks workgroups: the kernel's own grid, or the part of a larger grid that does this work)
 template <typename T, typename TOUT>
 LCE_DEV void dh_finish_body(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H, TOUT* out,
@@ -999,26 +1002,39 @@ LCE_DEV void dh_finish_body(const float* part, int S, int64_t stride, const int*
   for (int64_t q = bid * blockDim.x + threadIdx.x; q < n; q += nblocks * blockDim.x) {
     const int64_t t = q / per_row, c = (q - t * per_row) * 4;
     const int64_t pos = inv ? (int64_t)inv[t] : t;
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f};
     if (pos >= 0) {
       const float* src = part + pos * H + c;
-      a = *reinterpret_cast<const float4*>(src);
-      for (int s = 1; s < S; ++s) {
-        const float4 b = *reinterpret_cast<const float4*>(src + s * stride);
-        a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+      a = *reinterpret_cast<const f32x4_t*>(src);
+      int s = 1;
+      for (; s + 16 <= S; s += 16) {
+        f32x4_t b[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) b[i] = *reinterpret_cast<const f32x4_t*>(src + (s + i) * stride);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a += b[i];
       }
+      for (; s + 4 <= S; s += 4) {
+        f32x4_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = *reinterpret_cast<const f32x4_t*>(src + (s + i) * stride);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a += b[i];
+      }
+      for (; s < S; ++s) a += *reinterpret_cast<const f32x4_t*>(src + s * stride);
       if (lt.labels) {
         const float G = lt.g_lp[t * lt.g_stride] * lt.scale;
         const int64_t y = lt.labels[t] - lt.v0;
         if (G != 0.f && y >= 0 && y < lt.V) {
           const T* w = W + y * ldw + c;
-          a.x = __builtin_fmaf(G, (float)w[0], a.x); a.y = __builtin_fmaf(G, (float)w[1], a.y);
-          a.z = __builtin_fmaf(G, (float)w[2], a.z); a.w = __builtin_fmaf(G, (float)w[3], a.w);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(G, (float)w[e], a[e]);
         }
       }
     }
     TOUT* dst = out + t * H + c;
-    dst[0] = round_to<TOUT>(a.x); dst[1] = round_to<TOUT>(a.y); dst[2] = round_to<TOUT>(a.z); dst[3] = round_to<TOUT>(a.w);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e] = round_to<TOUT>(a[e]);
   }
 }
 
