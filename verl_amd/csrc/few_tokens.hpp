@@ -455,9 +455,9 @@ __global__ __launch_bounds__(512, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 // NT token rows and one K slice of the chunk's dS columns; wave w multiplies columns h0 + 64 (w % 4) .. +63 with half of the
 // token rows:  C[m = h][n = t] = sum_u W[vocab_at(u)][h] * dS[t][u].
 // A stage is 64 columns of dS: 64 rows of W (512 bytes of each, fetched in the order of dS's columns) and NT x 128
-// bytes of dS.  What bounds it is the read of W, and that by the bytes in flight: DEPTH stages are on their way in registers
-// (128 KB of W per CU up to 64 tokens, 96 KB beyond) while one is multiplied out of LDS, which holds two, so that a stage
-// costs one barrier.
+// bytes of dS.  What bounds it is the read of W, and that by the bytes in flight: four stages are on their way in registers
+// (128 KB of W per CU; three, 96 KB, beyond 64 tokens: step of 100 / 128 tokens at H=3584 674 / 686 us, four 667 / 678, H=5120 935 / 950,
+// four 923 / 945, others level) while one is multiplied out of LDS, which holds two, so that a stage costs one barrier.
 // The workgroups of one slice read the same dS.  Numbered across the XCDs, the neighbours of a slice read pieces of the same rows of W at
 // the same time; numbered within them (by_xcd), dS passes into each L2 about once instead of in all eight.  The second from 33 tokens
 // on, where dS is a tenth of W and more: frozen head, 64 tokens, H=3584 410.8 -> 406.0 us, 4096: 377.5 -> 368.2, 5120: 569.4 -> 565.0;
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(512, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 template <int KT>
 struct FewShape {  // KT: token positions, 64 up to 64 tokens, else 128
   static constexpr int HW = 256;                                     // columns of H per workgroup
-  static constexpr int DH_DEPTH = KT <= 64 ? 4 : 3;
+  static constexpr int DH_DEPTH = 4;
   static constexpr int DH_STAGE = 64 * HW * 2 + KT * 128;            // W rows, dS tile
   static constexpr int DH_LDS = 2 * DH_STAGE;
 };
