@@ -13,6 +13,8 @@
 // but 400 to 500 for both at once.  Everything is plain HIP with compiler-placed waits; K-major operands (hidden[t][.],
 // dS[t][.], W[v][.] in the gradients) are read through the transposing LDS read ds_read_b64_tr_b16.
 #pragma once
+#include <type_traits>
+
 #include "gemm_core.hpp"
 #include "lce_kernels.hpp"
 
@@ -80,7 +82,11 @@ struct FewFwdShape {
 // The products of W's rows [row0, vend64) with the NT hidden rows, 256 rows of W at a time; `pass(acc, m0, vbase, busy)` gets those of
 // rows vbase .. vbase + 31 (this wave's; busy: some exist) in acc[0][j][.], column j * 32 + lane % 32.  h_off: byte offset of hidden row
 // tid / 8 + 64 i (kBufNowhere: reads as zero) in the h_bytes behind h.
-template <typename TIN, int NT, int AUX, typename F>
+// HALF: a pass is whole turns of the loop over the DEPTH stages in flight and half a one (16 bits: H is a multiple of 128 but not of
+// 256), and every second pass starts at the second half of the ring.  Rounded up to whole turns, a seventh of the stages were zeros at
+// H=896: 1 / 40 / 64 tokens, V=151936, 50.7 / 51.7 / 52.1 -> 49.2 / 49.6 / 50.0 us.  (A branch around them in the loop costs more than they
+// do: 57 us; the waits behind it are for all loads.)
+template <typename TIN, int NT, int AUX, bool HALF, typename F>
 LCE_DEV void few_products(const TIN* W, int64_t ldw, int64_t row0, int64_t vend64, int64_t H, const TIN* h, int64_t h_bytes,
                           const uint32_t (&h_off)[FewFwdShape<TIN, NT>::HROWS / 64], char* lds, F&& pass) {
   typedef FewFwdShape<TIN, NT> S;
@@ -88,7 +94,7 @@ LCE_DEV void few_products(const TIN* W, int64_t ldw, int64_t row0, int64_t vend6
   constexpr int WL = S::BM / 64;  // 16-byte chunks of a W stage per thread: row tid / 8 + 64 i, chunk tid % 8
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
   const int vend = (int)vend64;
-  const int n_k = (int)(H / S::BK), n_kp = (n_k + DEPTH - 1) / DEPTH * DEPTH;  // stages of a pass, rounded up to turns of the loop
+  const int n_k = (int)(H / S::BK), n_kp = HALF ? n_k : (n_k + DEPTH - 1) / DEPTH * DEPTH;  // stages of a pass, of whole turns of the loop
 
   // rows beyond the range, tokens beyond T and stages beyond K read as zero
   const uint32_t w_row = (uint32_t)(ldw * sizeof(TIN));
@@ -118,46 +124,67 @@ LCE_DEV void few_products(const TIN* W, int64_t ldw, int64_t row0, int64_t vend6
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) fetch(pw[d], pb[d]);
   int buf = 0;
-  for (int64_t m0 = row0; m0 < vend64; m0 += S::BM) {
-    f32x16_t acc[1][FN];
+  f32x16_t acc[1][FN];
+  int64_t m0 = row0;
+  auto begin = [&] {
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
-    const int vbase = (int)m0 + wave * 32;  // this wave's first row
-    const bool busy = vbase < vend;         // (a short last pass leaves the LDS to the waves that have rows)
-    for (int k0 = 0; k0 < n_kp; k0 += DEPTH) {
+  };
+  // stages [D0, D1) of a turn
+  auto stages = [&](auto d0, auto d1) {
+    const bool busy = m0 + wave * 32 < vend;  // (a short last pass leaves the LDS to the waves that have rows)
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        char* st = lds + buf * S::STAGE;
-        buf ^= 1;
+    for (int d = d0.value; d < d1.value; ++d) {
+      char* st = lds + buf * S::STAGE;
+      buf ^= 1;
 #pragma unroll
-        for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4_t*>(st + put + i * 8192) = pw[d][i];
+      for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4_t*>(st + put + i * 8192) = pw[d][i];
 #pragma unroll
-        for (int i = 0; i < HL; ++i) *reinterpret_cast<u32x4_t*>(st + S::BM * 128 + put + i * 8192) = pb[d][i];
-        fetch(pw[d], pb[d]);
-        // (a buffer is written again two stages on: every wave has passed the barrier between, after its reads of this stage)
-        __syncthreads();
-        if (busy) {
+      for (int i = 0; i < HL; ++i) *reinterpret_cast<u32x4_t*>(st + S::BM * 128 + put + i * 8192) = pb[d][i];
+      fetch(pw[d], pb[d]);
+      // (a buffer is written again two stages on: every wave has passed the barrier between, after its reads of this stage)
+      __syncthreads();
+      if (busy) {
 #pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            const int c = ((2 * kk + hh) ^ sw) * 16;
-            const u32x4_t af = *reinterpret_cast<const u32x4_t*>(st + a_rd + c);
-            u32x4_t bf[FN];
+        for (int kk = 0; kk < 4; ++kk) {
+          const int c = ((2 * kk + hh) ^ sw) * 16;
+          const u32x4_t af = *reinterpret_cast<const u32x4_t*>(st + a_rd + c);
+          u32x4_t bf[FN];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const u32x4_t*>(st + b_rd + j * 4096 + c);
+          for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const u32x4_t*>(st + b_rd + j * 4096 + c);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) Mma<TIN>::run(acc[0][j], af, bf[j]);
-          }
+          for (int j = 0; j < FN; ++j) Mma<TIN>::run(acc[0][j], af, bf[j]);
         }
       }
     }
-    pass(acc, m0, vbase, busy);
+  };
+  auto end = [&] {
+    const int vbase = (int)m0 + wave * 32;  // this wave's first row
+    pass(acc, m0, vbase, vbase < vend);
+    m0 += S::BM;
+  };
+  constexpr std::integral_constant<int, 0> zero{};
+  constexpr std::integral_constant<int, DEPTH / 2> half{};
+  constexpr std::integral_constant<int, DEPTH> whole{};
+  while (m0 < vend64) {
+    begin();
+    for (int k0 = 0; k0 < (HALF ? n_k - DEPTH / 2 : n_kp); k0 += DEPTH) stages(zero, whole);
+    if constexpr (HALF) stages(zero, half);
+    end();
+    if constexpr (HALF) {
+      if (m0 >= vend64) break;
+      begin();
+      stages(half, whole);
+      for (int k0 = DEPTH / 2; k0 < n_k; k0 += DEPTH) stages(zero, whole);
+      end();
+    }
   }
 }
 
 // Forward.  AUX: cache policy of the loads of W
-template <typename TIN, int NT, int AUX>
+template <typename TIN, int NT, int AUX, bool HALF>
 LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
   typedef FewFwdShape<TIN, NT> S;
   constexpr int FN = S::FN, HL = S::HROWS / 64;
@@ -180,7 +207,7 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
   uint32_t h_off[HL];
 #pragma unroll
   for (int i = 0; i < HL; ++i) h_off[i] = (uint32_t)((tid >> 3) + 64 * i) * h_row + (tid & 7) * 16;
-  few_products<TIN, NT, AUX>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * h_row, h_off, lds,
+  few_products<TIN, NT, AUX, HALF>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * h_row, h_off, lds,
                              [&](f32x16_t (&acc)[1][FN], int64_t m0, int vbase, bool) {
     if constexpr (sizeof(TIN) == 2) if (p.xcache) {
       // the logits of this pass, for a backward that then has no need to recompute them.  A 32x32 block passes through 4 KB of
@@ -234,11 +261,11 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
 }
 
 // (which rows are read how: read_w_once, lce_host.hpp.  A branch around the whole body: none around a load.)
-template <typename TIN, int NT>
+template <typename TIN, int NT, bool HALF>
 __global__ __launch_bounds__(512, 2) void lce_fwd_few_kernel(FwdArgs<TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  if ((int64_t)blockIdx.x * p.split_stride < p.once_rows) fwd_few_body<TIN, NT, kBufNonTemporal>(p, lds);
-  else fwd_few_body<TIN, NT, 0>(p, lds);
+  if ((int64_t)blockIdx.x * p.split_stride < p.once_rows) fwd_few_body<TIN, NT, kBufNonTemporal, HALF>(p, lds);
+  else fwd_few_body<TIN, NT, 0, HALF>(p, lds);
 }
 
 template <typename TIN>

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(512, 2) void lce_ds_few_f32_kernel(FewF32Args p) {
     k[j] = p.tokc[j * 32 + ln];
     lab[j] = p.tokl[j * 32 + ln] - (int)p.lab0;
   }
-  few_products<float, NT, kBufNonTemporal>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * p.ldh * 4, h_off, lds,
+  few_products<float, NT, kBufNonTemporal, false>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * p.ldh * 4, h_off, lds,
                                            [&](f32x16_t (&acc)[1][FN], int64_t, int vbase, bool busy) {
     if (!busy) return;
 #pragma unroll

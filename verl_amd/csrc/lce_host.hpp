@@ -433,7 +433,9 @@ int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int6
   {
     ProfScope prof(PC_FWD, st);
     typedef FewFwdShape<TIN, NT> Shape;
-    auto kern = lce_fwd_few_kernel<TIN, NT>;
+    constexpr bool kHalves = sizeof(TIN) == 2;
+    const bool half = (H / Shape::BK) % Shape::DEPTH == Shape::DEPTH / 2;
+    auto kern = kHalves && half ? lce_fwd_few_kernel<TIN, NT, kHalves> : lce_fwd_few_kernel<TIN, NT, false>;
     allow_lds(kern, Shape::LDS_BYTES);
     hipLaunchKernelGGL(kern, dim3((unsigned)S), dim3(512), Shape::LDS_BYTES, st, p);
     int rc = check_launch("lce_fwd_few_kernel");
