@@ -16,6 +16,10 @@ DEV = "cuda:0"
     (17, 640, 65537),     # rows of a second pass in some workgroups
     (64, 896, 140001),    # three passes, the last one short
     (33, 256, 140001),    # whole turns
+    (65, 384, 90001),     # three blocks of 32 tokens from here on
+    (96, 512, 140001),
+    (80, 896, 20011),
+    (97, 384, 90001),     # the 256 x 128 tile
 ])
 def test_passes(T, H, V, dtype):
     from verl_amd.utils.kernel import kernels

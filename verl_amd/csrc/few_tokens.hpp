@@ -54,17 +54,19 @@ LCE_DEV void mma16(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
 LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Forward, up to 64 tokens.  Workgroup = 512 threads = 8 waves, one per CU; it owns a contiguous range of vocabulary rows (the
+// Forward, up to 96 tokens (NT: 64 or 96).  Workgroup = 512 threads = 8 waves, one per CU; it owns a contiguous range of vocabulary rows (the
 // same number for every workgroup) and goes through it in passes of 256 rows, for each of which K is streamed in stages of 64:
-// 256 rows of W x 128 bytes and 64 rows of hidden x 128 bytes.  What bounds it is the read of W, and that by the bytes in
+// 256 rows of W x 128 bytes and 64 or 128 rows of hidden x 128 bytes.  What bounds it is the read of W, and that by the bytes in
 // flight: DEPTH stages are on their way in registers (128 KB of W per CU) while one is multiplied out of LDS, which holds two,
 // so that a stage costs one barrier; and the stages of the next pass follow those of this one without a gap.
 // The products are those of the d_logits tiles, 32x32x16 blocks with k ascending (rows: vocabulary, columns: tokens), so logits
-// kept here have the bits that a backward without them recomputes.  A wave owns 32 rows x 64 tokens; in a short last pass the
+// kept here have the bits that a backward without them recomputes.  A wave owns 32 rows x NT tokens; in a short last pass the
 // waves without rows stand aside (64 tokens: 182 -> 174 us).
 // Measured, kernel and merge, against the 256 x 64 tile with a ring of whole LDS stages (H, V: before -> after): 64 tokens,
 // 3584, 152064: 184 -> 174 us; 4096, 128256: 175 -> 160; 896, 151936: 58 -> 51.5; the same access pattern without any
-// arithmetic takes 170, 163 and 41.  (128 tokens on 64 x 64 wave tiles: 223 us, the 256 x 128 tile takes 213.)
+// arithmetic takes 170, 163 and 41.  65 / 80 / 96 tokens against the 256 x 128 tile: 3584: 198 / 202 / 204 -> 186 / 193 / 197 us, 5120:
+// 283 / 288 / 293 -> 266 / 276 / 285, 4096: 172 / 172 / 173 -> 166 / 172 / 173, 896: 57 / 57 / 57.5 -> 56; forward + backward 3584: 635 /
+// 651 / 667 -> 622 / 639 / 655, 4096: 575 / 578 / 584 -> 560 / 567 / 577.  (97 to 128 tokens so: 206 / 211 -> 224 / 230, the tile stays.)
 // fp32 inputs run it up to 128 tokens, on the fp32 MFMA, which is the bound from some 40 tokens on (64 tokens, 1.09 G products of W's
 // elements: 445 us at its peak rate): the narrowest of 32, 64, 96 and 128 tokens that holds them.  Against the 256 x 64 and 256 x 128
 // tiles, H=3584: 1 to 32 tokens 750 -> 440 us, 64: 746 -> 673, 65 to 96: 1335 -> 936, 128: 1335 -> 1220; H=896: 202 -> 113, 202 -> 188,

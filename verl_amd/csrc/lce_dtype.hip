@@ -50,6 +50,7 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
 #if LCE_TU_DTYPE != 1
     case kSelT64: LCE_FEW(64);
     case kSelT128:
+      if (T <= 96) LCE_FEW(96);
       if (!read_w_once(V, ldw * (int64_t)sizeof(TuT), xcache)) LCE_RUN(VariantT128Plain);
       LCE_RUN(VariantT128);
 #else

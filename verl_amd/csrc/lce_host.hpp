@@ -365,7 +365,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
   int S = Cfg::BN > 128 ? forward_splits_256(ntt, nvt, max_splits) : bc * ((8 + nrb - 1) / nrb);
   if (S > nvt) S = nvt;
   if (S > max_splits) S = max_splits;
-  // The narrow token tiles serve the HBM-bound case (up to 128 tokens: one streaming read of W; 16-bit inputs of up to 64
+  // The narrow token tiles serve the HBM-bound case (up to 128 tokens: one streaming read of W; 16-bit inputs of up to 96
   // tokens have a kernel of their own, forward_few).  There each
   // split takes one contiguous range of rows, the same length for all, instead of whole tiles dealt round robin
   // (594 tiles over 256 splits would be 3 against 2, and a split's tiles would lie 256 tiles apart).  Measured
@@ -413,7 +413,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
                        entropy_b, shard_out, st);
 }
 
-// forward with at most 64 tokens of 16 bits or 128 of fp32 (few_tokens.hpp): one contiguous range of rows per workgroup, one
+// forward with at most 96 tokens of 16 bits or 128 of fp32 (few_tokens.hpp): one contiguous range of rows per workgroup, one
 // workgroup per CU; whole panels of the kept logits
 template <typename TIN, int NT>
 int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
@@ -428,7 +428,7 @@ int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int6
   p.parts = reinterpret_cast<f32x4_t*>(ws);
   p.xlabel = reinterpret_cast<float*>(ws + align256((size_t)S * T * 16));
   p.S = S; p.tile_step = 256; p.label_offset = label_offset; p.xcache = xcache; p.w_plane = p.h_plane = 0;
-  p.once_rows = read_w_once(V, ldw * (int64_t)sizeof(TIN), xcache) ? V : V - kMallBytes / 4 / (ldw * (int64_t)sizeof(TIN));
+  p.once_rows = read_w_once(V, ldw * (int64_t)sizeof(TIN), xcache) ? V : T > 64 ? 0 : V - kMallBytes / 4 / (ldw * (int64_t)sizeof(TIN));
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   {
     ProfScope prof(PC_FWD, st);

@@ -57,7 +57,7 @@ struct FwdArgs {
   // temperature) are kept for the backward: logit (t, v) at kept_logit(xcache, T, t, v).
   float* xcache;
   int64_t w_plane, h_plane;  // W and h in bfloat16 planes (GemmCfg16, TERMS == 6): bytes from plane to plane
-  int64_t once_rows;  // up to 64 tokens: workgroups whose rows start before this one read W with non-temporal loads
+  int64_t once_rows;  // up to 96 tokens: workgroups whose rows start before this one read W with non-temporal loads
 };
 
 // Kept logits lie in panels of 16 vocabulary rows, [panel][token][16] fp32: what one 16 x 16 block of a tile holds is one
