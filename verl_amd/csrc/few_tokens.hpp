@@ -623,7 +623,8 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 // columns [64 b, 64 b + 64) of dS, which lie within one group of the vocabulary order Perm (a whole group of the
 // eight-wave tiles' order, half a group of the 16x16x32 tiles'), and the first `nrows` compact token positions, of which it
 // writes as many as a reader takes: up to the tokens that take part, rounded up to the d_weight product's K granule (64, and
-// two slabs at least).  Positions beyond the tokens and columns beyond the chunk's rows (the grid covers whole 256-row
+// two slabs at least) for the tiles, and `exact`ly those for the streaming kernels, which read zeros behind them (1 / 8 / 24 tokens,
+// H=3584: step 559 / 569 / 580 -> 551 / 563 / 577 us, H=4096 528 / 538 / 550 -> 523 / 534 / 548; from 40 on level).  Positions beyond the tokens and columns beyond the chunk's rows (the grid covers whole 256-row
 // tiles) are written as zeros, as the tiles write them.  Eight lanes share a position: they read the 256 bytes of its
 // token's logits behind the 64 columns and write 128 bytes of dS.  Bound by HBM; the constants come from the per-position
 // table (worked out per workgroup they were six dependent loads and a logarithm per position) and four positions are on
@@ -632,14 +633,14 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 // on (a multiple of 16), of xtok tokens.
 // ------------------------------------------------------------------------------------------------------------------
 template <typename TIN, typename Perm>
-__global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t xtok, int nrows) {
+__global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t xtok, int nrows, bool exact) {
   static_assert(sizeof(TIN) == 2 && Perm::GV % 64 == 0, "16-bit d_logits, groups of the vocabulary order in multiples of 64 rows");
   constexpr int U = 4;
   const int tid = threadIdx.x, c = tid & 7;
   const int64_t u0 = (int64_t)blockIdx.x * 64;   // first of this workgroup's 64 columns of dS
   const int64_t g0 = u0 - u0 % Perm::GV;         // first row (= first column) of their group of the vocabulary order
   const int Tc = (int)(p.n_rows ? (int64_t)*p.n_rows : p.T);
-  const int used = Tc <= 64 ? 128 : (Tc + 63) / 64 * 64, end = used < nrows ? used : nrows;
+  const int used = exact ? Tc : Tc <= 64 ? 128 : (Tc + 63) / 64 * 64, end = used < nrows ? used : nrows;
   // columns c * 8 + (0..3) and c * 8 + (4..7) of the workgroup's 64 are two runs of four consecutive vocabulary rows
   // (both orders Perm keep what one lane of a d_logits tile holds together: four consecutive rows per register quad),
   // and the cache is padded to whole groups, so each run is one aligned 16-byte load

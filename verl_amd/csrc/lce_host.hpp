@@ -989,14 +989,14 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     if constexpr (sizeof(TIN) == 2 && Cfg::BM == 256) {
       if (xcache && L.tn && p.n_ds > 0) {
         // d_logits of this chunk from the logits the forward kept: no pass over W, no T x V x H product
-        const int nrows = L.few ? ((int)(T <= 64 ? 64 : 128) < (int)L.tpad ? (int)(T <= 64 ? 64 : 128) : (int)L.tpad) : (int)L.tpad;
+        const int nrows = L.few ? (int)T : (int)L.tpad;
         const int64_t c0 = p.ds.v0 - vocab_offset;  // the chunk's first row of W
         {
           ProfScope prof(PC_BWD_DS, st);
           DsArgs<TIN> dq = p.ds;
           dq.rows = rows;  // (the 16x16x32 tiles read the compact copy of hidden and no list; the cache is indexed by token)
           hipLaunchKernelGGL((ds_from_logits_kernel<TIN, KPerm<Cfg>>), dim3((unsigned)(round_up(p.ds.vrows, 256) / 64)), dim3(256), 0, st, dq,
-                             xcache + c0 * T, T, nrows);
+                             xcache + c0 * T, T, nrows, L.few);
           if ((rc = check_launch("ds_from_logits_kernel"))) return rc;
         }
         p.n_ds = 0;  // (what is left for the launch below: the gradient GEMMs of the previous chunk)
