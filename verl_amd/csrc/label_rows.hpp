@@ -338,7 +338,7 @@ __global__ __launch_bounds__(256) void token_prep_kernel(CoefArgs<T> a, LabelTer
 // lce_dh16_kernel has worked out from the same count of rows).  Workgroup n_dh + i: compact position
 // i of the token list; the first position of each label adds sum of G_t * hidden[t][:] over the positions with that
 // label, in order, to the label's row of d_weight (as dw_label_rows_kernel does over a sorted run).
-template <typename T, typename TOUT>
+template <typename T, typename TOUT, bool DEEP>
 __global__ __launch_bounds__(256) void token_finish_kernel(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H,
                                                            TOUT* d_hidden, LabelTerm lt, const T* W, int64_t ldw, int n_dh, const int* rows,
                                                            const int* n_rows, const uint32_t* keys, const T* h, int64_t ldh, TOUT* dW,
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void token_finish_kernel(const float* part, in
       S = by_rows.count(rows_n);
       stride = DhSlices::stride(rows_n, H);
     }
-    dh_finish_body<T, TOUT>(part, S, stride, inv, ntok, H, d_hidden, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)n_dh);
+    dh_finish_body<T, TOUT, DEEP>(part, S, stride, inv, ntok, H, d_hidden, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)n_dh);
     return;
   }
   constexpr int N = 16 / (int)sizeof(T);

@@ -128,8 +128,9 @@ int backward_few_f32(const float* h, int64_t ldh, const float* W, int64_t ldw, c
   ProfScope prof(PC_DH_FINISH, st);
   LabelTerm lt;
   lt.labels = nullptr; lt.v0 = vocab_offset; lt.V = V; lt.g_lp = dlogprobs; lt.g_stride = g_stride; lt.scale = 0.f;
-  hipLaunchKernelGGL((dh_finish_kernel<float, float>), dim3((unsigned)((T * (H / 4) + 255) / 256)), dim3(256), 0, st, q.dHp, L.ksplit, part_stride, inv, T,
-                     H, d_hidden, lt, W, ldw);
+  const int64_t blocks = (T * (H / 4) + 255) / 256;
+  auto finish = dh_sum_deep(L.ksplit, blocks) ? dh_finish_kernel<float, float, true> : dh_finish_kernel<float, float, false>;
+  hipLaunchKernelGGL(finish, dim3((unsigned)blocks), dim3(256), 0, st, q.dHp, L.ksplit, part_stride, inv, T, H, d_hidden, lt, W, ldw);
   return check_launch("dh_finish_kernel");
 }
 #endif

@@ -509,6 +509,11 @@ int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cos
   return best;
 }
 
+// Is the sum of the partials a chain of loads (dh_finish_body, DEEP)?  Many slices and few workgroups to hide it; either way, us: 100
+// tokens of H=3584 (18 slices, 350 workgroups) 10.6 / 8.6, 300 of 896 (32, 262) 15.5 / 11.5, 600 of 896 (21, 525) 17.0 / 14.9; 200 of 3584 (18,
+// 700) 12.6 / 15.0, 1000 of 896 (16, 875) 10.3 / 14.0, 333 of 3584 (9, 1165) 13.0 / 15.7, 1000 of 3584 37 / 44.
+bool dh_sum_deep(int slices, int64_t workgroups) { return slices > 8 && 2 * workgroups <= 5 * kNumCUs; }
+
 // The same choice for every number of row tiles that may turn out to take part, within the memory that `ksplit` partials of all
 // T rows have.  Forward + backward in us, slices counted for all tokens / this way: H=4096, V=128256, 1000 tokens, about 500 with
 // gradient 1646 / 1341, about 250: 1931 / 1761, 2000 tokens 3263 / 2555, 400: 1083 / 1029; H=5120 1500 tokens 4016 / 3346; level
@@ -1025,11 +1030,14 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
       const int n_lr = (L.sort_items && need_dw) ? (int)T : 0;
       const int64_t part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
       if (n_dh + n_lr > 0) {
+        const bool deep = dh_sum_deep(L.ksplit, dh_blocks);
+        auto finish_f32 = deep ? token_finish_kernel<TIN, float, true> : token_finish_kernel<TIN, float, false>;
+        auto finish = deep ? token_finish_kernel<TIN, TIN, true> : token_finish_kernel<TIN, TIN, false>;
         if (grads_f32)
-          hipLaunchKernelGGL((token_finish_kernel<TIN, float>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
+          hipLaunchKernelGGL(finish_f32, dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
                              T, H, static_cast<float*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<float*>(d_weight), by_rows);
         else
-          hipLaunchKernelGGL((token_finish_kernel<TIN, TIN>), dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
+          hipLaunchKernelGGL(finish, dim3((unsigned)(n_dh + n_lr)), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv,
                              T, H, static_cast<TIN*>(d_hidden), lt, W, ldw, n_dh, rows, n_rows, skeys[0], h, ldh, static_cast<TIN*>(d_weight), by_rows);
         if ((rc = check_launch("token_finish_kernel"))) return rc;
       }
@@ -1068,10 +1076,10 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
     if (blocks > 8192) blocks = 8192;
     const int64_t part_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
     if (grads_f32)
-      hipLaunchKernelGGL((dh_finish_kernel<TIN, float>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv, T, H,
+      hipLaunchKernelGGL((dh_finish_kernel<TIN, float, false>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv, T, H,
                          static_cast<float*>(d_hidden), lt, W, ldw);
     else
-      hipLaunchKernelGGL((dh_finish_kernel<TIN, TIN>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv, T, H,
+      hipLaunchKernelGGL((dh_finish_kernel<TIN, TIN, false>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit, part_stride, inv, T, H,
                          static_cast<TIN*>(d_hidden), lt, W, ldw);
     if ((rc = check_launch("dh_finish_kernel"))) return rc;
   }

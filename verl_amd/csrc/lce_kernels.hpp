@@ -991,11 +991,11 @@ struct LabelTerm {
 // without `inv`), or zeros where inv[t] < 0 (token without upstream gradient).  The sum runs in the
 // fixed order s = 0, 1, ..., so the result does not depend on scheduling.  H a multiple of 4.
 // With a label term, G_t * W[label_t][:] is added in fp32 before the one rounding.
-// Up to 64 slices, with a workgroup or less to a CU where there are few tokens: what bounds it is the chain of loads, so 16 of
-// them are in flight at a time (8 tokens of H=896, 64 slices: 19 us as the compiler had it, now 6 to 8; 128 tokens: 20, now 8.5; one column
-// per thread in place of four, for more workgroups, is no faster).
+// DEEP (dh_sum_deep): few tokens, so a workgroup or two to a CU, and up to 64 slices: what bounds it is the chain of loads, so 16 of
+// them are in flight at a time (8 tokens of H=896, 64 slices: 19 us, now 7; one column per thread in place of four, for more
+// workgroups, is no faster).  With many workgroups the registers cost more than the loads gain: 4096 tokens of H=4096 20 -> 27 us.
 // (bid of nblocks workgroups: the kernel's own grid, or the part of a larger grid that does this work)
-template <typename T, typename TOUT>
+template <typename T, typename TOUT, bool DEEP>
 LCE_DEV void dh_finish_body(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H, TOUT* out,
                             const LabelTerm& lt, const T* W, int64_t ldw, int64_t bid, int64_t nblocks) {
   const int64_t per_row = H / 4, n = ntok * per_row;
@@ -1007,14 +1007,14 @@ LCE_DEV void dh_finish_body(const float* part, int S, int64_t stride, const int*
       const float* src = part + pos * H + c;
       a = *reinterpret_cast<const f32x4_t*>(src);
       int s = 1;
-      for (; s + 16 <= S; s += 16) {
+      for (; DEEP && s + 16 <= S; s += 16) {
         f32x4_t b[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) b[i] = *reinterpret_cast<const f32x4_t*>(src + (s + i) * stride);
 #pragma unroll
         for (int i = 0; i < 16; ++i) a += b[i];
       }
-      for (; s + 4 <= S; s += 4) {
+      for (; DEEP && s + 4 <= S; s += 4) {
         f32x4_t b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) b[i] = *reinterpret_cast<const f32x4_t*>(src + (s + i) * stride);
@@ -1038,10 +1038,10 @@ LCE_DEV void dh_finish_body(const float* part, int S, int64_t stride, const int*
   }
 }
 
-template <typename T, typename TOUT>
+template <typename T, typename TOUT, bool DEEP>
 __global__ void dh_finish_kernel(const float* part, int S, int64_t stride, const int* inv, int64_t ntok, int64_t H, TOUT* out,
                                  LabelTerm lt, const T* W, int64_t ldw) {
-  dh_finish_body<T, TOUT>(part, S, stride, inv, ntok, H, out, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)gridDim.x);
+  dh_finish_body<T, TOUT, DEEP>(part, S, stride, inv, ntok, H, out, lt, W, ldw, (int64_t)blockIdx.x, (int64_t)gridDim.x);
 }
 
 // Tokens whose upstream gradients are both zero add nothing to either gradient.  The others are listed in order:

@@ -263,7 +263,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
     lt.labels = nullptr; lt.v0 = vocab_offset; lt.V = V; lt.g_lp = dlogprobs; lt.g_stride = g_stride; lt.scale = 0.f;
     int64_t blocks = (T * (H / 4) + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL((dh_finish_kernel<float, float>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit,
+    hipLaunchKernelGGL((dh_finish_kernel<float, float, false>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit,
                        (int64_t)(align256((size_t)T * H * 4) / 4), inv, T, H, d_hidden, lt, W, ldw);
     if ((rc = check_launch("dh_finish_kernel"))) return rc;
   }
