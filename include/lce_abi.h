@@ -334,9 +334,9 @@ int lce_num_variants(void);
  * which an XCD's consecutive blocks of d_logits tiles walk the chunk: -1 = chosen by size (default), 0 = along the
  * vocabulary, 1 = along the tokens.  LCE_OPT_DHIDDEN_KSPLIT (default 0 = by shape): K slices of the d_hidden GEMM, each
  * with its own fp32 partial that is summed in a fixed order afterwards (0..16; changes the workspace size).
- * LCE_OPT_FEW_TOKEN_GEMMS (default 1, 16-bit inputs): with at most 128 tokens both gradient GEMMs of the backward run
- * as one launch of streaming kernels; 0 = the 256 x 256 tile kernels, which the tests compare them with (changes the
- * workspace size). */
+ * LCE_OPT_FEW_TOKEN_GEMMS (default 1): with at most 128 tokens the gradient GEMMs of the backward, and with fp32 inputs
+ * its d_logits too, run as streaming kernels; 0 = the 256 x 256 tile kernels, which the tests compare them with (changes
+ * the workspace size). */
 enum {
   LCE_OPT_SPLIT_BACKWARD_LAUNCHES = 1,
   LCE_OPT_DLOGITS_TOKENS_FIRST = 2,
