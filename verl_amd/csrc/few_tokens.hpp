@@ -63,7 +63,7 @@ LCE_DEV int fw_swz(int r) { return ((r & 3) << 2) ^ ((r >> 3) & 3); }
 // kept here have the bits that a backward without them recomputes.  A wave owns 32 rows x NT tokens; in a short last pass the
 // waves without rows stand aside (64 tokens: 182 -> 174 us).
 // Measured, kernel and merge, against the 256 x 64 tile with a ring of whole LDS stages (H, V: before -> after): 64 tokens,
-// 3584, 152064: 184 -> 174 us; 4096, 128256: 175 -> 160; 896, 151936: 58 -> 51.5; the same access pattern without any
+// 3584, 152064: 184 -> 174 us; 4096, 128256: 175 -> 160; 896, 151936: 58 -> 50; the same access pattern without any
 // arithmetic takes 170, 163 and 41.  65 / 80 / 96 tokens against the 256 x 128 tile: 3584: 198 / 202 / 204 -> 186 / 193 / 197 us, 5120:
 // 283 / 288 / 293 -> 266 / 276 / 285, 4096: 172 / 172 / 173 -> 166 / 172 / 173, 896: 57 / 57 / 57.5 -> 56; forward + backward 3584: 635 /
 // 651 / 667 -> 622 / 639 / 655, 4096: 575 / 578 / 584 -> 560 / 567 / 577.  (97 to 128 tokens so: 206 / 211 -> 224 / 230, the tile stays.)
@@ -624,7 +624,8 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 // eight-wave tiles' order, half a group of the 16x16x32 tiles'), and the first `nrows` compact token positions, of which it
 // writes as many as a reader takes: up to the tokens that take part, rounded up to the d_weight product's K granule (64, and
 // two slabs at least) for the tiles, and `exact`ly those for the streaming kernels, which read zeros behind them (1 / 8 / 24 tokens,
-// H=3584: step 559 / 569 / 580 -> 551 / 563 / 577 us, H=4096 528 / 538 / 550 -> 523 / 534 / 548; from 40 on level).  Positions beyond the tokens and columns beyond the chunk's rows (the grid covers whole 256-row
+// H=3584: step 559 / 569 / 580 -> 551 / 563 / 577 us, H=4096 528 / 538 / 550 -> 523 / 534 / 548; from 40 on level).
+// Positions beyond the tokens and columns beyond the chunk's rows (the grid covers whole 256-row
 // tiles) are written as zeros, as the tiles write them.  Eight lanes share a position: they read the 256 bytes of its
 // token's logits behind the 64 columns and write 128 bytes of dS.  Bound by HBM; the constants come from the per-position
 // table (worked out per workgroup they were six dependent loads and a logarithm per position) and four positions are on
