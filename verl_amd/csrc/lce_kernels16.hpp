@@ -167,9 +167,13 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
       if constexpr (KEEP) {
         // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.  Issued AHEAD of the next
         // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
-        // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are
-        // issued 16 at a time and so many are waited for that, with the prologue's 32 loads behind them, fewer than 64
-        // operations are ever in flight.  Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
+        // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are issued two
+        // block columns at a time, and behind the last column, whichever it is, so many are waited for that with the
+        // prologue's loads behind them fewer than 64 operations are ever in flight (8 stores a column, 12 where the compiler gives
+        // lanes without a token a store of their own; tests/test_ring_loads_on_cpu.py counts them on the listing).
+        // Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
+        constexpr int kColumn = NB + NB / 2, kBehindLast = 24, kBetween = 32;
+        static_assert(kBetween + 2 * kColumn < 64 && 4 * kColumn < 64 && kBehindLast + 2 * (Cfg::HL + Cfg::HLB) < 64, "vmcnt range");
         const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
         // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
         const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
@@ -183,10 +187,10 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
             const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, kBufNonTemporal);
           }
-          if (j % 2 == 1 && j >= 3) {
+          if (j == NBN - 1 || (j % 2 == 1 && j >= 3)) {
             __builtin_amdgcn_sched_barrier(0);
-            if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<24>();
-            else GemmCore16<Cfg>::template wait_vm<32>();
+            if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<kBehindLast>();
+            else GemmCore16<Cfg>::template wait_vm<kBetween>();
           }
         }
         __builtin_amdgcn_sched_barrier(0);
