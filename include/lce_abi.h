@@ -29,8 +29,11 @@ extern "C" {
  * same).  For lce_forward,
  * lce_forward_keep_logits, lce_forward_shard and the lce_backward functions: a backward must be given the code of the
  * forward that its statistics come from, because the rounding errors of the logits that it recomputes cancel against those
- * of the statistics.  The planes want the whole workspace that the size queries answer (they answer alike for both codes);
- * with LCE_DTYPE_F32 what the fp32 MFMA needs is enough.  Every other entry point takes the first three codes. */
+ * of the statistics.  lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES the workspace the forward is fastest with
+ * (planes of at most 256 MB of the weight, or two fifths of its own bytes where that is more, next to those of hidden) and for
+ * LCE_DTYPE_F32 the least that is enough for either code; a forward on the planes is served with any size from there on, with
+ * the same results.  The backward's query answers what the code asked for needs (for LCE_DTYPE_F32: either code).  The fp32 MFMA
+ * itself needs what LCE_DTYPE_BF16 is answered in the forward.  Every other entry point takes the first three codes. */
 enum { LCE_DTYPE_BF16 = 0, LCE_DTYPE_F32 = 1, LCE_DTYPE_F16 = 2, LCE_DTYPE_F32_PLANES = 3 };
 enum { LCE_REDUCTION_NONE = 0, LCE_REDUCTION_SUM = 1, LCE_REDUCTION_MEAN = 2 }; /* verl/utils/kernel/kernels.py:102-126 */
 enum {
@@ -288,7 +291,8 @@ int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
  * d_logits buffer stays within 256 MiB): a byte count; lce_backward_workspace_bytes with vocab_chunk <= 0 then
  * returns the workspace of the widest chunk that fits it (never below 2048 columns, never above the bound
  * 0.25 * T * V * esz + 4 * V * H), and lce_backward with vocab_chunk <= 0 uses that chunk.  An explicit vocab_chunk
- * is not touched.  Takes the role of the reference's fixed vocab_per_split = 9504 (verl/utils/kernel/kernels.py:1666-1670).
+ * is not touched.  What lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES stays within it too, down to the least
+ * that is enough.  Takes the role of the reference's fixed vocab_per_split = 9504 (verl/utils/kernel/kernels.py:1666-1670).
  * LCE_OPT_LABEL_TERM_OUTSIDE (default 2, 16-bit inputs only) chooses the data format of the gradient of the logits:
  * 0 = the label's entry is rounded to 16 bits with the rest of the d_logits tile, which is the reference's format
  * (verl/utils/kernel/kernels.py:1666-1724); 1 = its one-hot part g_logprob / temperature * 1[v == label] is added to

@@ -199,11 +199,14 @@ static size_t forward_workspace_need(int64_t T, int64_t V, int max_splits) {
   return align256((size_t)forward_splits_upper_bound(T, V > 0 ? V : 1, max_splits) * (size_t)T * 16) + 2 * align256((size_t)T * 4);
 }
 
-// (answered for LCE_DTYPE_F32: enough for either code of fp32)
+// (answered for LCE_DTYPE_F32: the least that is enough for either code of fp32)
 size_t lce_forward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
   const size_t need = forward_workspace_need(T, V, kMaxSplits);
-  if (T <= 0 || H <= 0 || V <= 0 || (dtype != LCE_DTYPE_F32 && dtype != LCE_DTYPE_F32_PLANES) || !use_terms(tuning_snapshot(), T, H, V)) return need;
-  return dtype == LCE_DTYPE_F32 ? std::max(need, terms_fwd_plan(T, H, V).total) : terms_fwd_plan(T, H, V).total;
+  if (T <= 0 || H <= 0 || V <= 0 || (dtype != LCE_DTYPE_F32 && dtype != LCE_DTYPE_F32_PLANES)) return need;
+  const Tuning tu = tuning_snapshot();
+  if (!use_terms(tu, T, H, V)) return need;
+  if (dtype == LCE_DTYPE_F32) return std::max(need, terms_fwd_plan(T, H, V, 0).total);
+  return terms_fwd_plan(T, H, V, tu.ws_budget > 0 ? (size_t)tu.ws_budget : SIZE_MAX).total;
 }
 
 // shared body of lce_forward and lce_forward_shard
@@ -226,7 +229,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   if (!shard_out && (!logprobs || !entropy || !maximum || !accumulate || !entropy_b)) return fail(LCE_E_ARG, "null output pointer");
   const Tuning tu = tuning_snapshot();
   const bool terms = planes && use_terms(tu, T, H, V);
-  const size_t need = terms ? terms_fwd_plan(T, H, V).total : forward_workspace_need(T, V, max_splits);
+  const size_t need = terms ? terms_fwd_plan(T, H, V, 0).total : forward_workspace_need(T, V, max_splits);
   if (!workspace || workspace_bytes < need) return fail(LCE_E_WORKSPACE, "forward workspace too small: %zu < %zu", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
   int sel = tu.variant_fwd;
@@ -246,7 +249,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
-                         accumulate, entropy_b, ws, st, label_offset, shard_out, max_splits, xcache);
+                         accumulate, entropy_b, ws, workspace_bytes, st, label_offset, shard_out, max_splits, xcache);
 }
 
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype) {

@@ -61,8 +61,8 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
       if (T <= 96) LCE_FEW(96);
       LCE_FEW(128);
     case kSelTerms:
-      return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws, st,
-                           label_offset, shard_out);
+      return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws,
+                           ws_bytes, st, label_offset, shard_out);
 #endif
   }
 #undef LCE_FEW

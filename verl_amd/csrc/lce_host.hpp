@@ -70,8 +70,8 @@ enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8, k
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
 #define LCE_FWD_PARAMS                                                                                                      \
   const void *h, int64_t ldh, const void *W, int64_t ldw, const int64_t *labels, int64_t T, int64_t H, int64_t V,          \
-      float temperature, int reduction, float *lp, float *ent, float *mx, float *ac, float *eb, char *ws, hipStream_t st,   \
-      int64_t label_offset, float *shard_out, int max_splits, float *xcache
+      float temperature, int reduction, float *lp, float *ent, float *mx, float *ac, float *eb, char *ws, size_t ws_bytes,  \
+      hipStream_t st, int64_t label_offset, float *shard_out, int max_splits, float *xcache
 #define LCE_BWD_PARAMS                                                                                                      \
   const void *h, int64_t ldh, const void *W, int64_t ldw, const int64_t *labels, int64_t T, int64_t H, int64_t V,          \
       float temperature, int reduction, const float *mx, const float *ac, const float *eb, const float *glp,               \

@@ -21,22 +21,14 @@ struct TermsFwdPlan {
 
 int terms_fwd_splits(int ntt, int64_t rows) { return forward_splits_256(ntt, (int)((rows + 255) / 256)); }
 
-TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V) {
+TermsFwdPlan terms_fwd_plan_for(int64_t T, int64_t H, int64_t V, int64_t tiles) {  // tiles: of 256 vocabulary rows, in a chunk
   TermsFwdPlan p;
   const int ntt = (int)((T + 255) / 256);
-  // whole rounds of tiles over the CUs: as many as 256 MB of planes allow, which the memory-side cache then holds from the split to
-  // the product, but one at least, through memory or not (forward in us, chunks of 256 MB / one round: H=3584, 300 tokens 5698 /
-  // 3392, 1000: 6278 / 5528; H=5120, 300: 10600 / 4902, 1000: 10882 / 8064)
-  const int64_t most = ((int64_t)256 << 20) / (6 * H * 256);  // tiles of a chunk
-  const int64_t rounds = std::max<int64_t>(1, most * ntt / kNumCUs);
-  const int64_t tiles = std::max<int64_t>(1, rounds * kNumCUs / ntt);
   p.rows = tiles * 256;
   p.nchunks = (int)((V + p.rows - 1) / p.rows);
-  p.splits = 0;
-  for (int c = 0; c < p.nchunks; ++c) {
-    const int64_t rows = std::min<int64_t>(p.rows, V - c * p.rows);
-    p.splits += std::min<int>(terms_fwd_splits(ntt, rows), (int)((rows + 255) / 256));
-  }
+  auto splits = [&](int64_t rows) { return std::min<int>(terms_fwd_splits(ntt, rows), (int)((rows + 255) / 256)); };
+  p.splits = splits(V - (p.nchunks - 1) * p.rows);
+  if (p.nchunks > 1) p.splits += (p.nchunks - 1) * splits(p.rows);
   size_t o = align256((size_t)p.splits * T * 16);
   p.off_xlabel = o; o += align256((size_t)T * 4);
   p.off_lp = o;     o += align256((size_t)T * 4);
@@ -45,6 +37,29 @@ TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V) {
   p.off_w = o;      o += align256((size_t)std::min<int64_t>(p.rows, round_up(V, 64)) * 3 * H * 2);
   p.total = o;
   return p;
+}
+
+// The widest chunks that a workspace of `room` bytes has space for, between two bounds that are of shapes alone.  The lower
+// one, whose workspace is always enough: 256 MB of planes, which the memory-side cache holds from the split to the product, in
+// whole rounds of tiles over the CUs.  Where they hold less than a round (few tokens, a wide weight) the upper one is a round,
+// through memory, but at most two fifths of the weight's own bytes.  The same bits whatever the width: a tile is a split of
+// its own there.  Forward in us by MiB of workspace, H=5120, V=152064: 256 tokens 257: 10684, 610: 5654, 906: 4166, 1127: 3697
+// (taken), 1495: 3325; 300 tokens 260: 10478, 611: 5534, 905: 4391 (taken, a round); 1000 tokens 287: 10632, 489: 7728 (taken, a
+// round); H=4096, V=128256: 256 tokens 260: 5987, 764: 2749 (taken), 1514: 2135; 300 tokens 262: 5869, 616: 3172, 766: 2962 (taken).
+TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V, size_t room) {
+  const int64_t ntt = (T + 255) / 256, nvt = (V + 255) / 256, tile_bytes = 6 * H * 256;
+  const int64_t base = std::max<int64_t>(1, ((int64_t)256 << 20) / tile_bytes);  // tiles of a chunk
+  const int64_t rounds = base * ntt / kNumCUs;
+  if (rounds > 0) return terms_fwd_plan_for(T, H, V, std::max<int64_t>(1, rounds * kNumCUs / ntt));
+  const int64_t share = V * H * 4 * 2 / 5 / tile_bytes;
+  const int64_t most = std::max(base, std::min<int64_t>(kNumCUs / ntt, share));
+  // (chunks of one length: a shorter last one would take its round all the same)
+  int64_t n = (nvt + most - 1) / most;
+  const int64_t n_base = (nvt + base - 1) / base;
+  for (;; ++n) {
+    const TermsFwdPlan p = terms_fwd_plan_for(T, H, V, (nvt + n - 1) / n);
+    if (p.total <= room || n >= n_base) return p;
+  }
 }
 
 // ---- backward ---------------------------------------------------------------------------------
@@ -125,9 +140,9 @@ int launch_split(const SplitArgs& s, const SplitArgs* also, int* wide, hipStream
 }
 
 int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
-                  int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, hipStream_t st,
-                  int64_t label_offset, float* shard_out) {
-  const TermsFwdPlan pl = terms_fwd_plan(T, H, V);
+                  int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, size_t ws_bytes,
+                  hipStream_t st, int64_t label_offset, float* shard_out) {
+  const TermsFwdPlan pl = terms_fwd_plan(T, H, V, ws_bytes);
   bf16_t* h3 = reinterpret_cast<bf16_t*>(ws + pl.off_h);
   bf16_t* w3 = reinterpret_cast<bf16_t*>(ws + pl.off_w);
   int* wide = reinterpret_cast<int*>(ws + pl.off_wide);
