@@ -246,7 +246,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   if (terms) sel = kSelTerms;
-  if (xcache && sel != kSelT64 && sel != kSelT128 && sel != 0 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
+  if (xcache && sel != kSelT64 && sel != kSelT128 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
                          accumulate, entropy_b, ws, workspace_bytes, st, label_offset, shard_out, max_splits, xcache);

@@ -402,7 +402,10 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
         hipLaunchKernelGGL((lce_fwd16_kernel<Cfg, false>), dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
       }
     } else {
-      auto kern = sizeof(TIN) == 2 && xcache ? lce_fwd_kernel<Cfg, sizeof(TIN) == 2> : lce_fwd_kernel<Cfg, false>;  // (fp32 keeps none)
+      // (of these loops only the 128-token tile keeps logits, with W read once: forward_entry, read_w_once)
+      constexpr bool kKeeps = sizeof(TIN) == 2 && Cfg::BN == 128 && Cfg::A_AUX != 0;
+      if (xcache && !kKeeps) return fail(LCE_E_ARG, "forward: this tile cannot keep the logits");
+      auto kern = xcache ? lce_fwd_kernel<Cfg, kKeeps> : lce_fwd_kernel<Cfg, false>;
       allow_lds(kern, Cfg::LDS_BYTES);
       hipLaunchKernelGGL(kern, dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
     }

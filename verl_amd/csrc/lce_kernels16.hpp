@@ -814,11 +814,14 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_fwd16_kernel(FwdArgs<typena
   if (!p.map.decode(blockIdx.x, tt, s)) return;
   const int64_t n0 = (int64_t)tt * Cfg::BN, left = p.T - n0;
   if constexpr (Fwd16Tails<Cfg>::value) {
-    if (left <= 160) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<5>, KEEP>(p, n0, s, lds);
-    if constexpr (Cfg::NBN > 6) {
+    // (the weight read once is for a launch of one tile of tokens, and up to 192 that is the 192-wide one: forward_w_once)
+    constexpr bool kMoreThan192 = Cfg::A_ONCE && Cfg::NBN > 6;
+    if constexpr (!kMoreThan192)
+      if (left <= 160) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<5>, KEEP>(p, n0, s, lds);
+    if constexpr (!kMoreThan192 && Cfg::NBN > 6)
       if (left <= 192) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<6>, KEEP>(p, n0, s, lds);
+    if constexpr (Cfg::NBN > 6)
       if (left <= 224) return fwd16_body<typename Fwd16Tails<Cfg>::template Narrow<7>, KEEP>(p, n0, s, lds);
-    }
   }
   fwd16_body<Cfg, KEEP>(p, n0, s, lds);
 }

@@ -139,6 +139,7 @@ int launch_split(const SplitArgs& s, const SplitArgs* also, int* wide, hipStream
   return check_launch("split_again_kernel");
 }
 
+#if LCE_TU_PART == 0
 int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                   int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, size_t ws_bytes,
                   hipStream_t st, int64_t label_offset, float* shard_out) {
@@ -180,6 +181,7 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
                        entropy_b, shard_out, st);
 }
 
+#else
 int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                    int reduction, const float* maximum, const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
                    float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu) {
@@ -284,6 +286,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   }
   return LCE_OK;
 }
+#endif
 #endif
 
 }  // namespace
