@@ -287,8 +287,8 @@ int lce_ppo_forward_end(lce_ppo_call_t* call, void* stream, void* ticket);
 int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
 
 /* Product-level options (process-wide; every entry point works from one snapshot of the settings taken when it starts).
- * LCE_OPT_WORKSPACE_BUDGET (default 0 = the built-in rule, chunks of 8192 vocabulary columns or wider while one
- * d_logits buffer stays within 256 MiB): a byte count; lce_backward_workspace_bytes with vocab_chunk <= 0 then
+ * LCE_OPT_WORKSPACE_BUDGET (default 0 = the built-in rule: chunks of 16384 vocabulary columns while one d_logits buffer
+ * stays within 1 GiB, from 8192 columns on, wider while it stays within 256 MiB, narrower once two would pass 4 GiB): a byte count; lce_backward_workspace_bytes with vocab_chunk <= 0 then
  * returns the workspace of the widest chunk that fits it (never below 2048 columns, never above the bound
  * 0.25 * T * V * esz + 4 * V * H), and lce_backward with vocab_chunk <= 0 uses that chunk.  An explicit vocab_chunk
  * is not touched.  What lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES stays within it too, down to the least

@@ -1,4 +1,4 @@
-// Few tokens (gfx950).  16-bit inputs: the forward up to 64, d_hidden up to 128, d_weight up to 256, and d_logits from kept
+// Few tokens (gfx950).  16-bit inputs: the forward up to 96, d_hidden up to 128, d_weight up to 256, and d_logits from kept
 // logits; fp32 inputs: the forward up to 128.
 //
 // With T <= 128 every product is one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
@@ -485,8 +485,9 @@ __global__ __launch_bounds__(512, 2) void lce_dw_few_kernel(FewArgs<TIN> p) {
 // token rows:  C[m = h][n = t] = sum_u W[vocab_at(u)][h] * dS[t][u].
 // A stage is 64 columns of dS: 64 rows of W (512 bytes of each, fetched in the order of dS's columns) and NT x 128
 // bytes of dS.  What bounds it is the read of W, and that by the bytes in flight: four stages are on their way in registers
-// (128 KB of W per CU; three, 96 KB, beyond 64 tokens: step of 100 / 128 tokens at H=3584 674 / 686 us, four 667 / 678, H=5120 935 / 950,
-// four 923 / 945, others level) while one is multiplied out of LDS, which holds two, so that a stage costs one barrier.
+// (128 KB of W per CU) while one is multiplied out of LDS, which holds two, so that a stage costs one barrier.  Beyond 64 tokens, where
+// the tiles of dS take registers too, three stages were slower, us of a step: 100 / 128 tokens, H=3584, three 674 / 686, four 667 / 678;
+// H=5120 935 / 950, 923 / 945; other H level.
 // The workgroups of one slice read the same dS.  Numbered across the XCDs, the neighbours of a slice read pieces of the same rows of W at
 // the same time; numbered within them (by_xcd), dS passes into each L2 about once instead of in all eight.  The second from 33 tokens
 // on, where dS is a tenth of W and more: frozen head, 64 tokens, H=3584 410.8 -> 406.0 us, 4096: 377.5 -> 368.2, 5120: 569.4 -> 565.0;

@@ -14,7 +14,9 @@ struct FewF32Layout {
 // Which calls: shapes and diagnostic settings alone.  Measured, forward + backward in ms (the forward is the same), tiles of 256 x 256
 // with transposed copies of W / this way, H=3584, V=152064: 1 token 7.6 / 1.57, 32: 7.8 / 1.74, 64: 8.2 / 2.7, 100: 8.7 / 4.5, 128:
 // 8.8 / 4.6; H=896: 2.7 / 0.47, 2.8 / 0.50, 3.0 / 0.80, 3.1 / 1.31, 3.1 / 1.36; without d_weight, H=3584, 16 tokens 6.4 / 1.32.  Error
-// against float64 (2-norm; H=896, V=151936, 64 tokens): d_hidden 3.8e-6 / 3.8e-6, d_weight 1.2e-7 / 4.2e-8.
+// against float64 (2-norm; H=896, V=151936, 64 tokens): d_hidden 3.8e-6 / 3.8e-6, d_weight 1.2e-7 / 4.2e-8.  Where the line lies: the
+// kernels are laid out for 128 positions (hidden and its products take half the registers there), and from 129 to 255 tokens,
+// where the planes do not yet run, the tiles do (129: 11.2 ms, 255: 11.3, 256: 8.0); wider streams have not been tried.
 bool few_f32(const Tuning& tu, int64_t T) { return T <= 128 && !tu.variant_forced && tu.few_token_gemms && !tu.split_bwd; }
 
 FewF32Layout few_f32_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {

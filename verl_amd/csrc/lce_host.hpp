@@ -518,9 +518,10 @@ int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cos
 bool dh_sum_deep(int slices, int64_t workgroups) { return slices > 8 && 2 * workgroups <= 5 * kNumCUs; }
 
 // The same choice for every number of row tiles that may turn out to take part, within the memory that `ksplit` partials of all
-// T rows have.  Forward + backward in us, slices counted for all tokens / this way: H=4096, V=128256, 1000 tokens, about 500 with
-// gradient 1646 / 1341, about 250: 1931 / 1761, 2000 tokens 3263 / 2555, 400: 1083 / 1029; H=5120 1500 tokens 4016 / 3346; level
-// where every token has one and where the row tiles left fill the CUs as they are.
+// T rows have.  Forward + backward in us, bf16, slices counted for all tokens / this way, by the tokens with gradient: H=4096, V=128256,
+// 1000 tokens, all 2615 / 2615, 750: 2300 / 2245, 500: 2010 / 1865, 300: 1850 / 1700, 250: 1770 / 1470, 100: 1635 / 1350; 2000 tokens,
+// 1000: 3900 / 3550, 400: 3340 / 2607; H=5120, V=152064, 1500 tokens, all 5680 / 5680, 750: 4470 / 4000, 300: 3860 / 3082; H=3584, 333
+// tokens, 200: 1090 / 1090, 100: 922 / 868.
 DhSlices dh_slices_by_rows(int64_t T, int64_t H, int64_t vchunk, bool wide, int ksplit) {
   DhSlices d = {};
   d.tile_rows = wide ? 256 : 192;

@@ -80,11 +80,12 @@ def set_vocab_chunk(columns: int):
 
 
 def set_workspace_budget(num_bytes: int):
-    """Byte budget of the backward's workspace (process-wide; 0 = the library's default rule: chunks of 8192 vocabulary
-    columns, wider while one d_logits buffer stays within 256 MiB).  The library then picks the widest vocabulary chunk
-    whose workspace fits the budget (never fewer than 2048 columns) and never exceeds its own upper bound of a quarter of
-    one ``[T, V]`` tensor plus one fp32 ``[V, H]``.  An explicit ``set_vocab_chunk`` takes precedence.  The planes that an fp32
-    forward keeps of the weight stay within the budget too, down to 256 MB."""
+    """Byte budget of the backward's workspace (process-wide; 0 = the library's default rule: chunks of 16384 vocabulary
+    columns while one d_logits buffer stays within 1 GiB, from 8192 columns on, wider while it stays within 256 MiB, narrower
+    once two would pass 4 GiB).  The library then picks the widest vocabulary chunk whose workspace fits the budget (never
+    fewer than 2048 columns) and never exceeds its own upper bound of a quarter of one ``[T, V]`` tensor plus one fp32
+    ``[V, H]``.  An explicit ``set_vocab_chunk`` takes precedence.  The workspace of an fp32 forward on bfloat16 planes stays
+    within the budget too, down to some 256 MB."""
     _abi.check(_abi.load().lce_set_option(8, int(num_bytes)), "lce_set_option")
 
 
