@@ -29,7 +29,7 @@ extern "C" {
  * same).  For lce_forward,
  * lce_forward_keep_logits, lce_forward_shard and the lce_backward functions: a backward must be given the code of the
  * forward that its statistics come from, because the rounding errors of the logits that it recomputes cancel against those
- * of the statistics.  lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES the workspace the forward is fastest with
+ * of the statistics.  lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES the most that the forward makes use of
  * (planes of at most 256 MB of the weight, or two fifths of its own bytes where that is more, next to those of hidden) and for
  * LCE_DTYPE_F32 the least that is enough for either code; a forward on the planes is served with any size from there on, with
  * the same results.  The backward's query answers what the code asked for needs (for LCE_DTYPE_F32: either code).  The fp32 MFMA
@@ -288,11 +288,12 @@ int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
 
 /* Product-level options (process-wide; every entry point works from one snapshot of the settings taken when it starts).
  * LCE_OPT_WORKSPACE_BUDGET (default 0 = the built-in rule: chunks of 16384 vocabulary columns while one d_logits buffer
- * stays within 1 GiB, from 8192 columns on, wider while it stays within 256 MiB, narrower once two would pass 4 GiB): a byte count; lce_backward_workspace_bytes with vocab_chunk <= 0 then
- * returns the workspace of the widest chunk that fits it (never below 2048 columns, never above the bound
- * 0.25 * T * V * esz + 4 * V * H), and lce_backward with vocab_chunk <= 0 uses that chunk.  An explicit vocab_chunk
- * is not touched.  What lce_forward_workspace_bytes answers for LCE_DTYPE_F32_PLANES stays within it too, down to the least
- * that is enough.  Takes the role of the reference's fixed vocab_per_split = 9504 (verl/utils/kernel/kernels.py:1666-1670).
+ * stays within 1 GiB, from 8192 columns on, wider while it stays within 256 MiB, narrower once two would pass 4 GiB): a byte
+ * count; lce_backward_workspace_bytes with vocab_chunk <= 0 then returns the workspace of the widest chunk that fits it
+ * (never below 2048 columns, never above the bound 0.25 * T * V * esz + 4 * V * H), and lce_backward with vocab_chunk <= 0
+ * uses that chunk.  An explicit vocab_chunk is not touched.  What lce_forward_workspace_bytes answers for
+ * LCE_DTYPE_F32_PLANES stays within it too, down to the least that is enough.
+ * Takes the role of the reference's fixed vocab_per_split = 9504 (verl/utils/kernel/kernels.py:1666-1670).
  * LCE_OPT_LABEL_TERM_OUTSIDE (default 2, 16-bit inputs only) chooses the data format of the gradient of the logits:
  * 0 = the label's entry is rounded to 16 bits with the rest of the d_logits tile, which is the reference's format
  * (verl/utils/kernel/kernels.py:1666-1724); 1 = its one-hot part g_logprob / temperature * 1[v == label] is added to
