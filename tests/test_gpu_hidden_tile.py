@@ -1,0 +1,52 @@
+"""Gradient products on tiles of 224 hidden columns: hidden sizes of one tile (cut short), several, and several with a cut last one,
+through every kernel that has them: launches of their own (one chunk), combined launches (several chunks, d_hidden read back and
+added to), 16-bit and fp32 results, fp32 inputs on planes; against the oracle in float64."""
+
+import pytest
+import torch
+
+from oracle import lce_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,V,vchunk,keep", [
+    (150, 128, 9001, 0, 1.0),      # one tile, 128 of its columns; narrow tiles of tokens; the streaming d_weight
+    (300, 640, 20003, 0, 0.7),     # three tiles, the last one cut
+    (520, 896, 33001, 0, 1.0),     # whole tiles
+    (1025, 896, 33024, 0, 0.02),   # two slabs of K at most
+    (2100, 384, 40011, 8192, 0.6),
+    (700, 896, 36864, 4096, 1.0),
+])  # fmt: skip
+def test_gradients_on_narrow_tiles(T, H, V, vchunk, keep, dtype):
+    from verl_amd.utils.kernel import kernels
+
+    g = torch.Generator().manual_seed(T + H)
+    h = torch.randn(T, H, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(V, H, generator=g) * 0.03).to(dtype).to(DEV)
+    y = torch.randint(0, V, (T,), generator=g).to(DEV)
+    mask = (torch.rand(T, generator=g) < keep).float()
+    g_lp, g_ent = (torch.randn(T, generator=g) * mask).to(DEV), (torch.randn(T, generator=g) * mask).to(DEV)
+    *_, mx, ac, eb, cache = kernels.forward_keeping_logits(h, w, y, 0, 0.9)
+    rdh, rdw = O.lce_backward(g_lp, g_ent, h, w, y, 0.9, compute_dtype=torch.float64)
+    run = lambda f32, **kw: kernels.efficient_entropy_backward(g_lp, g_ent, h, w, y, mx, ac, eb, 0, f32, 0.9, **kw)  # noqa: E731
+    kernels.set_vocab_chunk(vchunk)
+    try:
+        for f32 in (False, True):
+            dh, dw = run(f32)
+            dh1, _ = run(f32, need_d_weight=False)
+            _, dw1 = run(f32, need_d_hidden=False)
+            assert torch.equal(dh, dh1) and torch.equal(dw, dw1)
+            if cache is not None:
+                dh2, dw2 = run(f32, logits_cache=cache)
+                assert torch.equal(dh, dh2) and torch.equal(dw, dw2)
+            # 16 bits: every element of the logits' gradient is rounded by 2^-9 (2^-12) of itself; fp32: the planes' own error
+            rel = 3e-6 if dtype == torch.float32 else 2.0**-7
+            for got, want in ((dh, rdh), (dw, rdw)):
+                assert ((got.double() - want).norm() / want.norm()).item() <= rel
+                assert (got.double() - want).abs().max().item() <= (1e-5 if dtype == torch.float32 else 2.0**-7) * want.abs().max().item()
+    finally:
+        kernels.set_vocab_chunk(0)
+    assert (dh[mask.to(DEV) == 0] == 0).all()

@@ -62,19 +62,20 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 // ONE fp32 product or partial sum costs, and the products themselves are exact.  Six bfloat16 MFMAs take six sixteenths
 // of the matrix pipe's time of the fp32 one.
 // A_ONCE_: the loads of A are marked non-temporal (A is read once, or nearly, and larger than the caches).
-template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0, int TERMS_ = 1, int A_ONCE_ = 0>
+// NBM_: 16-row blocks per wave along the MFMA rows: 8 for tiles of 256 rows, 7 for 224 (A K-major only: hidden_tile).
+template <typename TIN_, int TRANS_ = 0, int NBN_ = 8, int A_EARLY_ = 0, int TERMS_ = 1, int A_ONCE_ = 0, int NBM_ = 8>
 struct GemmCfg16 {
   typedef TIN_ TIN;
   static_assert(sizeof(TIN_) == 2, "16-bit operands");
   static constexpr bool CORE16 = true;
   static_assert(NBN_ == 8 || TRANS_ != 1, "both operands K-major: square tiles");
-  static constexpr int BM = 256, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
+  static constexpr int BM = 32 * NBM_, BN = 32 * NBN_, BKB = 128, BK = 64, NSTAGE = 5, SPLIT = 2, TRANS = TRANS_;
   static constexpr bool A_EARLY = A_EARLY_ != 0, A_ONCE = A_ONCE_ != 0;
   static constexpr int TERMS = TERMS_;
   static_assert(TERMS_ == 1 || TERMS_ == 6, "products per slab");
   static constexpr int WAVES_M = 2, WAVES_N = 2, NW = 4, NTHREADS = 256;
-  static constexpr int WM = 128, WN = 16 * NBN_;
-  static constexpr int NB = 8, NBN = NBN_;           // 16-row / 16-column blocks of a wave tile
+  static constexpr int WM = 16 * NBM_, WN = 16 * NBN_;
+  static constexpr int NB = NBM_, NBN = NBN_;        // 16-row / 16-column blocks of a wave tile
   static constexpr int STAGE_BYTES = 32768;          // one operand's slab: 256 rows x 128 bytes (or BN rows), or 64 k-rows x 512 bytes
   static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
   static constexpr int HL = 8, HLB = NBN_;           // wave-wide 16-byte-per-lane loads per wave and half slab of A, of B
@@ -121,6 +122,7 @@ struct GemmCore16 {
   // 16 rows x 4 chunks that a quarter wave reads for one fragment then fall into 64 different banks.
   LCE_DEV void init(const TIN* A, int64_t lda, int64_t m0, int64_t M, const TIN* B, int64_t ldb, int64_t n0, int64_t N,
                     const int* b_rows = nullptr) {
+    static_assert(Cfg::BM == 256, "row-major A: tiles of 256 rows");
     set_lane();
     a_base = reinterpret_cast<const char*>(A + m0 * lda);
     b_base = reinterpret_cast<const char*>(b_rows ? B : B + n0 * ldb);
@@ -146,8 +148,8 @@ struct GemmCore16 {
     b_rd = (uint32_t)(wave_n * Cfg::WN * 128) + off;
   }
 
-  // K-major operands: A[k][m0 + 0..256), B[k][n0 + 0..256) with row strides lda / ldb (elements); both must be
-  // allocated in whole 256-column tiles.  A ring slot holds 64 k-rows of 512 bytes; chunk c of row r sits at
+  // K-major operands: A[k][m0 + 0..BM), B[k][n0 + 0..256) with row strides lda / ldb (elements); both must be
+  // allocated in whole tiles.  A ring slot holds 64 k-rows of 512 bytes; chunk c of row r sits at
   // position c ^ swz(r), swz(r) = 4 (r % 4) ^ 2 ((r / 8) % 2), so that the eight k-rows that half a wave touches
   // in one transposing read fall into different banks.
   // The transposing read: in each group of 16 lanes, lane 4e + q supplies the address of X[k0 + e][x0 + 4q ..] and
@@ -164,7 +166,7 @@ struct GemmCore16 {
     for (int j = 0; j < HL; ++j) {
       const int row = (j * Cfg::NW + wave) * 2 + (lane >> 5);
       const int c = (lane & 31) ^ tn_swz(row);
-      va[j] = (uint32_t)((int64_t)row * lda * 2) + (uint32_t)(c * 16);
+      va[j] = (uint32_t)((int64_t)row * lda * 2) + (uint32_t)(a_chunk(c) * 16);
       vb[j] = (uint32_t)((int64_t)row * ldb * 2) + (b_pcol ? (uint32_t)((c >> 3) * b_pcol * 2) + (uint32_t)((c & 7) * 16) : (uint32_t)(c * 16));
     }
     reads_tn(lane);
@@ -173,8 +175,15 @@ struct GemmCore16 {
     const int g = ln >> 4, e = (ln & 15) >> 2, q = ln & 3;
     const int row = 8 * g + e;  // (k-step 0, first half of the octet)
     const uint32_t in_row = (uint32_t)((((q >> 1) ^ tn_swz(row)) * 16) + (q & 1) * 8);
-    a_rd = (uint32_t)(row * 512 + wave_m * Cfg::WM * 2) + in_row;
+    a_rd = (uint32_t)(row * 512 + wave_m * 256) + in_row;
     b_rd = (uint32_t)(row * 512 + wave_n * Cfg::WN * 2) + in_row;
+  }
+  // 16-byte chunk of a row of a K-major A that chunk c of the LDS row holds: each wave's columns begin at a multiple of 256 bytes
+  // there, whatever their number (the blocks' offsets are XORed in); what is left over repeats the last chunk
+  static LCE_DEV int a_chunk(int c) {
+    if (NB == 8) return c;
+    const int in = c & 15;
+    return (c >> 4) * 2 * NB + (in < 2 * NB ? in : 2 * NB - 1);
   }
   // another tile of the same matrices after init_tn
   LCE_DEV void move_tn(const TIN* A, int64_t m0, const TIN* B, int64_t n0, int64_t b_pcol) {
@@ -183,10 +192,10 @@ struct GemmCore16 {
   }
   static LCE_DEV int tn_swz(int row) { return ((row & 3) * 4) ^ (((row >> 3) & 1) * 2); }
 
-  // Mixed: A[k][m0 + 0..256) K-major as in init_tn, B row-major as in init (rows n0 .. of an N-row matrix, clamped).
+  // Mixed: A[k][m0 + 0..BM) K-major as in init_tn, B row-major as in init (rows n0 .. of an N-row matrix, clamped).
   // LDS row r of an A slab holds memory row perm(r) of the slab (perm: a permutation of 0..63, the order in which B's
   // K index was stored); rows at or beyond `kvalid` > 0 are replaced by rows that exist (B is zero there), and columns at
-  // or beyond `mcols` (a last tile of a width that is no multiple of 256) by the row's first chunk: in bounds, and they
+  // or beyond `mcols` (a last tile that is not full) by the row's first chunk: in bounds, and they
   // feed only results that the epilogue discards.  b_slab_bytes: from one K slab of B to the next (its rows' 128 bytes for
   // rows of ldb elements; a panel where B lies in panels of 64 columns).
   template <typename Perm>
@@ -206,7 +215,7 @@ struct GemmCore16 {
 #pragma unroll
     for (int j = 0; j < HL; ++j) {
       const int rowa = (j * Cfg::NW + wave) * 2 + (lane >> 5);
-      const int ca = (lane & 31) ^ tn_swz(rowa);
+      const int ca = a_chunk((lane & 31) ^ tn_swz(rowa));
       const int prow = (int)perm(rowa);
       const uint32_t col = (uint32_t)(((int64_t)ca * 8 < mcols ? ca : 0) * 16);
       va[j] = (uint32_t)((int64_t)prow * lda * 2) + col;
@@ -220,7 +229,7 @@ struct GemmCore16 {
     }
     const int g = lane >> 4, e = (lane & 15) >> 2, q = lane & 3;
     const int row = 8 * g + e;
-    a_rd = (uint32_t)(row * 512 + wave_m * Cfg::WM * 2) + (uint32_t)((((q >> 1) ^ tn_swz(row)) * 16) + (q & 1) * 8);
+    a_rd = (uint32_t)(row * 512 + wave_m * 256) + (uint32_t)((((q >> 1) ^ tn_swz(row)) * 16) + (q & 1) * 8);
     const int r16 = lane & 15;
     b_rd = (uint32_t)(wave_n * Cfg::WN * 128) + (uint32_t)(r16 * 128 + ((g ^ (r16 >> 1)) * 16));
   }
@@ -288,7 +297,7 @@ struct GemmCore16 {
                      u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NBN], char* lds, int dma_slot, int64_t dma_ks,
                      const char* dma_from = nullptr) const {
     constexpr int DMAS = DMA_B ? HLB : HL, EVERY = NB * NBN / DMAS;
-    static_assert(2 * NF <= NB * NBN && NB * NBN % DMAS == 0, "one fragment read after every second MFMA");
+    static_assert(2 * NF <= NB * NBN && DMAS * EVERY <= NB * NBN && EVERY > 3, "one fragment read after every second MFMA");
     static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
       constexpr int m = decltype(mc)::value;
       constexpr int i = m / NBN, j = m % NBN;
@@ -301,7 +310,7 @@ struct GemmCore16 {
       if constexpr (FIRST) Mma16<TIN>::first(acc[i][j], af[i], bf[j]);
       else Mma16<TIN>::run(acc[i][j], af[i], bf[j]);
       if constexpr ((m & 1) == 0 && m / 2 < NF) read_frag<m / 2, S_N>(ra_n, rb_n, af_n, bf_n);
-      if constexpr (m % EVERY == 3) {
+      if constexpr (m % EVERY == 3 && m / EVERY < DMAS) {
         constexpr int j8 = m / EVERY;
         if constexpr (FROM)
           __builtin_amdgcn_global_load_lds((gptr_t)(dma_from + (DMA_B ? vb[j8] : va[j8])), (lptr_t)(lds + dma_slot * SLOT + (j8 * Cfg::NW + wave) * 1024),
@@ -428,7 +437,7 @@ struct GemmCore16 {
   template <int STORES>
   LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
     static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
-    static_assert(NBN == NB && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "square tiles, B early");
+    static_assert(NBN == 8 && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "whole tiles, B early");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     int sb = s.sb;
     auto slab = [&](auto first, int it) {
@@ -456,7 +465,9 @@ struct GemmCore16 {
     // the next tile's first fragments are in registers from here on, whatever the compiler does with those meanwhile
     wait_lgkm<0>();
 #pragma unroll
-    for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(s.af[i]), "+v"(s.bf[i]));
+    for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(s.af[i]));
+#pragma unroll
+    for (int j = 0; j < NBN; ++j) asm volatile("" : "+v"(s.bf[j]));
     retire(acc);
   }
 

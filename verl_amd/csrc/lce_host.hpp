@@ -207,7 +207,7 @@ int block_rows(int nrow_tiles) { return TileMap::block_rows(nrow_tiles); }
 template <typename Cfg>
 GemmArgs<typename Cfg::TIN> make_gemm_args(const typename Cfg::TIN* A, int64_t lda, const typename Cfg::TIN* B, int64_t ldb,
                                            int64_t M, int64_t N, int64_t K, float* Cf, int64_t ldcf, typename Cfg::TIN* Ct,
-                                           int64_t ldct, int out_mode) {
+                                           int64_t ldct, int out_mode, int n_tile = 0) {  // n_tile: width of C's tiles (0: Cfg's)
   GemmArgs<typename Cfg::TIN> p;
   p.A = A; p.lda = lda; p.B = B; p.ldb = ldb; p.M = M; p.N = N; p.K = K;
   p.a_pcol = 0; p.a_plane = p.b_plane = 0;
@@ -215,7 +215,7 @@ GemmArgs<typename Cfg::TIN> make_gemm_args(const typename Cfg::TIN* A, int64_t l
   p.ksplit = 1; p.kslice = K; p.cf_split_stride = 0;
   p.m_dev = nullptr; p.k_dev = nullptr; p.k_gran = 1; p.tn = 0; p.b_rows_valid = 0; p.perm_rows = 0;
   // (the 16x16x32 loop takes its MFMA columns from A)
-  const int rm = Cfg::CORE16 ? Cfg::BN : Cfg::BM, rn = Cfg::CORE16 ? Cfg::BM : Cfg::BN;
+  const int rm = Cfg::CORE16 ? Cfg::BN : Cfg::BM, rn = n_tile ? n_tile : Cfg::CORE16 ? Cfg::BM : Cfg::BN;
   const int tm = (int)((M + rm - 1) / rm), tn = (int)((N + rn - 1) / rn);
   p.n_tiles = tn;
   p.map = TileMap::make(tm, tn, block_rows(tm), 1);
@@ -481,6 +481,19 @@ struct BwdLayout {
 // elements); for fp32 a vocab-major copy of the d_logits and a transposed hidden are built for it.
 bool dw_transposed_reads(size_t esz) { return esz == 2; }
 
+// Width of the gradient products' tiles along H on the 16x16x32 loop: 256, or 224 where those leave less of the last tile over.  H = 896
+// is four tiles either way, without a column of padding or with 128.  A 224-wide tile's slab is an eighth less matrix work behind
+// the same loads and takes some 0.92 of the time, hence the line: 896 and the narrow sizes below, not 2688 (12 tiles for 11).  H=896,
+// V=151936, forward + backward, 256 / 224 wide: bf16 500 tokens 577 -> 553 us, 1000: 1076 -> 1035, 4096: 3920 -> 3780, 16384: 14.98 -> 14.48 ms;
+// fp32 on planes 400 tokens 3101 -> 2995 us, 1024: 5854 -> 5670, 2000: 10862 -> 10465.
+int hidden_tile(int64_t H) { return (H + 223) / 224 * 12 < (H + 255) / 256 * 13 ? 224 : 256; }
+
+// the same loop on tiles of 224 hidden columns
+template <typename Cfg> struct Hidden224 { typedef Cfg type; };
+template <typename TIN, int TR, int NBN, int AE, int TERMS, int AO> struct Hidden224<GemmCfg16<TIN, TR, NBN, AE, TERMS, AO, 8>> {
+  typedef GemmCfg16<TIN, TR, NBN, AE, TERMS, AO, 7> type;
+};
+
 // The d_hidden GEMM has only ceil(T/256) * ceil(H/256) output tiles, each with a K loop as long as the
 // vocabulary chunk.  With few tokens one such tile takes longer than a CU's share of the whole launch
 // (d_logits tiles + both GEMMs) and would set the launch's duration; the K range is then cut into
@@ -499,7 +512,7 @@ int dh_ksplit(int64_t T, int64_t H, int64_t vchunk) {
 // tiles x 9 slices are one round of 264 slabs; 16 slices, what the mixed launch would take, two rounds of 149.)
 // `wide`: token tiles 256 wide, else 192, whose slabs take 0.82 of the time (28 tiles either way: 512 tokens 412 us, 333: 330).
 int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cost_out, int most = 32) {
-  const int64_t tiles = (wide ? (T + 255) / 256 : (T + 191) / 192) * ((H + 255) / 256), slabs = (vchunk + 63) / 64;
+  const int64_t ht = hidden_tile(H), tiles = (wide ? (T + 255) / 256 : (T + 191) / 192) * ((H + ht - 1) / ht), slabs = (vchunk + 63) / 64;
   const double per_slice = (double)T * H * 8.0 / 5.0e12 / 1.2e-6;
   int best = 1;
   double best_cost = -1.0;
@@ -813,10 +826,12 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
   const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN);
   // (the K-major d_weight tiles use the 160 KB split ring whatever ring the variant itself uses)
   const int chunk_lds = L.tn && Cfg::LDS_BYTES < 160 * 1024 ? 160 * 1024 : Cfg::LDS_BYTES;
+  const int h_tile = Cfg::CORE16 ? hidden_tile(H) : 0;
   auto launch_chunk = [&](const BwdChunkArgs<TIN>& q) {
     if constexpr (Cfg::CORE16) {
-      allow_lds(lce_bwd_chunk16_kernel<Cfg>, chunk_lds);
-      hipLaunchKernelGGL(lce_bwd_chunk16_kernel<Cfg>, dim3(q.n_gw + q.n_gh + q.n_ds), dim3(Cfg::NTHREADS), chunk_lds, st, q);
+      auto kern = h_tile == 224 ? lce_bwd_chunk16_kernel<Cfg, 7> : lce_bwd_chunk16_kernel<Cfg, 8>;
+      allow_lds(kern, chunk_lds);
+      hipLaunchKernelGGL(kern, dim3(q.n_gw + q.n_gh + q.n_ds), dim3(Cfg::NTHREADS), chunk_lds, st, q);
     } else {
       allow_lds(lce_bwd_chunk_kernel<Cfg>, chunk_lds);
       hipLaunchKernelGGL(lce_bwd_chunk_kernel<Cfg>, dim3(q.n_gw + q.n_gh + q.n_ds), dim3(Cfg::NTHREADS), chunk_lds, st, q);
@@ -886,7 +901,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           // (no d_hidden GEMM)
         } else if (L.tn_dh) {
           // W as it lies in memory (K-major for this product), fetched with transposing LDS reads
-          p.gh = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, W + v0 * ldw, ldw, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1);
+          p.gh = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, W + v0 * ldw, ldw, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1, h_tile);
           p.gh.tn = 2;
           p.gh.a_pcol = L.panels ? L.pcol : 0;
           p.gh.b_rows_valid = vrows;
@@ -913,7 +928,7 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
           // (no d_weight GEMM)
         } else if (L.tn) {
           // d_weight[v0 : v0 + vrows][H] = dS[tokens][vrows]^T . hidden[tokens][H], both operands K-major
-          p.gw = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, Ht, L.ldHt, vrows, H, round_up(T, 64), dw_f32, H, dw_t, H, grads_f32 ? 0 : 2);
+          p.gw = make_gemm_args<Cfg>(dS[cc & 1], L.ldS, Ht, L.ldHt, vrows, H, round_up(T, 64), dw_f32, H, dw_t, H, grads_f32 ? 0 : 2, h_tile);
           p.gw.tn = 1;
           p.gw.a_pcol = L.panels ? L.pcol : 0;
           p.gw.perm_rows = 1;
@@ -927,8 +942,8 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
         if constexpr (Cfg::CORE16) {
           // (one chunk: no d_logits tiles share this launch)
           if (L.mid && !tu.split_bwd && need_dh) {
-            auto launch_dh = [&](auto variant) {
-              typedef typename decltype(variant)::Cfg DhCfg;
+            auto launch_dh_on = [&](auto cfg) {
+              typedef decltype(cfg) DhCfg;
               GemmArgs<TIN> q = p.gh;
               const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
               q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
@@ -941,6 +956,10 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
               allow_lds(lce_dh16_kernel<DhCfg>, DhCfg::LDS_BYTES);
               hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3((unsigned)grid), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q, by_rows);
               return check_launch("lce_dh16_kernel");
+            };
+            auto launch_dh = [&](auto variant) {
+              typedef typename decltype(variant)::Cfg DhCfg;
+              return h_tile == 224 ? launch_dh_on(typename Hidden224<DhCfg>::type{}) : launch_dh_on(DhCfg{});
             };
             const bool once = need_dw && T <= (L.mid_192 ? 192 : 512);
             if (L.mid_192) rc = once ? launch_dh(VariantN192<TIN, 1>{}) : launch_dh(VariantN192<TIN, 0>{});
@@ -958,11 +977,11 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
             if (rc) return rc;
             p.n_gw = 0;
           } else if (L.mid && !tu.split_bwd && need_dw && dw_t && aligned16(dw_t)) {
-            const int64_t tiles = ((p.gw.M + 255) / 256) * ((p.gw.N + 255) / 256);
+            const int64_t tiles = ((p.gw.M + 255) / 256) * p.gw.n_tiles;
             ProfScope prof(PC_GEMM_DW, st);
-            allow_lds(lce_dw16_kernel<Cfg>, Cfg::LDS_BYTES);
-            hipLaunchKernelGGL(lce_dw16_kernel<Cfg>, dim3((unsigned)(tiles < kNumCUs ? p.gw.map.total : kNumCUs)), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st,
-                               p.gw);
+            auto kern = h_tile == 224 ? lce_dw16_kernel<typename Hidden224<Cfg>::type> : lce_dw16_kernel<Cfg>;
+            allow_lds(kern, Cfg::LDS_BYTES);
+            hipLaunchKernelGGL(kern, dim3((unsigned)(tiles < kNumCUs ? p.gw.map.total : kNumCUs)), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p.gw);
             if ((rc = check_launch("lce_dw16_kernel"))) return rc;
             p.n_gw = 0;
           }

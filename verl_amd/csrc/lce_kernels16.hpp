@@ -12,8 +12,8 @@ namespace lce {
 // vocabulary rows (one wave tile) the entries are ordered so that what a lane holds of two neighbouring blocks is one
 // 16-byte run and the four lane groups follow each other (64 contiguous bytes per token and store instruction):
 // row v = 16 i + 4 g + r  ->  position 32 (i / 2) + 8 g + 4 (i % 2) + r.  Tokens keep their order.
-template <typename TIN, int TR, int NBN, int AE, int TERMS, int AO>
-struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS, AO>> {
+template <typename TIN, int TR, int NBN, int AE, int TERMS, int AO, int NBM>
+struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS, AO, NBM>> {
   static constexpr int GT = 128, GV = 128;
   static __host__ __device__ __forceinline__ int64_t token(int64_t t) { return t; }
   static __host__ __device__ __forceinline__ int64_t token_at(int64_t u) { return u; }
@@ -413,7 +413,7 @@ LCE_DEV void gemm16_edge(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cf
   }
 }
 
-// A full wave tile in fp32, C (+)= acc (ACC: old values are read), as whole lines: one block column (16 rows x 128 columns) at a
+// A full wave tile in fp32, C (+)= acc (ACC: old values are read), as whole lines: one block column (16 rows x 128 or 112 columns) at a
 // time goes through 8 KB of LDS that belong to this wave, 16-byte chunk c of row r at c ^ r, and meets memory two rows x 512
 // bytes per instruction.  In the accumulators' own lane order, 16 rows x 64 bytes, reading and writing a tile took 38300
 // cycles, a sixteenth of the d_hidden GEMM's K loop, with one block column of old values on its way or with three; this way it
@@ -421,17 +421,20 @@ LCE_DEV void gemm16_edge(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cf
 template <typename Cfg, bool ACC>
 LCE_DEV void gemm16_f32_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t mw, int64_t nw, uint32_t stage) {
   // mw, nw: the wave tile's first row and column of C
-  constexpr int NB = Cfg::NB, NBN = Cfg::NBN, AHEAD = 2;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN, AHEAD = 2, PAIRS = 8;
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15, hi = lane >> 5, cl = lane & 31;
   const uint32_t wr = stage + (uint32_t)(l16 * 512 + (g4 ^ l16) * 16);   // chunk 4 i + g4: ^ i * 64
   const uint32_t rd = stage + (uint32_t)(hi * 512 + (cl ^ hi) * 16);     // row 2 k + hi: ^ k * 32, + k * 1024
   char* base = reinterpret_cast<char*>(p.Cf + mw * p.ldcf + nw);
   const uint32_t off = (uint32_t)(hi * p.ldcf * 4 + cl * 16);
   const int64_t row_bytes = p.ldcf * 4;
-  f32x4_t prev[AHEAD + 1][NB];
+  const bool has = NB == 8 || cl < 4 * NB;  // (the lane has a chunk of its row)
+  f32x4_t prev[AHEAD + 1][PAIRS];
   auto fetch = [&](int j) {
+    if (has) {
 #pragma unroll
-    for (int k = 0; k < NB; ++k) prev[j % (AHEAD + 1)][k] = *reinterpret_cast<const f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off);
+      for (int k = 0; k < PAIRS; ++k) prev[j % (AHEAD + 1)][k] = *reinterpret_cast<const f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off);
+    }
   };
   auto write = [&](int j) {
     GemmCore16<Cfg>::stay_column(acc, j);
@@ -449,26 +452,28 @@ LCE_DEV void gemm16_f32_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&ac
     if (ACC && j + AHEAD < NBN) fetch(j + AHEAD);
     if (j + 1 < NBN) write(j + 1);
     GemmCore16<Cfg>::template wait_lgkm<(j + 1 < NBN ? NB : 0)>();  // block column j is in LDS (j + 1's writes may be on their way)
-    u32x4_t v[NB];
-    static_for(std::make_integer_sequence<int, NB>{}, [&](auto kc) {
+    u32x4_t v[PAIRS];
+    static_for(std::make_integer_sequence<int, PAIRS>{}, [&](auto kc) {
       constexpr int k = decltype(kc)::value;
       v[k] = lds_read16<k * 1024>((rd ^ (uint32_t)(k * 32)) + (j & 1) * 8192);
     });
     GemmCore16<Cfg>::template wait_lgkm<0>();
 #pragma unroll
-    for (int k = 0; k < NB; ++k) asm volatile("" : "+v"(v[k]));  // (the reads are assembly, the compiler does not know when they return)
+    for (int k = 0; k < PAIRS; ++k) asm volatile("" : "+v"(v[k]));  // (the reads are assembly, the compiler does not know when they return)
+    if (has) {
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      f32x4_t x = __builtin_bit_cast(f32x4_t, v[k]);
-      if (ACC) x += prev[j % (AHEAD + 1)][k];
-      *reinterpret_cast<f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off) = x;
+      for (int k = 0; k < PAIRS; ++k) {
+        f32x4_t x = __builtin_bit_cast(f32x4_t, v[k]);
+        if (ACC) x += prev[j % (AHEAD + 1)][k];
+        *reinterpret_cast<f32x4_t*>(base + (16 * j + 2 * k) * row_bytes + off) = x;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   });
 }
 
 // C in fp32 (out_mode 0 or 1: the callers have no other).
-// CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2, NBN>: then B is K-major as it lies in memory, B[k][n] with row
+// CoreCfg: Cfg itself, or its mixed twin GemmCfg16<TIN, 2, ..>: then B is K-major as it lies in memory, B[k][n] with row
 // stride ldb, its rows in the order KPerm<Cfg>::vocab_at of A's columns (the d_hidden GEMM reading W in place: no W^T);
 // rows of B at or beyond p.b_rows_valid do not exist (A is zero in those columns).
 template <typename Cfg, typename CoreCfg = Cfg>
@@ -539,18 +544,18 @@ LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_
 // Non-temporal: unmarked, the lines of d_weight push the dS and the hidden that other workgroups are about to read out of the
 // caches (forward + backward, H=3584, V=152064: 333 tokens 1289 -> 1240 us, 512: 1624 -> 1588, 700: 2111 -> 2089, level from 1600 on).
 template <typename Cfg, typename PermCfg, bool FULL>
-LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NB], int64_t m0, int64_t n0,
+LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], int64_t m0, int64_t n0,
                                 int wave_m, int wave_n, uint32_t stage) {
   typedef typename Cfg::TIN TIN;
   typedef typename VecOf<TIN, 4>::type vec_t;
-  constexpr int NB = Cfg::NB;
+  constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
   const int lane = lane_anew(), g4 = lane >> 4, l16 = lane & 15;
   const uint32_t wr = stage + (uint32_t)(l16 * 256 + (((g4 >> 1) ^ l16) * 16) + (g4 & 1) * 8);  // chunk 2 i + g4 / 2: ^ i * 32
   const uint32_t rd = stage + (uint32_t)(g4 * 256 + ((l16 ^ g4) * 16));                          // row 4 k + g4: ^ k * 64, + k * 1024
   // the store of row 4 k + g4 of block column j, chunk l16: a uniform row pointer and one offset per lane
   const int64_t n = n0 + wave_m * Cfg::WM;
   const uint32_t off = (uint32_t)(g4 * p.ldct + l16 * 8) * (uint32_t)sizeof(TIN);
-  const bool n_ok = FULL || n + l16 * 8 < p.N;
+  const bool n_ok = (NB == 8 || l16 < 2 * NB) && (FULL || n + l16 * 8 < p.N);  // (the lane has a chunk of its row)
   const int64_t mw = m0 + wave_n * Cfg::WN;
   char* base = reinterpret_cast<char*>(p.Ct + mw * p.ldct + n);
   auto write = [&](auto jc) {
@@ -577,20 +582,20 @@ LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&
     for (int k = 0; k < 4; ++k) {
       constexpr int u0 = 16 * j;
       const int64_t row = KPerm<PermCfg>::vocab_at(u0 + 4 * k);  // (+ g4: four consecutive rows of C)
-      if (FULL || (n_ok && mw + row + g4 < p.M)) __builtin_nontemporal_store(v[k], reinterpret_cast<u32x4_t*>(base + row * p.ldct * (int64_t)sizeof(TIN) + off));
+      if (n_ok && (FULL || mw + row + g4 < p.M)) __builtin_nontemporal_store(v[k], reinterpret_cast<u32x4_t*>(base + row * p.ldct * (int64_t)sizeof(TIN) + off));
     }
   };
-  static_for(std::make_integer_sequence<int, NB + 1>{}, [&](auto jc) {
+  static_for(std::make_integer_sequence<int, NBN + 1>{}, [&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    if constexpr (j < NB) write(jc);
+    if constexpr (j < NBN) write(jc);
     if constexpr (j > 0) {
-      GemmCore16<Cfg>::template wait_lgkm<(j < NB ? NB : 0)>();  // block column j - 1 is in LDS (j's eight writes may be on their way)
+      GemmCore16<Cfg>::template wait_lgkm<(j < NBN ? NB : 0)>();  // block column j - 1 is in LDS (j's writes may be on their way)
       store(std::integral_constant<int, j - 1>{});
     }
   });
 }
 
-// C[m][n] = sum_k A[k][m] * B[k][n], both operands K-major and allocated in whole 256-column tiles, K (or *k_dev
+// C[m][n] = sum_k A[k][m] * B[k][n], both operands K-major and allocated in whole tiles, K (or *k_dev
 // rounded up to k_gran) a multiple of 64.  out_mode 0: Cf = acc; out_mode 2: Ct[PermCfg's vocab_at(m)][n] = (TIN)acc
 // (the rows of C are A's columns, which the d_logits epilogue leaves in KPerm::vocab order).
 template <typename Cfg, typename PermCfg>
@@ -603,31 +608,31 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
   }
   int tm, tn;
   if (!p.map.decode(bid, tm, tn)) return;
-  const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
+  const int64_t m0 = (int64_t)tm * Cfg::BN, n0 = (int64_t)tn * Cfg::BM;  // (MFMA rows = n, MFMA columns = m)
   GemmCore16<Cfg> g;
-  f32x4_t acc[Cfg::NB][Cfg::NB];
+  f32x4_t acc[Cfg::NB][Cfg::NBN];
   if (p.K > 0) {
     g.a_plane = p.b_plane;
     g.b_plane = p.a_plane;
-    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);  // MFMA rows = n, MFMA columns = m
+    g.init_tn(p.B, p.ldb, n0, p.A, p.lda, m0, p.a_pcol);
     g.run(lds, p.K, acc);
   } else {
     g.set_lane();
 #pragma unroll
     for (int i = 0; i < Cfg::NB; ++i)
 #pragma unroll
-      for (int j = 0; j < Cfg::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < Cfg::NBN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   if (p.out_mode == 2) {
     __syncthreads();  // (the ring is the store tiles' now)
     const uint32_t stage = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 8192;
-    if (m0 + Cfg::BM <= p.M && n0 + Cfg::BN <= p.N) gemm16_store_lines<Cfg, PermCfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
+    if (m0 + Cfg::BN <= p.M && n0 + Cfg::BM <= p.N) gemm16_store_lines<Cfg, PermCfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
     else gemm16_store_lines<Cfg, PermCfg, false>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
     return;
   }
   const int64_t nw = n0 + g.wave_m * Cfg::WM + 4 * (g.lane >> 4);
 #pragma unroll
-  for (int j = 0; j < Cfg::NB; ++j) {
+  for (int j = 0; j < Cfg::NBN; ++j) {
     const int u = g.wave_n * Cfg::WN + j * 16 + (g.lane & 15);  // row inside the tile, in the operand's column order
     const int64_t m = m0 + (p.perm_rows ? (int64_t)KPerm<PermCfg>::vocab_at(u) : (int64_t)u);
     GemmCore16<Cfg>::stay_column(acc, j);
@@ -649,8 +654,9 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  typedef GemmCfg16<typename Cfg::TIN, 1> TnCfg;
+  typedef GemmCfg16<typename Cfg::TIN, 1, 8, 0, 1, 0, Cfg::NB> TnCfg;
   typedef GemmCore16<TnCfg> Core;
+  constexpr int TM = TnCfg::BN, TN = TnCfg::BM;  // a tile's rows and columns of C (MFMA rows = n, MFMA columns = m)
   if (p.k_dev) {
     // (at least two slabs, which the stream wants: token_prep_kernel, and beyond its range gather_rows_kernel, zeroes that many
     // rows of hidden, the d_logits pass those of dS)
@@ -660,7 +666,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   const int nk = (int)(p.K / 64);
   Core g;
   g.set_lane();
-  f32x4_t acc[Cfg::NB][Cfg::NB];
+  f32x4_t acc[TnCfg::NB][TnCfg::NBN];
   int bid = blockIdx.x, tm = 0, tn = 0;
   auto next_tile = [&]() {  // the first tile at or behind bid (uniform over the workgroup)
     for (; bid < p.map.total; bid += gridDim.x)
@@ -670,26 +676,26 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   if (!next_tile()) return;
   if (nk == 0) {  // no token takes part
     for (bool more = true; more; bid += gridDim.x, more = next_tile())
-      for (int q = threadIdx.x; q < Cfg::BM * (Cfg::BN / 8); q += Cfg::NTHREADS) {
-        const int64_t m = (int64_t)tm * Cfg::BM + q / (Cfg::BN / 8), n = (int64_t)tn * Cfg::BN + q % (Cfg::BN / 8) * 8;
+      for (int q = threadIdx.x; q < TM * (TN / 8); q += Cfg::NTHREADS) {
+        const int64_t m = (int64_t)tm * TM + q / (TN / 8), n = (int64_t)tn * TN + q % (TN / 8) * 8;
         if (m < p.M && n < p.N) *reinterpret_cast<u32x4_t*>(p.Ct + m * p.ldct + n) = u32x4_t{0u, 0u, 0u, 0u};
       }
     return;
   }
   typename Core::Stream s;
-  g.init_tn(p.B, p.ldb, (int64_t)tn * Cfg::BN, p.A, p.lda, (int64_t)tm * Cfg::BM, p.a_pcol);  // MFMA rows = n, MFMA columns = m
+  g.init_tn(p.B, p.ldb, (int64_t)tn * TN, p.A, p.lda, (int64_t)tm * TM, p.a_pcol);
   g.prologue(lds, p.K);
   g.stream_begin(lds, s);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
   bool behind = false, more = true;
   while (more) {
-    const int64_t m0 = (int64_t)tm * Cfg::BM, n0 = (int64_t)tn * Cfg::BN;
+    const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
     bid += gridDim.x;
     more = next_tile();
     const char *a_next = g.a_base, *b_next = g.b_base;
     if (more) {
-      a_next = reinterpret_cast<const char*>(p.B + (int64_t)tn * Cfg::BN);
-      b_next = reinterpret_cast<const char*>(p.a_pcol ? p.A + (int64_t)tm * (Cfg::BM / 64) * p.a_pcol : p.A + (int64_t)tm * Cfg::BM);
+      a_next = reinterpret_cast<const char*>(p.B + (int64_t)tn * TN);
+      b_next = reinterpret_cast<const char*>(p.a_pcol ? p.A + (int64_t)tm * (TM / 64) * p.a_pcol : p.A + (int64_t)tm * TM);
     }
     g.reads_tn(lane_anew());
     g.template stream_tile<32>(lds, nk, acc, s, a_next, b_next, behind);
@@ -698,7 +704,7 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
     const int free_slot = s.sb + 4 >= 5 ? s.sb + 4 - 5 : s.sb + 4;
     const uint32_t stage = lds0 + (uint32_t)(free_slot * TnCfg::STAGE_BYTES) + g.wave * 8192;
     __builtin_amdgcn_sched_barrier(0);
-    behind = m0 + Cfg::BM <= p.M && n0 + Cfg::BN <= p.N;
+    behind = m0 + TM <= p.M && n0 + TN <= p.N;
     if (behind) gemm16_store_lines<TnCfg, Cfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
     else gemm16_store_lines<TnCfg, Cfg, false>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
     __builtin_amdgcn_sched_barrier(0);
@@ -850,24 +856,25 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typena
     p.cf_split_stride = DhSlices::stride(rows, p.N);
     p.map.ncol_tiles = p.n_tiles * p.ksplit;
   }
-  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY, 1, Cfg::A_ONCE>>(p, blockIdx.x, lds);
+  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY, 1, Cfg::A_ONCE, Cfg::NB>>(p, blockIdx.x, lds);
 }
 
-template <typename Cfg>
+// a tile of d_weight (p.tn == 1) or of d_hidden, NBM blocks of hidden columns to a wave
+template <typename Cfg, int NBM>
 LCE_DEV void any_gemm16_tile(const GemmArgs<typename Cfg::TIN>& p, int bid, char* lds) {
-  if (p.tn == 1) gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1, 8, 0, Cfg::TERMS>, Cfg>(p, bid, lds);
+  typedef typename Cfg::TIN TIN;
+  if (p.tn == 1) gemm16_tn_tile<GemmCfg16<TIN, 1, 8, 0, Cfg::TERMS, 0, NBM>, Cfg>(p, bid, lds);
   // (W early: the whole step 0.2 to 0.5 % faster from 2048 to 16384 tokens)
-  else if (p.tn == 2) gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, 8, 1, Cfg::TERMS>>(p, bid, lds);
-  else gemm16_tile<Cfg>(p, bid, lds);
+  else gemm16_tile<GemmCfg16<TIN, 0, 8, 0, Cfg::TERMS, 0, NBM>, GemmCfg16<TIN, 2, 8, 1, Cfg::TERMS, 0, NBM>>(p, bid, lds);
 }
 
 // one launch of the backward's steady state (see lce_bwd_chunk_kernel)
-template <typename Cfg>
+template <typename Cfg, int NBM>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_bwd_chunk16_kernel(BwdChunkArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int bid = blockIdx.x;
-  if (bid < p.n_gw) any_gemm16_tile<Cfg>(p.gw, bid, lds);
-  else if (bid < p.n_gw + p.n_gh) any_gemm16_tile<Cfg>(p.gh, bid - p.n_gw, lds);
+  if (bid < p.n_gw) any_gemm16_tile<Cfg, NBM>(p.gw, bid, lds);
+  else if (bid < p.n_gw + p.n_gh) any_gemm16_tile<Cfg, NBM>(p.gh, bid - p.n_gw, lds);
   else ds16_tile<Cfg>(p.ds, bid - p.n_gw - p.n_gh, lds);
 }
 

@@ -217,7 +217,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   if ((rc = check_launch("fill_zero_kernel"))) return rc;
   const SplitArgs sh = {h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows};
   if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
-  const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN);
+  const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN), h_tile = hidden_tile(H);
   // launch c: d_logits of chunk c and the gradient GEMMs of chunk c - 1, as in backward_impl
   for (int c = 0; c <= L.nchunks; ++c) {
     BwdChunkArgs<bf16_t> p;
@@ -243,7 +243,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
       const int64_t v0 = (int64_t)cc * L.vchunk, vrows = std::min(L.vchunk, V - v0);
       const int64_t kc = round_up(vrows, KPerm<Cfg>::GV);
       if (need_dh) {
-        p.gh = make_gemm_args<Cfg>(dS[cc & 1], 64, w3[cc & 1], 3 * H, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1);
+        p.gh = make_gemm_args<Cfg>(dS[cc & 1], 64, w3[cc & 1], 3 * H, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1, h_tile);
         p.gh.tn = 2; p.gh.b_rows_valid = vrows; p.gh.m_dev = n_rows;
         p.gh.a_pcol = L.pcol; p.gh.a_plane = L.plane * 2; p.gh.b_plane = H * 2;
         if (L.ksplit > 1) {
@@ -255,7 +255,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
         p.n_gh = p.gh.map.total;
       }
       if (need_dw) {
-        p.gw = make_gemm_args<Cfg>(dS[cc & 1], 64, h3, 3 * L.ldH, vrows, H, round_up(T, 64), d_weight + v0 * H, H, nullptr, 0, 0);
+        p.gw = make_gemm_args<Cfg>(dS[cc & 1], 64, h3, 3 * L.ldH, vrows, H, round_up(T, 64), d_weight + v0 * H, H, nullptr, 0, 0, h_tile);
         p.gw.tn = 1; p.gw.perm_rows = 1; p.gw.k_dev = n_rows; p.gw.k_gran = 64;
         p.gw.a_pcol = L.pcol; p.gw.a_plane = L.plane * 2; p.gw.b_plane = L.ldH * 2;
         p.n_gw = p.gw.map.total;
@@ -270,8 +270,9 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
       }
     }
     ProfScope prof(PC_BWD_CHUNK, st);
-    allow_lds(lce_bwd_chunk16_kernel<Cfg>, Cfg::LDS_BYTES);
-    hipLaunchKernelGGL(lce_bwd_chunk16_kernel<Cfg>, dim3(p.n_gw + p.n_gh + p.n_ds), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
+    auto kern = h_tile == 224 ? lce_bwd_chunk16_kernel<Cfg, 7> : lce_bwd_chunk16_kernel<Cfg, 8>;
+    allow_lds(kern, Cfg::LDS_BYTES);
+    hipLaunchKernelGGL(kern, dim3(p.n_gw + p.n_gh + p.n_ds), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
     if ((rc = check_launch("lce_bwd_chunk16_kernel"))) return rc;
   }
   if (need_dh) {
