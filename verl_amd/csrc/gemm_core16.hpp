@@ -57,8 +57,8 @@ LCE_DEV void static_for(std::integer_sequence<int, Is...>, F&& f) {
 // row of tiles (ragged token counts: less work for padding; the loop itself runs a few per cent below the square tile's rate).
 // A_EARLY_: the ring's early operand (see main) is A instead of B.
 // TERMS_: products per slab.  1: the operands are what they are.  6: fp32 operands, each held as three bfloat16 planes
-// x = x1 + x2 + x3 (exact: 3 x 8 significant bits); a slab is multiplied as a1 b1 + a1 b2 + a2 b1 + a1 b3 + a3 b1 + a2 b2 into
-// the same fp32 accumulators.  What is left out, a2 b3 + a3 b2 + a3 b3, is below 2^-26 of |a b|, a quarter of what rounding
+// x = x1 + x2 + x3 (exact: 3 x 8 significant bits); a slab is multiplied as a1 b3 + a1 b2 + a2 b2 + a2 b1 + a1 b1 + a3 b1 into
+// the same fp32 accumulators (main6).  What is left out, a2 b3 + a3 b2 + a3 b3, is below 2^-26 of |a b|, a quarter of what rounding
 // ONE fp32 product or partial sum costs, and the products themselves are exact.  Six bfloat16 MFMAs take six sixteenths
 // of the matrix pipe's time of the fp32 one.
 // A_ONCE_: the loads of A are marked non-temporal (A is read once, or nearly, and larger than the caches).
@@ -238,21 +238,14 @@ struct GemmCore16 {
   // load j of one operand's half slab number `ks` into ring slot `slot`
   LCE_DEV void dma(char* lds, int slot, int64_t ks, bool is_b, int j) const {
     char* dst = lds + slot * SLOT + (j * Cfg::NW + wave) * 1024;
-    int64_t plane = 0;
-    if constexpr (Cfg::TERMS == 6) {
-      // product number ks % 6 of slab ks / 6: planes (a, b) = (0,0) (0,1) (1,0) (0,2) (2,0) (1,1), two bits each
-      const int n = (int)ks, slab = n / 6, t = 2 * (n - 6 * slab);
-      plane = is_b ? ((0x484 >> t) & 3) * b_plane : ((0x610 >> t) & 3) * a_plane;
-      ks = slab;
-    }
     const char* src;
     if (Cfg::TRANS == 2 && !is_b) {
       // slabs with rows that do not exist take the last slab that has any, with its rows clamped (branch-free: the
       // hand-placed schedule of a k-step must stay one basic block)
       const bool tail = ks >= a_ks_full;
-      src = a_base + (tail ? a_ks_last : ks) * a_slab + plane + (tail ? va_tail[j] : va[j]);
+      src = a_base + (tail ? a_ks_last : ks) * a_slab + (tail ? va_tail[j] : va[j]);
     } else {
-      src = (is_b ? b_base + ks * b_slab + plane + vb[j] : a_base + ks * a_slab + plane + va[j]);
+      src = (is_b ? b_base + ks * b_slab + vb[j] : a_base + ks * a_slab + va[j]);
     }
     if (Cfg::A_ONCE && !is_b) __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, kBufNonTemporal);  // (constants after inlining)
     else __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
@@ -267,8 +260,10 @@ struct GemmCore16 {
   // ra / rb: LDS address of the slot plus a_rd / b_rd; S: k-step inside the slab
   template <int F, int S>
   LCE_DEV void read_frag(uint32_t ra, uint32_t rb, u32x4_t (&af)[NB], u32x4_t (&bf)[NBN]) const {
-    constexpr bool is_a = frag_is_a(F);
-    constexpr int blk = frag_blk(F);
+    read_block<frag_is_a(F), frag_blk(F), S>(ra, rb, af, bf);
+  }
+  template <bool is_a, int blk, int S>
+  LCE_DEV void read_block(uint32_t ra, uint32_t rb, u32x4_t (&af)[NB], u32x4_t (&bf)[NBN]) const {
     u32x4_t v;
     if constexpr (is_a ? TA : TB) {
       // block: 16 columns = 32 bytes further, inside the swizzled chunk bits; k-step: 32 rows; second half: 4 rows
@@ -332,7 +327,15 @@ struct GemmCore16 {
   // Issues the loads of the first two slabs (half slabs E0 L0 E1 L1 into slots 0..3; E = the early operand).  LDS must be
   // free: every wave past its last read of the previous tile and its own loads drained (a workgroup barrier after main()).
   LCE_DEV void prologue(char* lds, int64_t K) const {
-    const int64_t last = K / Cfg::BK * Cfg::TERMS - 1;
+    if constexpr (Cfg::TERMS == 6) {
+      fetch6<true>(lds, 0, 0, 2);
+      fetch6<false>(lds, 1, 0, 0);
+      fetch6<true>(lds, 2, 0, 1);
+      fetch6<false>(lds, 3, 0, 1);
+      fetch6<true>(lds, 4, 0, 0);
+      return;
+    }
+    const int64_t last = K / Cfg::BK - 1;
 #pragma unroll
     for (int hf = 0; hf < 4; ++hf) {
       const int64_t ks = hf / 2 < last ? hf / 2 : last;
@@ -350,7 +353,8 @@ struct GemmCore16 {
   // a half to arrive and L one slab.  Past the end
   // of K the loader re-fetches the last slab into slots nobody reads (a branch-free body), drained at the end.
   LCE_DEV void main(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {
-    const int nk = (int)(K / Cfg::BK) * Cfg::TERMS;
+    if constexpr (Cfg::TERMS == 6) return main6(lds, (int)(K / Cfg::BK), acc);
+    const int nk = (int)(K / Cfg::BK);
     const int64_t last = nk - 1;
     wait_vm<HL + HLB>();  // slab 0 has landed
     __builtin_amdgcn_s_barrier();
@@ -381,6 +385,134 @@ struct GemmCore16 {
     for (int it = 1; it < nk; ++it) slab(std::false_type{}, it);
     wait_vm<0>();    // drain the redundant tail fetches before LDS is reused
     wait_lgkm<0>();  // and the reads of the slab after the last
+    retire(acc);
+  }
+
+  // ---- TERMS == 6: a slab's six products -----------------------------------------------------------------------
+  // Consecutive products share an operand: a1 b3, a1 b2, a2 b2, a2 b1, a1 b1, a3 b1.  Its fragments stay in registers, so that a
+  // slab of K is seven half slabs read from LDS (a1 twice) and six fetched, where products that each bring both operands are
+  // twelve and twelve.  What that saves is energy: on such data the loop runs at the socket's power cap.  Against products that each
+  // bring both, H=896: 1024 tokens, forward 1422 -> 1287 us, forward + backward 5.84 -> 5.09 ms; 400 tokens 749 and 2761 for 806 and 2995;
+  // H=5120, 1000 tokens, forward 7.83 -> 7.00 ms.
+  // The fragments a k-step reads for the next one, WHAT: 1 of A, 2 of B, 3 both in kstep's order.
+  template <int WHAT>
+  struct Reads {
+    static constexpr int N = WHAT == 3 ? NF : WHAT == 1 ? NB : NBN;
+    static constexpr bool is_a(int f) { return WHAT == 3 ? frag_is_a(f) : WHAT == 1; }
+    static constexpr int blk(int f) { return WHAT == 3 ? frag_blk(f) : f; }
+    static constexpr int upto(int f) { return f < 0 ? 0 : WHAT == 3 ? GemmCore16::upto(f) : (f + 1) * (WHAT == 1 ? CA : CB); }
+    static constexpr int before(int m) { return (m + 1) / 2 > N ? N : (m + 1) / 2; }
+    // the last fragment that MFMA (i, j) is the first to depend on; -1: none
+    static constexpr int need(int i, int j) {
+      return WHAT == 3 ? (i == 0 ? 1 + j : j == 0 ? NBN + i : -1) : WHAT == 1 ? (j == 0 ? i : -1) : (i == 0 ? j : -1);
+    }
+  };
+  // half slab `ks` of plane `which`, its address in scalar registers (the compiler otherwise keeps the planes' addresses per lane)
+  struct Half6 {
+    const char* base;
+    bool tail;
+  };
+  template <bool IS_B>
+  LCE_DEV Half6 half6(int ks, int which) const {
+    const bool tail = Cfg::TRANS == 2 && !IS_B && ks >= a_ks_full;
+    Half6 h = {IS_B ? b_base + ks * b_slab + which * b_plane : a_base + (tail ? a_ks_last : ks) * a_slab + which * a_plane, tail};
+    asm volatile("" : "+s"(h.base));
+    return h;
+  }
+  template <bool IS_B>
+  LCE_DEV void load6(char* lds, int slot, Half6 h, int j) const {
+    const uint32_t at = IS_B ? vb[j < HLB ? j : 0] : Cfg::TRANS == 2 && h.tail ? va_tail[j] : va[j];
+    __builtin_amdgcn_global_load_lds((gptr_t)(h.base + at), (lptr_t)(lds + slot * SLOT + (j * Cfg::NW + wave) * 1024), 16, 0, 0);
+  }
+  template <bool IS_B>
+  LCE_DEV void fetch6(char* lds, int slot, int ks, int which) const {
+    const Half6 h = half6<IS_B>(ks, which);
+#pragma unroll
+    for (int j = 0; j < (IS_B ? HLB : HL); ++j) load6<IS_B>(lds, slot, h, j);
+  }
+
+  // One k-step.  CUR: what was read for it during the step before and may still be in flight (0: nothing).  NEXT: what is read for
+  // the next one, k-step S_N of its product.  LOAD: 1 / 2: the half slab `from` of A / B is fetched into `slot`.
+  template <int CUR, int NEXT, int S_N, int LOAD, bool FIRST = false>
+  LCE_DEV void kstep6(f32x4_t (&acc)[NB][NBN], const u32x4_t (&af)[NB], const u32x4_t (&bf)[NBN], uint32_t ra_n, uint32_t rb_n,
+                      u32x4_t (&af_n)[NB], u32x4_t (&bf_n)[NBN], char* lds = nullptr, int slot = 0, Half6 from = {}) const {
+    typedef Reads<NEXT> Nx;
+    constexpr int LOADS = LOAD == 1 ? HL : HLB, EVERY = NB * NBN / LOADS;
+    static_assert(2 * NF <= NB * NBN && EVERY > 3, "one fragment read after every second MFMA");
+    static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      constexpr int i = m / NBN, j = m % NBN;
+      if constexpr (CUR != 0) {
+        typedef Reads<CUR> Cu;
+        if constexpr (Cu::need(i, j) >= 0) {
+          constexpr int allow = Cu::upto(Cu::N - 1) - Cu::upto(Cu::need(i, j)) + Nx::upto(Nx::before(m) - 1);
+          wait_lgkm<(allow > 15 ? 15 : allow)>();
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FIRST) Mma16<TIN>::first(acc[i][j], af[i], bf[j]);
+      else Mma16<TIN>::run(acc[i][j], af[i], bf[j]);
+      if constexpr ((m & 1) == 0 && m / 2 < Nx::N) read_block<Nx::is_a(m / 2), Nx::blk(m / 2), S_N>(ra_n, rb_n, af_n, bf_n);
+      if constexpr (LOAD != 0 && m % EVERY == 3 && m / EVERY < LOADS) load6<LOAD == 2>(lds, slot, from, m / EVERY);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  // Half slabs are fetched in the order b3 a1 b2 a2 b1 | a3 b3' a1' b2' a2' b1' | ..., each into the slot that the product before
+  // has read for the last time (behind the barrier between a product's two k-steps), three to four products ahead of its own
+  // first read.  The waits count the loads behind the half slab that the next product is the first to read.
+  LCE_DEV void main6(char* lds, int nk, f32x4_t (&acc)[NB][NBN]) const {
+    const int last = nk - 1;
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    wait_vm<2 * HLB + HL>();
+    __builtin_amdgcn_s_barrier();
+    u32x4_t af[2][NB], bf[2][NBN];
+    static_for(std::make_integer_sequence<int, NF>{}, [&](auto fc) {
+      read_frag<decltype(fc)::value, 0>(lds0 + SLOT + a_rd, lds0 + b_rd, af[0], bf[0]);
+    });
+    int b3 = 0, a1 = 1, b2 = 2, a2 = 3, b1 = 4;  // slots; a3 follows b3
+    auto meet = [&](auto in_flight) {  // every wave's loads but so many have landed, every wave's reads have returned
+      constexpr int N = decltype(in_flight)::value;
+      if constexpr (N >= 0) wait_vm<N>();
+      wait_lgkm<0>();
+      __builtin_amdgcn_s_barrier();
+    };
+    constexpr std::integral_constant<int, HL + HLB> two{};
+    constexpr std::integral_constant<int, HL + 2 * HLB> three{};
+    constexpr std::integral_constant<int, -1> all_here{};
+    auto slab = [&](auto first, int it) {
+      constexpr bool FIRST = decltype(first)::value;
+      const int nx = it < last ? it + 1 : last;  // (past the end the last slab is fetched once more, into slots nobody reads)
+      auto ra = [&](int slot) { return lds0 + slot * SLOT + a_rd; };
+      auto rb = [&](int slot) { return lds0 + slot * SLOT + b_rd; };
+      kstep6<3, 3, 1, 0, FIRST>(acc, af[0], bf[0], ra(a1), rb(b3), af[1], bf[1]);  // a1 b3
+      meet(two);                                                                  // (b2)
+      kstep6<0, 2, 0, 1>(acc, af[1], bf[1], 0, rb(b2), af[0], bf[0], lds, b3, half6<false>(it, 2));
+      kstep6<2, 2, 1, 0>(acc, af[0], bf[0], 0, rb(b2), af[1], bf[1]);  // a1 b2
+      meet(two);                                                      // (a2)
+      kstep6<0, 1, 0, 2>(acc, af[1], bf[1], ra(a2), 0, af[0], bf[0], lds, b2, half6<true>(nx, 2));
+      kstep6<1, 1, 1, 0>(acc, af[0], bf[0], ra(a2), 0, af[1], bf[1]);  // a2 b2
+      meet(two);                                                      // (b1)
+      kstep6<0, 2, 0, 1>(acc, af[1], bf[1], 0, rb(b1), af[0], bf[0], lds, a2, half6<false>(nx, 0));
+      kstep6<2, 2, 1, 0>(acc, af[0], bf[0], 0, rb(b1), af[1], bf[1]);  // a2 b1
+      meet(all_here);
+      kstep6<0, 1, 0, 2>(acc, af[1], bf[1], ra(a1), 0, af[0], bf[0], lds, b1, half6<true>(nx, 1));
+      kstep6<1, 1, 1, 0>(acc, af[0], bf[0], ra(a1), 0, af[1], bf[1]);  // a1 b1
+      meet(three);                                                    // (a3)
+      kstep6<0, 1, 0, 1>(acc, af[1], bf[1], ra(b3), 0, af[0], bf[0], lds, a1, half6<false>(nx, 1));
+      kstep6<1, 1, 1, 0>(acc, af[0], bf[0], ra(b3), 0, af[1], bf[1]);  // a3 b1
+      meet(two);                                                      // (b3', a1')
+      kstep6<0, 3, 0, 2>(acc, af[1], bf[1], ra(a2), rb(b2), af[0], bf[0], lds, b3, half6<true>(nx, 0));
+      const int was_b3 = b3, was_a1 = a1;
+      b3 = b2;
+      b2 = b1;
+      b1 = was_b3;
+      a1 = a2;
+      a2 = was_a1;
+    };
+    slab(std::true_type{}, 0);
+    for (int it = 1; it < nk; ++it) slab(std::false_type{}, it);
+    wait_vm<0>();
+    wait_lgkm<0>();
     retire(acc);
   }
 
