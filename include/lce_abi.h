@@ -114,8 +114,10 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  * tokens and H=3584, 57 % at 1024), and keeping it saves the backward its pass over the weight and its T x V x H product
  * for the logits (64 tokens, H=3584, V=152064: 39 MB kept, 1.09 GB not read; 1024 tokens: a quarter of the matrix work).
  *   lce_logits_cache_max_tokens: the largest T for which a cache is offered: H / 2 for 16-bit inputs (the
- *     cache never exceeds the weight), or LCE_OPT_KEEP_LOGITS_TOKENS where that is lower; 0 for fp32 inputs and under diagnostic settings that force a tile variant.
- *   lce_logits_cache_bytes: size of the buffer for this shape, or 0 when T is beyond that: then pass NULL below.
+ *     cache never exceeds the weight), 4 H for LCE_DTYPE_F32_PLANES where the planes are used (of all rows of the weight up to H tokens,
+ *     beyond of as many of the first as are no larger than the weight), or LCE_OPT_KEEP_LOGITS_TOKENS where that is lower; 0 for
+ *     LCE_DTYPE_F32 and under diagnostic settings that force a tile variant.
+ *   lce_logits_cache_bytes: size of the buffer for this shape, or 0 where none is offered: then pass NULL below.
  *   lce_forward_keep_logits: lce_forward; with logits_cache != NULL it also writes hidden . weight^T there in fp32
  *     (private layout).  Same outputs, bit for bit.
  *   lce_backward_from_logits: lce_backward (grads_fp32 = 0) or lce_backward_f32 (grads_fp32 = 1; d_hidden, d_weight are
@@ -301,7 +303,7 @@ int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
  * with hidden . W[label] recomputed per token) is kept out of the tiles and added in fp32.  Changes the workspace size:
  * set it before querying lce_backward_workspace_bytes.
  * LCE_OPT_KEEP_LOGITS_TOKENS (default LCE_KEEP_LOGITS_NO_LIMIT; any count >= 0): the token count up to which
- * lce_logits_cache_bytes offers a cache, next to its own bound of H / 2 tokens; 0 makes every backward recompute its
+ * lce_logits_cache_bytes offers a cache, next to its own bounds; 0 makes every backward recompute its
  * logits, as the reference does at every size. */
 #define LCE_KEEP_LOGITS_NO_LIMIT ((int64_t)1 << 40)
 enum {

@@ -618,7 +618,7 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// d_logits of a vocabulary chunk from logits that the forward kept (tokens up to half the hidden size): what the
+// d_logits of a vocabulary chunk, or of its first rows, from logits that the forward kept (FwdArgs::xcache): what the
 // d_logits tiles compute from their accumulators, here from the kept x(t, v), element by element with the same
 // expressions, so the same bits.  One pass over 4 bytes per logit instead of a pass over W.  Workgroup b owns the 64
 // columns [64 b, 64 b + 64) of dS, which lie within one group of the vocabulary order Perm (a whole group of the
@@ -632,9 +632,10 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_kernel(FewArgs<TIN> p) {
 // table (worked out per workgroup they were six dependent loads and a logarithm per position) and four positions are on
 // their way at once.
 // p: the chunk's DsArgs (W, h, the tile map and the range are not used); x: the kept logits from the chunk's first row
-// on (a multiple of 16), of xtok tokens.
+// on (a multiple of 16), of xtok tokens.  TERMS == 6: d_logits in three planes, 10 bytes moved per logit; 25344 columns of 1024
+// tokens 51 us, 5.1 TB/s.
 // ------------------------------------------------------------------------------------------------------------------
-template <typename TIN, typename Perm>
+template <typename TIN, typename Perm, int TERMS = 1>
 __global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, const float* x, int64_t xtok, int nrows, bool exact) {
   static_assert(sizeof(TIN) == 2 && Perm::GV % 64 == 0, "16-bit d_logits, groups of the vocabulary order in multiples of 64 rows");
   constexpr int U = 4;
@@ -683,7 +684,10 @@ __global__ __launch_bounds__(256) void ds_from_logits_kernel(DsArgs<TIN> p, cons
         const bool dead = tok[u] < 0 || g0 + row >= p.vrows;
         d[e] = dlogit<true>(dead ? 0.f : v[u][e >> 2][e & 3], p.c, k[u][0], k[u][1], k[u][2], k[u][3], row == rel[u], dead, p.label_outside == 2);
       }
-      if (pos < end) store_run<TIN, 8>(ds_at(p.dS, p.ldS, p.pcol, pos, u0 + c * 8), d);
+      if (pos >= end) continue;
+      TIN* dst = ds_at(p.dS, p.ldS, p.pcol, pos, u0 + c * 8);
+      if constexpr (TERMS == 6) store_planes<TIN, 8>(dst, p.dS_plane, d);
+      else store_run<TIN, 8>(dst, d);
     }
   }
 }

@@ -246,22 +246,24 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   if (terms) sel = kSelTerms;
-  if (xcache && sel != kSelT64 && sel != kSelT128 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
+  if (xcache && !terms && sel != kSelT64 && sel != kSelT128 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
                          accumulate, entropy_b, ws, workspace_bytes, st, label_offset, shard_out, max_splits, xcache);
 }
 
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype) {
-  if (!known_dtype(dtype) || H <= 0) return 0;
+  const bool planes = dtype == LCE_DTYPE_F32_PLANES;
+  if (!(known_dtype(dtype) || planes) || H <= 0) return 0;
   const Tuning tu = tuning_snapshot();
   if (tu.variant_forced) return 0;  // (a forced tile variant may be one that cannot write the cache)
-  const int64_t most = logits_cache_max_tokens(H, esize(dtype));
+  const int64_t most = planes ? kTermsKeepTokens * H : logits_cache_max_tokens(H, esize(dtype));
   return most < tu.keep_logits_tokens ? most : tu.keep_logits_tokens;
 }
 
 size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
   if (V <= 0 || T < 1 || T > lce_logits_cache_max_tokens(H, dtype)) return 0;
+  if (dtype == LCE_DTYPE_F32_PLANES) return terms_cache_bytes(tuning_snapshot(), T, H, V);
   return (size_t)T * (size_t)logits_cache_row(V) * 4;
 }
 
@@ -270,7 +272,7 @@ int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight,
                             float* maximum, float* accumulate, float* entropy_b, void* workspace, size_t workspace_bytes,
                             void* logits_cache, size_t logits_cache_bytes, void* stream) {
   if (logits_cache) {
-    const size_t need = known_dtype(dtype) ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
+    const size_t need = known_dtype(dtype) || dtype == LCE_DTYPE_F32_PLANES ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
     if (need == 0) return fail(LCE_E_ARG, "lce_forward_keep_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");
@@ -407,7 +409,7 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
   char* ws = reinterpret_cast<char*>(align256(reinterpret_cast<size_t>(workspace)));
   return kBackward[dtype](terms ? kSelTerms : esz == 4 && few_f32(tu, T) ? kSelFewF32 : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
                           accumulate, entropy_b, dlogprobs, dentropy, d_hidden, d_weight, grads_f32, ws, vchunk, st, vocab_offset,
-                          tu, xcache);
+                          tu, planes && !terms ? nullptr : xcache);
 }
 
 int lce_backward_from_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,
@@ -416,7 +418,9 @@ int lce_backward_from_logits(const void* hidden, int64_t ldh, const void* weight
                              void* d_hidden, void* d_weight, int grads_fp32, void* workspace, size_t workspace_bytes, int64_t vchunk,
                              const void* logits_cache, size_t logits_cache_bytes, void* stream) {
   if (logits_cache) {
-    const size_t need = known_dtype(dtype) ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
+    // (a cache on planes was written under what was set then: nothing set since changes its size, at most whether it is read)
+    const size_t need = dtype == LCE_DTYPE_F32_PLANES ? (T > 0 && H > 0 && V > 0 ? terms_cache_bytes(Tuning(), T, H, V) : 0)
+                        : known_dtype(dtype)          ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
     if (need == 0) return fail(LCE_E_ARG, "lce_backward_from_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");

@@ -62,7 +62,7 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
       LCE_FEW(128);
     case kSelTerms:
       return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws,
-                           ws_bytes, st, label_offset, shard_out);
+                           ws_bytes, st, label_offset, shard_out, xcache);
 #endif
   }
 #undef LCE_FEW
@@ -96,7 +96,7 @@ int TU_FN(backward)(int sel, LCE_BWD_PARAMS) {
 #if LCE_TU_DTYPE == 1
     case kSelTerms:
       return backward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
-                            (float*)dw, ws, vchunk, st, vocab_offset, tu);
+                            (float*)dw, ws, vchunk, st, vocab_offset, tu, xcache);
     case kSelFewF32:
       return backward_few_f32((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
                               (float*)dw, ws, vchunk, st, vocab_offset, tu);

@@ -53,9 +53,10 @@ struct FwdArgs {
   int64_t split_stride, tile_step, split_span;
   TileMap map;       // rows = token tiles, cols = splits
   int64_t label_offset;  // W holds vocabulary rows [label_offset, label_offset + V) of a larger vocabulary (0 = all of it)
-  // When not null (offered while the tokens are at most half the hidden size), the raw logits h . W[v] (fp32, before the division by the
+  // When not null (offered while they are no larger than the weight), the raw logits h . W[v] (fp32, before the division by the
   // temperature) are kept for the backward: logit (t, v) at kept_logit(xcache, T, t, v).
   float* xcache;
+  int64_t keep_rows;  // operands in planes: of the first so many rows of W only (V, or a multiple of the tile's rows)
   int64_t w_plane, h_plane;  // W and h in bfloat16 planes (GemmCfg16, TERMS == 6): bytes from plane to plane
   int64_t once_rows;  // up to 96 tokens: workgroups whose rows start before this one read W with non-temporal loads
 };
@@ -470,6 +471,20 @@ LCE_DEV void store_run(T* dst, const float (&v)[N]) {
     for (int e = 0; e < PER; ++e) out[e] = round_to<T>(v[k + e]);
     if (STREAM) __builtin_nontemporal_store(out, reinterpret_cast<vec_t*>(dst + k));
     else *reinterpret_cast<vec_t*>(dst + k) = out;
+  }
+}
+
+// N fp32 values as the three terms whose sum they are (GemmCfg16, TERMS == 6), `plane` elements from term to term
+template <typename T, int N>
+LCE_DEV void store_planes(T* dst, int64_t plane, const float (&v)[N]) {
+  float rest[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) rest[q] = v[q];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    store_run<T, N>(dst + t * plane, rest);
+#pragma unroll
+    for (int q = 0; q < N; ++q) rest[q] -= (float)(T)rest[q];
   }
 }
 

@@ -164,7 +164,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
       g.main(lds, p.H, acc);
       const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
       const bool full = m0 + Cfg::BM <= vend64;
-      if constexpr (KEEP) {
+      if (KEEP && (Cfg::TERMS == 1 || m0 < p.keep_rows)) {
         // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.  Issued AHEAD of the next
         // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
         // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are issued two
@@ -172,8 +172,9 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
         // prologue's loads behind them fewer than 64 operations are ever in flight (8 stores a column, 12 where the compiler gives
         // lanes without a token a store of their own; tests/test_ring_loads_on_cpu.py counts them on the listing).
         // Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
-        constexpr int kColumn = NB + NB / 2, kBehindLast = 24, kBetween = 32;
-        static_assert(kBetween + 2 * kColumn < 64 && 4 * kColumn < 64 && kBehindLast + 2 * (Cfg::HL + Cfg::HLB) < 64, "vmcnt range");
+        constexpr int kColumn = NB + NB / 2, kBehindLast = Cfg::TERMS == 6 ? 16 : 24, kBetween = 32;
+        constexpr int kPrologue = Cfg::TERMS == 6 ? 2 * Cfg::HL + 3 * Cfg::HLB : 2 * (Cfg::HL + Cfg::HLB);
+        static_assert(kBetween + 2 * kColumn < 64 && 4 * kColumn < 64 && kBehindLast + kPrologue < 64, "vmcnt range");
         const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
         // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
         const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
@@ -291,19 +292,8 @@ LCE_DEV void ds16_epilogue(const DsArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cf
       }
       // rows of positions without a token are zeros (their constants make them so); they pad the d_weight GEMM's K
       TIN* dst = ds_at(p.dS, p.ldS, p.pcol, tok, vloc0 + ip * 32 + g4 * 8);
-      if constexpr (Cfg::TERMS == 6) {
-        float rest[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) rest[q] = d[q];
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-          store_run<TIN, 8>(dst + t * p.dS_plane, rest);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) rest[q] -= (float)(TIN)rest[q];
-        }
-      } else {
-        store_run<TIN, 8>(dst, d);
-      }
+      if constexpr (Cfg::TERMS == 6) store_planes<TIN, 8>(dst, p.dS_plane, d);
+      else store_run<TIN, 8>(dst, d);
     }
   }
 }

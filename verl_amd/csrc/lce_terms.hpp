@@ -2,7 +2,7 @@
 // multiplied as six products of planes (GemmCfg16, TERMS == 6).  The fp32 MFMA runs at 157 TFLOP/s dense, the bfloat16 one
 // at 2.5 PFLOP/s; six products for one leave 2.5 times the rate at the clocks both reach, against which stand the passes
 // that make the planes (10 bytes per element of W, forward and backward each).  Measured, fp32 MFMA / planes: H=896,
-// V=151936, 1024 tokens forward + backward 9.90 / 5.09 ms, 2000 tokens forward 4.11 / 2.23, 400 tokens forward 1.09 / 0.75;
+// V=151936, 1024 tokens forward + backward 9.90 / 4.67 ms (logits kept), 2000 tokens forward 4.11 / 2.23, 400 tokens forward 1.09 / 0.75;
 // H=5120, 1500 tokens, half with gradient 56.6 / 26.8.  Error against float64 (2-norm, relative; H=896, V=151936, 2000 tokens):
 // log-probs 7.7e-8 / 7.2e-8, entropies 5.9e-8 / 5.6e-8, d_hidden 1.0e-6 / 5.9e-7, d_weight 7.9e-7 / 4.1e-7: the products are
 // exact and a sixteenth as many partial sums are rounded.
@@ -124,6 +124,17 @@ bool use_terms(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
   return (double)terms_bwd_layout(Tuning(), T, H, V, 0).total + 512.0 <= (double)T * V + 4.0 * (double)V * H;
 }
 
+// Kept logits (see logits_cache_max_tokens) of a call on planes: of the first rows of W, as many as are no larger than the weight,
+// T * rows * 4 <= V * H * 4: all up to H tokens.  Offered up to 4 H tokens, where they are a quarter of the rows and save 2 %: a kept
+// logit is 4 bytes written and read once, a recomputed one 12 H operations, whatever T is.  Forward + backward, recomputed / kept,
+// us: H=896, 300 tokens 2620 / 2182, 600: 3868 / 3241, 1024: 5220 / 4674 (7/8 of the rows), 2000: 9480 / 8901, 3500: 16327 / 16031;
+// H=3584, 300: 10591 / 8015; H=4096, 2000: 33872 / 27158; d_hidden alone H=5120, 1500: 30957 / 21076.
+constexpr int64_t kTermsKeepTokens = 4;  // times H
+int64_t terms_kept_rows(int64_t T, int64_t H, int64_t V) { return T <= H ? V : V * H / T / 256 * 256; }
+size_t terms_cache_bytes(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
+  return T <= kTermsKeepTokens * H && use_terms(tu, T, H, V) ? (size_t)T * (size_t)logits_cache_row(terms_kept_rows(T, H, V)) * 4 : 0;
+}
+
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1
 typedef GemmCfg16<bf16_t, 0, 8, 0, 6> TermsCfg;
 
@@ -142,7 +153,7 @@ int launch_split(const SplitArgs& s, const SplitArgs* also, int* wide, hipStream
 #if LCE_TU_PART == 0
 int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                   int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, size_t ws_bytes,
-                  hipStream_t st, int64_t label_offset, float* shard_out) {
+                  hipStream_t st, int64_t label_offset, float* shard_out, float* xcache) {
   const TermsFwdPlan pl = terms_fwd_plan(T, H, V, ws_bytes);
   bf16_t* h3 = reinterpret_cast<bf16_t*>(ws + pl.off_h);
   bf16_t* w3 = reinterpret_cast<bf16_t*>(ws + pl.off_w);
@@ -158,7 +169,8 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
   p.w_plane = p.h_plane = H * 2;
   p.c = kLog2e / temperature;
   p.xlabel = reinterpret_cast<float*>(ws + pl.off_xlabel);
-  p.xcache = nullptr; p.once_rows = 0;
+  p.once_rows = 0;
+  const int64_t kept = xcache ? terms_kept_rows(T, H, V) : 0;
   f32x4_t* parts = reinterpret_cast<f32x4_t*>(ws);
   int done = 0;
   for (int c = 0; c < pl.nchunks; ++c) {
@@ -170,9 +182,12 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
     p.parts = parts + (int64_t)done * T;
     p.split_stride = TermsCfg::BM; p.tile_step = (int64_t)p.S * TermsCfg::BM; p.split_span = rows;
     p.map = TileMap::make(ntt, p.S, block_rows(ntt), 1);
+    p.keep_rows = std::min(rows, kept - v0);
+    p.xcache = p.keep_rows > 0 ? xcache + v0 * T : nullptr;
     ProfScope prof(PC_FWD, st);
-    allow_lds((lce_fwd16_kernel<TermsCfg, false>), TermsCfg::LDS_BYTES);
-    hipLaunchKernelGGL((lce_fwd16_kernel<TermsCfg, false>), dim3(p.map.total), dim3(TermsCfg::NTHREADS), TermsCfg::LDS_BYTES, st, p);
+    auto kern = p.xcache ? lce_fwd16_kernel<TermsCfg, true> : lce_fwd16_kernel<TermsCfg, false>;
+    allow_lds(kern, TermsCfg::LDS_BYTES);
+    hipLaunchKernelGGL(kern, dim3(p.map.total), dim3(TermsCfg::NTHREADS), TermsCfg::LDS_BYTES, st, p);
     if ((rc = check_launch("lce_fwd16_kernel"))) return rc;
     done += p.S;
   }
@@ -184,7 +199,8 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
 #else
 int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                    int reduction, const float* maximum, const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
-                   float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu) {
+                   float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu,
+                   const float* xcache) {
   typedef TermsCfg Cfg;
   const bool need_dh = d_hidden != nullptr, need_dw = d_weight != nullptr;
   const TermsBwdLayout L = terms_bwd_layout(tu, T, H, V, vchunk);
@@ -218,6 +234,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   const SplitArgs sh = {h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows};
   if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
   const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN), h_tile = hidden_tile(H);
+  const int64_t kept = xcache ? terms_kept_rows(T, H, V) : 0;
   // launch c: d_logits of chunk c and the gradient GEMMs of chunk c - 1, as in backward_impl
   for (int c = 0; c <= L.nchunks; ++c) {
     BwdChunkArgs<bf16_t> p;
@@ -235,8 +252,22 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
       d.dS = dS[c & 1]; d.ldS = 64; d.pcol = L.pcol; d.dST = nullptr; d.ldST = 0; d.tpad = L.tpad;
       d.rows = nullptr; d.n_rows = n_rows; d.label_outside = 0;
       d.tokc = tokc; d.tokl = tokl; d.lab0 = v0; d.range_rows = 0;
-      d.map = TileMap::make(ntt, (int)((vrows + Cfg::BM - 1) / Cfg::BM), block_rows(ntt), 0);
-      p.n_ds = d.map.total;
+      // the rows whose logits the forward kept, then tiles for the others
+      const int64_t k = std::min(vrows, kept - v0);
+      if (k > 0) {
+        ProfScope prof(PC_BWD_DS, st);
+        DsArgs<bf16_t> dq = d;
+        dq.rows = rows;  // (the tiles read the compact planes of hidden and no list; the cache is indexed by token)
+        dq.vrows = k;
+        hipLaunchKernelGGL((ds_from_logits_kernel<bf16_t, KPerm<Cfg>, Cfg::TERMS>), dim3((unsigned)(round_up(k, 256) / 64)), dim3(256), 0, st, dq,
+                           xcache + v0 * T, T, (int)L.tpad, false);
+        if ((rc = check_launch("ds_from_logits_kernel"))) return rc;
+        d.W += k * d.ldw; d.v0 += k; d.lab0 += k; d.vrows -= k; d.dS += k / 64 * d.pcol;
+      }
+      if (d.vrows > 0) {
+        d.map = TileMap::make(ntt, (int)((d.vrows + Cfg::BM - 1) / Cfg::BM), block_rows(ntt), 0);
+        p.n_ds = d.map.total;
+      }
     }
     if (c > 0) {
       const int cc = c - 1;
@@ -269,6 +300,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
         p.n_gh = 0;
       }
     }
+    if (p.n_gw + p.n_gh + p.n_ds == 0) continue;
     ProfScope prof(PC_BWD_CHUNK, st);
     auto kern = h_tile == 224 ? lce_bwd_chunk16_kernel<Cfg, 7> : lce_bwd_chunk16_kernel<Cfg, 8>;
     allow_lds(kern, Cfg::LDS_BYTES);
