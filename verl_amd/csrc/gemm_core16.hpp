@@ -35,6 +35,9 @@ struct Mma16<bf16_t> {
   static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
   }
+  static LCE_DEV void over(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // the same, in the registers of what acc was
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "+a"(acc) : "v"(a), "v"(b));
+  }
 };
 template <>
 struct Mma16<f16_t> {
@@ -43,6 +46,9 @@ struct Mma16<f16_t> {
   }
   static LCE_DEV void first(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // acc = a b
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
+  }
+  static LCE_DEV void over(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {  // the same, in the registers of what acc was
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "+a"(acc) : "v"(a), "v"(b));
   }
 };
 
@@ -561,46 +567,137 @@ struct GemmCore16 {
     });
     s.sb = 0;
   }
-  // One tile of nk >= 2 slabs at a_base / b_base; a_next / b_next: the next tile's (this one's again when there is none).
-  // STORES: with `stores_behind`, exactly that many stores of this wave lie between the loads of this tile's second slab
-  // and anything loaded here.  The first wait leaves them in flight; the second slab's needs them acknowledged, which
-  // gives them the time of a slab and a half.  Ring slot (s.sb + 4) % 5 is free when this returns, until the barrier that
-  // the caller places before the next call.
-  template <int STORES>
-  LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, bool stores_behind) const {
-    static_assert(Cfg::TRANS != 2 && HL + STORES < 64, "slab addresses, vmcnt range");
-    static_assert(NBN == 8 && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "whole tiles, B early");
+  // What slab `it` of nk fetches meanwhile: the slab two further on, beyond this tile's last (a_base / b_base) the first ones of
+  // the next tile (a_next / b_next; this one's again when there is none).
+  struct Ahead {
+    const char *a, *b;
+  };
+  LCE_DEV Ahead stream_ahead(int it, int nk, const char* a_next, const char* b_next) const {
+    const bool nx = it + 2 >= nk;
+    const int ks = nx ? it + 2 - nk : it + 2;
+    return {(nx ? a_next : a_base) + ks * a_slab, (nx ? b_next : b_base) + ks * b_slab};
+  }
+  static LCE_DEV int ring(int slot) { return slot >= 5 ? slot - 5 : slot; }
+
+  // Slab `it` of a tile of nk >= 2 slabs.  Ring slot (s.sb + 4) % 5 is free when this returns.
+  template <bool FIRST>
+  LCE_DEV void stream_slab(char* lds, int it, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next) const {
+    static_assert(Cfg::TRANS != 2 && NBN == 8 && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "whole tiles, B early");
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
-    int sb = s.sb;
-    auto slab = [&](auto first, int it) {
-      constexpr bool FIRST = decltype(first)::value;
-      u32x4_t af1[NB], bf1[NBN];  // the fragments of the slab's second k-step
-      const int sa = sb + 1 >= 5 ? sb + 1 - 5 : sb + 1;
-      const int nb = sb + 2 >= 5 ? sb + 2 - 5 : sb + 2;
-      const int na = sb + 3 >= 5 ? sb + 3 - 5 : sb + 3;
-      const int fr = sb + 4 >= 5 ? sb + 4 - 5 : sb + 4;
-      const bool nx = it + 2 >= nk;
-      const int ks = nx ? it + 2 - nk : it + 2;
-      const char* from_b = (nx ? b_next : b_base) + ks * b_slab;
-      const char* from_a = (nx ? a_next : a_base) + ks * a_slab;
-      kstep<true, 1, true, true, FIRST>(acc, s.af, s.bf, lds0 + sa * SLOT + a_rd, lds0 + sb * SLOT + b_rd, af1, bf1, lds, fr, 0, from_b);
-      if (FIRST && stores_behind) wait_vm<HL + STORES>();
-      else wait_vm<HL>();
-      wait_lgkm<0>();
-      __builtin_amdgcn_s_barrier();
-      kstep<false, 0, false, true>(acc, af1, bf1, lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, s.af, s.bf, lds, sb, 0, from_a);
-      sb = nb;
-    };
-    slab(std::true_type{}, 0);
-    for (int it = 1; it < nk; ++it) slab(std::false_type{}, it);
-    s.sb = sb;
-    // the next tile's first fragments are in registers from here on, whatever the compiler does with those meanwhile
+    u32x4_t af1[NB], bf1[NBN];  // the fragments of the slab's second k-step
+    const int sb = s.sb, sa = ring(sb + 1), nb = ring(sb + 2), na = ring(sb + 3), fr = ring(sb + 4);
+    const Ahead from = stream_ahead(it, nk, a_next, b_next);
+    kstep<true, 1, true, true, FIRST>(acc, s.af, s.bf, lds0 + sa * SLOT + a_rd, lds0 + sb * SLOT + b_rd, af1, bf1, lds, fr, 0, from.b);
+    wait_vm<HL>();
+    wait_lgkm<0>();
+    __builtin_amdgcn_s_barrier();
+    kstep<false, 0, false, true>(acc, af1, bf1, lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, s.af, s.bf, lds, sb, 0, from.a);
+    s.sb = nb;
+  }
+
+  // the next tile's first fragments are in registers from here on, whatever the compiler does with those meanwhile
+  static LCE_DEV void stream_settle(Stream& s) {
     wait_lgkm<0>();
 #pragma unroll
     for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(s.af[i]));
 #pragma unroll
     for (int j = 0; j < NBN; ++j) asm volatile("" : "+v"(s.bf[j]));
+  }
+
+  // One tile.
+  LCE_DEV void stream_tile(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next) const {
+    stream_slab<true>(lds, 0, nk, acc, s, a_next, b_next);
+    for (int it = 1; it < nk; ++it) stream_slab<false>(lds, it, nk, acc, s, a_next, b_next);
+    stream_settle(s);
     retire(acc);
+  }
+
+  // A tile's last slab when only its first k-step holds anything.  The next tile's first fragments are not read yet when it
+  // returns (stream_fragments).
+  LCE_DEV void stream_half_slab(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next) const {
+    const Ahead from = stream_ahead(nk - 1, nk, a_next, b_next);
+    const int fr = ring(s.sb + 4);
+    constexpr int EVERY = NB * NBN / HLB;
+    wait_lgkm<0>();
+    static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      Mma16<TIN>::run(acc[m / NBN][m % NBN], s.af[m / NBN], s.bf[m % NBN]);
+      if constexpr (m % EVERY == 3 && m / EVERY < HLB) fetch_b(lds, fr, from.b, m / EVERY);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    wait_vm<HLB>();
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int j = 0; j < HL; ++j) fetch_a(lds, s.sb, from.a, j);
+    s.sb = ring(s.sb + 2);
+  }
+  LCE_DEV void stream_fragments(char* lds, Stream& s) const {
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    static_for(std::make_integer_sequence<int, NF>{}, [&](auto fc) {
+      read_frag<decltype(fc)::value, 0>(lds0 + ring(s.sb + 1) * SLOT + a_rd, lds0 + s.sb * SLOT + b_rd, s.af, s.bf);
+    });
+  }
+  LCE_DEV void fetch_a(char* lds, int slot, const char* from, int j) const {
+    __builtin_amdgcn_global_load_lds((gptr_t)(from + va[j]), (lptr_t)(lds + slot * SLOT + (j * Cfg::NW + wave) * 1024), 16, 0, 0);
+  }
+  LCE_DEV void fetch_b(char* lds, int slot, const char* from, int j) const {
+    __builtin_amdgcn_global_load_lds((gptr_t)(from + vb[j]), (lptr_t)(lds + slot * SLOT + (j * Cfg::NW + wave) * 1024), 16, 0, 0);
+  }
+
+  // A tile's first slab, whose first k-step takes the finished tile out of the accumulators as it starts them anew: block (i, j) is
+  // handed to `out` (out.block<i, j>(value)) ahead of the MFMA that overwrites it, block columns in the outer loop, and
+  // out.send<j>() and out.store<j>() follow while column j + 1 goes through the matrix pipe: a column's NB LDS writes, then its
+  // out.READS LDS reads, then its out.STORES stores.  The finished tile meets LDS in ring slot (s.sb + 4) % 5, so that the B half
+  // that would be fetched into it comes with the A half, in the second k-step.  `last`: there is no next tile, and the accumulators
+  // hold nothing afterwards (a way out of a walk that read them elsewhere would have the compiler move them about).
+  template <typename Out>
+  LCE_DEV void stream_slab_over(char* lds, int nk, f32x4_t (&acc)[NB][NBN], Stream& s, const char* a_next, const char* b_next, Out& out, bool last) const {
+    static_assert(Cfg::TRANS != 2 && NBN == 8 && NB >= 7 && !AE && Cfg::TERMS == 1 && !Cfg::A_ONCE, "whole tiles, B early");
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    u32x4_t af1[NB], bf1[NBN];
+    const int sb = s.sb, sa = ring(sb + 1), nb = ring(sb + 2), na = ring(sb + 3), fr = ring(sb + 4);
+    const Ahead from = stream_ahead(0, nk, a_next, b_next);
+    const uint32_t ra = lds0 + sa * SLOT + a_rd, rb = lds0 + sb * SLOT + b_rd;
+    wait_lgkm<0>();
+    static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
+      constexpr int m = decltype(mc)::value, j = m / NB, i = m % NB;
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" : "+a"(acc[i][j]));  // (read here and not ahead of the first MFMA)
+      out.template block<i, j>(acc[i][j]);
+      Mma16<TIN>::over(acc[i][j], s.af[i], s.bf[j]);
+      if constexpr (j > 0 && i == 1) out.template send<j - 1>();  // (a wave's LDS operations are done in order)
+      if constexpr (j > 0 && i == 5) {
+        wait_lgkm<4>();  // (the writes of blocks 2 to 5 came behind those reads)
+        out.template store<j - 1>();
+      }
+      if constexpr (i == NB - 1) {
+        if constexpr (2 * j < NF) read_frag<2 * j, 1>(ra, rb, af1, bf1);
+        if constexpr (2 * j + 1 < NF) read_frag<2 * j + 1, 1>(ra, rb, af1, bf1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    out.template send<NBN - 1>();
+    wait_lgkm<0>();
+    out.template store<NBN - 1>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (last) return;
+    wait_vm<NBN * Out::STORES>();  // slab 1 has landed; the stores may be on their way
+    __builtin_amdgcn_s_barrier();
+    constexpr int LOADS = HLB + HL, EVERY = NB * NBN / LOADS;
+    static_assert(2 * NF <= NB * NBN && LOADS * EVERY <= NB * NBN, "one fragment read after every second MFMA");
+    static_for(std::make_integer_sequence<int, NB * NBN>{}, [&](auto mc) {
+      constexpr int m = decltype(mc)::value, l = m / EVERY;
+      __builtin_amdgcn_sched_barrier(0);
+      Mma16<TIN>::run(acc[m / NBN][m % NBN], af1[m / NBN], bf1[m % NBN]);
+      if constexpr ((m & 1) == 0 && m / 2 < NF) read_frag<m / 2, 0>(lds0 + na * SLOT + a_rd, lds0 + nb * SLOT + b_rd, s.af, s.bf);
+      if constexpr (m % EVERY == EVERY - 1 && l < LOADS) {
+        if constexpr (l < HLB) fetch_b(lds, fr, from.b, l);
+        else fetch_a(lds, sb, from.a, l - HLB);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    s.sb = nb;
   }
 
   LCE_DEV void run(char* lds, int64_t K, f32x4_t (&acc)[NB][NBN]) const {

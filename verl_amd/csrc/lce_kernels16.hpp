@@ -144,7 +144,7 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
       const int64_t next = m0 + p.tile_step;
       const bool flows = next + Cfg::BM <= vend64;
       const char* a_next = flows ? g.a_base + p.tile_step * p.ldw * 2 : g.a_base;
-      g.template stream_tile<0>(lds, nk, acc, st, a_next, g.b_base, false);
+      g.stream_tile(lds, nk, acc, st, a_next, g.b_base);
       g.a_base = a_next;
       const bool anew = next < vend64 && !flows;
       if (anew) {
@@ -524,13 +524,14 @@ LCE_DEV void gemm16_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, char* 
 
 // LDS write of 8 bytes as inline assembly, for the same reason as the reads: through the compiler it would wait for the
 // global->LDS loads in flight
-LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_write_b64 %0, %1" ::"v"(lds_addr), "v"(v)); }
+template <int OFF = 0>
+LCE_DEV void lds_write8(uint32_t lds_addr, const u32x2_t& v) { asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(lds_addr), "v"(v), "i"(OFF)); }
 
 // A finished wave tile in 16 bits, C[m][n] with rows in the operand's column order (PermCfg's vocab_at), leaves the wave as
 // whole lines: 16 rows x 128 columns (one block column) at a time go through 4 KB of LDS that belong to this wave, 16-byte
 // chunk c of row r at c ^ r, and are stored four rows x 256 bytes per instruction.  (A CU stores such runs three to four
 // times as fast as the accumulators' own lane order, 16 rows x 64 bytes.)  Two buffers in turn: block column j is
-// written while j - 1 is read back, so that neither waits for the other.  32 stores, exactly, when the tile is FULL.
+// written while j - 1 is read back, so that neither waits for the other.
 // Non-temporal: unmarked, the lines of d_weight push the dS and the hidden that other workgroups are about to read out of the
 // caches (forward + backward, H=3584, V=152064: 333 tokens 1289 -> 1240 us, 512: 1624 -> 1588, 700: 2111 -> 2089, level from 1600 on).
 template <typename Cfg, typename PermCfg, bool FULL>
@@ -585,6 +586,51 @@ LCE_DEV void gemm16_store_lines(const GemmArgs<typename Cfg::TIN>& p, f32x4_t (&
   });
 }
 
+// The same for a workgroup that walks tiles, block by block as the next tile's first k-step comes to them
+// (GemmCore16::stream_slab_over).  Rows and columns beyond C are stores to nowhere, so that their number is always the same.
+template <typename Cfg, typename PermCfg>
+struct LineStores16 {
+  typedef typename Cfg::TIN TIN;
+  static constexpr int STORES = 4;  // of a block column
+  buf_t out;
+  uint32_t wr, rd;
+  int at, row_bytes;
+  u32x4_t v[STORES];
+  LCE_DEV LineStores16(const GemmArgs<TIN>& p, int64_t m0, int64_t n0, int wave_m, int wave_n, uint32_t stage) {
+    const int lane = lane_anew(), g4 = lane >> 4, l16 = lane & 15;
+    wr = stage + (uint32_t)(l16 * 256 + (((g4 >> 1) ^ l16) * 16) + (g4 & 1) * 8);
+    rd = stage + (uint32_t)(g4 * 256 + ((l16 ^ g4) * 16));
+    const int64_t n = n0 + wave_m * Cfg::WM, mw = m0 + wave_n * Cfg::WN, left = p.M - mw;
+    row_bytes = (int)(p.ldct * (int64_t)sizeof(TIN));
+    out = make_buf(p.Ct + mw * p.ldct + n, (left < Cfg::WN ? left > 0 ? left : 0 : Cfg::WN) * row_bytes);
+    at = (Cfg::NB == 8 || l16 < 2 * Cfg::NB) && n + l16 * 8 < p.N ? g4 * row_bytes + l16 * 16 : kBufNowhere;
+  }
+  template <int I, int J>
+  LCE_DEV void block(const f32x4_t& acc) const {
+    typename VecOf<TIN, 4>::type o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = round_to<TIN>(acc[r]);
+    lds_write8<(J & 1) * 4096>(wr ^ (uint32_t)(I * 32), __builtin_bit_cast(u32x2_t, o));
+  }
+  template <int J>
+  LCE_DEV void send() {
+    static_for(std::make_integer_sequence<int, STORES>{}, [&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      v[k] = lds_read16<(J & 1) * 4096 + k * 1024>(rd ^ (uint32_t)(k * 64));
+    });
+  }
+  template <int J>
+  LCE_DEV void store() {
+#pragma unroll
+    for (int k = 0; k < STORES; ++k) asm volatile("" : "+v"(v[k]));
+#pragma unroll
+    for (int k = 0; k < STORES; ++k) {
+      const int row = (int)KPerm<PermCfg>::vocab_at(16 * J + 4 * k);
+      __builtin_amdgcn_raw_buffer_store_b128(v[k], out, at + row * row_bytes, 0, kBufNonTemporal);
+    }
+  }
+};
+
 // C[m][n] = sum_k A[k][m] * B[k][n], both operands K-major and allocated in whole tiles, K (or *k_dev
 // rounded up to k_gran) a multiple of 64.  out_mode 0: Cf = acc; out_mode 2: Ct[PermCfg's vocab_at(m)][n] = (TIN)acc
 // (the rows of C are A's columns, which the d_logits epilogue leaves in KPerm::vocab order).
@@ -638,9 +684,13 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
 
 // d_weight with tokens between the streaming kernels' range and the sizes where a tile's K loop hides everything else:
 // C[vocab_at(m)][n] = (TIN) sum_k A[k][m] B[k][n] as in gemm16_tn_tile (out_mode 2), by workgroups that stay (one per CU)
-// and walk the tiles, the K loops of successive tiles being one stream of slabs (GemmCore16::stream_tile).  With 333 tokens a
+// and walk the tiles, the K loops of successive tiles being one stream of slabs.  With 333 tokens a
 // tile is six slabs of 1.2 to 1.5 us, and a workgroup per tile paid another 9 us for its start, its first loads, the drain of
-// its last and its stores.
+// its last and its stores.  A finished tile leaves the accumulators during the next one's first k-step (stream_slab_over: 384
+// conversions beside 64 MFMAs, some 2800 cycles for 4400 + 1024 one behind the other), and a last slab of up to 32 tokens is one k-step: kernel at 333
+// tokens of H=3584 432 -> 416 us, 512: 496 -> 487, 1000: 908 -> 902; step 270: 1203 -> 1187, 333: 1268 -> 1251, 500: 1575 -> 1561, 400 of
+// H=5120 2117 -> 2089, from 1000 on level.  Without its stores it takes 347, 443 and 811: the 1.09 GB of results cost 45 to 90 us
+// wherever in the tile they are issued (workgroups set off by a quarter of a tile against each other: level).
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typename Cfg::TIN> p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -648,15 +698,14 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
   typedef GemmCore16<TnCfg> Core;
   constexpr int TM = TnCfg::BN, TN = TnCfg::BM;  // a tile's rows and columns of C (MFMA rows = n, MFMA columns = m)
   if (p.k_dev) {
-    // (at least two slabs, which the stream wants: token_prep_kernel, and beyond its range gather_rows_kernel, zeroes that many
-    // rows of hidden, the d_logits pass those of dS)
-    const int64_t k = *p.k_dev == 0 ? 0 : (*p.k_dev <= 64 ? 128 : ((int64_t)*p.k_dev + 63) / 64 * 64);
+    // whole k-steps of 32 (at least two slabs, which the stream wants: token_prep_kernel, and beyond its range gather_rows_kernel,
+    // zeroes that many rows of hidden, the d_logits pass those of dS)
+    const int64_t k = *p.k_dev == 0 ? 0 : (*p.k_dev <= 64 ? 128 : ((int64_t)*p.k_dev + 31) / 32 * 32);
     p.K = k < p.K ? k : p.K;
   }
-  const int nk = (int)(p.K / 64);
+  const int nk = (int)((p.K + 63) / 64);
   Core g;
   g.set_lane();
-  f32x4_t acc[TnCfg::NB][TnCfg::NBN];
   int bid = blockIdx.x, tm = 0, tn = 0;
   auto next_tile = [&]() {  // the first tile at or behind bid (uniform over the workgroup)
     for (; bid < p.map.total; bid += gridDim.x)
@@ -672,35 +721,51 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typena
       }
     return;
   }
-  typename Core::Stream s;
-  g.init_tn(p.B, p.ldb, (int64_t)tn * TN, p.A, p.lda, (int64_t)tm * TM, p.a_pcol);
-  g.prologue(lds, p.K);
-  g.stream_begin(lds, s);
-  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
-  bool behind = false, more = true;
-  while (more) {
-    const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
-    bid += gridDim.x;
-    more = next_tile();
-    const char *a_next = g.a_base, *b_next = g.b_base;
-    if (more) {
-      a_next = reinterpret_cast<const char*>(p.B + (int64_t)tn * TN);
-      b_next = reinterpret_cast<const char*>(p.a_pcol ? p.A + (int64_t)tm * (TM / 64) * p.a_pcol : p.A + (int64_t)tm * TM);
+  // (a loop of its own for a last slab that is half a slab: with one loop for both the fragments are moved from register to register)
+  auto walk = [&](auto half) {
+    constexpr bool HALF = decltype(half)::value;
+    f32x4_t acc[TnCfg::NB][TnCfg::NBN];
+    typename Core::Stream s;
+    int64_t m0, n0;  // this tile
+    const char *a_next, *b_next;
+    bool more;
+    auto look_ahead = [&]() {
+      m0 = (int64_t)tm * TM;
+      n0 = (int64_t)tn * TN;
+      bid += gridDim.x;
+      more = next_tile();
+      a_next = more ? reinterpret_cast<const char*>(p.B + (int64_t)tn * TN) : g.a_base;
+      b_next = more ? reinterpret_cast<const char*>(p.a_pcol ? p.A + (int64_t)tm * (TM / 64) * p.a_pcol : p.A + (int64_t)tm * TM) : g.b_base;
+    };
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds) + g.wave * 8192;
+    auto stage = [&]() { return lds0 + (uint32_t)(Core::ring(s.sb + 4) * TnCfg::STAGE_BYTES); };
+    g.init_tn(p.B, p.ldb, (int64_t)tn * TN, p.A, p.lda, (int64_t)tm * TM, p.a_pcol);
+    g.prologue(lds, (int64_t)nk * 64);
+    g.stream_begin(lds, s);
+    look_ahead();
+    g.template stream_slab<true>(lds, 0, nk, acc, s, a_next, b_next);
+    while (true) {
+      for (int it = 1; it < nk - HALF; ++it) g.template stream_slab<false>(lds, it, nk, acc, s, a_next, b_next);
+      if constexpr (HALF) g.stream_half_slab(lds, nk, acc, s, a_next, b_next);
+      else Core::stream_settle(s);
+      Core::retire(acc);
+      g.a_base = a_next;
+      g.b_base = b_next;
+      g.reads_tn(lane_anew());
+      if constexpr (HALF) {
+        g.stream_fragments(lds, s);
+        Core::stream_settle(s);
+      }
+      LineStores16<TnCfg, Cfg> done(p, m0, n0, g.wave_m, g.wave_n, stage());
+      const bool last = !more;
+      if (!last) look_ahead();
+      g.stream_slab_over(lds, nk, acc, s, a_next, b_next, done, last);
+      if (last) break;
     }
-    g.reads_tn(lane_anew());
-    g.template stream_tile<32>(lds, nk, acc, s, a_next, b_next, behind);
-    g.a_base = a_next;
-    g.b_base = b_next;
-    const int free_slot = s.sb + 4 >= 5 ? s.sb + 4 - 5 : s.sb + 4;
-    const uint32_t stage = lds0 + (uint32_t)(free_slot * TnCfg::STAGE_BYTES) + g.wave * 8192;
-    __builtin_amdgcn_sched_barrier(0);
-    behind = m0 + TM <= p.M && n0 + TN <= p.N;
-    if (behind) gemm16_store_lines<TnCfg, Cfg, true>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
-    else gemm16_store_lines<TnCfg, Cfg, false>(p, acc, m0, n0, g.wave_m, g.wave_n, stage);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();  // every wave has read its staged rows: the slot is the ring's again
-  }
-  Core::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
+    Core::template wait_vm<0>();
+  };
+  if (p.K % 64 != 0) walk(std::true_type{});
+  else walk(std::false_type{});
 }
 
 // fp32 rows as three bfloat16 planes, out[r] = three runs of ldo elements.  Row r is in[rows[r]] (in[r] without `rows`) for
