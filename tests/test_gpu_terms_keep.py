@@ -1,10 +1,13 @@
 """fp32 inputs on bfloat16 planes with kept logits: of every row of the weight up to as many tokens as the hidden size, of the
-first rows beyond.  Both ways to d_logits share all of their arithmetic, so the bits are those of the backward that recomputes."""
+first rows beyond.  Both ways to d_logits share all of their arithmetic: d_weight has the bits of the backward that recomputes,
+d_hidden, which sums chunks of another width, its error."""
 
 import importlib
 
 import pytest
 import torch
+
+from oracle import lce_oracle as O
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -16,6 +19,7 @@ DEV = "cuda:0"
     (700, 256, 50003, 2048, 0, 0.5),   # part of the rows: whole chunks, one cut in two, the others
     (1024, 256, 65536, 0, 1, 0.02),    # a quarter of them, the most tokens that keep any
     (640, 640, 33000, 0, 0, 0.0),      # no token takes part
+    (700, 256, 50003, 65536, 0, 1.0),  # part of the rows of one chunk
 ])  # fmt: skip
 def test_kept_logits_of_planes(T, H, V, vchunk, reduction, keep):
     from verl_amd import _abi
@@ -41,11 +45,21 @@ def test_kept_logits_of_planes(T, H, V, vchunk, reduction, keep):
         run = lambda **kw: kernels.efficient_entropy_backward(g_lp, g_ent, h, w, y, *kept[2:], reduction, False, 0.8, **kw)  # noqa: E731
         dh, dw = run()
         dh1, dw1 = run(logits_cache=cache)
-        assert torch.equal(dh, dh1) and torch.equal(dw, dw1)
-        assert torch.equal(dh, run(logits_cache=cache, need_d_weight=False)[0]) and torch.equal(dw, run(logits_cache=cache, need_d_hidden=False)[1])
+        assert torch.equal(dw, dw1)
+        assert torch.equal(dh1, run(logits_cache=cache, need_d_weight=False)[0]) and torch.equal(dw, run(logits_cache=cache, need_d_hidden=False)[1])
         torch.cuda.synchronize()
     finally:
         kernels.set_vocab_chunk(0)
+    full = g_lp if reduction == 0 else (g_lp / (T if reduction == 2 else 1)).expand(T)
+    # (an ignored label has no entry of its own; the oracle takes labels of the vocabulary only)
+    want = O.lce_backward(full, g_ent, h, w, y.clamp(min=0), 0.8, compute_dtype=torch.float64)[0]
+    want -= ((y < 0) * full / 0.8).double()[:, None] * w[0].double()
+    if want.norm() > 0:  # the bar of the planes' other tests; the two ways differ by less than either's own error allows
+        off, off1 = (((x.double() - want).norm() / want.norm()).item() for x in (dh, dh1))
+        print(f"T={T} H={H} V={V}: d_hidden against float64, recomputed {off:.2e}, kept {off1:.2e}")
+        assert off1 <= 3e-6 and off1 <= 1.25 * off
+    else:
+        assert (dh1 == 0).all()
 
 
 def test_which_fp32_calls_keep_logits():

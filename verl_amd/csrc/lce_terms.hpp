@@ -67,7 +67,14 @@ struct TermsBwdLayout {
   int64_t vchunk, tpad, pcol, plane, ldH;  // plane: elements from plane to plane of a d_logits panel
   size_t off_dS[2], off_W[2], off_H, off_dHacc, off_rows, off_inv, off_nrows, off_acounts, off_tokc, off_tokl, total;
   int nchunks, ksplit;
+  bool wide;  // chunks twice as wide where the forward kept the logits, with twice the K slices and partials of d_hidden
 };
+
+// upper bound of the workspace: a quarter of one [T, V] plus one fp32 [V, H], or the budget
+double terms_gate(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
+  const double gate = (double)T * V + 4.0 * (double)V * H;
+  return tu.ws_budget > 0 && (double)tu.ws_budget < gate ? (double)tu.ws_budget : gate;
+}
 
 TermsBwdLayout terms_bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
   TermsBwdLayout L;
@@ -79,19 +86,29 @@ TermsBwdLayout terms_bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int6
   L.pcol = 3 * L.plane + 64;
   L.ldH = round_up(H, 256) + 64;
   size_t o = 0;
-  for (int b = 0; b < 2; ++b) {
-    L.off_dS[b] = o; o += (b == 0 || L.nchunks > 1) ? align256((size_t)(L.vchunk / 64) * L.pcol * 2) : 0;
-    L.off_W[b] = o;  o += (b == 0 || L.nchunks > 1) ? align256((size_t)L.vchunk * 3 * H * 2) : 0;
-  }
+  // (the two of a kind follow each other without a gap: backward_terms has chunks that take both)
+  const bool two = L.nchunks > 1;
+  for (int b = 0; b < 2; ++b) { L.off_dS[b] = o; o += b == 0 || two ? (size_t)(L.vchunk / 64) * L.pcol * 2 : 0; }
+  o = align256(o);
+  for (int b = 0; b < 2; ++b) { L.off_W[b] = o; o += b == 0 || two ? (size_t)L.vchunk * 3 * H * 2 : 0; }
+  o = align256(o);
   L.off_H = o;       o += align256((size_t)L.tpad * 3 * L.ldH * 2);
-  L.off_dHacc = o;   o += (size_t)L.ksplit * align256((size_t)T * H * 4);
   L.off_rows = o;    o += align256((size_t)L.tpad * 4);
   L.off_inv = o;     o += align256((size_t)T * 4);
   L.off_nrows = o;   o += 256;
   L.off_acounts = o; o += align256((size_t)((T + kActiveBlock - 1) / kActiveBlock) * 4);
   L.off_tokc = o;    o += align256((size_t)L.tpad * 16);
   L.off_tokl = o;    o += align256((size_t)L.tpad * 4);
-  L.total = o;
+  L.off_dHacc = o;   o += (size_t)L.ksplit * align256((size_t)T * H * 4);
+  // The wide chunks, where a launch is few rounds of tiles and half of the rows at least are kept: forward + backward, us, H=896: 256
+  // tokens 1977 -> 1659, 300: 2177 -> 2155, 600: 3225 -> 3011, 1024: 4650 -> 4383 (d_hidden alone 3325 -> 3355), 1500: 6487 -> 6404; five
+  // rounds, H=4096, 2000: 26584 -> 26260; from eight rounds on they are level or slower: H=3584, 300: 7906 -> 7976, 600: 10999 -> 11174;
+  // H=5120, 1000: 21342 -> 21593; with 45 % of the rows, H=896, 2000: 8791 -> 8909.
+  const int64_t h_tile = hidden_tile(H);
+  const size_t more = (size_t)L.ksplit * align256((size_t)T * H * 4);
+  L.wide = two && L.vchunk >= 4096 && T <= 2 * H && tu.dh_ksplit == 0 && (L.vchunk / 256) * ((H + h_tile - 1) / h_tile) < 6 * kNumCUs &&
+           (double)(o + more) + 512.0 <= terms_gate(tu, T, H, V);
+  L.total = o + (L.wide ? more : 0);
   return L;
 }
 
@@ -99,8 +116,7 @@ TermsBwdLayout terms_bwd_layout_for(const Tuning& tu, int64_t T, int64_t H, int6
 // planes stay within 256 MB
 TermsBwdLayout terms_bwd_layout(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
   if (vchunk <= 0) {
-    double gate = (double)T * V + 4.0 * (double)V * H;
-    if (tu.ws_budget > 0 && (double)tu.ws_budget < gate) gate = (double)tu.ws_budget;
+    const double gate = terms_gate(tu, T, H, V);
     vchunk = std::min(round_up(V, 256), std::max<int64_t>(2048, (((int64_t)256 << 20) / (6 * T)) / 256 * 256));
     while (vchunk > 2048 && (double)terms_bwd_layout_for(tu, T, H, V, vchunk).total + 512.0 > gate) vchunk -= 1024;
     if (vchunk < 2048) vchunk = 2048;
@@ -235,58 +251,66 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
   const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN), h_tile = hidden_tile(H);
   const int64_t kept = xcache ? terms_kept_rows(T, H, V) : 0;
-  // launch c: d_logits of chunk c and the gradient GEMMs of chunk c - 1, as in backward_impl
-  for (int c = 0; c <= L.nchunks; ++c) {
+  // The chunks: of the rows whose logits the forward kept, then the others, whose d_logits tiles share a launch with the products of the
+  // chunk before.  The kept ones' d_logits are a pass of their own, so that both buffers may hold one chunk twice as wide (L.wide): half as
+  // many launches, each with a last round of tiles.  The last of them, where others follow, is of the usual width.
+  struct Chunk {
+    int64_t v0, rows;
+    int buf;
+    bool kept, alone;  // alone: its products share their launch with no d_logits tiles
+  };
+  std::vector<Chunk> chunks;
+  auto cut = [&](int64_t from, int64_t to, int64_t width, bool of_kept) {
+    const int64_t n = (to - from + width - 1) / width;
+    if (n > 0) width = round_up((to - from + n - 1) / n, 256);
+    for (int64_t v0 = from, c = 0; v0 < to; v0 += width, ++c) chunks.push_back({v0, std::min(width, to - v0), of_kept ? 0 : (int)(c & 1), of_kept, of_kept});
+  };
+  const int64_t joint = kept < V && L.nchunks > 1 ? std::min(kept, L.vchunk) : 0;
+  cut(0, kept - joint, L.wide ? 2 * L.vchunk : L.vchunk, true);
+  // K slices of a wide chunk no longer than a usual one's (the same error of d_hidden), or twice as many as that has, where d_hidden's
+  // tiles then fill their rounds over the CUs better by a tenth (1024 tokens of H=896, d_hidden alone: 3447 -> 3305 us)
+  int wide_slices = L.ksplit;
+  if (L.wide && !chunks.empty()) {
+    const int64_t tiles = ntt * ((H + h_tile - 1) / h_tile), rows = chunks[0].rows, slice = round_up((L.vchunk + L.ksplit - 1) / L.ksplit, Cfg::BK);
+    auto time = [&](int64_t s) { return (double)((tiles * s + kNumCUs - 1) / kNumCUs) * ((double)rows / (double)(s * Cfg::BK) + 2); };
+    wide_slices = (int)std::max<int64_t>(L.ksplit, (rows + slice - 1) / slice);
+    if (time(2 * L.ksplit) < 0.9 * time(wide_slices)) wide_slices = 2 * L.ksplit;
+  }
+  const int all_slices = std::max(wide_slices, L.ksplit);
+  if (joint > 0) chunks.push_back({kept - joint, joint, 1, true, false});
+  cut(kept, V, L.vchunk, false);
+  const int nchunks = (int)chunks.size();
+  auto launch = [&](BwdChunkArgs<bf16_t>& p) {
+    if (p.n_gw + p.n_gh + p.n_ds == 0) return (int)LCE_OK;
+    ProfScope prof(PC_BWD_CHUNK, st);
+    auto kern = h_tile == 224 ? lce_bwd_chunk16_kernel<Cfg, 7> : lce_bwd_chunk16_kernel<Cfg, 8>;
+    allow_lds(kern, Cfg::LDS_BYTES);
+    hipLaunchKernelGGL(kern, dim3(p.n_gw + p.n_gh + p.n_ds), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
+    return check_launch("lce_bwd_chunk16_kernel");
+  };
+  // step c: the gradient GEMMs of chunk c - 1 and d_logits of chunk c, in one launch as in backward_impl where neither is a pass or a launch of its own
+  for (int c = 0; c <= nchunks; ++c) {
     BwdChunkArgs<bf16_t> p;
     p.n_gw = p.n_gh = p.n_ds = 0;
-    if (c < L.nchunks) {
-      const int64_t v0 = (int64_t)c * L.vchunk, vrows = std::min(L.vchunk, V - v0);
-      // (the last reader of this buffer, d_hidden of chunk c - 2, ran in the launch before the last)
-      if ((rc = launch_split({W + v0 * ldw, ldw, vrows, H, w3[c & 1], H, vrows, nullptr, nullptr}, &sh, wide, st))) return rc;
-      DsArgs<bf16_t>& d = p.ds;
-      d.W = w3[c & 1]; d.ldw = 3 * H; d.h = h3; d.ldh = 3 * L.ldH; d.labels = labels; d.T = T; d.H = H;
-      d.w_plane = H * 2; d.h_plane = L.ldH * 2; d.dS_plane = L.plane;
-      d.v0 = vocab_offset + v0; d.vrows = vrows; d.rcp_tau = 1.0f / temperature; d.c = kLog2e / temperature;
-      d.maximum = maximum; d.accumulate = accumulate; d.entropy_b = entropy_b;
-      d.g_lp = dlogprobs; d.g_lp_stride = g_stride; d.g_lp_scale = g_scale; d.g_ent = dentropy;
-      d.dS = dS[c & 1]; d.ldS = 64; d.pcol = L.pcol; d.dST = nullptr; d.ldST = 0; d.tpad = L.tpad;
-      d.rows = nullptr; d.n_rows = n_rows; d.label_outside = 0;
-      d.tokc = tokc; d.tokl = tokl; d.lab0 = v0; d.range_rows = 0;
-      // the rows whose logits the forward kept, then tiles for the others
-      const int64_t k = std::min(vrows, kept - v0);
-      if (k > 0) {
-        ProfScope prof(PC_BWD_DS, st);
-        DsArgs<bf16_t> dq = d;
-        dq.rows = rows;  // (the tiles read the compact planes of hidden and no list; the cache is indexed by token)
-        dq.vrows = k;
-        hipLaunchKernelGGL((ds_from_logits_kernel<bf16_t, KPerm<Cfg>, Cfg::TERMS>), dim3((unsigned)(round_up(k, 256) / 64)), dim3(256), 0, st, dq,
-                           xcache + v0 * T, T, (int)L.tpad, false);
-        if ((rc = check_launch("ds_from_logits_kernel"))) return rc;
-        d.W += k * d.ldw; d.v0 += k; d.lab0 += k; d.vrows -= k; d.dS += k / 64 * d.pcol;
-      }
-      if (d.vrows > 0) {
-        d.map = TileMap::make(ntt, (int)((d.vrows + Cfg::BM - 1) / Cfg::BM), block_rows(ntt), 0);
-        p.n_ds = d.map.total;
-      }
-    }
     if (c > 0) {
-      const int cc = c - 1;
-      const int64_t v0 = (int64_t)cc * L.vchunk, vrows = std::min(L.vchunk, V - v0);
+      const Chunk& k = chunks[c - 1];
+      const int64_t v0 = k.v0, vrows = k.rows;
       const int64_t kc = round_up(vrows, KPerm<Cfg>::GV);
       if (need_dh) {
-        p.gh = make_gemm_args<Cfg>(dS[cc & 1], 64, w3[cc & 1], 3 * H, T, H, kc, dHacc, H, nullptr, 0, cc == 0 ? 0 : 1, h_tile);
+        p.gh = make_gemm_args<Cfg>(dS[k.buf], 64, w3[k.buf], 3 * H, T, H, kc, dHacc, H, nullptr, 0, c == 1 ? 0 : 1, h_tile);
         p.gh.tn = 2; p.gh.b_rows_valid = vrows; p.gh.m_dev = n_rows;
         p.gh.a_pcol = L.pcol; p.gh.a_plane = L.plane * 2; p.gh.b_plane = H * 2;
-        if (L.ksplit > 1) {
-          p.gh.ksplit = L.ksplit;
-          p.gh.kslice = round_up((kc + L.ksplit - 1) / L.ksplit, Cfg::BK);
-          p.gh.map = TileMap::make(p.gh.map.nrow_tiles, p.gh.n_tiles * L.ksplit, p.gh.map.br, p.gh.map.rows_fastest);
+        const int slices = k.alone ? wide_slices : L.ksplit;
+        if (slices > 1) {
+          p.gh.ksplit = slices;
+          p.gh.kslice = round_up((kc + slices - 1) / slices, Cfg::BK);
+          p.gh.map = TileMap::make(p.gh.map.nrow_tiles, p.gh.n_tiles * slices, p.gh.map.br, p.gh.map.rows_fastest);
           p.gh.cf_split_stride = (int64_t)(align256((size_t)T * H * 4) / 4);
         }
         p.n_gh = p.gh.map.total;
       }
       if (need_dw) {
-        p.gw = make_gemm_args<Cfg>(dS[cc & 1], 64, h3, 3 * L.ldH, vrows, H, round_up(T, 64), d_weight + v0 * H, H, nullptr, 0, 0, h_tile);
+        p.gw = make_gemm_args<Cfg>(dS[k.buf], 64, h3, 3 * L.ldH, vrows, H, round_up(T, 64), d_weight + v0 * H, H, nullptr, 0, 0, h_tile);
         p.gw.tn = 1; p.gw.perm_rows = 1; p.gw.k_dev = n_rows; p.gw.k_gran = 64;
         p.gw.a_pcol = L.pcol; p.gw.a_plane = L.plane * 2; p.gw.b_plane = L.ldH * 2;
         p.n_gw = p.gw.map.total;
@@ -299,13 +323,36 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
         p.n_gw = p.n_gh;
         p.n_gh = 0;
       }
+      if (k.alone || c == nchunks) {
+        if ((rc = launch(p))) return rc;
+        p.n_gw = p.n_gh = 0;
+      }
     }
-    if (p.n_gw + p.n_gh + p.n_ds == 0) continue;
-    ProfScope prof(PC_BWD_CHUNK, st);
-    auto kern = h_tile == 224 ? lce_bwd_chunk16_kernel<Cfg, 7> : lce_bwd_chunk16_kernel<Cfg, 8>;
-    allow_lds(kern, Cfg::LDS_BYTES);
-    hipLaunchKernelGGL(kern, dim3(p.n_gw + p.n_gh + p.n_ds), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
-    if ((rc = check_launch("lce_bwd_chunk16_kernel"))) return rc;
+    if (c == nchunks) break;
+    const Chunk& k = chunks[c];
+    const int64_t v0 = k.v0, vrows = k.rows;
+    // (the last reader of this buffer ran in the launch before the last)
+    if ((rc = launch_split({W + v0 * ldw, ldw, vrows, H, w3[k.buf], H, vrows, nullptr, nullptr}, &sh, wide, st))) return rc;
+    DsArgs<bf16_t>& d = p.ds;
+    d.W = w3[k.buf]; d.ldw = 3 * H; d.h = h3; d.ldh = 3 * L.ldH; d.labels = labels; d.T = T; d.H = H;
+    d.w_plane = H * 2; d.h_plane = L.ldH * 2; d.dS_plane = L.plane;
+    d.v0 = vocab_offset + v0; d.vrows = vrows; d.rcp_tau = 1.0f / temperature; d.c = kLog2e / temperature;
+    d.maximum = maximum; d.accumulate = accumulate; d.entropy_b = entropy_b;
+    d.g_lp = dlogprobs; d.g_lp_stride = g_stride; d.g_lp_scale = g_scale; d.g_ent = dentropy;
+    d.dS = dS[k.buf]; d.ldS = 64; d.pcol = L.pcol; d.dST = nullptr; d.ldST = 0; d.tpad = L.tpad;
+    d.rows = nullptr; d.n_rows = n_rows; d.label_outside = 0;
+    d.tokc = tokc; d.tokl = tokl; d.lab0 = v0; d.range_rows = 0;
+    if (k.kept) {
+      ProfScope prof(PC_BWD_DS, st);
+      d.rows = rows;  // (the tiles read the compact planes of hidden and no list; the cache is indexed by token)
+      hipLaunchKernelGGL((ds_from_logits_kernel<bf16_t, KPerm<Cfg>, Cfg::TERMS>), dim3((unsigned)(round_up(vrows, 256) / 64)), dim3(256), 0, st, d,
+                         xcache + v0 * T, T, (int)L.tpad, false);
+      if ((rc = check_launch("ds_from_logits_kernel"))) return rc;
+      continue;
+    }
+    d.map = TileMap::make(ntt, (int)((vrows + Cfg::BM - 1) / Cfg::BM), block_rows(ntt), 0);
+    p.n_ds = d.map.total;
+    if ((rc = launch(p))) return rc;
   }
   if (need_dh) {
     ProfScope prof(PC_DH_FINISH, st);
@@ -313,7 +360,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
     lt.labels = nullptr; lt.v0 = vocab_offset; lt.V = V; lt.g_lp = dlogprobs; lt.g_stride = g_stride; lt.scale = 0.f;
     int64_t blocks = (T * (H / 4) + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL((dh_finish_kernel<float, float, false>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, L.ksplit,
+    hipLaunchKernelGGL((dh_finish_kernel<float, float, false>), dim3((unsigned)blocks), dim3(256), 0, st, dHacc, all_slices,
                        (int64_t)(align256((size_t)T * H * 4) / 4), inv, T, H, d_hidden, lt, W, ldw);
     if ((rc = check_launch("dh_finish_kernel"))) return rc;
   }
