@@ -20,6 +20,7 @@ DEV = "cuda:0"
     (1024, 256, 65536, 0, 1, 0.02),    # a quarter of them, the most tokens that keep any
     (640, 640, 33000, 0, 0, 0.0),      # no token takes part
     (700, 256, 50003, 65536, 0, 1.0),  # part of the rows of one chunk
+    (890, 896, 52003, 0, 0, 1.0),      # the forward's last chunk on tiles of 128 tokens
 ])  # fmt: skip
 def test_kept_logits_of_planes(T, H, V, vchunk, reduction, keep):
     from verl_amd import _abi
@@ -38,6 +39,10 @@ def test_kept_logits_of_planes(T, H, V, vchunk, reduction, keep):
     plain = kernels.efficient_entropy_forward(h, w, y, reduction, 0.8)
     *kept, cache = kernels.forward_keeping_logits(h, w, y, reduction, 0.8)
     assert all(torch.equal(a, b) for a, b in zip(plain, kept))
+    if reduction == 0:
+        known = y >= 0
+        for got, want in zip(plain[:2], O.lce_forward(h, w, y.clamp(min=0), 0.8, compute_dtype=torch.float64)):
+            assert (got.double() - want)[known].abs().max() <= 1e-5 * want[known].abs().max()
     rows = V if T <= H else V * H // T // 256 * 256
     assert cache.numel() == T * ((rows + 63) // 64 * 64) * 4 <= (V + 63) * H * 4
     kernels.set_vocab_chunk(vchunk)

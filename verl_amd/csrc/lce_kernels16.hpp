@@ -100,7 +100,7 @@ struct Fwd16Stream {
 // 1004 -> 1016, 5003: 4049 -> 4080).
 template <typename Cfg>
 struct Fwd16Tails {
-  static constexpr bool value = Cfg::A_EARLY || Cfg::TERMS == 6;
+  static constexpr bool value = (Cfg::A_EARLY || Cfg::TERMS == 6) && Cfg::NBN > 5;
   template <int NBN>
   using Narrow = GemmCfg16<typename Cfg::TIN, 0, NBN, Cfg::A_EARLY, Cfg::TERMS, Cfg::A_ONCE>;
 };

@@ -39,20 +39,25 @@ TermsFwdPlan terms_fwd_plan_for(int64_t T, int64_t H, int64_t V, int64_t tiles) 
   return p;
 }
 
+// A chunk whose tiles would be half as many as the CUs or fewer is multiplied on tiles of 128 tokens instead of 256, which take 0.55 of the
+// time: all chunks of 256 tokens, and with more the last one where few rows are left for it.  Forward, us, 256 tokens: H=896 604 -> 529,
+// 3584: 2311 -> 2105, 4096: 2498 -> 2067, 5120: 3362 -> 3051; 1000 tokens of H=896 (eighteen tiles of rows in the last chunk) 1261 -> 1237.
+bool terms_fwd_half(int64_t ntt, int64_t rows) { return ntt * ((rows + 255) / 256) <= kNumCUs / 2; }
+
 // The widest chunks that a workspace of `room` bytes has space for, between two bounds that are of shapes alone.  The lower
 // one, whose workspace is always enough: 256 MB of planes, which the memory-side cache holds from the split to the product, in
 // whole rounds of tiles over the CUs.  Where they hold less than a round (few tokens, a wide weight) the upper one is a round,
 // through memory, but at most two fifths of the weight's own bytes.  The same bits whatever the width: a tile is a split of
-// its own there.  Forward in us by MiB of workspace, H=5120, V=152064: 256 tokens 257: 10684, 610: 5654, 906: 4166, 1127: 3697
-// (taken), 1495: 3325; 300 tokens 260: 10478, 611: 5534, 905: 4391 (taken, a round); 1000 tokens 287: 10632, 489: 7728 (taken, a
-// round); H=4096, V=128256: 256 tokens 260: 5987, 764: 2749 (taken), 1514: 2135; 300 tokens 262: 5869, 616: 3172, 766: 2962 (taken).
+// its own there.  Forward in us by MiB of workspace, H=5120, V=152064: 300 tokens 260: 10478, 611: 5534, 905: 4391 (taken, a round); 1000 tokens 287: 10632, 489: 7728 (taken, a
+// round); H=4096, V=128256: 300 tokens 262: 5869, 616: 3172, 766: 2962 (taken).
 TermsFwdPlan terms_fwd_plan(int64_t T, int64_t H, int64_t V, size_t room) {
   const int64_t ntt = (T + 255) / 256, nvt = (V + 255) / 256, tile_bytes = 6 * H * 256;
   const int64_t base = std::max<int64_t>(1, ((int64_t)256 << 20) / tile_bytes);  // tiles of a chunk
   const int64_t rounds = base * ntt / kNumCUs;
   if (rounds > 0) return terms_fwd_plan_for(T, H, V, std::max<int64_t>(1, rounds * kNumCUs / ntt));
   const int64_t share = V * H * 4 * 2 / 5 / tile_bytes;
-  const int64_t most = std::max(base, std::min<int64_t>(kNumCUs / ntt, share));
+  // (one tile of tokens is multiplied as two of 128: terms_fwd_half)
+  const int64_t most = ntt == 1 ? std::min<int64_t>(kNumCUs / 2, std::max(base, share)) : std::max(base, std::min<int64_t>(kNumCUs / ntt, share));
   // (chunks of one length: a shorter last one would take its round all the same)
   int64_t n = (nvt + most - 1) / most;
   const int64_t n_base = (nvt + base - 1) / base;
@@ -153,6 +158,7 @@ size_t terms_cache_bytes(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
 
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1
 typedef GemmCfg16<bf16_t, 0, 8, 0, 6> TermsCfg;
+typedef GemmCfg16<bf16_t, 0, 4, 0, 6> TermsHalfCfg;  // tiles of 128 tokens
 
 // The planes of one operand (`s`), and then, where that or the other one (`also`, null: not there yet) holds values that want
 // it, those of both once more (split_again_kernel).
@@ -197,13 +203,19 @@ int forward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, cons
     p.label_offset = label_offset + v0;
     p.parts = parts + (int64_t)done * T;
     p.split_stride = TermsCfg::BM; p.tile_step = (int64_t)p.S * TermsCfg::BM; p.split_span = rows;
-    p.map = TileMap::make(ntt, p.S, block_rows(ntt), 1);
     p.keep_rows = std::min(rows, kept - v0);
     p.xcache = p.keep_rows > 0 ? xcache + v0 * T : nullptr;
+    auto launch = [&](auto cfg) {
+      typedef decltype(cfg) Cfg;
+      const int tt = (int)((T + Cfg::BN - 1) / Cfg::BN);
+      p.map = TileMap::make(tt, p.S, block_rows(tt), 1);
+      auto kern = p.xcache ? lce_fwd16_kernel<Cfg, true> : lce_fwd16_kernel<Cfg, false>;
+      allow_lds(kern, Cfg::LDS_BYTES);
+      hipLaunchKernelGGL(kern, dim3(p.map.total), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, st, p);
+    };
     ProfScope prof(PC_FWD, st);
-    auto kern = p.xcache ? lce_fwd16_kernel<TermsCfg, true> : lce_fwd16_kernel<TermsCfg, false>;
-    allow_lds(kern, TermsCfg::LDS_BYTES);
-    hipLaunchKernelGGL(kern, dim3(p.map.total), dim3(TermsCfg::NTHREADS), TermsCfg::LDS_BYTES, st, p);
+    if (terms_fwd_half(ntt, rows)) launch(TermsHalfCfg{});
+    else launch(TermsCfg{});
     if ((rc = check_launch("lce_fwd16_kernel"))) return rc;
     done += p.S;
   }
