@@ -117,7 +117,9 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  *     cache never exceeds the weight), 4 H for LCE_DTYPE_F32_PLANES where the planes are used (of all rows of the weight up to H tokens,
  *     beyond of as many of the first as are no larger than the weight), or LCE_OPT_KEEP_LOGITS_TOKENS where that is lower; 0 for
  *     LCE_DTYPE_F32 and under diagnostic settings that force a tile variant.
- *   lce_logits_cache_bytes: size of the buffer for this shape, or 0 where none is offered: then pass NULL below.
+ *   lce_logits_cache_bytes: size of the buffer for this shape, or 0 where none is offered: then pass NULL below.  (fp32 with at
+ *     most LCE_F32_FEW_TOKENS and H tokens, either code: 0, as it has always answered; a caller that brings T * (V rounded up to 64) * 4
+ *     bytes all the same has its logits kept there under the limits of lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES).)
  *   lce_forward_keep_logits: lce_forward; with logits_cache != NULL it also writes hidden . weight^T there in fp32
  *     (private layout).  Same outputs, bit for bit.
  *   lce_backward_from_logits: lce_backward (grads_fp32 = 0) or lce_backward_f32 (grads_fp32 = 1; d_hidden, d_weight are
@@ -125,6 +127,7 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  *     and dtype, the gradient of the logits is computed from it with the same expressions, so both gradients are bit for
  *     bit those of lce_backward (LCE_DTYPE_F32_PLANES: d_weight; d_hidden may sum chunks of another width).  The cache is only
  *     read. */
+#define LCE_F32_FEW_TOKENS 128
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype);
 size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype);
 int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,

@@ -78,7 +78,7 @@ struct FewFwdShape {
   static constexpr int BK = 128 / (int)sizeof(TIN);  // K elements of a stage
   static constexpr int HROWS = (NT + 63) / 64 * 64;  // rows of a stage of hidden in LDS (64 are fetched at a time)
   static constexpr int STAGE = BM * 128 + HROWS * 128;
-  static constexpr int LDS_BYTES = 2 * STAGE + (sizeof(TIN) == 2 ? 8 * 4096 : 0);  // two stages, a store tile per wave
+  static constexpr int LDS_BYTES = 2 * STAGE + 8 * 4096;  // two stages, a store tile per wave
 };
 
 // The products of W's rows [row0, vend64) with the NT hidden rows, 256 rows of W at a time; `pass(acc, m0, vbase, busy)` gets those of
@@ -211,7 +211,7 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
   for (int i = 0; i < HL; ++i) h_off[i] = (uint32_t)((tid >> 3) + 64 * i) * h_row + (tid & 7) * 16;
   few_products<TIN, NT, AUX, HALF>(p.W, p.ldw, row0, vend64, p.H, p.h, p.T * h_row, h_off, lds,
                              [&](f32x16_t (&acc)[1][FN], int64_t m0, int vbase, bool) {
-    if constexpr (sizeof(TIN) == 2) if (p.xcache) {
+    if (p.xcache) {
       // the logits of this pass, for a backward that then has no need to recompute them.  A 32x32 block passes through 4 KB of
       // LDS of this wave's own and leaves it as whole lines, 1 KB (16 tokens x 16 rows of a panel) per store; rows in whole
       // fours, the last ones of W up to the end of the cache's panel.  Non-temporal (64 tokens, H=3584: step 632 -> 615 us,

@@ -1,5 +1,5 @@
 // fp32 inputs with at most 128 tokens: the backward as three streams, as in few_tokens.hpp, on the fp32 MFMA:
-//   d_logits    reads W once (the forward's products again) and writes [T, V]
+//   d_logits    reads W once (the forward's products again), or the logits that the forward kept, and writes [T, V]
 //   d_hidden    reads W once
 //   d_weight    writes [V, H] once
 // fp32 needs no transposing reads: v_mfma_f32_32x32x2_f32 takes one element per lane of either operand, so that a K-major operand
@@ -82,6 +82,22 @@ __global__ __launch_bounds__(512, 2) void lce_ds_few_f32_kernel(FewF32Args p) {
       }
     }
   });
+}
+
+// The same from logits that the forward kept (FwdArgs::xcache), x from the chunk's first row on: a workgroup per panel, eight lanes to a
+// position.  The same expressions, so the same bits.  Bound by HBM: 4 bytes read and 4 written per logit instead of a read of W.
+inline __global__ __launch_bounds__(256) void ds_few_f32_from_logits_kernel(FewF32Args p, const float* x) {
+  const int n = p.tokens(), v = 4 * (threadIdx.x & 7);
+  const int64_t u0 = (int64_t)blockIdx.x * 32;
+  for (int pos = threadIdx.x >> 3; pos < n; pos += 32) {
+    const f32x4_t k = p.tokc[pos];
+    const int64_t lab = p.tokl[pos] - p.lab0;
+    const f32x4_t z = load_vec<true>(reinterpret_cast<const f32x4_t*>(kept_logit(x, p.T, p.rows ? (int64_t)p.rows[pos] : pos, u0 + v)));
+    f32x4_t d;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d[r] = dlogit<true>(z[r], p.c, k[0], k[1], k[2], k[3], u0 + v + r == lab, u0 + v + r >= p.vrows, false);
+    *reinterpret_cast<f32x4_t*>(ds32_at(p.dS, p.pcol, pos, u0 + v)) = d;
+  }
 }
 
 // d_hidden.  Workgroup = 512 threads = 8 waves, one per CU; it owns columns [h0, h0 + 256) of the result for all positions and one K

@@ -272,7 +272,9 @@ int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight,
                             float* maximum, float* accumulate, float* entropy_b, void* workspace, size_t workspace_bytes,
                             void* logits_cache, size_t logits_cache_bytes, void* stream) {
   if (logits_cache) {
-    const size_t need = known_dtype(dtype) || dtype == LCE_DTYPE_F32_PLANES ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
+    const bool f32 = dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES;
+    size_t need = f32 || known_dtype(dtype) ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
+    if (f32 && need == 0 && T <= lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES)) need = few_f32_cache_bytes(T, H, V);
     if (need == 0) return fail(LCE_E_ARG, "lce_forward_keep_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");
@@ -409,7 +411,7 @@ static int backward_entry(const void* hidden, int64_t ldh, const void* weight, i
   char* ws = reinterpret_cast<char*>(align256(reinterpret_cast<size_t>(workspace)));
   return kBackward[dtype](terms ? kSelTerms : esz == 4 && few_f32(tu, T) ? kSelFewF32 : bwd_variant(tu, T, esz), hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, maximum,
                           accumulate, entropy_b, dlogprobs, dentropy, d_hidden, d_weight, grads_f32, ws, vchunk, st, vocab_offset,
-                          tu, planes && !terms ? nullptr : xcache);
+                          tu, esz == 4 && !terms && !few_f32(tu, T) ? nullptr : xcache);
 }
 
 int lce_backward_from_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,
@@ -418,9 +420,10 @@ int lce_backward_from_logits(const void* hidden, int64_t ldh, const void* weight
                              void* d_hidden, void* d_weight, int grads_fp32, void* workspace, size_t workspace_bytes, int64_t vchunk,
                              const void* logits_cache, size_t logits_cache_bytes, void* stream) {
   if (logits_cache) {
-    // (a cache on planes was written under what was set then: nothing set since changes its size, at most whether it is read)
-    const size_t need = dtype == LCE_DTYPE_F32_PLANES ? (T > 0 && H > 0 && V > 0 ? terms_cache_bytes(Tuning(), T, H, V) : 0)
-                        : known_dtype(dtype)          ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
+    // (a cache of fp32 logits was written under what was set then: nothing set since changes its size, at most whether it is read)
+    const bool f32 = dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES;
+    size_t need = f32 || !known_dtype(dtype) || T <= 0 ? 0 : lce_logits_cache_bytes(T, H, V, dtype);
+    if (f32 && T > 0 && H > 0 && V > 0) need = T <= kFewF32Tokens ? few_f32_cache_bytes(T, H, V) : dtype == LCE_DTYPE_F32 ? 0 : terms_cache_bytes(Tuning(), T, H, V);
     if (need == 0) return fail(LCE_E_ARG, "lce_backward_from_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");

@@ -99,7 +99,7 @@ int TU_FN(backward)(int sel, LCE_BWD_PARAMS) {
                             (float*)dw, ws, vchunk, st, vocab_offset, tu, xcache);
     case kSelFewF32:
       return backward_few_f32((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, mx, ac, eb, glp, gent, (float*)dh,
-                              (float*)dw, ws, vchunk, st, vocab_offset, tu);
+                              (float*)dw, ws, vchunk, st, vocab_offset, tu, xcache);
 #endif
   }
 #undef LCE_RUN

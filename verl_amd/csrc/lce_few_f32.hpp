@@ -13,11 +13,19 @@ struct FewF32Layout {
 
 // Which calls: shapes and diagnostic settings alone.  Measured, forward + backward in ms (the forward is the same), tiles of 256 x 256
 // with transposed copies of W / this way, H=3584, V=152064: 1 token 7.6 / 1.57, 32: 7.8 / 1.74, 64: 8.2 / 2.7, 100: 8.7 / 4.5, 128:
-// 8.8 / 4.6; H=896: 2.7 / 0.47, 2.8 / 0.50, 3.0 / 0.80, 3.1 / 1.31, 3.1 / 1.36; without d_weight, H=3584, 16 tokens 6.4 / 1.32.  Error
+// 8.8 / 4.6; H=896: 2.7 / 0.47, 2.8 / 0.50, 3.0 / 0.80, 3.1 / 1.31, 3.1 / 1.36; without d_weight, H=3584, 16 tokens 6.4 / 1.32.
+// With the forward's logits (few_f32_cache_bytes): H=3584, 12 tokens 1.59 -> 1.18, 64: 2.59 -> 1.94, 128: 4.58 -> 3.38; H=896, 1: 0.43 -> 0.33, 100:
+// 1.26 -> 0.96; without d_weight, H=5120, 19: 1.82 -> 1.20.  Error
 // against float64 (2-norm; H=896, V=151936, 64 tokens): d_hidden 3.8e-6 / 3.8e-6, d_weight 1.2e-7 / 4.2e-8.  Where the line lies: the
 // kernels are laid out for 128 positions (hidden and its products take half the registers there), and from 129 to 255 tokens,
-// where the planes do not yet run, the tiles do (129: 11.2 ms, 255: 11.3, 256: 8.0); wider streams have not been tried.
-bool few_f32(const Tuning& tu, int64_t T) { return T <= 128 && !tu.variant_forced && tu.few_token_gemms && !tu.split_bwd; }
+// where the planes do not yet run, the tiles do (129: 11.2 ms, 255: 11.3, 256: 6.0); wider streams have not been tried.
+constexpr int64_t kFewF32Tokens = LCE_F32_FEW_TOKENS;
+bool few_f32(const Tuning& tu, int64_t T) { return T <= kFewF32Tokens && !tu.variant_forced && tu.few_token_gemms && !tu.split_bwd; }
+
+// bytes of the logits that a forward of so few tokens keeps where it is handed the buffer
+size_t few_f32_cache_bytes(int64_t T, int64_t H, int64_t V) {
+  return T >= 1 && T <= kFewF32Tokens && T <= H && V > 0 ? (size_t)T * (size_t)logits_cache_row(V) * 4 : 0;
+}
 
 FewF32Layout few_f32_layout_for(const Tuning& tu, int64_t T, int64_t H, int64_t V, int64_t vchunk) {
   FewF32Layout L;
@@ -58,9 +66,13 @@ FewF32Layout few_f32_layout(const Tuning& tu, int64_t T, int64_t H, int64_t V, i
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1 && LCE_TU_PART == 1
 // d_logits, d_hidden and d_weight of one chunk
 template <int NT>
-int launch_few_f32(FewF32Args q, bool need_dh, bool need_dw, hipStream_t st) {
+int launch_few_f32(FewF32Args q, bool need_dh, bool need_dw, hipStream_t st, const float* x) {
   int rc;
-  {
+  if (x) {
+    ProfScope prof(PC_BWD_DS, st);
+    hipLaunchKernelGGL(ds_few_f32_from_logits_kernel, dim3((unsigned)((q.vrows + 31) / 32)), dim3(256), 0, st, q, x);
+    if ((rc = check_launch("ds_few_f32_from_logits_kernel"))) return rc;
+  } else {
     typedef FewFwdShape<float, NT> S;
     ProfScope prof(PC_BWD_DS, st);
     q.span = round_up((q.vrows + kNumCUs - 1) / kNumCUs, 32);
@@ -90,7 +102,8 @@ int launch_few_f32(FewF32Args q, bool need_dh, bool need_dw, hipStream_t st) {
 
 int backward_few_f32(const float* h, int64_t ldh, const float* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                      int reduction, const float* maximum, const float* accumulate, const float* entropy_b, const float* dlogprobs, const float* dentropy,
-                     float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu) {
+                     float* d_hidden, float* d_weight, char* ws, int64_t vchunk, hipStream_t st, int64_t vocab_offset, const Tuning& tu,
+                     const float* xcache) {
   const FewF32Layout L = few_f32_layout(tu, T, H, V, vchunk);
   int* rows = reinterpret_cast<int*>(ws + L.off_rows);
   int* inv = reinterpret_cast<int*>(ws + L.off_inv);
@@ -122,8 +135,9 @@ int backward_few_f32(const float* h, int64_t ldh, const float* W, int64_t ldw, c
     q.accumulate = c > 0;
     q.dW = d_weight ? d_weight + v0 * H : nullptr;
     const bool dh = d_hidden != nullptr, dw = d_weight != nullptr;
-    rc = L.nt == 32 ? launch_few_f32<32>(q, dh, dw, st) : L.nt == 64 ? launch_few_f32<64>(q, dh, dw, st)
-       : L.nt == 96 ? launch_few_f32<96>(q, dh, dw, st) : launch_few_f32<128>(q, dh, dw, st);
+    const float* x = xcache ? xcache + v0 * T : nullptr;
+    rc = L.nt == 32 ? launch_few_f32<32>(q, dh, dw, st, x) : L.nt == 64 ? launch_few_f32<64>(q, dh, dw, st, x)
+       : L.nt == 96 ? launch_few_f32<96>(q, dh, dw, st, x) : launch_few_f32<128>(q, dh, dw, st, x);
     if (rc) return rc;
   }
   if (!d_hidden) return LCE_OK;

@@ -129,6 +129,14 @@ def _check_inputs(hidden, weight, labels):
     return _abi.DTYPE_F32_PLANES if hidden.dtype == torch.float32 else _abi.dtype_code(hidden.dtype)
 
 
+def kept_logits_size(T: int, H: int, V: int, code: int) -> int:
+    """Bytes of the logits that a forward of this shape keeps for its backward (0: none)."""
+    lib = _abi.load()
+    if code == _abi.DTYPE_F32_PLANES and T <= min(128, H):  # (LCE_F32_FEW_TOKENS: the query answers 0 for them)
+        return T * ((V + 63) // 64 * 64) * 4 if 0 < T <= lib.lce_logits_cache_max_tokens(H, code) else 0
+    return lib.lce_logits_cache_bytes(T, H, V, code)
+
+
 def efficient_entropy_forward(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -144,7 +152,7 @@ def efficient_entropy_forward(
 def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0, dist_process_group=None, *, keep_logits=True):
     """``efficient_entropy_forward`` plus a sixth value: the kept logits for ``efficient_entropy_backward(...,
     logits_cache=)``, or ``None`` where the library keeps none (16-bit inputs: more tokens than half the hidden
-    size; fp32: fewer than 256 or more than four times the hidden size; ``keep_logits=False``).
+    size; fp32: 129 to 255, or more than four times the hidden size; ``keep_logits=False``).
     With few tokens fp32 ``[T, V]`` is a fraction of the weight itself, so the autograd node keeps it like any activation
     and the backward skips the pass over ``[V, H]`` and the ``T x V x H`` product that recompute it (not in the
     reference, which always recomputes)."""
@@ -170,7 +178,7 @@ def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0,
     with _abi.on_device(dev):
         ws_bytes = lib.lce_forward_workspace_bytes(T, H, V, code)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-        cache_bytes = lib.lce_logits_cache_bytes(T, H, V, code) if keep_logits else 0
+        cache_bytes = kept_logits_size(T, H, V, code) if keep_logits else 0
         if cache_bytes:
             cache = torch.empty((cache_bytes,), device=dev, dtype=torch.uint8)
         rc = lib.lce_forward_keep_logits(
