@@ -127,7 +127,7 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  *     and dtype, the gradient of the logits is computed from it with the same expressions, so both gradients are bit for
  *     bit those of lce_backward (LCE_DTYPE_F32_PLANES: d_weight; d_hidden may sum chunks of another width).  The cache is only
  *     read. */
-#define LCE_F32_FEW_TOKENS 128
+#define LCE_F32_FEW_TOKENS 255
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype);
 size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype);
 int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,
@@ -345,7 +345,7 @@ int lce_num_variants(void);
  * which an XCD's consecutive blocks of d_logits tiles walk the chunk: -1 = chosen by size (default), 0 = along the
  * vocabulary, 1 = along the tokens.  LCE_OPT_DHIDDEN_KSPLIT (default 0 = by shape): K slices of the d_hidden GEMM, each
  * with its own fp32 partial that is summed in a fixed order afterwards (0..16; changes the workspace size).
- * LCE_OPT_FEW_TOKEN_GEMMS (default 1): with at most 128 tokens the gradient GEMMs of the backward, and with fp32 inputs
+ * LCE_OPT_FEW_TOKEN_GEMMS (default 1): with at most 128 tokens (fp32: 255) the gradient GEMMs of the backward, and with fp32 inputs
  * its d_logits too, run as streaming kernels; 0 = the 256 x 256 tile kernels, which the tests compare them with (changes
  * the workspace size). */
 enum {

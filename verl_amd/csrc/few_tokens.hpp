@@ -1,5 +1,5 @@
 // Few tokens (gfx950).  16-bit inputs: the forward up to 96, d_hidden up to 128, d_weight up to 256, and d_logits from kept
-// logits; fp32 inputs: the forward up to 128.
+// logits; fp32 inputs: the forward up to 128 at a time.
 //
 // With T <= 128 every product is one streaming pass over a [V, H] matrix and bound by HBM, not by the matrix cores:
 //   logits      W[v] . hidden[t]                        reads W once; nothing is written (or the kept logits)
@@ -232,7 +232,7 @@ LCE_DEV void fwd_few_body(const FwdArgs<TIN>& p, char* lds) {
           const f32x4_t x4 = *reinterpret_cast<const f32x4_t*>(sC + (q >> 1) * 2048 + tl * 64 + ((p4 ^ ((tl >> 1) & 3)) * 16));
           const int v = vbase + 16 * (q >> 1) + 4 * p4;
           const int64_t t = j * 32 + tl;
-          if (t < p.T && v < vend) __builtin_nontemporal_store(x4, reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.T, t, v)));
+          if (t < p.T && v < vend) __builtin_nontemporal_store(x4, reinterpret_cast<f32x4_t*>(kept_logit(p.xcache, p.xtok, t, v)));
         }
       }
     }

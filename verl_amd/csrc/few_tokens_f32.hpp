@@ -1,4 +1,5 @@
-// fp32 inputs with at most 128 tokens: the backward as three streams, as in few_tokens.hpp, on the fp32 MFMA:
+// fp32 inputs with at most 255 tokens: the backward as three streams, as in few_tokens.hpp, on the fp32 MFMA (from 129 on the first two
+// in two groups of positions):
 //   d_logits    reads W once (the forward's products again), or the logits that the forward kept, and writes [T, V]
 //   d_hidden    reads W once
 //   d_weight    writes [V, H] once
@@ -31,10 +32,12 @@ struct FewF32Args {
   int ksplit, accumulate;       // accumulate: 0 store, 1 add to what is there (second and later chunks)
   float* dW;           // rows of d_weight of this chunk, [vrows][H]
   int n_su;            // d_weight: workgroups side by side along the vocabulary
+  int first;           // d_logits and d_hidden: this launch's first position (dS, tokc, tokl, rows and dHp point there)
+  int most;            // positions of a launch
 
   LCE_DEV int tokens() const {
-    const int t = (int)T;
-    return n_rows && *n_rows < t ? *n_rows : t;
+    const int t = (int)T, all = n_rows && *n_rows < t ? *n_rows : t, n = all - first;
+    return n < 0 ? 0 : n < most ? n : most;
   }
 };
 
@@ -121,6 +124,7 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_f32_kernel(FewF32Args p) {
   const int64_t k_begin = (int64_t)s * p.kslice, k_left = p.vrows - k_begin;
   const int n_st = k_left <= 0 ? 0 : (int)(((k_left < p.kslice ? k_left : p.kslice) + 31) / 32);  // stages
   const int n = p.tokens();
+  if (n == 0) return;  // (nobody reads partials of positions beyond the tokens)
   f32x16_t acc[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j)
@@ -208,21 +212,22 @@ __global__ __launch_bounds__(512, 2) void lce_dh_few_f32_kernel(FewF32Args p) {
 // d_weight.  Workgroup = 512 threads = 8 waves, one per CU; a wave keeps hidden of its 64 columns in registers as MFMA operands and the
 // workgroup walks the panels id / n_ht, id / n_ht + n_su, ... of dS:  C[m = v][n = h] = sum_t dS[t][v] hidden[t][h].  A lane holds one
 // column of 16 rows, 32 lanes a whole line of a row, so the results are stored as they lie.
+// (Beyond 128 positions it is 32 of its columns instead of 64: the same registers.)
 template <int KT>
 struct FewDwF32Shape {
-  static constexpr int HW = 512, TILE = (KT + 63) / 64 * 64 * 128, LDS_BYTES = 2 * TILE;
+  static constexpr int NB = KT > 128 ? 1 : 2, HW = 256 * NB, TILE = (KT + 63) / 64 * 64 * 128, LDS_BYTES = 2 * TILE;
 };
 
 template <int KT>
 __global__ __launch_bounds__(512, 2) void lce_dw_few_f32_kernel(FewF32Args p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   typedef FewDwF32Shape<KT> S;
-  constexpr int HW = S::HW, KP = KT / 2, BL = S::TILE / 8192, NB = 2;
+  constexpr int HW = S::HW, KP = KT / 2, BL = S::TILE / 8192, NB = S::NB;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, hh = lane >> 5, ln = lane & 31;
   const int n_ht = (int)((p.H + HW - 1) / HW);
   const int id = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);  // (as in lce_dw_few_kernel)
   if (id >= n_ht * p.n_su) return;
-  const int64_t h0 = (int64_t)(id % n_ht) * HW, hw = h0 + 64 * wave;
+  const int64_t h0 = (int64_t)(id % n_ht) * HW, hw = h0 + 32 * NB * wave;
   const int64_t n_pan = (p.vrows + 31) / 32;
   const int n = p.tokens();
   u32x4_t pre[BL];

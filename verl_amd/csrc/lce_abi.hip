@@ -201,7 +201,9 @@ static size_t forward_workspace_need(int64_t T, int64_t V, int max_splits) {
 
 // (answered for LCE_DTYPE_F32: the least that is enough for either code of fp32)
 size_t lce_forward_workspace_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
-  const size_t need = forward_workspace_need(T, V, kMaxSplits);
+  // (129 to 255 tokens of fp32: room for a split per CU of their first 128)
+  const bool twice = (dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES) && T > 128 && T <= kFewF32Tokens;
+  const size_t need = std::max(forward_workspace_need(T, V, kMaxSplits), twice ? (size_t)kNumCUs * 128 * 16 + 4096 : 0);
   if (T <= 0 || H <= 0 || V <= 0 || (dtype != LCE_DTYPE_F32 && dtype != LCE_DTYPE_F32_PLANES)) return need;
   const Tuning tu = tuning_snapshot();
   if (!use_terms(tu, T, H, V)) return need;
@@ -236,6 +238,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   if (!tu.variant_forced) {
     if (T <= 64) sel = kSelT64;
     else if (T <= 128) sel = kSelT128;
+    else if (esize(dtype) == 4 && T <= kFewF32Tokens) sel = kSelFewTwice;
     else if (esize(dtype) == 2 && forward_tiles_192(T, V)) sel = kSelN192;
     else if (esize(dtype) == 2) sel = T > kCore16MinTokensFwd ? kVariantCore16 : kSelWEarly;
     else if (T <= 512) sel = 0;  // W (the A operand) streams from HBM: give it the early slot
@@ -246,7 +249,7 @@ static int forward_entry(const void* hidden, int64_t ldh, const void* weight, in
   // (the square tile's stream of slabs wants two of them)
   if (sel == kVariantCore16 && esize(dtype) == 2 && H < 128) sel = kSelN192;
   if (terms) sel = kSelTerms;
-  if (xcache && !terms && sel != kSelT64 && sel != kSelT128 && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
+  if (xcache && !terms && sel != kSelT64 && sel != kSelT128 && sel != kSelFewTwice && !((sel == kVariantCore16 || sel == kSelN192 || sel == kSelWEarly) && esize(dtype) == 2))
     return fail(LCE_E_ARG, "forward: tile selector %d cannot keep the logits", sel);
   return kForward[dtype](sel, hidden, ldh, weight, ldw, labels, T, H, V, temperature, reduction, logprobs, entropy, maximum,
                          accumulate, entropy_b, ws, workspace_bytes, st, label_offset, shard_out, max_splits, xcache);

@@ -60,6 +60,9 @@ int TU_FN(forward)(int sel, LCE_FWD_PARAMS) {
     case kSelT128:
       if (T <= 96) LCE_FEW(96);
       LCE_FEW(128);
+    case kSelFewTwice:
+      return forward_few_twice((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws,
+                               ws_bytes, st, label_offset, shard_out, max_splits, xcache);
     case kSelTerms:
       return forward_terms((const float*)h, ldh, (const float*)W, ldw, labels, T, H, V, temperature, reduction, lp, ent, mx, ac, eb, ws,
                            ws_bytes, st, label_offset, shard_out, xcache);

@@ -63,8 +63,8 @@ struct Tuning {
 
 // tile selectors of the per-type launchers: 0..3 are the variants of lce_set_variant, then the two few-token forward tiles
 // and the 16x16x32 loop on tiles 192 tokens wide or with the weight early, the bfloat16 planes of fp32 inputs (lce_terms.hpp), and their backward with
-// few tokens (lce_few_f32.hpp)
-enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8, kSelWEarly = 9 };
+// few tokens, and their forward in two groups of tokens (lce_few_f32.hpp)
+enum { kSelT64 = 4, kSelT128 = 5, kSelN192 = 6, kSelTerms = 7, kSelFewF32 = 8, kSelWEarly = 9, kSelFewTwice = 10 };
 
 // The launchers of one element type each (lce_dtype.hip compiles them as separate objects).  `sel` is a tile selector;
 // the other arguments are those of forward_impl / backward_impl / launch_gemm below with untyped pointers.
@@ -421,7 +421,7 @@ int forward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::TI
 template <typename TIN, int NT>
 int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int64_t* labels, int64_t T, int64_t H, int64_t V, float temperature,
                 int reduction, float* logprobs, float* entropy, float* maximum, float* accumulate, float* entropy_b, char* ws, hipStream_t st,
-                int64_t label_offset, float* shard_out, int max_splits, float* xcache) {
+                int64_t label_offset, float* shard_out, int max_splits, float* xcache, int64_t xtok = 0) {
   const int most = max_splits < kNumCUs ? max_splits : kNumCUs;
   FwdArgs<TIN> p;
   p.split_stride = p.split_span = round_up((V + most - 1) / most, 16);
@@ -430,7 +430,7 @@ int forward_few(const TIN* h, int64_t ldh, const TIN* W, int64_t ldw, const int6
   p.c = kLog2e / temperature;
   p.parts = reinterpret_cast<f32x4_t*>(ws);
   p.xlabel = reinterpret_cast<float*>(ws + align256((size_t)S * T * 16));
-  p.S = S; p.tile_step = 256; p.label_offset = label_offset; p.xcache = xcache; p.w_plane = p.h_plane = 0;
+  p.S = S; p.tile_step = 256; p.label_offset = label_offset; p.xcache = xcache; p.xtok = xtok ? xtok : T; p.w_plane = p.h_plane = 0;
   p.once_rows = read_w_once(V, ldw * (int64_t)sizeof(TIN), xcache) ? V : T > 64 ? 0 : V - kMallBytes / 4 / (ldw * (int64_t)sizeof(TIN));
   float* lp_tok = reduction == LCE_REDUCTION_NONE ? logprobs : reinterpret_cast<float*>(ws + align256((size_t)S * T * 16) + align256((size_t)T * 4));
   {

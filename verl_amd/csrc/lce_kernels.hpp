@@ -58,6 +58,7 @@ struct FwdArgs {
   float* xcache;
   int64_t keep_rows;  // operands in planes: of the first so many rows of W only (V, or a multiple of the tile's rows)
   int64_t w_plane, h_plane;  // W and h in bfloat16 planes (GemmCfg16, TERMS == 6): bytes from plane to plane
+  int64_t xtok;       // streaming kernels: tokens of the kept logits (this launch may have some of them)
   int64_t once_rows;  // up to 96 tokens: workgroups whose rows start before this one read W with non-temporal loads
 };
 

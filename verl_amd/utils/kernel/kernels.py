@@ -132,7 +132,7 @@ def _check_inputs(hidden, weight, labels):
 def kept_logits_size(T: int, H: int, V: int, code: int) -> int:
     """Bytes of the logits that a forward of this shape keeps for its backward (0: none)."""
     lib = _abi.load()
-    if code == _abi.DTYPE_F32_PLANES and T <= min(128, H):  # (LCE_F32_FEW_TOKENS: the query answers 0 for them)
+    if code == _abi.DTYPE_F32_PLANES and T <= min(255, H):  # (LCE_F32_FEW_TOKENS: the query answers 0 for them)
         return T * ((V + 63) // 64 * 64) * 4 if 0 < T <= lib.lce_logits_cache_max_tokens(H, code) else 0
     return lib.lce_logits_cache_bytes(T, H, V, code)
 
@@ -152,7 +152,7 @@ def efficient_entropy_forward(
 def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0, dist_process_group=None, *, keep_logits=True):
     """``efficient_entropy_forward`` plus a sixth value: the kept logits for ``efficient_entropy_backward(...,
     logits_cache=)``, or ``None`` where the library keeps none (16-bit inputs: more tokens than half the hidden
-    size; fp32: 129 to 255, or more than four times the hidden size; ``keep_logits=False``).
+    size; fp32: four times the hidden size; ``keep_logits=False``).
     With few tokens fp32 ``[T, V]`` is a fraction of the weight itself, so the autograd node keeps it like any activation
     and the backward skips the pass over ``[V, H]`` and the ``T x V x H`` product that recompute it (not in the
     reference, which always recomputes)."""
