@@ -31,16 +31,17 @@ struct KPerm<GemmCfg16<TIN, TR, NBN, AE, TERMS, AO, NBM>> {
 // forward
 // ------------------------------------------------------------------------------------------------
 // folds one finished tile into the running per-token statistics (FULL: no padded vocabulary rows in the tile)
-template <typename Cfg, bool FULL>
+template <typename Cfg, bool FULL, typename F>
 LCE_DEV void fwd16_fold(const FwdArgs<typename Cfg::TIN>& p, f32x4_t (&acc)[Cfg::NB][Cfg::NBN], float (&m)[Cfg::NBN],
                         float (&a)[Cfg::NBN], float (&b)[Cfg::NBN], const int (&lab)[Cfg::NBN], int vbase, int vend, int64_t tok0, int g4,
-                        int l16) {
+                        int l16, F&& column) {
   constexpr int NB = Cfg::NB, NBN = Cfg::NBN;
 #pragma unroll
   for (int j = 0; j < NBN; ++j) {
     // One block column at a time (register pressure).  Its accumulators are in AGPRs up to here: the compiler otherwise reads
     // all 256 of a lane ahead of the first column and keeps other values in scratch memory meanwhile.
     GemmCore16<Cfg>::stay_column(acc, j);
+    column(j);
     float x[NB * 4];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -154,8 +155,8 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
         g.prologue(lds, p.H);
       }
       const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
-      if (m0 + Cfg::BM <= vend64) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
-      else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
+      if (m0 + Cfg::BM <= vend64) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16, [](int) {});
+      else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16, [](int) {});
       if (anew) g.stream_begin(lds, st);
     }
     GemmCore16<Cfg>::template wait_vm<0>();  // (the last tile's loads ahead, which nobody reads)
@@ -164,46 +165,64 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
       g.main(lds, p.H, acc);
       const int vbase = (int)m0 + g.wave_m * Cfg::WM;  // vocabulary index of this wave's first row
       const bool full = m0 + Cfg::BM <= vend64;
-      if (KEEP && (Cfg::TERMS == 1 || m0 < p.keep_rows)) {
-        // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.  Issued AHEAD of the next
-        // tile's first loads: the K loop waits on counts of outstanding vector-memory operations, and with the stores older
-        // than every load it waits for, those counts mean what they say.  The count is a 6-bit field: the stores are issued two
-        // block columns at a time, and behind the last column, whichever it is, so many are waited for that with the
-        // prologue's loads behind them fewer than 64 operations are ever in flight (8 stores a column, 12 where the compiler gives
-        // lanes without a token a store of their own; tests/test_ring_loads_on_cpu.py counts them on the listing).
-        // Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
-        constexpr int kColumn = NB + NB / 2, kBehindLast = Cfg::TERMS == 6 ? 16 : 24, kBetween = 32;
-        constexpr int kPrologue = Cfg::TERMS == 6 ? 2 * Cfg::HL + 3 * Cfg::HLB : 2 * (Cfg::HL + Cfg::HLB);
-        static_assert(kBetween + 2 * kColumn < 64 && 4 * kColumn < 64 && kBehindLast + kPrologue < 64, "vmcnt range");
-        const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
-        // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
-        const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
-        const int row_at = g4 * 16, panel = (int)p.T * 64;
+      auto fold = [&](auto&& column) {
+        if (full) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16, column);
+        else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16, column);
+      };
+      // With kept logits a column is stored just before it is folded in, so that the stores leave during the fold, and the next
+      // tile's first loads come behind both: the K loop waits on counts of outstanding vector-memory operations, and with the stores
+      // older than every load it waits for, those counts mean what they say.  (With six products there are not the registers for it:
+      // the stores first, then the loads, then the fold.)  Forward + backward against that order, us: H=896, 130 tokens 261 -> 258, 299
+      // with a frozen head 300 -> 295; H=3584, 256: 896 -> 892, 1000: 2934 -> 2922, 1700: 4849 -> 4833; H=5120, 400: 2068 -> 2055.
+      constexpr bool kWithFold = KEEP && Cfg::TERMS == 1;
+      if constexpr (KEEP) {
+        if (Cfg::TERMS == 1 || m0 < p.keep_rows) {
+          // a lane holds four consecutive vocabulary rows of a token per block: one 16-byte store.
+          // The count is a 6-bit field: four columns' stores, then two at a time, and behind the last column, whichever it is, so many
+          // are waited for that with the prologue's loads behind them fewer than 64 operations are ever in flight (8 stores a
+          // column, 12 where the compiler gives lanes without a token a store of their own; tests/test_ring_loads_on_cpu.py counts
+          // them on the listing).  Non-temporal: 130 tokens, H=3584, step 812 -> 794 us, 192: 859 -> 842, level from 333 on.
+          constexpr int kColumn = NB + NB / 2, kBehindLast = Cfg::TERMS == 6 ? 16 : 24, kBetween = 32;
+          constexpr int kPrologue = Cfg::TERMS == 6 ? 2 * Cfg::HL + 3 * Cfg::HLB : 2 * (Cfg::HL + Cfg::HLB);
+          static_assert(kBetween + 2 * kColumn < 64 && 4 * kColumn < 64 && kBehindLast + kPrologue < 64, "vmcnt range");
+          const int64_t t0 = n0 + g.wave_n * Cfg::WN + l16;
+          // the eight panels of this wave's rows; tokens beyond T and rows beyond the split (whole fours) are dropped
+          const buf_t kept = make_buf(kept_logit(p.xcache, p.T, 0, vbase), (int64_t)NB * p.T * 64);
+          const int row_at = g4 * 16, panel = (int)p.T * 64;
+          auto store = [&](int j) {
+            const int at = t0 + j * 16 < p.T ? (int)(t0 + j * 16) * 64 + row_at : kBufNowhere;
 #pragma unroll
-        for (int j = 0; j < NBN; ++j) {
-          GemmCore16<Cfg>::stay_column(acc, j);
-          const int at = t0 + j * 16 < p.T ? (int)(t0 + j * 16) * 64 + row_at : kBufNowhere;
+            for (int i = 0; i < NB; ++i) {
+              const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
+              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, kBufNonTemporal);
+            }
+            if (kWithFold) __builtin_amdgcn_sched_barrier(0);  // (ahead of the column's fold, all of them)
+            if (j % 2 == 1 && j >= 3 && j < NBN - 1) {
+              __builtin_amdgcn_sched_barrier(0);
+              GemmCore16<Cfg>::template wait_vm<kBetween>();
+            }
+          };
+          if constexpr (kWithFold) {
+            fold(store);
+          } else {
 #pragma unroll
-          for (int i = 0; i < NB; ++i) {
-            const int o = at == kBufNowhere || (!full && vbase + 16 * i + 4 * g4 >= vend) ? kBufNowhere : at + i * panel;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), kept, o, 0, kBufNonTemporal);
+            for (int j = 0; j < NBN; ++j) {
+              GemmCore16<Cfg>::stay_column(acc, j);
+              store(j);
+            }
           }
-          if (j == NBN - 1 || (j % 2 == 1 && j >= 3)) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (j == NBN - 1) GemmCore16<Cfg>::template wait_vm<kBehindLast>();
-            else GemmCore16<Cfg>::template wait_vm<kBetween>();
-          }
+          __builtin_amdgcn_sched_barrier(0);
+          GemmCore16<Cfg>::template wait_vm<kBehindLast>();
+          __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
       }
-      // the next tile's first slabs fly while this tile's statistics are folded in
       __syncthreads();  // every wave is past its last LDS read and has drained its own loads
       if (m0 + p.tile_step < vend64) {
         g.init(p.W, p.ldw, m0 + p.tile_step, vend64, p.h, p.ldh, n0, p.T);
         g.prologue(lds, p.H);
       }
-      if (full) fwd16_fold<Cfg, true>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
-      else fwd16_fold<Cfg, false>(p, acc, m, a, b, lab, vbase, vend, n0 + g.wave_n * Cfg::WN, g4, l16);
+      // the next tile's first slabs fly while this tile's statistics are folded in
+      if constexpr (!kWithFold) fold([](int) {});
     }
   }
   __syncthreads();
