@@ -530,20 +530,29 @@ int dh_ksplit_alone(int64_t T, int64_t H, int64_t vchunk, bool wide, double* cos
 // 700) 12.6 / 15.0, 1000 of 896 (16, 875) 10.3 / 14.0, 333 of 3584 (9, 1165) 13.0 / 15.7, 1000 of 3584 37 / 44.
 bool dh_sum_deep(int slices, int64_t workgroups) { return slices > 8 && 2 * workgroups <= 5 * kNumCUs; }
 
-// The same choice for every number of row tiles that may turn out to take part, within the memory that `ksplit` partials of all
-// T rows have.  Forward + backward in us, bf16, slices counted for all tokens / this way, by the tokens with gradient: H=4096, V=128256,
-// 1000 tokens, all 2615 / 2615, 750: 2300 / 2245, 500: 2010 / 1865, 300: 1850 / 1700, 250: 1770 / 1470, 100: 1635 / 1350; 2000 tokens,
+// The same choice, and that of the tiles' width, for every number of rows that may turn out to take part, within the memory that `ksplit`
+// partials of all T rows have.  Forward + backward in us, bf16, slices counted for all tokens / this way, by the tokens with gradient: H=4096,
+// V=128256, 1000 tokens, all 2615 / 2615, 750: 2300 / 2245, 500: 2010 / 1865, 300: 1850 / 1700, 250: 1770 / 1470, 100: 1635 / 1350; 2000 tokens,
 // 1000: 3900 / 3550, 400: 3340 / 2607; H=5120, V=152064, 1500 tokens, all 5680 / 5680, 750: 4470 / 4000, 300: 3860 / 3082; H=3584, 333
 // tokens, 200: 1090 / 1090, 100: 922 / 868.
+// The width of the tiles for all tokens / for these, 1000 tokens, d_hidden and d_weight with what surrounds them, H=4096: 100: 516 / 484, 300:
+// 900 / 787, 350: 942 / 828, 400: 999 / 954, 560: 1301 / 1185, from 600 on and at 200 to 256 level; H=3584, 300: 897 / 819, 560: 1339 / 1227;
+// forward + backward, 700 tokens with a frozen head 1438 / 1329, H=5120, 1500: 4901 / 4616, H=896, 700: 627 / 602.
 DhSlices dh_slices_by_rows(int64_t T, int64_t H, int64_t vchunk, bool wide, int ksplit) {
   DhSlices d = {};
-  d.tile_rows = wide ? 256 : 192;
-  const int all = d.tiles(T);
-  const int64_t room = (int64_t)ksplit * (int64_t)(align256((size_t)T * H * 4) / 4);
-  for (int r = 1; r <= all; ++r) {
-    const int64_t rows = std::min<int64_t>(T, (int64_t)r * d.tile_rows);
-    double cost;
-    d.n[r - 1] = r == all ? (uint8_t)ksplit : (uint8_t)dh_ksplit_alone(rows, H, vchunk, wide, &cost, (int)std::min<int64_t>(32, room / DhSlices::stride(rows, H)));
+  const int64_t room = (int64_t)ksplit * (int64_t)(align256((size_t)T * H * 4) / 4), tile = wide ? 256 : 192;
+  for (int b = 0; b <= DhSlices::bucket(T); ++b) {
+    const int64_t rows = std::min<int64_t>(T, 64 * (b + 1));
+    const int most = (int)std::min<int64_t>(32, room / DhSlices::stride(rows, H));
+    double c256, c192;
+    const int s256 = dh_ksplit_alone(rows, H, vchunk, true, &c256, most), s192 = dh_ksplit_alone(rows, H, vchunk, false, &c192, most);
+    bool narrow = c192 < c256;
+    if ((rows + tile - 1) / tile == (T + tile - 1) / tile && narrow == !wide) {  // (as many tiles as for all rows)
+      d.n[b] = (uint8_t)ksplit;
+    } else {
+      d.n[b] = (uint8_t)(narrow ? s192 : s256);
+    }
+    if (narrow) d.narrow |= 1u << b;
   }
   return d;
 }
@@ -942,28 +951,34 @@ int backward_impl(const typename Cfg::TIN* h, int64_t ldh, const typename Cfg::T
         if constexpr (Cfg::CORE16) {
           // (one chunk: no d_logits tiles share this launch)
           if (L.mid && !tu.split_bwd && need_dh) {
-            auto launch_dh_on = [&](auto cfg) {
-              typedef decltype(cfg) DhCfg;
+            auto launch_dh = [&](auto wide_cfg, auto narrow_cfg) {
+              typedef decltype(wide_cfg) Wide;
+              typedef decltype(narrow_cfg) Narrow;
               GemmArgs<TIN> q = p.gh;
-              const int tm = (int)((T + DhCfg::BN - 1) / DhCfg::BN);
+              const int tm = (int)(L.mid_192 ? (T + 191) / 192 : (T + 255) / 256);
               q.map = TileMap::make(tm, q.n_tiles * L.ksplit, block_rows(tm), 1);
               int grid = q.map.total;
               if (one_prep && tu.dh_ksplit <= 0) {
-                by_rows = dh_slices_by_rows(T, H, L.vchunk, DhCfg::BN == 256, L.ksplit);
-                for (int r = 1; r <= tm; ++r) grid = std::max(grid, TileMap::make(r, q.n_tiles * by_rows.n[r - 1], 1, 1).total);
+                by_rows = dh_slices_by_rows(T, H, L.vchunk, !L.mid_192, L.ksplit);
+                for (int b = 0; b <= DhSlices::bucket(T); ++b) {
+                  const int64_t rows = std::min<int64_t>(T, 64 * (b + 1)), tile = by_rows.tile(rows);
+                  grid = std::max(grid, TileMap::make((int)((rows + tile - 1) / tile), q.n_tiles * by_rows.n[b], 1, 1).total);
+                }
               }
               ProfScope prof(PC_GEMM_DH, st);
-              allow_lds(lce_dh16_kernel<DhCfg>, DhCfg::LDS_BYTES);
-              hipLaunchKernelGGL(lce_dh16_kernel<DhCfg>, dim3((unsigned)grid), dim3(DhCfg::NTHREADS), DhCfg::LDS_BYTES, st, q, by_rows);
+              auto kern = lce_dh16_kernel<Wide, Narrow>;
+              allow_lds(kern, Wide::LDS_BYTES);
+              hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(Wide::NTHREADS), Wide::LDS_BYTES, st, q, by_rows, L.mid_192);
               return check_launch("lce_dh16_kernel");
             };
-            auto launch_dh = [&](auto variant) {
-              typedef typename decltype(variant)::Cfg DhCfg;
-              return h_tile == 224 ? launch_dh_on(typename Hidden224<DhCfg>::type{}) : launch_dh_on(DhCfg{});
+            auto launch_on = [&](auto wide, auto narrow) {
+              typedef typename decltype(wide)::Cfg W;
+              typedef typename decltype(narrow)::Cfg N;
+              return h_tile == 224 ? launch_dh(typename Hidden224<W>::type{}, typename Hidden224<N>::type{}) : launch_dh(W{}, N{});
             };
-            const bool once = need_dw && T <= (L.mid_192 ? 192 : 512);
-            if (L.mid_192) rc = once ? launch_dh(VariantN192<TIN, 1>{}) : launch_dh(VariantN192<TIN, 0>{});
-            else rc = once ? launch_dh(VariantWEarly<TIN, 1>{}) : launch_dh(VariantWEarly<TIN, 0>{});
+            if (need_dw && T <= 192) rc = launch_on(VariantWEarly<TIN, 1>{}, VariantN192<TIN, 1>{});
+            else if (need_dw && T <= 512) rc = launch_on(VariantWEarly<TIN, 1>{}, VariantN192<TIN, 0>{});
+            else rc = launch_on(VariantWEarly<TIN, 0>{}, VariantN192<TIN, 0>{});
             if (rc) return rc;
             p.n_gh = 0;
           }

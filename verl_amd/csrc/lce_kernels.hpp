@@ -697,15 +697,17 @@ LCE_DEV void ds_tile(const DsArgs<typename Cfg::TIN>& p, int bid, char* lds) {
 //   out_mode 0: Cf = acc           1: Cf += acc
 //            2: Ct = (TIN)acc      3: Ct = (TIN)(Cf + acc)
 // ------------------------------------------------------------------------------------------------
-// K slices of a d_hidden product that is a launch of its own, by the row tiles that take part: only the device knows how many
-// tokens have a gradient, and slices counted for all of them leave the CUs of the other rows' tiles idle.  With r tiles (of tile_rows
-// rows) n[r - 1] slices, whose fp32 partials lie stride(rows) elements apart.  n[0] == 0: not in use.
-constexpr int kDhRowTiles = 11;
+// Tile width and K slices of a d_hidden product that is a launch of its own, by the rows that take part: only the device knows how many
+// tokens have a gradient; slices counted for all of them leave the CUs of the other rows' tiles idle, and a width that fits all of them
+// may not fit these.  For 64 (b - 1) + 1 to 64 b rows, tiles 192 rows wide where bit b - 1 of `narrow` is set and 256 otherwise, n[b - 1]
+// slices, whose fp32 partials lie stride(rows) elements apart.  n[0] == 0: not in use.
+constexpr int kDhRows = 2048;
 struct DhSlices {
-  uint8_t n[kDhRowTiles];
-  int tile_rows;
-  LCE_HOST_DEV int tiles(int64_t rows) const { return rows > tile_rows ? (int)((rows + tile_rows - 1) / tile_rows) : 1; }
-  LCE_HOST_DEV int count(int64_t rows) const { return n[tiles(rows) - 1]; }
+  uint8_t n[kDhRows / 64];
+  uint32_t narrow;
+  LCE_HOST_DEV static int bucket(int64_t rows) { return rows > 64 ? (int)((rows + 63) / 64) - 1 : 0; }
+  LCE_HOST_DEV int count(int64_t rows) const { return n[bucket(rows)]; }
+  LCE_HOST_DEV int tile(int64_t rows) const { return narrow >> bucket(rows) & 1 ? 192 : 256; }
   LCE_HOST_DEV static int64_t stride(int64_t rows, int64_t H) { return (rows * H + 63) / 64 * 64; }
 };
 

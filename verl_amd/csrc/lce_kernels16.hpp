@@ -918,19 +918,22 @@ __global__ __launch_bounds__(Cfg::NTHREADS) void gemm16_tn_kernel(GemmArgs<typen
   gemm16_tn_tile<GemmCfg16<typename Cfg::TIN, 1>, Cfg>(p, blockIdx.x, lds);
 }
 
-// d_hidden on its own: C[m][n] (+)= sum_k A[m][k] B[k][n] as in gemm16_tile's mixed mode (W read in place); with `by_rows` in use
-// the K slices are those of the rows that take part
-template <typename Cfg>
-__global__ __launch_bounds__(Cfg::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Cfg::TIN> p, DhSlices by_rows) {
+// d_hidden on its own: C[m][n] (+)= sum_k A[m][k] B[k][n] as in gemm16_tile's mixed mode (W read in place), on tiles of 256 or 192 tokens;
+// with `by_rows` in use the width and the K slices are those of the rows that take part
+template <typename Wide, typename Narrow>
+__global__ __launch_bounds__(Wide::NTHREADS) void lce_dh16_kernel(GemmArgs<typename Wide::TIN> p, DhSlices by_rows, bool narrow) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   if (by_rows.n[0]) {
     const int64_t rows = *p.m_dev;
+    narrow = by_rows.tile(rows) == 192;
     p.ksplit = by_rows.count(rows);
-    p.kslice = ((p.K + p.ksplit - 1) / p.ksplit + Cfg::BK - 1) / Cfg::BK * Cfg::BK;
+    p.kslice = ((p.K + p.ksplit - 1) / p.ksplit + Wide::BK - 1) / Wide::BK * Wide::BK;
     p.cf_split_stride = DhSlices::stride(rows, p.N);
     p.map.ncol_tiles = p.n_tiles * p.ksplit;
+    p.map.br = 8;  // (what TileMap::with_rows narrows to the tiles there are)
   }
-  gemm16_tile<Cfg, GemmCfg16<typename Cfg::TIN, 2, Cfg::NBN, Cfg::A_EARLY, 1, Cfg::A_ONCE, Cfg::NB>>(p, blockIdx.x, lds);
+  if (narrow) gemm16_tile<Narrow, GemmCfg16<typename Wide::TIN, 2, Narrow::NBN, Narrow::A_EARLY, 1, Narrow::A_ONCE, Narrow::NB>>(p, blockIdx.x, lds);
+  else gemm16_tile<Wide, GemmCfg16<typename Wide::TIN, 2, Wide::NBN, Wide::A_EARLY, 1, Wide::A_ONCE, Wide::NB>>(p, blockIdx.x, lds);
 }
 
 // a tile of d_weight (p.tn == 1) or of d_hidden, NBM blocks of hidden columns to a wave
