@@ -2,7 +2,7 @@
 // multiplied as six products of planes (GemmCfg16, TERMS == 6).  The fp32 MFMA runs at 157 TFLOP/s dense, the bfloat16 one
 // at 2.5 PFLOP/s; six products for one leave 2.5 times the rate at the clocks both reach, against which stand the passes
 // that make the planes (10 bytes per element of W, forward and backward each).  Measured, fp32 MFMA / planes: H=896,
-// V=151936, 1024 tokens forward + backward 9.90 / 4.67 ms (logits kept), 2000 tokens forward 4.11 / 2.23, 400 tokens forward 1.09 / 0.75;
+// V=151936, 1024 tokens forward + backward 9.90 / 4.30 ms (logits kept), 2000 tokens forward 4.11 / 2.23, 400 tokens forward 1.09 / 0.75;
 // H=5120, 1500 tokens, half with gradient 56.6 / 26.8.  Error against float64 (2-norm, relative; H=896, V=151936, 2000 tokens):
 // log-probs 7.7e-8 / 7.2e-8, entropies 5.9e-8 / 5.6e-8, d_hidden 1.0e-6 / 5.9e-7, d_weight 7.9e-7 / 4.1e-7: the products are
 // exact and a sixteenth as many partial sums are rounded.
