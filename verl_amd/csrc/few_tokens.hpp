@@ -83,7 +83,7 @@ struct FewFwdShape {
 
 // The products of W's rows [row0, vend64) with the NT hidden rows, 256 rows of W at a time; `pass(acc, m0, vbase, busy)` gets those of
 // rows vbase .. vbase + 31 (this wave's; busy: some exist) in acc[0][j][.], column j * 32 + lane % 32.  h_off: byte offset of hidden row
-// tid / 8 + 64 i (kBufNowhere: reads as zero) in the h_bytes behind h.
+// tid / 8 + 64 i (beyond h_bytes: reads as zero) in the h_bytes behind h.
 // HALF: a pass is whole turns of the loop over the DEPTH stages in flight and half a one (16 bits: H is a multiple of 128 but not of
 // 256), and every second pass starts at the second half of the ring.  Rounded up to whole turns, a seventh of the stages were zeros at
 // H=896: 1 / 40 / 64 tokens, V=151936, 50.7 / 51.7 / 52.1 -> 49.2 / 49.6 / 50.0 us.  (A branch around them in the loop costs more than they

@@ -10,6 +10,12 @@
 
 namespace lce {
 
+// An offset beyond ONE descriptor over all rows of hidden: with 255 rows of up to 16 MiB (lce_abi.hip, check_common) that spans more than
+// the 2 GiB which kBufNowhere lies beyond.  Nothing is added to it but the 16 bytes of a load.
+constexpr int kFewF32Rows = 255;
+constexpr int kFewF32Nowhere = (int)0xff000000u;
+static_assert(kFewF32Rows * ((int64_t)16 << 20) <= (int64_t)0xff000000u, "beyond the last row of hidden");
+
 // d_logits lie in panels of 32 columns, [panel][token position][32], `pcol` elements from panel to panel.
 template <typename P>
 LCE_DEV P ds32_at(P dS, int64_t pcol, int64_t t, int64_t v) { return dS + (v >> 5) * pcol + t * 32 + (v & 31); }
@@ -58,7 +64,7 @@ __global__ __launch_bounds__(512, 2) void lce_ds_few_f32_kernel(FewF32Args p) {
 #pragma unroll
   for (int i = 0; i < HL; ++i) {
     const int pos = (tid >> 3) + 64 * i;
-    h_off[i] = pos < n ? (uint32_t)((p.rows ? (int64_t)p.rows[pos] : pos) * p.ldh * 4) + (tid & 7) * 16 : (uint32_t)kBufNowhere;
+    h_off[i] = pos < n ? (uint32_t)((p.rows ? (int64_t)p.rows[pos] : pos) * p.ldh * 4) + (tid & 7) * 16 : (uint32_t)kFewF32Nowhere;
   }
   f32x4_t k[FN];
   int lab[FN];
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(512, 2) void lce_dw_few_f32_kernel(FewF32Args p) {
 #pragma unroll
     for (int x = 0; x < NB; ++x) {
       const int64_t col = hw + 32 * x + ln;
-      hf[kp][x] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(hid, tok >= 0 && col < p.H ? (int)((tok * p.ldh + col) * 4) : kBufNowhere, 0, 0));
+      hf[kp][x] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(hid, tok >= 0 && col < p.H ? (int)((tok * p.ldh + col) * 4) : kFewF32Nowhere, 0, 0));
     }
   }
   stash(lds);

@@ -41,7 +41,7 @@ typedef __amdgpu_buffer_rsrc_t buf_t;
 LCE_DEV buf_t make_buf(const void* p, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
 }
-constexpr int kBufNowhere = (int)0x80000000u;  // an offset beyond any buffer it is used with (those span less than 2 GiB)
+constexpr int kBufNowhere = (int)0x80000000u;  // an offset beyond any buffer it is used with (those span at most 2 GiB)
 constexpr int kBufNonTemporal = 2;
 
 typedef const void __attribute__((address_space(1))) * gptr_t;

@@ -24,6 +24,7 @@ struct FewF32Layout {
 // 2544 -> 2151, 255: 2542 -> 2433; H=896, 255: level.  Error of d_hidden against float64: 200 tokens, H=896, 1.03e-6 / 6.7e-7, H=3584 1.37e-6 /
 // 1.15e-6.  From 256 on the planes run (H=3584: 6.0 ms), with large vocabularies.
 constexpr int64_t kFewF32Tokens = LCE_F32_FEW_TOKENS;
+static_assert(kFewF32Tokens <= kFewF32Rows, "rows of hidden behind one descriptor");
 bool few_f32(const Tuning& tu, int64_t T) { return T <= kFewF32Tokens && !tu.variant_forced && tu.few_token_gemms && !tu.split_bwd; }
 
 // bytes of the logits that a forward of so few tokens keeps where it is handed the buffer
