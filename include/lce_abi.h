@@ -125,8 +125,8 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  *   lce_backward_from_logits: lce_backward (grads_fp32 = 0) or lce_backward_f32 (grads_fp32 = 1; d_hidden, d_weight are
  *     float* then); with logits_cache != NULL, as written by lce_forward_keep_logits for the same hidden, weight, T, H, V
  *     and dtype, the gradient of the logits is computed from it with the same expressions, so both gradients are bit for
- *     bit those of lce_backward (LCE_DTYPE_F32_PLANES: d_weight; d_hidden may sum chunks of another width).  The cache is only
- *     read. */
+ *     bit those of lce_backward (on planes but for inputs of 2^59 and more, which the planes hold in another way from
+ *     the chunk of the weight on that has the first).  The cache is only read. */
 #define LCE_F32_FEW_TOKENS 255
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype);
 size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype);

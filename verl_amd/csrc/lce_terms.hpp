@@ -72,7 +72,7 @@ struct TermsBwdLayout {
   int64_t vchunk, tpad, pcol, plane, ldH;  // plane: elements from plane to plane of a d_logits panel
   size_t off_dS[2], off_W[2], off_H, off_dHacc, off_rows, off_inv, off_nrows, off_acounts, off_tokc, off_tokl, total;
   int nchunks, ksplit;
-  bool wide;  // chunks twice as wide where the forward kept the logits, with twice the K slices and partials of d_hidden
+  bool wide;  // the chunks of kept rows are twice as wide, with twice the K slices and partials of d_hidden (TermsChunks)
 };
 
 // upper bound of the workspace: a quarter of one [T, V] plus one fp32 [V, H], or the budget
@@ -154,6 +154,47 @@ constexpr int64_t kTermsKeepTokens = 4;  // times H
 int64_t terms_kept_rows(int64_t T, int64_t H, int64_t V) { return T <= H ? V : V * H / T / 256 * 256; }
 size_t terms_cache_bytes(const Tuning& tu, int64_t T, int64_t H, int64_t V) {
   return T <= kTermsKeepTokens * H && use_terms(tu, T, H, V) ? (size_t)T * (size_t)logits_cache_row(terms_kept_rows(T, H, V)) * 4 : 0;
+}
+
+// The chunks of a backward: of the rows whose logits a forward of this shape keeps, then the others.  With the logits at hand the
+// first ones' d_logits are a pass of their own, so that both buffers may hold one chunk twice as wide (L.wide): half as many
+// launches, each with a last round of tiles.  The last of them, where others follow, is of the usual width, and its products share a
+// launch with the d_logits tiles of the first of the others.  The list is one of shapes and settings, whether this call has the logits or
+// not: the chunks and their K slices are the order of d_hidden's sums, and whether a forward kept its logits depends on what other
+// graphs hold at that moment.  Without them a wide chunk's d_logits tiles are a launch of their own.  That costs such a backward up to 4 %
+// (d_hidden alone up to 10 %) against chunks that share their launches, us: H=896, 300 tokens 1825 -> 1905, 600: 2820 -> 2790 (d_hidden alone 2018
+// -> 2230), 1024: 3810 -> 3900, 1500: 5240 -> 5415; H=4096, 2000: 24580 -> 25480; with the logits it is the same.
+struct TermsChunks {
+  struct Chunk {
+    int64_t v0, rows;
+    int buf;
+    bool kept, wide;
+  };
+  int64_t to[3], width[3];  // the kept rows but the last chunk of them, that chunk, the others: end, rows of a chunk
+  int n[3], wide;           // chunks; how many of them, from the first on, are wide
+  bool two;
+  int count() const { return n[0] + n[1] + n[2]; }
+  Chunk at(int c) const {
+    const int r = c < n[0] ? 0 : c < n[0] + n[1] ? 1 : 2, first = r == 0 ? 0 : r == 1 ? n[0] : n[0] + n[1];
+    const int64_t v0 = (r ? to[r - 1] : 0) + (c - first) * width[r];
+    return {v0, std::min(width[r], to[r] - v0), c < wide || !two ? 0 : (c & 1), r < 2, c < wide};
+  }
+};
+TermsChunks terms_chunks(const TermsBwdLayout& L, int64_t T, int64_t H, int64_t V) {
+  TermsChunks t;
+  const int64_t kept = T <= kTermsKeepTokens * H ? terms_kept_rows(T, H, V) : 0;
+  t.two = L.nchunks > 1;
+  t.to[1] = kept;
+  t.to[0] = kept - (kept < V && t.two ? std::min(kept, L.vchunk) : 0);
+  t.to[2] = V;
+  for (int r = 0; r < 3; ++r) {
+    const int64_t rows = t.to[r] - (r ? t.to[r - 1] : 0), most = r == 0 && L.wide ? 2 * L.vchunk : L.vchunk;
+    t.n[r] = (int)((rows + most - 1) / most);
+    t.width[r] = t.n[r] > 0 ? round_up((rows + t.n[r] - 1) / t.n[r], 256) : most;
+    t.n[r] = (int)((rows + t.width[r] - 1) / t.width[r]);
+  }
+  t.wide = L.wide ? t.n[0] : 0;
+  return t;
 }
 
 #if defined(LCE_TU_DTYPE) && LCE_TU_DTYPE == 1
@@ -262,36 +303,23 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
   const SplitArgs sh = {h, ldh, T, H, h3, L.ldH, L.tpad, rows, n_rows};
   if ((rc = launch_split(sh, nullptr, wide, st))) return rc;
   const int ntt = (int)((T + Cfg::BN - 1) / Cfg::BN), h_tile = hidden_tile(H);
-  const int64_t kept = xcache ? terms_kept_rows(T, H, V) : 0;
-  // The chunks: of the rows whose logits the forward kept, then the others, whose d_logits tiles share a launch with the products of the
-  // chunk before.  The kept ones' d_logits are a pass of their own, so that both buffers may hold one chunk twice as wide (L.wide): half as
-  // many launches, each with a last round of tiles.  The last of them, where others follow, is of the usual width.
-  struct Chunk {
-    int64_t v0, rows;
-    int buf;
-    bool kept, alone;  // alone: its products share their launch with no d_logits tiles
-  };
-  std::vector<Chunk> chunks;
-  auto cut = [&](int64_t from, int64_t to, int64_t width, bool of_kept) {
-    const int64_t n = (to - from + width - 1) / width;
-    if (n > 0) width = round_up((to - from + n - 1) / n, 256);
-    for (int64_t v0 = from, c = 0; v0 < to; v0 += width, ++c) chunks.push_back({v0, std::min(width, to - v0), of_kept ? 0 : (int)(c & 1), of_kept, of_kept});
-  };
-  const int64_t joint = kept < V && L.nchunks > 1 ? std::min(kept, L.vchunk) : 0;
-  cut(0, kept - joint, L.wide ? 2 * L.vchunk : L.vchunk, true);
   // K slices of a wide chunk no longer than a usual one's (the same error of d_hidden), or twice as many as that has, where d_hidden's
   // tiles then fill their rounds over the CUs better by a tenth (1024 tokens of H=896, d_hidden alone: 3447 -> 3305 us)
+  const TermsChunks chunks = terms_chunks(L, T, H, V);
   int wide_slices = L.ksplit;
-  if (L.wide && !chunks.empty()) {
-    const int64_t tiles = ntt * ((H + h_tile - 1) / h_tile), rows = chunks[0].rows, slice = round_up((L.vchunk + L.ksplit - 1) / L.ksplit, Cfg::BK);
+  if (chunks.wide > 0) {
+    const int64_t tiles = ntt * ((H + h_tile - 1) / h_tile), rows = chunks.at(0).rows, slice = round_up((L.vchunk + L.ksplit - 1) / L.ksplit, Cfg::BK);
     auto time = [&](int64_t s) { return (double)((tiles * s + kNumCUs - 1) / kNumCUs) * ((double)rows / (double)(s * Cfg::BK) + 2); };
     wide_slices = (int)std::max<int64_t>(L.ksplit, (rows + slice - 1) / slice);
     if (time(2 * L.ksplit) < 0.9 * time(wide_slices)) wide_slices = 2 * L.ksplit;
   }
   const int all_slices = std::max(wide_slices, L.ksplit);
-  if (joint > 0) chunks.push_back({kept - joint, joint, 1, true, false});
-  cut(kept, V, L.vchunk, false);
-  const int nchunks = (int)chunks.size();
+  const int nchunks = chunks.count();
+  // d_logits of a kept chunk, where the caller has the logits, are a pass of their own instead of tiles
+  auto from_cache = [&](int c) { return xcache && c < nchunks && chunks.at(c).kept; };
+  // Does chunk c share its products' launch with the d_logits tiles of the next one?  Not where those are no tiles, or where the two are not in
+  // different buffers: a wide chunk is in both, and with a single chunk's layout there is but one.
+  auto shares = [&](int c) { return L.nchunks > 1 && c + 1 < nchunks && !chunks.at(c).wide && !from_cache(c + 1); };
   auto launch = [&](BwdChunkArgs<bf16_t>& p) {
     if (p.n_gw + p.n_gh + p.n_ds == 0) return (int)LCE_OK;
     ProfScope prof(PC_BWD_CHUNK, st);
@@ -305,14 +333,14 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
     BwdChunkArgs<bf16_t> p;
     p.n_gw = p.n_gh = p.n_ds = 0;
     if (c > 0) {
-      const Chunk& k = chunks[c - 1];
+      const TermsChunks::Chunk k = chunks.at(c - 1);
       const int64_t v0 = k.v0, vrows = k.rows;
       const int64_t kc = round_up(vrows, KPerm<Cfg>::GV);
       if (need_dh) {
         p.gh = make_gemm_args<Cfg>(dS[k.buf], 64, w3[k.buf], 3 * H, T, H, kc, dHacc, H, nullptr, 0, c == 1 ? 0 : 1, h_tile);
         p.gh.tn = 2; p.gh.b_rows_valid = vrows; p.gh.m_dev = n_rows;
         p.gh.a_pcol = L.pcol; p.gh.a_plane = L.plane * 2; p.gh.b_plane = H * 2;
-        const int slices = k.alone ? wide_slices : L.ksplit;
+        const int slices = k.wide ? wide_slices : L.ksplit;
         if (slices > 1) {
           p.gh.ksplit = slices;
           p.gh.kslice = round_up((kc + slices - 1) / slices, Cfg::BK);
@@ -335,15 +363,15 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
         p.n_gw = p.n_gh;
         p.n_gh = 0;
       }
-      if (k.alone || c == nchunks) {
+      if (!shares(c - 1)) {
         if ((rc = launch(p))) return rc;
         p.n_gw = p.n_gh = 0;
       }
     }
     if (c == nchunks) break;
-    const Chunk& k = chunks[c];
+    const TermsChunks::Chunk k = chunks.at(c);
     const int64_t v0 = k.v0, vrows = k.rows;
-    // (the last reader of this buffer ran in the launch before the last)
+    // (the last reader of this buffer ran in an earlier launch)
     if ((rc = launch_split({W + v0 * ldw, ldw, vrows, H, w3[k.buf], H, vrows, nullptr, nullptr}, &sh, wide, st))) return rc;
     DsArgs<bf16_t>& d = p.ds;
     d.W = w3[k.buf]; d.ldw = 3 * H; d.h = h3; d.ldh = 3 * L.ldH; d.labels = labels; d.T = T; d.H = H;
@@ -354,7 +382,7 @@ int backward_terms(const float* h, int64_t ldh, const float* W, int64_t ldw, con
     d.dS = dS[k.buf]; d.ldS = 64; d.pcol = L.pcol; d.dST = nullptr; d.ldST = 0; d.tpad = L.tpad;
     d.rows = nullptr; d.n_rows = n_rows; d.label_outside = 0;
     d.tokc = tokc; d.tokl = tokl; d.lab0 = v0; d.range_rows = 0;
-    if (k.kept) {
+    if (from_cache(c)) {
       ProfScope prof(PC_BWD_DS, st);
       d.rows = rows;  // (the tiles read the compact planes of hidden and no list; the cache is indexed by token)
       hipLaunchKernelGGL((ds_from_logits_kernel<bf16_t, KPerm<Cfg>, Cfg::TERMS>), dim3((unsigned)(round_up(vrows, 256) / 64)), dim3(256), 0, st, d,

@@ -214,7 +214,7 @@ def efficient_entropy_backward(
     ``need_d_hidden`` / ``need_d_weight`` (not in the reference, which always computes both): ``False`` leaves that
     gradient's GEMM out, a third of the backward's work, and returns ``None`` in its place, e.g. for a frozen lm-head
     under LoRA.  ``logits_cache``: the sixth value of ``forward_keeping_logits`` for the same inputs; the gradients are
-    bit for bit the same with and without it (fp32: ``d_weight``; ``d_hidden`` may be summed in another order)."""
+    bit for bit the same with and without it."""
     if not (need_d_hidden or need_d_weight):
         return None, None
     _require_single_rank(dist_process_group)
