@@ -153,6 +153,7 @@ def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0,
     """``efficient_entropy_forward`` plus a sixth value: the kept logits for ``efficient_entropy_backward(...,
     logits_cache=)``, or ``None`` where the library keeps none (16-bit inputs: more tokens than half the hidden
     size; fp32: four times the hidden size; ``keep_logits=False``).
+    ``None`` too where there is no memory for them.
     With few tokens fp32 ``[T, V]`` is a fraction of the weight itself, so the autograd node keeps it like any activation
     and the backward skips the pass over ``[V, H]`` and the ``T x V x H`` product that recompute it (not in the
     reference, which always recomputes)."""
@@ -180,7 +181,10 @@ def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0,
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
         cache_bytes = kept_logits_size(T, H, V, code) if keep_logits else 0
         if cache_bytes:
-            cache = torch.empty((cache_bytes,), device=dev, dtype=torch.uint8)
+            try:
+                cache = torch.empty((cache_bytes,), device=dev, dtype=torch.uint8)
+            except torch.cuda.OutOfMemoryError:  # (a backward that recomputes them may still fit)
+                cache_bytes = 0
         rc = lib.lce_forward_keep_logits(
             hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), labels.data_ptr(), T, H, V, code,
             float(temperature), reduction, logprobs.data_ptr(), entropy.data_ptr(), maximum.data_ptr(),
