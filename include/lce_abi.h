@@ -20,7 +20,8 @@ extern "C" {
 #endif
 
 /* 11: the PPO loss as a pair (lce_ppo_forward .. lce_ppo_backward, lce_ppo_call_t), the logits twins in the caller's types,
- *     larger PPO and fp32 workspaces, another layout of the kept logits */
+ *     larger PPO and fp32 workspaces, another layout of the kept logits; since then lce_kept_logits_bytes was added, and nothing else
+ *     changed its meaning */
 #define LCE_ABI_VERSION 11
 
 /* LCE_DTYPE_F32_PLANES: fp32 tensors like LCE_DTYPE_F32, with leave to take their products on the bfloat16 matrix pipe, every
@@ -117,9 +118,9 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
  *     cache never exceeds the weight), 4 H for LCE_DTYPE_F32_PLANES where the planes are used (of all rows of the weight up to H tokens,
  *     beyond of as many of the first as are no larger than the weight), or LCE_OPT_KEEP_LOGITS_TOKENS where that is lower; 0 for
  *     LCE_DTYPE_F32 and under diagnostic settings that force a tile variant.
- *   lce_logits_cache_bytes: size of the buffer for this shape, or 0 where none is offered: then pass NULL below.  (fp32 with at
- *     most LCE_F32_FEW_TOKENS and H tokens, either code: 0, as it has always answered; a caller that brings T * (V rounded up to 64) * 4
- *     bytes all the same has its logits kept there under the limits of lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES).)
+ *   lce_kept_logits_bytes: size of the buffer for this shape, or 0 where none is taken: then pass NULL below.  For fp32, either code,
+ *     also with at most LCE_F32_FEW_TOKENS and H tokens, under the limits of lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES).
+ *   lce_logits_cache_bytes: the same, but 0 for those few tokens of fp32, as it has always answered.
  *   lce_forward_keep_logits: lce_forward; with logits_cache != NULL it also writes hidden . weight^T there in fp32
  *     (private layout).  Same outputs, bit for bit.
  *   lce_backward_from_logits: lce_backward (grads_fp32 = 0) or lce_backward_f32 (grads_fp32 = 1; d_hidden, d_weight are
@@ -130,6 +131,7 @@ int lce_backward_f32(const void* hidden, int64_t ldh, const void* weight, int64_
 #define LCE_F32_FEW_TOKENS 255
 int64_t lce_logits_cache_max_tokens(int64_t H, int dtype);
 size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype);
+size_t lce_kept_logits_bytes(int64_t T, int64_t H, int64_t V, int dtype);
 int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,
                             int64_t H, int64_t V, int dtype, float temperature, int reduction, float* logprobs, float* entropy,
                             float* maximum, float* accumulate, float* entropy_b, void* workspace, size_t workspace_bytes,

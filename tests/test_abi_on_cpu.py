@@ -369,3 +369,44 @@ def test_tile_map_covers_every_tile_once_and_balances_the_xcds(tmp_path):
     subprocess.run(["g++", "-O1", "-std=c++17", "-o", exe, os.path.join(here, "tile_map_check.cpp")], check=True, timeout=300)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout + r.stderr
+
+
+def test_the_query_of_the_kept_logits_agrees_with_the_call():
+    """lce_kept_logits_bytes is what lce_forward_keep_logits takes, for every code: a byte less is refused by its size, no other
+    shape takes a buffer at all.  (Checked ahead of any launch.)"""
+    lib = _abi.load()
+    room = torch.zeros(64)
+    at = (room.data_ptr() + 15) // 16 * 16
+
+    def call(T, H, V, code, cache_bytes):
+        rc = lib.lce_forward_keep_logits(at, H, at, H, at, T, H, V, code, 1.0, 0, at, at, at, at, at, at, 0, at, cache_bytes, None)
+        return rc, lib.lce_last_error().decode()
+
+    def check(T, H, V, code):
+        need = lib.lce_kept_logits_bytes(T, H, V, code)
+        old = lib.lce_logits_cache_bytes(T, H, V, code)
+        few = code in (_abi.DTYPE_F32, _abi.DTYPE_F32_PLANES) and T <= 255
+        assert (old in (0, need)) if few else old == need
+        if need == 0:
+            rc, text = call(T, H, V, code, 1 << 40)
+            assert rc == -1 and "no logits are kept" in text
+            return 0
+        rc, text = call(T, H, V, code, need - 1)
+        assert rc == -2 and f"logits cache too small: {need - 1} < {need}" in text
+        rc, text = call(T, H, V, code, need)
+        assert rc == -2 and "forward workspace too small" in text  # (past the cache's checks)
+        return need
+
+    H, V = 512, 40011
+    row = (V + 63) // 64 * 64 * 4
+    for code in (_abi.DTYPE_BF16, _abi.DTYPE_F16):
+        assert [check(T, H, V, code) // row for T in (1, 255, 256, 257)] == [1, 255, 256, 0]
+    assert [check(T, H, V, _abi.DTYPE_F32) // row for T in (1, 128, 129, 255, 256)] == [1, 128, 129, 255, 0]
+    assert [check(T, H, V, _abi.DTYPE_F32_PLANES) // row for T in (1, 255, 256, 512)] == [1, 255, 256, 512]
+    assert check(2048, H, V, _abi.DTYPE_F32_PLANES) == 2048 * (V * H // 2048 // 256 * 256) * 4 and check(2049, H, V, _abi.DTYPE_F32_PLANES) == 0
+    assert check(65, 64, V, _abi.DTYPE_F32) == 0 and check(0, H, V, _abi.DTYPE_F32) == 0 and lib.lce_kept_logits_bytes(8, H, V, 9) == 0
+    try:
+        assert lib.lce_set_option(11, 100) == 0
+        assert check(100, H, V, _abi.DTYPE_F32) > 0 and check(101, H, V, _abi.DTYPE_F32_PLANES) == 0
+    finally:
+        lib.lce_set_option(11, 1 << 40)

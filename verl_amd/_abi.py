@@ -36,6 +36,7 @@ SYMBOLS = {
     ),
     "lce_logits_cache_max_tokens": (_i64, [_i64, _i]),
     "lce_logits_cache_bytes": (_sz, [_i64, _i64, _i64, _i]),
+    "lce_kept_logits_bytes": (_sz, [_i64, _i64, _i64, _i]),
     "lce_forward_keep_logits": (
         _i,
         [_p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i, _f, _i, _p, _p, _p, _p, _p, _p, _sz, _p, _sz, _p],
@@ -113,7 +114,9 @@ def load() -> ctypes.CDLL:
         if lib.lce_abi_version() != ABI_VERSION:
             raise LceError(f"ABI version mismatch: library {lib.lce_abi_version()}, binding {ABI_VERSION}")
         for name, (res, args) in SYMBOLS.items():
-            fn = getattr(lib, name)
+            fn = getattr(lib, name, None)
+            if fn is None:
+                raise LceError(f"{LIB_PATH} has no {name}: it was built from older sources, build it again")
             fn.restype = res
             fn.argtypes = args
         _lib = lib

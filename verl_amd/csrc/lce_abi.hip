@@ -270,15 +270,19 @@ size_t lce_logits_cache_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
   return (size_t)T * (size_t)logits_cache_row(V) * 4;
 }
 
+size_t lce_kept_logits_bytes(int64_t T, int64_t H, int64_t V, int dtype) {
+  const bool f32 = dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES;
+  const size_t few = f32 && T <= lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES) ? few_f32_cache_bytes(T, H, V) : 0;
+  return few ? few : lce_logits_cache_bytes(T, H, V, dtype);
+}
+
 int lce_forward_keep_logits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const int64_t* labels, int64_t T,
                             int64_t H, int64_t V, int dtype, float temperature, int reduction, float* logprobs, float* entropy,
                             float* maximum, float* accumulate, float* entropy_b, void* workspace, size_t workspace_bytes,
                             void* logits_cache, size_t logits_cache_bytes, void* stream) {
   if (logits_cache) {
-    const bool f32 = dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES;
-    size_t need = f32 || known_dtype(dtype) ? lce_logits_cache_bytes(T, H, V, dtype) : 0;
-    if (f32 && need == 0 && T <= lce_logits_cache_max_tokens(H, LCE_DTYPE_F32_PLANES)) need = few_f32_cache_bytes(T, H, V);
-    if (need == 0) return fail(LCE_E_ARG, "lce_forward_keep_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
+    const size_t need = lce_kept_logits_bytes(T, H, V, dtype);
+    if (need == 0) return fail(LCE_E_ARG, "lce_forward_keep_logits: no logits are kept for this shape (lce_kept_logits_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");
   }
@@ -427,7 +431,7 @@ int lce_backward_from_logits(const void* hidden, int64_t ldh, const void* weight
     const bool f32 = dtype == LCE_DTYPE_F32 || dtype == LCE_DTYPE_F32_PLANES;
     size_t need = f32 || !known_dtype(dtype) || T <= 0 ? 0 : lce_logits_cache_bytes(T, H, V, dtype);
     if (f32 && T > 0 && H > 0 && V > 0) need = T <= kFewF32Tokens ? few_f32_cache_bytes(T, H, V) : dtype == LCE_DTYPE_F32 ? 0 : terms_cache_bytes(Tuning(), T, H, V);
-    if (need == 0) return fail(LCE_E_ARG, "lce_backward_from_logits: no logits are kept for this shape (lce_logits_cache_bytes is 0): pass NULL");
+    if (need == 0) return fail(LCE_E_ARG, "lce_backward_from_logits: no logits are kept for this shape (lce_kept_logits_bytes is 0): pass NULL");
     if (logits_cache_bytes < need) return fail(LCE_E_WORKSPACE, "logits cache too small: %zu < %zu", logits_cache_bytes, need);
     if (reinterpret_cast<size_t>(logits_cache) % 16 != 0) return fail(LCE_E_ARG, "logits cache must be 16-byte aligned");
   }

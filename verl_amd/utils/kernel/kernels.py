@@ -131,10 +131,7 @@ def _check_inputs(hidden, weight, labels):
 
 def kept_logits_size(T: int, H: int, V: int, code: int) -> int:
     """Bytes of the logits that a forward of this shape keeps for its backward (0: none)."""
-    lib = _abi.load()
-    if code == _abi.DTYPE_F32_PLANES and T <= min(255, H):  # (LCE_F32_FEW_TOKENS: the query answers 0 for them)
-        return T * ((V + 63) // 64 * 64) * 4 if 0 < T <= lib.lce_logits_cache_max_tokens(H, code) else 0
-    return lib.lce_logits_cache_bytes(T, H, V, code)
+    return _abi.load().lce_kept_logits_bytes(T, H, V, code)
 
 
 def efficient_entropy_forward(
