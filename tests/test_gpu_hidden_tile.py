@@ -53,3 +53,51 @@ def test_gradients_on_narrow_tiles(T, H, V, vchunk, keep, dtype):
     finally:
         kernels.set_vocab_chunk(0)
     assert (dh[mask.to(DEV) == 0] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,V,vchunk", [
+    (300, 1088, 9001, 0),      # five tiles, the last one cut
+    (700, 1344, 12007, 4096),  # six whole ones, several chunks
+    (1030, 3136, 5003, 0),     # fourteen for thirteen of 256
+])  # fmt: skip
+def test_hidden_sizes_that_are_multiples_of_64(T, H, V, vchunk, dtype):
+    """The other sizes with narrow tiles, which only the C ABI takes: row strides that no tile divides."""
+    from verl_amd import _abi
+
+    lib = _abi.load()
+    g = torch.Generator().manual_seed(H)
+    h = torch.randn(T, H, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(V, H, generator=g) * 0.03).to(dtype).to(DEV)
+    y = torch.randint(0, V, (T,), generator=g).to(DEV)
+    on = torch.rand(T, generator=g) < 0.8
+    g_lp, g_ent = (torch.randn(T, generator=g) * on).to(DEV), (torch.randn(T, generator=g) * on).to(DEV)
+    code = _abi.DTYPE_F32_PLANES if dtype == torch.float32 else _abi.dtype_code(dtype)
+    st = _abi.current_stream(h.device)
+    common = (h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, 0.9, 0)
+    out = torch.empty(5, T, device=DEV)
+    need, kept = lib.lce_forward_workspace_bytes(T, H, V, code), lib.lce_kept_logits_bytes(T, H, V, code)
+    ws, cache = torch.empty(need, device=DEV, dtype=torch.uint8), torch.empty(max(kept, 16), device=DEV, dtype=torch.uint8)
+    rc = lib.lce_forward_keep_logits(*common, *(o.data_ptr() for o in out), ws.data_ptr(), need, cache.data_ptr() if kept else None, kept, st)
+    _abi.check(rc, "lce_forward_keep_logits")
+    need = lib.lce_backward_workspace_bytes(T, H, V, code, vchunk)
+    ws = torch.empty(need, device=DEV, dtype=torch.uint8)
+    rdh, rdw = O.lce_backward(g_lp, g_ent, h, w, y, 0.9, compute_dtype=torch.float64)
+    results = []
+    for x, n in ((None, 0), (cache.data_ptr(), kept)):
+        if x is not None and kept == 0:
+            continue
+        dh, dw = torch.full((T, H), 7.0, device=DEV), torch.full((V, H), 7.0, device=DEV)
+        ws.fill_(0xFF)  # (NaN)
+        rc = lib.lce_backward_from_logits(*common, *(o.data_ptr() for o in out[2:]), g_lp.data_ptr(), g_ent.data_ptr(), dh.data_ptr(),
+                                          dw.data_ptr(), 1, ws.data_ptr(), need, vchunk, x, n, st)  # fmt: skip
+        _abi.check(rc, "lce_backward_from_logits")
+        # (the bars of the test above)
+        rel = 3e-6 if dtype == torch.float32 else 2.0**-7
+        for got, want in ((dh, rdh), (dw, rdw)):
+            assert ((got.double() - want).norm() / want.norm()).item() <= rel
+            assert (got.double() - want).abs().max().item() <= (1e-5 if dtype == torch.float32 else 2.0**-7) * want.abs().max().item()
+        assert (dh[~on.to(DEV)] == 0).all()
+        results.append((dh, dw))
+    for dh, dw in results[1:]:
+        assert torch.equal(dh, results[0][0]) and torch.equal(dw, results[0][1])

@@ -483,9 +483,12 @@ bool dw_transposed_reads(size_t esz) { return esz == 2; }
 
 // Width of the gradient products' tiles along H on the 16x16x32 loop: 256, or 224 where those leave less of the last tile over.  H = 896
 // is four tiles either way, without a column of padding or with 128.  A 224-wide tile's slab is an eighth less matrix work behind
-// the same loads and takes some 0.92 of the time, hence the line: 896 and the narrow sizes below, not 2688 (12 tiles for 11).  H=896,
+// the same loads and takes some 0.92 of the time, hence the line: as many tiles (up to 224, 257 to 448, 513 to 672, 769 to 896, 1025 to 1120, 1281
+// to 1344, 1537 to 1568), or more where that is less than a twelfth of them (3136: 14 for 13; not 2688, 12 for 11).  H=896,
 // V=151936, forward + backward, 256 / 224 wide: bf16 500 tokens 577 -> 553 us, 1000: 1076 -> 1035, 4096: 3920 -> 3780, 16384: 14.98 -> 14.48 ms;
-// fp32 on planes 400 tokens 3101 -> 2995 us, 1024: 5854 -> 5670, 2000: 10862 -> 10465.
+// fp32 on planes 400 tokens 3101 -> 2995 us, 1024: 5854 -> 5670, 2000: 10862 -> 10465.  Backward alone, V=152064, 500 / 4096 tokens of bf16 and 1024
+// of fp32: H=640 430 -> 398, 2378 -> 2290, 3361 -> 3137; 1088: 554 -> 533, 3723 -> 3515, 5038 -> 4744; 1344: 638 -> 613, 4320 -> 4058, 6063 -> 5709;
+// 3136: 1355 -> 1299, 9070 -> 8866, 12968 -> 12658.
 int hidden_tile(int64_t H) { return (H + 223) / 224 * 12 < (H + 255) / 256 * 13 ? 224 : 256; }
 
 // the same loop on tiles of 224 hidden columns
