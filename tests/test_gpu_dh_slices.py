@@ -5,7 +5,7 @@ nothing written beyond the workspace that the library asks for."""
 import pytest
 import torch
 
-from oracle import lce_oracle as O
+from tiles_part import check_tiles_part
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -45,7 +45,13 @@ def test_counts_of_tokens_with_a_gradient(T, H, V, active, dtype):
             g_lp.data_ptr(), g_ent.data_ptr(), dh.data_ptr(), None, ws.data_ptr(), need, 0, _abi.current_stream(h.device),
         )  # fmt: skip
         assert rc == 0
-        want = O.lce_backward(g_lp, g_ent, h, w, y, 1.0)[0].double()
+        dh32 = torch.empty(T, H, device=DEV)
+        rc = lib.lce_backward_f32(
+            h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, 1.0, 0, mx.data_ptr(), acc.data_ptr(), eb.data_ptr(),
+            g_lp.data_ptr(), g_ent.data_ptr(), dh32.data_ptr(), None, ws.data_ptr(), need, 0, _abi.current_stream(h.device),
+        )  # fmt: skip
+        assert rc == 0
+        want = check_tiles_part(dh32, None, g_lp, g_ent, h, w, y)[0]
         assert (ws[need:] == 0x5A).all()
         assert torch.count_nonzero(dh[~on]) == 0
         # the bar of the other backward tests: half an ulp of the result, 16-bit rounding of the logits' gradient

@@ -5,7 +5,7 @@ beyond the workspace."""
 import pytest
 import torch
 
-from oracle import lce_oracle as O
+from tiles_part import check_tiles_part
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -37,13 +37,19 @@ def test_counts_on_either_side_of_a_width(T, H, V, active, dtype):
         g_lp, g_ent = base_lp * on, base_ent * on
         ws[need:] = 0x5A
         dh, dw = torch.empty_like(h), torch.empty_like(w)
-        rc = lib.lce_backward(
-            h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, 1.0, 0, mx.data_ptr(), acc.data_ptr(), eb.data_ptr(),
-            g_lp.data_ptr(), g_ent.data_ptr(), dh.data_ptr(), dw.data_ptr(), ws.data_ptr(), need, 0, _abi.current_stream(h.device),
-        )  # fmt: skip
-        assert rc == 0
-        want = O.lce_backward(g_lp, g_ent, h, w, y, 1.0)[0].double()
+        dh32, dw32 = (torch.empty(x.shape, device=DEV) for x in (h, w))
+        for entry, a, b in ((lib.lce_backward, dh, dw), (lib.lce_backward_f32, dh32, dw32), (lib.lce_backward_f32, dh32, None)):
+            ws[:need] = 0xFF  # (NaN)
+            rc = entry(
+                h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), T, H, V, code, 1.0, 0, mx.data_ptr(), acc.data_ptr(), eb.data_ptr(),
+                g_lp.data_ptr(), g_ent.data_ptr(), a.data_ptr(), _abi.ptr(b), ws.data_ptr(), need, 0, _abi.current_stream(h.device),
+            )  # fmt: skip
+            assert rc == 0
+            if entry is lib.lce_backward_f32:
+                want, want_w = check_tiles_part(a, b, g_lp, g_ent, h, w, y)
         assert (ws[need:] == 0x5A).all()
-        assert torch.count_nonzero(dh[~on]) == 0
-        # the bar of the other backward tests: half an ulp of the result, 16-bit rounding of the logits' gradient
-        assert ((dh.double() - want).abs() <= 2e-2 + 2.0**-7 * want.abs()).all(), n
+        assert torch.count_nonzero(dh[~on]) == 0 and torch.count_nonzero(dh32[~on]) == 0
+        # in 16 bits the same sums, rounded once: half an ulp, 2^-8 (2^-11) of the value, 2^-25 of fp16's smallest ones
+        half = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+        assert ((dh.float() - dh32).abs() <= half * dh32.abs() + 2.0**-25).all(), n
+        assert ((dw.double() - want_w).norm() / want_w.norm()).item() <= 2.0**-8, n
