@@ -309,7 +309,7 @@ int lce_ppo_backward(const lce_ppo_call_t* call, void* stream);
  * with hidden . W[label] recomputed per token) is kept out of the tiles and added in fp32.  Changes the workspace size:
  * set it before querying lce_backward_workspace_bytes.
  * LCE_OPT_KEEP_LOGITS_TOKENS (default LCE_KEEP_LOGITS_NO_LIMIT; any count >= 0): the token count up to which
- * lce_logits_cache_bytes offers a cache, next to its own bounds; 0 makes every backward recompute its
+ * lce_kept_logits_bytes offers a cache, next to its own bounds; 0 makes every backward recompute its
  * logits, as the reference does at every size. */
 #define LCE_KEEP_LOGITS_NO_LIMIT ((int64_t)1 << 40)
 enum {

@@ -301,9 +301,9 @@ bool forward_tiles_192(int64_t T, int64_t V) {
 }
 
 // Kept logits: fp32, T * logits_cache_row(V) of them in panels (kept_logit), element (t, v) = hidden[t] . W[v].  A backward that is given them
-// computes d_logits from 4 bytes per logit instead of from a pass over W and a T x V x H product.  Offered for 16-bit
-// inputs while the cache is no larger than the weight it came from: T * V * 4 <= V * H * 2, i.e. up to H / 2 tokens;
-// beyond that nothing of size T x V is ever kept.
+// computes d_logits from 4 bytes per logit instead of from a pass over W and a T x V x H product.  Never larger than the weight they
+// came from.  16-bit inputs: T * V * 4 <= V * H * 2, i.e. up to H / 2 tokens, and nothing beyond; fp32 inputs: all of them up to H tokens, of
+// the first rows of W up to 4 H where the planes run (few_f32_cache_bytes, terms_cache_bytes).
 int64_t logits_cache_row(int64_t V) { return round_up(V, 64); }
 int64_t logits_cache_max_tokens(int64_t H, size_t esz) { return esz == 2 ? H / 2 : 0; }
 
@@ -540,7 +540,9 @@ bool dh_sum_deep(int slices, int64_t workgroups) { return slices > 8 && 2 * work
 // tokens, 200: 1090 / 1090, 100: 922 / 868.
 // The width of the tiles for all tokens / for these, 1000 tokens, d_hidden and d_weight with what surrounds them, H=4096: 100: 516 / 484, 300:
 // 900 / 787, 350: 942 / 828, 400: 999 / 954, 560: 1301 / 1185, from 600 on and at 200 to 256 level; H=3584, 300: 897 / 819, 560: 1339 / 1227;
-// forward + backward, 700 tokens with a frozen head 1438 / 1329, H=5120, 1500: 4901 / 4616, H=896, 700: 627 / 602.
+// forward + backward, 700 tokens with a frozen head 1438 / 1329, H=5120, 1500: 4901 / 4616, H=896, 700: 627 / 602; the whole step of 1000 tokens
+// of fp16, H=4096, fixed masks, nine runs a side that differ by up to 0.5 %: 200: 1510 / 1510, 300: 1782 / 1683, 350: 1832 / 1724, 400: 1888 / 1854,
+// 560: 2187 / 2082, 700: 2304 / 2310, all: 2714 / 2713; H=5120, 300 of 700, frozen head: 1707 / 1548.
 DhSlices dh_slices_by_rows(int64_t T, int64_t H, int64_t vchunk, bool wide, int ksplit) {
   DhSlices d = {};
   const int64_t room = (int64_t)ksplit * (int64_t)(align256((size_t)T * H * 4) / 4), tile = wide ? 256 : 192;

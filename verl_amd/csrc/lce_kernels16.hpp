@@ -172,8 +172,9 @@ LCE_DEV void fwd16_body(const FwdArgs<typename Cfg::TIN>& p, int64_t n0, int s, 
       // With kept logits a column is stored just before it is folded in, so that the stores leave during the fold, and the next
       // tile's first loads come behind both: the K loop waits on counts of outstanding vector-memory operations, and with the stores
       // older than every load it waits for, those counts mean what they say.  (With six products there are not the registers for it:
-      // the stores first, then the loads, then the fold.)  Forward + backward against that order, us: H=896, 130 tokens 261 -> 258, 299
-      // with a frozen head 300 -> 295; H=3584, 256: 896 -> 892, 1000: 2934 -> 2922, 1700: 4849 -> 4833; H=5120, 400: 2068 -> 2055.
+      // the stores first, then the loads, then the fold.)  Forward + backward against that order, us, nine runs a side in turn: H=896, 300
+      // tokens with a frozen head 302.9 -> 296.4; H=3584, 333: 1228 -> 1216, 512: 1535 -> 1524, 1000: 2921 -> 2902 (2911 to 2925, 2897 to 2904), 1700:
+      // 4817 -> 4800; 0.2 to 0.3 % and within the runs' spread for 400 of H=5120 and 1000 of H=4096.
       constexpr bool kWithFold = KEEP && Cfg::TERMS == 1;
       if constexpr (KEEP) {
         if (Cfg::TERMS == 1 || m0 < p.keep_rows) {
@@ -707,8 +708,9 @@ LCE_DEV void gemm16_tn_tile(const GemmArgs<typename Cfg::TIN>& pin, int bid, cha
 // tile is six slabs of 1.2 to 1.5 us, and a workgroup per tile paid another 9 us for its start, its first loads, the drain of
 // its last and its stores.  A finished tile leaves the accumulators during the next one's first k-step (stream_slab_over: 384
 // conversions beside 64 MFMAs, some 2800 cycles for 4400 + 1024 one behind the other), and a last slab of up to 32 tokens is one k-step: kernel at 333
-// tokens of H=3584 432 -> 416 us, 512: 496 -> 487, 1000: 908 -> 902; step 270: 1203 -> 1187, 333: 1268 -> 1251, 500: 1575 -> 1561, 400 of
-// H=5120 2117 -> 2089, from 1000 on level.  Without its stores it takes 347, 443 and 811: the 1.09 GB of results cost 45 to 90 us
+// tokens of H=3584 432 -> 416 us, 512: 496 -> 487, 1000: 908 -> 902.  Forward + backward with neither / the first / both: 270 tokens 1181 / 1173 / 1163,
+// 333: 1234 / 1226 / 1216, 600: 2037 / 2027 / 2018; where the last slab is a whole one 384: 1279 / 1271 / 1272, 500: 1541 / 1534 / 1535, 1000: 2922 /
+// 2914 / 2917 (runs of a side differ by up to 0.5 %).  Without its stores it takes 347, 443 and 811: the 1.09 GB of results cost 45 to 90 us
 // wherever in the tile they are issued (workgroups set off by a quarter of a tile against each other: level).
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NTHREADS) void lce_dw16_kernel(GemmArgs<typename Cfg::TIN> p) {

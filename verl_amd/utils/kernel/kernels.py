@@ -148,9 +148,9 @@ def efficient_entropy_forward(
 
 def forward_keeping_logits(hidden, weight, labels, reduction=2, temperature=1.0, dist_process_group=None, *, keep_logits=True):
     """``efficient_entropy_forward`` plus a sixth value: the kept logits for ``efficient_entropy_backward(...,
-    logits_cache=)``, or ``None`` where the library keeps none (16-bit inputs: more tokens than half the hidden
-    size; fp32: four times the hidden size; ``keep_logits=False``).
-    ``None`` too where there is no memory for them.
+    logits_cache=)``, or ``None``: with ``keep_logits=False``, where the library keeps none (``kept_logits_size``; 16-bit
+    inputs: more tokens than half the hidden size; fp32: more than the hidden size with at most 255 tokens, beyond those more
+    than four times the hidden size or a vocabulary too small for the planes), and where there is no memory for them.
     With few tokens fp32 ``[T, V]`` is a fraction of the weight itself, so the autograd node keeps it like any activation
     and the backward skips the pass over ``[V, H]`` and the ``T x V x H`` product that recompute it (not in the
     reference, which always recomputes)."""
